@@ -287,6 +287,37 @@ int32_t qllm_fp4_gemm_bf16_tall_split(const qllm_fp4_matrix* matrix,
                                       uint32_t segment_count, uint32_t batch,
                                       void* stream);
 
+/* The three with a workspace (16-byte aligned, at least
+ * qllm_fp4_tall_workspace_bytes()) in which a launch may leave parts of its sums:
+ * a batch whose tiles are too few for the GPU is cut along K over more
+ * workgroups, and a second launch adds the parts in order and does the epilogue.
+ * NULL: one launch, as above. */
+size_t qllm_fp4_tall_workspace_bytes(void);
+int32_t qllm_fp4_gemm_bf16_tall_cut(const qllm_fp4_matrix* matrix, const void* input,
+                                    size_t input_bytes, void* output,
+                                    uint32_t output_kind, const float* residual,
+                                    uint32_t batch, void* workspace,
+                                    size_t workspace_bytes, void* stream);
+int32_t qllm_fp4_swiglu_bf16_tall_cut(const qllm_fp4_matrix* gate,
+                                      const qllm_fp4_matrix* up, const void* input,
+                                      size_t input_bytes, void* output_bf16,
+                                      uint32_t batch, void* workspace,
+                                      size_t workspace_bytes, void* stream);
+int32_t qllm_fp4_gemm_bf16_tall_split_cut(const qllm_fp4_matrix* matrix,
+                                          const void* input, size_t input_bytes,
+                                          const qllm_gemm_segment* segments,
+                                          uint32_t segment_count, uint32_t batch,
+                                          void* workspace, size_t workspace_bytes,
+                                          void* stream);
+/* The parts alone, F32 [parts][batch][rows], for a norm that adds them
+ * (qllm_rms_norm_residual_batch); parts: 1 .. 16 and at most padded_columns / 64.
+ * qllm_fp4_tall_parts: into how many a batch is best cut (1 = not at all); their
+ * bytes are at most qllm_fp4_tall_workspace_bytes() where that is more than 1. */
+uint32_t qllm_fp4_tall_parts(const qllm_fp4_matrix* matrix, uint32_t batch);
+int32_t qllm_fp4_gemm_bf16_tall_partial(const qllm_fp4_matrix* matrix, const void* input,
+                                        size_t input_bytes, float* partials,
+                                        uint32_t parts, uint32_t batch, void* stream);
+
 /* replaces fp4_embedding_batch (transformer_kernels.hpp:68-70).  A token
  * outside the matrix (tokens[r] >= rows; a device-side selection over logits
  * without a finite maximum yields 0xffffffff) reads nothing and gives a row of

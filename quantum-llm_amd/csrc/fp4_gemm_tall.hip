@@ -11,7 +11,10 @@
 // its weights straight from the provider's streaming layout - the 16-byte
 // piece a lane loads per (tile, chunk) is its B operand for the chunk's four
 // instructions, no LDS and no shuffle - and shares the activation tile of the
-// chunk through LDS (double-buffered, one barrier per 64 columns of K).
+// chunk through LDS (double-buffered, one barrier per 64 columns of K).  Batches
+// whose tiles are too few for the GPU - short prompts, and long ones against
+// matrices of few rows - are cut along K and use lower workgroups
+// (fp4_gemm_short_kernel, plan_tall).
 //
 // Scale schemes:
 //  * UE8M0 per 32: the power-of-two scale is folded into the nibble -> bf16
@@ -68,6 +71,11 @@ struct TallArgs {
   uint32_t batch;
   uint32_t m_tiles;
   uint32_t n_tiles;
+  // K cut over `splits` workgroups per tile: part p of a tile sums its share of
+  // the chunks into partials[p][batch][rows] (SWIGLU: partials[p][2][batch]
+  // [rows], gate before up), and whoever reads them adds the parts in order
+  uint32_t splits;
+  float* partials;
   void* output;                  // [batch, rows]
   uint32_t output_kind;
   const float* residual;
@@ -77,6 +85,13 @@ struct TallArgs {
   uint32_t segment_kind[3];
   void* segment_output[3];
 };
+
+// Workgroups are dealt to the eight XCDs in turn, so XCD x runs the ids x,
+// x + 8, ...: the position that gives each XCD a contiguous range instead.
+__device__ __forceinline__ uint32_t xcd_contiguous(uint32_t id, uint32_t total) {
+  const uint32_t xcd = id % 8u;
+  return xcd * (total / 8u) + min(xcd, total % 8u) + id / 8u;
+}
 
 __device__ __forceinline__ void store_value(void* output, uint32_t kind,
                                             size_t index, float value) {
@@ -165,8 +180,121 @@ struct Operand<kSchemeF16> {
   }
 };
 
-// Workgroup (m_tile, n_tile): activation rows [128 m_tile, +128), weight rows
-// [256 n_tile, +256).
+// Where the output columns from `column` on go: the matrix's output, or the
+// segment that holds them (segments are multiples of 32 rows).
+struct Destination {
+  void* output;
+  uint32_t kind;
+  uint32_t width;
+  uint32_t first;   // the destination's first column in the matrix
+};
+__device__ __forceinline__ Destination destination_of(const TallArgs& args,
+                                                      uint32_t column) {
+  if (!args.segments) return {args.output, args.output_kind, args.rows, 0u};
+  uint32_t segment = 0, first = 0;
+  while (segment + 1u < args.segments &&
+         column >= first + args.segment_rows[segment]) {
+    first += args.segment_rows[segment];
+    ++segment;
+  }
+  return {args.segment_output[segment], args.segment_kind[segment],
+          args.segment_rows[segment], first};
+}
+
+// bf16(bf16(silu(gate)) * up), the rounding points of the SiLU-product launch
+__device__ __forceinline__ uint16_t swiglu_bits(float gate, float up) {
+  const float activated = bf16_round(gate / (1.0f + expf(-gate)));
+  return static_cast<uint16_t>(f32_to_bf16_bits(activated * up));
+}
+
+// Stores a wave's accumulators.  D register i of lane (n, g): activation row
+// first_m + 16 mt + 4 g + i, weight row 32 tile + 16 j + n.
+template <int MT, int T, bool SWIGLU>
+__device__ __forceinline__ void store_tiles(const TallArgs& args, uint32_t part,
+                                            uint32_t first_m,
+                                            const uint32_t (&tile_index)[T],
+                                            uint32_t tile_count,
+                                            const f32x4 (&acc)[MT][T][2]) {
+  const uint32_t n = threadIdx.x & 15u;
+  const uint32_t g = (threadIdx.x & 63u) >> 4;
+  if (args.splits > 1u) {
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      if (tile_index[t] >= tile_count) continue;
+      const uint32_t plane = SWIGLU ? part * 2u + t : part;
+#pragma unroll
+      for (uint32_t j = 0; j < 2u; ++j) {
+        const uint32_t column = tile_index[t] * kTileRows + 16u * j + n;
+        if (column >= args.rows) continue;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (uint32_t i = 0; i < 4u; ++i) {
+            const uint32_t row = first_m + 16u * mt + 4u * g + i;
+            if (row >= args.batch) continue;
+            args.partials[(static_cast<size_t>(plane) * args.batch + row) *
+                              args.rows + column] = acc[mt][t][j][i];
+          }
+      }
+    }
+    return;
+  }
+  if constexpr (SWIGLU) {
+    if (tile_index[0] >= tile_count) return;
+#pragma unroll
+    for (uint32_t j = 0; j < 2u; ++j) {
+      const uint32_t column = tile_index[0] * kTileRows + 16u * j + n;
+      if (column >= args.rows) continue;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) {
+          const uint32_t row = first_m + 16u * mt + 4u * g + i;
+          if (row >= args.batch) continue;
+          static_cast<uint16_t*>(args.output)[static_cast<size_t>(row) * args.rows +
+                                              column] =
+              swiglu_bits(acc[mt][0][j][i], acc[mt][1][j][i]);
+        }
+    }
+    return;
+  }
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    if (tile_index[t] >= tile_count) continue;
+    const uint32_t tile_first = tile_index[t] * kTileRows;
+    const Destination to = destination_of(args, tile_first);
+    const bool add = args.residual && !args.segments;
+#pragma unroll
+    for (uint32_t j = 0; j < 2u; ++j) {
+      const uint32_t column = tile_first + 16u * j + n;
+      if (column >= args.rows) continue;
+      // the residual's values are fetched together: it may be the output itself,
+      // and a load after a store would wait for every one before it
+      float rest[MT][4];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) {
+          const uint32_t row = min(first_m + 16u * mt + 4u * g + i, args.batch - 1u);
+          rest[mt][i] =
+              add ? args.residual[static_cast<size_t>(row) * args.rows + column] : 0.0f;
+        }
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) {
+          const uint32_t row = first_m + 16u * mt + 4u * g + i;
+          if (row >= args.batch) continue;
+          store_value(to.output, to.kind,
+                      static_cast<size_t>(row) * to.width + (column - to.first),
+                      add ? acc[mt][t][j][i] + rest[mt][i] : acc[mt][t][j][i]);
+        }
+    }
+  }
+}
+
+// Workgroup (part, m_tile, n_tile): activation rows [128 m_tile, +128), weight
+// rows [256 n_tile, +256), chunks of the part.
 //
 // SWIGLU: a wave's two tiles are the same 32 rows of the gate and of the up
 // matrix (a workgroup covers 128 rows of each), and the epilogue writes
@@ -187,15 +315,17 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_tall_kernel(
   const uint32_t K = args.padded_columns;
   const uint32_t chunks = K / kChunk;
 
-  // Workgroups are dealt to the eight XCDs in turn, so XCD x runs the ids
-  // x, x + 8, ...: give it a contiguous range of tiles instead.  Within the
+  // An XCD gets a contiguous range of tiles.  Within the
   // range the tiles go band by band (kBand activation tiles high), column by
   // column: the 64 workgroups an XCD runs at a time then cover about 8 x 8
   // tiles and fetch 8 + 8 operand tiles per K step into its L2 rather than
   // 64 + 1.
-  const uint32_t total = args.m_tiles * args.n_tiles;
-  const uint32_t xcd = blockIdx.x % 8u;
-  const uint32_t id = xcd * (total / 8u) + min(xcd, total % 8u) + blockIdx.x / 8u;
+  const uint32_t tiles = args.m_tiles * args.n_tiles;
+  const uint32_t position = xcd_contiguous(blockIdx.x, tiles * args.splits);
+  const uint32_t part = position / tiles;
+  const uint32_t id = position - part * tiles;
+  const uint32_t first_chunk = chunks * part / args.splits;
+  const uint32_t end_chunk = chunks * (part + 1u) / args.splits;
   const uint32_t band_tiles = kBand * args.n_tiles;
   const uint32_t band = id / band_tiles;
   const uint32_t in_band = id - band * band_tiles;
@@ -283,14 +413,14 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_tall_kernel(
     }
   };
 
-  fetch_activations(0u);
-  fetch_weights(std::integral_constant<int, 0>{}, 0u);
+  fetch_activations(first_chunk);
+  fetch_weights(std::integral_constant<int, 0>{}, first_chunk);
   store_activations(0u);
 
   const auto step = [&]<int slot>(std::integral_constant<int, slot>,
                                   uint32_t chunk) {
     __syncthreads();   // tile[slot] is complete; tile[slot ^ 1] is free
-    const uint32_t next = chunk + 1u < chunks ? chunk + 1u : chunk;
+    const uint32_t next = chunk + 1u < end_chunk ? chunk + 1u : chunk;
     fetch_activations(next);
     fetch_weights(std::integral_constant<int, slot ^ 1>{}, next);
     // the loads stay here, a whole step ahead of their use (left alone, the
@@ -328,74 +458,269 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_tall_kernel(
         }
       }
     }
-    if (chunk + 1u < chunks) store_activations(slot ^ 1u);
+    if (chunk + 1u < end_chunk) store_activations(slot ^ 1u);
   };
-  for (uint32_t chunk = 0; chunk < chunks; chunk += 2u) {
+  for (uint32_t chunk = first_chunk; chunk < end_chunk; chunk += 2u) {
     step(std::integral_constant<int, 0>{}, chunk);
-    if (chunk + 1u < chunks) step(std::integral_constant<int, 1>{}, chunk + 1u);
+    if (chunk + 1u < end_chunk) step(std::integral_constant<int, 1>{}, chunk + 1u);
   }
 
-  // D register i of lane (n, g): activation row 16 mt + 4 g + i, weight row
-  // 32 tile + 16 j + n
-  if constexpr (SWIGLU) {
-    if (tile_index[0] >= tile_count) return;
+  store_tiles<kTilesM, kTilesPerWave, SWIGLU>(args, part, first_m, tile_index,
+                                              tile_count, acc);
+}
+
+// Short batches: up to 64 rows a workgroup (16 MT), 128 weight rows (SWIGLU: of
+// each of the two matrices).  Here the weights' way from memory is what there is
+// to hide, not the matrix cores' time: a wave keeps its weights of the next four
+// chunks on their way in registers (with the one of fp4_gemm_tall_kernel a step
+// waits out most of a memory round trip), the activations of the next two steps
+// likewise, and a step covers 4 / MT chunks so that its barrier costs the same
+// whatever the height.
+template <int SCHEME, int MT, int T, bool SWIGLU>
+__global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
+    const TallArgs args) {
+  using Op = Operand<SCHEME>;
+  using Vector = typename Op::Vector;
+  constexpr bool F16 = SCHEME == kSchemeF16;
+  static_assert(!SWIGLU || T == 2);
+  constexpr uint32_t kAhead = 4;                    // chunks of weights in flight
+  constexpr uint32_t kSpan = 4 / MT;                // chunks per step
+  constexpr uint32_t kRow = kSpan * kChunk * 2u + 16u;
+  constexpr uint32_t kPieces = 16u * MT * kSpan * 8u / (kWaves * 64u);
+  static_assert(kPieces * kWaves * 64u == 16u * MT * kSpan * 8u);
+  __shared__ __attribute__((aligned(16))) uint8_t tile[2][16 * MT * kRow];
+
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t n = lane & 15u;
+  const uint32_t g = lane >> 4;
+  const uint32_t K = args.padded_columns;
+  const uint32_t chunks = K / kChunk;
+
+  // activation tiles of one weight tile run side by side on an XCD, then the
+  // weight tiles of a part: weights and activations come from its L2
+  const uint32_t tiles = args.m_tiles * args.n_tiles;
+  const uint32_t position = xcd_contiguous(blockIdx.x, tiles * args.splits);
+  const uint32_t part = position / tiles;
+  const uint32_t id = position - part * tiles;
+  const uint32_t first_m = id % args.m_tiles * (16u * MT);
+  const uint32_t n_tile = id / args.m_tiles;
+  const uint32_t first_chunk = chunks * part / args.splits;
+  const uint32_t end_chunk = chunks * (part + 1u) / args.splits;
+
+  const uint32_t tile_count = (args.rows + kTileRows - 1u) / kTileRows;
+  const uint8_t* weight_stream[T];
+  const uint8_t* scale_stream[T];
+  uint32_t tile_index[T];
 #pragma unroll
-    for (uint32_t j = 0; j < 2u; ++j) {
-      const uint32_t column = tile_index[0] * kTileRows + 16u * j + n;
-      if (column >= args.rows) continue;
+  for (int t = 0; t < T; ++t) {
+    tile_index[t] = SWIGLU ? n_tile * kWaves + wave : (n_tile * kWaves + wave) * T + t;
+    const size_t stream = min(tile_index[t], tile_count - 1u);
+    weight_stream[t] = (SWIGLU && t ? args.up_weights : args.weights) +
+                       stream * chunks * (kTileRows * 32u) + lane * 16u;
+    scale_stream[t] = (SWIGLU && t ? args.up_scales : args.scales) +
+                      stream * chunks * (kTileRows * (F16 ? 8u : 2u)) +
+                      (F16 ? ((g >> 1) * 16u + n) * 8u : n * 4u);
+  }
+
+  // piece p of a step's activations: row p / (8 kSpan), 16 bytes at column
+  // piece p % (8 kSpan).  Rows past the batch read its last row and are not
+  // stored; columns past K read its last ones and meet no weights.
+  const uint8_t* source_row[kPieces];
+  uint32_t source_column[kPieces], target[kPieces];
 #pragma unroll
-      for (uint32_t mt = 0; mt < kTilesM; ++mt)
+  for (uint32_t p = 0; p < kPieces; ++p) {
+    const uint32_t piece = p * kWaves * 64u + threadIdx.x;
+    const uint32_t row = piece / (8u * kSpan);
+    source_column[p] = piece % (8u * kSpan) * 16u;
+    target[p] = row * kRow + source_column[p];
+    source_row[p] = reinterpret_cast<const uint8_t*>(args.activations) +
+                    static_cast<size_t>(min(first_m + row, args.batch - 1u)) * K * 2u;
+  }
+  const uint32_t fragment_offset = n * kRow + g * 16u;
+
+  f32x4 acc[MT][T][2];
 #pragma unroll
-        for (uint32_t i = 0; i < 4u; ++i) {
-          const uint32_t row = first_m + 16u * mt + 4u * g + i;
-          if (row >= args.batch) continue;
-          const float gate = acc[mt][0][j][i];
-          const float activated = bf16_round(gate / (1.0f + expf(-gate)));
-          static_cast<uint16_t*>(args.output)[static_cast<size_t>(row) * args.rows +
-                                              column] =
-              static_cast<uint16_t>(f32_to_bf16_bits(activated * acc[mt][1][j][i]));
-        }
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (uint32_t j = 0; j < 2u; ++j) acc[mt][t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  uint4 staged[2][kPieces];
+  const auto fetch_activations = [&]<int slot>(std::integral_constant<int, slot>,
+                                               uint32_t chunk) {
+#pragma unroll
+    for (uint32_t p = 0; p < kPieces; ++p)
+      staged[slot][p] = *reinterpret_cast<const uint4*>(
+          source_row[p] + min(chunk * (kChunk * 2u) + source_column[p], K * 2u - 16u));
+  };
+  const auto store_activations = [&]<int slot>(std::integral_constant<int, slot>) {
+#pragma unroll
+    for (uint32_t p = 0; p < kPieces; ++p) {
+      uint4 v = staged[slot][p];
+      v.x = Op::stage(v.x); v.y = Op::stage(v.y);
+      v.z = Op::stage(v.z); v.w = Op::stage(v.w);
+      *reinterpret_cast<uint4*>(&tile[slot][target[p]]) = v;
     }
+  };
+  uint4 codes[kAhead][T];
+  uint2 scales[kAhead][T];
+  const auto fetch_weights = [&]<int slot>(std::integral_constant<int, slot>,
+                                           uint32_t chunk) {
+    // past the part's end every lane reads one line of the activations: the
+    // next chunk would go to memory for nothing
+    const auto* idle = reinterpret_cast<const uint8_t*>(args.activations);
+    const bool live = chunk < end_chunk;
+    const size_t at = chunk;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      codes[slot][t] = *reinterpret_cast<const uint4*>(
+          live ? weight_stream[t] + at * (kTileRows * 32u) : idle);
+      if constexpr (F16) {
+        scales[slot][t] = *reinterpret_cast<const uint2*>(
+            live ? scale_stream[t] + at * (kTileRows * 8u) : idle);
+      } else {
+        scales[slot][t].x = *reinterpret_cast<const uint32_t*>(
+            live ? scale_stream[t] + at * (kTileRows * 2u) : idle);
+        scales[slot][t].y = 0u;
+      }
+    }
+  };
+
+  const auto multiply = [&]<int slot, int buffer, int c>(
+                            std::integral_constant<int, slot>,
+                            std::integral_constant<int, buffer>,
+                            std::integral_constant<int, c>) {
+#pragma unroll
+    for (uint32_t s = 0; s < 2u; ++s) {
+      Vector a[MT];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        a[mt] = __builtin_bit_cast(
+            Vector, *reinterpret_cast<const uint4*>(&tile[buffer][
+                        mt * 16u * kRow + fragment_offset + c * 128u + s * 64u]));
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const uint4 q = codes[slot][t];
+        const uint32_t packed[4] = {q.x, q.y, q.z, q.w};   // index 2j + s
+#pragma unroll
+        for (uint32_t j = 0; j < 2u; ++j) {
+          const uint32_t word = j ? scales[slot][t].y : scales[slot][t].x;
+          const uint32_t f16_bits = s ? word >> 16 : word & 0xffffu;
+          const float fold =
+              F16 ? 1.0f
+                  : ue8m0_to_f32((scales[slot][t].x >> (8u * (2u * j + s))) & 0xffu);
+          Vector w[Op::kParts];
+          Op::weights(packed[2u * j + s], fold, f16_bits, w);
+#pragma unroll
+          for (int half = 0; half < Op::kParts; ++half)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+              acc[mt][t][j] = Op::mfma(a[mt], w[half], acc[mt][t][j]);
+        }
+      }
+    }
+  };
+
+  using std::integral_constant;
+  // in the order in which the loop waits for them
+  fetch_activations(integral_constant<int, 0>{}, first_chunk);
+  fetch_weights(integral_constant<int, 0>{}, first_chunk);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_activations(integral_constant<int, 1>{}, first_chunk + kSpan);
+  fetch_weights(integral_constant<int, 1>{}, first_chunk + 1u);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_weights(integral_constant<int, 2>{}, first_chunk + 2u);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_weights(integral_constant<int, 3>{}, first_chunk + 3u);
+  __builtin_amdgcn_sched_barrier(0);
+  store_activations(integral_constant<int, 0>{});
+
+  // a chunk's weights are refilled as soon as they have been multiplied
+  const auto one_chunk = [&]<int slot, int buffer, int c>(
+                             integral_constant<int, slot> s,
+                             integral_constant<int, buffer> b,
+                             integral_constant<int, c> in_step, uint32_t chunk) {
+    if (chunk < end_chunk) multiply(s, b, in_step);
+    // the loads stay here: moved up they would need registers of their own and
+    // copies at the loop's end, which wait for them, moved down they come late
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_weights(s, chunk + kAhead);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  const auto step = [&]<int first_slot, int buffer>(integral_constant<int, first_slot>,
+                                                    integral_constant<int, buffer> b,
+                                                    uint32_t chunk) {
+    __syncthreads();   // tile[buffer] is complete; the other one is free
+    fetch_activations(b, chunk + 2u * kSpan);
+    __builtin_amdgcn_sched_barrier(0);
+    one_chunk(integral_constant<int, first_slot>{}, b, integral_constant<int, 0>{}, chunk);
+    if constexpr (kSpan > 1)
+      one_chunk(integral_constant<int, first_slot + 1>{}, b,
+                integral_constant<int, 1>{}, chunk + 1u);
+    if constexpr (kSpan > 2) {
+      one_chunk(integral_constant<int, first_slot + 2>{}, b,
+                integral_constant<int, 2>{}, chunk + 2u);
+      one_chunk(integral_constant<int, first_slot + 3>{}, b,
+                integral_constant<int, 3>{}, chunk + 3u);
+    }
+    store_activations(integral_constant<int, buffer ^ 1>{});
+  };
+  constexpr integral_constant<int, 0> even;
+  constexpr integral_constant<int, 1> odd;
+  // Whole rounds of four chunks (eight at MT = 1): a step past the part's end
+  // makes its loads and multiplies nothing, so that every wait can count on the
+  // same loads having been made since.
+  for (uint32_t chunk = first_chunk; chunk < end_chunk;) {
+    step(even, even, chunk);
+    chunk += kSpan;
+    step(integral_constant<int, kSpan % kAhead>{}, odd, chunk);
+    chunk += kSpan;
+    if constexpr (kSpan == 1) {
+      step(integral_constant<int, 2>{}, even, chunk);
+      chunk += kSpan;
+      step(integral_constant<int, 3>{}, odd, chunk);
+      chunk += kSpan;
+    }
+  }
+  store_tiles<MT, T, SWIGLU>(args, part, first_m, tile_index, tile_count, acc);
+}
+
+// Adds the parts of a launch whose K was cut, four columns per thread, and
+// stores what its epilogue would have stored.
+template <bool SWIGLU>
+__global__ __launch_bounds__(256) void tall_parts_kernel(const TallArgs args) {
+  const uint32_t column = (blockIdx.x * 256u + threadIdx.x) * 4u;
+  const uint32_t row = blockIdx.y;
+  if (column >= args.rows) return;
+  const size_t plane = static_cast<size_t>(args.batch) * args.rows;
+  const float* source =
+      args.partials + static_cast<size_t>(row) * args.rows + column;
+  const size_t step = SWIGLU ? 2u * plane : plane;
+  f32x4 sum = *reinterpret_cast<const f32x4*>(source);
+  f32x4 up{};
+  if constexpr (SWIGLU) up = *reinterpret_cast<const f32x4*>(source + plane);
+  for (uint32_t part = 1; part < args.splits; ++part) {
+    source += step;
+    sum += *reinterpret_cast<const f32x4*>(source);
+    if constexpr (SWIGLU) up += *reinterpret_cast<const f32x4*>(source + plane);
+  }
+  if constexpr (SWIGLU) {
+    uint16_t* out = static_cast<uint16_t*>(args.output) +
+                    static_cast<size_t>(row) * args.rows + column;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[i] = swiglu_bits(sum[i], up[i]);
     return;
   }
+  const Destination to = destination_of(args, column);
 #pragma unroll
-  for (uint32_t t = 0; t < kTilesPerWave; ++t) {
-    if (tile_index[t] >= tile_count) continue;
-    const uint32_t tile_first = tile_index[t] * kTileRows;
-    // destination of the tile's columns (segments are multiples of 32 rows)
-    void* destination = args.output;
-    uint32_t kind = args.output_kind;
-    uint32_t width = args.rows;
-    uint32_t local_first = tile_first;
-    if (args.segments) {
-      uint32_t segment = 0;
-      while (segment + 1u < args.segments &&
-             local_first >= args.segment_rows[segment]) {
-        local_first -= args.segment_rows[segment];
-        ++segment;
-      }
-      destination = args.segment_output[segment];
-      kind = args.segment_kind[segment];
-      width = args.segment_rows[segment];
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < 2u; ++j) {
-      const uint32_t column = tile_first + 16u * j + n;
-      if (column >= args.rows) continue;
-      const uint32_t local_column = local_first + 16u * j + n;
-#pragma unroll
-      for (uint32_t mt = 0; mt < kTilesM; ++mt)
-#pragma unroll
-        for (uint32_t i = 0; i < 4u; ++i) {
-          const uint32_t row = first_m + 16u * mt + 4u * g + i;
-          if (row >= args.batch) continue;
-          float value = acc[mt][t][j][i];
-          if (args.residual && !args.segments)
-            value += args.residual[static_cast<size_t>(row) * args.rows + column];
-          store_value(destination, kind,
-                      static_cast<size_t>(row) * width + local_column, value);
-        }
-    }
+  for (int i = 0; i < 4; ++i) {
+    float value = sum[i];
+    if (args.residual && !args.segments)
+      value += args.residual[static_cast<size_t>(row) * args.rows + column + i];
+    store_value(to.output, to.kind,
+                static_cast<size_t>(row) * to.width + (column + i - to.first), value);
   }
 }
 
@@ -408,21 +733,167 @@ bool tall_matrix_ok(const qllm_fp4_matrix* m) {
          (m->tile_rows == 0u || m->tile_rows == kTileRows);
 }
 
-int32_t launch_tall(TallArgs args, uint32_t scheme, hipStream_t stream) {
-  args.m_tiles = (args.batch + kRowsM - 1u) / kRowsM;
+// How a launch is laid out: 16 `height` rows of activations per workgroup and
+// `splits` parts of K.
+//
+// Chosen by what the busiest CU will take.  With W workgroups per part it runs
+// n = ceil(W splits / 256) of them, each over ceil(chunks / splits) chunks; a
+// chunk costs `alone` ns where n = 1 (its round trips and barriers show) and
+// n * `shared` where workgroups hide each other's.  Parts are written and read
+// once more, at 6.2 TB/s, and take a launch of their own where no norm adds
+// them.  The constants are a fit to 1300 timed launches over weights that come
+// from memory (nine matrices of [2048, 2048] to [17408, 5120], 8 to 3000 rows;
+// 7 % root mean square error; the chosen layout is 1.5 % slower than the best of
+// those timed on average).  What it gives over one workgroup per 128 rows and
+// tile: [5120, 17408] with binary16 scales, 48 rows 400 -> 27 us, 300 rows
+// 404 -> 97, 1000 rows 405 -> 254, 2000 rows 668 -> 498; [10240, 5120] 127 ->
+// 25, 135 -> 73, 211 -> 190, 333 -> 327; gate and up of [17408, 5120] 129 -> 54,
+// 221 -> 195, then unchanged.
+struct TallPlan {
+  uint32_t height;
+  uint32_t splits;
+};
+
+constexpr uint32_t kMaximumParts = 16;
+constexpr size_t kPartsBytes = size_t{128} << 20;
+
+struct ChunkCost {
+  float alone, shared;   // ns
+};
+// [scheme][SwiGLU][log2 height]
+constexpr ChunkCost kChunkCost[2][2][4] = {
+    {{{160.f, 150.f}, {195.f, 180.f}, {365.f, 250.f}, {1160.f, 780.f}},
+     {{250.f, 325.f}, {335.f, 345.f}, {605.f, 420.f}, {1215.f, 780.f}}},
+    {{{220.f, 230.f}, {300.f, 280.f}, {545.f, 390.f}, {1690.f, 1265.f}},
+     {{380.f, 440.f}, {515.f, 500.f}, {985.f, 715.f}, {1710.f, 1230.f}}}};
+
+uint32_t weight_rows_of(uint32_t height, bool swiglu) {
+  return (height == 8u && !swiglu ? kTilesN : kWaves) * kTileRows;
+}
+
+uint32_t workgroups_of(uint32_t rows, uint32_t batch, uint32_t height, bool swiglu) {
+  const uint32_t weight_rows = weight_rows_of(height, swiglu);
+  return (batch + 16u * height - 1u) / (16u * height) *
+         ((rows + weight_rows - 1u) / weight_rows);
+}
+
+size_t parts_bytes(uint32_t rows, uint32_t batch, uint32_t splits, bool swiglu) {
+  return splits > 1u ? size_t{splits} * (swiglu ? 2u : 1u) * batch * rows * 4u : 0u;
+}
+
+// At most `workspace_bytes` of parts; `separate`: they are added by a launch of
+// their own.
+TallPlan plan_tall(uint32_t rows, uint32_t padded_columns, uint32_t batch,
+                   uint32_t scheme, bool swiglu, bool separate,
+                   size_t workspace_bytes, uint32_t fixed_splits = 0u) {
+  const uint32_t chunks = padded_columns / kChunk;
+  const uint32_t first = fixed_splits ? fixed_splits : 1u;
+  // A part has two rounds of a workgroup's four chunks in flight at least; parts
+  // are added four columns at a time, a row per grid row.  Matrices far below the
+  // timed ones, which no decoder layer has, stay whole: the fit says nothing there.
+  const bool whole = rows % 4u || batch > 65535u || chunks < 16u ||
+                     uint64_t{rows} * padded_columns < (1u << 20);
+  const uint32_t last = fixed_splits                  ? fixed_splits
+                        : whole                       ? 1u
+                        : chunks / 8u < kMaximumParts ? chunks / 8u
+                                                      : kMaximumParts;
+  TallPlan best{};
+  double least = 0.0;
+  for (uint32_t log_height = 0; log_height < 4u; ++log_height) {
+    const uint32_t height = 1u << log_height;
+    // the lowest that holds the batch, or one of the two highest
+    if (height < 4u ? batch > 16u * height || (height == 2u && batch <= 16u)
+                    : batch <= 8u * height)
+      continue;
+    const ChunkCost cost = kChunkCost[scheme][swiglu][log_height];
+    const uint32_t workgroups = workgroups_of(rows, batch, height, swiglu);
+    for (uint32_t splits = first; splits <= last; ++splits) {
+      const size_t bytes = parts_bytes(rows, batch, splits, swiglu);
+      if (!fixed_splits && bytes > workspace_bytes) break;
+      const uint64_t on_one = (uint64_t{workgroups} * splits + 255u) / 256u;
+      const double chunk =
+          on_one > 1u && on_one * cost.shared > cost.alone ? on_one * cost.shared
+                                                           : cost.alone;
+      const double time = (chunks + splits - 1u) / splits * chunk +
+                          (separate ? 2.0 : 1.0) * bytes / 6200.0 +
+                          (separate && splits > 1u ? 4300.0 : 0.0);
+      if (!best.height || time < least) {
+        best = {height, splits};
+        least = time;
+      }
+    }
+  }
+  return best;
+}
+
+template <int SCHEME>
+void start_tall(const TallArgs& args, uint32_t height, bool swiglu, uint32_t grid,
+                hipStream_t stream) {
+  constexpr uint32_t kThreads = kWaves * 64;
+  switch (height) {
+    case 1:
+      if (swiglu)
+        fp4_gemm_short_kernel<SCHEME, 1, 2, true><<<grid, kThreads, 0, stream>>>(args);
+      else
+        fp4_gemm_short_kernel<SCHEME, 1, 1, false><<<grid, kThreads, 0, stream>>>(args);
+      break;
+    case 2:
+      if (swiglu)
+        fp4_gemm_short_kernel<SCHEME, 2, 2, true><<<grid, kThreads, 0, stream>>>(args);
+      else
+        fp4_gemm_short_kernel<SCHEME, 2, 1, false><<<grid, kThreads, 0, stream>>>(args);
+      break;
+    case 4:
+      if (swiglu)
+        fp4_gemm_short_kernel<SCHEME, 4, 2, true><<<grid, kThreads, 0, stream>>>(args);
+      else
+        fp4_gemm_short_kernel<SCHEME, 4, 1, false><<<grid, kThreads, 0, stream>>>(args);
+      break;
+    default:
+      if (swiglu)
+        fp4_gemm_tall_kernel<SCHEME, true><<<grid, kThreads, 0, stream>>>(args);
+      else
+        fp4_gemm_tall_kernel<SCHEME><<<grid, kThreads, 0, stream>>>(args);
+  }
+}
+
+// The parts of a cut launch stay in args.partials.
+int32_t launch_tall(TallArgs args, uint32_t scheme, const TallPlan& plan,
+                    hipStream_t stream) {
   const bool swiglu = args.up_weights != nullptr;
-  const uint32_t rows_per_workgroup = (swiglu ? kWaves : kTilesN) * kTileRows;
-  args.n_tiles = (args.rows + rows_per_workgroup - 1u) / rows_per_workgroup;
-  const uint32_t grid = args.m_tiles * args.n_tiles;
-  if (swiglu && scheme == QLLM_SCALE_F16_BLOCK16)
-    fp4_gemm_tall_kernel<kSchemeF16, true><<<grid, kWaves * 64, 0, stream>>>(args);
-  else if (swiglu)
-    fp4_gemm_tall_kernel<kSchemeUe8m0, true><<<grid, kWaves * 64, 0, stream>>>(args);
-  else if (scheme == QLLM_SCALE_F16_BLOCK16)
-    fp4_gemm_tall_kernel<kSchemeF16><<<grid, kWaves * 64, 0, stream>>>(args);
+  const uint32_t weight_rows = weight_rows_of(plan.height, swiglu);
+  args.m_tiles = (args.batch + 16u * plan.height - 1u) / (16u * plan.height);
+  args.n_tiles = (args.rows + weight_rows - 1u) / weight_rows;
+  args.splits = plan.splits;
+  const uint32_t grid = args.m_tiles * args.n_tiles * plan.splits;
+  if (scheme == QLLM_SCALE_F16_BLOCK16)
+    start_tall<kSchemeF16>(args, plan.height, swiglu, grid, stream);
   else
-    fp4_gemm_tall_kernel<kSchemeUe8m0><<<grid, kWaves * 64, 0, stream>>>(args);
+    start_tall<kSchemeUe8m0>(args, plan.height, swiglu, grid, stream);
   return launched("tall FP4 GEMM");
+}
+
+int32_t add_parts(const TallArgs& args, hipStream_t stream) {
+  const dim3 grid((args.rows / 4u + 255u) / 256u, args.batch);
+  if (args.up_weights)
+    tall_parts_kernel<true><<<grid, 256, 0, stream>>>(args);
+  else
+    tall_parts_kernel<false><<<grid, 256, 0, stream>>>(args);
+  return launched("tall FP4 GEMM parts");
+}
+
+// One launch, or - where the plan cuts K and `workspace` holds the parts - two.
+int32_t run_tall(TallArgs args, uint32_t scheme, void* workspace,
+                 size_t workspace_bytes, hipStream_t stream) {
+  const bool swiglu = args.up_weights != nullptr;
+  const TallPlan plan =
+      plan_tall(args.rows, args.padded_columns, args.batch, scheme, swiglu, true,
+                workspace ? workspace_bytes : 0u);
+  args.partials = static_cast<float*>(workspace);
+  args.splits = plan.splits;
+  const int32_t status = launch_tall(args, scheme, plan, stream);
+  if (status != QLLM_OK || plan.splits == 1u) return status;
+  return add_parts(args, stream);
 }
 
 }  // namespace
@@ -430,31 +901,101 @@ int32_t launch_tall(TallArgs args, uint32_t scheme, hipStream_t stream) {
 
 using namespace qllm;
 
-extern "C" int32_t qllm_fp4_gemm_bf16_tall(const qllm_fp4_matrix* matrix,
-                                           const void* input, size_t input_bytes,
-                                           void* output, uint32_t output_kind,
-                                           const float* residual, uint32_t batch,
-                                           void* stream) {
-  if (!tall_matrix_ok(matrix) || !input || !output || !batch ||
-      batch > (1u << 20) || output_kind > QLLM_OUT_BF16 ||
+namespace {
+
+// The arguments of a launch over `matrix` after the checks that all forms share.
+bool tall_arguments(const qllm_fp4_matrix* matrix, const void* input,
+                    size_t input_bytes, uint32_t batch, TallArgs& args) {
+  if (!tall_matrix_ok(matrix) || !input || !batch || batch > (1u << 20) ||
       (reinterpret_cast<uintptr_t>(input) & 15u) ||
       input_bytes < static_cast<size_t>(batch) * matrix->padded_columns * 2u)
-    return fail(QLLM_INVALID_ARGUMENT, "invalid tall FP4 GEMM");
-  if (residual && output_kind == QLLM_OUT_BF16 &&
-      static_cast<const void*>(residual) == output)
-    return fail(QLLM_INVALID_ARGUMENT,
-                "tall FP4 GEMM: bf16 output cannot alias the f32 residual");
-  TallArgs args{};
+    return false;
   args.weights = matrix->weights;
   args.scales = static_cast<const uint8_t*>(matrix->scales);
   args.activations = static_cast<const uint16_t*>(input);
   args.rows = matrix->rows;
   args.padded_columns = matrix->padded_columns;
   args.batch = batch;
+  return true;
+}
+
+bool workspace_ok(const void* workspace) {
+  return (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0u;
+}
+
+}  // namespace
+
+extern "C" size_t qllm_fp4_tall_workspace_bytes(void) { return kPartsBytes; }
+
+extern "C" uint32_t qllm_fp4_tall_parts(const qllm_fp4_matrix* matrix, uint32_t batch) {
+  if (!tall_matrix_ok(matrix) || !batch) return 1u;
+  return plan_tall(matrix->rows, matrix->padded_columns, batch, matrix->scale_scheme,
+                   false, false, kPartsBytes).splits;
+}
+
+extern "C" int32_t qllm_fp4_gemm_bf16_tall_partial(const qllm_fp4_matrix* matrix,
+                                                   const void* input, size_t input_bytes,
+                                                   float* partials, uint32_t parts,
+                                                   uint32_t batch, void* stream) {
+  TallArgs args{};
+  if (!tall_arguments(matrix, input, input_bytes, batch, args) || !partials ||
+      !parts || parts > kMaximumParts || parts > matrix->padded_columns / kChunk ||
+      !workspace_ok(partials))
+    return fail(QLLM_INVALID_ARGUMENT, "invalid partial tall FP4 GEMM");
+  const TallPlan plan = plan_tall(args.rows, args.padded_columns, batch,
+                                  matrix->scale_scheme, false, false, 0u, parts);
+  args.partials = partials;
+  args.output = partials;   // of a single part
+  args.output_kind = QLLM_OUT_F32;
+  return launch_tall(args, matrix->scale_scheme, plan, as_stream(stream));
+}
+
+extern "C" int32_t qllm_fp4_gemm_bf16_tall_cut(const qllm_fp4_matrix* matrix,
+                                               const void* input, size_t input_bytes,
+                                               void* output, uint32_t output_kind,
+                                               const float* residual, uint32_t batch,
+                                               void* workspace, size_t workspace_bytes,
+                                               void* stream) {
+  TallArgs args{};
+  if (!tall_arguments(matrix, input, input_bytes, batch, args) || !output ||
+      output_kind > QLLM_OUT_BF16 || !workspace_ok(workspace))
+    return fail(QLLM_INVALID_ARGUMENT, "invalid tall FP4 GEMM");
+  if (residual && output_kind == QLLM_OUT_BF16 &&
+      static_cast<const void*>(residual) == output)
+    return fail(QLLM_INVALID_ARGUMENT,
+                "tall FP4 GEMM: bf16 output cannot alias the f32 residual");
   args.output = output;
   args.output_kind = output_kind;
   args.residual = residual;
-  return launch_tall(args, matrix->scale_scheme, as_stream(stream));
+  return run_tall(args, matrix->scale_scheme, workspace, workspace_bytes,
+                  as_stream(stream));
+}
+
+extern "C" int32_t qllm_fp4_gemm_bf16_tall(const qllm_fp4_matrix* matrix,
+                                           const void* input, size_t input_bytes,
+                                           void* output, uint32_t output_kind,
+                                           const float* residual, uint32_t batch,
+                                           void* stream) {
+  return qllm_fp4_gemm_bf16_tall_cut(matrix, input, input_bytes, output, output_kind,
+                                     residual, batch, nullptr, 0u, stream);
+}
+
+extern "C" int32_t qllm_fp4_swiglu_bf16_tall_cut(const qllm_fp4_matrix* gate,
+                                                 const qllm_fp4_matrix* up,
+                                                 const void* input, size_t input_bytes,
+                                                 void* output_bf16, uint32_t batch,
+                                                 void* workspace, size_t workspace_bytes,
+                                                 void* stream) {
+  TallArgs args{};
+  if (!tall_arguments(gate, input, input_bytes, batch, args) || !tall_matrix_ok(up) ||
+      gate->rows != up->rows || gate->padded_columns != up->padded_columns ||
+      gate->scale_scheme != up->scale_scheme || !output_bf16 || !workspace_ok(workspace))
+    return fail(QLLM_INVALID_ARGUMENT, "invalid tall FP4 SwiGLU");
+  args.up_weights = up->weights;
+  args.up_scales = static_cast<const uint8_t*>(up->scales);
+  args.output = output_bf16;
+  args.output_kind = QLLM_OUT_BF16;
+  return run_tall(args, gate->scale_scheme, workspace, workspace_bytes, as_stream(stream));
 }
 
 extern "C" int32_t qllm_fp4_swiglu_bf16_tall(const qllm_fp4_matrix* gate,
@@ -462,37 +1003,18 @@ extern "C" int32_t qllm_fp4_swiglu_bf16_tall(const qllm_fp4_matrix* gate,
                                              const void* input, size_t input_bytes,
                                              void* output_bf16, uint32_t batch,
                                              void* stream) {
-  if (!tall_matrix_ok(gate) || !tall_matrix_ok(up) || gate->rows != up->rows ||
-      gate->padded_columns != up->padded_columns ||
-      gate->scale_scheme != up->scale_scheme || !input || !output_bf16 ||
-      !batch || batch > (1u << 20) ||
-      (reinterpret_cast<uintptr_t>(input) & 15u) ||
-      input_bytes < static_cast<size_t>(batch) * gate->padded_columns * 2u)
-    return fail(QLLM_INVALID_ARGUMENT, "invalid tall FP4 SwiGLU");
-  TallArgs args{};
-  args.weights = gate->weights;
-  args.scales = static_cast<const uint8_t*>(gate->scales);
-  args.up_weights = up->weights;
-  args.up_scales = static_cast<const uint8_t*>(up->scales);
-  args.activations = static_cast<const uint16_t*>(input);
-  args.rows = gate->rows;
-  args.padded_columns = gate->padded_columns;
-  args.batch = batch;
-  args.output = output_bf16;
-  args.output_kind = QLLM_OUT_BF16;
-  return launch_tall(args, gate->scale_scheme, as_stream(stream));
+  return qllm_fp4_swiglu_bf16_tall_cut(gate, up, input, input_bytes, output_bf16, batch,
+                                       nullptr, 0u, stream);
 }
 
-extern "C" int32_t qllm_fp4_gemm_bf16_tall_split(
+extern "C" int32_t qllm_fp4_gemm_bf16_tall_split_cut(
     const qllm_fp4_matrix* matrix, const void* input, size_t input_bytes,
     const qllm_gemm_segment* segments, uint32_t segment_count, uint32_t batch,
-    void* stream) {
-  if (!tall_matrix_ok(matrix) || !input || !segments || !segment_count ||
-      segment_count > 3u || !batch || batch > (1u << 20) ||
-      (reinterpret_cast<uintptr_t>(input) & 15u) ||
-      input_bytes < static_cast<size_t>(batch) * matrix->padded_columns * 2u)
-    return fail(QLLM_INVALID_ARGUMENT, "invalid split tall FP4 GEMM");
+    void* workspace, size_t workspace_bytes, void* stream) {
   TallArgs args{};
+  if (!tall_arguments(matrix, input, input_bytes, batch, args) || !segments ||
+      !segment_count || segment_count > 3u || !workspace_ok(workspace))
+    return fail(QLLM_INVALID_ARGUMENT, "invalid split tall FP4 GEMM");
   uint64_t total = 0;
   for (uint32_t index = 0; index < segment_count; ++index) {
     if (!segments[index].output || !segments[index].rows ||
@@ -508,11 +1030,14 @@ extern "C" int32_t qllm_fp4_gemm_bf16_tall_split(
     return fail(QLLM_INVALID_ARGUMENT,
                 "split tall FP4 GEMM: segments do not cover the matrix");
   args.segments = segment_count;
-  args.weights = matrix->weights;
-  args.scales = static_cast<const uint8_t*>(matrix->scales);
-  args.activations = static_cast<const uint16_t*>(input);
-  args.rows = matrix->rows;
-  args.padded_columns = matrix->padded_columns;
-  args.batch = batch;
-  return launch_tall(args, matrix->scale_scheme, as_stream(stream));
+  return run_tall(args, matrix->scale_scheme, workspace, workspace_bytes,
+                  as_stream(stream));
+}
+
+extern "C" int32_t qllm_fp4_gemm_bf16_tall_split(
+    const qllm_fp4_matrix* matrix, const void* input, size_t input_bytes,
+    const qllm_gemm_segment* segments, uint32_t segment_count, uint32_t batch,
+    void* stream) {
+  return qllm_fp4_gemm_bf16_tall_split_cut(matrix, input, input_bytes, segments,
+                                           segment_count, batch, nullptr, 0u, stream);
 }

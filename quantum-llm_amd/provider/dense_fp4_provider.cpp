@@ -1591,9 +1591,9 @@ void Mi355DenseFp4Provider::enqueue_mtp_prefill(
       embedding, mtp_.embedding_norm, prefill_hidden_, mtp_.hidden_norm,
       fusion_input, rows, g_.hidden, g_.norm_epsilon, g_.zero_centered_norm,
       stream));
-  status_check(qllm_fp4_gemm_bf16_tall(&mtp_.fusion.descriptor, fusion_input,
-                                       2U * hidden_bytes, prefill_hidden_,
-                                       QLLM_OUT_F32, nullptr, rows, stream));
+  status_check(qllm_fp4_gemm_bf16_tall_cut(
+      &mtp_.fusion.descriptor, fusion_input, 2U * hidden_bytes, prefill_hidden_,
+      QLLM_OUT_F32, nullptr, rows, prefill_parts_, prefill_parts_bytes_, stream));
   status_check(qllm_rms_norm_batch(prefill_hidden_, layer.input_norm, nullptr,
                                    prefill_normalized_, g_.hidden, rows,
                                    g_.hidden, g_.norm_epsilon,
@@ -1603,9 +1603,9 @@ void Mi355DenseFp4Provider::enqueue_mtp_prefill(
       {prefill_query_, layer.qkv.descriptor.rows - 2U * kv_rows, QLLM_OUT_F32},
       {prefill_key_, kv_rows, QLLM_OUT_F32},
       {prefill_value_, kv_rows, QLLM_OUT_F32}};
-  status_check(qllm_fp4_gemm_bf16_tall_split(&layer.qkv.descriptor,
-                                             prefill_normalized_, hidden_bytes,
-                                             projections, 3U, rows, stream));
+  status_check(qllm_fp4_gemm_bf16_tall_split_cut(
+      &layer.qkv.descriptor, prefill_normalized_, hidden_bytes, projections, 3U,
+      rows, prefill_parts_, prefill_parts_bytes_, stream));
   const auto pages = const_cast<const void* const*>(device_page_table_);
   // the proposer's cache lags the target's by one token: record `position`
   // carries rotary position `position` + 1 (enqueue_mtp)
@@ -1660,6 +1660,8 @@ void Mi355DenseFp4Provider::ensure_prefill_workspace(std::uint32_t rows) {
   prefill_attention_ = static_cast<std::uint16_t*>(
       allocate(n * g_.query_heads * g_.head_dim * 2U));
   prefill_embedding_ = static_cast<float*>(allocate(n * g_.hidden * 4U));
+  prefill_parts_bytes_ = qllm_fp4_tall_workspace_bytes();
+  prefill_parts_ = static_cast<float*>(allocate(prefill_parts_bytes_));
   // the MLP's activation; the proposer's fusion input [rows, 2 hidden] too
   prefill_activation_ = static_cast<std::uint16_t*>(allocate(
       n * std::max<std::size_t>(g_.intermediate, 2U * g_.hidden) * 2U));
@@ -1753,20 +1755,48 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
                                             prefill_tokens_, prefill_hidden_,
                                             rows, stream));
       const std::size_t hidden_bytes = std::size_t{rows} * g_.hidden * 2U;
+      // A projection onto the residual stream whose launch is cut along K leaves
+      // its parts to the norm that follows, as in a verify step.
+      std::uint32_t parts = 0U;
+      const auto normalise = [&](const float* weight) {
+        if (parts)
+          status_check(qllm_rms_norm_residual_batch(
+              prefill_hidden_, prefill_parts_, parts, weight, prefill_normalized_,
+              rows, g_.hidden, g_.norm_epsilon, g_.zero_centered_norm, stream));
+        else
+          status_check(qllm_rms_norm_batch(
+              prefill_hidden_, weight, nullptr, prefill_normalized_, g_.hidden,
+              rows, g_.hidden, g_.norm_epsilon, g_.zero_centered_norm, stream));
+        parts = 0U;
+      };
+      const auto project = [&](const qllm_fp4_matrix& matrix,
+                               const std::uint16_t* input, std::size_t bytes,
+                               bool norm_follows) {
+        const std::uint32_t cut =
+            norm_follows && rows <= 65535U && g_.hidden <= 16384U
+                ? qllm_fp4_tall_parts(&matrix, rows)
+                : 1U;
+        if (cut > 1U) {
+          status_check(qllm_fp4_gemm_bf16_tall_partial(
+              &matrix, input, bytes, prefill_parts_, cut, rows, stream));
+          parts = cut;
+        } else {
+          status_check(qllm_fp4_gemm_bf16_tall_cut(
+              &matrix, input, bytes, prefill_hidden_, QLLM_OUT_F32,
+              prefill_hidden_, rows, prefill_parts_, prefill_parts_bytes_, stream));
+        }
+      };
       for (std::uint32_t index = 0; index < g_.layers; ++index) {
         const auto& layer = layers_[index];
-        status_check(qllm_rms_norm_batch(
-            prefill_hidden_, layer.input_norm, nullptr, prefill_normalized_,
-            g_.hidden, rows, g_.hidden, g_.norm_epsilon, g_.zero_centered_norm,
-            stream));
+        normalise(layer.input_norm);
         const std::uint32_t kv_rows = g_.kv_heads * g_.head_dim;
         const qllm_gemm_segment projections[3] = {
             {prefill_query_, layer.qkv.descriptor.rows - 2U * kv_rows, QLLM_OUT_F32},
             {prefill_key_, kv_rows, QLLM_OUT_F32},
             {prefill_value_, kv_rows, QLLM_OUT_F32}};
-        status_check(qllm_fp4_gemm_bf16_tall_split(
+        status_check(qllm_fp4_gemm_bf16_tall_split_cut(
             &layer.qkv.descriptor, prefill_normalized_, hidden_bytes,
-            projections, 3U, rows, stream));
+            projections, 3U, rows, prefill_parts_, prefill_parts_bytes_, stream));
         // attention in row batches of the verify step's size: each batch sees
         // the cache up to and including its own rows
         if (g_.kv_encoding == KvEncoding::q4_f16_per_head) {
@@ -1844,23 +1874,19 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
           launch.stream = stream;
           status_check(qllm_attention_paged_f16_batched(&launch, attention_batch));
         }
-        status_check(qllm_fp4_gemm_bf16_tall(
-            &layer.output.descriptor, prefill_attention_,
-            std::size_t{rows} * attention_width * 2U, prefill_hidden_,
-            QLLM_OUT_F32, prefill_hidden_, rows, stream));
-        status_check(qllm_rms_norm_batch(
-            prefill_hidden_, layer.post_attention_norm, nullptr,
-            prefill_normalized_, g_.hidden, rows, g_.hidden, g_.norm_epsilon,
-            g_.zero_centered_norm, stream));
+        project(layer.output.descriptor, prefill_attention_,
+                std::size_t{rows} * attention_width * 2U, true);
+        normalise(layer.post_attention_norm);
         // gate and up in one launch; silu(gate) * up leaves it in bf16 with
         // the verify step's rounding points
-        status_check(qllm_fp4_swiglu_bf16_tall(
+        status_check(qllm_fp4_swiglu_bf16_tall_cut(
             &layer.gate.descriptor, &layer.up.descriptor, prefill_normalized_,
-            hidden_bytes, prefill_activation_, rows, stream));
-        status_check(qllm_fp4_gemm_bf16_tall(
-            &layer.down.descriptor, prefill_activation_,
-            std::size_t{rows} * g_.intermediate * 2U, prefill_hidden_,
-            QLLM_OUT_F32, prefill_hidden_, rows, stream));
+            hidden_bytes, prefill_activation_, rows, prefill_parts_,
+            prefill_parts_bytes_, stream));
+        // (the last layer's sum is complete: its rows are read as they are)
+        project(layer.down.descriptor, prefill_activation_,
+                std::size_t{rows} * g_.intermediate * 2U,
+                index + 1U < g_.layers);
       }
       if (done + rows == count) {
         // last row -> the verify step's buffers, then the head on that row

@@ -173,3 +173,67 @@ def test_tall_gemm_rejects_row_major(device):
     with pytest.raises(qh.QllmError, match="invalid tall"):
         qh.call("qllm_fp4_gemm_bf16_tall", matrix, qh.ptr(act), act.numel() * 2,
                 qh.ptr(out), qh.OUT_F32, None, 16, None)
+
+
+@pytest.mark.parametrize("rows,padded,batch", [
+    (96, 64, 1), (132, 576, 15), (4, 1024, 16), (260, 832, 17), (1056, 192, 33),
+    (640, 1088, 64), (388, 1024, 65), (2048, 5120, 48), (1024, 1216, 300)])
+@pytest.mark.parametrize("scheme", [ol.SCALE_UE8M0_BLOCK32, ol.SCALE_F16_BLOCK16])
+def test_launches_cut_along_k_match_the_oracle(device, scheme, rows, padded, batch):
+    """Workgroup heights at their edges (1, 16 / 17, 32 / 33, 64 / 65 rows), parts
+    that share the chunks unevenly or hold one chunk each, ragged weight rows:
+    the forms with a workspace, every number of parts, and gate and up."""
+    rng = np.random.default_rng(rows + batch)
+    act = ol.bf16_round(rng.standard_normal((batch, padded)).astype(np.float32))
+    d_act = gu.device_tensor(ol.bf16_bits(act), device)
+    residual = rng.standard_normal((batch, rows)).astype(np.float32)
+    d_residual = gu.device_tensor(residual, device)
+    matrices, wants, keep = [], [], []
+    for _ in range(2):
+        codes, scales = synth.fp4_matrix(rng, rows, padded, scheme)
+        wants.append(ol.fp4_linear_f64(codes, scales, scheme, rows, padded, act))
+        d_codes, d_scales = gu.device_tensor(codes, device), gu.device_tensor(scales, device)
+        matrix, kept = qh.prepack(
+            qh.fp4_matrix(d_codes, d_scales, rows, padded, padded, scheme), device)
+        matrices.append(matrix)
+        keep.append((d_codes, d_scales, kept))
+    size = qh.call("qllm_fp4_tall_workspace_bytes")
+    workspace = torch.empty(size, dtype=torch.uint8, device=device)
+    # F32 sums of at most `padded` exact products, in any order
+    bound = 2e-6 * np.sqrt(padded) * np.abs(wants[0]).max()
+
+    for space, count in ((workspace, size), (None, 0)):
+        out = torch.full((batch, rows), np.nan, device=device)
+        qh.call("qllm_fp4_gemm_bf16_tall_cut", matrices[0], qh.ptr(d_act),
+                d_act.numel() * 2, qh.ptr(out), qh.OUT_F32, qh.ptr(d_residual), batch,
+                qh.ptr(space), count, None)
+        assert np.abs(out.cpu().numpy() - residual - wants[0]).max() < bound + 1e-6
+    out = torch.full((batch, rows), np.nan, dtype=torch.bfloat16, device=device)
+    qh.call("qllm_fp4_swiglu_bf16_tall_cut", matrices[0], matrices[1], qh.ptr(d_act),
+            d_act.numel() * 2, qh.ptr(out), batch, qh.ptr(workspace), size, None)
+    want = ol.silu_product(wants[0], wants[1], True)
+    # two roundings to bf16 (the gate's SiLU, the product), each of which may fall
+    # to the neighbouring value, at most 2^-7 of it away
+    error = np.abs(out.float().cpu().numpy() - want)
+    assert (error <= 2.0 ** -6 * np.abs(want) + 4 * bound * (1 + np.abs(wants[1]))).all()
+    if rows % 32 == 0:
+        segments = (qh.GemmSegment * 2)()
+        parts = [torch.full((batch, n), np.nan, device=device) for n in (32, rows - 32)]
+        for segment, part in zip(segments, parts):
+            segment.output, segment.rows = qh.ptr(part), part.shape[1]
+            segment.output_kind = qh.OUT_F32
+        qh.call("qllm_fp4_gemm_bf16_tall_split_cut", matrices[0], qh.ptr(d_act),
+                d_act.numel() * 2, ctypes.addressof(segments), 2, batch,
+                qh.ptr(workspace), size, None)
+        got = torch.cat(parts, dim=1).cpu().numpy()
+        assert np.abs(got - wants[0]).max() < bound
+    assert 1 <= qh.call("qllm_fp4_tall_parts", matrices[0], batch) <= 16
+    for count in range(1, min(16, padded // 64) + 1):
+        sums = torch.full((count, batch, rows), np.nan, device=device)
+        qh.call("qllm_fp4_gemm_bf16_tall_partial", matrices[0], qh.ptr(d_act),
+                d_act.numel() * 2, qh.ptr(sums), count, batch, None)
+        assert np.abs(sums.sum(0).cpu().numpy() - wants[0]).max() < bound
+    for count in (0, 17, padded // 64 + 1):
+        with pytest.raises(qh.QllmError, match="invalid partial"):
+            qh.call("qllm_fp4_gemm_bf16_tall_partial", matrices[0], qh.ptr(d_act),
+                    d_act.numel() * 2, qh.ptr(workspace), count, batch, None)
