@@ -975,8 +975,8 @@ typedef struct qllm_linear_segment {
 
 /* Up to 8 segments in one launch, the same `batch` input rows for all of them.
  * bf16: up to 64 rows stream the weights once with K cut over a workgroup's
- * waves, more rows go through the tall tiles.  F32: plain 32-bit
- * multiply-adds. */
+ * waves, more rows go through the tall tiles.  F32: the same, every input value
+ * in three bf16 parts that hold all of it. */
 int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32_t count,
                           uint32_t batch, uint32_t element, void* stream);
 

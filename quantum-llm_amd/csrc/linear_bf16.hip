@@ -18,7 +18,13 @@
 //    prefetched one step ahead in registers.  An XCD gets a contiguous range
 //    of the grid walked in bands of activation tiles, so operands are shared
 //    in its L2.
-//  * F32 mode: plain 32-bit multiply-adds from the same packed weights.
+//  * F32 mode runs on the same kernels: a 32-bit activation is the sum of three
+//    bf16 values (its 24 significant bits, eight at a time), their products with
+//    a bf16 weight are exact in 32 bits, and all three go into the same F32
+//    accumulator.  Nothing of the activation is lost; against 64 bits a product
+//    is 2 to 4 times closer than a chain of multiply-adds over K was (of
+//    [11264, 2048] 1.9e-7 up to 64 rows and 4.9e-7 above, 8.1e-7 before), and
+//    it takes 13 us for one row and 73 for 333 instead of 330 and 440.
 #include "common.hpp"
 #include "mixed_common.hpp"
 
@@ -65,9 +71,66 @@ __device__ __forceinline__ void store_gated(const qllm_linear_segment& s, uint32
     store_element(out + i, activate(s.activation, gate[i]) * up[i]);
 }
 
+// ---- operands -----------------------------------------------------------------
+
+// Eight consecutive input values of a row as they come from memory, and as
+// operands of the matrix instructions: bf16 as it is, F32 in three bf16 parts.
+template <bool F32>
+struct Input;
+
+template <>
+struct Input<false> {
+  static constexpr int kParts = 1;
+  using Element = uint16_t;
+  using Raw = i32x4;
+  static __device__ __forceinline__ Raw load(const uint16_t* source) {
+    return *reinterpret_cast<const i32x4*>(source);
+  }
+  static __device__ __forceinline__ void split(const Raw& raw, i32x4 (&out)[1]) {
+    out[0] = raw;
+  }
+};
+
+template <>
+struct Input<true> {
+  static constexpr int kParts = 3;
+  using Element = float;
+  struct Raw {
+    f32x4 low, high;
+  };
+  static __device__ __forceinline__ Raw load(const float* source) {
+    const f32x4* vector = reinterpret_cast<const f32x4*>(source);
+    return {vector[0], vector[1]};
+  }
+  // The upper 16 bits of x are its first eight significant bits, x minus those
+  // has sixteen left, and so on: every difference is exact.  An infinity is its
+  // first part alone; a NaN reaches the second one whatever its bits are.
+  static __device__ __forceinline__ void split(const Raw& raw, i32x4 (&out)[3]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t part[3][2];
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const int at = 2 * i + half;
+        float rest = at < 4 ? raw.low[at] : raw.high[at - 4];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          part[p][half] = __float_as_uint(rest);
+          const float top = __uint_as_float(part[p][half] & 0xffff0000u);
+          rest = fabsf(rest) == INFINITY ? 0.0f : rest - top;
+        }
+      }
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        out[p][i] = static_cast<int>(
+            __builtin_amdgcn_perm(part[p][1], part[p][0], 0x07060302u));
+    }
+  }
+};
+
 // ---- up to 64 rows ------------------------------------------------------------
 
-template <int MT, int TILES, int UNROLL>
+template <bool F32, int MT, int TILES, int UNROLL>
 __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_t unit,
                                            uint32_t batch, f32x4* scratch) {
   const uint32_t wave = threadIdx.x / kWave;
@@ -84,18 +147,28 @@ __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_
 
   const i32x4* weights = static_cast<const i32x4*>(s.weights) +
                          size_t{tile} * TILES * chunks * kWave + lane;
-  const uint16_t* input[MT];
+  using In = Input<F32>;
+  using Element = typename In::Element;
+  const Element* input[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const uint32_t row = min(mt * 16u + lane % 16u, batch - 1u);
-    input[mt] = static_cast<const uint16_t*>(s.input) + size_t{row} * s.input_stride +
+    input[mt] = static_cast<const Element*>(s.input) + size_t{row} * s.input_stride +
                 8u * (lane / 16u);
   }
   f32x4 sum[TILES][MT] = {};
+  const auto multiply = [&](const i32x4 (&w)[TILES], const typename In::Raw& raw, int mt) {
+    i32x4 x[In::kParts];
+    In::split(raw, x);
+#pragma unroll
+    for (int p = 0; p < In::kParts; ++p)
+#pragma unroll
+      for (int t = 0; t < TILES; ++t) sum[t][mt] = mfma_bf16(w[t], x[p], sum[t][mt]);
+  };
   uint32_t chunk = begin;
   for (; chunk + UNROLL <= end; chunk += UNROLL) {
     i32x4 w[UNROLL][TILES];
-    i32x4 x[UNROLL][MT];
+    typename In::Raw x[UNROLL][MT];
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
@@ -105,25 +178,20 @@ __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-        x[u][mt] = *reinterpret_cast<const i32x4*>(input[mt] + (chunk + u) * 32u);
+      for (int mt = 0; mt < MT; ++mt) x[u][mt] = In::load(input[mt] + (chunk + u) * 32u);
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
-      for (int t = 0; t < TILES; ++t)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-          sum[t][mt] = mfma_bf16(w[u][t], x[u][mt], sum[t][mt]);
+      for (int mt = 0; mt < MT; ++mt) multiply(w[u], x[u][mt], mt);
   }
-  for (; chunk < end; ++chunk)
+  for (; chunk < end; ++chunk) {
+    i32x4 w[TILES];
 #pragma unroll
-    for (int t = 0; t < TILES; ++t) {
-      const i32x4 w = weights[(size_t{static_cast<uint32_t>(t)} * chunks + chunk) * kWave];
+    for (int t = 0; t < TILES; ++t)
+      w[t] = weights[(size_t{static_cast<uint32_t>(t)} * chunks + chunk) * kWave];
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-        sum[t][mt] = mfma_bf16(
-            w, *reinterpret_cast<const i32x4*>(input[mt] + chunk * 32u), sum[t][mt]);
-    }
+    for (int mt = 0; mt < MT; ++mt) multiply(w, In::load(input[mt] + chunk * 32u), mt);
+  }
 
 #pragma unroll
   for (int t = 0; t < TILES; ++t)
@@ -145,7 +213,7 @@ __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_
     const uint32_t n = tile * 16u + 4u * (at / 16u);
     if (m >= batch) continue;
     if constexpr (TILES == 2) {
-      store_gated<uint16_t>(s, m, n, total[0], total[1]);
+      store_gated<Element>(s, m, n, total[0], total[1]);
     } else {
       float* base = static_cast<float*>(s.output) +
                     size_t{part} * batch * s.output_stride;
@@ -154,27 +222,33 @@ __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_
   }
 }
 
-template <int MT>
+template <bool F32, int MT>
 __global__ __launch_bounds__(kSmallWaves* kWave) void linear_small_kernel(LinearArgs args) {
   __shared__ f32x4 scratch[2 * MT * kSmallWaves * kWave];
   const uint32_t index = segment_of(args, blockIdx.x);
   const qllm_linear_segment& s = args.segment[index];
   const uint32_t unit = blockIdx.x - args.first_unit[index];
+  // (F32 input takes twice the registers in flight)
+  constexpr int kUnroll = F32 && MT > 2 ? 2 : MT > 1 ? 4 : 8;
   if (s.epilogue == QLLM_LINEAR_GATED)
-    small_unit<MT, 2, (MT > 1 ? 2 : 4)>(s, unit, args.batch, scratch);
+    small_unit<F32, MT, 2, (kUnroll > 2 ? kUnroll / 2 : kUnroll)>(s, unit, args.batch,
+                                                                  scratch);
   else
-    small_unit<MT, 1, (MT > 1 ? 4 : 8)>(s, unit, args.batch, scratch);
+    small_unit<F32, MT, 1, kUnroll>(s, unit, args.batch, scratch);
 }
 
 // ---- tall batches --------------------------------------------------------------
 
-template <int NT, int MT>
+template <bool F32, int NT, int MT>
 __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
+  using In = Input<F32>;
+  using Element = typename In::Element;
+  constexpr int kParts = In::kParts;
   constexpr uint32_t kRowsM = MT * 16u;
   constexpr uint32_t kPieces = kRowsM * 8u;           // 16-byte pieces of a tile
   constexpr uint32_t kLoads = kPieces / 256u;
   static_assert(kPieces % 256u == 0u);
-  __shared__ i32x4 tile[2][kPieces];
+  __shared__ i32x4 tile[2][kParts][kPieces];
 
   const uint32_t m_tiles = (args.batch + kRowsM - 1u) / kRowsM;
   // contiguous ranges of workgroups per XCD (consecutive ids go round the XCDs)
@@ -208,36 +282,43 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
                  size_t{min(first_tile + t, weight_tiles - 1u)} * chunks * kWave + lane;
 
   // piece p of the tile: row p / 8, swizzled slot p % 8
-  const i32x4* source[kLoads];
+  const Element* source[kLoads];
 #pragma unroll
   for (uint32_t i = 0; i < kLoads; ++i) {
     const uint32_t piece = i * 256u + threadIdx.x;
     const uint32_t row = piece / 8u;
     const uint32_t column = (piece % 8u) ^ (row % 8u);
     const uint32_t batch_row = min(m_tile * kRowsM + row, args.batch - 1u);
-    source[i] = reinterpret_cast<const i32x4*>(
-        static_cast<const uint16_t*>(s.input) + size_t{batch_row} * s.input_stride +
-        column * 8u);
+    source[i] = static_cast<const Element*>(s.input) +
+                size_t{batch_row} * s.input_stride + column * 8u;
   }
 
   f32x4 sum[NT][MT] = {};
-  i32x4 staged[kLoads];
+  typename In::Raw staged[kLoads];
+  const auto store_staged = [&](uint32_t buffer) {
+#pragma unroll
+    for (uint32_t i = 0; i < kLoads; ++i) {
+      i32x4 parts[kParts];
+      In::split(staged[i], parts);
+#pragma unroll
+      for (int p = 0; p < kParts; ++p) tile[buffer][p][i * 256u + threadIdx.x] = parts[p];
+    }
+  };
   i32x4 held[2][2][NT];   // [step parity][half of 32 columns][tile]
 #pragma unroll
-  for (uint32_t i = 0; i < kLoads; ++i) staged[i] = source[i][0];
+  for (uint32_t i = 0; i < kLoads; ++i) staged[i] = In::load(source[i]);
 #pragma unroll
   for (int half = 0; half < 2; ++half)
 #pragma unroll
     for (int t = 0; t < NT; ++t) held[0][half][t] = weights[t][half * kWave];
-#pragma unroll
-  for (uint32_t i = 0; i < kLoads; ++i) tile[0][i * 256u + threadIdx.x] = staged[i];
+  store_staged(0u);
   __syncthreads();
 
   const auto step_at = [&](uint32_t step, auto parity) {
     constexpr int P = decltype(parity)::value;
     const uint32_t next = min(step + 1u, steps - 1u);   // the last step re-reads itself
 #pragma unroll
-    for (uint32_t i = 0; i < kLoads; ++i) staged[i] = source[i][next * 8u];
+    for (uint32_t i = 0; i < kLoads; ++i) staged[i] = In::load(source[i] + next * 64u);
 #pragma unroll
     for (int half = 0; half < 2; ++half)
 #pragma unroll
@@ -245,22 +326,23 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
         held[1 - P][half][t] = weights[t][(next * 2u + half) * kWave];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      i32x4 x[MT];
+    for (int half = 0; half < 2; ++half)
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const uint32_t row = mt * 16u + lane % 16u;
-        const uint32_t column = half * 4u + lane / 16u;
-        x[mt] = tile[P][row * 8u + (column ^ (row % 8u))];
+      for (int p = 0; p < kParts; ++p) {
+        i32x4 x[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          const uint32_t row = mt * 16u + lane % 16u;
+          const uint32_t column = half * 4u + lane / 16u;
+          x[mt] = tile[P][p][row * 8u + (column ^ (row % 8u))];
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+            sum[t][mt] = mfma_bf16(held[P][half][t], x[mt], sum[t][mt]);
       }
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-          sum[t][mt] = mfma_bf16(held[P][half][t], x[mt], sum[t][mt]);
-    }
-#pragma unroll
-    for (uint32_t i = 0; i < kLoads; ++i) tile[1 - P][i * 256u + threadIdx.x] = staged[i];
+    store_staged(1 - P);
     __syncthreads();
   };
   uint32_t step = 0;
@@ -270,6 +352,26 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
   }
   if (step < steps) step_at(step, std::integral_constant<int, 0>{});
 
+  if (s.epilogue == QLLM_LINEAR_ADD) {
+    // what the sums are added to comes first: every load after a store would
+    // wait for all before it
+    const bool vectors = s.output_stride % 4u == 0u;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const uint32_t m = min(m_tile * kRowsM + mt * 16u + lane % 16u, args.batch - 1u);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const uint32_t n = (first_tile + t) * 16u + 4u * (lane / 16u);
+        const float* out = static_cast<const float*>(s.output) + size_t{m} * s.output_stride;
+        if (vectors && n + 4u <= s.output_columns) {
+          sum[t][mt] += *reinterpret_cast<const f32x4*>(out + n);
+        } else {
+          for (uint32_t i = 0; i < 4u; ++i)
+            if (n + i < s.output_columns) sum[t][mt][i] += out[n + i];
+        }
+      }
+    }
+  }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const uint32_t m = m_tile * kRowsM + mt * 16u + lane % 16u;
@@ -281,7 +383,7 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
           const uint32_t at = first_tile + t;
           if (at >= weight_tiles) continue;
           const uint32_t n = at / 2u * 16u + 4u * (lane / 16u);
-          if (n + 4u <= s.output_columns && s.output_stride % 4u == 0u) {
+          if (!F32 && n + 4u <= s.output_columns && s.output_stride % 4u == 0u) {
             const f32x4 gate = sum[t][mt];
             const f32x4 up = sum[t + 1][mt];
             uint32_t bits[4];
@@ -293,7 +395,7 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
                 i32x2{static_cast<int>(bits[0] | bits[1] << 16),
                       static_cast<int>(bits[2] | bits[3] << 16)};
           } else {
-            store_gated<uint16_t>(s, m, n, sum[t][mt], sum[t + 1][mt]);
+            store_gated<Element>(s, m, n, sum[t][mt], sum[t + 1][mt]);
           }
         }
       }
@@ -302,83 +404,7 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
       for (int t = 0; t < NT; ++t)
         if (first_tile + t < weight_tiles)
           store_four(s, static_cast<float*>(s.output), m,
-                     (first_tile + t) * 16u + 4u * (lane / 16u), sum[t][mt],
-                     s.epilogue == QLLM_LINEAR_ADD);
-    }
-  }
-}
-
-// ---- F32 mode --------------------------------------------------------------------
-
-// 64 batch rows x 64 packed weight rows per workgroup, 4 x 4 products per
-// thread; a thread's weight rows are 16 apart, so the two tiles of a gated
-// pair meet in it.
-__global__ __launch_bounds__(256) void linear_f32_kernel(LinearArgs args) {
-  __shared__ float x_tile[32][65];
-  __shared__ float w_tile[32][65];
-  const uint32_t index = segment_of(args, blockIdx.x);
-  const qllm_linear_segment& s = args.segment[index];
-  const uint32_t unit = blockIdx.x - args.first_unit[index];
-  const uint32_t n_tiles = (s.rows + 63u) / 64u;
-  const uint32_t m_tiles = (args.batch + 63u) / 64u;
-  const uint32_t parts = s.epilogue == QLLM_LINEAR_PARTIALS ? s.splits : 1u;
-  const uint32_t part = unit / (n_tiles * m_tiles);
-  const uint32_t rest = unit % (n_tiles * m_tiles);
-  const uint32_t m0 = rest / n_tiles * 64u;
-  const uint32_t n0 = rest % n_tiles * 64u;
-  const uint32_t chunks = s.columns / 32u;
-  const uint32_t begin = chunks * part / parts;
-  const uint32_t end = chunks * (part + 1u) / parts;
-  const auto* weights = static_cast<const uint16_t*>(s.weights);
-  const auto* input = static_cast<const float*>(s.input);
-  const uint32_t tx = threadIdx.x % 16u;
-  const uint32_t ty = threadIdx.x / 16u;
-  float sum[4][4] = {};
-  for (uint32_t chunk = begin; chunk < end; ++chunk) {
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < 64u * 32u; i += 256u) {
-      const uint32_t k = i % 32u;
-      const uint32_t row = i / 32u;
-      const uint32_t m = min(m0 + row, args.batch - 1u);
-      x_tile[k][row] = input[size_t{m} * s.input_stride + chunk * 32u + k];
-      const uint32_t n = n0 + row;
-      w_tile[k][row] =
-          n < s.rows ? bf16_bits_to_f32(weights[(size_t{n / 16u} * chunks + chunk) * 512u +
-                                                (k / 8u * 16u + n % 16u) * 8u + k % 8u])
-                     : 0.0f;
-    }
-    __syncthreads();
-    for (uint32_t k = 0; k < 32u; ++k) {
-      float x[4], w[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        x[i] = x_tile[k][ty * 4u + i];
-        w[i] = w_tile[k][tx + 16u * i];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sum[i][j] = fmaf(x[i], w[j], sum[i][j]);
-    }
-  }
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t m = m0 + ty * 4u + i;
-    if (m >= args.batch) continue;
-    if (s.epilogue == QLLM_LINEAR_GATED) {
-      for (int j = 0; j < 4; j += 2) {
-        const uint32_t n = n0 / 2u + j * 8u + tx;
-        if (n0 + j * 16u + tx < s.rows && n < s.output_columns)
-          static_cast<float*>(s.output)[size_t{m} * s.output_stride + n] =
-              activate(s.activation, sum[i][j]) * sum[i][j + 1];
-      }
-      continue;
-    }
-    float* out = static_cast<float*>(s.output) +
-                 (size_t{part} * args.batch + m) * s.output_stride;
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t n = n0 + tx + 16u * j;
-      if (n >= s.rows || n >= s.output_columns) continue;
-      out[n] = s.epilogue == QLLM_LINEAR_ADD ? out[n] + sum[i][j] : sum[i][j];
+                     (first_tile + t) * 16u + 4u * (lane / 16u), sum[t][mt], false);
     }
   }
 }
@@ -415,13 +441,19 @@ uint32_t tall_units(const qllm_linear_segment& s, uint32_t batch) {
   return (s.rows + 64u * NT - 1u) / (64u * NT) * ((batch + 16u * MT - 1u) / (16u * MT));
 }
 
-template <int NT, int MT>
+template <bool F32, int NT, int MT>
 int32_t launch_tall(LinearArgs& args, hipStream_t stream) {
   args.first_unit[0] = 0;
   for (uint32_t i = 0; i < args.count; ++i)
     args.first_unit[i + 1] = args.first_unit[i] + tall_units<NT, MT>(args.segment[i], args.batch);
-  linear_tall_kernel<NT, MT><<<args.first_unit[args.count], 256, 0, stream>>>(args);
-  return launched("tall bf16 linear");
+  linear_tall_kernel<F32, NT, MT><<<args.first_unit[args.count], 256, 0, stream>>>(args);
+  return launched("tall linear");
+}
+
+template <bool F32, int MT>
+void launch_small(const LinearArgs& args, hipStream_t stream) {
+  linear_small_kernel<F32, MT>
+      <<<args.first_unit[args.count], kSmallWaves * kWave, 0, stream>>>(args);
 }
 
 template <int NT, int MT>
@@ -496,16 +528,7 @@ extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32
     args.segment[i] = s;
   }
   const auto hip_stream = as_stream(stream);
-  if (element == QLLM_ELEMENT_F32) {
-    for (uint32_t i = 0; i < count; ++i) {
-      const qllm_linear_segment& s = segments[i];
-      const uint32_t parts = s.epilogue == QLLM_LINEAR_PARTIALS ? s.splits : 1u;
-      args.first_unit[i + 1] = args.first_unit[i] +
-                               (s.rows + 63u) / 64u * ((batch + 63u) / 64u) * parts;
-    }
-    linear_f32_kernel<<<args.first_unit[count], 256, 0, hip_stream>>>(args);
-    return launched("F32 linear");
-  }
+  const bool f32 = element == QLLM_ELEMENT_F32;
   if (batch <= 64u) {
     for (uint32_t i = 0; i < count; ++i) {
       const qllm_linear_segment& s = segments[i];
@@ -513,18 +536,20 @@ extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32
       const uint32_t tile_rows = s.epilogue == QLLM_LINEAR_GATED ? 32u : 16u;
       args.first_unit[i + 1] = args.first_unit[i] + s.rows / tile_rows * parts;
     }
-    const uint32_t units = args.first_unit[count];
-    const uint32_t threads = kSmallWaves * kWave;
     if (batch <= 16u)
-      linear_small_kernel<1><<<units, threads, 0, hip_stream>>>(args);
+      f32 ? launch_small<true, 1>(args, hip_stream) : launch_small<false, 1>(args, hip_stream);
     else if (batch <= 32u)
-      linear_small_kernel<2><<<units, threads, 0, hip_stream>>>(args);
+      f32 ? launch_small<true, 2>(args, hip_stream) : launch_small<false, 2>(args, hip_stream);
     else
-      linear_small_kernel<4><<<units, threads, 0, hip_stream>>>(args);
-    return launched("small-batch bf16 linear");
+      f32 ? launch_small<true, 4>(args, hip_stream) : launch_small<false, 4>(args, hip_stream);
+    return launched("small-batch linear");
   }
+  // F32: three parts of 64 activation rows fit a workgroup's LDS twice over
+  if (f32)
+    return all_tall_units<4, 4>(args) >= 384u ? launch_tall<true, 4, 4>(args, hip_stream)
+                                              : launch_tall<true, 2, 4>(args, hip_stream);
   // the largest tiles that still give every CU two workgroups to hold
-  if (all_tall_units<4, 8>(args) >= 512u) return launch_tall<4, 8>(args, hip_stream);
-  if (all_tall_units<2, 8>(args) >= 384u) return launch_tall<2, 8>(args, hip_stream);
-  return launch_tall<2, 4>(args, hip_stream);
+  if (all_tall_units<4, 8>(args) >= 512u) return launch_tall<false, 4, 8>(args, hip_stream);
+  if (all_tall_units<2, 8>(args) >= 384u) return launch_tall<false, 2, 8>(args, hip_stream);
+  return launch_tall<false, 2, 4>(args, hip_stream);
 }

@@ -1078,7 +1078,7 @@ void Mi355MixedProvider::enqueue_sandwich(Block& block, std::uint32_t rows,
   };
   const auto project = [&](const Matrix& matrix, std::uint32_t splits,
                            const DeviceBuffer& post_norm) {
-    const bool split = g_.element == QLLM_ELEMENT_BF16 && rows <= kSmallBatch;
+    const bool split = rows <= kSmallBatch;
     qllm_linear_segment s{};
     s.weights = matrix.data.get();
     s.input = joined_.get();

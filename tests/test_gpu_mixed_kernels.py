@@ -61,6 +61,44 @@ def test_linear_segments_of_every_epilogue(device, element, batch):
     assert torch.all(gated[:, 45:] == 0)
 
 
+@pytest.mark.parametrize("batch", [1, 16, 17, 33, 64, 65, 200])
+def test_linear_takes_all_bits_of_32_bit_inputs(device, batch):
+    """Inputs with 24 significant bits over 60 powers of two, the largest finite
+    value, infinities and a NaN whose upper half reads as an infinity."""
+    rng = np.random.default_rng(batch)
+    matrix = mm.bf16(rng.standard_normal((70, 192)) / 14)
+    matrix[:, 190] = 0.25
+    x = (rng.standard_normal((batch, 192)) * np.exp2(rng.integers(-30, 31, (batch, 192)))
+         ).astype(np.float32)
+    odd = batch // 2
+    special = {0: np.float32(3.4028235e38), 1: np.inf, 2: -np.inf,
+               3: np.uint32(0x7f800001).view(np.float32)}.items()
+    weights = packed(device, [(matrix, 0, 1, 0)], 70, 192)
+    out = torch.zeros((batch, 72), device=device)
+
+    def run(values):
+        d_x = padded_input(device, values, 192, F32)
+        segment = qh.LinearSegment(qh.ptr(weights), qh.ptr(d_x), qh.ptr(out), 80, 192, 192,
+                                   72, 70, qh.LINEAR_STORE, 0, 0)
+        qh.call("qllm_linear_batch", ctypes.byref(segment), 1, batch, F32, None)
+        return out[:, :70].cpu().numpy().astype(np.float64)
+
+    # every product is exact, every one of the 3 x 192 additions of a sum rounds
+    # by at most 2^-24 of the magnitudes' sum, in whatever order
+    magnitude = np.abs(x.astype(np.float64)) @ np.abs(matrix.T.astype(np.float64))
+    bound = 3 * 192 * 2.0 ** -24 * magnitude
+    want = x.astype(np.float64) @ matrix.T.astype(np.float64)
+    assert (np.abs(run(x) - want) <= bound).all()
+    for _, value in special:
+        changed = np.zeros_like(x)
+        changed[odd, 190] = value
+        with np.errstate(invalid="ignore"):
+            expected = changed[odd, 190].astype(np.float64) * 0.25
+        got = run(changed)
+        assert np.array_equal(got[odd], np.full(70, expected), equal_nan=True)
+        assert not np.delete(got, odd, axis=0).any()
+
+
 @pytest.mark.parametrize("element", [F32, BF16])
 @pytest.mark.parametrize("splits", [1, 3, 7])
 def test_linear_partials_and_side_by_side_columns(device, element, splits):
