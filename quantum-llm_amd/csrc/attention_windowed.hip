@@ -15,7 +15,8 @@
 //    and low halves (together 16 bits of mantissa), lets the matrix cores mix
 //    them over heads - the mix matrix is bf16 as stored, so both products are
 //    exact and added in F32 - and multiplies the mixed weights with the values.
-//  * general: one workgroup per row, any size, bf16 or F32 arithmetic.
+//  * general: any size, plain F32 arithmetic on bf16 or F32 elements.  A few rows
+//    take the split form's three launches; more, a workgroup per row.
 //
 // Keys lie in fragments of 16 tokens x 32 dimensions and values, transposed, in
 // fragments of 16 dimensions x 32 tokens: every operand load of a wave is one
@@ -184,6 +185,43 @@ struct AttentionArgs {
   uint32_t value_splits;
 };
 
+// q . key over `dim` dimensions, 16 bytes of a key's fragment row (32 dimensions,
+// then 512 elements to the next) at a time.
+template <typename T>
+__device__ __forceinline__ float key_product(const float* q, const T* key, uint32_t dim) {
+  constexpr uint32_t kVector = 16u / sizeof(T);
+  float sum[2] = {0.0f, 0.0f};
+  uint32_t d = 0;
+#pragma unroll 4
+  for (; d + kVector <= dim; d += kVector) {
+    const i32x4 raw = *reinterpret_cast<const i32x4*>(key + size_t{d / 32u} * 512u + d % 32u);
+    const T* element = reinterpret_cast<const T*>(&raw);
+#pragma unroll
+    for (uint32_t i = 0; i < kVector; ++i)
+      sum[i % 2u] = fmaf(q[d + i], load_element(element + i), sum[i % 2u]);
+  }
+  for (; d < dim; ++d)
+    sum[0] = fmaf(q[d], load_element(key + size_t{d / 32u} * 512u + d % 32u), sum[0]);
+  return sum[0] + sum[1];
+}
+
+// The sum over a tile's 32 keys of weight x value, one dimension (32 consecutive
+// elements), added to `total`.
+template <typename T>
+__device__ __forceinline__ float value_product(const float* weights, const T* values,
+                                               float total) {
+  constexpr uint32_t kVector = 16u / sizeof(T);
+#pragma unroll
+  for (uint32_t j = 0; j < kTileKeys; j += kVector) {
+    const i32x4 raw = *reinterpret_cast<const i32x4*>(values + j);
+    const T* element = reinterpret_cast<const T*>(&raw);
+#pragma unroll
+    for (uint32_t i = 0; i < kVector; ++i)
+      total = fmaf(weights[j + i], load_element(element + i), total);
+  }
+  return total;
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void general_attention_kernel(AttentionArgs args) {
   extern __shared__ float shared[];
@@ -219,11 +257,7 @@ __global__ __launch_bounds__(256) void general_attention_kernel(AttentionArgs ar
       if (visible(a, position, key)) {
         const uint32_t slot = key % a.page_tokens;
         const T* k = page + key_block(a, head / group, slot) + slot % 16u * 32u;
-        score = 0.0f;
-        for (uint32_t d = 0; d < a.dim; ++d)
-          score = fmaf(q[head * a.dim + d],
-                       load_element(k + size_t{d / 32u} * 512u + d % 32u), score);
-        score *= a.scale;
+        score = key_product(q + head * a.dim, k, a.dim) * a.scale;
       }
       weights[i] = score;
     }
@@ -270,11 +304,8 @@ __global__ __launch_bounds__(256) void general_attention_kernel(AttentionArgs ar
     for (uint32_t i = threadIdx.x; i < heads * a.vdim; i += blockDim.x) {
       const uint32_t h = i / a.vdim;
       const T* v = page + value_block(a, h / group, slot) + size_t{i % a.vdim} * 32u;
-      float total = out[i];
       // slots past the row's position may hold anything: their weight is zero
-      for (uint32_t j = 0; j < kTileKeys; ++j)
-        total = fmaf(mixed[h * kTileKeys + j], load_element(v + j), total);
-      out[i] = total;
+      out[i] = value_product(mixed + h * kTileKeys, v, out[i]);
     }
     __syncthreads();
   }
@@ -284,6 +315,145 @@ __global__ __launch_bounds__(256) void general_attention_kernel(AttentionArgs ar
     store_element(static_cast<T*>(run.output) + size_t{row} * run.output_stride + i,
                   out[i] * gate);
   }
+}
+
+// A few rows in plain F32.  One workgroup per row took 750 us for a token of 16
+// heads over 340 keys - one CU's round trips, every score twice; dealt over the
+// score and value splits of the form below it takes 53 us (scores 25,
+// values 23, sum 5).
+//
+// Scores of the workgroup's tiles for all heads, 32 lanes per (head, tile), and
+// the heads' maxima and sums over those tiles.
+template <typename T>
+__global__ __launch_bounds__(256) void general_scores_kernel(AttentionArgs args) {
+  extern __shared__ float shared[];
+  const Attention& a = args.attention;
+  const uint32_t heads = a.query_heads;
+  const uint32_t group = heads / a.kv_heads;
+  float* q = shared;                        // [heads][dim]
+  float* maximum = q + heads * a.dim;       // [heads]
+  float* total = maximum + heads;           // [heads]
+  const uint32_t row = blockIdx.y;
+  const uint32_t position = a.step[kStepPosition] + row;
+  const TileRange range = tiles_for(a, position, position);
+  const T* query =
+      static_cast<const T*>(args.launch.query) + size_t{row} * heads * a.key_stride;
+  for (uint32_t i = threadIdx.x; i < heads * a.dim; i += blockDim.x)
+    q[i] = load_element(query + size_t{i / a.dim} * a.key_stride + i % a.dim);
+  for (uint32_t h = threadIdx.x; h < heads; h += blockDim.x) {
+    maximum[h] = -INFINITY;
+    total[h] = 0.0f;
+  }
+  __syncthreads();
+  const uint32_t begin = static_cast<uint32_t>(uint64_t{range.count} * blockIdx.x / gridDim.x);
+  const uint32_t end =
+      static_cast<uint32_t>(uint64_t{range.count} * (blockIdx.x + 1u) / gridDim.x);
+  for (uint32_t ordinal = begin; ordinal < end; ++ordinal) {
+    const uint32_t key = range.tile(ordinal) * kTileKeys + threadIdx.x % kTileKeys;
+    const T* page = page_of<const T>(a, key);
+    const uint32_t slot = key % a.page_tokens;
+    // (a head's lanes are the same ones in every tile)
+    for (uint32_t head = threadIdx.x / kTileKeys; head < heads;
+         head += blockDim.x / kTileKeys) {
+      float score = -INFINITY;
+      if (visible(a, position, key))
+        score = key_product(q + head * a.dim,
+                            page + key_block(a, head / group, slot) + slot % 16u * 32u,
+                            a.dim) * a.scale;
+      args.scores[(size_t{row} * heads + head) * args.capacity +
+                  size_t{ordinal} * kTileKeys + threadIdx.x % kTileKeys] = score;
+      float top = score;
+      for (int offset = 16; offset > 0; offset >>= 1)
+        top = fmaxf(top, __shfl_xor(top, offset, kWave));
+      const float fresh = fmaxf(maximum[head], top);
+      float share = fresh > -INFINITY ? expf(score - fresh) : 0.0f;
+      for (int offset = 16; offset > 0; offset >>= 1)
+        share += __shfl_xor(share, offset, kWave);
+      if (threadIdx.x % kTileKeys == 0u && fresh > -INFINITY) {
+        total[head] = total[head] * expf(maximum[head] - fresh) + share;
+        maximum[head] = fresh;
+      }
+    }
+  }
+  __syncthreads();
+  for (uint32_t h = threadIdx.x; h < heads; h += blockDim.x) {
+    float* out =
+        args.maxima + ((size_t{row} * args.score_splits + blockIdx.x) * heads + h) * 2u;
+    out[0] = maximum[h];
+    out[1] = total[h];
+  }
+}
+
+// Normalised and mixed weights of the workgroup's tiles times the values of one
+// key/value head.
+template <typename T>
+__global__ __launch_bounds__(256) void general_values_kernel(AttentionArgs args) {
+  extern __shared__ float shared[];
+  const Attention& a = args.attention;
+  const uint32_t heads = a.query_heads;
+  const uint32_t group = heads / a.kv_heads;
+  float* maximum = shared;                        // [heads]
+  float* total = maximum + heads;                 // [heads]
+  float* weights = total + heads;                 // [heads][32]
+  float* mixed = weights + heads * kTileKeys;     // [group][32]
+  float* out = mixed + group * kTileKeys;         // [group][vdim]
+  const uint32_t row = blockIdx.z;
+  const uint32_t kv = blockIdx.y;
+  const uint32_t position = a.step[kStepPosition] + row;
+  const TileRange range = tiles_for(a, position, position);
+  for (uint32_t h = threadIdx.x / kWave; h < heads; h += blockDim.x / kWave) {
+    const uint32_t lane = threadIdx.x % kWave;   // a score split (at most 64)
+    float m = -INFINITY;
+    float t = 0.0f;
+    if (lane < args.score_splits) {
+      const float* pair =
+          args.maxima + ((size_t{row} * args.score_splits + lane) * heads + h) * 2u;
+      m = pair[0];
+      t = pair[1];
+    }
+    const float top = wave_max(m);
+    t = wave_sum(m > -INFINITY ? t * expf(m - top) : 0.0f);
+    if (lane == 0u) {
+      maximum[h] = top;
+      total[h] = t;
+    }
+  }
+  for (uint32_t i = threadIdx.x; i < group * a.vdim; i += blockDim.x) out[i] = 0.0f;
+  __syncthreads();
+  const uint32_t begin = static_cast<uint32_t>(uint64_t{range.count} * blockIdx.x / gridDim.x);
+  const uint32_t end =
+      static_cast<uint32_t>(uint64_t{range.count} * (blockIdx.x + 1u) / gridDim.x);
+  for (uint32_t ordinal = begin; ordinal < end; ++ordinal) {
+    const uint32_t key0 = range.tile(ordinal) * kTileKeys;
+    const float* scores =
+        args.scores + size_t{row} * heads * args.capacity + size_t{ordinal} * kTileKeys;
+    for (uint32_t i = threadIdx.x; i < heads * kTileKeys; i += blockDim.x) {
+      const uint32_t h = i / kTileKeys;
+      weights[i] = expf(scores[size_t{h} * args.capacity + i % kTileKeys] - maximum[h]) /
+                   total[h];
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < group * kTileKeys; i += blockDim.x) {
+      const uint32_t h = kv * group + i / kTileKeys;
+      float sum = 0.0f;
+      if (a.head_mix) {
+        const float* mix = a.head_mix + size_t{h} * heads;
+        for (uint32_t g = 0; g < heads; ++g)
+          sum = fmaf(mix[g], weights[g * kTileKeys + i % kTileKeys], sum);
+      } else {
+        sum = weights[h * kTileKeys + i % kTileKeys];
+      }
+      mixed[i] = sum;
+    }
+    __syncthreads();
+    const T* values = page_of<const T>(a, key0) + value_block(a, kv, key0 % a.page_tokens);
+    for (uint32_t i = threadIdx.x; i < group * a.vdim; i += blockDim.x)
+      out[i] = value_product(mixed + i / a.vdim * kTileKeys,
+                             values + size_t{i % a.vdim} * 32u, out[i]);
+  }
+  for (uint32_t i = threadIdx.x; i < group * a.vdim; i += blockDim.x)
+    args.partials[((size_t{row} * args.value_splits + blockIdx.x) * heads + kv * group) *
+                      a.vdim + i] = out[i];
 }
 
 // ---- split form (decode) -----------------------------------------------------------
@@ -488,6 +658,7 @@ __global__ __launch_bounds__(256) void split_values_kernel(AttentionArgs args) {
   }
 }
 
+template <typename T>
 __global__ void split_combine_kernel(AttentionArgs args) {
   const Attention& a = args.attention;
   const auto& run = args.launch;
@@ -506,7 +677,7 @@ __global__ void split_combine_kernel(AttentionArgs args) {
     float total = 0.0f;
 #pragma unroll
     for (uint32_t s = 0; s < kMaximumValueSplits; ++s) total += part[s];
-    store_element(static_cast<uint16_t*>(run.output) + size_t{row} * run.output_stride +
+    store_element(static_cast<T*>(run.output) + size_t{row} * run.output_stride +
                       head * a.vdim + d,
                   total * gate);
   }
@@ -1023,6 +1194,39 @@ size_t general_bytes(const Attention& a) {
   return size_t{a.query_heads} * (a.dim + 2u * kTileKeys + a.vdim + 2u) * 4u;
 }
 
+size_t general_scores_bytes(const Attention& a) {
+  return size_t{a.query_heads} * (a.dim + 2u) * 4u;
+}
+
+size_t general_values_bytes(const Attention& a) {
+  const size_t group = a.query_heads / a.kv_heads;
+  return (size_t{a.query_heads} * (2u + kTileKeys) + group * (kTileKeys + a.vdim)) * 4u;
+}
+
+// The parts of a split launch's workspace.
+void place_splits(AttentionArgs& args) {
+  const Attention& a = args.attention;
+  const uint32_t tiles = maximum_tiles(a, args.launch.maximum_position);
+  args.capacity = tiles * kTileKeys;
+  args.score_splits = score_splits_for(tiles);
+  args.value_splits = value_splits_for(tiles);
+  args.scores = static_cast<float*>(args.launch.workspace);
+  args.maxima = args.scores + size_t{args.launch.rows} * a.query_heads * args.capacity;
+  args.partials =
+      args.maxima + size_t{args.launch.rows} * args.score_splits * a.query_heads * 2u;
+}
+
+template <typename T>
+void launch_general_splits(const AttentionArgs& args, hipStream_t stream) {
+  const Attention& a = args.attention;
+  const uint32_t rows = args.launch.rows;
+  general_scores_kernel<T>
+      <<<dim3(args.score_splits, rows), 256, general_scores_bytes(a), stream>>>(args);
+  general_values_kernel<T><<<dim3(args.value_splits, a.kv_heads, rows), 256,
+                             general_values_bytes(a), stream>>>(args);
+  split_combine_kernel<T><<<dim3(a.query_heads, rows), 64, 0, stream>>>(args);
+}
+
 bool split_stride(uint32_t stride) {
   return stride == 64u || stride == 128u || stride == 256u;
 }
@@ -1105,6 +1309,21 @@ extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* a
     if (general_bytes(a) > kMaximumLds)
       return fail(QLLM_INVALID_ARGUMENT,
                   "windowed attention: heads and dimensions exceed the general kernel");
+    // Up to the split form's rows a workgroup per row leaves the chip idle (one row
+    // over 340 keys: 750 us against 53); a caller that brought no workspace
+    // for the splits, and heads whose buffers pass 64 KiB, stay with it.
+    if (launch->rows <= kSplitRows && launch->workspace &&
+        (reinterpret_cast<uintptr_t>(launch->workspace) & 15u) == 0u &&
+        launch->workspace_bytes >= qllm_windowed_attention_workspace_bytes(
+                                       attention, launch->rows, launch->maximum_position) &&
+        general_scores_bytes(a) <= 65536u && general_values_bytes(a) <= 65536u) {
+      place_splits(args);
+      if (a.element == QLLM_ELEMENT_F32)
+        launch_general_splits<float>(args, hip_stream);
+      else
+        launch_general_splits<uint16_t>(args, hip_stream);
+      return launched("windowed split attention");
+    }
     if (general_bytes(a) > 65536u) {
       const void* kernel = a.element == QLLM_ELEMENT_F32
                                ? reinterpret_cast<const void*>(general_attention_kernel<float>)
@@ -1140,13 +1359,7 @@ extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* a
           qllm_windowed_attention_workspace_bytes(attention, launch->rows,
                                                   launch->maximum_position))
     return fail(QLLM_INVALID_ARGUMENT, "windowed attention workspace is too small");
-  const uint32_t tiles = maximum_tiles(a, launch->maximum_position);
-  args.capacity = tiles * kTileKeys;
-  args.score_splits = score_splits_for(tiles);
-  args.value_splits = value_splits_for(tiles);
-  args.scores = static_cast<float*>(launch->workspace);
-  args.maxima = args.scores + size_t{launch->rows} * a.query_heads * args.capacity;
-  args.partials = args.maxima + size_t{launch->rows} * args.score_splits * a.query_heads * 2u;
+  place_splits(args);
   const dim3 score_grid(args.score_splits, a.kv_heads, launch->rows);
   if (a.key_stride == 64u)
     split_scores_kernel<2><<<score_grid, 256, 0, hip_stream>>>(args);
@@ -1169,6 +1382,7 @@ extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* a
     values(std::integral_constant<int, 8>{});
   else
     values(std::integral_constant<int, 16>{});
-  split_combine_kernel<<<dim3(a.query_heads, launch->rows), 64, 0, hip_stream>>>(args);
+  split_combine_kernel<uint16_t>
+      <<<dim3(a.query_heads, launch->rows), 64, 0, hip_stream>>>(args);
   return launched("windowed split attention");
 }

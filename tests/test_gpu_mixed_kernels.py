@@ -302,6 +302,25 @@ class Attention:
         return (out * mo.sigmoid(gate)[:, :, None]).reshape(rows, -1)
 
 
+@pytest.mark.parametrize("element,heads,kv,dim,vdim,window", [
+    (F32, 16, 4, 128, 128, 0), (F32, 5, 1, 40, 24, 700), (F32, 40, 2, 32, 32, 100),
+    (BF16, 40, 2, 32, 32, 0)])
+def test_general_splits_equal_a_workgroup_per_row(device, element, heads, kv, dim, vdim,
+                                                  window):
+    """One to four rows over a long context, dealt over workgroups, against the same
+    rows as the end of a batch that takes a workgroup for each."""
+    rng = np.random.default_rng(heads)
+    total, scale = 1300, 1.0 / np.sqrt(dim)
+    mix = mm.bf16(np.eye(heads) + 0.2 * rng.standard_normal((heads, heads)))
+    layer = Attention(device, element, heads, kv, dim, vdim, window, 3, mix, scale,
+                      context=1344)
+    projections = mm.bf16(rng.standard_normal((total, layer.stride)))
+    whole = layer.run(projections, 0)
+    for rows in (1, 2, 3, 4):
+        again = layer.run(projections[total - rows:], total - rows)
+        close(again, whole[total - rows:], element)
+
+
 def stand_out(rng, layer, projections, pairs, head, strength=None):
     """Makes the score of (query row, key row) of one head stand out: the key
     becomes the query direction (unrotated dimensions or rotary 0 assumed)."""
