@@ -897,6 +897,16 @@ int32_t qllm_apply_presence_penalty_rows(float* logits, size_t row_stride,
 int32_t qllm_mark_presence(uint8_t* emitted, const uint32_t* tokens,
                            uint32_t token_count, uint32_t count, void* stream);
 
+/* The same for up to 16 tokens in host memory, read before the call returns: they
+ * travel in the launch's arguments, with no copy. */
+int32_t qllm_mark_presence_values(uint8_t* emitted, const uint32_t* host_tokens,
+                                  uint32_t count, uint32_t vocabulary, void* stream);
+
+/* Up to 16 words from host memory (read before the call returns) to device memory:
+ * a launch that carries them instead of a copy. */
+int32_t qllm_store_words(uint32_t* destination, const uint32_t* host_words,
+                         uint32_t count, void* stream);
+
 /* ---- mixed-layer decoders -------------------------------------------------------
  *
  * Kernels of decoders whose layers differ: windowed attention with mixed heads

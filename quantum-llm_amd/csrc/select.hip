@@ -6,12 +6,14 @@
 // NaN never selected.
 #include "common.hpp"
 
+#include <algorithm>
 #include <mutex>
 
 namespace qllm {
 namespace {
 
 constexpr uint32_t kNoIndex = 0xffffffffu;
+constexpr uint32_t kMaximumWords = 16;   // words that travel in a launch
 constexpr uint32_t kArgmaxChunk = 2048;   // items per stage-1 block
 constexpr uint32_t kTopkChunk = 4096;     // items per stage-1 block
 constexpr uint32_t kTopkThreads = 256;
@@ -410,6 +412,24 @@ __global__ __launch_bounds__(256) void presence_penalty_rows_kernel(
   }
 }
 
+// A few words that travel in a launch's arguments instead of through a copy.
+struct Words {
+  uint32_t value[kMaximumWords];
+};
+
+__global__ __launch_bounds__(64) void store_words_kernel(uint32_t* destination, Words words,
+                                                         uint32_t count) {
+  if (threadIdx.x < count) destination[threadIdx.x] = words.value[threadIdx.x];
+}
+
+__global__ __launch_bounds__(64) void mark_values_kernel(uint8_t* emitted, Words tokens,
+                                                         uint32_t count,
+                                                         uint32_t vocabulary) {
+  if (threadIdx.x >= count) return;
+  const uint32_t token = tokens.value[threadIdx.x];
+  if (token < vocabulary) emitted[token] = 1u;
+}
+
 __global__ __launch_bounds__(64) void mark_presence_kernel(
     uint8_t* emitted, const uint32_t* tokens, uint32_t token_count,
     uint32_t count) {
@@ -620,6 +640,27 @@ extern "C" int32_t qllm_apply_presence_penalty_rows(
                                  as_stream(stream)>>>(
       logits, row_stride, emitted, drafts, rows, count, penalty);
   return launched("presence penalty rows");
+}
+
+extern "C" int32_t qllm_store_words(uint32_t* destination, const uint32_t* host_words,
+                                    uint32_t count, void* stream) {
+  if (!destination || !host_words || !count || count > kMaximumWords)
+    return fail(QLLM_INVALID_ARGUMENT, "invalid word store");
+  Words words{};
+  std::copy_n(host_words, count, words.value);
+  store_words_kernel<<<1, 64, 0, as_stream(stream)>>>(destination, words, count);
+  return launched("word store");
+}
+
+extern "C" int32_t qllm_mark_presence_values(uint8_t* emitted, const uint32_t* host_tokens,
+                                             uint32_t count, uint32_t vocabulary,
+                                             void* stream) {
+  if (!emitted || !host_tokens || !count || count > kMaximumWords || !vocabulary)
+    return fail(QLLM_INVALID_ARGUMENT, "invalid presence marks");
+  Words tokens{};
+  std::copy_n(host_tokens, count, tokens.value);
+  mark_values_kernel<<<1, 64, 0, as_stream(stream)>>>(emitted, tokens, count, vocabulary);
+  return launched("presence marks");
 }
 
 extern "C" int32_t qllm_mark_presence(uint8_t* emitted, const uint32_t* tokens,

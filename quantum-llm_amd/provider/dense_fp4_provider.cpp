@@ -196,7 +196,7 @@ void Mi355DenseFp4Provider::allocate_workspaces() {
       std::max<std::size_t>({g_.hidden, g_.intermediate,
                              std::size_t{g_.query_heads} * g_.head_dim});
   // tokens (up to 8) and the four position words of a pass lie side by side,
-  // so that one copy from pinned host memory uploads both
+  // so that one launch brings both
   tokens_ = static_cast<std::uint32_t*>(device_alloc((8U + 4U) * 4U));
   positions_ = tokens_ + 8U;
   {
@@ -1933,10 +1933,7 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
       predicted = selector_->select(logits_, presence_, argmax_tokens_, request,
                                     first_position + count - 1U);
     } else {
-      hip_check(hipMemcpyAsync(&predicted, argmax_tokens_, sizeof(predicted),
-                               hipMemcpyDeviceToHost, hip_stream),
-                "copy the prompt's prediction");
-      hip_check(hipStreamSynchronize(hip_stream), "prompt prefill");
+      predicted = selector_->read_token(argmax_tokens_);
     }
     prefill_tokens_total_ += count;
     if (state) {
@@ -2003,15 +2000,12 @@ er::Status Mi355DenseFp4Provider::run_target_graph(const std::uint32_t* tokens,
       return {er::ErrorCode::invalid_argument, "target program is not prepared"};
     ensure_pages(first_position + rows - 1U);
     const auto stream = static_cast<hipStream_t>(stream_);
-    // The stream is idle here (every pass ends with a wait), so the pinned
-    // words of the previous pass have been read.
-    std::copy(tokens, tokens + rows, staging_->target);
+    std::uint32_t words[12]{};
+    std::copy(tokens, tokens + rows, words);
     const std::uint32_t positions[4] = {first_position, first_position,
                                         first_position + 1U, rows};
-    std::copy(positions, positions + 4, staging_->target + 8);
-    hip_check(hipMemcpyAsync(tokens_, staging_->target, sizeof(staging_->target),
-                             hipMemcpyHostToDevice, stream),
-              "upload target tokens and positions");
+    std::copy(positions, positions + 4, words + 8);
+    status_check(qllm_store_words(tokens_, words, 12U, stream_));
     if (!graphs_[rows]) {
       hip_check(hipStreamSynchronize(stream), "drain stream before capture");
       hipGraph_t graph{};
@@ -2663,12 +2657,10 @@ void Mi355DenseFp4Provider::propose_with_graphs(
   ensure_pages(committed_length + drafts - 2U);
   const std::uint32_t positions[4] = {first_position, first_position + 1U,
                                       first_position + 1U, 0U};
-  std::copy(tokens.begin(), tokens.end(), staging_->proposer);
-  std::copy(positions, positions + 4, staging_->proposer + 8);
-  hip_check(hipMemcpyAsync(mtp_tokens_, staging_->proposer,
-                           sizeof(staging_->proposer), hipMemcpyHostToDevice,
-                           stream),
-            "upload MTP tokens and positions");
+  std::uint32_t words[12]{};
+  std::copy(tokens.begin(), tokens.end(), words);
+  std::copy(positions, positions + 4, words + 8);
+  status_check(qllm_store_words(mtp_tokens_, words, 12U, stream_));
   state.draft_predictions.clear();
   state.draft_predictions.reserve(drafts);
   const bool greedy =
@@ -2696,13 +2688,8 @@ void Mi355DenseFp4Provider::propose_with_graphs(
     for (std::uint32_t depth = 0; depth < drafts; ++depth) {
       if (depth) {
         // the device chained its own argmax; the sampled draft replaces it
-        // (pinned word: the previous pass ended with a wait, and the copy is
-        // ordered before the pass launched next)
-        staging_->proposer[0] = state.draft_predictions.back().token;
-        hip_check(hipMemcpyAsync(mtp_tokens_, staging_->proposer,
-                                 sizeof(std::uint32_t), hipMemcpyHostToDevice,
-                                 stream),
-                  "upload sampled MTP draft");
+        const std::uint32_t sampled = state.draft_predictions.back().token;
+        status_check(qllm_store_words(mtp_tokens_, &sampled, 1U, stream_));
       }
       launch_mtp_graph(depth ? 1U : rows, depth != 0U);
       DraftPrediction prediction;

@@ -440,11 +440,9 @@ class Mi355DenseFp4Provider final : public DecoderProvider {
   std::int8_t* query_operands_{};       // Q4H attention operands of a batch
   float* query_operand_scales_{};
   float* rope_table_{};                 // [max_rows, rotary_dim / 2] (cos, sin)
-  // Pinned host words for the small per-pass transfers: 8 tokens + 4
-  // position words up (target pass, proposer pass), 8 chosen tokens down.
+  // Pinned host words for the chosen tokens that come down after a pass (what
+  // goes up - 8 tokens, 4 position words - travels in a launch's arguments).
   struct HostStaging {
-    std::uint32_t target[12];
-    std::uint32_t proposer[12];
     std::uint32_t download[8];
   };
   HostStaging* staging_ = nullptr;

@@ -913,9 +913,13 @@ void Mi355MixedProvider::begin_batch(MixedRequestState& state,
   words[2] = rows;
   words[3] = 0U;
   std::copy(tokens.begin(), tokens.end(), words + kStepWords);
-  hip_check(hipMemcpyAsync(step_.get(), words, (kStepWords + rows) * 4U,
-                           hipMemcpyHostToDevice, stream),
-            "upload batch words");
+  if (rows == 1U)
+    status_check(qllm_store_words(step_.as<std::uint32_t>(), words, kStepWords + 1U,
+                                  stream_));
+  else
+    hip_check(hipMemcpyAsync(step_.get(), words, (kStepWords + rows) * 4U,
+                             hipMemcpyHostToDevice, stream),
+              "upload batch words");
   batch_rows_ = rows;
 }
 

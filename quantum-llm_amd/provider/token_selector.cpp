@@ -16,12 +16,10 @@ TokenSelector::TokenSelector(void* stream, std::uint32_t vocabulary, void* works
                              std::size_t workspace_bytes)
     : stream_(stream), vocabulary_(vocabulary), workspace_(workspace),
       workspace_bytes_(workspace_bytes),
-      device_(8U * kMaximumTopK * (4U + 4U) + 8U * 4U, "allocate token selection") {
-  // top-k logits of up to 8 rows, then their tokens: one buffer, one readback;
-  // the marks follow
+      device_(8U * kMaximumTopK * (4U + 4U), "allocate token selection") {
+  // top-k logits of up to 8 rows, then their tokens: one buffer, one readback
   top_logits_ = device_.as<float>();
   top_tokens_ = reinterpret_cast<std::uint32_t*>(top_logits_ + 8U * kMaximumTopK);
-  mark_tokens_ = top_tokens_ + 8U * kMaximumTopK;
   void* pinned = nullptr;
   hip_check(hipHostMalloc(&pinned, sizeof(Staging), hipHostMallocDefault),
             "allocate pinned staging");
@@ -43,18 +41,21 @@ std::size_t TokenSelector::workspace_bytes(std::uint32_t vocabulary,
 void TokenSelector::mark(
     std::uint8_t* emitted, std::span<const std::uint32_t> tokens) {
   if (tokens.empty()) return;
-  if (tokens.size() > 8U) throw std::runtime_error("too many presence marks");
-  const auto stream = static_cast<hipStream_t>(stream_);
-  // the pinned words are free: every pass that used them ended with a wait
-  std::copy(tokens.begin(), tokens.end(), staging_->marks);
-  hip_check(hipMemcpyAsync(mark_tokens_, staging_->marks, tokens.size() * 4U,
-                           hipMemcpyHostToDevice, stream),
-            "upload presence marks");
-  status_check(qllm_mark_presence(emitted, mark_tokens_,
-                                  static_cast<std::uint32_t>(tokens.size()),
-                                  vocabulary_, stream_));
+  status_check(qllm_mark_presence_values(emitted, tokens.data(),
+                                         static_cast<std::uint32_t>(tokens.size()),
+                                         vocabulary_, stream_));
 }
 
+// One word of device memory, through pinned memory: a copy to pageable memory is
+// staged and waited for twice.
+std::uint32_t TokenSelector::read_token(const std::uint32_t* device_token) {
+  const auto stream = static_cast<hipStream_t>(stream_);
+  hip_check(hipMemcpyAsync(&staging_->token, device_token, sizeof(std::uint32_t),
+                           hipMemcpyDeviceToHost, stream),
+            "copy greedy token");
+  hip_check(hipStreamSynchronize(stream), "copy greedy token");
+  return staging_->token;
+}
 
 // The head's token for a request (run_head with a request, :8433-8517): the
 // presence penalty from the first output position on, arg-max at temperature
@@ -81,10 +82,7 @@ std::uint32_t TokenSelector::select(float* logits, std::uint8_t* presence,
   const auto temperature = request_parameter(request, "sampling_temperature_ppm");
   std::uint32_t selected{};
   if (temperature == 0U) {
-    hip_check(hipMemcpyAsync(&selected, argmax_tokens, sizeof(selected),
-                             hipMemcpyDeviceToHost, stream),
-              "copy greedy token");
-    hip_check(hipStreamSynchronize(stream), "copy greedy token");
+    selected = read_token(argmax_tokens);
     // a row without a finite logit selects nothing (0xffffffff): reported
     // before the presence bytes or the caller's state change
     if (selected >= vocabulary_)
@@ -167,14 +165,7 @@ er::SamplingDistribution TokenSelector::distribution(
                                      workspace_, workspace_bytes_,
                                      stream_));
   }
-  if (temperature == 0U) {
-    std::uint32_t token{};
-    hip_check(hipMemcpyAsync(&token, device_argmax, sizeof(token),
-                             hipMemcpyDeviceToHost, stream),
-              "copy exact greedy token");
-    hip_check(hipStreamSynchronize(stream), "copy exact greedy token");
-    return {{{token, 1.0}}};
-  }
+  if (temperature == 0U) return {{{read_token(device_argmax), 1.0}}};
   const auto top_p = static_cast<std::uint32_t>(
       request_parameter(request, "sampling_top_p_ppm"));
   const auto min_p = static_cast<std::uint32_t>(

@@ -42,7 +42,9 @@ class TokenSelector final {
   [[nodiscard]] std::vector<er::SamplingDistribution> top_k_distributions(
       const float* logits, std::uint32_t vocabulary, std::size_t stride,
       std::uint32_t rows, const er::ProgramRequestContext& request);
-  // emitted[token] = 1 for every token (one upload, one launch)
+  // A selection on the device, after everything enqueued so far.
+  [[nodiscard]] std::uint32_t read_token(const std::uint32_t* device_token);
+  // emitted[token] = 1 for every token (one launch)
   void mark(std::uint8_t* emitted, std::span<const std::uint32_t> tokens);
 
   [[nodiscard]] std::uint64_t gpu_calls() const noexcept { return gpu_calls_; }
@@ -54,7 +56,7 @@ class TokenSelector final {
   struct Staging final {
     float top_logits[8 * kMaximumTopK];            // top-k readback: logits of all
     std::uint32_t top_tokens[8 * kMaximumTopK];    // rows, then their tokens
-    std::uint32_t marks[8];                        // tokens whose byte is set
+    std::uint32_t token;                           // one row's selection
   };
   void* stream_{};
   std::uint32_t vocabulary_{};
@@ -63,7 +65,6 @@ class TokenSelector final {
   DeviceBuffer device_;
   float* top_logits_{};
   std::uint32_t* top_tokens_{};
-  std::uint32_t* mark_tokens_{};
   Staging* staging_{};
   std::uint64_t gpu_calls_{};
   std::uint64_t logit_transfer_bytes_{};

@@ -476,3 +476,27 @@ def test_norm_of_partial_sums_with_and_without_a_residual(device):
     assert np.array_equal(got_sum, want)
     normed = ol.rms_norm_rows(want, weight, 1e-6, True)
     assert (np.abs(got_out - normed) <= np.abs(normed) * 2.0 ** -8 + 2e-5).all()
+
+
+@pytest.mark.parametrize("count", [1, 5, 16])
+def test_words_and_marks_travel_in_a_launch(device, count):
+    """Host words are read before the call returns; marks outside the vocabulary
+    are ignored; more than sixteen are turned down."""
+    words = np.arange(7, 7 + count, dtype=np.uint32)
+    target = torch.zeros(20, dtype=torch.int32, device=device)
+    marks = np.array([(3 * i) % 40 for i in range(count)], dtype=np.uint32)
+    marks[-1] = 0xffffffff
+    emitted = torch.zeros(32, dtype=torch.uint8, device=device)
+    qh.call("qllm_store_words", qh.ptr(target), words.ctypes.data, count, None)
+    qh.call("qllm_mark_presence_values", qh.ptr(emitted), marks.ctypes.data, count, 32, None)
+    expected = np.zeros(32, dtype=np.uint8)
+    expected[[m for m in marks if m < 32]] = 1
+    kept = words.copy()
+    words[:] = 0
+    assert np.array_equal(target.cpu().numpy()[:count], kept.astype(np.int32))
+    assert not target.cpu().numpy()[count:].any()
+    assert np.array_equal(emitted.cpu().numpy(), expected)
+    for name, arguments in (("qllm_store_words", ()), ("qllm_mark_presence_values", (32,))):
+        with pytest.raises(qh.QllmError, match="invalid"):
+            qh.call(name, qh.ptr(target), np.zeros(17, np.uint32).ctypes.data, 17, *arguments,
+                    None)
