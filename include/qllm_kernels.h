@@ -630,6 +630,19 @@ int32_t qllm_rope_table(float* table, uint32_t rows, uint32_t rotary_dim,
                         uint32_t first_rotary_position, float rope_theta,
                         int32_t bf16_activations,
                         const uint32_t* device_positions, void* stream);
+/* Rotary and K/V store of a batch whose (cos, sin) pairs lie in rope_table
+ * [rows][rotary_dim / 2][2]: head norms (weights may be NULL) and rotation of query
+ * and key rows in place, then the rows' records in the layer's pages - Q4H, or
+ * binary16 with f16_pages; page_table NULL: rotation only.  Values and bytes equal
+ * qllm_qkv_rope_cache_paged_q4h_batch, or qllm_qkv_rope_batch followed by
+ * qllm_store_kv_paged_f16_batch.  head_dim 128 or 256. */
+int32_t qllm_qkv_rope_table_batch(
+    float* query, uint32_t query_stride, float* key, const float* value,
+    const float* q_norm_weight, const float* k_norm_weight, const float* rope_table,
+    const void* const* page_table, int32_t f16_pages, uint32_t full_attention_layer,
+    uint32_t page_tokens, uint32_t first_cache_position, uint32_t rows,
+    uint32_t query_heads, uint32_t kv_heads, uint32_t head_dim, uint32_t rotary_dim,
+    float epsilon, int32_t bf16_activations, void* stream);
 /* Many micro-batches in one launch (prompt prefill): the launch's `rows` rows
  * are attended in batches of `batch_rows` consecutive rows, batch b exactly as
  * a launch of its own with first_context_tokens + b * batch_rows would be

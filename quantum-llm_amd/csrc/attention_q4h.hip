@@ -2107,6 +2107,169 @@ __global__ __launch_bounds__(64) void qkv_rope_q4h_kernel(
   }
 }
 
+// ---- rotary and store from a table ------------------------------------------------
+
+struct TableRopeArgs {
+  float* query;
+  uint32_t query_stride;
+  float* key;
+  const float* value;
+  const float* q_weight;
+  const float* k_weight;
+  const float2* table;             // [rows][rotary_dim / 2]
+  const void* const* page_table;   // null: rotary only
+  uint32_t layer;
+  uint32_t page_tokens;
+  uint32_t first_cache_position;
+  uint32_t rows;
+  uint32_t query_heads;
+  uint32_t kv_heads;
+  uint32_t rotary_dim;
+  float epsilon;
+  bool bf16_activations;
+};
+
+enum StoreKind { kStoreQ4h, kStoreF16 };
+
+// qkv_rope_q4h_kernel's work (and f16_store_kernel's) for the rows of a prompt or
+// of a verify step with the exact cache: same arithmetic, same bytes.  What bounds
+// it is memory: a row of 72 heads of 128 is 37 KB in and 34 KB out.  The kernel
+// above computes a power, a sine and a cosine per element, for every head again,
+// and has one row of a head in flight per wave (16384 rows of 64 + 8 heads 898 us,
+// 300 rows 41); here cosine and sine come from the table of the pass, and a wave
+// fetches R rows before it works on the first (280 us, 4.3 TB/s, and 11; 3001 rows of
+// 24 + 4 heads of 256, with gates and norms, 114 -> 56).
+// N = head_dim / 64; lane l holds elements l, l + 64, ...
+template <int N, int R, int STORE>
+__global__ __launch_bounds__(256) void table_rope_kernel(const TableRopeArgs args) {
+  constexpr uint32_t D = 64u * N;
+  __shared__ float rows_of_waves[4][D];
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = threadIdx.x >> 6;
+  float* const scratch = rows_of_waves[wave];
+  const uint32_t first = (blockIdx.y * 4u + wave) * R;
+  if (first >= args.rows) return;
+  const bool is_query = blockIdx.x < args.query_heads;
+  const uint32_t head = is_query ? blockIdx.x : blockIdx.x - args.query_heads;
+  const size_t row_step = is_query ? size_t{args.query_heads} * args.query_stride
+                                   : size_t{args.kv_heads} * D;
+  float* const base = is_query ? args.query + size_t{head} * args.query_stride
+                               : args.key + size_t{head} * D;
+  const float* const weight = is_query ? args.q_weight : args.k_weight;
+  const bool stores = !is_query && args.page_table;
+  const uint32_t half = args.rotary_dim / 2u;
+
+  float x[R][N], v[R][N];
+  float2 turn[R][N];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const size_t row = min(first + r, args.rows - 1u);
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const uint32_t index = lane + 64u * k;
+      x[r][k] = base[row * row_step + index];
+      v[r][k] = stores ? args.value[row * row_step + size_t{head} * D + index] : 0.0f;
+      turn[r][k] = index < args.rotary_dim
+                       ? args.table[row * half + (index < half ? index : index - half)]
+                       : make_float2(1.0f, 0.0f);
+    }
+  }
+  float factor[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) factor[k] = weight ? 1.0f + weight[lane + 64u * k] : 1.0f;
+
+  // one wave's LDS: its reads and writes stay in the order they are written in
+  const auto settle = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const uint32_t row = first + r;
+    if (row >= args.rows) break;
+    if (weight) {
+      float square = 0.0f;
+#pragma unroll
+      for (int k = 0; k < N; ++k) square = fmaf(x[r][k], x[r][k], square);
+      square = wave_sum(square);
+      const float inverse = rsqrtf(square / static_cast<float>(D) + args.epsilon);
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        const float value = x[r][k] * inverse * factor[k];
+        x[r][k] = args.bf16_activations ? bf16_round(value) : value;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) scratch[lane + 64u * k] = x[r][k];
+    settle();
+    float turned[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const uint32_t index = lane + 64u * k;
+      float result = x[r][k];
+      if (index < args.rotary_dim) {
+        const float other =
+            index < half ? -scratch[index + half] : scratch[index - half];
+        result = __fmaf_rn(x[r][k], turn[r][k].x, __fmul_rn(other, turn[r][k].y));
+      }
+      turned[k] = args.bf16_activations ? bf16_round(result) : result;
+      base[row * row_step + index] = turned[k];
+    }
+    settle();
+    if (!stores) continue;
+    const uint32_t position = args.first_cache_position + row;
+    const uint32_t slot = position % args.page_tokens;
+    uint8_t* const page = static_cast<uint8_t*>(
+        const_cast<void*>(args.page_table[position / args.page_tokens]));
+    if constexpr (STORE == kStoreF16) {
+      const size_t width = size_t{args.kv_heads} * D;
+      const size_t page_values = args.page_tokens * width;
+      uint16_t* const keys = reinterpret_cast<uint16_t*>(page) +
+                             size_t{args.layer} * 2u * page_values + slot * width +
+                             size_t{head} * D;
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        keys[lane + 64u * k] = static_cast<uint16_t>(f32_to_f16_bits(turned[k]));
+        keys[page_values + lane + 64u * k] =
+            static_cast<uint16_t>(f32_to_f16_bits(v[r][k]));
+      }
+    } else {
+      const Q4hPlanes planes =
+          q4h_planes(page, args.layer, args.page_tokens, args.kv_heads, D);
+      const size_t record = size_t{head} * args.page_tokens + slot;
+#pragma unroll
+      for (int k = 0; k < N; ++k) scratch[lane + 64u * k] = turned[k];
+      settle();
+      q4h_encode_record(scratch, D, const_cast<uint8_t*>(planes.key_codes) + record * (D / 2u),
+                        const_cast<uint8_t*>(planes.key_scales) + record * 2u, lane);
+      settle();
+#pragma unroll
+      for (int k = 0; k < N; ++k) scratch[lane + 64u * k] = v[r][k];
+      settle();
+      q4h_encode_record(scratch, D,
+                        const_cast<uint8_t*>(planes.value_codes) + record * (D / 2u),
+                        const_cast<uint8_t*>(planes.value_scales) + record * 2u, lane);
+      settle();
+    }
+  }
+}
+
+template <int STORE>
+void launch_table_rope(const TableRopeArgs& args, uint32_t head_dim, hipStream_t stream) {
+  // four rows a wave once that still gives every SIMD a few waves
+  const uint32_t heads = args.query_heads + args.kv_heads;
+  const bool several = uint64_t{heads} * args.rows >= 16384u;
+  const dim3 grid(heads, (args.rows + (several ? 15u : 3u)) / (several ? 16u : 4u));
+  if (head_dim == 128u && several)
+    table_rope_kernel<2, 4, STORE><<<grid, 256, 0, stream>>>(args);
+  else if (head_dim == 128u)
+    table_rope_kernel<2, 1, STORE><<<grid, 256, 0, stream>>>(args);
+  else if (several)
+    table_rope_kernel<4, 4, STORE><<<grid, 256, 0, stream>>>(args);
+  else
+    table_rope_kernel<4, 1, STORE><<<grid, 256, 0, stream>>>(args);
+}
+
 // transformer_kernels.cu:4391-4416
 __global__ __launch_bounds__(64) void quantize_queries_q8_kernel(
     const float* query, uint32_t query_stride, int8_t* q8, float* scales,
@@ -2683,4 +2846,31 @@ extern "C" int32_t qllm_rope_table(float* table, uint32_t rows,
       reinterpret_cast<float2*>(table), rotary_dim, first_rotary_position,
       rope_theta, bf16_activations != 0, device_positions);
   return launched("rotary table");
+}
+
+extern "C" int32_t qllm_qkv_rope_table_batch(
+    float* query, uint32_t query_stride, float* key, const float* value,
+    const float* q_norm_weight, const float* k_norm_weight, const float* rope_table,
+    const void* const* page_table, int32_t f16_pages, uint32_t full_attention_layer,
+    uint32_t page_tokens, uint32_t first_cache_position, uint32_t rows,
+    uint32_t query_heads, uint32_t kv_heads, uint32_t head_dim, uint32_t rotary_dim,
+    float epsilon, int32_t bf16_activations, void* stream) {
+  if (!query || !key || !rope_table || (page_table && (!value || !page_tokens)) ||
+      !rows || rows > 16u * 65535u || !query_heads || !kv_heads ||
+      query_heads < kv_heads || query_heads % kv_heads ||
+      (head_dim != 128u && head_dim != 256u) || query_stride < head_dim || !rotary_dim ||
+      rotary_dim > head_dim || rotary_dim % 2u || !(epsilon > 0.0f) ||
+      (reinterpret_cast<uintptr_t>(rope_table) & 7u) ||
+      first_cache_position > 0xffffffffu - (rows - 1u))
+    return fail(QLLM_INVALID_ARGUMENT, "invalid QKV rope batch from a table");
+  const TableRopeArgs args{query, query_stride, key, value, q_norm_weight, k_norm_weight,
+                           reinterpret_cast<const float2*>(rope_table), page_table,
+                           full_attention_layer, page_tokens, first_cache_position, rows,
+                           query_heads, kv_heads, rotary_dim, epsilon,
+                           bf16_activations != 0};
+  if (f16_pages)
+    launch_table_rope<kStoreF16>(args, head_dim, as_stream(stream));
+  else
+    launch_table_rope<kStoreQ4h>(args, head_dim, as_stream(stream));
+  return launched("QKV rope batch from a table");
 }

@@ -292,10 +292,10 @@ void Mi355DenseFp4Provider::allocate_workspaces() {
               "clear query operands");
     hip_check(hipMemset(query_operand_scales_, 0, scale_bytes),
               "clear query operand scales");
-    // (cos, sin) of a batch's rotary angles, computed once per pass
-    rope_table_ = static_cast<float*>(
-        device_alloc(std::size_t{max_rows_} * g_.rotary_dim * 4U));
   }
+  // (cos, sin) of a batch's rotary angles, computed once per pass
+  rope_table_ = static_cast<float*>(
+      device_alloc(std::size_t{max_rows_} * g_.rotary_dim * 4U));
 
   // the heads' tile maxima: 32 vocabulary rows per tile
   const std::size_t head_maxima_bytes =
@@ -1245,14 +1245,11 @@ void Mi355DenseFp4Provider::enqueue_attention(
       status_check(qllm_attention_paged_q4h(&launch));
     }
   } else {
-    status_check(qllm_qkv_rope_batch(
-        query, query_stride, key, layer.query_norm, layer.key_norm,
-        first_position, rows, g_.query_heads, g_.kv_heads, g_.head_dim,
-        g_.rotary_dim, g_.norm_epsilon, g_.rope_theta, 0, stream));
-    status_check(qllm_store_kv_paged_f16_batch(
-        key, value, const_cast<const void* const*>(device_page_table_),
-        index, g_.kv_page_tokens, first_position, rows, g_.kv_heads,
-        g_.head_dim, stream));
+    status_check(qllm_qkv_rope_table_batch(
+        query, query_stride, key, value, layer.query_norm, layer.key_norm, rope_table_,
+        const_cast<const void* const*>(device_page_table_), 1, index,
+        g_.kv_page_tokens, first_position, rows, g_.query_heads, g_.kv_heads,
+        g_.head_dim, g_.rotary_dim, g_.norm_epsilon, 0, stream));
     qllm_f16_attention_launch launch{};
     launch.query = query;
     launch.device_pages = const_cast<const void* const*>(device_page_table_);
@@ -1305,7 +1302,6 @@ std::uint32_t Mi355DenseFp4Provider::prompt_attention_splits(
 void Mi355DenseFp4Provider::enqueue_rope_table(std::uint32_t rows,
                                                std::uint32_t first_position,
                                                bool deferred_positions) {
-  if (!rope_table_) return;
   status_check(qllm_rope_table(rope_table_, rows, g_.rotary_dim, first_position,
                                g_.rope_theta, 0,
                                deferred_positions ? positions_ : nullptr,
@@ -1660,6 +1656,7 @@ void Mi355DenseFp4Provider::ensure_prefill_workspace(std::uint32_t rows) {
   prefill_attention_ = static_cast<std::uint16_t*>(
       allocate(n * g_.query_heads * g_.head_dim * 2U));
   prefill_embedding_ = static_cast<float*>(allocate(n * g_.hidden * 4U));
+  prefill_rope_table_ = static_cast<float*>(allocate(n * g_.rotary_dim * 4U));
   prefill_parts_bytes_ = qllm_fp4_tall_workspace_bytes();
   prefill_parts_ = static_cast<float*>(allocate(prefill_parts_bytes_));
   // the MLP's activation; the proposer's fusion input [rows, 2 hidden] too
@@ -1754,6 +1751,8 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
       status_check(qllm_fp4_embedding_batch(&embedding_.descriptor,
                                             prefill_tokens_, prefill_hidden_,
                                             rows, stream));
+      status_check(qllm_rope_table(prefill_rope_table_, rows, g_.rotary_dim, position,
+                                   g_.rope_theta, 0, nullptr, stream));
       const std::size_t hidden_bytes = std::size_t{rows} * g_.hidden * 2U;
       // A projection onto the residual stream whose launch is cut along K leaves
       // its parts to the norm that follows, as in a verify step.
@@ -1804,11 +1803,11 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
           const std::uint32_t query_stride =
               g_.head_dim * (g_.output_gated ? 2U : 1U);
           const auto pages = const_cast<const void* const*>(device_page_table_);
-          status_check(qllm_qkv_rope_cache_paged_q4h_batch(
+          status_check(qllm_qkv_rope_table_batch(
               prefill_query_, query_stride, prefill_key_, prefill_value_,
-              layer.query_norm, layer.key_norm, pages, index, g_.kv_page_tokens,
-              position, position, rows, g_.query_heads, g_.kv_heads, g_.head_dim,
-              g_.rotary_dim, g_.norm_epsilon, g_.rope_theta, 0, stream));
+              layer.query_norm, layer.key_norm, prefill_rope_table_, pages, 0, index,
+              g_.kv_page_tokens, position, rows, g_.query_heads, g_.kv_heads,
+              g_.head_dim, g_.rotary_dim, g_.norm_epsilon, 0, stream));
           qllm_q4h_attention_launch launch{};
           launch.query = prefill_query_;
           launch.page_table = pages;
@@ -1844,14 +1843,11 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
           const std::uint32_t query_stride =
               g_.head_dim * (g_.output_gated ? 2U : 1U);
           const auto pages = const_cast<const void* const*>(device_page_table_);
-          status_check(qllm_qkv_rope_batch(
-              prefill_query_, query_stride, prefill_key_, layer.query_norm,
-              layer.key_norm, position, rows, g_.query_heads, g_.kv_heads,
-              g_.head_dim, g_.rotary_dim, g_.norm_epsilon, g_.rope_theta, 0,
-              stream));
-          status_check(qllm_store_kv_paged_f16_batch(
-              prefill_key_, prefill_value_, pages, index, g_.kv_page_tokens,
-              position, rows, g_.kv_heads, g_.head_dim, stream));
+          status_check(qllm_qkv_rope_table_batch(
+              prefill_query_, query_stride, prefill_key_, prefill_value_,
+              layer.query_norm, layer.key_norm, prefill_rope_table_, pages, 1, index,
+              g_.kv_page_tokens, position, rows, g_.query_heads, g_.kv_heads,
+              g_.head_dim, g_.rotary_dim, g_.norm_epsilon, 0, stream));
           qllm_f16_attention_launch launch{};
           launch.query = prefill_query_;
           launch.device_pages = pages;

@@ -497,6 +497,7 @@ class Mi355DenseFp4Provider final : public DecoderProvider {
   std::uint16_t* prefill_attention_{};    // bf16 [rows, query_heads * head_dim]
   float* prefill_embedding_{};
   std::uint16_t* prefill_activation_{};   // bf16 [rows, intermediate]
+  float* prefill_rope_table_{};           // [rows, rotary_dim / 2] (cos, sin)
   float* prefill_parts_{};                // parts of projections cut along K
   std::size_t prefill_parts_bytes_{};
   // split partials of the batched prompt attention: [rows, splits, heads(, d)]

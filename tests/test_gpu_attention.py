@@ -442,3 +442,60 @@ def test_fused_rotary_attention_equals_the_two_launches(device, tokens, rows, Q,
     for index, (a, b) in enumerate(zip(plain_pages, fused_pages)):
         assert np.array_equal(a, b), index
     assert not np.array_equal(plain_pages[-1], pages[-1])   # the batch was stored
+
+
+@pytest.mark.parametrize("rows,first", [(1, 0), (5, 61), (17, 4), (333, 190)])
+@pytest.mark.parametrize("head_dim,rotary,heads,kv,gated,qk_norm,rounded", [
+    (128, 128, 16, 4, False, False, 0), (128, 40, 6, 2, True, True, 1),
+    (256, 64, 48, 4, True, True, 0), (256, 256, 2, 1, False, False, 0)])
+@pytest.mark.parametrize("f16", [0, 1])
+def test_rotary_and_store_from_a_table_equal_their_own_angles(
+        device, rows, first, head_dim, rotary, heads, kv, gated, qk_norm, rounded, f16):
+    """Queries, keys and page bytes bit for bit as from the launches that compute
+    cosine and sine themselves: one row and four rows a wave, last waves with fewer,
+    rows across pages, partners in the same lane and in others."""
+    rng = np.random.default_rng(rows + rotary)
+    page_tokens, layer, theta, eps = 64, 1, 1.0e6, 1.0e-6
+    stride = head_dim * (2 if gated else 1)
+    value = torch.from_numpy(rng.standard_normal((rows, kv, head_dim)).astype(np.float32)
+                             ).to(device)
+    query = torch.from_numpy(rng.standard_normal((rows, heads, stride)).astype(np.float32)
+                             ).to(device)
+    key = torch.from_numpy(rng.standard_normal((rows, kv, head_dim)).astype(np.float32)
+                           ).to(device)
+    norms = [torch.from_numpy(rng.standard_normal(head_dim).astype(np.float32)).to(device)
+             if qk_norm else None for _ in range(2)]
+    per_layer = (page_tokens * kv * head_dim * 4 if f16
+                 else page_tokens * kv * 2 * (head_dim // 2 + 2))
+    count = (first + rows + page_tokens - 1) // page_tokens
+    table = torch.empty((rows, rotary // 2, 2), device=device)
+    qh.call("qllm_rope_table", qh.ptr(table), rows, rotary, first, theta, rounded, None, None)
+    results = []
+    for from_table in (False, True):
+        q, k = query.clone(), key.clone()
+        pages = torch.zeros((count, 2 * per_layer), dtype=torch.uint8, device=device)
+        pointers = torch.tensor([p.data_ptr() for p in pages], dtype=torch.int64,
+                                device=device)
+        if from_table:
+            qh.call("qllm_qkv_rope_table_batch", qh.ptr(q), stride, qh.ptr(k), qh.ptr(value),
+                    qh.ptr(norms[0]), qh.ptr(norms[1]), qh.ptr(table), qh.ptr(pointers), f16,
+                    layer, page_tokens, first, rows, heads, kv, head_dim, rotary, eps,
+                    rounded, None)
+        elif f16:
+            qh.call("qllm_qkv_rope_batch", qh.ptr(q), stride, qh.ptr(k), qh.ptr(norms[0]),
+                    qh.ptr(norms[1]), first, rows, heads, kv, head_dim, rotary, eps, theta,
+                    rounded, None)
+            qh.call("qllm_store_kv_paged_f16_batch", qh.ptr(k), qh.ptr(value),
+                    qh.ptr(pointers), layer, page_tokens, first, rows, kv, head_dim, None)
+        else:
+            qh.call("qllm_qkv_rope_cache_paged_q4h_batch", qh.ptr(q), stride, qh.ptr(k),
+                    qh.ptr(value), qh.ptr(norms[0]), qh.ptr(norms[1]), qh.ptr(pointers),
+                    layer, page_tokens, first, first, rows, heads, kv, head_dim, rotary, eps,
+                    theta, rounded, None)
+        results.append([t.cpu().numpy().view(np.uint8) for t in (q, k, pages)])
+    for old, new in zip(*results):
+        assert np.array_equal(old, new)
+    with pytest.raises(qh.QllmError, match="invalid QKV rope batch from a table"):
+        qh.call("qllm_qkv_rope_table_batch", qh.ptr(query), stride, qh.ptr(key),
+                qh.ptr(value), None, None, qh.ptr(table), None, 0, 0, 64, 0, rows, heads, kv,
+                64, 64, eps, 0, None)
