@@ -977,7 +977,7 @@ enum qllm_linear_epilogue {
    * [m][n] = activation(gate product) * up product; n < rows / 2 */
   QLLM_LINEAR_GATED = 2,
   /* output f32 [split][m][n]: the product cut along K in `splits` parts, which
-   * the norm that follows adds (qllm_stream_norm).  At most 64 batch rows. */
+   * the norm that follows adds (qllm_stream_norm). */
   QLLM_LINEAR_PARTIALS = 3
 };
 
@@ -1002,6 +1002,12 @@ typedef struct qllm_linear_segment {
  * in three bf16 parts that hold all of it. */
 int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32_t count,
                           uint32_t batch, uint32_t element, void* stream);
+/* Into how many parts a matrix alone in a launch of more than 64 rows is best cut
+ * (1 = not at all); parts x batch is at most QLLM_LINEAR_PART_ROWS where that is
+ * more than 1. */
+#define QLLM_LINEAR_PART_ROWS 8192u
+uint32_t qllm_linear_parts(uint32_t rows, uint32_t columns, uint32_t batch,
+                           uint32_t element);
 
 /* x[row] = table[token] * scale; a token outside the table gives zeros. */
 int32_t qllm_embedding_bf16_batch(const void* table_bf16, uint32_t vocabulary,

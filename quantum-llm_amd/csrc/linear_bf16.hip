@@ -28,6 +28,10 @@
 #include "common.hpp"
 #include "mixed_common.hpp"
 
+#include <algorithm>
+#include <cmath>
+#include <iterator>
+
 namespace qllm {
 namespace {
 
@@ -259,8 +263,10 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
   }
   const uint32_t index = segment_of(args, work);
   const qllm_linear_segment& s = args.segment[index];
-  const uint32_t unit = work - args.first_unit[index];
   const uint32_t n_tiles = (s.rows + 64u * NT - 1u) / (64u * NT);
+  const uint32_t parts = s.epilogue == QLLM_LINEAR_PARTIALS ? s.splits : 1u;
+  const uint32_t part = (work - args.first_unit[index]) / (n_tiles * m_tiles);
+  const uint32_t unit = (work - args.first_unit[index]) % (n_tiles * m_tiles);
   // bands of kBandTiles activation tiles, walked column by column
   const uint32_t band = unit / (kBandTiles * n_tiles);
   const uint32_t band_rows = min(kBandTiles, m_tiles - band * kBandTiles);
@@ -272,6 +278,8 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
   const uint32_t lane = threadIdx.x % kWave;
   const uint32_t chunks = s.columns / 32u;
   const uint32_t steps = s.columns / 64u;
+  const uint32_t first_step = steps * part / parts;
+  const uint32_t end_step = steps * (part + 1u) / parts;
   const uint32_t weight_tiles = s.rows / 16u;
   const uint32_t first_tile = (n_tile * 4u + wave) * NT;
 
@@ -295,35 +303,40 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
 
   f32x4 sum[NT][MT] = {};
   typename In::Raw staged[kLoads];
-  const auto store_staged = [&](uint32_t buffer) {
+  i32x4 held[2][2][NT];   // [step parity][half of 32 columns][tile]
+  const auto fetch_input = [&](uint32_t step) {
+#pragma unroll
+    for (uint32_t i = 0; i < kLoads; ++i) staged[i] = In::load(source[i] + step * 64u);
+  };
+  const auto store_input = [&](uint32_t buffer) {
 #pragma unroll
     for (uint32_t i = 0; i < kLoads; ++i) {
-      i32x4 parts[kParts];
-      In::split(staged[i], parts);
+      i32x4 split[kParts];
+      In::split(staged[i], split);
 #pragma unroll
-      for (int p = 0; p < kParts; ++p) tile[buffer][p][i * 256u + threadIdx.x] = parts[p];
+      for (int p = 0; p < kParts; ++p) tile[buffer][p][i * 256u + threadIdx.x] = split[p];
     }
   };
-  i32x4 held[2][2][NT];   // [step parity][half of 32 columns][tile]
-#pragma unroll
-  for (uint32_t i = 0; i < kLoads; ++i) staged[i] = In::load(source[i]);
-#pragma unroll
-  for (int half = 0; half < 2; ++half)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) held[0][half][t] = weights[t][half * kWave];
-  store_staged(0u);
-  __syncthreads();
-
-  const auto step_at = [&](uint32_t step, auto parity) {
-    constexpr int P = decltype(parity)::value;
-    const uint32_t next = min(step + 1u, steps - 1u);   // the last step re-reads itself
-#pragma unroll
-    for (uint32_t i = 0; i < kLoads; ++i) staged[i] = In::load(source[i] + next * 64u);
+  const auto fetch_weights = [&](auto slot, uint32_t step) {
 #pragma unroll
     for (int half = 0; half < 2; ++half)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
-        held[1 - P][half][t] = weights[t][(next * 2u + half) * kWave];
+        held[slot][half][t] = weights[t][(step * 2u + half) * kWave];
+  };
+  constexpr std::integral_constant<int, 0> even;
+  constexpr std::integral_constant<int, 1> odd;
+  // (a part without steps, of more parts than steps, loads the last one for nothing)
+  fetch_input(min(first_step, steps - 1u));
+  fetch_weights(even, min(first_step, steps - 1u));
+  store_input(0u);
+  __syncthreads();
+
+  const auto step_at = [&](uint32_t step, auto parity) {
+    constexpr int P = decltype(parity)::value;
+    const uint32_t next = min(step + 1u, end_step - 1u);   // the last one re-reads itself
+    fetch_input(next);
+    fetch_weights(std::integral_constant<int, 1 - P>{}, next);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int half = 0; half < 2; ++half)
@@ -342,34 +355,37 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
           for (int t = 0; t < NT; ++t)
             sum[t][mt] = mfma_bf16(held[P][half][t], x[mt], sum[t][mt]);
       }
-    store_staged(1 - P);
+    store_input(1 - P);
     __syncthreads();
   };
-  uint32_t step = 0;
-  for (; step + 2u <= steps; step += 2u) {
-    step_at(step, std::integral_constant<int, 0>{});
-    step_at(step + 1u, std::integral_constant<int, 1>{});
+  uint32_t step = first_step;
+  for (; step + 2u <= end_step; step += 2u) {
+    step_at(step, even);
+    step_at(step + 1u, odd);
   }
-  if (step < steps) step_at(step, std::integral_constant<int, 0>{});
+  if (step < end_step) step_at(step, even);
 
+  // What the sums are added to is fetched before anything is stored, and - where
+  // the wave's tiles are whole - all of it at once: every load after a store would
+  // wait for all before it.
   if (s.epilogue == QLLM_LINEAR_ADD) {
-    // what the sums are added to comes first: every load after a store would
-    // wait for all before it
-    const bool vectors = s.output_stride % 4u == 0u;
+    const bool whole =
+        s.output_stride % 4u == 0u && (first_tile + NT) * 16u <= s.output_columns;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const uint32_t m = min(m_tile * kRowsM + mt * 16u + lane % 16u, args.batch - 1u);
+      const float* out = static_cast<const float*>(s.output) + size_t{m} * s.output_stride +
+                         first_tile * 16u + 4u * (lane / 16u);
+      if (whole) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const uint32_t n = (first_tile + t) * 16u + 4u * (lane / 16u);
-        const float* out = static_cast<const float*>(s.output) + size_t{m} * s.output_stride;
-        if (vectors && n + 4u <= s.output_columns) {
-          sum[t][mt] += *reinterpret_cast<const f32x4*>(out + n);
-        } else {
-          for (uint32_t i = 0; i < 4u; ++i)
-            if (n + i < s.output_columns) sum[t][mt][i] += out[n + i];
-        }
+        for (int t = 0; t < NT; ++t)
+          sum[t][mt] += *reinterpret_cast<const f32x4*>(out + t * 16);
+        continue;
       }
+      for (int t = 0; t < NT; ++t)
+        for (uint32_t i = 0; i < 4u; ++i)
+          if (first_tile * 16u + 4u * (lane / 16u) + t * 16u + i < s.output_columns)
+            sum[t][mt][i] += out[t * 16 + i];
     }
   }
 #pragma unroll
@@ -403,8 +419,10 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         if (first_tile + t < weight_tiles)
-          store_four(s, static_cast<float*>(s.output), m,
-                     (first_tile + t) * 16u + 4u * (lane / 16u), sum[t][mt], false);
+          store_four(s,
+                     static_cast<float*>(s.output) +
+                         size_t{part} * args.batch * s.output_stride,
+                     m, (first_tile + t) * 16u + 4u * (lane / 16u), sum[t][mt], false);
     }
   }
 }
@@ -436,17 +454,84 @@ bool aligned16(const void* pointer) {
   return (reinterpret_cast<uintptr_t>(pointer) & 15u) == 0u;
 }
 
-template <int NT, int MT>
-uint32_t tall_units(const qllm_linear_segment& s, uint32_t batch) {
-  return (s.rows + 64u * NT - 1u) / (64u * NT) * ((batch + 16u * MT - 1u) / (16u * MT));
+uint32_t parts_of(const qllm_linear_segment& s) {
+  return s.epilogue == QLLM_LINEAR_PARTIALS ? s.splits : 1u;
+}
+
+// The forms of the tall kernel: NT weight tiles of 16 rows a wave, MT activation
+// tiles of 16 rows a workgroup.
+//
+// Which one, and how many parts of K where the caller can take parts, follows from
+// what the busiest CU will take: n = ceil(workgroups / 256) workgroups over their
+// steps of 64 columns, a step `alone` ns for n = 1 and n * `shared` where workgroups
+// hide each other's round trips, and parts written and read at 6.5 TB/s.  The
+// constants are a fit to 1150 timed launches over weights from memory (eight
+// matrices of [2048, 2048] to [24576, 4096], 66 to 3000 rows; 8 % root mean square
+// error); the layout it picks is 0.7 % slower than the best of those timed, the
+// rule before it - largest tiles that give two workgroups a CU, K never cut - 68 %:
+// [2048, 7680] 100 rows 62 -> 13 us, 1000 rows 60 -> 40, 3000 rows 117 -> 93; in 32
+// bits 100 rows 141 -> 20, 500 rows 143 -> 47.
+struct TallForm {
+  uint32_t nt, mt;
+  float alone, shared;
+};
+constexpr TallForm kTallForms[] = {
+    {2, 4, 435.f, 325.f}, {2, 8, 725.f, 515.f}, {4, 8, 1130.f, 895.f}};
+constexpr TallForm kTallFormsF32[] = {{2, 4, 1105.f, 775.f}, {4, 4, 1525.f, 1230.f}};
+
+uint64_t tall_units(const TallForm& form, uint32_t rows, uint32_t batch) {
+  return uint64_t{(rows + 64u * form.nt - 1u) / (64u * form.nt)} *
+         ((batch + 16u * form.mt - 1u) / (16u * form.mt));
+}
+
+// Time of `units` workgroups that run `steps` steps on average.
+double tall_time(const TallForm& form, double units, double steps) {
+  const double on_one = std::ceil(units / 256.0);
+  return steps * std::max<double>(form.alone, on_one * form.shared);
+}
+
+// Calls visit(form, index) for the forms of an element type.
+template <typename Visit>
+void each_form(bool f32, const Visit& visit) {
+  if (f32)
+    for (uint32_t i = 0; i < std::size(kTallFormsF32); ++i) visit(kTallFormsF32[i], i);
+  else
+    for (uint32_t i = 0; i < std::size(kTallForms); ++i) visit(kTallForms[i], i);
+}
+
+// The form for a launch whose parts are given.
+uint32_t tall_form(const LinearArgs& args, bool f32) {
+  uint32_t best = 0;
+  double least = 0.0;
+  each_form(f32, [&](const TallForm& form, uint32_t index) {
+    double units = 0.0;
+    double work = 0.0;
+    for (uint32_t i = 0; i < args.count; ++i) {
+      const auto& s = args.segment[i];
+      const double own = static_cast<double>(tall_units(form, s.rows, args.batch));
+      units += own * parts_of(s);
+      work += own * (s.columns / 64u);
+    }
+    const double time = tall_time(form, units, work / units);
+    if (index == 0u || time < least) {
+      best = index;
+      least = time;
+    }
+  });
+  return best;
 }
 
 template <bool F32, int NT, int MT>
 int32_t launch_tall(LinearArgs& args, hipStream_t stream) {
   args.first_unit[0] = 0;
   for (uint32_t i = 0; i < args.count; ++i)
-    args.first_unit[i + 1] = args.first_unit[i] + tall_units<NT, MT>(args.segment[i], args.batch);
-  linear_tall_kernel<F32, NT, MT><<<args.first_unit[args.count], 256, 0, stream>>>(args);
+    args.first_unit[i + 1] =
+        args.first_unit[i] +
+        static_cast<uint32_t>(tall_units({NT, MT, 0.f, 0.f}, args.segment[i].rows,
+                                         args.batch)) *
+            parts_of(args.segment[i]);
+  linear_tall_kernel<F32, NT, MT>
+      <<<args.first_unit[args.count], 256, 0, stream>>>(args);
   return launched("tall linear");
 }
 
@@ -454,14 +539,6 @@ template <bool F32, int MT>
 void launch_small(const LinearArgs& args, hipStream_t stream) {
   linear_small_kernel<F32, MT>
       <<<args.first_unit[args.count], kSmallWaves * kWave, 0, stream>>>(args);
-}
-
-template <int NT, int MT>
-uint32_t all_tall_units(const LinearArgs& args) {
-  uint32_t units = 0;
-  for (uint32_t i = 0; i < args.count; ++i)
-    units += tall_units<NT, MT>(args.segment[i], args.batch);
-  return units;
 }
 
 }  // namespace
@@ -522,7 +599,7 @@ extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32
         s.input_stride % 8u || !s.output_columns ||
         s.output_columns > outputs || s.output_stride < s.output_columns ||
         s.epilogue > QLLM_LINEAR_PARTIALS || s.activation > QLLM_ACTIVATION_SILU ||
-        (partials && (!s.splits || s.splits > 16u || batch > 64u)) ||
+        (partials && (!s.splits || s.splits > 16u)) ||
         !aligned16(s.weights) || !aligned16(s.input) || !aligned16(s.output))
       return fail(QLLM_INVALID_ARGUMENT, "invalid linear segment");
     args.segment[i] = s;
@@ -544,12 +621,31 @@ extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32
       f32 ? launch_small<true, 4>(args, hip_stream) : launch_small<false, 4>(args, hip_stream);
     return launched("small-batch linear");
   }
-  // F32: three parts of 64 activation rows fit a workgroup's LDS twice over
+  const uint32_t form = tall_form(args, f32);
   if (f32)
-    return all_tall_units<4, 4>(args) >= 384u ? launch_tall<true, 4, 4>(args, hip_stream)
-                                              : launch_tall<true, 2, 4>(args, hip_stream);
-  // the largest tiles that still give every CU two workgroups to hold
-  if (all_tall_units<4, 8>(args) >= 512u) return launch_tall<false, 4, 8>(args, hip_stream);
-  if (all_tall_units<2, 8>(args) >= 384u) return launch_tall<false, 2, 8>(args, hip_stream);
-  return launch_tall<false, 2, 4>(args, hip_stream);
+    return form ? launch_tall<true, 4, 4>(args, hip_stream)
+                : launch_tall<true, 2, 4>(args, hip_stream);
+  if (form == 2u) return launch_tall<false, 4, 8>(args, hip_stream);
+  return form ? launch_tall<false, 2, 8>(args, hip_stream)
+              : launch_tall<false, 2, 4>(args, hip_stream);
+}
+
+extern "C" uint32_t qllm_linear_parts(uint32_t rows, uint32_t columns, uint32_t batch,
+                                      uint32_t element) {
+  const uint32_t steps = columns / 64u;
+  uint32_t best = 1u;
+  double least = 0.0;
+  each_form(element == QLLM_ELEMENT_F32, [&](const TallForm& form, uint32_t) {
+    const double units = static_cast<double>(tall_units(form, rows, batch));
+    for (uint32_t parts = 1; parts <= 16u && parts <= std::max(steps, 1u); ++parts) {
+      if (parts > 1u && uint64_t{parts} * batch > QLLM_LINEAR_PART_ROWS) break;
+      const double time = tall_time(form, units * parts, (steps + parts - 1u) / parts) +
+                          parts * 4.0 * batch * rows / 6500.0;
+      if (least == 0.0 || time < least) {
+        best = parts;
+        least = time;
+      }
+    }
+  });
+  return best;
 }

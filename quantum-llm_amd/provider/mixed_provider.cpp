@@ -772,7 +772,10 @@ void Mi355MixedProvider::ensure_workspace(std::uint32_t rows, std::uint32_t last
     const Block& block = *item;
     partial_rows = std::max<std::size_t>(
         partial_rows, std::max(block.splits, block.down_splits) * kSmallBatch);
-    if (block.sandwich) partial_rows = std::max<std::size_t>(partial_rows, size);
+    partial_rows = std::max<std::size_t>(
+        partial_rows,
+        std::max<std::size_t>(size, std::min<std::size_t>(std::size_t{16U} * size,
+                                                          QLLM_LINEAR_PART_ROWS)));
     if (block.kind == Kind::attention) {
       const auto& a = block.attention;
       query = std::max(query, std::size_t{a.query_heads} * a.key_stride);
@@ -1069,8 +1072,16 @@ qllm_stream_norm_launch Mi355MixedProvider::stream_norm(std::uint32_t rows, floa
   return norm;
 }
 
+// Parts of K of a projection onto the stream, which the next norm adds.
+std::uint32_t Mi355MixedProvider::parts_for(const Matrix& matrix, std::uint32_t few_rows,
+                                            std::uint32_t rows) const {
+  return rows <= kSmallBatch ? few_rows
+                             : qllm_linear_parts(matrix.rows, matrix.columns, rows,
+                                                 g_.element);
+}
+
 // Mixer and feed-forward one after the other; each leaves its output as partial
-// sums (a single one, from a tall batch) that the next norm takes.
+// sums that the next norm takes.
 void Mi355MixedProvider::enqueue_sandwich(Block& block, std::uint32_t rows,
                                           std::uint32_t last_position) {
   const auto normed = [&](const DeviceBuffer& weight) {
@@ -1082,7 +1093,7 @@ void Mi355MixedProvider::enqueue_sandwich(Block& block, std::uint32_t rows,
   };
   const auto project = [&](const Matrix& matrix, std::uint32_t splits,
                            const DeviceBuffer& post_norm) {
-    const bool split = rows <= kSmallBatch;
+    const std::uint32_t parts = parts_for(matrix, splits, rows);
     qllm_linear_segment s{};
     s.weights = matrix.data.get();
     s.input = joined_.get();
@@ -1092,10 +1103,10 @@ void Mi355MixedProvider::enqueue_sandwich(Block& block, std::uint32_t rows,
     s.input_stride = matrix.columns;
     s.output_stride = round_up(g_.hidden, 4U);
     s.output_columns = g_.hidden;
-    s.epilogue = split ? QLLM_LINEAR_PARTIALS : QLLM_LINEAR_STORE;
-    s.splits = split ? splits : 0U;
+    s.epilogue = QLLM_LINEAR_PARTIALS;
+    s.splits = parts;
     status_check(qllm_linear_batch(&s, 1U, rows, g_.element, stream_));
-    pending_partials_ = split ? splits : 1U;
+    pending_partials_ = parts;
     pending_branch_ = {post_norm.as<float>(), block.residual_scale, block.epsilon};
   };
   qllm_linear_segment s{};
@@ -1201,12 +1212,13 @@ void Mi355MixedProvider::enqueue_block(Block& block, std::uint32_t rows,
   s.columns = block.output.columns;
   s.input_stride = block.output.columns;
   s.output_columns = g_.hidden;
-  if (g_.element == QLLM_ELEMENT_BF16 && rows <= kSmallBatch) {
+  if (const auto parts = parts_for(block.output, block.splits, rows);
+      rows <= kSmallBatch || parts > 1U) {
     s.output = partials_.get();
     s.output_stride = round_up(g_.hidden, 4U);
     s.epilogue = QLLM_LINEAR_PARTIALS;
-    s.splits = block.splits;
-    pending_partials_ = block.splits;
+    s.splits = parts;
+    pending_partials_ = parts;
   } else {
     s.output = hidden_[stream_index_].get();
     s.output_stride = g_.hidden;

@@ -155,6 +155,8 @@ class Mi355MixedProvider final : public DecoderProvider {
   void enqueue_sandwich(Block& block, std::uint32_t rows, std::uint32_t last_position);
   void enqueue_mixer(Block& block, std::uint32_t rows, std::uint32_t last_position);
   // Norm launch over the stream with what partial sums are pending.
+  [[nodiscard]] std::uint32_t parts_for(const Matrix& matrix, std::uint32_t few_rows,
+                                        std::uint32_t rows) const;
   [[nodiscard]] qllm_stream_norm_launch stream_norm(std::uint32_t rows, float epsilon);
   void enqueue_latent(Block& block, std::uint32_t rows, std::uint32_t last_position);
   void enqueue_attention(Block& block, std::uint32_t rows, std::uint32_t last_position);

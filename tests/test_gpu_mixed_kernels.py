@@ -118,6 +118,31 @@ def test_linear_partials_and_side_by_side_columns(device, element, splits):
     close(out.sum(0)[:, :50], want, F32)
 
 
+@pytest.mark.parametrize("element", [F32, BF16])
+@pytest.mark.parametrize("rows,columns,batch", [
+    (50, 192, 65), (300, 512, 129), (33, 64, 200), (1100, 1984, 67)])
+def test_linear_partials_of_tall_batches(device, element, rows, columns, batch):
+    """Parts of every count of a batch of more than 64 rows, among them more parts
+    than steps of K, uneven shares and ragged tiles; the count the library advises."""
+    rng = np.random.default_rng(rows)
+    matrix = mm.bf16(rng.standard_normal((rows, columns)) / np.sqrt(columns))
+    x = mm.bf16(rng.standard_normal((batch, columns)))
+    weights = packed(device, [(matrix, 0, 1, 0)], rows, columns)
+    d_x = padded_input(device, x, columns, element)
+    stride = padded(rows, 4) + 4
+    want = x.astype(np.float64) @ matrix.T.astype(np.float64)
+    advised = qh.call("qllm_linear_parts", padded(rows, 16), columns, batch, element)
+    assert 1 <= advised <= 16 and (advised == 1 or advised * batch <= 8192)
+    for parts in sorted({1, 2, 3, 7, 16, advised}):
+        out = torch.full((parts, batch, stride), 7.0, device=device)
+        segment = qh.LinearSegment(qh.ptr(weights), qh.ptr(d_x), qh.ptr(out),
+                                   padded(rows, 16), columns, columns, stride, rows,
+                                   qh.LINEAR_PARTIALS, 0, parts)
+        qh.call("qllm_linear_batch", ctypes.byref(segment), 1, batch, element, None)
+        close(out[:, :, :rows].sum(0), want, F32)
+        assert torch.all(out[:, :, rows:] == 7.0)
+
+
 def test_linear_tall_tiles_of_all_sizes(device):
     rng = np.random.default_rng(3)
     for rows, columns, batch in ((2100, 128, 700), (4096, 64, 1030), (300, 320, 129)):
