@@ -35,6 +35,7 @@
 //    2^-11 in that weight).  Checkpoint scales lie well inside.
 #include "common.hpp"
 
+#include <iterator>
 #include <type_traits>
 
 namespace qllm {
@@ -469,12 +470,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_tall_kernel(
                                               tile_count, acc);
 }
 
-// Short batches: up to 64 rows a workgroup (16 MT), 128 weight rows (SWIGLU: of
-// each of the two matrices).  Here the weights' way from memory is what there is
+// Short batches: 16, 32, 48 or 64 rows a workgroup (16 MT), 128 weight rows (SWIGLU:
+// of each of the two matrices).  Here the weights' way from memory is what there is
 // to hide, not the matrix cores' time: a wave keeps its weights of the next four
 // chunks on their way in registers (with the one of fp4_gemm_tall_kernel a step
 // waits out most of a memory round trip), the activations of the next two steps
-// likewise, and a step covers 4 / MT chunks so that its barrier costs the same
+// likewise, and a step covers so many chunks that its barrier costs about the same
 // whatever the height.
 template <int SCHEME, int MT, int T, bool SWIGLU>
 __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
@@ -484,7 +485,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
   constexpr bool F16 = SCHEME == kSchemeF16;
   static_assert(!SWIGLU || T == 2);
   constexpr uint32_t kAhead = 4;                    // chunks of weights in flight
-  constexpr uint32_t kSpan = 4 / MT;                // chunks per step
+  constexpr uint32_t kSpan = MT == 3 ? 2 : 4 / MT;  // chunks per step
   constexpr uint32_t kRow = kSpan * kChunk * 2u + 16u;
   constexpr uint32_t kPieces = 16u * MT * kSpan * 8u / (kWaves * 64u);
   static_assert(kPieces * kWaves * 64u == 16u * MT * kSpan * 8u);
@@ -733,8 +734,8 @@ bool tall_matrix_ok(const qllm_fp4_matrix* m) {
          (m->tile_rows == 0u || m->tile_rows == kTileRows);
 }
 
-// How a launch is laid out: 16 `height` rows of activations per workgroup and
-// `splits` parts of K.
+// How a launch is laid out: 16 `height` rows of activations per workgroup (height 1,
+// 2, 3, 4 or 8) and `splits` parts of K.
 //
 // Chosen by what the busiest CU will take.  With W workgroups per part it runs
 // n = ceil(W splits / 256) of them, each over ceil(chunks / splits) chunks; a
@@ -760,12 +761,14 @@ constexpr size_t kPartsBytes = size_t{128} << 20;
 struct ChunkCost {
   float alone, shared;   // ns
 };
-// [scheme][SwiGLU][log2 height]
-constexpr ChunkCost kChunkCost[2][2][4] = {
-    {{{160.f, 150.f}, {195.f, 180.f}, {365.f, 250.f}, {1160.f, 780.f}},
-     {{250.f, 325.f}, {335.f, 345.f}, {605.f, 420.f}, {1215.f, 780.f}}},
-    {{{220.f, 230.f}, {300.f, 280.f}, {545.f, 390.f}, {1690.f, 1265.f}},
-     {{380.f, 440.f}, {515.f, 500.f}, {985.f, 715.f}, {1710.f, 1230.f}}}};
+constexpr uint32_t kHeights[] = {1u, 2u, 3u, 4u, 8u};
+// [scheme][SwiGLU][height]; 48 rows, which joined later, at the share of the 64-row
+// workgroup's cost that 48 rows of the 27B widths took (86 %)
+constexpr ChunkCost kChunkCost[2][2][5] = {
+    {{{160.f, 150.f}, {195.f, 180.f}, {315.f, 215.f}, {365.f, 250.f}, {1160.f, 780.f}},
+     {{250.f, 325.f}, {335.f, 345.f}, {520.f, 360.f}, {605.f, 420.f}, {1215.f, 780.f}}},
+    {{{220.f, 230.f}, {300.f, 280.f}, {470.f, 335.f}, {545.f, 390.f}, {1690.f, 1265.f}},
+     {{380.f, 440.f}, {515.f, 500.f}, {845.f, 615.f}, {985.f, 715.f}, {1710.f, 1230.f}}}};
 
 uint32_t weight_rows_of(uint32_t height, bool swiglu) {
   return (height == 8u && !swiglu ? kTilesN : kWaves) * kTileRows;
@@ -799,13 +802,13 @@ TallPlan plan_tall(uint32_t rows, uint32_t padded_columns, uint32_t batch,
                                                       : kMaximumParts;
   TallPlan best{};
   double least = 0.0;
-  for (uint32_t log_height = 0; log_height < 4u; ++log_height) {
-    const uint32_t height = 1u << log_height;
-    // the lowest that holds the batch, or one of the two highest
-    if (height < 4u ? batch > 16u * height || (height == 2u && batch <= 16u)
-                    : batch <= 8u * height)
-      continue;
-    const ChunkCost cost = kChunkCost[scheme][swiglu][log_height];
+  for (uint32_t index = 0; index < std::size(kHeights); ++index) {
+    const uint32_t height = kHeights[index];
+    // one or two tiles of rows where they hold the batch, else the higher ones, and
+    // none of which a lower one would hold the batch
+    if (height < 3u ? batch > 16u * height : batch <= 32u) continue;
+    if (index && batch <= 16u * kHeights[index - 1u]) continue;
+    const ChunkCost cost = kChunkCost[scheme][swiglu][index];
     const uint32_t workgroups = workgroups_of(rows, batch, height, swiglu);
     for (uint32_t splits = first; splits <= last; ++splits) {
       const size_t bytes = parts_bytes(rows, batch, splits, swiglu);
@@ -842,6 +845,12 @@ void start_tall(const TallArgs& args, uint32_t height, bool swiglu, uint32_t gri
         fp4_gemm_short_kernel<SCHEME, 2, 2, true><<<grid, kThreads, 0, stream>>>(args);
       else
         fp4_gemm_short_kernel<SCHEME, 2, 1, false><<<grid, kThreads, 0, stream>>>(args);
+      break;
+    case 3:
+      if (swiglu)
+        fp4_gemm_short_kernel<SCHEME, 3, 2, true><<<grid, kThreads, 0, stream>>>(args);
+      else
+        fp4_gemm_short_kernel<SCHEME, 3, 1, false><<<grid, kThreads, 0, stream>>>(args);
       break;
     case 4:
       if (swiglu)

@@ -177,7 +177,8 @@ def test_tall_gemm_rejects_row_major(device):
 
 @pytest.mark.parametrize("rows,padded,batch", [
     (96, 64, 1), (132, 576, 15), (4, 1024, 16), (260, 832, 17), (1056, 192, 33),
-    (640, 1088, 64), (388, 1024, 65), (2048, 5120, 48), (1024, 1216, 300)])
+    (640, 1088, 64), (388, 1024, 65), (2048, 5120, 48), (1024, 1216, 300),
+    (160, 1024, 49), (2048, 2112, 97)])
 @pytest.mark.parametrize("scheme", [ol.SCALE_UE8M0_BLOCK32, ol.SCALE_F16_BLOCK16])
 def test_launches_cut_along_k_match_the_oracle(device, scheme, rows, padded, batch):
     """Workgroup heights at their edges (1, 16 / 17, 32 / 33, 64 / 65 rows), parts
