@@ -325,7 +325,7 @@ __global__ __launch_bounds__(256) void general_attention_kernel(AttentionArgs ar
 // Scores of the workgroup's tiles for all heads, 32 lanes per (head, tile), and
 // the heads' maxima and sums over those tiles.
 template <typename T>
-__global__ __launch_bounds__(256) void general_scores_kernel(AttentionArgs args) {
+__global__ __launch_bounds__(512) void general_scores_kernel(AttentionArgs args) {
   extern __shared__ float shared[];
   const Attention& a = args.attention;
   const uint32_t heads = a.query_heads;
@@ -1194,6 +1194,17 @@ size_t general_bytes(const Attention& a) {
   return size_t{a.query_heads} * (a.dim + 2u * kTileKeys + a.vdim + 2u) * 4u;
 }
 
+// The general form's workgroups take a tile each where there is room: their scores
+// and values are plain multiply-adds, 4 us a tile and head group (16 heads, 340 keys:
+// scores 25 us two tiles at a time, values 23 four at a time).
+uint32_t general_score_splits_for(uint32_t tiles) {
+  return tiles < kMaximumScoreSplits ? tiles : kMaximumScoreSplits;
+}
+
+uint32_t general_value_splits_for(uint32_t tiles) {
+  return tiles < kMaximumValueSplits ? tiles : kMaximumValueSplits;
+}
+
 size_t general_scores_bytes(const Attention& a) {
   return size_t{a.query_heads} * (a.dim + 2u) * 4u;
 }
@@ -1204,12 +1215,12 @@ size_t general_values_bytes(const Attention& a) {
 }
 
 // The parts of a split launch's workspace.
-void place_splits(AttentionArgs& args) {
+void place_splits(AttentionArgs& args, bool general) {
   const Attention& a = args.attention;
   const uint32_t tiles = maximum_tiles(a, args.launch.maximum_position);
   args.capacity = tiles * kTileKeys;
-  args.score_splits = score_splits_for(tiles);
-  args.value_splits = value_splits_for(tiles);
+  args.score_splits = general ? general_score_splits_for(tiles) : score_splits_for(tiles);
+  args.value_splits = general ? general_value_splits_for(tiles) : value_splits_for(tiles);
   args.scores = static_cast<float*>(args.launch.workspace);
   args.maxima = args.scores + size_t{args.launch.rows} * a.query_heads * args.capacity;
   args.partials =
@@ -1221,7 +1232,7 @@ void launch_general_splits(const AttentionArgs& args, hipStream_t stream) {
   const Attention& a = args.attention;
   const uint32_t rows = args.launch.rows;
   general_scores_kernel<T>
-      <<<dim3(args.score_splits, rows), 256, general_scores_bytes(a), stream>>>(args);
+      <<<dim3(args.score_splits, rows), 512, general_scores_bytes(a), stream>>>(args);
   general_values_kernel<T><<<dim3(args.value_splits, a.kv_heads, rows), 256,
                              general_values_bytes(a), stream>>>(args);
   split_combine_kernel<T><<<dim3(a.query_heads, rows), 64, 0, stream>>>(args);
@@ -1288,8 +1299,9 @@ extern "C" size_t qllm_windowed_attention_workspace_bytes(
   const uint32_t tiles = maximum_tiles(*attention, maximum_position);
   const size_t heads = attention->query_heads;
   const size_t split = kSplitRows * heads * 4u *
-                       (size_t{tiles} * kTileKeys + size_t{score_splits_for(tiles)} * 2u +
-                        size_t{value_splits_for(tiles)} * attention->vdim);
+                       (size_t{tiles} * kTileKeys +
+                        size_t{general_score_splits_for(tiles)} * 2u +
+                        size_t{general_value_splits_for(tiles)} * attention->vdim);
   const size_t prompt = size_t{rows} * heads * 4u;   // denominators
   return split > prompt ? split : prompt;
 }
@@ -1317,7 +1329,7 @@ extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* a
         launch->workspace_bytes >= qllm_windowed_attention_workspace_bytes(
                                        attention, launch->rows, launch->maximum_position) &&
         general_scores_bytes(a) <= 65536u && general_values_bytes(a) <= 65536u) {
-      place_splits(args);
+      place_splits(args, true);
       if (a.element == QLLM_ELEMENT_F32)
         launch_general_splits<float>(args, hip_stream);
       else
@@ -1359,7 +1371,7 @@ extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* a
           qllm_windowed_attention_workspace_bytes(attention, launch->rows,
                                                   launch->maximum_position))
     return fail(QLLM_INVALID_ARGUMENT, "windowed attention workspace is too small");
-  place_splits(args);
+  place_splits(args, false);
   const dim3 score_grid(args.score_splits, a.kv_heads, launch->rows);
   if (a.key_stride == 64u)
     split_scores_kernel<2><<<score_grid, 256, 0, hip_stream>>>(args);
