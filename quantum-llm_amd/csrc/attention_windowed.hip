@@ -15,8 +15,8 @@
 //    and low halves (together 16 bits of mantissa), lets the matrix cores mix
 //    them over heads - the mix matrix is bf16 as stored, so both products are
 //    exact and added in F32 - and multiplies the mixed weights with the values.
-//  * general: any size, plain F32 arithmetic on bf16 or F32 elements.  A few rows
-//    take the split form's three launches; more, a workgroup per row.
+//  * general: any size, F32 arithmetic on bf16 or F32 elements.  A few rows take
+//    the split form's three launches; more, the 32-bit matrix instructions.
 //
 // Keys lie in fragments of 16 tokens x 32 dimensions and values, transposed, in
 // fragments of 16 dimensions x 32 tokens: every operand load of a wave is one
@@ -222,105 +222,273 @@ __device__ __forceinline__ float value_product(const float* weights, const T* va
   return total;
 }
 
+// Four consecutive elements as F32; the address is aligned to an element only.
+__device__ __forceinline__ f32x4 four_elements(const float* from) {
+  struct __attribute__((packed, aligned(4))) Raw { f32x4 value; };
+  return reinterpret_cast<const Raw*>(from)->value;
+}
+__device__ __forceinline__ f32x4 four_elements(const uint16_t* from) {
+  struct __attribute__((packed, aligned(2))) Raw { uint16_t value[4]; };
+  const Raw raw = *reinterpret_cast<const Raw*>(from);
+  return f32x4{load_element(raw.value), load_element(raw.value + 1),
+               load_element(raw.value + 2), load_element(raw.value + 3)};
+}
+
+// sum += a b, 16 x 16 outputs over 4 x 4 terms of 32 bits: a lane holds term
+// 4 (lane / 16) + i of row (column) lane % 16 in a[i] (b[i]).
+__device__ __forceinline__ void add_products(const f32x4& a, const f32x4& b, f32x4& sum) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], sum, 0, 0, 0);
+}
+
+// Head dimensions of any number in elements of either type, every product and sum
+// in F32 on the matrix cores.  A matrix operand's 16 columns are the query heads
+// of one key/value head times the workgroup's rows.  With mixed heads a workgroup
+// owns all heads of its rows, without it those of one operand.
+//
+// A first walk over the visible tiles takes each head's maximum and sum, the
+// waves' units being (operand, tile); the second takes `tiles` tiles a round:
+// their scores again, normalised into LDS, the mix over heads, and the mixed
+// weights times the values, units being (operand, 16 value dimensions).
+//
+// As plain multiply-adds, a workgroup per row, this was bound by the lines that
+// its loads touch (64 a load of keys, each query head its own): 350 us for rows 0
+// .. 332 of 16 heads on 4, 128 dimensions, and 1740 us for rows 0 .. 999; now 91
+// and 279 us, of which the matrix instructions are about 30 and 80.
+struct GeneralArgs {
+  AttentionArgs base;
+  uint32_t rows;    // of a workgroup
+  uint32_t tiles;   // of a round
+  uint32_t pitch;   // floats from one head's weights to the next one's
+};
+
 template <typename T>
-__global__ __launch_bounds__(256) void general_attention_kernel(AttentionArgs args) {
-  extern __shared__ float shared[];
-  const Attention& a = args.attention;
-  const auto& run = args.launch;
+__global__ __launch_bounds__(1024) void general_attention_kernel(GeneralArgs args) {
+  extern __shared__ __attribute__((aligned(16))) float shared[];
+  const Attention& a = args.base.attention;
+  const auto& run = args.base.launch;
   const uint32_t heads = a.query_heads;
   const uint32_t group = heads / a.kv_heads;
-  float* q = shared;                                   // [heads][dim]
-  float* weights = q + heads * a.dim;                  // [heads][32]
-  float* mixed = weights + heads * kTileKeys;          // [heads][32]
-  float* out = mixed + heads * kTileKeys;              // [heads][vdim]
-  float* maximum = out + heads * a.vdim;               // [heads]
-  float* sum = maximum + heads;                        // [heads]
-  const uint32_t row = blockIdx.x;
-  const uint32_t position = a.step[kStepPosition] + row;
-  const TileRange range = tiles_for(a, position, position);
+  const uint32_t per = min(group, 16u);                // heads of an operand
+  const uint32_t operands_per_kv = (group + 15u) / 16u;
+  const uint32_t operands = a.head_mix ? a.kv_heads * operands_per_kv : 1u;
+  const uint32_t first_operand = a.head_mix ? 0u : blockIdx.y;
+  const uint32_t first_head =
+      a.head_mix ? 0u
+                 : first_operand / operands_per_kv * group + first_operand % operands_per_kv * 16u;
+  const uint32_t span = a.head_mix ? heads : min(16u, group - first_operand % operands_per_kv * 16u);
+  const uint32_t row0 = (gridDim.x - 1u - blockIdx.x) * args.rows;   // long rows first
+  const uint32_t here = min(args.rows, run.rows - row0);
+  const uint32_t position0 = a.step[kStepPosition] + row0;
+  const TileRange range = tiles_for(a, position0, position0 + here - 1u);
+  const uint32_t wave = threadIdx.x / kWave;
+  const uint32_t waves = blockDim.x / kWave;
+  const uint32_t column = threadIdx.x % 16u;
+  const uint32_t quarter = threadIdx.x % kWave / 16u;
 
-  const T* query = static_cast<const T*>(run.query) + size_t{row} * heads * a.key_stride;
-  for (uint32_t i = threadIdx.x; i < heads * a.dim; i += blockDim.x)
-    q[i] = load_element(query + size_t{i / a.dim} * a.key_stride + i % a.dim);
-  for (uint32_t i = threadIdx.x; i < heads * a.vdim; i += blockDim.x) out[i] = 0.0f;
-  for (uint32_t h = threadIdx.x; h < heads; h += blockDim.x) {
-    maximum[h] = -INFINITY;
-    sum[h] = 0.0f;
+  const uint32_t lines = args.rows * span;             // (row, head) pairs
+  float* const out = shared;                           // [lines][vdim]
+  float* const maximum = out + lines * a.vdim;         // [lines]
+  float* const sum = maximum + lines;                  // [lines]
+  // (16-byte aligned: the sizes in front are rounded up)
+  float* const weights = shared + ((lines * (a.vdim + 2u) + 3u) & ~3u);   // [lines][pitch]
+  float* const mixed = a.head_mix ? weights + lines * args.pitch : weights;
+  float* const found = weights;                        // [part][operand][16][2]
+
+  struct Column {
+    uint32_t row, head, line;
+    bool used;
+  };
+  // the row, head and line that a column of an operand stands for
+  const auto column_of = [&](uint32_t operand, uint32_t index) {
+    const uint32_t kv = operand / operands_per_kv;
+    const uint32_t base = operand % operands_per_kv * 16u;
+    const uint32_t in_group = base + index % per;
+    Column c{index / per, 0u, 0u, index / per < here && in_group < group};
+    if (!c.used) c.row = 0u;
+    c.head = kv * group + (c.used ? in_group : base);
+    c.line = c.row * span + c.head - first_head;
+    return c;
+  };
+  // s[half][i]: key 16 half + 4 quarter + i of the tile with column `c`
+  const auto scores = [&](uint32_t operand, const Column& c, uint32_t tile, f32x4 (&s)[2]) {
+    const uint32_t key0 = tile * kTileKeys;
+    const T* const keys = page_of<const T>(a, key0) +
+                          key_block(a, operand / operands_per_kv, key0 % a.page_tokens) +
+                          column * 32u + 4u * quarter;
+    const T* const query = static_cast<const T*>(run.query) +
+                           (size_t{row0 + c.row} * heads + c.head) * a.key_stride + 4u * quarter;
+    s[0] = s[1] = f32x4{};
+    const auto step = [&](uint32_t d) {
+      const f32x4 q = four_elements(query + d);
+#pragma unroll
+      for (uint32_t half = 0; half < 2u; ++half)
+        add_products(four_elements(keys + size_t{half} * 16u * a.key_stride + d / 32u * 512u +
+                                   d % 32u), q, s[half]);
+    };
+    uint32_t d = 0;
+    for (; d + 64u <= a.dim; d += 64u) {
+#pragma unroll
+      for (uint32_t i = 0; i < 64u; i += 16u) step(d + i);
+    }
+    for (; d + 16u <= a.dim; d += 16u) step(d);
+    if (d < a.dim) {   // what lies past the last dimension may be anything
+      f32x4 q = four_elements(query + d);
+#pragma unroll
+      for (uint32_t half = 0; half < 2u; ++half) {
+        f32x4 k = four_elements(keys + size_t{half} * 16u * a.key_stride + d / 32u * 512u +
+                                d % 32u);
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i)
+          if (d + 4u * quarter + i >= a.dim) q[i] = k[i] = 0.0f;
+        add_products(k, q, s[half]);
+      }
+    }
+#pragma unroll
+    for (uint32_t half = 0; half < 2u; ++half)
+#pragma unroll
+      for (uint32_t i = 0; i < 4u; ++i)
+        s[half][i] = visible(a, position0 + c.row, key0 + half * 16u + 4u * quarter + i)
+                         ? s[half][i] * a.scale
+                         : -INFINITY;
+  };
+  const auto merge = [](float& m, float& t, float other_m, float other_t) {
+    const float fresh = fmaxf(m, other_m);
+    if (fresh == -INFINITY) return;
+    t = t * expf(m - fresh) + other_t * expf(other_m - fresh);
+    m = fresh;
+  };
+
+  const uint32_t at_once = min(operands, waves);
+  const uint32_t parts = waves / at_once;   // waves of an operand
+  const uint32_t part = wave / at_once;
+  if (part < parts) {
+    for (uint32_t operand = wave % at_once; operand < operands; operand += at_once) {
+      const Column c = column_of(first_operand + operand, column);
+      float m = -INFINITY;
+      float t = 0.0f;
+      for (uint32_t ordinal = part; ordinal < range.count; ordinal += parts) {
+        f32x4 s[2];
+        scores(first_operand + operand, c, range.tile(ordinal), s);
+        float top = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) top = fmaxf(top, s[i / 4][i % 4]);
+        if (top == -INFINITY) continue;
+        const float fresh = fmaxf(m, top);
+        t *= expf(m - fresh);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) t += expf(s[i / 4][i % 4] - fresh);
+        m = fresh;
+      }
+      merge(m, t, __shfl_xor(m, 16, kWave), __shfl_xor(t, 16, kWave));
+      merge(m, t, __shfl_xor(m, 32, kWave), __shfl_xor(t, 32, kWave));
+      if (quarter == 0u) {
+        float* const pair = found + ((part * operands + operand) * 16u + column) * 2u;
+        pair[0] = m;
+        pair[1] = t;
+      }
+    }
+  }
+  for (uint32_t i = threadIdx.x; i < lines * a.vdim; i += blockDim.x) out[i] = 0.0f;
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < operands * 16u; i += blockDim.x) {
+    const Column c = column_of(first_operand + i / 16u, i % 16u);
+    float m = -INFINITY;
+    float t = 0.0f;
+    for (uint32_t p = 0; p < parts; ++p) {
+      const float* const pair = found + (p * operands * 16u + i) * 2u;
+      merge(m, t, pair[0], pair[1]);
+    }
+    if (c.used) {
+      maximum[c.line] = m;
+      sum[c.line] = t;
+    }
   }
   __syncthreads();
 
-  const auto score_tile = [&](uint32_t tile, const T* page) {
-    for (uint32_t i = threadIdx.x; i < heads * kTileKeys; i += blockDim.x) {
-      const uint32_t head = i / kTileKeys;
-      const uint32_t key = tile * kTileKeys + i % kTileKeys;
-      float score = -INFINITY;
-      if (visible(a, position, key)) {
-        const uint32_t slot = key % a.page_tokens;
-        const T* k = page + key_block(a, head / group, slot) + slot % 16u * 32u;
-        score = key_product(q + head * a.dim, k, a.dim) * a.scale;
-      }
-      weights[i] = score;
-    }
-    __syncthreads();
-  };
-
-  for (uint32_t ordinal = 0; ordinal < range.count; ++ordinal) {
-    const uint32_t tile = range.tile(ordinal);
-    score_tile(tile, page_of<const T>(a, tile * kTileKeys));
-    for (uint32_t h = threadIdx.x; h < heads; h += blockDim.x) {
-      float m = maximum[h];
-      for (uint32_t j = 0; j < kTileKeys; ++j) m = fmaxf(m, weights[h * kTileKeys + j]);
-      if (m > -INFINITY) {
-        float s = sum[h] * expf(maximum[h] - m);
-        for (uint32_t j = 0; j < kTileKeys; ++j) s += expf(weights[h * kTileKeys + j] - m);
-        sum[h] = s;
-        maximum[h] = m;
+  for (uint32_t ordinal = 0; ordinal < range.count; ordinal += args.tiles) {
+    const uint32_t tiles = min(args.tiles, range.count - ordinal);
+    for (uint32_t unit = wave; unit < operands * tiles; unit += waves) {
+      const uint32_t operand = first_operand + unit % operands;
+      const uint32_t tile = unit / operands;
+      const Column c = column_of(operand, column);
+      f32x4 s[2];
+      scores(operand, c, range.tile(ordinal + tile), s);
+      if (!c.used) continue;
+      float* const line = weights + c.line * args.pitch + tile * kTileKeys + 4u * quarter;
+      const float top = maximum[c.line];
+      const float total = sum[c.line];
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[half][i] = expf(s[half][i] - top) / total;
+        *reinterpret_cast<f32x4*>(line + half * 16) = s[half];
       }
     }
     __syncthreads();
+    if (a.head_mix) {
+      const uint32_t fours = tiles * (kTileKeys / 4u);
+      for (uint32_t i = threadIdx.x; i < here * heads * fours; i += blockDim.x) {
+        const uint32_t line = i / fours;
+        const uint32_t at = i % fours * 4u;
+        const float* const mix = a.head_mix + size_t{line % heads} * heads;
+        const float* from = weights + line / heads * heads * args.pitch + at;
+        f32x4 total = {};
+#pragma unroll 4
+        for (uint32_t g = 0; g < heads; ++g, from += args.pitch) {
+          const f32x4 weight = *reinterpret_cast<const f32x4*>(from);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) total[j] = fmaf(mix[g], weight[j], total[j]);
+        }
+        *reinterpret_cast<f32x4*>(mixed + line * args.pitch + at) = total;
+      }
+      __syncthreads();
+    }
+    const uint32_t pieces = (a.vdim + 15u) / 16u;
+    for (uint32_t unit = wave; unit < operands * pieces; unit += waves) {
+      const uint32_t operand = first_operand + unit / pieces;
+      const uint32_t d = unit % pieces * 16u + column;
+      const uint32_t kv = operand / operands_per_kv;
+      const float* const line =
+          mixed + column_of(operand, column).line * args.pitch + 4u * quarter;
+      f32x4 total = {};
+      for (uint32_t tile = 0; tile < tiles; ++tile) {
+        const uint32_t key0 = range.tile(ordinal + tile) * kTileKeys;
+        // slots past a row's position may hold anything finite: their weight is zero
+        const T* const values = page_of<const T>(a, key0) +
+                                value_block(a, kv, key0 % a.page_tokens) + d * 32u +
+                                4u * quarter;
+#pragma unroll
+        for (uint32_t half = 0; half < 2u; ++half)
+          add_products(*reinterpret_cast<const f32x4*>(line + tile * kTileKeys + half * 16u),
+                       four_elements(values + half * 16u), total);
+      }
+      if (d >= a.vdim) continue;
+#pragma unroll
+      for (uint32_t i = 0; i < 4u; ++i) {
+        const Column c = column_of(operand, 4u * quarter + i);
+        if (c.used) out[c.line * a.vdim + d] += total[i];
+      }
+    }
+    if (!a.head_mix) __syncthreads();   // with a mix the next two barriers are enough
   }
-  for (uint32_t ordinal = 0; ordinal < range.count; ++ordinal) {
-    const uint32_t tile = range.tile(ordinal);
-    const T* page = page_of<const T>(a, tile * kTileKeys);
-    score_tile(tile, page);
-    for (uint32_t i = threadIdx.x; i < heads * kTileKeys; i += blockDim.x) {
-      const uint32_t h = i / kTileKeys;
-      weights[i] = expf(weights[i] - maximum[h]) / sum[h];
-    }
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < heads * kTileKeys; i += blockDim.x) {
-      if (!a.head_mix) {
-        mixed[i] = weights[i];
-        continue;
-      }
-      const float* mix = a.head_mix + size_t{i / kTileKeys} * heads;
-      float total = 0.0f;
-      for (uint32_t g = 0; g < heads; ++g)
-        total = fmaf(mix[g], weights[g * kTileKeys + i % kTileKeys], total);
-      mixed[i] = total;
-    }
-    __syncthreads();
-    const uint32_t slot = tile * kTileKeys % a.page_tokens;
-    for (uint32_t i = threadIdx.x; i < heads * a.vdim; i += blockDim.x) {
-      const uint32_t h = i / a.vdim;
-      const T* v = page + value_block(a, h / group, slot) + size_t{i % a.vdim} * 32u;
-      // slots past the row's position may hold anything: their weight is zero
-      out[i] = value_product(mixed + h * kTileKeys, v, out[i]);
-    }
-    __syncthreads();
-  }
-  for (uint32_t i = threadIdx.x; i < heads * a.vdim; i += blockDim.x) {
-    const float gate =
-        run.gate ? sigmoid_f32(run.gate[size_t{row} * run.gate_stride + i / a.vdim]) : 1.0f;
-    store_element(static_cast<T*>(run.output) + size_t{row} * run.output_stride + i,
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < here * span * a.vdim; i += blockDim.x) {
+    const uint32_t line = i / a.vdim;
+    const size_t row = row0 + line / span;
+    const uint32_t head = first_head + line % span;
+    const float gate = run.gate ? sigmoid_f32(run.gate[row * run.gate_stride + head]) : 1.0f;
+    store_element(static_cast<T*>(run.output) + row * run.output_stride +
+                      size_t{head} * a.vdim + i % a.vdim,
                   out[i] * gate);
   }
 }
 
-// A few rows in plain F32.  One workgroup per row took 750 us for a token of 16
-// heads over 340 keys - one CU's round trips, every score twice; dealt over the
-// score and value splits of the form below it takes 53 us (scores 25,
-// values 23, sum 5).
+// A few rows in plain F32.  A workgroup takes 84 us for a token of 16 heads over
+// 340 keys and 259 over 1300 - one CU's round trips, every score twice; dealt over
+// the score and value splits of the form below it takes 24 and 32 us (scores
+// 12, values 10, sum 3 over 340).
 //
 // Scores of the workgroup's tiles for all heads, 32 lanes per (head, tile), and
 // the heads' maxima and sums over those tiles.
@@ -1190,13 +1358,65 @@ uint32_t value_splits_for(uint32_t tiles) {
   return wanted < kMaximumValueSplits ? wanted : kMaximumValueSplits;
 }
 
-size_t general_bytes(const Attention& a) {
-  return size_t{a.query_heads} * (a.dim + 2u * kTileKeys + a.vdim + 2u) * 4u;
+// What a workgroup of the general kernel keeps in LDS.
+size_t general_bytes(const GeneralArgs& args, uint32_t waves) {
+  const Attention& a = args.base.attention;
+  const size_t group = a.query_heads / a.kv_heads;
+  const size_t operands = a.head_mix ? a.kv_heads * ((group + 15u) / 16u) : 1u;
+  const size_t lines = args.rows * (a.head_mix ? a.query_heads : group < 16u ? group : 16u);
+  const size_t weights = lines * args.pitch * (a.head_mix ? 2u : 1u);
+  const size_t parts = operands < waves ? waves / operands : 1u;
+  const size_t found = parts * operands * 32u;
+  return (((lines * (a.vdim + 2u) + 3u) & ~size_t{3}) + (weights > found ? weights : found)) * 4u;
+}
+
+// Rows, tiles and pitch of the general kernel's workgroups, as their LDS holds them.
+// A row of an operand costs its workgroup little (the operand's 16 columns are
+// multiplied whether used or not), so rows are only put together when a workgroup
+// each would go round the compute units more than once.
+bool plan_general(GeneralArgs& args, uint32_t& waves, uint32_t groups_per_row) {
+  const Attention& a = args.base.attention;
+  const uint32_t group = a.query_heads / a.kv_heads;
+  const uint32_t operands = a.head_mix ? a.kv_heads * ((group + 15u) / 16u) : 1u;
+  const uint32_t most = group < 16u ? 16u / group : 1u;
+  const uint64_t wanted = (uint64_t{args.base.launch.rows} * groups_per_row + 255u) / 256u;
+  args.rows = static_cast<uint32_t>(wanted < most ? wanted : most);
+  args.tiles = operands < waves ? waves / operands : 1u;
+  const auto fits = [&](uint32_t pad) {
+    args.pitch = args.tiles * kTileKeys + pad;
+    return general_bytes(args, waves) <= kMaximumLds;
+  };
+  while (!fits(4u) && args.tiles > 1u) --args.tiles;
+  while (!fits(4u) && args.rows > 1u) --args.rows;
+  while (!fits(4u) && !fits(0u) && waves > 1u) waves /= 2u;
+  return fits(4u) || fits(0u);
+}
+
+template <typename T>
+int32_t launch_general(const AttentionArgs& base, hipStream_t stream) {
+  const Attention& a = base.attention;
+  uint32_t waves = a.head_mix ? 16u : 8u;
+  const uint32_t group = a.query_heads / a.kv_heads;
+  const uint32_t own = a.head_mix ? 1u : a.kv_heads * ((group + 15u) / 16u);
+  GeneralArgs args{base, 1u, 1u, 0u};
+  if (!plan_general(args, waves, own))
+    return fail(QLLM_INVALID_ARGUMENT,
+                "windowed attention: heads and dimensions exceed the general kernel");
+  const size_t bytes = general_bytes(args, waves);
+  if (bytes > 65536u) {
+    const auto raised =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(general_attention_kernel<T>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kMaximumLds);
+    if (raised != hipSuccess) return checked(raised, "windowed attention LDS");
+  }
+  const uint32_t blocks = (base.launch.rows + args.rows - 1u) / args.rows;
+  general_attention_kernel<T><<<dim3(blocks, own), waves * kWave, bytes, stream>>>(args);
+  return launched("windowed attention");
 }
 
 // The general form's workgroups take a tile each where there is room: their scores
-// and values are plain multiply-adds, 4 us a tile and head group (16 heads, 340 keys:
-// scores 25 us two tiles at a time, values 23 four at a time).
+// and values are plain multiply-adds, and 16 heads over 340 keys took 25 us of
+// scores two tiles a workgroup and 23 of values four, against 12 and 10.
 uint32_t general_score_splits_for(uint32_t tiles) {
   return tiles < kMaximumScoreSplits ? tiles : kMaximumScoreSplits;
 }
@@ -1318,11 +1538,12 @@ extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* a
   AttentionArgs args{a, *launch, nullptr, nullptr, nullptr, 0u, 0u, 0u};
   const uint32_t form = qllm_windowed_attention_form(attention, launch->rows);
   if (form == QLLM_ATTENTION_GENERAL) {
-    if (general_bytes(a) > kMaximumLds)
+    // (whatever the rows: what a workgroup with all heads of one row may hold)
+    if (size_t{a.query_heads} * (a.dim + 2u * kTileKeys + a.vdim + 2u) * 4u > kMaximumLds)
       return fail(QLLM_INVALID_ARGUMENT,
                   "windowed attention: heads and dimensions exceed the general kernel");
-    // Up to the split form's rows a workgroup per row leaves the chip idle (one row
-    // over 340 keys: 750 us against 53); a caller that brought no workspace
+    // Up to the split form's rows a workgroup per row leaves the chip idle (one or
+    // four rows over 340 keys: 84 us against 24); a caller that brought no workspace
     // for the splits, and heads whose buffers pass 64 KiB, stay with it.
     if (launch->rows <= kSplitRows && launch->workspace &&
         (reinterpret_cast<uintptr_t>(launch->workspace) & 15u) == 0u &&
@@ -1336,22 +1557,8 @@ extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* a
         launch_general_splits<uint16_t>(args, hip_stream);
       return launched("windowed split attention");
     }
-    if (general_bytes(a) > 65536u) {
-      const void* kernel = a.element == QLLM_ELEMENT_F32
-                               ? reinterpret_cast<const void*>(general_attention_kernel<float>)
-                               : reinterpret_cast<const void*>(
-                                     general_attention_kernel<uint16_t>);
-      const auto raised = hipFuncSetAttribute(
-          kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kMaximumLds);
-      if (raised != hipSuccess) return checked(raised, "windowed attention LDS");
-    }
-    if (a.element == QLLM_ELEMENT_F32)
-      general_attention_kernel<float>
-          <<<launch->rows, 256, general_bytes(a), hip_stream>>>(args);
-    else
-      general_attention_kernel<uint16_t>
-          <<<launch->rows, 256, general_bytes(a), hip_stream>>>(args);
-    return launched("windowed attention");
+    return a.element == QLLM_ELEMENT_F32 ? launch_general<float>(args, hip_stream)
+                                         : launch_general<uint16_t>(args, hip_stream);
   }
   if (form == QLLM_ATTENTION_PROMPT) {
     if (!launch->workspace ||

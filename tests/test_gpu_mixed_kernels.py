@@ -346,6 +346,34 @@ def test_general_splits_equal_a_workgroup_per_row(device, element, heads, kv, di
         close(again, whole[total - rows:], element)
 
 
+@pytest.mark.parametrize("element", [F32, BF16])
+@pytest.mark.parametrize("heads,kv,dim,vdim,window,sinks,mixed,rows", [
+    (16, 4, 112, 144, 100, 5, True, 530),     # three rows a workgroup
+    (6, 2, 72, 20, 0, 0, True, 259),          # a short last workgroup, a rest of dimensions
+    (6, 2, 72, 20, 50, 33, False, 259),       # a workgroup per operand
+    (20, 1, 320, 30, 64, 0, True, 40),        # two operands of one key/value head
+    (40, 2, 24, 320, 0, 0, False, 40),
+    (5, 5, 16, 16, 20, 1, True, 700),         # one head an operand
+    (72, 72, 4, 496, 30, 0, True, 34),        # LDS holds one tile and no padding
+], ids=str)
+def test_general_prompts_match_the_oracle(device, element, heads, kv, dim, vdim, window, sinks,
+                                          mixed, rows):
+    """Rows of the general form: several to a workgroup, operands of more than 16
+    heads, remainders of dimensions and workgroups."""
+    rng = np.random.default_rng(rows)
+    scale = 1.0 / np.sqrt(dim)
+    mix = mm.bf16(np.eye(heads) + 0.2 * rng.standard_normal((heads, heads)))
+    layer = Attention(device, element, heads, kv, dim, vdim, window, sinks,
+                      mix if mixed else None, scale, context=704,
+                      strides=(padded(dim, 32), padded(vdim, 16)))
+    assert qh.call("qllm_windowed_attention_form", ctypes.byref(layer.layer),
+                   rows) == qh.ATTENTION_GENERAL
+    projections = mm.bf16(rng.standard_normal((rows, layer.stride)))
+    want = layer.expected(projections, window, sinks,
+                          (mix if mixed else np.eye(heads)).astype(np.float64), scale)
+    close(layer.run(projections, 0), want, element)
+
+
 def stand_out(rng, layer, projections, pairs, head, strength=None):
     """Makes the score of (query row, key row) of one head stand out: the key
     becomes the query direction (unrotated dimensions or rotary 0 assumed)."""
