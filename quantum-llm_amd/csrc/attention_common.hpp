@@ -170,6 +170,7 @@ __device__ __forceinline__ void q8_encode_record(const float* source,
 // besides their tiles, in tiles' worth of time - the deal is over
 // context_tiles + tail_work tiles of which the last tail_work do not exist, so
 // those waves walk that many fewer.
+template <int WAVES = kSplitWaves>
 __device__ __forceinline__ void wave_tile_range(uint32_t context_tiles,
                                                 uint32_t tile_tokens,
                                                 uint32_t split_tokens,
@@ -181,8 +182,8 @@ __device__ __forceinline__ void wave_tile_range(uint32_t context_tiles,
   if (split_tokens == 0u) {
     // floor(slot * tiles / slots) in 32-bit arithmetic: with tiles = q * slots
     // + r it is slot * q + floor(slot * r / slots), and slot * r < slots^2
-    const uint32_t slots = splits * kSplitWaves;
-    const uint32_t slot = split * kSplitWaves + wave;
+    const uint32_t slots = splits * WAVES;
+    const uint32_t slot = split * WAVES + wave;
     const uint32_t dealt = context_tiles + tail_work;
     const uint32_t quotient = dealt / slots;
     const uint32_t remainder = dealt - quotient * slots;
@@ -193,8 +194,8 @@ __device__ __forceinline__ void wave_tile_range(uint32_t context_tiles,
     const uint32_t split_tiles = split_tokens / tile_tokens;
     const uint32_t begin = min(split * split_tiles, context_tiles);
     const uint32_t count = min(begin + split_tiles, context_tiles) - begin;
-    tile_first = begin + wave * count / kSplitWaves;
-    tile_last = begin + (wave + 1u) * count / kSplitWaves;
+    tile_first = begin + wave * count / WAVES;
+    tile_last = begin + (wave + 1u) * count / WAVES;
   }
 }
 
@@ -210,27 +211,29 @@ struct PartialTarget {
   uint32_t matrix_rows;    // rows * group
 };
 
-// Merges the eight wave states of a workgroup and writes the split partial.
+// Merges the wave states of a workgroup (of eight waves unless said otherwise) and writes the split partial.
 // A wave's state: per row tile rt (16 matrix rows; lane (col = lane%16, quad =
 // lane/16) owns matrix row 16*rt + col) the running maximum (log2 units) and
 // sum, and out[dt][rt] = O^T elements d = 16*dt + 4*quad .. +3 of that row.
 //  1. every wave publishes its (max, sum) per row; all waves derive the
 //     merged maximum and bring their own accumulators to it.
 //  2. the accumulators are summed reduce-scatter style, eight 1 KiB register
-//     vectors (one per receiving wave) at a time: each wave drops the eight
-//     vectors of the group into LDS, lane-linear (no bank conflicts), and
-//     wave v adds up vector v of all eight waves in a fixed order.  Wave v
-//     ends up owning vectors v, v+8, ... of the result and writes them out.
-// `pool` needs 64 KiB of LDS, `summary` 512*RT bytes per wave; both may
+//     vectors at a time: each wave drops the eight vectors of the group into
+//     LDS, lane-linear (no bank conflicts), and wave v adds up vectors v,
+//     v + WAVES, ... of all waves in a fixed order, owns them in the result and
+//     writes them out.
+// `pool` needs 8 KiB of LDS per wave, `summary` 512*RT bytes; both may
 // overlap whatever the tile loop used (the function starts with a barrier).
-template <int D, int RT>
+template <int D, int RT, int WAVES = kSplitWaves>
 __device__ __forceinline__ void merge_wave_states(
     float (&running_max)[RT], float (&running_sum)[RT],
     f32x4 (&out)[D / 16][RT], float* pool, float2* summary, uint32_t wave,
     uint32_t lane, const PartialTarget& target) {
   constexpr int DT = D / 16;
   constexpr int VECTORS = DT * RT;   // f32x4 accumulator vectors per wave
-  static_assert(VECTORS % kSplitWaves == 0, "vectors are dealt to 8 waves");
+  constexpr int ROUND = 8;           // vectors of a round
+  constexpr int OWN = ROUND / WAVES;
+  static_assert(VECTORS % ROUND == 0 && ROUND % WAVES == 0, "vectors are dealt to the waves");
   const uint32_t col = lane & 15u;
   const uint32_t quad = lane >> 4;
   __syncthreads();  // tiles done: the LDS they used is free
@@ -242,16 +245,16 @@ __device__ __forceinline__ void merge_wave_states(
   float merged_max[RT], merged_sum[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
-    float2 part[kSplitWaves];
+    float2 part[WAVES];
     float maximum = kMaskedMax;
 #pragma unroll
-    for (int w = 0; w < kSplitWaves; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       part[w] = summary[(w * RT + rt) * 64 + lane];
       maximum = fmaxf(maximum, part[w].x);
     }
     float sum = 0.0f;
 #pragma unroll
-    for (int w = 0; w < kSplitWaves; ++w)
+    for (int w = 0; w < WAVES; ++w)
       sum = fmaf(part[w].y, __builtin_amdgcn_exp2f(part[w].x - maximum), sum);
     const float factor = __builtin_amdgcn_exp2f(running_max[rt] - maximum);
 #pragma unroll
@@ -261,29 +264,32 @@ __device__ __forceinline__ void merge_wave_states(
     merged_max[rt] = maximum;
     merged_sum[rt] = sum;
   }
-  f32x4 merged[VECTORS / kSplitWaves];
+  f32x4 merged[VECTORS / WAVES];
 #pragma unroll
-  for (int group_index = 0; group_index < VECTORS / kSplitWaves; ++group_index) {
+  for (int group_index = 0; group_index < VECTORS / ROUND; ++group_index) {
 #pragma unroll
-    for (int v = 0; v < kSplitWaves; ++v) {
-      const int k = group_index * kSplitWaves + v;
-      *reinterpret_cast<f32x4*>(pool + ((wave * kSplitWaves + v) * 64 + lane) * 4u) =
+    for (int v = 0; v < ROUND; ++v) {
+      const int k = group_index * ROUND + v;
+      *reinterpret_cast<f32x4*>(pool + ((wave * ROUND + v) * 64 + lane) * 4u) =
           out[k / RT][k % RT];
     }
     __syncthreads();
-    f32x4 total = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int w = 0; w < kSplitWaves; ++w)
-      total += *reinterpret_cast<const f32x4*>(
-          pool + ((w * kSplitWaves + wave) * 64 + lane) * 4u);
-    merged[group_index] = total;
+    for (int own = 0; own < OWN; ++own) {
+      f32x4 total = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w)
+        total += *reinterpret_cast<const f32x4*>(
+            pool + ((w * ROUND + own * WAVES + wave) * 64 + lane) * 4u);
+      merged[group_index * OWN + own] = total;
+    }
     __syncthreads();
   }
 
   // partials: wave v writes the vectors it owns, wave 0 also max and sum
 #pragma unroll
-  for (int group_index = 0; group_index < VECTORS / kSplitWaves; ++group_index) {
-    const uint32_t k = group_index * kSplitWaves + wave;
+  for (int group_index = 0; group_index < VECTORS / WAVES; ++group_index) {
+    const uint32_t k = group_index * WAVES + wave;
     const uint32_t dt = k / RT;
     const uint32_t rt = k % RT;
     const uint32_t matrix_row = 16u * rt + col;

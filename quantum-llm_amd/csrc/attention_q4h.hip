@@ -432,9 +432,10 @@ __global__ void rope_table_kernel(float2* table, uint32_t rotary_dim,
 // the staged tile before it is read (the cache pages need not hold them yet);
 // the workgroup that owns the context's last tile also writes them to the
 // pages for later steps.
-template <int D, int RT, bool FUSED = false>
-__global__ __launch_bounds__(kSplitWaves * 64) void q4h_attention_split_kernel(
+template <int D, int RT, bool FUSED = false, int WAVES = kSplitWaves>
+__global__ __launch_bounds__(WAVES * 64, 2) void q4h_attention_split_kernel(
     const SplitArgs launch_args) {
+  static_assert(!FUSED || WAVES == kSplitWaves, "the fused work is dealt to eight waves");
   // a batched launch narrows the arguments to the batch of this grid layer
   SplitArgs args = launch_args;
   if (!FUSED && launch_args.batch_rows) {
@@ -481,7 +482,7 @@ __global__ __launch_bounds__(kSplitWaves * 64) void q4h_attention_split_kernel(
   // with the tile after the next.
   constexpr int DEPTH = 1;
   __shared__ __attribute__((aligned(16)))
-  uint8_t stage[kSplitWaves * STAGE * DEPTH];
+  uint8_t stage[WAVES * STAGE * DEPTH];
   // query operands in MFMA order, then per matrix row its scale and the number
   // of tokens it may attend
   __shared__ __attribute__((aligned(16)))
@@ -506,10 +507,11 @@ __global__ __launch_bounds__(kSplitWaves * 64) void q4h_attention_split_kernel(
   // (fused: the workgroup at the end of the context also encodes the batch's
   // K/V records, lays them over its tiles and writes them to their pages -
   // about two tiles' worth of time for each of its waves.  The plain kernel
-  // deals the same way, so that both add up a context in the same order.)
-  constexpr uint32_t kTailWork = 2u * kSplitWaves;
-  wave_tile_range(context_tiles, 64u, args.split_tokens, split, gridDim.y, wave,
-                  tile_first, tile_last, kTailWork);
+  // deals the same way, so that both add up a context in the same order; not so
+  // the smaller workgroups of long prompts.)
+  constexpr uint32_t kTailWork = WAVES == kSplitWaves ? 2u * kSplitWaves : 0u;
+  wave_tile_range<WAVES>(context_tiles, 64u, args.split_tokens, split, gridDim.y, wave,
+                         tile_first, tile_last, kTailWork);
 
   // the wave's staging areas: tile t of the wave uses area t % DEPTH
   uint8_t* const stage_base = stage + wave * (STAGE * DEPTH);
@@ -596,8 +598,8 @@ __global__ __launch_bounds__(kSplitWaves * 64) void q4h_attention_split_kernel(
   // The F32 query row is quantised here to 15 bits and split into two int8
   // planes, q = scale * (128*hi + lo) with hi in [-127,127], lo in [-64,63],
   // so the integer scores carry the query to ~3e-5 relative instead of the
-  // 4e-3 of a single Q8 plane.  The operands are published in MFMA order.
-  static_assert(RT * KSTEPS <= kSplitWaves, "one wave per operand pair");
+  // 4e-3 of a single Q8 plane.  The operands are published in MFMA order, a
+  // wave per pair of planes (a workgroup of fewer waves goes round).
   // fused mode: scratch of the per-wave rotary, then the batch's fresh K/V
   // records [K codes | V codes | K scale | V scale] of this KV head
   constexpr int RECORD = D + 16;
@@ -896,14 +898,14 @@ __global__ __launch_bounds__(kSplitWaves * 64) void q4h_attention_split_kernel(
     const uint8_t* planes = uniform_pointer(
         args.query_operands + static_cast<size_t>(kv_head) * kPlanes * 1024u);
 #pragma unroll
-    for (uint32_t plane = 0; plane < (kPlanes + kSplitWaves - 1u) / kSplitWaves;
+    for (uint32_t plane = 0; plane < (kPlanes + WAVES - 1u) / WAVES;
          ++plane) {
-      const uint32_t index = plane * kSplitWaves + wave;
+      const uint32_t index = plane * WAVES + wave;
       if (index < kPlanes)
         copy16_to_lds(planes + index * 1024u, lane_now * 16u,
                       exchange_lds + index * 1024u);
     }
-    if (wave == kSplitWaves - 1u && lane_now < RT * 16u) {
+    if (wave == WAVES - 1u && lane_now < RT * 16u) {
       const uint8_t* scales = uniform_pointer(reinterpret_cast<const uint8_t*>(
           args.query_operand_scales + static_cast<size_t>(kv_head) * RT * 16u));
       copy4_to_lds(scales, lane_now * 4u, exchange_lds + kPlanes * 1024u);
@@ -919,74 +921,77 @@ __global__ __launch_bounds__(kSplitWaves * 64) void q4h_attention_split_kernel(
   } else if (args.query_operands) {
     // the operands were asked for before the tiles
     vmem_wait_units<KS_LOADS>(halves_after_operands);
-  } else if (wave < static_cast<uint32_t>(RT * KSTEPS)) {
-    // wave u builds k-step u % KSTEPS of row tile u / KSTEPS (the row's scale
-    // needs the whole row, so every such wave reads all of it)
-    const uint32_t rt = wave / KSTEPS;
-    const uint32_t step = wave % KSTEPS;
-    const uint32_t matrix_row = 16u * rt + col;
-    const bool valid = matrix_row < matrix_rows;
-    const uint32_t row = valid ? matrix_row / group : 0u;
-    const uint32_t head = kv_head * group + (valid ? matrix_row % group : 0u);
-    const size_t record = static_cast<size_t>(row) * args.query_heads + head;
-    float values[16];
-    float maximum = 0.0f;
+  } else {
+#pragma unroll 1
+    for (uint32_t pair = wave; pair < static_cast<uint32_t>(RT * KSTEPS); pair += WAVES) {
+      // pair u is k-step u % KSTEPS of row tile u / KSTEPS (the row's scale needs
+      // the whole row, so every such wave reads all of it)
+      const uint32_t rt = pair / KSTEPS;
+      const uint32_t step = pair % KSTEPS;
+      const uint32_t matrix_row = 16u * rt + col;
+      const bool valid = matrix_row < matrix_rows;
+      const uint32_t row = valid ? matrix_row / group : 0u;
+      const uint32_t head = kv_head * group + (valid ? matrix_row % group : 0u);
+      const size_t record = static_cast<size_t>(row) * args.query_heads + head;
+      float values[16];
+      float maximum = 0.0f;
 #pragma unroll
-    for (int h = 0; h < KSTEPS; ++h) {
-      const uint32_t d0 = 128u * (h / 2) + 32u * quad + 16u * (h % 2);
+      for (int h = 0; h < KSTEPS; ++h) {
+        const uint32_t d0 = 128u * (h / 2) + 32u * quad + 16u * (h % 2);
 #pragma unroll
-      for (int piece = 0; piece < 4; ++piece) {
-        float4 loaded = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (valid)
-          loaded = *reinterpret_cast<const float4*>(
-              args.query + record * args.query_stride + d0 + 4u * piece);
-        if (static_cast<uint32_t>(h) == step) {
-          values[4 * piece + 0] = loaded.x;
-          values[4 * piece + 1] = loaded.y;
-          values[4 * piece + 2] = loaded.z;
-          values[4 * piece + 3] = loaded.w;
+        for (int piece = 0; piece < 4; ++piece) {
+          float4 loaded = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+          if (valid)
+            loaded = *reinterpret_cast<const float4*>(
+                args.query + record * args.query_stride + d0 + 4u * piece);
+          if (static_cast<uint32_t>(h) == step) {
+            values[4 * piece + 0] = loaded.x;
+            values[4 * piece + 1] = loaded.y;
+            values[4 * piece + 2] = loaded.z;
+            values[4 * piece + 3] = loaded.w;
+          }
+          maximum = fmaxf(maximum, fmaxf(fmaxf(fabsf(loaded.x), fabsf(loaded.y)),
+                                         fmaxf(fabsf(loaded.z), fabsf(loaded.w))));
         }
-        maximum = fmaxf(maximum, fmaxf(fmaxf(fabsf(loaded.x), fabsf(loaded.y)),
-                                       fmaxf(fabsf(loaded.z), fabsf(loaded.w))));
       }
-    }
-    maximum = quad_row_max(maximum);
-    const float scale = fmaxf(maximum * (1.0f / 16319.0f), 0x1p-100f);
-    const float inverse = 1.0f / scale;
-    if (quad == 0u && step == 0u) {
-      exchange_scale[16 * rt + col] =
-          scale * (1.4426950408889634f / (16.0f * sqrtf(static_cast<float>(D))));
-      exchange_limit[16 * rt + col] = first_context_tokens + row;
-    }
-    uint32_t high_bytes[16], low_bytes[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      int quantized = __float2int_rn(values[j] * inverse);
-      quantized = max(-16319, min(16319, quantized));
-      const int high = (quantized + 64) >> 7;  // floor((v+64)/128)
-      const int low = quantized - (high << 7);
-      high_bytes[j] = static_cast<uint32_t>(high) & 0xffu;
-      low_bytes[j] = static_cast<uint32_t>(low) & 0xffu;
-    }
-    // byte order inside each 8-element half: even d first, then odd d,
-    // matching the order in which the key nibbles are widened
-    const int order[16] = {0, 2, 4, 6, 1, 3, 5, 7, 8, 10, 12, 14, 9, 11, 13, 15};
-    i32x4 high_operand, low_operand;
-#pragma unroll
-    for (int word = 0; word < 4; ++word) {
-      uint32_t high_word = 0u, low_word = 0u;
-#pragma unroll
-      for (int byte = 0; byte < 4; ++byte) {
-        high_word |= high_bytes[order[4 * word + byte]] << (8 * byte);
-        low_word |= low_bytes[order[4 * word + byte]] << (8 * byte);
+      maximum = quad_row_max(maximum);
+      const float scale = fmaxf(maximum * (1.0f / 16319.0f), 0x1p-100f);
+      const float inverse = 1.0f / scale;
+      if (quad == 0u && step == 0u) {
+        exchange_scale[16 * rt + col] =
+            scale * (1.4426950408889634f / (16.0f * sqrtf(static_cast<float>(D))));
+        exchange_limit[16 * rt + col] = first_context_tokens + row;
       }
-      high_operand[word] = static_cast<int>(high_word);
-      low_operand[word] = static_cast<int>(low_word);
+      uint32_t high_bytes[16], low_bytes[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        int quantized = __float2int_rn(values[j] * inverse);
+        quantized = max(-16319, min(16319, quantized));
+        const int high = (quantized + 64) >> 7;  // floor((v+64)/128)
+        const int low = quantized - (high << 7);
+        high_bytes[j] = static_cast<uint32_t>(high) & 0xffu;
+        low_bytes[j] = static_cast<uint32_t>(low) & 0xffu;
+      }
+      // byte order inside each 8-element half: even d first, then odd d,
+      // matching the order in which the key nibbles are widened
+      const int order[16] = {0, 2, 4, 6, 1, 3, 5, 7, 8, 10, 12, 14, 9, 11, 13, 15};
+      i32x4 high_operand, low_operand;
+#pragma unroll
+      for (int word = 0; word < 4; ++word) {
+        uint32_t high_word = 0u, low_word = 0u;
+#pragma unroll
+        for (int byte = 0; byte < 4; ++byte) {
+          high_word |= high_bytes[order[4 * word + byte]] << (8 * byte);
+          low_word |= low_bytes[order[4 * word + byte]] << (8 * byte);
+        }
+        high_operand[word] = static_cast<int>(high_word);
+        low_operand[word] = static_cast<int>(low_word);
+      }
+      *reinterpret_cast<i32x4*>(exchange + (pair * 2u + 0u) * 1024u + lane * 16u) =
+          high_operand;
+      *reinterpret_cast<i32x4*>(exchange + (pair * 2u + 1u) * 1024u + lane * 16u) =
+          low_operand;
     }
-    *reinterpret_cast<i32x4*>(exchange + (wave * 2u + 0u) * 1024u + lane * 16u) =
-        high_operand;
-    *reinterpret_cast<i32x4*>(exchange + (wave * 2u + 1u) * 1024u + lane * 16u) =
-        low_operand;
   }
   __syncthreads();
 
@@ -1309,19 +1314,19 @@ __global__ __launch_bounds__(kSplitWaves * 64) void q4h_attention_split_kernel(
                           : kMaskedMax;
   }
 
-  // ---- merge the eight wave states, write the split partial ------------------
-  static_assert(kSplitWaves * kSplitWaves * 1024 <= kSplitWaves * STAGE,
+  // ---- merge the wave states, write the split partial ------------------
+  static_assert(WAVES * 8 * 1024 <= WAVES * STAGE,
                 "merge pool does not fit the staging memory");
-  static_assert(kSplitWaves * RT * 64 * 8 <= sizeof(exchange),
+  static_assert(WAVES * RT * 64 * 8 <= sizeof(exchange),
                 "row summaries do not fit the exchange area");
   const PartialTarget target{args.partial_maxima, args.partial_sums,
                              args.partial_outputs, args.maximum_splits,
                              args.query_heads, kv_head, split, group,
                              matrix_rows};
-  merge_wave_states<D, RT>(running_max, running_sum, out,
-                           reinterpret_cast<float*>(stage),
-                           reinterpret_cast<float2*>(exchange), wave, lane,
-                           target);
+  merge_wave_states<D, RT, WAVES>(running_max, running_sum, out,
+                                  reinterpret_cast<float*>(stage),
+                                  reinterpret_cast<float2*>(exchange), wave, lane,
+                                  target);
 }
 
 // ---- prompt attention: eight row batches share every cache tile -------------
@@ -2654,9 +2659,25 @@ extern "C" int32_t qllm_attention_paged_q4h_batched(
   args.batch_rows = batch_rows;
   const dim3 grid(launch->kv_heads, splits, batches);
   const hipStream_t stream = as_stream(launch->stream);
-  int32_t status = launch->head_dim == 128u
-                       ? launch_split<128>(args, row_tiles, grid, stream)
-                       : launch_split<256>(args, row_tiles, grid, stream);
+  // At head_dim 256 a workgroup of eight waves fills a compute unit's LDS, and its
+  // prologue and the merge of its states, 20 us, stand between two workgroups; of two
+  // waves three fit and hide each other's, but a tile costs them 1.03 us of the compute
+  // unit against 0.86.  24 heads on 4, five rows a batch: whole prompts of 960 / 3001
+  // rows (768 / 2404 workgroups, 8 / 24 tiles on average) 84 / 383 us with eight
+  // waves, 68 / 303 with two; 320 rows over 4320 tokens cut three ways (768, 22) 119
+  // and 101; 1000 rows over 9000 (800, 133) 512 and 603.  Where fewer workgroups than
+  // three a compute unit leave waves idle, eight share a context better: 640 rows
+  // over 4640 tokens (512, 66) 171 us against 220.
+  const uint64_t middle = uint64_t{launch->first_context_tokens} + launch->rows / 2u;
+  int32_t status = QLLM_OK;
+  if (launch->head_dim == 256u && row_tiles == 2u &&
+      uint64_t{grid.x} * grid.y * grid.z >= 768u && middle <= uint64_t{splits} * 48u * 64u) {
+    q4h_attention_split_kernel<256, 2, false, 2><<<grid, 128, 0, stream>>>(args);
+    status = launched("Q4H attention split");
+  } else {
+    status = launch->head_dim == 128u ? launch_split<128>(args, row_tiles, grid, stream)
+                                      : launch_split<256>(args, row_tiles, grid, stream);
+  }
   if (status != QLLM_OK) return status;
   // partials are laid out by global row, which is what the combine indexes
   return launch_attention_combine(

@@ -1275,7 +1275,7 @@ void Mi355DenseFp4Provider::enqueue_attention(
 }
 
 // Context splits of a batched (prompt) attention launch.  Every workgroup pays
-// a prologue and a merge of its eight wave states whatever its share of the
+// a prologue and a merge of its wave states whatever its share of the
 // context, so the context is cut only as far as it takes to give every CU a
 // workgroup: a full chunk's row batches need no cut at all (a 32768-token
 // prompt: 5.50 s with eight splits, 5.09 / 4.91 / 4.79 s with four / two / one).

@@ -216,6 +216,45 @@ def test_batched_launch_equals_one_launch_per_batch(device, total, first, Q, KV,
             qh.call("qllm_attention_paged_q4h_batched", launch, total)
 
 
+@pytest.mark.parametrize("total,first,Q,KV,batch,splits", [
+    (958, 1, 24, 4, 5, 1),      # 768 workgroups: two waves each; the last has 3 rows
+    (93, 70, 16, 8, 16, 16),    # splits without a tile
+    (120, 1000, 12, 2, 5, 16)])
+def test_large_batched_launches_of_256_dimensions(device, total, first, Q, KV, batch, splits):
+    """Workgroups of two waves: the oracle's attention, and up to the rounding of
+    the probabilities what launches of a batch each compute."""
+    rng = np.random.default_rng(total)
+    d, page_tokens, tokens = 256, 64, first + total - 1
+    keys = rng.standard_normal((tokens, KV, d)).astype(np.float32)
+    values = rng.standard_normal((tokens, KV, d)).astype(np.float32)
+    pages = synth.q4h_pages(keys, values, page_tokens, 1, 0)
+    query = ol.bf16_round(rng.standard_normal((total, Q, 2 * d)).astype(np.float32))
+    d_pages = [gu.device_tensor(page, device) for page in pages]
+    table = torch.tensor([page.data_ptr() for page in d_pages], dtype=torch.int64,
+                         device=device)
+    d_query = gu.device_tensor(query, device)
+    maxima = torch.zeros((total, splits, Q), device=device)
+    sums = torch.zeros_like(maxima)
+    outputs = torch.zeros((total, splits, Q, d), device=device)
+    out = torch.full((total, Q, d), float("nan"), device=device)
+    launch = qh.Q4hAttentionLaunch(
+        qh.ptr(d_query), 0, 0, qh.ptr(table), qh.ptr(out), qh.ptr(maxima), qh.ptr(sums),
+        qh.ptr(outputs), first, total, 0, page_tokens, Q, KV, d, 0, splits, 2 * d, 1,
+        qh.OUT_F32, None)
+    qh.call("qllm_attention_paged_q4h_batched", launch, batch)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    shape = ol.AttentionShape(total, Q, KV, d, first, page_tokens, 0, 1)
+    gu.assert_close(got, ol.attention_q4h(shape, query, pages, "f64"), what="batched attention")
+    # (binary16 probabilities are rounded relative to each wave's running maximum)
+    for row in (0, total // batch // 2 * batch, (total - 1) // batch * batch):
+        rows = min(batch, total - row)
+        single = gu.q4h_attention(device, pages, query[row:row + rows], rows, Q, KV, d,
+                                  first + row, page_tokens, 0, 1, balanced_splits=splits)
+        gu.assert_close(got[row:row + rows], single, rtol=3e-3, atol=3e-4,
+                        what="batched vs single")
+
+
 @pytest.mark.parametrize("total,first,Q,KV,gated,batch,splits", [
     (100, 300, 64, 8, False, 6, 1),      # 17 batches: three workgroup layers, the last part empty
     (100, 300, 64, 8, False, 6, 3),      # the tiles cut over three splits
