@@ -8,7 +8,8 @@
 //  * split (one to four rows, decode): scores of all visible keys once, 16 keys
 //    per wave, with each workgroup's maximum and sum; then, per key/value head,
 //    normalise, mix (F32) and multiply with the values, the visible tiles dealt
-//    over workgroups; then the partial outputs are added and gated.
+//    over workgroups; then the partial outputs are added and gated (few tiles: one
+//    workgroup has them all and gates its sums itself).
 //  * prompt: a first walk over the visible keys takes every row's softmax
 //    denominator.  In a second, a workgroup owns 16 query rows and all heads: it
 //    recomputes the scores, leaves the normalised weights in LDS as bf16 high
@@ -713,12 +714,15 @@ __global__ __launch_bounds__(256) void split_scores_kernel(AttentionArgs args) {
 
 constexpr uint32_t kMixRow = 40;   // bf16 values per LDS row of mixed weights (32 + pad)
 
-// NV = value_stride / 16, GROUP = query heads per key/value head at most.
-template <int NV, int GROUP>
-__global__ __launch_bounds__(256) void split_values_kernel(AttentionArgs args) {
+// NV = value_stride / 16, GROUP = query heads per key/value head at most.  The
+// launch is a chain of round trips (its tiles are a few KiB each): a wave's first
+// values and scores set out before the maxima are merged.  With eight waves a
+// workgroup takes all tiles of its heads and writes the gated outputs itself.
+template <int NV, int GROUP, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void split_values_kernel(AttentionArgs args) {
   __shared__ float row_maximum[64], row_inverse[64];
   __shared__ __attribute__((aligned(16))) float mix[64][GROUP];
-  __shared__ __attribute__((aligned(16))) uint16_t mixed[4][16 * kMixRow];
+  __shared__ __attribute__((aligned(16))) uint16_t mixed[WAVES][16 * kMixRow];
   __shared__ f32x4 gathered[NV * kWave];
   const Attention& a = args.attention;
   const uint32_t row = blockIdx.z;
@@ -730,9 +734,34 @@ __global__ __launch_bounds__(256) void split_values_kernel(AttentionArgs args) {
   const uint32_t wave = threadIdx.x / kWave;
   const uint32_t lane = threadIdx.x % kWave;
 
+  const uint32_t begin = static_cast<uint32_t>(uint64_t{range.count} * blockIdx.x / gridDim.x);
+  const uint32_t end =
+      static_cast<uint32_t>(uint64_t{range.count} * (blockIdx.x + 1u) / gridDim.x);
+  // a tile's values, and the scores of key lane % 32 with eight heads of parity lane / 32
+  i32x4 v[NV];
+  float raw[8];
+  const auto fetch_scores = [&](uint32_t ordinal, uint32_t g0) {
+    const float* scores = args.scores + size_t{row} * heads * args.capacity +
+                          size_t{ordinal} * kTileKeys + lane % 32u;
+#pragma unroll
+    for (uint32_t i = 0; i < 8u; ++i)
+      raw[i] = scores[static_cast<size_t>(min(g0 + 2u * i, heads - 1u)) * args.capacity];
+  };
+  const auto fetch = [&](uint32_t ordinal) {
+    const uint32_t key0 = range.tile(ordinal) * kTileKeys;
+    const i32x4* values = reinterpret_cast<const i32x4*>(
+                              page_of<const uint16_t>(a, key0) +
+                              value_block(a, kv, key0 % a.page_tokens)) +
+                          lane % 16u * 4u + lane / 16u;
+#pragma unroll
+    for (int t = 0; t < NV; ++t) v[t] = values[t * kWave];
+    fetch_scores(ordinal, lane / 32u);
+  };
+  if (begin + wave < end) fetch(begin + wave);
+
   // a wave per head, a lane per score split (at most 64)
 #pragma unroll 4
-  for (uint32_t h = wave; h < heads; h += 4u) {
+  for (uint32_t h = wave; h < heads; h += WAVES) {
     float m = -INFINITY;
     float t = 0.0f;
     if (lane < args.score_splits) {
@@ -755,32 +784,16 @@ __global__ __launch_bounds__(256) void split_values_kernel(AttentionArgs args) {
     const float value = a.head_mix ? a.head_mix[size_t{h} * heads + g] : (h == g ? 1.0f : 0.0f);
     mix[g][in_group] = in_group < group ? value : 0.0f;
   }
-  for (uint32_t i = threadIdx.x; i < 4u * 16u * kMixRow; i += blockDim.x)
+  for (uint32_t i = threadIdx.x; i < WAVES * 16u * kMixRow; i += blockDim.x)
     mixed[0][i] = 0u;
   __syncthreads();
 
   f32x4 sum[NV] = {};
-  const uint32_t begin = static_cast<uint32_t>(uint64_t{range.count} * blockIdx.x / gridDim.x);
-  const uint32_t end =
-      static_cast<uint32_t>(uint64_t{range.count} * (blockIdx.x + 1u) / gridDim.x);
-  for (uint32_t ordinal = begin + wave; ordinal < end; ordinal += 4u) {
-    const uint32_t key0 = range.tile(ordinal) * kTileKeys;
-    const i32x4* values = reinterpret_cast<const i32x4*>(
-                              page_of<const uint16_t>(a, key0) +
-                              value_block(a, kv, key0 % a.page_tokens)) +
-                          lane % 16u * 4u + lane / 16u;
-    i32x4 v[NV];
-#pragma unroll
-    for (int t = 0; t < NV; ++t) v[t] = values[t * kWave];
-    // lane: key lane % 32, heads of parity lane / 32
-    const float* scores = args.scores + size_t{row} * heads * args.capacity +
-                          size_t{ordinal} * kTileKeys + lane % 32u;
+  for (uint32_t ordinal = begin + wave; ordinal < end; ordinal += WAVES) {
+    if (ordinal != begin + wave) fetch(ordinal);
     float share[GROUP] = {};
     for (uint32_t g0 = lane / 32u; g0 < heads; g0 += 16u) {
-      float raw[8];
-#pragma unroll
-      for (uint32_t i = 0; i < 8u; ++i)
-        raw[i] = scores[size_t{min(g0 + 2u * i, heads - 1u)} * args.capacity];
+      if (g0 >= 2u) fetch_scores(ordinal, g0);
 #pragma unroll
       for (uint32_t i = 0; i < 8u; ++i) {
         const uint32_t g = min(g0 + 2u * i, heads - 1u);
@@ -807,7 +820,7 @@ __global__ __launch_bounds__(256) void split_values_kernel(AttentionArgs args) {
     __builtin_amdgcn_wave_barrier();
   }
   // the waves' sums in order
-  for (uint32_t turn = 0; turn < 4u; ++turn) {
+  for (uint32_t turn = 0; turn < static_cast<uint32_t>(WAVES); ++turn) {
     if (wave == turn)
 #pragma unroll
       for (int t = 0; t < NV; ++t)
@@ -819,9 +832,18 @@ __global__ __launch_bounds__(256) void split_values_kernel(AttentionArgs args) {
     if (d >= a.vdim) continue;
     for (uint32_t j = 0; j < 4u; ++j) {
       const uint32_t h = 4u * (i % kWave / 16u) + j;
-      if (h < group)
+      if (h >= group) continue;
+      if constexpr (WAVES == 8) {
+        const auto& run = args.launch;
+        const uint32_t head = kv * group + h;
+        const float gate =
+            run.gate ? sigmoid_f32(run.gate[size_t{row} * run.gate_stride + head]) : 1.0f;
+        store_element(static_cast<uint16_t*>(run.output) + size_t{row} * run.output_stride +
+                          head * a.vdim + d, gathered[i][j] * gate);
+      } else {
         args.partials[((size_t{row} * args.value_splits + blockIdx.x) * heads + kv * group +
                        h) * a.vdim + d] = gathered[i][j];
+      }
     }
   }
 }
@@ -1353,7 +1375,16 @@ uint32_t score_splits_for(uint32_t tiles) {
   return wanted < kMaximumScoreSplits ? wanted : kMaximumScoreSplits;
 }
 
-uint32_t value_splits_for(uint32_t tiles) {
+// Up to two tiles a wave, one workgroup of eight waves per key/value head saves the
+// launch that adds the splits: one row of 16 heads on 4, 128 dimensions, 16.2 -> 13.6
+// us over 6 tiles, 16.5 -> 15.4 over 11 and 16.5 -> 16.1 over 16.  (More heads to a
+// key/value head want more registers than eight waves have.)
+bool whole_values(const Attention& a, uint32_t tiles) {
+  return tiles <= 16u && a.query_heads / a.kv_heads <= 4u;
+}
+
+uint32_t value_splits_for(const Attention& a, uint32_t tiles) {
+  if (whole_values(a, tiles)) return 1u;
   const uint32_t wanted = (tiles + 3u) / 4u;
   return wanted < kMaximumValueSplits ? wanted : kMaximumValueSplits;
 }
@@ -1440,7 +1471,7 @@ void place_splits(AttentionArgs& args, bool general) {
   const uint32_t tiles = maximum_tiles(a, args.launch.maximum_position);
   args.capacity = tiles * kTileKeys;
   args.score_splits = general ? general_score_splits_for(tiles) : score_splits_for(tiles);
-  args.value_splits = general ? general_value_splits_for(tiles) : value_splits_for(tiles);
+  args.value_splits = general ? general_value_splits_for(tiles) : value_splits_for(a, tiles);
   args.scores = static_cast<float*>(args.launch.workspace);
   args.maxima = args.scores + size_t{args.launch.rows} * a.query_heads * args.capacity;
   args.partials =
@@ -1588,12 +1619,15 @@ extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* a
     split_scores_kernel<8><<<score_grid, 256, 0, hip_stream>>>(args);
   const dim3 value_grid(args.value_splits, a.kv_heads, launch->rows);
   const bool narrow = a.query_heads / a.kv_heads <= 4u;
+  const bool whole = whole_values(a, args.capacity / kTileKeys);
   const auto values = [&](auto nv) {
     constexpr int NV = decltype(nv)::value;
-    if (narrow)
-      split_values_kernel<NV, 4><<<value_grid, 256, 0, hip_stream>>>(args);
+    if (whole)
+      split_values_kernel<NV, 4, 8><<<value_grid, 512, 0, hip_stream>>>(args);
+    else if (narrow)
+      split_values_kernel<NV, 4, 4><<<value_grid, 256, 0, hip_stream>>>(args);
     else
-      split_values_kernel<NV, 16><<<value_grid, 256, 0, hip_stream>>>(args);
+      split_values_kernel<NV, 16, 4><<<value_grid, 256, 0, hip_stream>>>(args);
   };
   if (a.value_stride == 64u)
     values(std::integral_constant<int, 4>{});
@@ -1601,7 +1635,8 @@ extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* a
     values(std::integral_constant<int, 8>{});
   else
     values(std::integral_constant<int, 16>{});
-  split_combine_kernel<uint16_t>
-      <<<dim3(a.query_heads, launch->rows), 64, 0, hip_stream>>>(args);
+  if (!whole)
+    split_combine_kernel<uint16_t>
+        <<<dim3(a.query_heads, launch->rows), 64, 0, hip_stream>>>(args);
   return launched("windowed split attention");
 }

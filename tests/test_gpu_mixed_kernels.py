@@ -374,6 +374,21 @@ def test_general_prompts_match_the_oracle(device, element, heads, kv, dim, vdim,
     close(layer.run(projections, 0), want, element)
 
 
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(16, 4, 128, 128), (6, 3, 64, 56),
+                                               (4, 1, 250, 230), (12, 2, 64, 64)])
+@pytest.mark.parametrize("keys", [256, 257, 511, 512, 513])   # tiles of eight waves, and past them
+def test_split_rows_at_the_edges_of_their_forms(device, heads, kv, dim, vdim, keys):
+    rng = np.random.default_rng(keys + heads)
+    scale = 1.0 / np.sqrt(dim)
+    mix = mm.bf16(np.eye(heads) + 0.2 * rng.standard_normal((heads, heads)))
+    layer = Attention(device, BF16, heads, kv, dim, vdim, 0, 0, mix, scale, context=576)
+    projections = mm.bf16(rng.standard_normal((keys, layer.stride)))
+    want = layer.expected(projections, 0, 0, mix.astype(np.float64), scale)
+    layer.run(projections[:keys - 5], 0)
+    close(layer.run(projections[keys - 5:keys - 1], keys - 5), want[keys - 5:keys - 1], BF16)
+    close(layer.run(projections[keys - 1:], keys - 1), want[keys - 1:], BF16)
+
+
 def stand_out(rng, layer, projections, pairs, head, strength=None):
     """Makes the score of (query row, key row) of one head stand out: the key
     becomes the query direction (unrotated dimensions or rotary 0 assumed)."""
