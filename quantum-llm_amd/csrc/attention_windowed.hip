@@ -543,6 +543,9 @@ __global__ __launch_bounds__(512) void general_scores_kernel(AttentionArgs args)
         maximum[head] = fresh;
       }
     }
+    // the next tile's lanes read what one lane of their half wave wrote here
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
   __syncthreads();
   for (uint32_t h = threadIdx.x; h < heads; h += blockDim.x) {

@@ -346,6 +346,28 @@ def test_general_splits_equal_a_workgroup_per_row(device, element, heads, kv, di
         close(again, whole[total - rows:], element)
 
 
+@pytest.mark.parametrize("element,heads,kv,dim,vdim,window", [
+    (F32, 5, 1, 40, 24, 0), (F32, 33, 3, 16, 16, 2400), (BF16, 34, 2, 32, 32, 0)])
+def test_general_splits_with_several_tiles_a_workgroup(device, element, heads, kv, dim, vdim,
+                                                       window):
+    """More tiles than score splits: a head's running maximum and sum pass from one
+    tile's lanes to the next one's.  Odd head counts leave half waves without a head."""
+    rng = np.random.default_rng(heads)
+    total, scale = 4200, 2.0 / np.sqrt(dim)      # 132 tiles in 64 splits
+    layer = Attention(device, element, heads, kv, dim, vdim, window, 3, None, scale,
+                      context=4224)
+    projections = mm.bf16(rng.standard_normal((total, layer.stride)))
+    # maxima that grow from tile to tile, and one that comes first
+    keys = slice(heads * dim, (heads + kv) * dim)
+    projections[:, keys] *= np.linspace(0.25, 1.5, total)[:, None]
+    projections[64, keys] *= 4.0
+    projections = mm.bf16(projections)
+    whole = layer.run(projections, 0)
+    for rows in (1, 4):
+        again = layer.run(projections[total - rows:], total - rows)
+        close(again, whole[total - rows:], element)
+
+
 @pytest.mark.parametrize("element", [F32, BF16])
 @pytest.mark.parametrize("heads,kv,dim,vdim,window,sinks,mixed,rows", [
     (16, 4, 112, 144, 100, 5, True, 530),     # three rows a workgroup
