@@ -2605,8 +2605,11 @@ extern "C" int32_t qllm_quantize_gqa_queries_q8(
   return launched("GQA query Q8 quantization");
 }
 
-extern "C" int32_t qllm_attention_paged_q4h_batched(
-    const qllm_q4h_attention_launch* launch, uint32_t batch_rows) {
+namespace {
+
+// any_order: workgroups may deal a batch's tiles otherwise than a launch of its own
+int32_t attend_batches(const qllm_q4h_attention_launch* launch, uint32_t batch_rows,
+                       bool any_order) {
   if (!launch || !launch->query || !launch->page_table || !launch->output ||
       (reinterpret_cast<uintptr_t>(launch->query) & 15u) ||
       launch->query_stride % 4u || !launch->partial_maxima ||
@@ -2670,7 +2673,7 @@ extern "C" int32_t qllm_attention_paged_q4h_batched(
   // over 4640 tokens (512, 66) 171 us against 220.
   const uint64_t middle = uint64_t{launch->first_context_tokens} + launch->rows / 2u;
   int32_t status = QLLM_OK;
-  if (launch->head_dim == 256u && row_tiles == 2u &&
+  if (any_order && launch->head_dim == 256u && row_tiles == 2u &&
       uint64_t{grid.x} * grid.y * grid.z >= 768u && middle <= uint64_t{splits} * 48u * 64u) {
     q4h_attention_split_kernel<256, 2, false, 2><<<grid, 128, 0, stream>>>(args);
     status = launched("Q4H attention split");
@@ -2686,6 +2689,18 @@ extern "C" int32_t qllm_attention_paged_q4h_batched(
       launch->output, launch->output_kind, launch->first_context_tokens,
       launch->maximum_splits, launch->split_tokens, launch->rows,
       launch->query_heads, launch->head_dim, nullptr, stream);
+}
+
+}  // namespace
+
+extern "C" int32_t qllm_attention_paged_q4h_batched(
+    const qllm_q4h_attention_launch* launch, uint32_t batch_rows) {
+  return attend_batches(launch, batch_rows, false);
+}
+
+extern "C" int32_t qllm_attention_paged_q4h_batched_any_order(
+    const qllm_q4h_attention_launch* launch, uint32_t batch_rows) {
+  return attend_batches(launch, batch_rows, true);
 }
 
 extern "C" int32_t qllm_attention_paged_q4h_prompt(

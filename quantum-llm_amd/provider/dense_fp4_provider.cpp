@@ -1837,7 +1837,7 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
           } else {
             launch.maximum_splits = prefill_splits_for(rows, attention_batch);
             status_check(
-                qllm_attention_paged_q4h_batched(&launch, attention_batch));
+                qllm_attention_paged_q4h_batched_any_order(&launch, attention_batch));
           }
         } else {
           const std::uint32_t query_stride =

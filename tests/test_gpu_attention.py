@@ -221,8 +221,10 @@ def test_batched_launch_equals_one_launch_per_batch(device, total, first, Q, KV,
     (93, 70, 16, 8, 16, 16),    # splits without a tile
     (120, 1000, 12, 2, 5, 16)])
 def test_large_batched_launches_of_256_dimensions(device, total, first, Q, KV, batch, splits):
-    """Workgroups of two waves: the oracle's attention, and up to the rounding of
-    the probabilities what launches of a batch each compute."""
+    """Batches enough for workgroups of two waves: the launch that is free in its
+    order takes them and gives the oracle's attention and, up to the rounding of the
+    probabilities, what launches of a batch each compute; the other one gives those
+    bit for bit."""
     rng = np.random.default_rng(total)
     d, page_tokens, tokens = 256, 64, first + total - 1
     keys = rng.standard_normal((tokens, KV, d)).astype(np.float32)
@@ -243,7 +245,13 @@ def test_large_batched_launches_of_256_dimensions(device, total, first, Q, KV, b
         qh.OUT_F32, None)
     qh.call("qllm_attention_paged_q4h_batched", launch, batch)
     torch.cuda.synchronize()
+    exact_order = out.cpu().numpy()
+    out.fill_(float("nan"))
+    qh.call("qllm_attention_paged_q4h_batched_any_order", launch, batch)
+    torch.cuda.synchronize()
     got = out.cpu().numpy()
+    if splits == 1:   # (waves of one tile each merge to the same bits)
+        assert not np.array_equal(got, exact_order)
     shape = ol.AttentionShape(total, Q, KV, d, first, page_tokens, 0, 1)
     gu.assert_close(got, ol.attention_q4h(shape, query, pages, "f64"), what="batched attention")
     # (binary16 probabilities are rounded relative to each wave's running maximum)
@@ -253,6 +261,7 @@ def test_large_batched_launches_of_256_dimensions(device, total, first, Q, KV, b
                                   first + row, page_tokens, 0, 1, balanced_splits=splits)
         gu.assert_close(got[row:row + rows], single, rtol=3e-3, atol=3e-4,
                         what="batched vs single")
+        assert np.array_equal(exact_order[row:row + rows], single), row
 
 
 @pytest.mark.parametrize("total,first,Q,KV,gated,batch,splits", [
