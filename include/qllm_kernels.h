@@ -287,12 +287,16 @@ int32_t qllm_fp4_gemm_bf16_tall_split(const qllm_fp4_matrix* matrix,
                                       uint32_t segment_count, uint32_t batch,
                                       void* stream);
 
-/* The three with a workspace (16-byte aligned, at least
- * qllm_fp4_tall_workspace_bytes()) in which a launch may leave parts of its sums:
- * a batch whose tiles are too few for the GPU is cut along K over more
- * workgroups, and a second launch adds the parts in order and does the epilogue.
+/* The three with a workspace (16-byte aligned) in which a launch may leave parts of
+ * its sums: a batch whose tiles are too few for the GPU is cut along K over more
+ * workgroups, and a second launch adds the parts in order and does the epilogue.  No
+ * launch has a use for more than qllm_fp4_tall_workspace_bytes(), those over one
+ * matrix (swiglu: gate and up of its shape) with 1 .. batch rows none for more than
+ * qllm_fp4_tall_parts_bytes(); with less it is cut less.
  * NULL: one launch, as above. */
 size_t qllm_fp4_tall_workspace_bytes(void);
+size_t qllm_fp4_tall_parts_bytes(const qllm_fp4_matrix* matrix, int32_t swiglu,
+                                 uint32_t batch);
 int32_t qllm_fp4_gemm_bf16_tall_cut(const qllm_fp4_matrix* matrix, const void* input,
                                     size_t input_bytes, void* output,
                                     uint32_t output_kind, const float* residual,
@@ -312,7 +316,7 @@ int32_t qllm_fp4_gemm_bf16_tall_split_cut(const qllm_fp4_matrix* matrix,
 /* The parts alone, F32 [parts][batch][rows], for a norm that adds them
  * (qllm_rms_norm_residual_batch); parts: 1 .. 16 and at most padded_columns / 64.
  * qllm_fp4_tall_parts: into how many a batch is best cut (1 = not at all); their
- * bytes are at most qllm_fp4_tall_workspace_bytes() where that is more than 1. */
+ * bytes are at most qllm_fp4_tall_parts_bytes() where that is more than 1. */
 uint32_t qllm_fp4_tall_parts(const qllm_fp4_matrix* matrix, uint32_t batch);
 int32_t qllm_fp4_gemm_bf16_tall_partial(const qllm_fp4_matrix* matrix, const void* input,
                                         size_t input_bytes, float* partials,

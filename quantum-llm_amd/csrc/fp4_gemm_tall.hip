@@ -35,6 +35,7 @@
 //    2^-11 in that weight).  Checkpoint scales lie well inside.
 #include "common.hpp"
 
+#include <algorithm>
 #include <iterator>
 #include <type_traits>
 
@@ -940,6 +941,28 @@ extern "C" uint32_t qllm_fp4_tall_parts(const qllm_fp4_matrix* matrix, uint32_t 
   if (!tall_matrix_ok(matrix) || !batch) return 1u;
   return plan_tall(matrix->rows, matrix->padded_columns, batch, matrix->scale_scheme,
                    false, false, kPartsBytes).splits;
+}
+
+extern "C" size_t qllm_fp4_tall_parts_bytes(const qllm_fp4_matrix* matrix, int32_t swiglu,
+                                            uint32_t batch) {
+  if (!tall_matrix_ok(matrix)) return 0u;
+  const uint32_t rows = matrix->rows;
+  size_t most = 0;
+  // Within 16 batch rows the workgroups of every height stay the same in number and a
+  // row makes the parts cost more, so the first row of 16 asks for the most parts.
+  for (uint64_t first = 1u; first <= batch; first += 16u) {
+    const uint32_t row = static_cast<uint32_t>(first);
+    if (parts_bytes(rows, row, 2u, swiglu) > kPartsBytes) break;
+    const uint32_t last = static_cast<uint32_t>(std::min<uint64_t>(first + 15u, batch));
+    for (const bool separate : {true, false}) {
+      if (!separate && swiglu) continue;
+      const TallPlan plan = plan_tall(rows, matrix->padded_columns, row,
+                                      matrix->scale_scheme, swiglu, separate, kPartsBytes);
+      most = std::max(most, std::min(parts_bytes(rows, last, plan.splits, swiglu),
+                                     kPartsBytes));
+    }
+  }
+  return most;
 }
 
 extern "C" int32_t qllm_fp4_gemm_bf16_tall_partial(const qllm_fp4_matrix* matrix,

@@ -678,6 +678,8 @@ er::PrepareOperationResult Mi355DenseFp4Provider::prepare(
       layer.qkv = concatenate_rows({query, key, value});
       require_shape(layer.output, g_.hidden, g_.query_heads * g_.head_dim,
                     "output_projection");
+      note_prompt_parts(layer.qkv);
+      note_prompt_parts(layer.output);
       if (g_.qk_norm) {
         layer.query_norm =
             upload_f32(tensor_for(context.tensors, "query_norm"), g_.head_dim);
@@ -703,6 +705,8 @@ er::PrepareOperationResult Mi355DenseFp4Provider::prepare(
       require_shape(layer.gate, g_.intermediate, g_.hidden, "gate_projection");
       require_shape(layer.up, g_.intermediate, g_.hidden, "up_projection");
       require_shape(layer.down, g_.hidden, g_.intermediate, "down_projection");
+      note_prompt_parts(layer.gate, true);
+      note_prompt_parts(layer.down);
       prepared->kind = PreparedOperation::Kind::ffn;
       prepared->layer = ffn_ops_;
       ++ffn_ops_;
@@ -793,6 +797,8 @@ void Mi355DenseFp4Provider::prepare_mtp(
   require_shape(value, g_.kv_heads * g_.head_dim, g_.hidden,
                 "layer.0.value_projection");
   layer.qkv = concatenate_rows({query, key, value});
+  note_prompt_parts(mtp_.fusion);
+  note_prompt_parts(layer.qkv);
   layer.output =
       upload_matrix(tensor_for(tensors, "layer.0.output_projection"), true);
   require_shape(layer.output, g_.hidden, g_.query_heads * g_.head_dim,
@@ -1617,14 +1623,28 @@ void Mi355DenseFp4Provider::enqueue_mtp_prefill(
   // MLP would compute.
 }
 
+// Room for the parts of a projection's launches over prompts, when it is loaded.
+void Mi355DenseFp4Provider::note_prompt_parts(const DeviceFp4Matrix& matrix, bool swiglu) {
+  const auto& descriptor = matrix.descriptor;
+  if (!noted_parts_.insert({descriptor.rows, descriptor.padded_columns,
+                            descriptor.scale_scheme, swiglu ? 1U : 0U}).second)
+    return;
+  wanted_parts_bytes_ = std::max(
+      wanted_parts_bytes_,
+      qllm_fp4_tall_parts_bytes(&descriptor, swiglu,
+                                std::min(prefill_chunk_rows(), g_.max_context)));
+}
+
 // The buffers of a prompt pass of up to `rows` rows.  A longer prompt than any
 // before replaces them by larger ones (the stream is idle between prefills).
 void Mi355DenseFp4Provider::ensure_prefill_workspace(std::uint32_t rows) {
-  if (rows <= prefill_rows_) return;
+  if (rows <= prefill_rows_ && wanted_parts_bytes_ <= prefill_parts_bytes_) return;
+  rows = std::max(rows, prefill_rows_);
   const auto release = [this] {
     for (void* pointer : prefill_allocations_) (void)hipFree(pointer);
     prefill_allocations_.clear();
     prefill_rows_ = 0U;
+    prefill_parts_bytes_ = 0U;
   };
   if (prefill_rows_) {
     hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream_)),
@@ -1657,8 +1677,9 @@ void Mi355DenseFp4Provider::ensure_prefill_workspace(std::uint32_t rows) {
       allocate(n * g_.query_heads * g_.head_dim * 2U));
   prefill_embedding_ = static_cast<float*>(allocate(n * g_.hidden * 4U));
   prefill_rope_table_ = static_cast<float*>(allocate(n * g_.rotary_dim * 4U));
-  prefill_parts_bytes_ = qllm_fp4_tall_workspace_bytes();
-  prefill_parts_ = static_cast<float*>(allocate(prefill_parts_bytes_));
+  prefill_parts_ = static_cast<float*>(
+      allocate(std::max<std::size_t>(wanted_parts_bytes_, 16U)));
+  prefill_parts_bytes_ = wanted_parts_bytes_;
   // the MLP's activation; the proposer's fusion input [rows, 2 hidden] too
   prefill_activation_ = static_cast<std::uint16_t*>(allocate(
       n * std::max<std::size_t>(g_.intermediate, 2U * g_.hidden) * 2U));
@@ -1775,7 +1796,8 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
             norm_follows && rows <= 65535U && g_.hidden <= 16384U
                 ? qllm_fp4_tall_parts(&matrix, rows)
                 : 1U;
-        if (cut > 1U) {
+        if (cut > 1U &&
+            std::size_t{cut} * rows * g_.hidden * 4U <= prefill_parts_bytes_) {
           status_check(qllm_fp4_gemm_bf16_tall_partial(
               &matrix, input, bytes, prefill_parts_, cut, rows, stream));
           parts = cut;

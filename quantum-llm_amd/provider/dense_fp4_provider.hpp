@@ -9,12 +9,14 @@
 // the gfx950 kernels of include/qllm_kernels.h on one HIP stream.
 #pragma once
 
+#include <array>
 #include <atomic>
 #include <cstdint>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <optional>
+#include <set>
 #include <span>
 #include <string>
 #include <vector>
@@ -375,6 +377,7 @@ class Mi355DenseFp4Provider final : public DecoderProvider {
                          const float* qkv_partials = nullptr,
                          std::uint32_t qkv_partial_count = 0U);
   // buffers for `rows` prompt rows at a time (allocated on first use)
+  void note_prompt_parts(const DeviceFp4Matrix& matrix, bool swiglu = false);
   void ensure_prefill_workspace(std::uint32_t rows);
   void enqueue_mtp(std::uint32_t rows, const float* previous_hidden,
                    bool produce_logits, std::uint32_t cache_position,
@@ -500,6 +503,8 @@ class Mi355DenseFp4Provider final : public DecoderProvider {
   float* prefill_rope_table_{};           // [rows, rotary_dim / 2] (cos, sin)
   float* prefill_parts_{};                // parts of projections cut along K
   std::size_t prefill_parts_bytes_{};
+  std::size_t wanted_parts_bytes_{};      // most that a prompt's projections leave
+  std::set<std::array<std::uint32_t, 4>> noted_parts_;   // shapes it was taken over
   // split partials of the batched prompt attention: [rows, splits, heads(, d)]
   std::uint32_t prefill_splits_{};
   float* prefill_partial_maxima_{};

@@ -2,6 +2,7 @@
 against the same prompt fed through the verify step's own row-batch pass."""
 import numpy as np
 import pytest
+import torch
 
 import oracle_lib as ol
 import qllm_provider as qp
@@ -170,4 +171,20 @@ def test_prefill_rejects_bad_prompts(device):
         provider.prefill(np.arange(200, dtype=np.uint32) % 7, 0)       # beyond the context
     with pytest.raises(qp.ProviderError, match="vocabulary"):
         provider.prefill(np.array([1, 99999], dtype=np.uint32), 0)
+    provider.close()
+
+
+def test_workspace_of_a_narrow_decoder_is_narrow(device):
+    """What the first prompt sets aside follows the decoder's widths and context: no
+    projection of this one is cut along K, so no parts are kept."""
+    rng, model, build = make("reference", 7, max_context=512)
+    provider = build()
+    provider.run_target(rng.integers(0, model.vocabulary, 5).astype(np.uint32), 0)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info(device)[0]
+    provider.prefill(rng.integers(0, model.vocabulary, 300).astype(np.uint32), 0)
+    torch.cuda.synchronize()
+    # 512 rows of 256 to 1024 floats a row in a dozen buffers, split partials of 300
+    # rows x 8 splits x 8 heads x 130 floats, whole allocation units
+    assert before - torch.cuda.mem_get_info(device)[0] < 64 << 20
     provider.close()
