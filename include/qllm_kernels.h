@@ -1020,6 +1020,9 @@ int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32_t count,
 #define QLLM_LINEAR_PART_ROWS 8192u
 uint32_t qllm_linear_parts(uint32_t rows, uint32_t columns, uint32_t batch,
                            uint32_t element);
+/* The most parts x rows it asks for with 65 .. batch rows; 0 = none is cut. */
+uint32_t qllm_linear_part_rows(uint32_t rows, uint32_t columns, uint32_t batch,
+                               uint32_t element);
 
 /* x[row] = table[token] * scale; a token outside the table gives zeros. */
 int32_t qllm_embedding_bf16_batch(const void* table_bf16, uint32_t vocabulary,

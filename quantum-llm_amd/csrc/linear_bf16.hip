@@ -693,6 +693,23 @@ extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32
               : launch_tall<false, 2, 4>(args, hip_stream);
 }
 
+extern "C" uint32_t qllm_linear_part_rows(uint32_t rows, uint32_t columns, uint32_t batch,
+                                          uint32_t element) {
+  uint32_t most = 0u;
+  // Within 64 batch rows the workgroups of every form stay the same in number and a row
+  // makes the parts cost more, so the first row of 64 asks for the most parts.
+  for (uint64_t first = 65u; first <= batch && 2u * first <= QLLM_LINEAR_PART_ROWS;
+       first += 64u) {
+    const uint32_t parts =
+        qllm_linear_parts(rows, columns, static_cast<uint32_t>(first), element);
+    const uint64_t last = std::min<uint64_t>(first + 63u, batch);
+    if (parts > 1u)
+      most = std::max(most, static_cast<uint32_t>(std::min<uint64_t>(
+                                parts * last, QLLM_LINEAR_PART_ROWS)));
+  }
+  return most;
+}
+
 extern "C" uint32_t qllm_linear_parts(uint32_t rows, uint32_t columns, uint32_t batch,
                                       uint32_t element) {
   const uint32_t steps = columns / 64u;

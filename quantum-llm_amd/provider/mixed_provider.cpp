@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <set>
 #include <stdexcept>
 
 namespace qllm {
@@ -768,14 +769,17 @@ void Mi355MixedProvider::ensure_workspace(std::uint32_t rows, std::uint32_t last
   std::size_t query_rank = 0U;
   std::size_t query_width = 0U;
   std::size_t partial_rows = 0U;
+  std::set<std::pair<std::uint32_t, std::uint32_t>> shapes;   // a model has few
   for (const auto& item : blocks_) {
     const Block& block = *item;
     partial_rows = std::max<std::size_t>(
         partial_rows, std::max(block.splits, block.down_splits) * kSmallBatch);
-    partial_rows = std::max<std::size_t>(
-        partial_rows,
-        std::max<std::size_t>(size, std::min<std::size_t>(std::size_t{16U} * size,
-                                                          QLLM_LINEAR_PART_ROWS)));
+    if (block.sandwich) partial_rows = std::max<std::size_t>(partial_rows, size);
+    for (const Matrix* matrix : {&block.output, &block.down})
+      if (matrix->rows && shapes.insert({matrix->rows, matrix->columns}).second)
+        partial_rows = std::max<std::size_t>(
+            partial_rows,
+            qllm_linear_part_rows(matrix->rows, matrix->columns, size, g_.element));
     if (block.kind == Kind::attention) {
       const auto& a = block.attention;
       query = std::max(query, std::size_t{a.query_heads} * a.key_stride);
@@ -802,6 +806,7 @@ void Mi355MixedProvider::ensure_workspace(std::uint32_t rows, std::uint32_t last
   shift_last_ = zeroed(std::size_t{round_up(g_.hidden, 4U)} * 4U, "allocate shifted row");
   partials_ = zeroed(partial_rows * round_up(g_.hidden, 4U) * 4U,
                      "allocate partial sums");
+  partial_rows_ = static_cast<std::uint32_t>(partial_rows);
   scratch_ = zeroed(scratch, "allocate mixer scratch");
   scratch_bytes_ = scratch;
   hip_check(hipDeviceSynchronize(), "clear workspace");
@@ -1075,9 +1080,9 @@ qllm_stream_norm_launch Mi355MixedProvider::stream_norm(std::uint32_t rows, floa
 // Parts of K of a projection onto the stream, which the next norm adds.
 std::uint32_t Mi355MixedProvider::parts_for(const Matrix& matrix, std::uint32_t few_rows,
                                             std::uint32_t rows) const {
-  return rows <= kSmallBatch ? few_rows
-                             : qllm_linear_parts(matrix.rows, matrix.columns, rows,
-                                                 g_.element);
+  if (rows <= kSmallBatch) return few_rows;
+  return std::min(qllm_linear_parts(matrix.rows, matrix.columns, rows, g_.element),
+                  std::max(1U, partial_rows_ / rows));
 }
 
 // Mixer and feed-forward one after the other; each leaves its output as partial

@@ -220,7 +220,8 @@ class Mi355MixedProvider final : public DecoderProvider {
   DeviceBuffer queries_;         // F32, from query latents
   DeviceBuffer kept_values_;
   DeviceBuffer shift_last_;
-  DeviceBuffer partials_;
+  DeviceBuffer partials_;          // [partial_rows_, hidden padded to 4]
+  std::uint32_t partial_rows_{};
   DeviceBuffer scratch_;         // attention splits, recurrence preparation
   std::size_t scratch_bytes_{};
   DeviceBuffer head_input_;

@@ -279,6 +279,7 @@ SIGNATURES = {
     "qllm_linear_packed_bytes": (c_size_t, [c_uint32, c_uint32]),
     "qllm_linear_pack_strided": (c_int32, [c_void_p, c_uint32, c_uint32, c_uint64, c_uint64, c_void_p, c_uint32, c_uint32, c_uint32, c_uint32, c_void_p]),
     "qllm_linear_pack": (c_int32, [c_void_p, c_uint32, c_uint32, c_void_p, c_uint32, c_uint32, c_uint32, c_uint32, c_void_p]),
+    "qllm_linear_part_rows": (c_uint32, [c_uint32, c_uint32, c_uint32, c_uint32]),
     "qllm_linear_parts": (c_uint32, [c_uint32, c_uint32, c_uint32, c_uint32]),
     "qllm_linear_batch": (c_int32, [POINTER(LinearSegment), c_uint32, c_uint32, c_uint32, c_void_p]),
     "qllm_embedding_bf16_batch": (c_int32, [c_void_p, c_uint32, c_void_p, c_void_p, c_uint32, c_uint32, c_float, c_void_p]),

@@ -5,6 +5,7 @@ import os
 
 import numpy as np
 import pytest
+import torch
 
 import mixed_model as mm
 import mixer_oracle as mo
@@ -141,6 +142,24 @@ def test_long_decoding_lets_expired_pages_go(tmp_path):
         assert model.telemetry("provider_graph_launches") > 400
         model.end(request)
         model.close()
+
+
+def test_partial_sums_take_the_room_their_matrices_ask_for(tmp_path):
+    """Output launches of this model leave at most 1024 rows of parts at 512 tokens."""
+    config = mm.configuration(64, 2048, [mm.attention(4, 1, 32, 32, 200, 0)], [512])
+    path = mm.write_folder(tmp_path / "m", config, mm.random_weights(config, 2))
+    model = qp.Model(path, 1024, kv_page_tokens=64)
+    request = model.begin()
+    model.step(request, np.arange(5) % 64, [4])
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    model.step(request, np.arange(512) % 64, [511])
+    torch.cuda.synchronize()
+    # 8 MiB of parts (64 MiB, were every batch cut sixteen ways), 4 MiB a buffer of
+    # 512 rows of 2048 floats
+    assert before - torch.cuda.mem_get_info()[0] < 48 << 20
+    model.end(request)
+    model.close()
 
 
 def test_context_limit_and_bad_batches(mixed):

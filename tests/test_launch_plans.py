@@ -31,3 +31,20 @@ def test_parts_of_prompts_fit_what_is_set_aside(rows, padded, most, scheme):
             assert room <= max(needed * 1.35, 16 * 16 * 16 * rows)
     assert room <= most and (room > 0) == (most > 0)
     assert qh.call("qllm_fp4_tall_parts_bytes", m, 1, 40) <= 16 * 2 * 48 * rows * 4
+
+
+@pytest.mark.parametrize("element", [qh.ELEMENT_BF16, qh.ELEMENT_F32])
+@pytest.mark.parametrize("rows,columns", [(2048, 640), (2048, 7680), (4096, 16384), (512, 1024),
+                                          (16, 64), (5120, 5120)])
+def test_part_rows_of_linears_cover_what_is_advised(rows, columns, element):
+    needed = 0
+    for batch in range(65, 4200):
+        parts = qh.call("qllm_linear_parts", rows, columns, batch, element)
+        assert parts == 1 or parts * batch <= 8192
+        if parts > 1:
+            needed = max(needed, parts * batch)
+        if batch in (65, 100, 128, 512, 1000, 4199):
+            room = qh.call("qllm_linear_part_rows", rows, columns, batch, element)
+            # (asked for 64 rows at a time)
+            assert needed <= room <= max(needed * 1.35, 16 * 128)
+    assert qh.call("qllm_linear_part_rows", rows, columns, 64, element) == 0
