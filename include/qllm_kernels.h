@@ -322,6 +322,16 @@ int32_t qllm_fp4_gemm_bf16_tall_partial(const qllm_fp4_matrix* matrix, const voi
                                         size_t input_bytes, float* partials,
                                         uint32_t parts, uint32_t batch, void* stream);
 
+/* How a launch is laid out: batch and weight rows of a workgroup, parts of K. */
+typedef struct qllm_launch_layout {
+  uint32_t batch_rows, weight_rows, parts;
+} qllm_launch_layout;
+/* Of a tall launch over `matrix` (swiglu: and another of its shape) with that much
+ * workspace, or - parts not 0 - of a partial one with so many parts. */
+int32_t qllm_fp4_tall_layout(const qllm_fp4_matrix* matrix, int32_t swiglu, uint32_t batch,
+                             size_t workspace_bytes, uint32_t parts,
+                             qllm_launch_layout* layout);
+
 /* replaces fp4_embedding_batch (transformer_kernels.hpp:68-70).  A token
  * outside the matrix (tokens[r] >= rows; a device-side selection over logits
  * without a finite maximum yields 0xffffffff) reads nothing and gives a row of
@@ -1020,6 +1030,9 @@ int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32_t count,
 #define QLLM_LINEAR_PART_ROWS 8192u
 uint32_t qllm_linear_parts(uint32_t rows, uint32_t columns, uint32_t batch,
                            uint32_t element);
+/* Of a launch of these segments: `parts` are those of the first one. */
+int32_t qllm_linear_layout(const qllm_linear_segment* segments, uint32_t count,
+                           uint32_t batch, uint32_t element, qllm_launch_layout* layout);
 /* The most parts x rows it asks for with 65 .. batch rows; 0 = none is cut. */
 uint32_t qllm_linear_part_rows(uint32_t rows, uint32_t columns, uint32_t batch,
                                uint32_t element);

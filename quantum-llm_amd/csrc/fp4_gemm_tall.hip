@@ -943,6 +943,19 @@ extern "C" uint32_t qllm_fp4_tall_parts(const qllm_fp4_matrix* matrix, uint32_t 
                    false, false, kPartsBytes).splits;
 }
 
+extern "C" int32_t qllm_fp4_tall_layout(const qllm_fp4_matrix* matrix, int32_t swiglu,
+                                        uint32_t batch, size_t workspace_bytes,
+                                        uint32_t parts, qllm_launch_layout* layout) {
+  if (!tall_matrix_ok(matrix) || !batch || batch > (1u << 20) || parts > kMaximumParts ||
+      parts > matrix->padded_columns / kChunk || (parts && swiglu) || !layout)
+    return fail(QLLM_INVALID_ARGUMENT, "invalid tall FP4 GEMM layout");
+  const TallPlan plan =
+      plan_tall(matrix->rows, matrix->padded_columns, batch, matrix->scale_scheme, swiglu,
+                parts == 0u, workspace_bytes, parts);
+  *layout = {16u * plan.height, weight_rows_of(plan.height, swiglu), plan.splits};
+  return QLLM_OK;
+}
+
 extern "C" size_t qllm_fp4_tall_parts_bytes(const qllm_fp4_matrix* matrix, int32_t swiglu,
                                             uint32_t batch) {
   if (!tall_matrix_ok(matrix)) return 0u;

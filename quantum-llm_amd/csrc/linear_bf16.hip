@@ -644,12 +644,13 @@ extern "C" int32_t qllm_linear_pack_strided(const void* source_bf16, uint32_t ro
   return launched("linear pack");
 }
 
-extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32_t count,
-                                     uint32_t batch, uint32_t element, void* stream) {
+namespace {
+
+int32_t linear_arguments(const qllm_linear_segment* segments, uint32_t count,
+                         uint32_t batch, uint32_t element, LinearArgs& args) {
   if (!segments || !count || count > kMaximumSegments || !batch ||
       element > QLLM_ELEMENT_F32)
     return fail(QLLM_INVALID_ARGUMENT, "invalid linear batch");
-  LinearArgs args{};
   args.count = count;
   args.batch = batch;
   for (uint32_t i = 0; i < count; ++i) {
@@ -667,6 +668,37 @@ extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32
       return fail(QLLM_INVALID_ARGUMENT, "invalid linear segment");
     args.segment[i] = s;
   }
+  return QLLM_OK;
+}
+
+// batch rows of a workgroup of the form for up to 64
+uint32_t small_rows(uint32_t batch) { return batch <= 16u ? 16u : batch <= 32u ? 32u : 64u; }
+
+}  // namespace
+
+extern "C" int32_t qllm_linear_layout(const qllm_linear_segment* segments, uint32_t count,
+                                      uint32_t batch, uint32_t element,
+                                      qllm_launch_layout* layout) {
+  LinearArgs args{};
+  if (!layout) return fail(QLLM_INVALID_ARGUMENT, "invalid linear layout");
+  if (const int32_t status = linear_arguments(segments, count, batch, element, args))
+    return status;
+  const bool f32 = element == QLLM_ELEMENT_F32;
+  if (batch <= 64u) {
+    *layout = {small_rows(batch), 16u, parts_of(args.segment[0])};
+    return QLLM_OK;
+  }
+  const uint32_t form = tall_form(args, f32);
+  const TallForm& tile = f32 ? kTallFormsF32[form] : kTallForms[form];
+  *layout = {16u * tile.mt, 64u * tile.nt, parts_of(args.segment[0])};
+  return QLLM_OK;
+}
+
+extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32_t count,
+                                     uint32_t batch, uint32_t element, void* stream) {
+  LinearArgs args{};
+  if (const int32_t status = linear_arguments(segments, count, batch, element, args))
+    return status;
   const auto hip_stream = as_stream(stream);
   const bool f32 = element == QLLM_ELEMENT_F32;
   if (batch <= 64u) {
@@ -676,9 +708,9 @@ extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32
       const uint32_t tile_rows = s.epilogue == QLLM_LINEAR_GATED ? 32u : 16u;
       args.first_unit[i + 1] = args.first_unit[i] + s.rows / tile_rows * parts;
     }
-    if (batch <= 16u)
+    if (small_rows(batch) == 16u)
       f32 ? launch_small<true, 1>(args, hip_stream) : launch_small<false, 1>(args, hip_stream);
-    else if (batch <= 32u)
+    else if (small_rows(batch) == 32u)
       f32 ? launch_small<true, 2>(args, hip_stream) : launch_small<false, 2>(args, hip_stream);
     else
       f32 ? launch_small<true, 4>(args, hip_stream) : launch_small<false, 4>(args, hip_stream);

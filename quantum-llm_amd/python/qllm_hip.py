@@ -37,6 +37,10 @@ class Fp4Matrix(Structure):
                 ("layout", c_uint32), ("tile_rows", c_uint32)]
 
 
+class LaunchLayout(Structure):
+    _fields_ = [("batch_rows", c_uint32), ("weight_rows", c_uint32), ("parts", c_uint32)]
+
+
 class RolloutStep(Structure):
     _fields_ = [("next_token", c_void_p), ("draft_tokens", c_void_p),
                 ("capacity", c_uint32), ("rows", c_uint32),
@@ -205,6 +209,7 @@ SIGNATURES = {
     "qllm_fp4_gemm_bf16_tall": (c_int32, [POINTER(Fp4Matrix), c_void_p, c_size_t, c_void_p, c_uint32, c_void_p, c_uint32, c_void_p]),
     "qllm_fp4_swiglu_bf16_tall": (c_int32, [POINTER(Fp4Matrix), POINTER(Fp4Matrix), c_void_p, c_size_t, c_void_p, c_uint32, c_void_p]),
     "qllm_fp4_tall_workspace_bytes": (c_size_t, []),
+    "qllm_fp4_tall_layout": (c_int32, [POINTER(Fp4Matrix), c_int32, c_uint32, c_size_t, c_uint32, POINTER(LaunchLayout)]),
     "qllm_fp4_tall_parts_bytes": (c_size_t, [POINTER(Fp4Matrix), c_int32, c_uint32]),
     "qllm_fp4_tall_parts": (c_uint32, [POINTER(Fp4Matrix), c_uint32]),
     "qllm_fp4_gemm_bf16_tall_cut": (c_int32, [POINTER(Fp4Matrix), c_void_p, c_size_t, c_void_p, c_uint32, c_void_p, c_uint32, c_void_p, c_size_t, c_void_p]),
@@ -279,6 +284,7 @@ SIGNATURES = {
     "qllm_linear_packed_bytes": (c_size_t, [c_uint32, c_uint32]),
     "qllm_linear_pack_strided": (c_int32, [c_void_p, c_uint32, c_uint32, c_uint64, c_uint64, c_void_p, c_uint32, c_uint32, c_uint32, c_uint32, c_void_p]),
     "qllm_linear_pack": (c_int32, [c_void_p, c_uint32, c_uint32, c_void_p, c_uint32, c_uint32, c_uint32, c_uint32, c_void_p]),
+    "qllm_linear_layout": (c_int32, [POINTER(LinearSegment), c_uint32, c_uint32, c_uint32, POINTER(LaunchLayout)]),
     "qllm_linear_part_rows": (c_uint32, [c_uint32, c_uint32, c_uint32, c_uint32]),
     "qllm_linear_parts": (c_uint32, [c_uint32, c_uint32, c_uint32, c_uint32]),
     "qllm_linear_batch": (c_int32, [POINTER(LinearSegment), c_uint32, c_uint32, c_uint32, c_void_p]),

@@ -492,7 +492,7 @@ def test_fused_rotary_attention_equals_the_two_launches(device, tokens, rows, Q,
     assert not np.array_equal(plain_pages[-1], pages[-1])   # the batch was stored
 
 
-@pytest.mark.parametrize("rows,first", [(1, 0), (5, 61), (17, 4), (333, 190)])
+@pytest.mark.parametrize("rows,first", [(1, 0), (5, 61), (17, 4), (333, 190), (2060, 30)])
 @pytest.mark.parametrize("head_dim,rotary,heads,kv,gated,qk_norm,rounded", [
     (128, 128, 16, 4, False, False, 0), (128, 40, 6, 2, True, True, 1),
     (256, 64, 48, 4, True, True, 0), (256, 256, 2, 1, False, False, 0)])
@@ -500,8 +500,9 @@ def test_fused_rotary_attention_equals_the_two_launches(device, tokens, rows, Q,
 def test_rotary_and_store_from_a_table_equal_their_own_angles(
         device, rows, first, head_dim, rotary, heads, kv, gated, qk_norm, rounded, f16):
     """Queries, keys and page bytes bit for bit as from the launches that compute
-    cosine and sine themselves: one row and four rows a wave, last waves with fewer,
-    rows across pages, partners in the same lane and in others."""
+    cosine and sine themselves: one row and (from 16384 rows of heads on: 2060 rows of
+    8 and 20 heads of 128, 333 and more of 52 heads of 256) four rows a wave, last waves with
+    fewer, rows across pages, partners in the same lane and in others."""
     rng = np.random.default_rng(rows + rotary)
     page_tokens, layer, theta, eps = 64, 1, 1.0e6, 1.0e-6
     stride = head_dim * (2 if gated else 1)

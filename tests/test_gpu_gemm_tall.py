@@ -35,8 +35,9 @@ def tall(device, codes, scales, scheme, rows, padded, act, out_kind=qh.OUT_F32,
     (2048, 1024, 1024), (512, 8192, 130)])
 @pytest.mark.parametrize("scheme", [ol.SCALE_UE8M0_BLOCK32, ol.SCALE_F16_BLOCK16])
 def test_tall_gemm_matches_oracle(device, scheme, rows, padded, batch):
-    """Ragged shapes: batches that are no multiple of 128, weight rows that are
-    no multiple of 256 or 32, a single chunk of K."""
+    """Ragged shapes, in workgroups of 16, 48 and 64 batch rows: batches and weight
+    rows that are no multiple of theirs or of 32, a single chunk of K.  (Larger
+    batches: test_every_layout_matches_the_product.)"""
     rng = np.random.default_rng(rows + batch)
     codes, scales = synth.fp4_matrix(rng, rows, padded, scheme)
     act = ol.bf16_round(rng.standard_normal((batch, padded)).astype(np.float32))
@@ -181,9 +182,10 @@ def test_tall_gemm_rejects_row_major(device):
     (160, 1024, 49), (2048, 2112, 97)])
 @pytest.mark.parametrize("scheme", [ol.SCALE_UE8M0_BLOCK32, ol.SCALE_F16_BLOCK16])
 def test_launches_cut_along_k_match_the_oracle(device, scheme, rows, padded, batch):
-    """Workgroup heights at their edges (1, 16 / 17, 32 / 33, 64 / 65 rows), parts
-    that share the chunks unevenly or hold one chunk each, ragged weight rows:
-    the forms with a workspace, every number of parts, and gate and up."""
+    """Workgroup heights at their edges (1, 16 / 17, 32 / 33, 64 / 65 rows) and
+    ragged weight rows through the forms with a workspace; parts that share the
+    chunks unevenly or hold one chunk each, every number of them; gate and up.
+    Matrices under 2^20 elements take one launch with a workspace too."""
     rng = np.random.default_rng(rows + batch)
     act = ol.bf16_round(rng.standard_normal((batch, padded)).astype(np.float32))
     d_act = gu.device_tensor(ol.bf16_bits(act), device)
@@ -228,7 +230,8 @@ def test_launches_cut_along_k_match_the_oracle(device, scheme, rows, padded, bat
                 qh.ptr(workspace), size, None)
         got = torch.cat(parts, dim=1).cpu().numpy()
         assert np.abs(got - wants[0]).max() < bound
-    assert 1 <= qh.call("qllm_fp4_tall_parts", matrices[0], batch) <= 16
+    advised = qh.call("qllm_fp4_tall_parts", matrices[0], batch)
+    assert (advised > 1) == (rows * padded >= 1 << 20) and advised <= 16
     for count in range(1, min(16, padded // 64) + 1):
         sums = torch.full((count, batch, rows), np.nan, device=device)
         qh.call("qllm_fp4_gemm_bf16_tall_partial", matrices[0], qh.ptr(d_act),
@@ -238,3 +241,110 @@ def test_launches_cut_along_k_match_the_oracle(device, scheme, rows, padded, bat
         with pytest.raises(qh.QllmError, match="invalid partial"):
             qh.call("qllm_fp4_gemm_bf16_tall_partial", matrices[0], qh.ptr(d_act),
                     d_act.numel() * 2, qh.ptr(workspace), count, batch, None)
+
+
+UE8M0, F16 = ol.SCALE_UE8M0_BLOCK32, ol.SCALE_F16_BLOCK16
+
+
+# (batch rows of a workgroup, whether K is cut) of a plain and of a gate-and-up launch
+@pytest.mark.parametrize("scheme,rows,padded,batch,plain,swiglu", [
+    (UE8M0, 2100, 8896, 1000, (128, True), (48, True)),
+    (UE8M0, 2112, 8896, 1000, (128, True), (48, True)),
+    (F16, 2100, 8896, 1000, (128, True), (128, True)),
+    (F16, 1088, 11200, 1500, (128, True), (128, True)),
+    (UE8M0, 1088, 11200, 900, (64, True), (128, True)),
+    (UE8M0, 5092, 128, 3001, (128, False), (128, False)),
+    (F16, 5092, 128, 3001, (128, False), (128, False)),
+    (UE8M0, 5120, 64, 3001, (128, False), (128, False)),
+    (UE8M0, 3072, 64, 500, (64, False), (64, False)),
+    (F16, 3072, 64, 500, (64, False), (64, False)),
+    (UE8M0, 3072, 2048, 100, (64, True), (64, True)),
+    (F16, 1536, 4096, 100, (64, True), (64, True)),
+    (UE8M0, 1100, 2112, 100, (48, True), (48, True)),
+    (F16, 1100, 2112, 48, (48, True), (48, True)),
+    (F16, 1088, 2112, 33, (48, True), (48, True)),
+    (UE8M0, 1100, 2112, 20, (32, True), (32, True)),
+    (F16, 1100, 2112, 20, (32, True), (32, True)),
+    (F16, 1088, 2112, 16, (16, True), (16, True))])
+def test_every_layout_matches_the_product(device, scheme, rows, padded, batch, plain, swiglu):
+    """Every height of a workgroup, whole and cut along K, against the product in 64
+    bits: weight rows and batches that end inside a workgroup, every output kind,
+    a residual that is the output, segments of different kinds, gate and up."""
+    rng = np.random.default_rng(rows + batch)
+    act = ol.bf16_round(rng.standard_normal((batch, padded)).astype(np.float32))
+    d_act = gu.device_tensor(ol.bf16_bits(act), device)
+    act64 = torch.from_numpy(act).to(device, torch.float64)
+    matrices, wants, keep = [], [], []
+    for _ in range(2):
+        codes, scales = synth.fp4_matrix(rng, rows, padded, scheme)
+        values = torch.from_numpy(synth.dequantize(codes, scales, scheme)).to(device)
+        wants.append((act64 @ values.T).cpu().numpy())
+        tensors = gu.device_tensor(codes, device), gu.device_tensor(scales, device)
+        matrix, kept = qh.prepack(qh.fp4_matrix(*tensors, rows, padded, padded, scheme),
+                                  device)
+        matrices.append(matrix)
+        keep.append((tensors, kept))
+    del values
+    want = wants[0]
+    size = qh.call("qllm_fp4_tall_workspace_bytes")
+    workspace = torch.full((size // 4,), float("nan"), device=device)   # parts are written first
+
+    def layout(gate_and_up, parts=0):
+        found = qh.LaunchLayout()
+        qh.call("qllm_fp4_tall_layout", matrices[0], gate_and_up, batch, size, parts,
+                ctypes.byref(found))
+        return found.batch_rows, found.parts
+
+    own = layout(0)[1]
+    assert [(height, parts > 1) for height, parts in (layout(0), layout(1))] == [plain, swiglu]
+    # F32 sums of `padded` exact products, in any order
+    bound = 2e-6 * np.sqrt(padded) * np.abs(want).max()
+
+    def run(kind, residual=None, in_place=False):
+        out = torch.full((batch, rows), float("nan"), device=device,
+                         dtype=torch.bfloat16 if kind == qh.OUT_BF16 else torch.float32)
+        if in_place:
+            out.copy_(residual)
+            residual = out
+        qh.call("qllm_fp4_gemm_bf16_tall_cut", matrices[0], qh.ptr(d_act),
+                d_act.numel() * 2, qh.ptr(out), kind, qh.ptr(residual), batch,
+                qh.ptr(workspace), size, None)
+        return out.double().cpu().numpy()
+
+    rest = torch.from_numpy(rng.standard_normal((batch, rows)).astype(np.float32)).to(device)
+    rest64 = rest.double().cpu().numpy()
+    assert np.abs(run(qh.OUT_F32) - want).max() < bound
+    sums = run(qh.OUT_F32, rest)
+    assert np.abs(sums - rest64 - want).max() < bound + 1e-6
+    assert np.array_equal(run(qh.OUT_F32, rest, in_place=True), sums)
+    rounded = run(qh.OUT_F32_BF16_ROUNDED)
+    assert np.array_equal(run(qh.OUT_BF16), rounded)
+    assert (np.abs(rounded - want) <= 2.0 ** -8 * np.abs(want) + 1.01 * bound).all()
+    if rows % 32 == 0:
+        widths, kinds = (64, 32, rows - 96), (qh.OUT_F32, qh.OUT_BF16,
+                                              qh.OUT_F32_BF16_ROUNDED)
+        outs = [torch.full((batch, n), float("nan"), device=device,
+                           dtype=torch.bfloat16 if k == qh.OUT_BF16 else torch.float32)
+                for n, k in zip(widths, kinds)]
+        segments = (qh.GemmSegment * 3)(*[qh.GemmSegment(qh.ptr(o), n, k)
+                                          for o, n, k in zip(outs, widths, kinds)])
+        qh.call("qllm_fp4_gemm_bf16_tall_split_cut", matrices[0], qh.ptr(d_act),
+                d_act.numel() * 2, ctypes.addressof(segments), 3, batch,
+                qh.ptr(workspace), size, None)
+        got = np.concatenate([o.double().cpu().numpy() for o in outs], axis=1)
+        assert np.array_equal(got[:, 64:], rounded[:, 64:])
+        assert np.array_equal(got[:, :64], run(qh.OUT_F32)[:, :64])
+    out = torch.full((batch, rows), float("nan"), dtype=torch.bfloat16, device=device)
+    qh.call("qllm_fp4_swiglu_bf16_tall_cut", matrices[0], matrices[1], qh.ptr(d_act),
+            d_act.numel() * 2, qh.ptr(out), batch, qh.ptr(workspace), size, None)
+    product = ol.silu_product(want, wants[1], True)
+    # two roundings to bf16 (the gate's SiLU, the product), each of which may fall
+    # to the neighbouring value, at most 2^-7 of it away
+    error = np.abs(out.double().cpu().numpy() - product)
+    assert (error <= 2.0 ** -6 * np.abs(product) + 4 * bound * (1 + np.abs(wants[1]))).all()
+    assert layout(0, own) == (plain[0], own)
+    for parts in {own, min(2, padded // 64)}:
+        sums = torch.full((parts, batch, rows), float("nan"), device=device)
+        qh.call("qllm_fp4_gemm_bf16_tall_partial", matrices[0], qh.ptr(d_act),
+                d_act.numel() * 2, qh.ptr(sums), parts, batch, None)
+        assert np.abs(sums.double().sum(0).cpu().numpy() - want).max() < bound

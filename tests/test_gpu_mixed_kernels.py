@@ -187,6 +187,8 @@ def test_linear_partials_of_tall_batches(device, element, rows, columns, batch):
 
 
 def test_linear_tall_tiles_of_all_sizes(device):
+    """Ragged tiles of 64 batch rows (the larger ones:
+    test_linear_tall_forms_of_every_epilogue)."""
     rng = np.random.default_rng(3)
     for rows, columns, batch in ((2100, 128, 700), (4096, 64, 1030), (300, 320, 129)):
         w = mm.bf16(rng.standard_normal((rows, columns)) / 12)
@@ -200,6 +202,62 @@ def test_linear_tall_tiles_of_all_sizes(device):
         qh.call("qllm_linear_batch", ctypes.byref(segment), 1, batch, BF16, None)
         torch.cuda.synchronize()
         close(out[:, :rows], x.astype(np.float64) @ w.T.astype(np.float64), F32)
+
+
+# (batch rows, weight rows) of a workgroup of a whole launch and of one in parts
+@pytest.mark.parametrize("element,rows,columns,batch,whole,parts,cut", [
+    (BF16, 2090, 192, 2900, (128, 128), 2, (128, 256)),
+    (BF16, 8170, 192, 1901, (128, 256), 5, (128, 256)),     # more parts than steps of K
+    (BF16, 4070, 320, 1000, (64, 128), 3, (128, 128)),
+    (BF16, 12270, 192, 333, (64, 128), 5, (128, 256)),
+    (F32, 2090, 192, 2900, (64, 256), 3, (64, 256)),
+    (F32, 12270, 192, 333, (64, 128), 2, (64, 256)),
+    (F32, 4070, 192, 70, (64, 128), 5, (64, 256))])
+def test_linear_tall_forms_of_every_epilogue(device, element, rows, columns, batch, whole,
+                                             parts, cut):
+    """Every form of the tall launch, with the epilogues of which a layer makes use:
+    rows and batches that end inside a workgroup, strides of no whole vectors."""
+    rng = np.random.default_rng(rows + batch)
+    w = mm.bf16(rng.standard_normal((rows, columns)) / np.sqrt(columns))
+    x = mm.bf16(rng.standard_normal((batch, columns)))
+    want = x.astype(np.float64) @ w.T.astype(np.float64)
+    weights, d_x = packed(device, [(w, 0, 1, 0)], rows, columns), padded_input(device, x,
+                                                                              columns, element)
+
+    def run(out, stride, epilogue, count, form, matrix=weights, height=rows, outputs=rows):
+        segment = qh.LinearSegment(qh.ptr(matrix), qh.ptr(d_x), qh.ptr(out),
+                                   padded(height, 16), columns, columns, stride, outputs,
+                                   epilogue, 0, count)
+        found = qh.LaunchLayout()
+        qh.call("qllm_linear_layout", ctypes.byref(segment), 1, batch, element,
+                ctypes.byref(found))
+        assert (found.batch_rows, found.weight_rows) == form
+        qh.call("qllm_linear_batch", ctypes.byref(segment), 1, batch, element, None)
+        torch.cuda.synchronize()
+
+    stride = padded(rows, 4)
+    out = torch.full((batch, stride), 7.0, device=device)
+    run(out, stride, qh.LINEAR_STORE, 0, whole)
+    close(out[:, :rows], want, F32, "store")
+    assert torch.all(out[:, rows:] == 7.0)
+    for stride in (padded(rows, 4), rows + 1):
+        base = rng.standard_normal((batch, stride)).astype(np.float32)
+        out = on(device, base)
+        run(out, stride, qh.LINEAR_ADD, 0, whole)
+        close(out[:, :rows], base[:, :rows] + want, F32, "add")
+        assert np.array_equal(out[:, rows:].cpu().numpy(), base[:, rows:])
+        out = torch.full((parts, batch, stride), 7.0, device=device)
+        run(out, stride, qh.LINEAR_PARTIALS, parts, cut)
+        close(out[:, :, :rows].double().sum(0), want, F32, "partials")
+        assert torch.all(out[:, :, rows:] == 7.0)
+    half = rows // 2
+    pair = packed(device, [(w[:half], 0, 2, 0), (w[half:2 * half], 1, 2, 0)],
+                  2 * padded(half, 16), columns)
+    out = torch.zeros((batch, padded(half, 4)), dtype=torch_type(element), device=device)
+    run(out, padded(half, 4), qh.LINEAR_GATED, 0, whole, pair, 2 * padded(half, 16), half)
+    gated = mo.gelu_tanh(want[:, :half]) * want[:, half:2 * half]
+    close(out[:, :half], gated, element, "gated")
+    assert torch.all(out[:, half:] == 0)
 
 
 # ---- stream ---------------------------------------------------------------------
