@@ -1021,7 +1021,8 @@ typedef struct qllm_linear_segment {
 /* Up to 8 segments in one launch, the same `batch` input rows for all of them.
  * bf16: up to 64 rows stream the weights once with K cut over a workgroup's
  * waves, more rows go through the tall tiles.  F32: the same, every input value
- * in three bf16 parts that hold all of it. */
+ * in three bf16 parts that hold all of it (of one below 2^-110, all but less than
+ * 2^-133). */
 int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32_t count,
                           uint32_t batch, uint32_t element, void* stream);
 /* Into how many parts a matrix alone in a launch of more than 64 rows is best cut

@@ -21,10 +21,11 @@
 //  * F32 mode runs on the same kernels: a 32-bit activation is the sum of three
 //    bf16 values (its 24 significant bits, eight at a time), their products with
 //    a bf16 weight are exact in 32 bits, and all three go into the same F32
-//    accumulator.  Nothing of the activation is lost; against 64 bits a product
-//    is 2 to 4 times closer than a chain of multiply-adds over K was (of
-//    [11264, 2048] 1.9e-7 up to 64 rows and 4.9e-7 above, 8.1e-7 before), and
-//    it takes 13 us for one row and 73 for 333 instead of 330 and 440.
+//    accumulator.  Down to 2^-110 nothing of the activation is lost; below, where
+//    the third part passes bf16's smallest step, what is lost is less than 2^-133.
+//    Against 64 bits a product is 2 to 4 times closer than a chain of multiply-adds
+//    over K was (of [11264, 2048] 1.9e-7 up to 64 rows and 4.9e-7 above, 8.1e-7
+//    before), and it takes 13 us for one row and 73 for 333 instead of 330 and 440.
 #include "common.hpp"
 #include "mixed_common.hpp"
 
@@ -107,8 +108,9 @@ struct Input<true> {
     return {vector[0], vector[1]};
   }
   // The upper 16 bits of x are its first eight significant bits, x minus those
-  // has sixteen left, and so on: every difference is exact.  An infinity is its
-  // first part alone; a NaN reaches the second one whatever its bits are.
+  // has sixteen left, and so on: every difference is exact, and with |x| >= 2^-110
+  // the last one is a bf16.  An infinity is its first part alone; a NaN reaches the
+  // second one whatever its bits are.
   static __device__ __forceinline__ void split(const Raw& raw, i32x4 (&out)[3]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

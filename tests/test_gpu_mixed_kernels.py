@@ -99,6 +99,29 @@ def test_linear_takes_all_bits_of_32_bit_inputs(device, batch):
         assert not np.delete(got, odd, axis=0).any()
 
 
+@pytest.mark.parametrize("batch", [16, 64, 200])
+def test_linear_takes_small_32_bit_inputs(device, batch):
+    """One input a row, weights of one: all of 24 significant bits from 2^-110 on,
+    below within bf16's smallest step."""
+    rng = np.random.default_rng(batch)
+    exponents = np.linspace(-149, -96, batch).astype(int)
+    values = ((1.0 + rng.integers(0, 1 << 23, batch) * 2.0 ** -23) *
+              np.exp2(exponents.astype(np.float64)) *
+              rng.choice([-1.0, 1.0], batch)).astype(np.float32)
+    x = np.zeros((batch, 64), dtype=np.float32)
+    x[np.arange(batch), np.arange(batch) % 64] = values
+    weights = packed(device, [(np.ones((16, 64), dtype=np.float32), 0, 1, 0)], 16, 64)
+    d_x = padded_input(device, x, 64, F32)
+    out = torch.zeros((batch, 16), device=device)
+    segment = qh.LinearSegment(qh.ptr(weights), qh.ptr(d_x), qh.ptr(out), 16, 64, 64, 16, 16,
+                               qh.LINEAR_STORE, 0, 0)
+    qh.call("qllm_linear_batch", ctypes.byref(segment), 1, batch, F32, None)
+    got = out.cpu().numpy().astype(np.float64)
+    error = np.abs(got - values[:, None].astype(np.float64))
+    assert not error[np.abs(values) >= 2.0 ** -110].any()
+    assert (error < 2.0 ** -133).all()
+
+
 @pytest.mark.parametrize("batch", [1, 16, 17, 33, 64, 65, 200])
 @pytest.mark.parametrize("epilogue", ["store", "gated"])
 def test_weights_that_are_no_numbers_meet_32_bit_inputs(device, batch, epilogue):
