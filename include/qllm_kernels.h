@@ -257,8 +257,8 @@ int32_t qllm_fp4_swiglu_bf16(const qllm_fp4_matrix* gate,
 /* The GEMM for tall batches (prompt prefill): any batch, a matrix in the tiled
  * layout with 32-row tiles, input bf16 [batch, padded_columns] (16-byte
  * aligned), output [batch, rows] in `output_kind`, optional F32 residual of
- * the same shape.  Workgroups of 16 to 128 batch rows x 256 weight rows on the
- * matrix cores.  With UE8M0 scales the arithmetic is the reference's (exact
+ * the same shape.  Workgroups of 16 to 64 batch rows x 128 weight rows or of 128 x
+ * 256 (gate and up: 128 of each matrix) on the matrix cores.  With UE8M0 scales the arithmetic is the reference's (exact
  * bf16 operands, F32 accumulation); with binary16 scales the scaled weights
  * and the activations enter as binary16 (see the kernel's header).
  * replaces fp4_gemm_bf16_block32 at batch > 8 (transformer_kernels.cu:

@@ -211,7 +211,8 @@ struct PartialTarget {
   uint32_t matrix_rows;    // rows * group
 };
 
-// Merges the wave states of a workgroup (of eight waves unless said otherwise) and writes the split partial.
+// Merges the wave states of a workgroup (of eight waves unless said otherwise) and
+// writes the split partial.
 // A wave's state: per row tile rt (16 matrix rows; lane (col = lane%16, quad =
 // lane/16) owns matrix row 16*rt + col) the running maximum (log2 units) and
 // sum, and out[dt][rt] = O^T elements d = 16*dt + 4*quad .. +3 of that row.
@@ -222,7 +223,7 @@ struct PartialTarget {
 //     LDS, lane-linear (no bank conflicts), and wave v adds up vectors v,
 //     v + WAVES, ... of all waves in a fixed order, owns them in the result and
 //     writes them out.
-// `pool` needs 8 KiB of LDS per wave, `summary` 512*RT bytes; both may
+// `pool` needs 8 KiB of LDS per wave, `summary` 512*RT bytes per wave; both may
 // overlap whatever the tile loop used (the function starts with a barrier).
 template <int D, int RT, int WAVES = kSplitWaves>
 __device__ __forceinline__ void merge_wave_states(

@@ -2665,12 +2665,12 @@ int32_t attend_batches(const qllm_q4h_attention_launch* launch, uint32_t batch_r
   // At head_dim 256 a workgroup of eight waves fills a compute unit's LDS, and its
   // prologue and the merge of its states, 20 us, stand between two workgroups; of two
   // waves three fit and hide each other's, but a tile costs them 1.03 us of the compute
-  // unit against 0.86.  24 heads on 4, five rows a batch: whole prompts of 960 / 3001
-  // rows (768 / 2404 workgroups, 8 / 24 tiles on average) 84 / 383 us with eight
-  // waves, 68 / 303 with two; 320 rows over 4320 tokens cut three ways (768, 22) 119
-  // and 101; 1000 rows over 9000 (800, 133) 512 and 603.  Where fewer workgroups than
-  // three a compute unit leave waves idle, eight share a context better: 640 rows
-  // over 4640 tokens (512, 66) 171 us against 220.
+  // unit against 0.86.  24 heads on 4, five rows a batch (no other geometry was timed):
+  // whole prompts of 960 / 3001 rows (768 / 2404 workgroups, 8 / 24 tiles on average)
+  // 84 / 383 us with eight waves, 68 / 303 with two; 320 rows over 4320 tokens cut
+  // three ways (768, 22) 119 and 101; 1000 rows over 9000 (800, 133) 512 and 603.
+  // Where fewer workgroups than three a compute unit leave waves idle, eight share a
+  // context better: 640 rows over 4640 tokens (512, 66) 171 us against 220.
   const uint64_t middle = uint64_t{launch->first_context_tokens} + launch->rows / 2u;
   int32_t status = QLLM_OK;
   if (any_order && launch->head_dim == 256u && row_tiles == 2u &&

@@ -1381,7 +1381,12 @@ uint32_t score_splits_for(uint32_t tiles) {
 // Up to two tiles a wave, one workgroup of eight waves per key/value head saves the
 // launch that adds the splits: one row of 16 heads on 4, 128 dimensions, 16.2 -> 13.6
 // us over 6 tiles, 16.5 -> 15.4 over 11 and 16.5 -> 16.1 over 16.  (More heads to a
-// key/value head want more registers than eight waves have.)
+// key/value head want more registers than eight waves have.)  `tiles` are the most
+// that a row up to the launch's maximum_position sees.  A captured step names the
+// model's last position there: it comes this way where the window and the kept
+// tokens, or the model's context, are within 16 tiles, however short the request is
+// so far.  (A turn of 100 + 32 tokens with a window of 1024: 8.01 ms in a model of 140
+// positions, 8.07 in one of 32768, whose tokens take the other launches.)
 bool whole_values(const Attention& a, uint32_t tiles) {
   return tiles <= 16u && a.query_heads / a.kv_heads <= 4u;
 }
@@ -1450,7 +1455,9 @@ int32_t launch_general(const AttentionArgs& base, hipStream_t stream) {
 
 // The general form's workgroups take a tile each where there is room: their scores
 // and values are plain multiply-adds, and 16 heads over 340 keys took 25 us of
-// scores two tiles a workgroup and 23 of values four, against 12 and 10.
+// scores two tiles a workgroup and 23 of values four, against 12 and 10.  (`tiles` as
+// above: workgroups past the request's last tile find nothing to do.  A 32-bit turn
+// of 333 + 8 tokens takes 3.30 ms in models of 349 and of 32768 positions.)
 uint32_t general_score_splits_for(uint32_t tiles) {
   return tiles < kMaximumScoreSplits ? tiles : kMaximumScoreSplits;
 }

@@ -744,9 +744,9 @@ bool tall_matrix_ok(const qllm_fp4_matrix* m) {
 // n * `shared` where workgroups hide each other's.  Parts are written and read
 // once more, at 6.2 TB/s, and take a launch of their own where no norm adds
 // them.  The constants are a fit to 1300 timed launches over weights that come
-// from memory (nine matrices of [2048, 2048] to [17408, 5120], 8 to 3000 rows;
-// 7 % root mean square error; the chosen layout is 1.5 % slower than the best of
-// those timed on average).  What it gives over one workgroup per 128 rows and
+// from memory (nine matrices of [2048, 2048] to [17408, 5120], 8 to 3000 rows,
+// heights 1, 2, 4 and 8; 7 % root mean square error; the chosen layout is 1.5 %
+// slower than the best of those timed on average).  What it gives over one workgroup per 128 rows and
 // tile: [5120, 17408] with binary16 scales, 48 rows 400 -> 27 us, 300 rows
 // 404 -> 97, 1000 rows 405 -> 254, 2000 rows 668 -> 498; [10240, 5120] 127 ->
 // 25, 135 -> 73, 211 -> 190, 333 -> 327; gate and up of [17408, 5120] 129 -> 54,
@@ -763,8 +763,9 @@ struct ChunkCost {
   float alone, shared;   // ns
 };
 constexpr uint32_t kHeights[] = {1u, 2u, 3u, 4u, 8u};
-// [scheme][SwiGLU][height]; 48 rows, which joined later, at the share of the 64-row
-// workgroup's cost that 48 rows of the 27B widths took (86 %)
+// [scheme][SwiGLU][height].  Those of 48 rows are no part of the fit: 86 % of the
+// 64-row workgroup's, the share that 48 rows of the 27B widths took; other widths
+// were not timed at that height.
 constexpr ChunkCost kChunkCost[2][2][5] = {
     {{{160.f, 150.f}, {195.f, 180.f}, {315.f, 215.f}, {365.f, 250.f}, {1160.f, 780.f}},
      {{250.f, 325.f}, {335.f, 345.f}, {520.f, 360.f}, {605.f, 420.f}, {1215.f, 780.f}}},
