@@ -1585,8 +1585,13 @@ extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* a
                   "windowed attention: heads and dimensions exceed the general kernel");
     // Up to the split form's rows a workgroup per row leaves the chip idle (one or
     // four rows over 340 keys: 84 us against 24); a caller that brought no workspace
-    // for the splits, and heads whose buffers pass 64 KiB, stay with it.
-    if (launch->rows <= kSplitRows && launch->workspace &&
+    // for the splits, and heads whose buffers pass 64 KiB, stay with it.  So do rows
+    // that see one tile, which leaves nothing to deal: three launches take 12 us for 5
+    // heads of 16 + 64 dimensions and 22 for 16 on 4 of 128 + 128, one 8.7 and 15.5;
+    // wide heads' chains are longer than the launches saved (8 of 256 + 256: 20 and 34).
+    const bool one_tile = maximum_tiles(a, launch->maximum_position) == 1u &&
+                          uint64_t{a.dim} + a.vdim <= 256u;
+    if (launch->rows <= kSplitRows && launch->workspace && !one_tile &&
         (reinterpret_cast<uintptr_t>(launch->workspace) & 15u) == 0u &&
         launch->workspace_bytes >= qllm_windowed_attention_workspace_bytes(
                                        attention, launch->rows, launch->maximum_position) &&

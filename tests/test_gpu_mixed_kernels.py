@@ -470,6 +470,25 @@ def test_general_splits_equal_a_workgroup_per_row(device, element, heads, kv, di
         close(again, whole[total - rows:], element)
 
 
+@pytest.mark.parametrize("element,heads,kv,dim,vdim", [
+    (F32, 5, 1, 16, 64), (F32, 16, 4, 128, 128), (F32, 4, 2, 128, 144), (BF16, 40, 2, 24, 32)])
+@pytest.mark.parametrize("keys", [4, 31, 32, 33, 64, 65])
+def test_general_rows_over_a_tile_or_two(device, element, heads, kv, dim, vdim, keys):
+    """A few rows at the edges between one launch and three: one visible tile, and
+    dimensions of 256 together."""
+    rng = np.random.default_rng(keys + heads)
+    scale = 1.0 / np.sqrt(dim)
+    mix = mm.bf16(np.eye(heads) + 0.2 * rng.standard_normal((heads, heads)))
+    layer = Attention(device, element, heads, kv, dim, vdim, 0, 0, mix, scale, context=128,
+                      strides=(padded(dim, 32), padded(vdim, 16)))
+    projections = mm.bf16(rng.standard_normal((keys, layer.stride)))
+    want = layer.expected(projections, 0, 0, mix.astype(np.float64), scale)
+    if keys > 4:
+        layer.run(projections[:keys - 4], 0)
+    close(layer.run(projections[keys - 4:], keys - 4), want[keys - 4:], element)
+    close(layer.run(projections[keys - 1:], keys - 1), want[keys - 1:], element)
+
+
 @pytest.mark.parametrize("element,heads,kv,dim,vdim,window", [
     (F32, 5, 1, 40, 24, 0), (F32, 33, 3, 16, 16, 2400), (BF16, 34, 2, 32, 32, 0)])
 def test_general_splits_with_several_tiles_a_workgroup(device, element, heads, kv, dim, vdim,
