@@ -122,20 +122,21 @@ def test_linear_takes_small_32_bit_inputs(device, batch):
     assert (error < 2.0 ** -133).all()
 
 
-@pytest.mark.parametrize("batch", [1, 16, 17, 33, 64, 65, 200])
+@pytest.mark.parametrize("batch", [1, 16, 17, 33, 64, 65, 200, 1000])
 @pytest.mark.parametrize("epilogue", ["store", "gated"])
 def test_weights_that_are_no_numbers_meet_32_bit_inputs(device, batch, epilogue):
     """Infinite and NaN weights give what a multiply-add gives, whichever parts of
     an input are zero: inputs of one, sixteen and 24 significant bits, zeros,
     infinities."""
     rng = np.random.default_rng(batch)
+    rows = 2112 if batch == 1000 else 64     # (the wider form of the tall launch)
     inputs = np.array([1.0, -1.5, 1.0 + 2.0 ** -15, 1.0 + 2.0 ** -23, -3.0e-30, 0.0, np.inf,
                        -np.inf], dtype=np.float32)
     x = np.zeros((batch, 192), dtype=np.float32)
     x[:, 7] = inputs[np.arange(batch) % len(inputs)]
     x[:, 100] = rng.standard_normal(batch)
-    matrix = mm.bf16(rng.standard_normal((64, 192)))
-    matrix[:, 7] = np.array([np.inf, -np.inf, np.nan, 0.5], dtype=np.float32)[np.arange(64) % 4]
+    matrix = mm.bf16(rng.standard_normal((rows, 192)))
+    matrix[:, 7] = np.resize(np.array([np.inf, -np.inf, np.nan, 0.5], dtype=np.float32), rows)
     x[:, 150] = 30.0     # the gate's input, and silu(30) is 30 in 32 bits
     d_x = padded_input(device, x, 192, F32)
     matrix[:, 150] = 0.0
@@ -143,19 +144,19 @@ def test_weights_that_are_no_numbers_meet_32_bit_inputs(device, batch, epilogue)
         products = [x[:, k, None].astype(np.float64) * matrix[:, k] for k in (7, 100)]
         want = products[0] + products[1]
     if epilogue == "store":
-        weights = packed(device, [(matrix, 0, 1, 0)], 64, 192)
-        out = torch.zeros((batch, 64), device=device)
-        segment = qh.LinearSegment(qh.ptr(weights), qh.ptr(d_x), qh.ptr(out), 64, 192, 192,
-                                   64, 64, qh.LINEAR_STORE, 0, 0)
+        weights = packed(device, [(matrix, 0, 1, 0)], rows, 192)
+        out = torch.zeros((batch, rows), device=device)
+        segment = qh.LinearSegment(qh.ptr(weights), qh.ptr(d_x), qh.ptr(out), rows, 192, 192,
+                                   rows, rows, qh.LINEAR_STORE, 0, 0)
     else:
-        gate = np.zeros((64, 192), dtype=np.float32)
+        gate = np.zeros((rows, 192), dtype=np.float32)
         gate[:, 150] = 1.0
         want, products = 30.0 * want, [30.0 * p for p in products]
         want[np.isinf(x[:, 7])] = np.nan      # meets the gate's zeros
-        weights = packed(device, [(gate, 0, 2, 0), (matrix, 1, 2, 0)], 128, 192)
-        out = torch.zeros((batch, 64), device=device)
-        segment = qh.LinearSegment(qh.ptr(weights), qh.ptr(d_x), qh.ptr(out), 128, 192, 192,
-                                   64, 64, qh.LINEAR_GATED, 1, 0)   # SiLU
+        weights = packed(device, [(gate, 0, 2, 0), (matrix, 1, 2, 0)], 2 * rows, 192)
+        out = torch.zeros((batch, rows), device=device)
+        segment = qh.LinearSegment(qh.ptr(weights), qh.ptr(d_x), qh.ptr(out), 2 * rows, 192,
+                                   192, rows, rows, qh.LINEAR_GATED, 1, 0)   # SiLU
     qh.call("qllm_linear_batch", ctypes.byref(segment), 1, batch, F32, None)
     got = out.cpu().numpy().astype(np.float64)
     finite = np.isfinite(want)
