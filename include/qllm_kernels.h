@@ -331,6 +331,10 @@ typedef struct qllm_launch_layout {
 int32_t qllm_fp4_tall_layout(const qllm_fp4_matrix* matrix, int32_t swiglu, uint32_t batch,
                              size_t workspace_bytes, uint32_t parts,
                              qllm_launch_layout* layout);
+/* Parts of each workgroup's tile past the last full round of the compute units, where
+ * the launch cuts only those; 0: it cuts all of them (layout.parts) or none. */
+uint32_t qllm_fp4_tall_tail_parts(const qllm_fp4_matrix* matrix, int32_t swiglu,
+                                  uint32_t batch, size_t workspace_bytes);
 
 /* replaces fp4_embedding_batch (transformer_kernels.hpp:68-70).  A token
  * outside the matrix (tokens[r] >= rows; a device-side selection over logits

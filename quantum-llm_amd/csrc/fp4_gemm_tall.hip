@@ -53,9 +53,14 @@ constexpr uint32_t kTilesPerWave = 2;    // 32-row weight tiles per wave
 constexpr uint32_t kTilesN = kWaves * kTilesPerWave;   // per workgroup
 constexpr uint32_t kTileRows = 32;
 constexpr uint32_t kBand = 8;            // activation tiles per band of the grid
-// LDS row of the activation tile: 64 values of 16 bits plus 16 bytes, so that
-// the sixteen rows a fragment load touches fall on different banks
-constexpr uint32_t kLdsRow = kChunk * 2u + 16u;
+constexpr uint32_t kLowestTail = 5;      // height from which on tiles may be cut alone
+// LDS row of the activation tile: 64 values of 16 bits in eight pieces, piece p of
+// row r at p ^ (r % 8), so that a fragment load meets no bank conflict (with rows
+// 16 bytes longer instead, every one of them cost four more cycles)
+constexpr uint32_t kLdsRow = kChunk * 2u;
+__device__ __forceinline__ uint32_t swizzled(uint32_t piece, uint32_t row) {
+  return (piece ^ (row % 8u)) * 16u;
+}
 
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
@@ -77,6 +82,11 @@ struct TallArgs {
   // the chunks into partials[p][batch][rows] (SWIGLU: partials[p][2][batch]
   // [rows], gate before up), and whoever reads them adds the parts in order
   uint32_t splits;
+  // With `cut` only the last tiles are cut: the first `whole` run whole, each of the
+  // others is `cut` pieces, whose accumulators go to partials as they stand in the
+  // registers ([piece][vector of a thread][thread]), for tall_tail_kernel
+  uint32_t whole;
+  uint32_t cut;
   float* partials;
   void* output;                  // [batch, rows]
   uint32_t output_kind;
@@ -93,6 +103,66 @@ struct TallArgs {
 __device__ __forceinline__ uint32_t xcd_contiguous(uint32_t id, uint32_t total) {
   const uint32_t xcd = id % 8u;
   return xcd * (total / 8u) + min(xcd, total % 8u) + id / 8u;
+}
+
+// What a workgroup does: chunks [first_chunk, end_chunk) of tile (m_tile, n_tile), as
+// part `part` of the launch or piece `piece` of a cut tile.
+struct Work {
+  uint32_t m_tile, n_tile;
+  uint32_t first_chunk, end_chunk;
+  uint32_t part, piece;
+  bool is_piece;
+};
+
+// Tiles go band by band (kBand activation tiles high), column by column: the 64
+// workgroups an XCD runs at a time then cover about 8 x 8 tiles and fetch 8 + 8
+// operand tiles per K step into its L2 rather than 64 + 1.
+__device__ __forceinline__ void place_tile(const TallArgs& args, uint32_t id,
+                                           uint32_t& m_tile, uint32_t& n_tile) {
+  const uint32_t band_tiles = kBand * args.n_tiles;
+  const uint32_t band = id / band_tiles;
+  const uint32_t in_band = id - band * band_tiles;
+  const uint32_t height = min(kBand, args.m_tiles - band * kBand);
+  m_tile = band * kBand + in_band % height;
+  n_tile = in_band / height;
+}
+
+// An XCD gets a contiguous range of a part's tiles, or - launches that may be TAILED -
+// of the whole tiles and then of the pieces.
+template <bool TAILED>
+__device__ __forceinline__ Work work_of(const TallArgs& args, uint32_t chunks) {
+  const uint32_t tiles = args.m_tiles * args.n_tiles;
+  Work work{};
+  uint32_t id, share = 0u, shares = 1u;
+  if constexpr (!TAILED) {
+    // (the low workgroups of short launches: no band is higher than the batch)
+    const uint32_t position = xcd_contiguous(blockIdx.x, tiles * args.splits);
+    work.part = position / tiles;
+    id = position - work.part * tiles;
+    work.n_tile = id / args.m_tiles;
+    work.m_tile = id - work.n_tile * args.m_tiles;
+    work.first_chunk = chunks * work.part / args.splits;
+    work.end_chunk = chunks * (work.part + 1u) / args.splits;
+    return work;
+  }
+  if (args.cut && blockIdx.x >= args.whole) {
+    work.is_piece = true;
+    work.piece = xcd_contiguous(blockIdx.x - args.whole, (tiles - args.whole) * args.cut);
+    id = args.whole + work.piece / args.cut;
+    share = work.piece % args.cut;
+    shares = args.cut;
+  } else if (args.cut) {
+    id = xcd_contiguous(blockIdx.x, args.whole);
+  } else {
+    const uint32_t position = xcd_contiguous(blockIdx.x, tiles * args.splits);
+    work.part = share = position / tiles;
+    id = position - share * tiles;
+    shares = args.splits;
+  }
+  work.first_chunk = chunks * share / shares;
+  work.end_chunk = chunks * (share + 1u) / shares;
+  place_tile(args, id, work.m_tile, work.n_tile);
+  return work;
 }
 
 __device__ __forceinline__ void store_value(void* output, uint32_t kind,
@@ -209,6 +279,29 @@ __device__ __forceinline__ uint16_t swiglu_bits(float gate, float up) {
   return static_cast<uint16_t>(f32_to_bf16_bits(activated * up));
 }
 
+// A piece's accumulators, vector q of thread i at ((piece Q + q) 256 + i) of
+// args.partials (Q vectors a thread).
+template <int MT, int T>
+__device__ __forceinline__ void store_piece(const TallArgs& args, uint32_t piece,
+                                            const f32x4 (&acc)[MT][T][2]) {
+  f32x4* target = reinterpret_cast<f32x4*>(args.partials) +
+                  static_cast<size_t>(piece) * (MT * T * 2u * kWaves * 64u) + threadIdx.x;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        target[((mt * T + t) * 2 + j) * (kWaves * 64u)] = acc[mt][t][j];
+}
+
+// The weight tiles of a wave: 32 rows of the gate matrix and the same of the up
+// matrix, or T tiles side by side.
+template <int T, bool SWIGLU>
+__device__ __forceinline__ uint32_t weight_tile(uint32_t n_tile, uint32_t wave, uint32_t t) {
+  return SWIGLU ? n_tile * kWaves + wave : (n_tile * kWaves + wave) * T + t;
+}
+
 // Stores a wave's accumulators.  D register i of lane (n, g): activation row
 // first_m + 16 mt + 4 g + i, weight row 32 tile + 16 j + n.
 template <int MT, int T, bool SWIGLU>
@@ -317,24 +410,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_tall_kernel(
   const uint32_t K = args.padded_columns;
   const uint32_t chunks = K / kChunk;
 
-  // An XCD gets a contiguous range of tiles.  Within the
-  // range the tiles go band by band (kBand activation tiles high), column by
-  // column: the 64 workgroups an XCD runs at a time then cover about 8 x 8
-  // tiles and fetch 8 + 8 operand tiles per K step into its L2 rather than
-  // 64 + 1.
-  const uint32_t tiles = args.m_tiles * args.n_tiles;
-  const uint32_t position = xcd_contiguous(blockIdx.x, tiles * args.splits);
-  const uint32_t part = position / tiles;
-  const uint32_t id = position - part * tiles;
-  const uint32_t first_chunk = chunks * part / args.splits;
-  const uint32_t end_chunk = chunks * (part + 1u) / args.splits;
-  const uint32_t band_tiles = kBand * args.n_tiles;
-  const uint32_t band = id / band_tiles;
-  const uint32_t in_band = id - band * band_tiles;
-  const uint32_t height = min(kBand, args.m_tiles - band * kBand);
-  const uint32_t m_tile = band * kBand + in_band % height;
-  const uint32_t n_tile = in_band / height;
-  const uint32_t first_m = m_tile * kRowsM;
+  const Work work = work_of<true>(args, chunks);
+  const uint32_t first_chunk = work.first_chunk;
+  const uint32_t end_chunk = work.end_chunk;
+  const uint32_t first_m = work.m_tile * kRowsM;
 
   // weight streams of this wave's tiles (tiles past the matrix repeat the last
   // one and are not stored)
@@ -344,8 +423,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_tall_kernel(
   uint32_t tile_index[kTilesPerWave];
 #pragma unroll
   for (uint32_t t = 0; t < kTilesPerWave; ++t) {
-    tile_index[t] = SWIGLU ? n_tile * kWaves + wave
-                           : n_tile * kTilesN + wave * kTilesPerWave + t;
+    tile_index[t] = weight_tile<kTilesPerWave, SWIGLU>(work.n_tile, wave, t);
     const size_t stream = min(tile_index[t], tile_count - 1u);
     weight_stream[t] = (SWIGLU && t ? args.up_weights : args.weights) +
                        stream * chunks * (kTileRows * 32u) + (g * 16u + n) * 16u;
@@ -365,9 +443,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_tall_kernel(
       reinterpret_cast<const uint8_t*>(args.activations) +
       (static_cast<size_t>(stage_live ? first_m + stage_row : 0u) * K +
        stage_half * 32u) * 2u;
-  const uint32_t stage_target = stage_row * kLdsRow + stage_half * 64u;
+  const uint32_t stage_target = stage_row * kLdsRow;
   // fragment of m-tile mt, span s: row 16 mt + n, columns 32 s + 8 g .. + 8
-  const uint32_t fragment_offset = n * kLdsRow + g * 16u;
+  const uint32_t fragment_offset[2] = {n * kLdsRow + swizzled(g, n),
+                                       n * kLdsRow + swizzled(g + 4u, n)};
 
   f32x4 acc[kTilesM][kTilesPerWave][2];
 #pragma unroll
@@ -390,7 +469,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_tall_kernel(
       uint4 v = staged[piece];
       v.x = Op::stage(v.x); v.y = Op::stage(v.y);
       v.z = Op::stage(v.z); v.w = Op::stage(v.w);
-      *reinterpret_cast<uint4*>(&tile[buffer][stage_target + piece * 16u]) = v;
+      *reinterpret_cast<uint4*>(
+          &tile[buffer][stage_target + swizzled(stage_half * 4u + piece, stage_row)]) = v;
     }
   };
   // (slot indices are compile-time constants throughout: an array indexed by a
@@ -437,7 +517,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_tall_kernel(
       for (uint32_t mt = 0; mt < kTilesM; ++mt)
         a[mt] = __builtin_bit_cast(
             Vector, *reinterpret_cast<const uint4*>(
-                        current + mt * 16u * kLdsRow + fragment_offset + s * 64u));
+                        current + mt * 16u * kLdsRow + fragment_offset[s]));
 #pragma unroll
       for (uint32_t t = 0; t < kTilesPerWave; ++t) {
         const uint4 q = codes[slot][t];
@@ -467,17 +547,25 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_tall_kernel(
     if (chunk + 1u < end_chunk) step(std::integral_constant<int, 1>{}, chunk + 1u);
   }
 
-  store_tiles<kTilesM, kTilesPerWave, SWIGLU>(args, part, first_m, tile_index,
-                                              tile_count, acc);
+  if (work.is_piece)
+    store_piece<kTilesM, kTilesPerWave>(args, work.piece, acc);
+  else
+    store_tiles<kTilesM, kTilesPerWave, SWIGLU>(args, work.part, first_m, tile_index,
+                                                tile_count, acc);
 }
 
-// Short batches: 16, 32, 48 or 64 rows a workgroup (16 MT), 128 weight rows (SWIGLU:
-// of each of the two matrices).  Here the weights' way from memory is what there is
-// to hide, not the matrix cores' time: a wave keeps its weights of the next four
-// chunks on their way in registers (with the one of fp4_gemm_tall_kernel a step
-// waits out most of a memory round trip), the activations of the next two steps
-// likewise, and a step covers so many chunks that its barrier costs about the same
-// whatever the height.
+// Short batches: 16 MT rows a workgroup, 128 T weight rows (SWIGLU: 128 of each of
+// the two matrices).  Up to 64 rows the weights' way from memory is what there is to
+// hide, not the matrix cores' time: a wave keeps its weights of the next four chunks
+// on their way in registers (with the one of fp4_gemm_tall_kernel a step waits out
+// most of a memory round trip), the activations of the next two steps likewise, and a
+// step covers so many chunks that its barrier costs about the same whatever the
+// height.  80 and 112 rows, where registers hold two chunks of weights, stand between
+// those and fp4_gemm_tall_kernel's 128 so that fewer rows of a batch's last workgroups
+// are padding; a weight's conversion, three vector instructions a pair of binary16
+// scaled ones, serves that many more rows (gate and up of [17408, 5120], two
+// workgroups a CU: matrix cores busy 60 % of the time with 64 rows, 65 with 80, 75
+// with 112, 74 with 128).
 template <int SCHEME, int MT, int T, bool SWIGLU>
 __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
     const TallArgs args) {
@@ -485,11 +573,13 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
   using Vector = typename Op::Vector;
   constexpr bool F16 = SCHEME == kSchemeF16;
   static_assert(!SWIGLU || T == 2);
-  constexpr uint32_t kAhead = 4;                    // chunks of weights in flight
-  constexpr uint32_t kSpan = MT == 3 ? 2 : 4 / MT;  // chunks per step
-  constexpr uint32_t kRow = kSpan * kChunk * 2u + 16u;
-  constexpr uint32_t kPieces = 16u * MT * kSpan * 8u / (kWaves * 64u);
-  static_assert(kPieces * kWaves * 64u == 16u * MT * kSpan * 8u);
+  constexpr uint32_t kAhead = MT > 4 ? 2 : 4;       // chunks of weights in flight
+  constexpr uint32_t kSpan = MT > 4 ? 1 : MT == 3 ? 2 : 4 / MT;  // chunks per step
+  constexpr uint32_t kRow = kSpan * kLdsRow;
+  // 16-byte pieces of a step's activations, of the workgroup and of a thread (an odd
+  // height's last ones are the same piece for half of the threads)
+  constexpr uint32_t kAllPieces = 16u * MT * kSpan * 8u;
+  constexpr uint32_t kPieces = (kAllPieces + kWaves * 64u - 1u) / (kWaves * 64u);
   __shared__ __attribute__((aligned(16))) uint8_t tile[2][16 * MT * kRow];
 
   const uint32_t lane = threadIdx.x & 63u;
@@ -499,16 +589,13 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
   const uint32_t K = args.padded_columns;
   const uint32_t chunks = K / kChunk;
 
-  // activation tiles of one weight tile run side by side on an XCD, then the
-  // weight tiles of a part: weights and activations come from its L2
-  const uint32_t tiles = args.m_tiles * args.n_tiles;
-  const uint32_t position = xcd_contiguous(blockIdx.x, tiles * args.splits);
-  const uint32_t part = position / tiles;
-  const uint32_t id = position - part * tiles;
-  const uint32_t first_m = id % args.m_tiles * (16u * MT);
-  const uint32_t n_tile = id / args.m_tiles;
-  const uint32_t first_chunk = chunks * part / args.splits;
-  const uint32_t end_chunk = chunks * (part + 1u) / args.splits;
+  // activation tiles of one weight tile run side by side on an XCD, then the weight
+  // tiles of a part: weights and activations come from its L2
+  constexpr bool kTailed = MT >= static_cast<int>(kLowestTail);
+  const Work work = work_of<kTailed>(args, chunks);
+  const uint32_t first_m = work.m_tile * (16u * MT);
+  const uint32_t first_chunk = work.first_chunk;
+  const uint32_t end_chunk = work.end_chunk;
 
   const uint32_t tile_count = (args.rows + kTileRows - 1u) / kTileRows;
   const uint8_t* weight_stream[T];
@@ -516,7 +603,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
   uint32_t tile_index[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) {
-    tile_index[t] = SWIGLU ? n_tile * kWaves + wave : (n_tile * kWaves + wave) * T + t;
+    tile_index[t] = weight_tile<T, SWIGLU>(work.n_tile, wave, t);
     const size_t stream = min(tile_index[t], tile_count - 1u);
     weight_stream[t] = (SWIGLU && t ? args.up_weights : args.weights) +
                        stream * chunks * (kTileRows * 32u) + lane * 16u;
@@ -532,14 +619,16 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
   uint32_t source_column[kPieces], target[kPieces];
 #pragma unroll
   for (uint32_t p = 0; p < kPieces; ++p) {
-    const uint32_t piece = p * kWaves * 64u + threadIdx.x;
+    const uint32_t piece = min(p * kWaves * 64u + threadIdx.x, kAllPieces - 1u);
     const uint32_t row = piece / (8u * kSpan);
     source_column[p] = piece % (8u * kSpan) * 16u;
-    target[p] = row * kRow + source_column[p];
+    target[p] = row * kRow + source_column[p] / kLdsRow * kLdsRow +
+                swizzled(source_column[p] % kLdsRow / 16u, row);
     source_row[p] = reinterpret_cast<const uint8_t*>(args.activations) +
                     static_cast<size_t>(min(first_m + row, args.batch - 1u)) * K * 2u;
   }
-  const uint32_t fragment_offset = n * kRow + g * 16u;
+  const uint32_t fragment_offset[2] = {n * kRow + swizzled(g, n),
+                                       n * kRow + swizzled(g + 4u, n)};
 
   f32x4 acc[MT][T][2];
 #pragma unroll
@@ -601,7 +690,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
       for (int mt = 0; mt < MT; ++mt)
         a[mt] = __builtin_bit_cast(
             Vector, *reinterpret_cast<const uint4*>(&tile[buffer][
-                        mt * 16u * kRow + fragment_offset + c * 128u + s * 64u]));
+                        mt * 16u * kRow + fragment_offset[s] + c * kLdsRow]));
 #pragma unroll
       for (int t = 0; t < T; ++t) {
         const uint4 q = codes[slot][t];
@@ -633,10 +722,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
   fetch_activations(integral_constant<int, 1>{}, first_chunk + kSpan);
   fetch_weights(integral_constant<int, 1>{}, first_chunk + 1u);
   __builtin_amdgcn_sched_barrier(0);
-  fetch_weights(integral_constant<int, 2>{}, first_chunk + 2u);
-  __builtin_amdgcn_sched_barrier(0);
-  fetch_weights(integral_constant<int, 3>{}, first_chunk + 3u);
-  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (kAhead > 2) {
+    fetch_weights(integral_constant<int, 2>{}, first_chunk + 2u);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_weights(integral_constant<int, 3>{}, first_chunk + 3u);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   store_activations(integral_constant<int, 0>{});
 
   // a chunk's weights are refilled as soon as they have been multiplied
@@ -671,7 +762,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
   };
   constexpr integral_constant<int, 0> even;
   constexpr integral_constant<int, 1> odd;
-  // Whole rounds of four chunks (eight at MT = 1): a step past the part's end
+  // Whole rounds of kAhead chunks (eight at MT = 1): a step past the part's end
   // makes its loads and multiplies nothing, so that every wait can count on the
   // same loads having been made since.
   for (uint32_t chunk = first_chunk; chunk < end_chunk;) {
@@ -679,14 +770,44 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
     chunk += kSpan;
     step(integral_constant<int, kSpan % kAhead>{}, odd, chunk);
     chunk += kSpan;
-    if constexpr (kSpan == 1) {
+    if constexpr (kSpan == 1 && kAhead == 4) {
       step(integral_constant<int, 2>{}, even, chunk);
       chunk += kSpan;
       step(integral_constant<int, 3>{}, odd, chunk);
       chunk += kSpan;
     }
   }
-  store_tiles<MT, T, SWIGLU>(args, part, first_m, tile_index, tile_count, acc);
+  if (kTailed && work.is_piece)
+    store_piece<MT, T>(args, work.piece, acc);
+  else
+    store_tiles<MT, T, SWIGLU>(args, work.part, first_m, tile_index, tile_count, acc);
+}
+
+// Adds the pieces of a cut tile in their order and stores the tile as a whole one's
+// workgroup would have, sixteen activation rows a workgroup (grid: tiles, MT).
+template <int MT, int T, bool SWIGLU>
+__global__ __launch_bounds__(kWaves * 64) void tall_tail_kernel(const TallArgs args) {
+  constexpr uint32_t kVectors = MT * T * 2u;
+  const uint32_t mt = blockIdx.y;
+  const f32x4* source = reinterpret_cast<const f32x4*>(args.partials) +
+                        (static_cast<size_t>(blockIdx.x) * args.cut * kVectors +
+                         mt * (T * 2u)) * (kWaves * 64u) + threadIdx.x;
+  f32x4 acc[1][T][2] = {};
+  for (uint32_t piece = 0; piece < args.cut; ++piece) {
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        acc[0][t][j] += source[static_cast<size_t>(t * 2 + j) * (kWaves * 64u)];
+    source += static_cast<size_t>(kVectors) * (kWaves * 64u);
+  }
+  uint32_t m_tile, n_tile, tile_index[T];
+  place_tile(args, args.whole + blockIdx.x, m_tile, n_tile);
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+    tile_index[t] = weight_tile<T, SWIGLU>(n_tile, threadIdx.x / 64u, t);
+  store_tiles<1, T, SWIGLU>(args, 0u, m_tile * (16u * MT) + 16u * mt, tile_index,
+                            (args.rows + kTileRows - 1u) / kTileRows, acc);
 }
 
 // Adds the parts of a launch whose K was cut, four columns per thread, and
@@ -736,7 +857,7 @@ bool tall_matrix_ok(const qllm_fp4_matrix* m) {
 }
 
 // How a launch is laid out: 16 `height` rows of activations per workgroup (height 1,
-// 2, 3, 4 or 8) and `splits` parts of K.
+// 2, 3, 4, 5, 7 or 8) and `splits` parts of K.
 //
 // Chosen by what the busiest CU will take.  With W workgroups per part it runs
 // n = ceil(W splits / 256) of them, each over ceil(chunks / splits) chunks; a
@@ -751,29 +872,50 @@ bool tall_matrix_ok(const qllm_fp4_matrix* m) {
 // 404 -> 97, 1000 rows 405 -> 254, 2000 rows 668 -> 498; [10240, 5120] 127 ->
 // 25, 135 -> 73, 211 -> 190, 333 -> 327; gate and up of [17408, 5120] 129 -> 54,
 // 221 -> 195, then unchanged.
+//
+// Where parts are added by a launch of their own, the tiles past the last full round of
+// the CUs may be cut instead of all of them: `cut` pieces each, the others run whole, as
+// where 500 rows by gate and up of [17408, 5120] are 544 tiles, of which the last 32 took
+// a CU's time for two again.  With that and the heights of 80 and 112 rows the four
+// linears of a layer of the 27B widths, binary16 scales, take 0.87 of the time for 80
+// rows, 0.92 for 300, 0.91 for 500, 0.93 for 1000, 0.98 for 1500 and 0.91 for 5000 (300
+// rows: 417 -> 382 us; 1000: 1102 -> 1021), with UE8M0 scales 0.92, 0.97, 0.95, 0.96, 0.94
+// and 0.91.
 struct TallPlan {
   uint32_t height;
   uint32_t splits;
+  uint32_t cut;   // 0: no tile is cut by itself
 };
 
 constexpr uint32_t kMaximumParts = 16;
+constexpr uint32_t kComputeUnits = 256;
 constexpr size_t kPartsBytes = size_t{128} << 20;
+constexpr uint32_t kMostPieces = 2u * kComputeUnits;   // of cut tiles
 
 struct ChunkCost {
   float alone, shared;   // ns
 };
-constexpr uint32_t kHeights[] = {1u, 2u, 3u, 4u, 8u};
-// [scheme][SwiGLU][height].  Those of 48 rows are no part of the fit: 86 % of the
-// 64-row workgroup's, the share that 48 rows of the 27B widths took; other widths
-// were not timed at that height.
-constexpr ChunkCost kChunkCost[2][2][5] = {
-    {{{160.f, 150.f}, {195.f, 180.f}, {315.f, 215.f}, {365.f, 250.f}, {1160.f, 780.f}},
-     {{250.f, 325.f}, {335.f, 345.f}, {520.f, 360.f}, {605.f, 420.f}, {1215.f, 780.f}}},
-    {{{220.f, 230.f}, {300.f, 280.f}, {470.f, 335.f}, {545.f, 390.f}, {1690.f, 1265.f}},
-     {{380.f, 440.f}, {515.f, 500.f}, {845.f, 615.f}, {985.f, 715.f}, {1710.f, 1230.f}}}};
+// Workgroups of 80 and 112 rows and cut tiles: not for matrices of fewer rows, which
+// were not timed with them.
+constexpr uint32_t kLowestTimedRows = 3072;
+constexpr uint32_t kHeights[] = {1u, 2u, 3u, 4u, 5u, 7u, 8u};
+// [scheme][SwiGLU][height].  Those of 80 and 112 rows are a fit of their own, to 410
+// launches of the 27B widths over 80 to 784 rows (4 to 8 % root mean square error), brought
+// to the scale of the others by the heights of 64 and 128 rows in it.  Those of 48 rows are
+// no part of a fit: 86 % of the 64-row workgroup's, the share that 48 rows of the 27B
+// widths took; other widths were not timed at that height.
+constexpr ChunkCost kChunkCost[2][2][7] = {
+    {{{160.f, 150.f}, {195.f, 180.f}, {315.f, 215.f}, {365.f, 250.f}, {770.f, 530.f},
+      {980.f, 690.f}, {1160.f, 780.f}},
+     {{250.f, 325.f}, {335.f, 345.f}, {520.f, 360.f}, {605.f, 420.f}, {790.f, 535.f},
+      {1000.f, 705.f}, {1215.f, 780.f}}},
+    {{{220.f, 230.f}, {300.f, 280.f}, {470.f, 335.f}, {545.f, 390.f}, {1150.f, 875.f},
+      {1440.f, 1120.f}, {1690.f, 1265.f}},
+     {{380.f, 440.f}, {515.f, 500.f}, {845.f, 615.f}, {985.f, 715.f}, {1150.f, 860.f},
+      {1440.f, 1110.f}, {1710.f, 1230.f}}}};
 
 uint32_t weight_rows_of(uint32_t height, bool swiglu) {
-  return (height == 8u && !swiglu ? kTilesN : kWaves) * kTileRows;
+  return (height >= 5u && !swiglu ? kTilesN : kWaves) * kTileRows;
 }
 
 uint32_t workgroups_of(uint32_t rows, uint32_t batch, uint32_t height, bool swiglu) {
@@ -784,6 +926,20 @@ uint32_t workgroups_of(uint32_t rows, uint32_t batch, uint32_t height, bool swig
 
 size_t parts_bytes(uint32_t rows, uint32_t batch, uint32_t splits, bool swiglu) {
   return splits > 1u ? size_t{splits} * (swiglu ? 2u : 1u) * batch * rows * 4u : 0u;
+}
+
+// Tiles that a plan with `cut` cuts: those past the last full round of the CUs.
+uint32_t tail_tiles_of(uint32_t workgroups) { return workgroups % kComputeUnits; }
+
+size_t piece_bytes(uint32_t height, bool swiglu) {
+  return size_t{16u} * height * weight_rows_of(height, swiglu) * (swiglu ? 8u : 4u);
+}
+
+// Bytes of workspace that a plan takes.
+size_t plan_bytes(const TallPlan& plan, uint32_t rows, uint32_t batch, bool swiglu) {
+  if (!plan.cut) return parts_bytes(rows, batch, plan.splits, swiglu);
+  return piece_bytes(plan.height, swiglu) * plan.cut *
+         tail_tiles_of(workgroups_of(rows, batch, plan.height, swiglu));
 }
 
 // At most `workspace_bytes` of parts; `separate`: they are added by a launch of
@@ -804,28 +960,48 @@ TallPlan plan_tall(uint32_t rows, uint32_t padded_columns, uint32_t batch,
                                                       : kMaximumParts;
   TallPlan best{};
   double least = 0.0;
+  const auto offer = [&](const TallPlan& plan, double time) {
+    if (best.height && time >= least) return;
+    best = plan;
+    least = time;
+  };
+  const bool timed = rows >= kLowestTimedRows;
+  uint32_t lower = 0;   // the height before
   for (uint32_t index = 0; index < std::size(kHeights); ++index) {
     const uint32_t height = kHeights[index];
+    if (!timed && (height == 5u || height == 7u)) continue;
     // one or two tiles of rows where they hold the batch, else the higher ones, and
     // none of which a lower one would hold the batch
     if (height < 3u ? batch > 16u * height : batch <= 32u) continue;
-    if (index && batch <= 16u * kHeights[index - 1u]) continue;
+    if (index && batch <= 16u * lower) continue;
+    lower = height;
     const ChunkCost cost = kChunkCost[scheme][swiglu][index];
     const uint32_t workgroups = workgroups_of(rows, batch, height, swiglu);
     for (uint32_t splits = first; splits <= last; ++splits) {
       const size_t bytes = parts_bytes(rows, batch, splits, swiglu);
       if (!fixed_splits && bytes > workspace_bytes) break;
-      const uint64_t on_one = (uint64_t{workgroups} * splits + 255u) / 256u;
+      const uint64_t on_one =
+          (uint64_t{workgroups} * splits + kComputeUnits - 1u) / kComputeUnits;
       const double chunk =
           on_one > 1u && on_one * cost.shared > cost.alone ? on_one * cost.shared
                                                            : cost.alone;
       const double time = (chunks + splits - 1u) / splits * chunk +
                           (separate ? 2.0 : 1.0) * bytes / 6200.0 +
                           (separate && splits > 1u ? 4300.0 : 0.0);
-      if (!best.height || time < least) {
-        best = {height, splits};
-        least = time;
-      }
+      offer({height, splits, 0u}, time);
+    }
+    // (whole tiles on every CU, so that two workgroups share it all the way)
+    const uint32_t tail = tail_tiles_of(workgroups);
+    if (!separate || whole || !timed || height < kLowestTail || tail == workgroups || !tail) continue;
+    for (uint32_t cut = 2u; cut <= last && tail * cut <= kMostPieces; ++cut) {
+      const TallPlan plan{height, 1u, cut};
+      const size_t bytes = plan_bytes(plan, rows, batch, swiglu);
+      if (bytes > workspace_bytes) break;
+      const double rounds =
+          workgroups / kComputeUnits +
+          static_cast<double>((tail * cut + kComputeUnits - 1u) / kComputeUnits) / cut;
+      offer(plan, chunks * std::max<double>(rounds * cost.shared, cost.alone) +
+                      2.0 * bytes / 6200.0 + 4300.0);
     }
   }
   return best;
@@ -860,11 +1036,47 @@ void start_tall(const TallArgs& args, uint32_t height, bool swiglu, uint32_t gri
       else
         fp4_gemm_short_kernel<SCHEME, 4, 1, false><<<grid, kThreads, 0, stream>>>(args);
       break;
+    case 5:
+      if (swiglu)
+        fp4_gemm_short_kernel<SCHEME, 5, 2, true><<<grid, kThreads, 0, stream>>>(args);
+      else
+        fp4_gemm_short_kernel<SCHEME, 5, 2, false><<<grid, kThreads, 0, stream>>>(args);
+      break;
+    case 7:
+      if (swiglu)
+        fp4_gemm_short_kernel<SCHEME, 7, 2, true><<<grid, kThreads, 0, stream>>>(args);
+      else
+        fp4_gemm_short_kernel<SCHEME, 7, 2, false><<<grid, kThreads, 0, stream>>>(args);
+      break;
     default:
       if (swiglu)
         fp4_gemm_tall_kernel<SCHEME, true><<<grid, kThreads, 0, stream>>>(args);
       else
         fp4_gemm_tall_kernel<SCHEME><<<grid, kThreads, 0, stream>>>(args);
+  }
+}
+
+void start_tail(const TallArgs& args, uint32_t height, uint32_t tail, hipStream_t stream) {
+  const dim3 grid(tail, height);
+  constexpr uint32_t kThreads = kWaves * 64;
+  switch (height) {
+    case 5:
+      if (args.up_weights)
+        tall_tail_kernel<5, 2, true><<<grid, kThreads, 0, stream>>>(args);
+      else
+        tall_tail_kernel<5, 2, false><<<grid, kThreads, 0, stream>>>(args);
+      break;
+    case 7:
+      if (args.up_weights)
+        tall_tail_kernel<7, 2, true><<<grid, kThreads, 0, stream>>>(args);
+      else
+        tall_tail_kernel<7, 2, false><<<grid, kThreads, 0, stream>>>(args);
+      break;
+    default:
+      if (args.up_weights)
+        tall_tail_kernel<8, 2, true><<<grid, kThreads, 0, stream>>>(args);
+      else
+        tall_tail_kernel<8, 2, false><<<grid, kThreads, 0, stream>>>(args);
   }
 }
 
@@ -876,11 +1088,17 @@ int32_t launch_tall(TallArgs args, uint32_t scheme, const TallPlan& plan,
   args.m_tiles = (args.batch + 16u * plan.height - 1u) / (16u * plan.height);
   args.n_tiles = (args.rows + weight_rows - 1u) / weight_rows;
   args.splits = plan.splits;
-  const uint32_t grid = args.m_tiles * args.n_tiles * plan.splits;
+  args.cut = plan.cut;
+  const uint32_t tiles = args.m_tiles * args.n_tiles;
+  const uint32_t tail = tail_tiles_of(tiles);
+  args.whole = tiles - tail;
+  const uint32_t grid =
+      plan.cut ? args.whole + tail * plan.cut : tiles * plan.splits;
   if (scheme == QLLM_SCALE_F16_BLOCK16)
     start_tall<kSchemeF16>(args, plan.height, swiglu, grid, stream);
   else
     start_tall<kSchemeUe8m0>(args, plan.height, swiglu, grid, stream);
+  if (plan.cut) start_tail(args, plan.height, tail, stream);
   return launched("tall FP4 GEMM");
 }
 
@@ -957,6 +1175,13 @@ extern "C" int32_t qllm_fp4_tall_layout(const qllm_fp4_matrix* matrix, int32_t s
   return QLLM_OK;
 }
 
+extern "C" uint32_t qllm_fp4_tall_tail_parts(const qllm_fp4_matrix* matrix, int32_t swiglu,
+                                             uint32_t batch, size_t workspace_bytes) {
+  if (!tall_matrix_ok(matrix) || !batch || batch > (1u << 20)) return 0u;
+  return plan_tall(matrix->rows, matrix->padded_columns, batch, matrix->scale_scheme,
+                   swiglu, true, workspace_bytes).cut;
+}
+
 extern "C" size_t qllm_fp4_tall_parts_bytes(const qllm_fp4_matrix* matrix, int32_t swiglu,
                                             uint32_t batch) {
   if (!tall_matrix_ok(matrix)) return 0u;
@@ -966,14 +1191,23 @@ extern "C" size_t qllm_fp4_tall_parts_bytes(const qllm_fp4_matrix* matrix, int32
   // row makes the parts cost more, so the first row of 16 asks for the most parts.
   for (uint64_t first = 1u; first <= batch; first += 16u) {
     const uint32_t row = static_cast<uint32_t>(first);
-    if (parts_bytes(rows, row, 2u, swiglu) > kPartsBytes) break;
+    if (parts_bytes(rows, row, 2u, swiglu) > kPartsBytes) {
+      // no launch of so many rows is cut as a whole: the room of the most pieces
+      if (rows >= kLowestTimedRows && rows % 4u == 0u && matrix->padded_columns >= 16u * kChunk)
+        most = std::max(most, kMostPieces * piece_bytes(kHeights[std::size(kHeights) - 1u],
+                                                        swiglu));
+      break;
+    }
     const uint32_t last = static_cast<uint32_t>(std::min<uint64_t>(first + 15u, batch));
     for (const bool separate : {true, false}) {
       if (!separate && swiglu) continue;
-      const TallPlan plan = plan_tall(rows, matrix->padded_columns, row,
-                                      matrix->scale_scheme, swiglu, separate, kPartsBytes);
-      most = std::max(most, std::min(parts_bytes(rows, last, plan.splits, swiglu),
-                                     kPartsBytes));
+      // (a cut tile's pieces are the same all along, so a plan that has them at any of
+      // the rows has them at the last one)
+      for (const uint32_t at : {row, last}) {
+        const TallPlan plan = plan_tall(rows, matrix->padded_columns, at,
+                                        matrix->scale_scheme, swiglu, separate, kPartsBytes);
+        most = std::max(most, std::min(plan_bytes(plan, rows, last, swiglu), kPartsBytes));
+      }
     }
   }
   return most;

@@ -210,6 +210,7 @@ SIGNATURES = {
     "qllm_fp4_swiglu_bf16_tall": (c_int32, [POINTER(Fp4Matrix), POINTER(Fp4Matrix), c_void_p, c_size_t, c_void_p, c_uint32, c_void_p]),
     "qllm_fp4_tall_workspace_bytes": (c_size_t, []),
     "qllm_fp4_tall_layout": (c_int32, [POINTER(Fp4Matrix), c_int32, c_uint32, c_size_t, c_uint32, POINTER(LaunchLayout)]),
+    "qllm_fp4_tall_tail_parts": (c_uint32, [POINTER(Fp4Matrix), c_int32, c_uint32, c_size_t]),
     "qllm_fp4_tall_parts_bytes": (c_size_t, [POINTER(Fp4Matrix), c_int32, c_uint32]),
     "qllm_fp4_tall_parts": (c_uint32, [POINTER(Fp4Matrix), c_uint32]),
     "qllm_fp4_gemm_bf16_tall_cut": (c_int32, [POINTER(Fp4Matrix), c_void_p, c_size_t, c_void_p, c_uint32, c_void_p, c_uint32, c_void_p, c_size_t, c_void_p]),

@@ -348,3 +348,86 @@ def test_every_layout_matches_the_product(device, scheme, rows, padded, batch, p
         qh.call("qllm_fp4_gemm_bf16_tall_partial", matrices[0], qh.ptr(d_act),
                 d_act.numel() * 2, qh.ptr(sums), parts, batch, None)
         assert np.abs(sums.double().sum(0).cpu().numpy() - want).max() < bound
+
+
+# (as above; parts of the tiles past the last full round of the compute units, 0: whole)
+@pytest.mark.parametrize("scheme,rows,padded,batch,plain,swiglu,tails", [
+    (F16, 8228, 2112, 1254, (128, False), (128, False), (3, 0)),
+    (F16, 5100, 2112, 1360, (80, False), (128, False), (3, 0)),
+    (F16, 6176, 4160, 1201, (112, False), (128, False), (4, 0)),
+    (UE8M0, 8228, 2112, 1254, (80, False), (128, False), (4, 0)),
+    (F16, 4100, 2112, 1254, (64, False), (80, False), (0, 4)),
+    (F16, 5100, 2112, 777, (48, False), (112, False), (0, 4)),
+    (UE8M0, 4100, 4160, 1201, (64, False), (112, False), (0, 2)),
+    (UE8M0, 6176, 2112, 1307, (80, False), (128, False), (0, 4)),
+    (F16, 6180, 2112, 66, (48, True), (80, True), (0, 0)),
+    (UE8M0, 6180, 1024, 1003, (112, False), (112, False), (0, 0))])
+def test_cut_last_tiles_match_the_product(device, scheme, rows, padded, batch, plain, swiglu,
+                                          tails):
+    """Workgroups of 80 and 112 batch rows, and launches that cut the tiles of their last
+    round alone: batches and weight rows that end inside a workgroup, a residual that is
+    the output, segments, gate and up; no more workspace than asked for."""
+    rng = np.random.default_rng(rows + batch)
+    act = ol.bf16_round(rng.standard_normal((batch, padded)).astype(np.float32))
+    d_act = gu.device_tensor(ol.bf16_bits(act), device)
+    act64 = torch.from_numpy(act).to(device, torch.float64)
+    matrices, wants, keep = [], [], []
+    for _ in range(2):
+        codes, scales = synth.fp4_matrix(rng, rows, padded, scheme)
+        values = torch.from_numpy(synth.dequantize(codes, scales, scheme)).to(device)
+        wants.append(act64 @ values.T)
+        tensors = gu.device_tensor(codes, device), gu.device_tensor(scales, device)
+        matrix, kept = qh.prepack(qh.fp4_matrix(*tensors, rows, padded, padded, scheme),
+                                  device)
+        matrices.append(matrix)
+        keep.append((tensors, kept))
+    del values
+    size = max(qh.call("qllm_fp4_tall_parts_bytes", matrices[0], kind, batch)
+               for kind in (0, 1))
+    workspace = torch.full((size // 4 + 4,), float("nan"), device=device)
+
+    for gate_and_up, expected in ((0, plain), (1, swiglu)):
+        found = qh.LaunchLayout()
+        qh.call("qllm_fp4_tall_layout", matrices[0], gate_and_up, batch, size, 0,
+                ctypes.byref(found))
+        assert (found.batch_rows, found.parts > 1) == expected
+        assert qh.call("qllm_fp4_tall_tail_parts", matrices[0], gate_and_up, batch,
+                       size) == tails[gate_and_up]
+        assert qh.call("qllm_fp4_tall_tail_parts", matrices[0], gate_and_up, batch, 0) == 0
+    # F32 sums of `padded` exact products, in any order
+    want = wants[0]
+    bound = 2e-6 * np.sqrt(padded) * want.abs().max().item()
+    rest = torch.randn((batch, rows), device=device)
+
+    def run(kind, residual=None):
+        out = torch.full((batch, rows), float("nan"), device=device,
+                         dtype=torch.bfloat16 if kind == qh.OUT_BF16 else torch.float32)
+        if residual is not None:
+            residual = out.copy_(residual)
+        qh.call("qllm_fp4_gemm_bf16_tall_cut", matrices[0], qh.ptr(d_act),
+                d_act.numel() * 2, qh.ptr(out), kind, qh.ptr(residual), batch,
+                qh.ptr(workspace), size, None)
+        return out
+
+    product = run(qh.OUT_F32)
+    assert (product.double() - want).abs().max() < bound
+    assert torch.equal(run(qh.OUT_BF16), product.bfloat16())
+    # (the product and the residual are added once more in F32)
+    assert (run(qh.OUT_F32, rest).double() - rest.double() - want).abs().max() < bound + 1e-6
+    if rows % 32 == 0:
+        widths = 64, rows - 64
+        outs = [torch.full((batch, n), float("nan"), device=device) for n in widths]
+        segments = (qh.GemmSegment * 2)(*[qh.GemmSegment(qh.ptr(o), n, qh.OUT_F32)
+                                          for o, n in zip(outs, widths)])
+        qh.call("qllm_fp4_gemm_bf16_tall_split_cut", matrices[0], qh.ptr(d_act),
+                d_act.numel() * 2, ctypes.addressof(segments), 2, batch,
+                qh.ptr(workspace), size, None)
+        assert torch.equal(torch.cat(outs, dim=1), product)
+    out = torch.full((batch, rows), float("nan"), dtype=torch.bfloat16, device=device)
+    qh.call("qllm_fp4_swiglu_bf16_tall_cut", matrices[0], matrices[1], qh.ptr(d_act),
+            d_act.numel() * 2, qh.ptr(out), batch, qh.ptr(workspace), size, None)
+    product = torch.nn.functional.silu(want).float().bfloat16().double() * wants[1]
+    # two roundings to bf16 (the gate's SiLU, the product), each of which may fall
+    # to the neighbouring value, at most 2^-7 of it away
+    error = (out.double() - product).abs()
+    assert (error <= 2.0 ** -6 * product.abs() + 4 * bound * (1 + wants[1].abs())).all()
