@@ -1091,6 +1091,17 @@ typedef struct qllm_stream_norm_launch {
   float branch_epsilon;
 } qllm_stream_norm_launch;
 int32_t qllm_stream_norm(const qllm_stream_norm_launch* launch, void* stream);
+/* The same where the stream begins: its rows are those of qllm_embedding_bf16_batch,
+ * looked up by this launch and written to `stream_out` (`input` is not read; no partial
+ * sums, no gather). */
+typedef struct qllm_token_rows {
+  const void* table;           /* bf16 [vocabulary][width] */
+  const uint32_t* tokens;      /* device, [rows] */
+  uint32_t vocabulary;
+  float scale;
+} qllm_token_rows;
+int32_t qllm_stream_norm_tokens(const qllm_stream_norm_launch* launch,
+                                const qllm_token_rows* tokens, void* stream);
 
 /* ---- windowed attention with mixed heads ---------------------------------- */
 

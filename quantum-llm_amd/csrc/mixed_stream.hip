@@ -1,5 +1,5 @@
-// The residual stream of mixed-layer decoders: embedding lookup and the norm
-// kernel every layer starts with - the partial sums of the projection before
+// The residual stream of mixed-layer decoders: embedding lookup (by itself or as the
+// first norm's input) and the norm kernel every layer starts with - the partial sums of the projection before
 // it added to the stream, the row's root mean square taken once, up to two
 // normalised copies written (a parallel layer feeds its mixer and its
 // feed-forward from the same row), or the token-shift blends of a mixer that
@@ -9,12 +9,34 @@
 namespace qllm {
 namespace {
 
-constexpr int kHeld = 4;   // 16-byte pieces of a row a thread keeps in registers
+constexpr int kHeld = 4;   // most 16-byte pieces of a row a thread keeps in registers
 
 struct NormArgs {
   qllm_stream_norm_launch launch;
   qllm_token_shift shift;
+  qllm_token_rows tokens;   // TABLE: the stream's rows are these, not launch.input
 };
+
+__device__ __forceinline__ const uint16_t* table_row(const NormArgs& args, uint32_t row) {
+  const uint32_t token = args.tokens.tokens[row];
+  return token < args.tokens.vocabulary
+             ? static_cast<const uint16_t*>(args.tokens.table) +
+                   size_t{token} * args.launch.width
+             : nullptr;
+}
+
+__device__ __forceinline__ f32x4 table_value4(const NormArgs& args, uint32_t row,
+                                              uint32_t piece) {
+  const uint16_t* values = table_row(args, row);
+  if (!values) return f32x4{};
+  const i32x2 bits = reinterpret_cast<const i32x2*>(values)[piece];
+  f32x4 value;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    value[c] = bf16_bits_to_f32(static_cast<uint32_t>(bits[c / 2]) >> (16 * (c % 2)) & 0xffffu) *
+               args.tokens.scale;
+  return value;
+}
 
 // The stream with the partial sums added; with a branch norm the sums alone.
 __device__ __forceinline__ f32x4 stream_value4(const qllm_stream_norm_launch& l,
@@ -69,96 +91,132 @@ __device__ __forceinline__ void pad_row(void* output, uint32_t row, uint32_t wid
     store_element(static_cast<T*>(output) + size_t{row} * stride + c, 0.0f);
 }
 
-// Rows whose width is a multiple of 4 and fits kHeld pieces per thread.
-template <typename T>
+// Rows whose width is a multiple of 4 and fits HELD pieces per thread.
+//
+// For a decoded token this is one workgroup whose time is the memory round trips it
+// waits for one after the other, 0.7 to 1.5 us each.  So all that it needs - partial
+// sums, norm weights, the previous token's row and the blends - is asked for before
+// the first sum over the row, with HELD = 1 (a thread per 16 bytes; registers of more
+// pieces would not hold it, and many rows hide each other's trips).  With the lookup of
+// the first layer's rows in the same launch (TABLE) a token of four layers takes 236 ->
+// 227 us at width 2048, 263 -> 253 in 32 bits.
+template <typename T, int HELD, bool TABLE>
 __global__ __launch_bounds__(1024) void stream_norm_wide_kernel(NormArgs args) {
   __shared__ float scratch[16];
   const qllm_stream_norm_launch& l = args.launch;
+  const qllm_token_shift& shift = args.shift;
   const uint32_t row = blockIdx.x;
-  const uint32_t source = l.gather ? l.gather[row] : row;
+  const uint32_t source = !TABLE && l.gather ? l.gather[row] : row;
   const uint32_t pieces = l.width / 4u;
-  f32x4 held[kHeld];
+  const bool shifted = l.shift != nullptr;
+  // (the request's slot is a load of its own that an address waits for)
+  const f32x4* carried =
+      shifted && row == 0u
+          ? reinterpret_cast<const f32x4*>(shift.previous +
+                                           l.step[kStepSlot] * shift.slot_stride)
+          : nullptr;
+  const bool writes = TABLE || (l.partial_count && !l.branch_weight);
+  f32x4 held[HELD], weight[2][HELD], before[HELD], mu[HELD == 1 ? 6 : 1];
   float squares = 0.0f;
 #pragma unroll
-  for (int i = 0; i < kHeld; ++i) {
+  for (int i = 0; i < HELD; ++i) {
+    const uint32_t piece = min(threadIdx.x + i * blockDim.x, pieces - 1u);
+#pragma unroll
+    for (int output = 0; output < 2; ++output)
+      if (l.weight[output])
+        weight[output][i] = reinterpret_cast<const f32x4*>(l.weight[output])[piece];
+    if (l.branch_weight)
+      before[i] = reinterpret_cast<const f32x4*>(l.input + size_t{row} * l.width)[piece];
+    if constexpr (HELD == 1)
+      if (shifted) {
+#pragma unroll
+        for (uint32_t s = 0; s < 6u; ++s)
+          if (s < shift.count) mu[s] = reinterpret_cast<const f32x4*>(shift.mu[s])[piece];
+        if (carried) before[i] = carried[piece];
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < HELD; ++i) {
     const uint32_t piece = threadIdx.x + i * blockDim.x;
     held[i] = f32x4{};
     if (piece >= pieces) continue;
-    held[i] = stream_value4(l, source, piece);
-    if (l.partial_count && !l.branch_weight)
+    held[i] = TABLE ? table_value4(args, row, piece) : stream_value4(l, source, piece);
+    if (writes)
       reinterpret_cast<f32x4*>(l.stream_out + size_t{row} * l.width)[piece] = held[i];
 #pragma unroll
     for (int c = 0; c < 4; ++c) squares = fmaf(held[i][c], held[i][c], squares);
   }
-  if (l.branch_weight) {
-    f32x4 before[kHeld], weight[kHeld];
+  if (!TABLE && l.branch_weight) {
+    f32x4 branch[HELD];
 #pragma unroll
-    for (int i = 0; i < kHeld; ++i) {
-      const uint32_t piece = threadIdx.x + i * blockDim.x;
-      if (piece >= pieces) continue;
-      before[i] = reinterpret_cast<const f32x4*>(l.input + size_t{row} * l.width)[piece];
-      weight[i] = reinterpret_cast<const f32x4*>(l.branch_weight)[piece];
-    }
+    for (int i = 0; i < HELD; ++i)
+      branch[i] = reinterpret_cast<const f32x4*>(
+          l.branch_weight)[min(threadIdx.x + i * blockDim.x, pieces - 1u)];
     const float unit =
         inverse_rms(block_sum(squares, scratch), l.width, l.branch_epsilon);
     squares = 0.0f;
 #pragma unroll
-    for (int i = 0; i < kHeld; ++i) {
+    for (int i = 0; i < HELD; ++i) {
       const uint32_t piece = threadIdx.x + i * blockDim.x;
       if (piece >= pieces) continue;
-      held[i] = before[i] + held[i] * unit * weight[i] * l.branch_scale;
+      held[i] = before[i] + held[i] * unit * branch[i] * l.branch_scale;
       reinterpret_cast<f32x4*>(l.stream_out + size_t{row} * l.width)[piece] = held[i];
 #pragma unroll
       for (int c = 0; c < 4; ++c) squares = fmaf(held[i][c], held[i][c], squares);
     }
   }
   const float inverse = inverse_rms(block_sum(squares, scratch), l.width, l.epsilon);
-  const bool shifted = l.shift != nullptr;
 #pragma unroll
   for (int output = 0; output < 2; ++output) {
     if (!l.weight[output] || (shifted && output == 0)) continue;
 #pragma unroll
-    for (int i = 0; i < kHeld; ++i) {
+    for (int i = 0; i < HELD; ++i) {
       const uint32_t piece = threadIdx.x + i * blockDim.x;
       if (piece >= pieces) continue;
-      const f32x4 weight = reinterpret_cast<const f32x4*>(l.weight[output])[piece];
       put4<T>(l.output[output], size_t{row} * l.stride[output] + piece * 4u,
-              held[i] * inverse * weight);
+              held[i] * inverse * weight[output][i]);
     }
     pad_row<T>(l.output[output], row, l.width, l.stride[output]);
   }
   if (!shifted) return;
 
-  const qllm_token_shift& shift = args.shift;
-  f32x4 before[kHeld];
-  float before_squares = 0.0f;
+  float before_inverse = 0.0f;
+  if (row == 0u) {   // takes the norm the request carries, already weighted
+    if constexpr (HELD > 1) {
 #pragma unroll
-  for (int i = 0; i < kHeld; ++i) {
-    const uint32_t piece = threadIdx.x + i * blockDim.x;
-    before[i] = f32x4{};
-    if (piece >= pieces) continue;
-    before[i] = row == 0u
-                    ? reinterpret_cast<const f32x4*>(
-                          shift.previous + l.step[kStepSlot] * shift.slot_stride)[piece]
-                    : stream_value4(l, row - 1u, piece);
+      for (int i = 0; i < HELD; ++i)
+        before[i] = carried[min(threadIdx.x + i * blockDim.x, pieces - 1u)];
+    }
+  } else {
+    float before_squares = 0.0f;
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-      before_squares = fmaf(before[i][c], before[i][c], before_squares);
+    for (int i = 0; i < HELD; ++i) {
+      const uint32_t piece = threadIdx.x + i * blockDim.x;
+      before[i] = f32x4{};
+      if (piece >= pieces) continue;
+      before[i] = TABLE ? table_value4(args, row - 1u, piece)
+                        : stream_value4(l, row - 1u, piece);
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        before_squares = fmaf(before[i][c], before[i][c], before_squares);
+    }
+    before_inverse = inverse_rms(block_sum(before_squares, scratch), l.width, l.epsilon);
   }
-  // row 0 takes the norm the request carries, already weighted
-  const float before_inverse =
-      inverse_rms(block_sum(before_squares, scratch), l.width, l.epsilon);
 #pragma unroll
-  for (int i = 0; i < kHeld; ++i) {
+  for (int i = 0; i < HELD; ++i) {
     const uint32_t piece = threadIdx.x + i * blockDim.x;
     if (piece >= pieces) continue;
-    const f32x4 weight = reinterpret_cast<const f32x4*>(l.weight[0])[piece];
-    const f32x4 here = held[i] * inverse * weight;
-    const f32x4 there = row == 0u ? before[i] : before[i] * before_inverse * weight;
-    for (uint32_t s = 0; s < shift.count; ++s) {
-      const f32x4 mu = reinterpret_cast<const f32x4*>(shift.mu[s])[piece];
+    const f32x4 here = held[i] * inverse * weight[0][i];
+    const f32x4 there =
+        row == 0u ? before[i] : before[i] * before_inverse * weight[0][i];
+#pragma unroll
+    for (uint32_t s = 0; s < 6u; ++s) {
+      if (s >= shift.count) break;
+      const f32x4 blend =
+          HELD == 1 ? mu[s % (HELD == 1 ? 6u : 1u)]
+                    : reinterpret_cast<const f32x4*>(shift.mu[s])[piece];
       put4<T>(shift.output[s], size_t{row} * l.stride[0] + piece * 4u,
-              here + (there - here) * mu);
+              here + (there - here) * blend);
     }
     if (row + 1u == l.rows) reinterpret_cast<f32x4*>(shift.last)[piece] = here;
   }
@@ -166,13 +224,21 @@ __global__ __launch_bounds__(1024) void stream_norm_wide_kernel(NormArgs args) {
     pad_row<T>(shift.output[s], row, l.width, l.stride[0]);
 }
 
-template <typename T>
+template <typename T, bool TABLE>
 __global__ __launch_bounds__(256) void stream_norm_narrow_kernel(NormArgs args) {
   __shared__ float scratch[16];
   const qllm_stream_norm_launch& l = args.launch;
   const uint32_t row = blockIdx.x;
-  const uint32_t source = l.gather ? l.gather[row] : row;
+  const uint32_t source = !TABLE && l.gather ? l.gather[row] : row;
   const bool shifted = l.shift != nullptr;
+  const auto own_value = [&](uint32_t at, uint32_t c) {
+    if constexpr (TABLE) {
+      const uint16_t* values = table_row(args, at);
+      return values ? bf16_bits_to_f32(values[c]) * args.tokens.scale : 0.0f;
+    } else {
+      return stream_value(l, at, c);
+    }
+  };
   const float* carried =
       shifted && row == 0u ? args.shift.previous + l.step[kStepSlot] * args.shift.slot_stride
                            : nullptr;
@@ -189,17 +255,17 @@ __global__ __launch_bounds__(256) void stream_norm_narrow_kernel(NormArgs args) 
                   l.branch_scale;
   }
   const auto here_value = [&](uint32_t c) {
-    const float value = stream_value(l, source, c);
+    const float value = own_value(source, c);
     return l.branch_weight ? l.input[size_t{row} * l.width + c] +
                                  value * unit_branch * l.branch_weight[c]
                            : value;
   };
   for (uint32_t c = threadIdx.x; c < l.width; c += blockDim.x) {
     const float value = here_value(c);
-    if (l.partial_count) l.stream_out[size_t{row} * l.width + c] = value;
+    if (TABLE || l.partial_count) l.stream_out[size_t{row} * l.width + c] = value;
     squares = fmaf(value, value, squares);
     if (shifted && !carried) {
-      const float before = stream_value(l, row - 1u, c);
+      const float before = own_value(row - 1u, c);
       before_squares = fmaf(before, before, before_squares);
     }
   }
@@ -217,7 +283,7 @@ __global__ __launch_bounds__(256) void stream_norm_narrow_kernel(NormArgs args) 
     const float here = unit * l.weight[0][c];
     const float there =
         carried ? carried[c]
-                : stream_value(l, row - 1u, c) * before_inverse * l.weight[0][c];
+                : own_value(row - 1u, c) * before_inverse * l.weight[0][c];
     for (uint32_t s = 0; s < args.shift.count; ++s)
       store_element(static_cast<T*>(args.shift.output[s]) + size_t{row} * l.stride[0] + c,
                     here + (there - here) * args.shift.mu[s][c]);
@@ -262,11 +328,29 @@ extern "C" int32_t qllm_embedding_bf16_batch(const void* table_bf16, uint32_t vo
   return launched("bf16 embedding lookup");
 }
 
-extern "C" int32_t qllm_stream_norm(const qllm_stream_norm_launch* launch, void* stream) {
+namespace {
+
+template <typename T, bool TABLE>
+void launch_norm(const NormArgs& args, bool wide, hipStream_t stream) {
+  const qllm_stream_norm_launch& l = args.launch;
+  const uint32_t pieces = l.width / 4u;
+  uint32_t threads = l.rows <= 16u ? 1024u : 256u;
+  while (threads > 64u && threads / 2u >= pieces) threads /= 2u;
+  if (pieces > threads * kHeld) threads = 1024u;
+  if (!wide || pieces > threads * kHeld)
+    stream_norm_narrow_kernel<T, TABLE><<<l.rows, 256, 0, stream>>>(args);
+  else if (pieces <= threads)
+    stream_norm_wide_kernel<T, 1, TABLE><<<l.rows, threads, 0, stream>>>(args);
+  else
+    stream_norm_wide_kernel<T, kHeld, TABLE><<<l.rows, threads, 0, stream>>>(args);
+}
+
+int32_t norm_rows(const qllm_stream_norm_launch* launch, const qllm_token_rows* tokens,
+                  void* stream) {
   if (!launch || !launch->input || !launch->rows || !launch->width ||
       launch->element > QLLM_ELEMENT_F32 ||
       (launch->partial_count &&
-       (!launch->partials || !launch->stream_out || launch->stream_out == launch->input ||
+       (tokens || !launch->partials || !launch->stream_out || launch->stream_out == launch->input ||
         launch->partial_stride < launch->width || launch->gather)) ||
       (launch->branch_weight && (!launch->partial_count || launch->shift)))
     return fail(QLLM_INVALID_ARGUMENT, "invalid stream norm");
@@ -281,7 +365,7 @@ extern "C" int32_t qllm_stream_norm(const qllm_stream_norm_launch* launch, void*
     wide = wide && aligned16(launch->weight[i]) && aligned16(launch->output[i]) &&
            launch->stride[i] % 4u == 0u;
   }
-  NormArgs args{*launch, {}};
+  NormArgs args{*launch, {}, {}};
   if (const auto* shift = launch->shift) {
     if (!shift->count || shift->count > 6u || !shift->previous || !shift->last ||
         !launch->step || launch->gather || !launch->weight[0])
@@ -295,20 +379,32 @@ extern "C" int32_t qllm_stream_norm(const qllm_stream_norm_launch* launch, void*
            shift->slot_stride % 4u == 0u;
     args.shift = *shift;
   }
-  const uint32_t pieces = launch->width / 4u;
-  uint32_t threads = launch->rows <= 16u ? 1024u : 256u;
-  while (threads > 64u && threads / 2u >= pieces) threads /= 2u;
-  if (pieces > threads * kHeld) threads = 1024u;
-  wide = wide && pieces <= threads * kHeld;
+  if (tokens) {
+    args.tokens = *tokens;
+    wide = wide && (reinterpret_cast<uintptr_t>(tokens->table) & 7u) == 0u;
+  }
   const auto hip_stream = as_stream(stream);
-  const bool f32 = launch->element == QLLM_ELEMENT_F32;
-  if (wide && f32)
-    stream_norm_wide_kernel<float><<<launch->rows, threads, 0, hip_stream>>>(args);
-  else if (wide)
-    stream_norm_wide_kernel<uint16_t><<<launch->rows, threads, 0, hip_stream>>>(args);
-  else if (f32)
-    stream_norm_narrow_kernel<float><<<launch->rows, 256, 0, hip_stream>>>(args);
+  if (launch->element == QLLM_ELEMENT_F32)
+    tokens ? launch_norm<float, true>(args, wide, hip_stream)
+           : launch_norm<float, false>(args, wide, hip_stream);
   else
-    stream_norm_narrow_kernel<uint16_t><<<launch->rows, 256, 0, hip_stream>>>(args);
+    tokens ? launch_norm<uint16_t, true>(args, wide, hip_stream)
+           : launch_norm<uint16_t, false>(args, wide, hip_stream);
   return launched("stream norm");
+}
+
+}  // namespace
+
+extern "C" int32_t qllm_stream_norm(const qllm_stream_norm_launch* launch, void* stream) {
+  return norm_rows(launch, nullptr, stream);
+}
+
+extern "C" int32_t qllm_stream_norm_tokens(const qllm_stream_norm_launch* launch,
+                                           const qllm_token_rows* tokens, void* stream) {
+  if (!launch || !tokens || !tokens->table || !tokens->tokens || !tokens->vocabulary ||
+      !launch->stream_out || launch->gather || launch->partial_count)
+    return fail(QLLM_INVALID_ARGUMENT, "invalid stream norm of tokens");
+  qllm_stream_norm_launch own = *launch;
+  own.input = own.stream_out;
+  return norm_rows(&own, tokens, stream);
 }

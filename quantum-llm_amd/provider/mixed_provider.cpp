@@ -931,13 +931,28 @@ void Mi355MixedProvider::begin_batch(MixedRequestState& state,
   batch_rows_ = rows;
 }
 
-void Mi355MixedProvider::enqueue_embedding(std::uint32_t rows) {
+// `with_norm`: the first block's norm looks the rows up itself.
+void Mi355MixedProvider::enqueue_embedding(std::uint32_t rows, bool with_norm) {
   stream_index_ = 0U;
   pending_partials_ = 0U;
   pending_branch_ = {};
+  pending_tokens_ = with_norm && !blocks_.empty();
+  if (pending_tokens_) return;
   status_check(qllm_embedding_bf16_batch(
       embedding_.get(), g_.vocabulary, step_.as<std::uint32_t>() + kStepWords,
       hidden_[0].as<float>(), rows, g_.hidden, embedding_scale_, stream_));
+}
+
+void Mi355MixedProvider::enqueue_norm(const qllm_stream_norm_launch& norm) {
+  if (!std::exchange(pending_tokens_, false)) {
+    status_check(qllm_stream_norm(&norm, stream_));
+    return;
+  }
+  const qllm_token_rows tokens{embedding_.get(), step_.as<std::uint32_t>() + kStepWords,
+                               g_.vocabulary, embedding_scale_};
+  qllm_stream_norm_launch first = norm;
+  first.stream_out = hidden_[0].as<float>();
+  status_check(qllm_stream_norm_tokens(&first, &tokens, stream_));
 }
 
 void Mi355MixedProvider::enqueue_attention(Block& block, std::uint32_t rows,
@@ -1094,7 +1109,7 @@ void Mi355MixedProvider::enqueue_sandwich(Block& block, std::uint32_t rows,
     norm.weight[0] = weight.as<float>();
     norm.output[0] = inputs_.get();
     norm.stride[0] = mixer_stride_;
-    status_check(qllm_stream_norm(&norm, stream_));
+    enqueue_norm(norm);
   };
   const auto project = [&](const Matrix& matrix, std::uint32_t splits,
                            const DeviceBuffer& post_norm) {
@@ -1176,7 +1191,7 @@ void Mi355MixedProvider::enqueue_block(Block& block, std::uint32_t rows,
     shift.last = shift_last_.as<float>();
     norm.shift = &shift;
   }
-  status_check(qllm_stream_norm(&norm, stream_));
+  enqueue_norm(norm);
 
   std::vector<qllm_linear_segment> segments;
   for (const auto& projection : block.projections) {
@@ -1235,7 +1250,7 @@ void Mi355MixedProvider::enqueue_block(Block& block, std::uint32_t rows,
 void Mi355MixedProvider::settle_stream(std::uint32_t rows) {
   if (!pending_partials_) return;
   const auto norm = stream_norm(rows, final_epsilon_);
-  status_check(qllm_stream_norm(&norm, stream_));
+  enqueue_norm(norm);
 }
 
 // Final norm and head on `count` rows: those from `first` on, or with `gather`
@@ -1249,7 +1264,7 @@ void Mi355MixedProvider::enqueue_head(std::uint32_t batch_rows, std::uint32_t fi
   norm.output[0] = head_input_.get();
   norm.stride[0] = mixer_stride_;
   norm.gather = gather ? gather_.as<std::uint32_t>() : nullptr;
-  status_check(qllm_stream_norm(&norm, stream_));
+  enqueue_norm(norm);
   qllm_linear_segment s{};
   s.weights = head_.data.get();
   s.input = head_input_.get();
@@ -1322,7 +1337,7 @@ Mi355MixedProvider::HeadResult Mi355MixedProvider::finish_batch(
 void Mi355MixedProvider::launch_step_graph() {
   const auto stream = static_cast<hipStream_t>(stream_);
   const auto enqueue = [this] {
-    enqueue_embedding(1U);
+    enqueue_embedding(1U, true);
     for (auto& block : blocks_) enqueue_block(*block, 1U, g_.max_context - 1U);
     enqueue_head(1U, 0U, 1U, false);
     status_check(qllm_argmax_batch(logits_.as<float>(), g_.vocabulary, 1U,
@@ -1439,7 +1454,7 @@ er::OperationExecutionHandle Mi355MixedProvider::execute(
       const auto tokens = host_u32_batch(input("token_ids"), kTokenAbi,
                                          "embedding token batch", g_.chunk_rows);
       begin_batch(*state, tokens, state->position);
-      enqueue_embedding(batch_rows_);
+      enqueue_embedding(batch_rows_, false);
       values.emplace("hidden", hidden_value(batch_rows_));
     } else if (operation->kind == Kind::head) {
       const auto rows = require_rows();
@@ -1490,7 +1505,7 @@ er::OperationExecutionHandle Mi355MixedProvider::execute_program_sequence(
     if (single) {
       launch_step_graph();
     } else {
-      enqueue_embedding(batch_rows_);
+      enqueue_embedding(batch_rows_, true);
       for (auto& block : blocks_) enqueue_block(*block, batch_rows_, positions.back());
     }
     auto result = finish_batch(*state, batch_rows_, invocation.request, single);

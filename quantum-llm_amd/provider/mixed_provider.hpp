@@ -150,7 +150,8 @@ class Mi355MixedProvider final : public DecoderProvider {
   void ensure_workspace(std::uint32_t rows, std::uint32_t last_position);
   void begin_batch(MixedRequestState& state, std::span<const std::uint32_t> tokens,
                    std::uint32_t first_position);
-  void enqueue_embedding(std::uint32_t rows);
+  void enqueue_embedding(std::uint32_t rows, bool with_norm);
+  void enqueue_norm(const qllm_stream_norm_launch& norm);
   void enqueue_block(Block& block, std::uint32_t rows, std::uint32_t last_position);
   void enqueue_sandwich(Block& block, std::uint32_t rows, std::uint32_t last_position);
   void enqueue_mixer(Block& block, std::uint32_t rows, std::uint32_t last_position);
@@ -235,6 +236,7 @@ class Mi355MixedProvider final : public DecoderProvider {
   std::size_t staging_words_{};
 
   std::uint32_t stream_index_{}; // which of hidden_ holds the stream
+  bool pending_tokens_{};   // the stream's rows are still to be looked up
   std::uint32_t pending_partials_{};
   // the norm pending partial sums pass on their way into the stream, if any
   struct Branch final {

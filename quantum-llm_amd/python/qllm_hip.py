@@ -115,6 +115,11 @@ class TokenShift(Structure):
                 ("previous", c_void_p), ("slot_stride", c_uint64), ("last", c_void_p)]
 
 
+class TokenRows(Structure):
+    _fields_ = [("table", c_void_p), ("tokens", c_void_p), ("vocabulary", c_uint32),
+                ("scale", c_float)]
+
+
 class StreamNormLaunch(Structure):
     _fields_ = [("input", c_void_p), ("stream_out", c_void_p), ("partials", c_void_p),
                 ("partial_count", c_uint32), ("partial_stride", c_uint32),
@@ -291,6 +296,7 @@ SIGNATURES = {
     "qllm_linear_batch": (c_int32, [POINTER(LinearSegment), c_uint32, c_uint32, c_uint32, c_void_p]),
     "qllm_embedding_bf16_batch": (c_int32, [c_void_p, c_uint32, c_void_p, c_void_p, c_uint32, c_uint32, c_float, c_void_p]),
     "qllm_stream_norm": (c_int32, [POINTER(StreamNormLaunch), c_void_p]),
+    "qllm_stream_norm_tokens": (c_int32, [POINTER(StreamNormLaunch), POINTER(TokenRows), c_void_p]),
     "qllm_windowed_layer_bytes": (c_size_t, [c_uint32, c_uint32, c_uint32, c_uint32, c_uint32]),
     "qllm_windowed_rope_store": (c_int32, [POINTER(WindowedAttention), POINTER(RopeStoreLaunch), c_void_p]),
     "qllm_windowed_attention_workspace_bytes": (c_size_t, [POINTER(WindowedAttention), c_uint32, c_uint32]),

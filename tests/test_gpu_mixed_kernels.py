@@ -367,6 +367,52 @@ def test_token_shift_carries_the_last_norm(device, element, width):
         carried[slot_stride:slot_stride + width] = last[:width]
 
 
+@pytest.mark.parametrize("element", [F32, BF16])
+@pytest.mark.parametrize("width,rows", [(64, 1), (90, 3), (2048, 1), (2048, 20), (4096, 17),
+                                        (8192, 2)])
+@pytest.mark.parametrize("shifted", [False, True])
+def test_first_norm_looks_its_rows_up(device, element, width, rows, shifted):
+    """Rows of a thread per piece, of several and of no whole pieces: the same bits as the
+    lookup and the norm by themselves, a token outside the table among them."""
+    rng = np.random.default_rng(width + rows)
+    vocabulary, stride = 50, padded(width, 64)
+    table = on(device, mm.bf16(rng.standard_normal((vocabulary, width))), torch.bfloat16)
+    ids = rng.integers(0, vocabulary, rows)
+    ids[rows // 2] = vocabulary if rows > 1 else ids[0]
+    ids = on(device, ids.astype(np.int32), torch.int32)
+    weights = [on(device, w) for w in rng.standard_normal((2, width)).astype(np.float32)]
+    mus = [on(device, m) for m in rng.uniform(0, 1, (6, width)).astype(np.float32)]
+    carried = on(device, rng.standard_normal(padded(width, 4)).astype(np.float32))
+    step = steps(device, 0, slot=0)
+
+    def run(together):
+        x = torch.full((rows, width), 7.0, device=device)
+        outs = [torch.full((rows, stride), 9.0, dtype=torch_type(element), device=device)
+                for _ in range(8)]
+        last = torch.zeros(padded(width, 4), device=device)
+        shift = qh.TokenShift(6, (ctypes.c_void_p * 6)(*map(qh.ptr, mus)),
+                              (ctypes.c_void_p * 6)(*map(qh.ptr, outs[2:])), qh.ptr(carried),
+                              padded(width, 4), qh.ptr(last))
+        launch = qh.StreamNormLaunch(
+            None if together else qh.ptr(x), qh.ptr(x) if together else None, None, 0, 0,
+            (ctypes.c_void_p * 2)(*map(qh.ptr, weights)),
+            (ctypes.c_void_p * 2)(*map(qh.ptr, outs[:2])),
+            (ctypes.c_uint32 * 2)(stride, stride), rows, width, 1e-5, element,
+            ctypes.pointer(shift) if shifted else None, None, qh.ptr(step))
+        if together:
+            qh.call("qllm_stream_norm_tokens", ctypes.byref(launch),
+                    ctypes.byref(qh.TokenRows(qh.ptr(table), qh.ptr(ids), vocabulary, 0.75)),
+                    None)
+        else:
+            qh.call("qllm_embedding_bf16_batch", qh.ptr(table), vocabulary, qh.ptr(ids),
+                    qh.ptr(x), rows, width, 0.75, None)
+            qh.call("qllm_stream_norm", ctypes.byref(launch), None)
+        return [x, last, *outs]
+
+    for one, two in zip(run(True), run(False)):
+        assert torch.equal(one, two)
+
+
 # ---- attention -------------------------------------------------------------------
 
 
