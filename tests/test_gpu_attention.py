@@ -216,6 +216,47 @@ def test_batched_launch_equals_one_launch_per_batch(device, total, first, Q, KV,
             qh.call("qllm_attention_paged_q4h_batched", launch, total)
 
 
+@pytest.mark.parametrize("splits", [1, 2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("d,gated,kind", [(128, False, qh.OUT_BF16), (256, True, qh.OUT_F32)])
+@pytest.mark.parametrize("shift", [0, 2])       # output values past a 16-byte line
+def test_splits_are_added_alike_in_every_form(device, splits, d, gated, kind, shift):
+    """Few splits are added four dimensions a thread, more of them and outputs off a
+    16-byte line one a thread: the oracle's attention either way, and the same bits
+    whatever the line.  Short contexts leave splits without a tile."""
+    rng = np.random.default_rng(splits)
+    rows, Q, KV, page_tokens, first = 33, 8, 2, 64, 130
+    tokens = first + rows - 1
+    keys = rng.standard_normal((tokens, KV, d)).astype(np.float32)
+    values = rng.standard_normal((tokens, KV, d)).astype(np.float32)
+    pages = synth.q4h_pages(keys, values, page_tokens, 1, 0)
+    stride = d * (2 if gated else 1)
+    query = ol.bf16_round(rng.standard_normal((rows, Q, stride)).astype(np.float32))
+    d_pages = [gu.device_tensor(page, device) for page in pages]
+    table = torch.tensor([page.data_ptr() for page in d_pages], dtype=torch.int64,
+                         device=device)
+    d_query = gu.device_tensor(query, device)
+    maxima = torch.zeros((rows, splits, Q), device=device)
+    sums = torch.zeros_like(maxima)
+    outputs = torch.zeros((rows, splits, Q, d), device=device)
+    type_ = torch.bfloat16 if kind == qh.OUT_BF16 else torch.float32
+    got = []
+    for off in (0, shift):
+        out = torch.zeros(rows * Q * d + 8, dtype=type_, device=device)
+        launch = qh.Q4hAttentionLaunch(
+            qh.ptr(d_query), 0, 0, qh.ptr(table), out.data_ptr() + off * out.element_size(),
+            qh.ptr(maxima), qh.ptr(sums), qh.ptr(outputs), first, rows, 0, page_tokens, Q, KV,
+            d, 0, splits, stride, int(gated), kind, None)
+        qh.call("qllm_attention_paged_q4h_batched", launch, 6)
+        torch.cuda.synchronize()
+        got.append(out[off:off + rows * Q * d].float().cpu().numpy().reshape(rows, Q, d))
+    assert np.array_equal(*got)
+    shape = ol.AttentionShape(rows, Q, KV, d, first, page_tokens, 0, int(gated))
+    want = ol.attention_q4h(shape, query, pages, "f64")
+    # a bf16 output is half of 2^-8 away from its value at most
+    gu.assert_close(got[0], want, rtol=1e-2 if kind == qh.OUT_BF16 else 1e-3, atol=1e-3,
+                    what="attention")
+
+
 @pytest.mark.parametrize("total,first,Q,KV,batch,splits", [
     (958, 1, 24, 4, 5, 1),      # 768 workgroups: two waves each; the last has 3 rows
     (93, 70, 16, 8, 16, 16),    # splits without a tile
