@@ -1187,6 +1187,13 @@ uint32_t qllm_windowed_attention_form(const qllm_windowed_attention* attention,
 int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* attention,
                                      const qllm_attention_launch* launch,
                                      void* stream);
+/* One row: qllm_windowed_rope_store, then qllm_windowed_attention_rows.  In the
+ * split form the launch of the scores rotates and stores the token itself, and
+ * query_out is not written. */
+int32_t qllm_windowed_attention_token(const qllm_windowed_attention* attention,
+                                      const qllm_rope_store_launch* store,
+                                      const qllm_attention_launch* launch,
+                                      void* stream);
 
 /* ---- latent attention ------------------------------------------------------- */
 

@@ -630,11 +630,47 @@ __global__ __launch_bounds__(256) void general_values_kernel(AttentionArgs args)
 
 // ---- split form (decode) -----------------------------------------------------------
 
+// Eight dimensions of a projection from d on, rotated pair by pair ((cos, sin) per
+// pair in `turns`), as a matrix operand; zeros from `dim` on.
+__device__ __forceinline__ i32x4 turned_operand(const f32x4 (&x)[2], uint32_t d, uint32_t dim,
+                                                uint32_t rotary_dims, const float2* turns) {
+  i32x4 operand;
+#pragma unroll
+  for (uint32_t i = 0; i < 4u; ++i) {
+    const float u = x[i / 2u][i % 2u * 2u];
+    const float v = x[i / 2u][i % 2u * 2u + 1u];
+    const bool turns_here = d + 2u * i < rotary_dims;
+    const float2 turn = turns[turns_here ? d / 2u + i : 0u];
+    const float first = u * turn.x - v * turn.y;
+    const float second = v * turn.x + u * turn.y;
+    operand[i] = static_cast<int>(turns_here ? pack_bf16(first, second) : pack_bf16(u, v));
+  }
+  return d < dim ? operand : i32x4{};
+}
+
+// Eight dimensions of a projection row; places past the last eight repeat them.
+__device__ __forceinline__ void fetch_eight(f32x4 (&x)[2], const float* row, uint32_t d,
+                                            uint32_t dim) {
+  const float* from = row + min(d, dim - 8u);
+  x[0] = four_elements(from);
+  x[1] = four_elements(from + 4);
+}
+
 // NK = key_stride / 32.
-template <int NK>
-__global__ __launch_bounds__(256) void split_scores_kernel(AttentionArgs args) {
+//
+// FRESH: the launch of one token, which also does what rope_store_kernel does for
+// it.  A wave rotates the queries that it needs from the projections, with one table
+// of angles per workgroup; the wave whose sixteen keys hold the token's lays the
+// rotated key over what its page held and stores it; the values go to their page from
+// the first workgroup, before the launch that reads them.  A launch less on a chain
+// of launches that wait for each other: 16 heads on 4 of 128 dimensions, 5 tiles, 4.7
+// us and 4.7 in two launches, 6.5 in one.
+template <int NK, bool FRESH>
+__global__ __launch_bounds__(256) void split_scores_kernel(AttentionArgs args,
+                                                           qllm_rope_store_launch store) {
   __shared__ float wave_maximum[4][16];
   __shared__ float wave_total[4][16];
+  __shared__ float2 turns[FRESH ? NK * 16 : 1];
   const Attention& a = args.attention;
   const uint32_t row = blockIdx.z;
   const uint32_t kv = blockIdx.y;
@@ -646,16 +682,64 @@ __global__ __launch_bounds__(256) void split_scores_kernel(AttentionArgs args) {
   const uint32_t in_group = lane % 16u;
   const uint32_t head = kv * group + min(in_group, group - 1u);
 
-  i32x4 q[NK];
-  const uint16_t* query = static_cast<const uint16_t*>(args.launch.query) +
-                          (size_t{row} * a.query_heads + head) * a.key_stride +
-                          8u * (lane / 16u);
-#pragma unroll
-  for (int c = 0; c < NK; ++c) q[c] = *reinterpret_cast<const i32x4*>(query + c * 32);
-
   const uint32_t units = range.count * 2u;   // of 16 keys
   const uint32_t begin = static_cast<uint32_t>(uint64_t{units} * blockIdx.x / gridDim.x);
   const uint32_t end = static_cast<uint32_t>(uint64_t{units} * (blockIdx.x + 1u) / gridDim.x);
+  i32x4 q[NK];
+  // the token's key is in the last tile, and this wave's if its unit is
+  const uint32_t own_unit = 2u * (range.count - 1u) + position % kTileKeys / 16u;
+  i32x4 own_key[FRESH ? NK : 1];
+  if constexpr (FRESH) {
+    const uint32_t d0 = 8u * (lane / 16u);
+    const bool owner = own_unit >= begin && own_unit < end && (own_unit - begin) % 4u == wave;
+    f32x4 raw[NK][2], raw_key[NK][2];
+#pragma unroll
+    for (int c = 0; c < NK; ++c)
+      fetch_eight(raw[c], store.projections + store.query_column + head * a.dim, c * 32u + d0,
+                  a.dim);
+    if (owner)
+#pragma unroll
+      for (int c = 0; c < NK; ++c)
+        fetch_eight(raw_key[c], store.projections + store.key_column + kv * a.dim,
+                    c * 32u + d0, a.dim);
+    if (threadIdx.x < store.rotary_dims / 2u) {
+      // the angle is reduced to one turn before it becomes F32
+      constexpr double kTurn = 6.283185307179586476925286766559;
+      double angle = static_cast<double>(position) * store.frequencies[threadIdx.x];
+      angle -= kTurn * rint(angle / kTurn);
+      float sine, cosine;
+      sincosf(static_cast<float>(angle), &sine, &cosine);
+      turns[threadIdx.x] = make_float2(cosine, sine);
+    }
+    if (blockIdx.x == 0u && threadIdx.x < a.vdim) {
+      const uint32_t slot = position % a.page_tokens;
+      const uint32_t at = kv * a.vdim + threadIdx.x;
+      float value = store.projections[store.value_column + at];
+      if (store.values_out) store.values_out[at] = value;
+      if (store.first_values) {
+        const float share = *store.value_share;
+        value = (1.0f - share) * value + share * store.first_values[at];
+      }
+      store_element(page_of<uint16_t>(a, position) + value_block(a, kv, slot) +
+                        size_t{threadIdx.x} * 32u + slot % 32u,
+                    value);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < NK; ++c)
+      q[c] = turned_operand(raw[c], c * 32u + d0, a.dim, store.rotary_dims, turns);
+    if (owner)
+#pragma unroll
+      for (int c = 0; c < NK; ++c)
+        own_key[c] = turned_operand(raw_key[c], c * 32u + d0, a.dim, store.rotary_dims, turns);
+  } else {
+    const uint16_t* query = static_cast<const uint16_t*>(args.launch.query) +
+                            (size_t{row} * a.query_heads + head) * a.key_stride +
+                            8u * (lane / 16u);
+#pragma unroll
+    for (int c = 0; c < NK; ++c) q[c] = *reinterpret_cast<const i32x4*>(query + c * 32);
+  }
+
   float maximum = -INFINITY;
   float total = 0.0f;
   float* scores =
@@ -663,12 +747,19 @@ __global__ __launch_bounds__(256) void split_scores_kernel(AttentionArgs args) {
   for (uint32_t unit = begin + wave; unit < end; unit += 4u) {
     const uint32_t key0 = range.tile(unit / 2u) * kTileKeys + unit % 2u * 16u;
     const uint32_t slot = key0 % a.page_tokens;
-    const i32x4* keys = reinterpret_cast<const i32x4*>(page_of<const uint16_t>(a, key0) +
-                                                       key_block(a, kv, slot)) +
-                        lane % 16u * 4u + lane / 16u;
+    i32x4* keys = reinterpret_cast<i32x4*>(page_of<uint16_t>(a, key0) +
+                                           key_block(a, kv, slot)) +
+                  lane % 16u * 4u + lane / 16u;
     i32x4 k[NK];
 #pragma unroll
     for (int c = 0; c < NK; ++c) k[c] = keys[c * kWave];
+    if constexpr (FRESH)
+      if (unit == own_unit && lane % 16u == position % 16u)
+#pragma unroll
+        for (int c = 0; c < NK; ++c) {
+          k[c] = own_key[c];
+          keys[c * kWave] = own_key[c];
+        }
     f32x4 s = {};
 #pragma unroll
     for (int c = 0; c < NK; ++c) s = mfma_bf16(k[c], q[c], s);
@@ -719,14 +810,17 @@ constexpr uint32_t kMixRow = 40;   // bf16 values per LDS row of mixed weights (
 
 // NV = value_stride / 16, GROUP = query heads per key/value head at most.  The
 // launch is a chain of round trips (its tiles are a few KiB each): a wave's first
-// values and scores set out before the maxima are merged.  With eight waves a
-// workgroup takes all tiles of its heads and writes the gated outputs itself.
+// values and scores and the gates set out before the maxima are merged.  With eight
+// waves a workgroup takes all tiles of its heads and writes the gated outputs itself.
+// 16 heads on 4 of 128 dimensions over 5 tiles: 9.7 us with the waves' sums added one
+// wave after the other, a head's splits by a whole wave and the gates fetched last,
+// 7.2 now.
 template <int NV, int GROUP, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void split_values_kernel(AttentionArgs args) {
   __shared__ float row_maximum[64], row_inverse[64];
   __shared__ __attribute__((aligned(16))) float mix[64][GROUP];
   __shared__ __attribute__((aligned(16))) uint16_t mixed[WAVES][16 * kMixRow];
-  __shared__ f32x4 gathered[NV * kWave];
+  __shared__ f32x4 gathered[WAVES][NV * kWave];
   const Attention& a = args.attention;
   const uint32_t row = blockIdx.z;
   const uint32_t kv = blockIdx.y;
@@ -762,22 +856,42 @@ __global__ __launch_bounds__(WAVES * 64) void split_values_kernel(AttentionArgs 
   };
   if (begin + wave < end) fetch(begin + wave);
 
-  // a wave per head, a lane per score split (at most 64)
-#pragma unroll 4
-  for (uint32_t h = wave; h < heads; h += WAVES) {
-    float m = -INFINITY;
-    float t = 0.0f;
-    if (lane < args.score_splits) {
+  // the gates of this lane's outputs, needed last
+  float gate[4];
+  if constexpr (WAVES == 8) {
+    const auto& run = args.launch;
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; ++j)
+      gate[j] = run.gate ? run.gate[size_t{row} * run.gate_stride + kv * group +
+                                    min(4u * (lane / 16u) + j, group - 1u)]
+                         : 0.0f;
+  }
+
+  // sixteen lanes per head, each every sixteenth of its score splits (at most 64)
+  constexpr uint32_t kEach = kMaximumScoreSplits / 16u;
+  for (uint32_t h0 = wave * 4u; h0 < heads; h0 += WAVES * 4u) {
+    const uint32_t h = min(h0 + lane / 16u, heads - 1u);
+    float m[kEach], t[kEach];
+    float top = -INFINITY;
+#pragma unroll
+    for (uint32_t i = 0; i < kEach; ++i) {
+      const uint32_t split = i * 16u + lane % 16u;
       const float* pair =
-          args.maxima + ((size_t{row} * args.score_splits + lane) * heads + h) * 2u;
-      m = pair[0];
-      t = pair[1];
+          args.maxima +
+          ((size_t{row} * args.score_splits + min(split, args.score_splits - 1u)) * heads + h) *
+              2u;
+      m[i] = split < args.score_splits ? pair[0] : -INFINITY;
+      t[i] = pair[1];
+      top = fmaxf(top, m[i]);
     }
-    const float top = wave_max(m);
-    t = wave_sum(t * expf(m - top));
-    if (lane == 0u) {
+    top = row16_max(top);
+    float total = 0.0f;
+#pragma unroll
+    for (uint32_t i = 0; i < kEach; ++i) total += t[i] * expf(m[i] - top);
+    total = row16_sum(total);
+    if (lane % 16u == 0u) {
       row_maximum[h] = top;
-      row_inverse[h] = 1.0f / t;
+      row_inverse[h] = 1.0f / total;
     }
   }
   for (uint32_t i = threadIdx.x; i < heads * GROUP; i += blockDim.x) {
@@ -823,29 +937,33 @@ __global__ __launch_bounds__(WAVES * 64) void split_values_kernel(AttentionArgs 
     __builtin_amdgcn_wave_barrier();
   }
   // the waves' sums in order
-  for (uint32_t turn = 0; turn < static_cast<uint32_t>(WAVES); ++turn) {
-    if (wave == turn)
+  const uint32_t live = min(end - begin, static_cast<uint32_t>(WAVES));
+  if (wave < live)
 #pragma unroll
-      for (int t = 0; t < NV; ++t)
-        gathered[t * kWave + lane] = turn == 0u ? sum[t] : gathered[t * kWave + lane] + sum[t];
-    __syncthreads();
-  }
+    for (int t = 0; t < NV; ++t) gathered[wave][t * kWave + lane] = sum[t];
+  __syncthreads();
   for (uint32_t i = threadIdx.x; i < NV * kWave; i += blockDim.x) {
+    f32x4 part[WAVES];
+#pragma unroll
+    for (uint32_t w = 0; w < WAVES; ++w) part[w] = gathered[live ? min(w, live - 1u) : 0u][i];
+    f32x4 total = live ? part[0] : f32x4{};
+#pragma unroll
+    for (uint32_t w = 1; w < WAVES; ++w) total = w < live ? total + part[w] : total;
     const uint32_t d = i / kWave * 16u + i % 16u;
     if (d >= a.vdim) continue;
+#pragma unroll
     for (uint32_t j = 0; j < 4u; ++j) {
-      const uint32_t h = 4u * (i % kWave / 16u) + j;
+      const uint32_t h = 4u * (lane / 16u) + j;
       if (h >= group) continue;
       if constexpr (WAVES == 8) {
         const auto& run = args.launch;
         const uint32_t head = kv * group + h;
-        const float gate =
-            run.gate ? sigmoid_f32(run.gate[size_t{row} * run.gate_stride + head]) : 1.0f;
+        const float open = run.gate ? sigmoid_f32(gate[j]) : 1.0f;
         store_element(static_cast<uint16_t*>(run.output) + size_t{row} * run.output_stride +
-                          head * a.vdim + d, gathered[i][j] * gate);
+                          head * a.vdim + d, total[j] * open);
       } else {
         args.partials[((size_t{row} * args.value_splits + blockIdx.x) * heads + kv * group +
-                       h) * a.vdim + d] = gathered[i][j];
+                       h) * a.vdim + d] = total[j];
       }
     }
   }
@@ -1364,6 +1482,17 @@ bool valid_geometry(const Attention& a) {
          a.pages_per_slot && a.element <= QLLM_ELEMENT_F32;
 }
 
+bool valid_store(const Attention* attention, const qllm_rope_store_launch* launch) {
+  return attention && launch && valid_geometry(*attention) && launch->projections &&
+         launch->query_out && launch->rows && launch->rotary_dims % 2u == 0u &&
+         launch->rotary_dims <= attention->dim &&
+         (!launch->rotary_dims || launch->frequencies) &&
+         (!launch->first_values || launch->value_share) &&
+         launch->query_column + attention->query_heads * attention->dim <= launch->stride &&
+         launch->key_column + attention->kv_heads * attention->dim <= launch->stride &&
+         launch->value_column + attention->kv_heads * attention->vdim <= launch->stride;
+}
+
 // Most tiles a row at or below maximum_position sees.
 uint32_t maximum_tiles(const Attention& a, uint32_t maximum_position) {
   const uint64_t all = maximum_position / kTileKeys + 1u;
@@ -1380,7 +1509,7 @@ uint32_t score_splits_for(uint32_t tiles) {
 
 // Up to two tiles a wave, one workgroup of eight waves per key/value head saves the
 // launch that adds the splits: one row of 16 heads on 4, 128 dimensions, 16.2 -> 13.6
-// us over 6 tiles, 16.5 -> 15.4 over 11 and 16.5 -> 16.1 over 16.  (More heads to a
+// us over 6 tiles, 16.5 -> 15.4 over 11 and 16.5 -> 16.1 over 16 (with the scores).  (More heads to a
 // key/value head want more registers than eight waves have.)  `tiles` are the most
 // that a row up to the launch's maximum_position sees.  A captured step names the
 // model's last position there: it comes this way where the window and the kept
@@ -1499,6 +1628,49 @@ void launch_general_splits(const AttentionArgs& args, hipStream_t stream) {
   split_combine_kernel<T><<<dim3(a.query_heads, rows), 64, 0, stream>>>(args);
 }
 
+// `store`: the launch of one token rotates and stores it as well.
+int32_t launch_splits(AttentionArgs& args, const qllm_rope_store_launch* store,
+                      hipStream_t stream) {
+  const Attention& a = args.attention;
+  place_splits(args, false);
+  const dim3 score_grid(args.score_splits, a.kv_heads, args.launch.rows);
+  const auto scores = [&](auto nk) {
+    constexpr int NK = decltype(nk)::value;
+    if (store)
+      split_scores_kernel<NK, true><<<score_grid, 256, 0, stream>>>(args, *store);
+    else
+      split_scores_kernel<NK, false><<<score_grid, 256, 0, stream>>>(args, {});
+  };
+  if (a.key_stride == 64u)
+    scores(std::integral_constant<int, 2>{});
+  else if (a.key_stride == 128u)
+    scores(std::integral_constant<int, 4>{});
+  else
+    scores(std::integral_constant<int, 8>{});
+  const dim3 value_grid(args.value_splits, a.kv_heads, args.launch.rows);
+  const bool narrow = a.query_heads / a.kv_heads <= 4u;
+  const bool whole = whole_values(a, args.capacity / kTileKeys);
+  const auto values = [&](auto nv) {
+    constexpr int NV = decltype(nv)::value;
+    if (whole)
+      split_values_kernel<NV, 4, 8><<<value_grid, 512, 0, stream>>>(args);
+    else if (narrow)
+      split_values_kernel<NV, 4, 4><<<value_grid, 256, 0, stream>>>(args);
+    else
+      split_values_kernel<NV, 16, 4><<<value_grid, 256, 0, stream>>>(args);
+  };
+  if (a.value_stride == 64u)
+    values(std::integral_constant<int, 4>{});
+  else if (a.value_stride == 128u)
+    values(std::integral_constant<int, 8>{});
+  else
+    values(std::integral_constant<int, 16>{});
+  if (!whole)
+    split_combine_kernel<uint16_t>
+        <<<dim3(a.query_heads, args.launch.rows), 64, 0, stream>>>(args);
+  return launched("windowed split attention");
+}
+
 bool split_stride(uint32_t stride) {
   return stride == 64u || stride == 128u || stride == 256u;
 }
@@ -1518,14 +1690,7 @@ extern "C" size_t qllm_windowed_layer_bytes(uint32_t page_tokens, uint32_t kv_he
 extern "C" int32_t qllm_windowed_rope_store(const qllm_windowed_attention* attention,
                                             const qllm_rope_store_launch* launch,
                                             void* stream) {
-  if (!attention || !launch || !valid_geometry(*attention) || !launch->projections ||
-      !launch->query_out || !launch->rows || launch->rotary_dims % 2u ||
-      launch->rotary_dims > attention->dim ||
-      (launch->rotary_dims && !launch->frequencies) ||
-      (launch->first_values && !launch->value_share) ||
-      launch->query_column + attention->query_heads * attention->dim > launch->stride ||
-      launch->key_column + attention->kv_heads * attention->dim > launch->stride ||
-      launch->value_column + attention->kv_heads * attention->vdim > launch->stride)
+  if (!valid_store(attention, launch))
     return fail(QLLM_INVALID_ARGUMENT, "invalid windowed rotary store");
   RopeArgs args{*attention, *launch, launch->rows > 64u ? 8u : 1u};
   const uint32_t units = attention->query_heads + 2u * attention->kv_heads;
@@ -1567,9 +1732,10 @@ extern "C" size_t qllm_windowed_attention_workspace_bytes(
   return split > prompt ? split : prompt;
 }
 
-extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* attention,
-                                                const qllm_attention_launch* launch,
-                                                void* stream) {
+namespace {
+// `store`: of the one row, in the split form.
+int32_t attend(const qllm_windowed_attention* attention, const qllm_rope_store_launch* store,
+               const qllm_attention_launch* launch, void* stream) {
   if (!attention || !launch || !valid_geometry(*attention) || !launch->query ||
       !launch->output || !launch->rows ||
       launch->output_stride < attention->query_heads * attention->vdim)
@@ -1624,34 +1790,26 @@ extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* a
           qllm_windowed_attention_workspace_bytes(attention, launch->rows,
                                                   launch->maximum_position))
     return fail(QLLM_INVALID_ARGUMENT, "windowed attention workspace is too small");
-  place_splits(args, false);
-  const dim3 score_grid(args.score_splits, a.kv_heads, launch->rows);
-  if (a.key_stride == 64u)
-    split_scores_kernel<2><<<score_grid, 256, 0, hip_stream>>>(args);
-  else if (a.key_stride == 128u)
-    split_scores_kernel<4><<<score_grid, 256, 0, hip_stream>>>(args);
-  else
-    split_scores_kernel<8><<<score_grid, 256, 0, hip_stream>>>(args);
-  const dim3 value_grid(args.value_splits, a.kv_heads, launch->rows);
-  const bool narrow = a.query_heads / a.kv_heads <= 4u;
-  const bool whole = whole_values(a, args.capacity / kTileKeys);
-  const auto values = [&](auto nv) {
-    constexpr int NV = decltype(nv)::value;
-    if (whole)
-      split_values_kernel<NV, 4, 8><<<value_grid, 512, 0, hip_stream>>>(args);
-    else if (narrow)
-      split_values_kernel<NV, 4, 4><<<value_grid, 256, 0, hip_stream>>>(args);
-    else
-      split_values_kernel<NV, 16, 4><<<value_grid, 256, 0, hip_stream>>>(args);
-  };
-  if (a.value_stride == 64u)
-    values(std::integral_constant<int, 4>{});
-  else if (a.value_stride == 128u)
-    values(std::integral_constant<int, 8>{});
-  else
-    values(std::integral_constant<int, 16>{});
-  if (!whole)
-    split_combine_kernel<uint16_t>
-        <<<dim3(a.query_heads, launch->rows), 64, 0, hip_stream>>>(args);
-  return launched("windowed split attention");
+  return launch_splits(args, store, hip_stream);
+}
+}  // namespace
+
+extern "C" int32_t qllm_windowed_attention_rows(const qllm_windowed_attention* attention,
+                                                const qllm_attention_launch* launch,
+                                                void* stream) {
+  return attend(attention, nullptr, launch, stream);
+}
+
+extern "C" int32_t qllm_windowed_attention_token(const qllm_windowed_attention* attention,
+                                                 const qllm_rope_store_launch* store,
+                                                 const qllm_attention_launch* launch,
+                                                 void* stream) {
+  if (!valid_store(attention, store) || !launch || launch->rows != 1u || store->rows != 1u)
+    return fail(QLLM_INVALID_ARGUMENT, "invalid windowed attention of a token");
+  // (operands are formed of eight dimensions each)
+  if (qllm_windowed_attention_form(attention, 1u) == QLLM_ATTENTION_SPLIT &&
+      attention->dim % 8u == 0u)
+    return attend(attention, store, launch, stream);
+  const int32_t status = qllm_windowed_rope_store(attention, store, stream);
+  return status != QLLM_OK ? status : attend(attention, nullptr, launch, stream);
 }

@@ -55,6 +55,20 @@ __device__ __forceinline__ float row16_sum(float value) {
   return value;
 }
 
+// Maximum over the 16 lanes of a row (every lane gets it).
+__device__ __forceinline__ float row16_max(float value) {
+  const auto rotated = [](float v, auto control) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                           decltype(control)::value, 0xf, 0xf, true));
+  };
+  value = fmaxf(value, rotated(value, std::integral_constant<int, 0x121>{}));   // row_ror:1
+  value = fmaxf(value, rotated(value, std::integral_constant<int, 0x122>{}));   // row_ror:2
+  value = fmaxf(value, rotated(value, std::integral_constant<int, 0x124>{}));   // row_ror:4
+  value = fmaxf(value, rotated(value, std::integral_constant<int, 0x128>{}));   // row_ror:8
+  return value;
+}
+
 // Sixteen values per lane, sixteen lanes per row: lane i of a row returns the
 // row's sum of value[i].  Halves of the values change hands with a partner
 // lane in four steps (partners that differ in lane bit 3, 2, 1, 0; together

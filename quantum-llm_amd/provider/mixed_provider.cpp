@@ -973,7 +973,6 @@ void Mi355MixedProvider::enqueue_attention(Block& block, std::uint32_t rows,
   }
   store.query_out = query_.get();
   store.rows = rows;
-  status_check(qllm_windowed_rope_store(&block.attention, &store, stream_));
 
   qllm_attention_launch launch{};
   launch.query = query_.get();
@@ -986,6 +985,11 @@ void Mi355MixedProvider::enqueue_attention(Block& block, std::uint32_t rows,
   launch.maximum_position = last_position;
   launch.workspace = scratch_.get();
   launch.workspace_bytes = scratch_bytes_;
+  if (rows == 1U) {
+    status_check(qllm_windowed_attention_token(&block.attention, &store, &launch, stream_));
+    return;
+  }
+  status_check(qllm_windowed_rope_store(&block.attention, &store, stream_));
   status_check(qllm_windowed_attention_rows(&block.attention, &launch, stream_));
 }
 

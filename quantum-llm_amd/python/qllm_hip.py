@@ -302,6 +302,7 @@ SIGNATURES = {
     "qllm_windowed_attention_workspace_bytes": (c_size_t, [POINTER(WindowedAttention), c_uint32, c_uint32]),
     "qllm_windowed_attention_form": (c_uint32, [POINTER(WindowedAttention), c_uint32]),
     "qllm_windowed_attention_rows": (c_int32, [POINTER(WindowedAttention), POINTER(AttentionLaunch), c_void_p]),
+    "qllm_windowed_attention_token": (c_int32, [POINTER(WindowedAttention), POINTER(RopeStoreLaunch), POINTER(AttentionLaunch), c_void_p]),
     "qllm_latent_layer_bytes": (c_size_t, [c_uint32, c_uint32, c_uint32, c_uint32]),
     "qllm_latent_store": (c_int32, [POINTER(LatentAttention), POINTER(LatentStoreLaunch), c_void_p]),
     "qllm_latent_attention_form": (c_uint32, [POINTER(LatentAttention), c_uint32]),

@@ -448,7 +448,8 @@ class Attention:
             heads, kv, dim, vdim, key, value, window, sinks, scale, qh.ptr(self.mix),
             page_tokens, pages, self.offset, qh.ptr(self.table), qh.ptr(self.step), element)
 
-    def run(self, projections, position, slot=0, first=None, share=None):
+    def run(self, projections, position, slot=0, first=None, share=None, token=False):
+        """`token`: a single row's launches as one call."""
         rows = projections.shape[0]
         d = on(self.device, projections)
         self.step.copy_(torch.tensor([position, slot, rows, 0], dtype=torch.int32))
@@ -462,7 +463,9 @@ class Attention:
         store = qh.RopeStoreLaunch(
             qh.ptr(d), self.stride, 0, at[0], at[1], self.rotary, qh.ptr(self.frequencies),
             qh.ptr(d_first), qh.ptr(d_share), qh.ptr(kept), qh.ptr(query), rows)
-        qh.call("qllm_windowed_rope_store", ctypes.byref(self.layer), ctypes.byref(store), None)
+        if not token:
+            qh.call("qllm_windowed_rope_store", ctypes.byref(self.layer), ctypes.byref(store),
+                    None)
         size = qh.call("qllm_windowed_attention_workspace_bytes", ctypes.byref(self.layer),
                        rows, position + rows - 1)
         workspace = torch.zeros(max(size, 16), dtype=torch.uint8, device=self.device)
@@ -471,8 +474,12 @@ class Attention:
         launch = qh.AttentionLaunch(
             qh.ptr(query), d.data_ptr() + 4 * gate, self.stride, qh.ptr(out),
             self.heads * self.vdim, rows, position + rows - 1, qh.ptr(workspace), size)
-        qh.call("qllm_windowed_attention_rows", ctypes.byref(self.layer), ctypes.byref(launch),
-                None)
+        if token:
+            qh.call("qllm_windowed_attention_token", ctypes.byref(self.layer),
+                    ctypes.byref(store), ctypes.byref(launch), None)
+        else:
+            qh.call("qllm_windowed_attention_rows", ctypes.byref(self.layer),
+                    ctypes.byref(launch), None)
         torch.cuda.synchronize()
         assert np.array_equal(
             kept.cpu().numpy(),
@@ -496,6 +503,41 @@ class Attention:
         out = mo.attention_core(q, k, v, where, where, scale, window or rows, sinks,
                                 np.eye(self.heads) if mix is None else mix)
         return (out * mo.sigmoid(gate)[:, :, None]).reshape(rows, -1)
+
+
+@pytest.mark.parametrize("element,heads,kv,dim,vdim,rotary,window,sinks", [
+    (BF16, 16, 4, 128, 128, 128, 0, 0), (BF16, 8, 1, 64, 40, 16, 40, 3),
+    (BF16, 6, 2, 200, 256, 64, 33, 40), (BF16, 4, 4, 24, 16, 0, 0, 0),
+    (BF16, 4, 2, 36, 32, 36, 0, 0),      # dimensions not in eights: the two launches
+    (F32, 4, 2, 40, 24, 40, 0, 3)])      # the general form likewise
+def test_a_token_in_one_call(device, element, heads, kv, dim, vdim, rotary, window, sinks):
+    """The token's rotation and store inside the launch of its scores: outputs and
+    pages are the two launches', at the places of a token in a key fragment, a tile
+    and a page, and at pages that held something else before."""
+    rng = np.random.default_rng(dim)
+    mix = mm.bf16(np.eye(heads) + 0.2 * rng.standard_normal((heads, heads)))
+    total = 131
+    one, two = (Attention(device, element, heads, kv, dim, vdim, window, sinks, mix,
+                          dim ** -0.5, rotary) for _ in range(2))
+    projections = mm.bf16(rng.standard_normal((total, one.stride)))
+    first = mm.bf16(rng.standard_normal((total, kv * vdim)))
+    for page in one.pages + two.pages:
+        page.fill_(0x3f)                 # 0.75 in either type
+    at = 0
+    for position in (0, 1, 15, 16, 31, 32, 63, 64, 100, 127, 128, 130):
+        for layer in (one, two):
+            if position > at:
+                layer.run(projections[at:position], at)
+        share = 0.25 if position % 2 else None
+        row = slice(position, position + 1)
+        blend = dict(first=None if share is None else first[row], share=share)
+        got = one.run(projections[row], position, token=True, **blend)
+        want = two.run(projections[row], position, **blend)
+        assert np.array_equal(got, want), position
+        assert np.all(np.isfinite(want))
+        at = position + 1
+    for left, right in zip(one.pages, two.pages):
+        assert torch.equal(left, right)
 
 
 @pytest.mark.parametrize("element,heads,kv,dim,vdim,window", [
