@@ -818,6 +818,20 @@ class Recurrence:
         return mo.rms(out, 1e-5).reshape(rows, n) * self.norm * gated, np.stack(states)
 
 
+@pytest.mark.parametrize("kind", [qh.RECURRENCE_DELTA, qh.RECURRENCE_BONUS])
+@pytest.mark.parametrize("dim,rank", [(64, 8), (64, 36), (24, 96), (64, 120), (256, 128),
+                                      (64, 136), (1, 256)])
+def test_recurrence_steps_of_any_rank(device, kind, dim, rank):
+    """Single tokens at the edges of the low-rank rows that a thread holds (pieces of
+    eight, at most sixteen of them) and of the parts that are added side by side."""
+    rng = np.random.default_rng(dim + rank)
+    layer = Recurrence(device, F32, kind, 2, dim, rank, rng)
+    projections = mm.bf16(rng.standard_normal((5, layer.stride)))
+    want, _ = layer.expected(projections)
+    got = [layer.run(projections[at:at + 1]) for at in range(5)]
+    close(np.concatenate(got), want, F32, "outputs", factor=2.0)
+
+
 @pytest.mark.parametrize("element", [F32, BF16])
 @pytest.mark.parametrize("kind", [qh.RECURRENCE_DELTA, qh.RECURRENCE_BONUS])
 @pytest.mark.parametrize("heads,dim,rank", [(3, 64, 16), (2, 24, 8), (1, 128, 40), (5, 16, 1),
