@@ -28,7 +28,10 @@ constexpr uint32_t kFragment = 512;          // elements, 16 x 32
 constexpr uint32_t kSplitRows = 32;          // rows of the split form
 constexpr uint32_t kMaximumSplits = 128;      // two for a lane when the parts are added
 constexpr uint32_t kSplitsFirst = 64;         // of one tile each, before they take several
-constexpr uint32_t kValueThreads = 1024;
+constexpr uint32_t kValueThreads = 512;
+constexpr uint32_t kValueTiles = kValueThreads / 256u;   // of sixteen values, per workgroup
+
+typedef __attribute__((ext_vector_type(2))) float f32x2;
 constexpr float kLog2e = 1.4426950408889634f;
 
 using Latent = qllm_latent_attention;
@@ -196,14 +199,15 @@ __device__ __forceinline__ bool in_fours(const Latent& a, const qllm_latent_laun
 }
 
 // Gates of N times four values of a head, the first four from n on, the others 16
-// apart; no load depends on whether they exist.
+// apart, as they are stored (zeros without gates); no load depends on whether they
+// exist.
 template <int N>
-__device__ __forceinline__ void take_gates(f32x4 (&gate)[N], const Latent& a,
+__device__ __forceinline__ void load_gates(f32x4 (&gate)[N], const Latent& a,
                                            const qllm_latent_launch& run, uint32_t row,
                                            uint32_t head, uint32_t n) {
   if (!run.gate) {
 #pragma unroll
-    for (int t = 0; t < N; ++t) gate[t] = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
+    for (int t = 0; t < N; ++t) gate[t] = f32x4{};
     return;
   }
   const float* source = run.gate + size_t{row} * run.gate_stride + head * a.vdim;
@@ -218,10 +222,16 @@ __device__ __forceinline__ void take_gates(f32x4 (&gate)[N], const Latent& a,
       for (uint32_t i = 0; i < 4u; ++i)
         gate[t][i] = source[min(n + t * 16u + i, a.vdim - 1u)];
   }
+}
+
+// What the outputs are multiplied with.
+template <int N>
+__device__ __forceinline__ void open_gates(f32x4 (&gate)[N], const qllm_latent_launch& run) {
 #pragma unroll
   for (int t = 0; t < N; ++t)
 #pragma unroll
-    for (uint32_t i = 0; i < 4u; ++i) gate[t][i] = sigmoid_f32(gate[t][i]);
+    for (uint32_t i = 0; i < 4u; ++i)
+      gate[t][i] = run.gate ? sigmoid_f32(gate[t][i]) : 1.0f;
 }
 
 __device__ __forceinline__ void store_four(const Latent& a, const qllm_latent_launch& run,
@@ -382,8 +392,40 @@ __global__ __launch_bounds__(256) void latent_query_kernel(AttentionArgs args) {
                          (size_t{head} * tiles + tile) * chunks * kWave + lane;
   const float* q = source + size_t{min(column, rows - 1u)} * run.query_stride;
   f32x4 sum = {};
-  for (uint32_t c = 0; c < chunks_of(a.dim); ++c)
-    sum = mfma_bf16(weights[c * kWave], query_operand(q, c * 32u + 8u * quarter, a.dim), sum);
+  const uint32_t count = chunks_of(a.dim);
+  if (a.dim % 8u == 0u && (width | run.query_stride) % 4u == 0u &&
+      (reinterpret_cast<uintptr_t>(run.query) & 15u) == 0u) {
+    // four chunks' weights and queries in one round trip: one row of 16 heads of 128
+    // dimensions 6.0 -> 3.1 us against a chunk after the other
+    for (uint32_t c0 = 0; c0 < count; c0 += 4u) {
+      i32x4 w[4];
+      f32x4 x[4][2];
+#pragma unroll
+      for (uint32_t i = 0; i < 4u; ++i) {
+        const uint32_t c = min(c0 + i, count - 1u);
+        w[i] = weights[c * kWave];
+        const f32x4* from = reinterpret_cast<const f32x4*>(
+            q + min(c * 32u + 8u * quarter, a.dim - 8u));
+        x[i][0] = from[0];
+        x[i][1] = from[1];
+      }
+#pragma unroll
+      for (uint32_t i = 0; i < 4u; ++i) {
+        if (c0 + i >= count) continue;
+        i32x4 operand;
+#pragma unroll
+        for (uint32_t j = 0; j < 4u; ++j)
+          operand[j] = static_cast<int>(
+              pack_bf16(x[i][j / 2u][j % 2u * 2u], x[i][j / 2u][j % 2u * 2u + 1u]));
+        if ((c0 + i) * 32u + 8u * quarter >= a.dim) operand = i32x4{};
+        sum = mfma_bf16(w[i], operand, sum);
+      }
+    }
+  } else {
+    for (uint32_t c = 0; c < count; ++c)
+      sum = mfma_bf16(weights[c * kWave], query_operand(q, c * 32u + 8u * quarter, a.dim),
+                      sum);
+  }
   if (column < rows)
     *reinterpret_cast<i32x2*>(out + column * out_row + tile * 16u + 4u * quarter) =
         i32x2{static_cast<int>(pack_bf16(sum[0], sum[1])),
@@ -587,8 +629,19 @@ __host__ __device__ __forceinline__ uint32_t added_quads(const Latent& a) {
   return quads > kValueThreads ? quads : kValueThreads;
 }
 
-// The parts of one head and up to 16 rows added, then through the value map: a
-// wave per 16 values and half of the latent.
+// The parts of one head and up to 16 rows added, then through the value map: two
+// tiles of 16 values to a workgroup, a wave per tile and quarter of the latent.
+//
+// Bound by what one compute unit has to fetch and the round trips it waits for: with
+// a workgroup per head that held all of its values, one row of 16 heads of 512 latent
+// and 128 own values took 8.5 us for 33 parts (200 KiB a workgroup), and 9.2 - 10.4
+// with parts and weights all asked for at once; here a workgroup adds the parts again
+// for every 32 values but fetches a quarter of the weights: 6.6 us.
+//
+// Everything that depends on nothing is asked for first, in the order in which it is
+// waited for: the row's maxima (a wave per row), this thread's first parts, this
+// wave's weights, the gates.  Places past the end are clamped and no load is left
+// out, so that each wait leaves the later loads in flight.
 __global__ __launch_bounds__(kValueThreads) void latent_value_kernel(AttentionArgs args) {
   extern __shared__ f32x4 dynamic[];
   __shared__ float share[16][kMaximumSplits];
@@ -607,40 +660,62 @@ __global__ __launch_bounds__(kValueThreads) void latent_value_kernel(AttentionAr
       reinterpret_cast<uint16_t*>(added + added_quads(a));         // [16][stride]
   const uint32_t wave = threadIdx.x / kWave;
   const uint32_t lane = threadIdx.x % kWave;
-
-  // this wave's first weights, on their way meanwhile
   const uint32_t column = lane % 16u;
   const uint32_t quarter = lane / 16u;
-  const uint32_t chunks = packed_chunks(a.rank);
-  const uint32_t half_chunks = (chunks_of(a.rank) + 1u) / 2u;
-  const uint32_t units = value_tiles(a) * 2u;
-  constexpr uint32_t kAhead = 8;
-  i32x4 ahead[kAhead];
-  const auto weights_of = [&](uint32_t unit) {
-    return static_cast<const i32x4*>(a.value_up) +
-           ((size_t{head} * value_tiles(a) + unit / 2u) * chunks + unit % 2u * half_chunks) *
-               kWave + lane;
-  };
-  const auto count_of = [&](uint32_t unit) {
-    return unit % 2u ? chunks_of(a.rank) - half_chunks : half_chunks;
-  };
-  if (wave < units)
-#pragma unroll
-    for (uint32_t c = 0; c < kAhead; ++c)
-      if (c < count_of(wave)) ahead[c] = weights_of(wave)[c * kWave];
 
-  if (wave < rows) {
-    const uint32_t item = (row0 + wave) * a.heads + head;
-    constexpr uint32_t kEach = kMaximumSplits / kWave;
+  constexpr uint32_t kEach = kMaximumSplits / kWave;
+  constexpr uint32_t kWaves = kValueThreads / kWave;
+  const auto pair_of = [&](uint32_t row, uint32_t i) {
+    return *reinterpret_cast<const f32x2*>(
+        args.maxima + (static_cast<size_t>(min(i * kWave + lane, args.splits - 1u)) * items +
+                       size_t{row0 + row} * a.heads + head) * 2u);
+  };
+  f32x2 pairs[kEach];
+#pragma unroll
+  for (uint32_t i = 0; i < kEach; ++i) pairs[i] = pair_of(min(wave, rows - 1u), i);
+  // a row's parts over as many groups as there are; every group a row if not
+  const uint32_t per_row = max(groups / rows, 1u);
+  const uint32_t group = threadIdx.x / quads;
+  const uint32_t quad = threadIdx.x % quads;
+  const uint32_t mine = group % per_row;
+  constexpr uint32_t kPieces = 10;
+  f32x4 piece[kPieces];
+  const auto fetch_parts = [&](uint32_t row, uint32_t first) {
+    const f32x4* part = reinterpret_cast<const f32x4*>(args.sums) +
+                        (size_t{row0 + row} * a.heads + head) * quads + quad;
+#pragma unroll
+    for (uint32_t s = 0; s < kPieces; ++s)
+      piece[s] =
+          part[static_cast<size_t>(min(first + s * per_row, args.splits - 1u)) * items * quads];
+  };
+  fetch_parts(min(group / per_row, rows - 1u), mine);
+  bool fetched = true;
+  const uint32_t chunks = chunks_of(a.rank);
+  const uint32_t quarter_chunks = (chunks + 3u) / 4u;         // at most four
+  const uint32_t value_tile = blockIdx.z * kValueTiles + wave / 4u;
+  const uint32_t chunk0 = wave % 4u * quarter_chunks;
+  i32x4 weights[4];
+  const i32x4* const map =
+      static_cast<const i32x4*>(a.value_up) +
+      (size_t{head} * value_tiles(a) + min(value_tile, value_tiles(a) - 1u)) *
+          packed_chunks(a.rank) * kWave + lane;
+#pragma unroll
+  for (uint32_t c = 0; c < 4u; ++c) weights[c] = map[min(chunk0 + c, chunks - 1u) * kWave];
+  const uint32_t n = value_tile * 16u + 4u * quarter;
+  f32x4 gate[1];
+  load_gates(gate, a, run, row0 + min(column, rows - 1u), head, n);
+
+  for (uint32_t row = wave; row < rows; row += kWaves) {
+    if (row != wave)
+#pragma unroll
+      for (uint32_t i = 0; i < kEach; ++i) pairs[i] = pair_of(row, i);
     float m[kEach], t[kEach];
     float top = -INFINITY;
 #pragma unroll
     for (uint32_t i = 0; i < kEach; ++i) {
-      const uint32_t split = i * kWave + lane;
-      const float* pair =
-          args.maxima + (size_t{min(split, args.splits - 1u)} * items + item) * 2u;
-      m[i] = split < args.splits ? pair[0] : -INFINITY;
-      t[i] = split < args.splits ? pair[1] : 0.0f;
+      const bool exists = i * kWave + lane < args.splits;
+      m[i] = exists ? pairs[i][0] : -INFINITY;
+      t[i] = exists ? pairs[i][1] : 0.0f;
       top = fmaxf(top, m[i]);
     }
     top = wave_max(top);
@@ -652,30 +727,22 @@ __global__ __launch_bounds__(kValueThreads) void latent_value_kernel(AttentionAr
     }
     total = wave_sum(total);
 #pragma unroll
-    for (uint32_t i = 0; i < kEach; ++i) share[wave][i * kWave + lane] = m[i] / total;
+    for (uint32_t i = 0; i < kEach; ++i) share[row][i * kWave + lane] = m[i] / total;
   }
   __syncthreads();
-  // a row's parts over as many groups as there are; every group a row if not
-  const uint32_t per_row = max(groups / rows, 1u);
-  const uint32_t group = threadIdx.x / quads;
-  const uint32_t quad = threadIdx.x % quads;
   if (group < groups)
     for (uint32_t row = group / per_row; row < rows; row += groups / per_row) {
-      const uint32_t mine = group % per_row;
-      const f32x4* part = reinterpret_cast<const f32x4*>(args.sums) +
-                          size_t{(row0 + row) * a.heads + head} * quads + quad;
       f32x4 sum = {};
-      for (uint32_t first = mine; first < args.splits; first += 8u * per_row) {
-        f32x4 piece[8];
+      for (uint32_t first = mine; first < args.splits; first += kPieces * per_row) {
+        if (!fetched) fetch_parts(row, first);
+        fetched = false;
         // a part whose share is zero may never have been written
 #pragma unroll
-        for (uint32_t s = 0; s < 8u; ++s) {
+        for (uint32_t s = 0; s < kPieces; ++s) {
           const uint32_t split = first + s * per_row;
           const float weight = split < args.splits ? share[row][split] : 0.0f;
-          piece[s] = weight > 0.0f ? part[size_t{split} * items * quads] * weight : f32x4{};
+          sum += weight > 0.0f ? piece[s] * weight : f32x4{};
         }
-#pragma unroll
-        for (uint32_t s = 0; s < 8u; ++s) sum += piece[s];
       }
       added[(row * per_row + mine) * quads + quad] = sum;
     }
@@ -685,39 +752,35 @@ __global__ __launch_bounds__(kValueThreads) void latent_value_kernel(AttentionAr
     const uint32_t at = i % quads;
     f32x4 sum = {};
     if (row < rows)
-      for (uint32_t p = 0; p < per_row; ++p) sum += added[(row * per_row + p) * quads + at];
+      for (uint32_t first = 0; first < per_row; first += 4u) {
+        f32x4 four[4];
+#pragma unroll
+        for (uint32_t p = 0; p < 4u; ++p)
+          four[p] = added[(row * per_row + min(first + p, per_row - 1u)) * quads + at];
+#pragma unroll
+        for (uint32_t p = 0; p < 4u; ++p) sum += first + p < per_row ? four[p] : f32x4{};
+      }
     *reinterpret_cast<i32x2*>(mean + row * stride + at * 4u) =
         i32x2{static_cast<int>(pack_bf16(sum[0], sum[1])),
               static_cast<int>(pack_bf16(sum[2], sum[3]))};
   }
   __syncthreads();
-  for (uint32_t base = 0; base < units; base += kValueThreads / kWave) {
-    const uint32_t unit = base + wave;
-    f32x4 sum = {};
-    if (unit < units) {
-      const uint16_t* operand =
-          mean + column * stride + unit % 2u * half_chunks * 32u + 8u * quarter;
-      const uint32_t count = count_of(unit);
+  f32x4 sum = {};
 #pragma unroll
-      for (uint32_t c = 0; c < kAhead; ++c) {
-        if (c >= count) continue;
-        const i32x4 w = base ? weights_of(unit)[c * kWave] : ahead[c];
-        sum = mfma_bf16(w, *reinterpret_cast<const i32x4*>(operand + c * 32u), sum);
-      }
-      for (uint32_t c = kAhead; c < count; ++c)
-        sum = mfma_bf16(weights_of(unit)[c * kWave],
-                        *reinterpret_cast<const i32x4*>(operand + c * 32u), sum);
-      if (unit % 2u) added[wave * kWave + lane] = sum;
-    }
-    __syncthreads();
-    if (unit < units && unit % 2u == 0u && column < rows) {
-      sum += added[(wave + 1u) * kWave + lane];
-      const uint32_t n = unit / 2u * 16u + 4u * quarter;
-      f32x4 gate[1];
-      take_gates(gate, a, run, row0 + column, head, n);
-      store_four(a, run, row0 + column, head, n, sum * gate[0]);
-    }
-    __syncthreads();
+  for (uint32_t c = 0; c < 4u; ++c) {
+    if (c >= quarter_chunks || chunk0 + c >= chunks) continue;
+    sum = mfma_bf16(weights[c],
+                    *reinterpret_cast<const i32x4*>(mean + column * stride +
+                                                    (chunk0 + c) * 32u + 8u * quarter),
+                    sum);
+  }
+  added[wave * kWave + lane] = sum;
+  __syncthreads();
+  if (wave % 4u == 0u && value_tile < value_tiles(a) && column < rows) {
+    sum = (added[wave * kWave + lane] + added[(wave + 1u) * kWave + lane]) +
+          (added[(wave + 2u) * kWave + lane] + added[(wave + 3u) * kWave + lane]);
+    open_gates(gate, run);
+    store_four(a, run, row0 + column, head, n, sum * gate[0]);
   }
 }
 
@@ -1049,7 +1112,8 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(AttentionArgs arg
     if (row >= run.rows) continue;
     const float inverse = 1.0f / total[m];
     f32x4 gate[NV];
-    take_gates(gate, a, run, row, head, 4u * quarter);
+    load_gates(gate, a, run, row, head, 4u * quarter);
+    open_gates(gate, run);
 #pragma unroll
     for (int t = 0; t < NV; ++t)
       store_four(a, run, row, head, t * 16u + 4u * quarter, out[m][t] * inverse * gate[t]);
@@ -1254,7 +1318,8 @@ extern "C" int32_t qllm_latent_attention_rows(const qllm_latent_attention* atten
     latent_split_kernel<4><<<grid, 256, 0, hip_stream>>>(args);
   else
     latent_split_kernel<8><<<grid, 256, 0, hip_stream>>>(args);
-  latent_value_kernel<<<dim3(a.heads, row_tiles), kValueThreads, value_bytes(a),
+  const uint32_t value_parts = (value_tiles(a) + kValueTiles - 1u) / kValueTiles;
+  latent_value_kernel<<<dim3(a.heads, row_tiles, value_parts), kValueThreads, value_bytes(a),
                         hip_stream>>>(args);
   return launched("latent split attention");
 }
