@@ -432,10 +432,10 @@ __global__ void rope_table_kernel(float2* table, uint32_t rotary_dim,
 // the staged tile before it is read (the cache pages need not hold them yet);
 // the workgroup that owns the context's last tile also writes them to the
 // pages for later steps.
-template <int D, int RT, bool FUSED = false, int WAVES = kSplitWaves>
-__global__ __launch_bounds__(WAVES * 64, 2) void q4h_attention_split_kernel(
+template <int D, int RT, bool FUSED = false>
+__global__ __launch_bounds__(kSplitWaves * 64, 2) void q4h_attention_split_kernel(
     const SplitArgs launch_args) {
-  static_assert(!FUSED || WAVES == kSplitWaves, "the fused work is dealt to eight waves");
+  constexpr int WAVES = kSplitWaves;
   // a batched launch narrows the arguments to the batch of this grid layer
   SplitArgs args = launch_args;
   if (!FUSED && launch_args.batch_rows) {
@@ -507,9 +507,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void q4h_attention_split_kernel(
   // (fused: the workgroup at the end of the context also encodes the batch's
   // K/V records, lays them over its tiles and writes them to their pages -
   // about two tiles' worth of time for each of its waves.  The plain kernel
-  // deals the same way, so that both add up a context in the same order; not so
-  // the smaller workgroups of long prompts.)
-  constexpr uint32_t kTailWork = WAVES == kSplitWaves ? 2u * kSplitWaves : 0u;
+  // deals the same way, so that both add up a context in the same order.)
+  constexpr uint32_t kTailWork = 2u * kSplitWaves;
   wave_tile_range<WAVES>(context_tiles, 64u, args.split_tokens, split, gridDim.y, wave,
                          tile_first, tile_last, kTailWork);
 
@@ -1353,11 +1352,23 @@ __global__ __launch_bounds__(WAVES * 64, 2) void q4h_attention_split_kernel(
 // split partial itself - no states are merged.
 constexpr int kPromptBatches = 8;
 
+// Bound by vector instructions and by what eight waves wait for between two barriers
+// (counters, 16384 rows of 64 heads on 8: vector pipes 63 %, matrix cores 35 %).  The
+// queries are quantised in one pass over them, a tile's page is looked up an iteration
+// before its loads, and K codes, query operands and V operands are read ahead of the
+// instructions that use them: 300 rows 36.9 -> 30.0 us, 16384 rows 5.66 -> 5.67 ms.
+//
+// At head_dim 256 a wave owns one row tile, sixteen consecutive (row, head) pairs
+// whatever the group, with its query operands in registers: two row tiles' and their
+// accumulators do not fit, and LDS has no room next to 32 KiB of V operands.  Rows of
+// codes are 128 bytes there, so their 16-byte pieces are swizzled by the row.  3001
+// rows of 24 heads on 4: 281 us with a workgroup of two waves for every five rows,
+// each of which converted its own V codes, 197 here.
 template <int D>
 __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kernel(
     const SplitArgs args) {
-  static_assert(D == 128, "LDS holds eight batches' query operands at 128 only");
-  constexpr int RT = 3;
+  constexpr bool WIDE = D == 256;
+  constexpr int RT = WIDE ? 1 : 3;
   constexpr int KSTEPS = D / 64;
   constexpr int DT = D / 16;
   constexpr int ROW = D / 2;
@@ -1368,7 +1379,8 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
   constexpr int CONV_KS = CONV_V;                   // K scales, F32 per token
   constexpr int CONV_VS = CONV_KS + 256;            // V scale pairs
   constexpr int CONV = CONV_VS + 128;
-  __shared__ __attribute__((aligned(16))) uint8_t q_operands_all[kPromptBatches * Q_BYTES];
+  __shared__ __attribute__((aligned(16)))
+  uint8_t q_operands_all[WIDE ? 16 : kPromptBatches * Q_BYTES];
   __shared__ float q_scales[kPromptBatches * RT * 16];
   __shared__ uint32_t q_limits[kPromptBatches * RT * 16];
   __shared__ __attribute__((aligned(16))) uint8_t converted[2 * CONV];
@@ -1384,24 +1396,28 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
   const uint32_t splits = gridDim.y;
   const uint32_t group = args.query_heads / args.kv_heads;
 
-  // this wave's batch
-  const uint32_t batches = (args.rows + args.batch_rows - 1u) / args.batch_rows;
+  // this wave's batch: matrix rows first_matrix_row .. of all rows * group, row by row
+  const uint32_t all_matrix_rows = args.rows * group;
+  const uint32_t per_batch = WIDE ? RT * 16u : args.batch_rows * group;
+  const uint32_t batches = (all_matrix_rows + per_batch - 1u) / per_batch;
   // (the workgroups with the longest contexts are dispatched first)
   const uint32_t first_batch = (gridDim.z - 1u - blockIdx.z) * kPromptBatches;
   const uint32_t batch = first_batch + wave;
   const bool live = batch < batches;
-  const uint32_t first_row = live ? batch * args.batch_rows : 0u;
-  const uint32_t batch_rows = live ? min(args.batch_rows, args.rows - first_row) : 0u;
-  const uint32_t matrix_rows = batch_rows * group;
+  const uint32_t first_matrix_row = live ? batch * per_batch : 0u;
+  const uint32_t matrix_rows =
+      live ? min(per_batch, all_matrix_rows - first_matrix_row) : 0u;
+  const uint32_t first_row = first_matrix_row / group;
   const uint32_t first_context_tokens = args.first_context_tokens + first_row;
-  const uint32_t batch_tiles =
-      live ? (first_context_tokens + batch_rows - 1u + 63u) / 64u : 0u;
+  // tiles that the matrix row sees, and all before it
+  const auto tiles_of = [&](uint32_t matrix_row) {
+    return (args.first_context_tokens + matrix_row / group + 63u) / 64u;
+  };
+  const uint32_t batch_tiles = live ? tiles_of(first_matrix_row + matrix_rows - 1u) : 0u;
   // the workgroup's tiles: those of its last batch, cut by the grid's splits
   const uint32_t last_batch = min(first_batch + kPromptBatches, batches) - 1u;
-  const uint32_t workgroup_context =
-      args.first_context_tokens +
-      min((last_batch + 1u) * args.batch_rows, args.rows) - 1u;
-  const uint32_t workgroup_tiles = (workgroup_context + 63u) / 64u;
+  const uint32_t workgroup_tiles =
+      tiles_of(min((last_batch + 1u) * per_batch, all_matrix_rows) - 1u);
   const uint32_t quotient = workgroup_tiles / splits;
   const uint32_t remainder = workgroup_tiles - quotient * splits;
   const uint32_t tile_first = split * quotient + split * remainder / splits;
@@ -1423,11 +1439,20 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
   // holds token 16 ((R / 4) % 4) + 4 (R / 16) + R % 4); waves 0 and 1 also the
   // tile's K and V scales (lanes 0..31 fetch tokens 2l, 2l + 1; the others
   // repeat them)
-  const auto send_values = [&](uint32_t tile) {
+  constexpr uint32_t kPieces = ROW / 16;         // 16-byte pieces of a row of codes
+  constexpr uint32_t kPasses = CODES / 4096;     // KiB a wave sends of either codes
+  // where row `row` keeps piece `piece`
+  const auto place = [](uint32_t piece, uint32_t row) {
+    return WIDE ? piece ^ (row & 7u) : piece;
+  };
+  // The page of a tile, fetched an iteration before its loads set out: the first thing
+  // behind a barrier would otherwise be every wave's wait for a page table entry.
+  const auto page_for = [&](uint32_t tile) {
+    return uniform_page(args.page_table, tile * 64u / args.page_tokens);
+  };
+  const auto send_values = [&](uint32_t tile, const void* page) {
     const uint32_t lane_now = fresh_lane_index();
-    const uint32_t lane_row = lane_now >> 2;
     const uint32_t tile_begin = tile * 64u;
-    const void* page = uniform_page(args.page_table, tile_begin / args.page_tokens);
     const Q4hPlanes planes =
         q4h_planes(page, args.layer, args.page_tokens, args.kv_heads, D);
     const size_t record0 = static_cast<size_t>(kv_head) * args.page_tokens +
@@ -1435,10 +1460,15 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
     const uint32_t target = raw_values_lds + (tile & 1u) * RAW_V;
     const uint8_t* rows = uniform_pointer(planes.value_codes +
                                           (record0 + 4u * wave) * ROW);
-    copy16_to_lds(rows,
-                  (16u * ((lane_row >> 2) & 3u) + (lane_row & 3u)) * ROW +
-                      (lane_now & 3u) * 16u,
-                  target + wave * 1024u);
+#pragma unroll
+    for (uint32_t pass = 0; pass < kPasses; ++pass) {
+      // LDS row 16 wave + lane_row
+      const uint32_t lane_row = lane_now / kPieces + pass * (64u / kPieces);
+      copy16_to_lds(rows,
+                    (16u * ((lane_row >> 2) & 3u) + (lane_row & 3u)) * ROW +
+                        place(lane_now % kPieces, lane_row) * 16u,
+                    target + (wave * kPasses + pass) * 1024u);
+    }
     if (wave < 2u) {
       const uint8_t* scales = uniform_pointer(
           planes.key_scales + record0 * 2u + wave * value_scale_distance);
@@ -1446,29 +1476,39 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
     }
   };
   // waves 4..7: a quarter of the tile's K codes each
-  const auto send_keys = [&](uint32_t tile) {
+  const auto send_keys = [&](uint32_t tile, const void* page) {
     const uint32_t lane_now = fresh_lane_index();
     const uint32_t tile_begin = tile * 64u;
-    const void* page = uniform_page(args.page_table, tile_begin / args.page_tokens);
     const Q4hPlanes planes =
         q4h_planes(page, args.layer, args.page_tokens, args.kv_heads, D);
     const size_t record0 = static_cast<size_t>(kv_head) * args.page_tokens +
                            tile_begin % args.page_tokens;
-    const uint8_t* rows = uniform_pointer(planes.key_codes + record0 * ROW +
-                                          (wave - 4u) * 1024u);
-    copy16_to_lds(rows, lane_now * 16u,
-                  raw_keys_lds + (tile & 1u) * CODES + (wave - 4u) * 1024u);
+#pragma unroll
+    for (uint32_t pass = 0; pass < kPasses; ++pass) {
+      const uint32_t part = (wave - 4u) * kPasses + pass;
+      copy16_to_lds(uniform_pointer(planes.key_codes + record0 * ROW + part * 1024u),
+                    lane_now / kPieces * ROW +
+                        place(lane_now % kPieces, lane_now / kPieces) * 16u,
+                    raw_keys_lds + (tile & 1u) * CODES + part * 1024u);
+    }
   };
   const auto convert = [&](uint32_t tile) {
     uint8_t* target = converted + (tile & 1u) * CONV;
     const uint32_t source = raw_values_lds + (tile & 1u) * RAW_V;
     const uint32_t lane_now = fresh_lane_index();
-    // V: row tile `wave` of head_dim, both halves of the 64 tokens
-    u32x2 transposed;
+    // V: row tiles `wave` (and wave + 8) of head_dim, both halves of the 64 tokens
+    constexpr int OWN = DT / kPromptBatches;
+    u32x2 transposed[OWN];
     {
-      const uint32_t address =
-          source + (16u * (lane_now >> 4) + (lane_now & 15u)) * ROW + wave * 8u;
-      asm volatile("ds_read_b64_tr_b4 %0, %1" : "=v"(transposed) : "v"(address));
+      const uint32_t row = lane_now;   // 16 (lane / 16) + lane % 16
+#pragma unroll
+      for (int own = 0; own < OWN; ++own) {
+        const uint32_t dt = wave + own * kPromptBatches;
+        const uint32_t address =
+            source + row * ROW +
+            (WIDE ? place(dt / 2u, row) * 16u + dt % 2u * 8u : dt * 8u);
+        asm volatile("ds_read_b64_tr_b4 %0, %1" : "=v"(transposed[own]) : "v"(address));
+      }
     }
     uint32_t first_scale = 0u, second_scale = 0u;
     if (wave == 6u) {
@@ -1482,12 +1522,16 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
       asm volatile("ds_read_u16 %0, %1" : "=v"(first_scale) : "v"(address));
       asm volatile("ds_read_u16 %0, %1 offset:32" : "=v"(second_scale) : "v"(address));
     }
+    // (each register once: a second mention would be a copy made before the wait)
     asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(transposed), "+v"(first_scale), "+v"(second_scale)
+                 : "+v"(transposed[0]), "+v"(first_scale), "+v"(second_scale)
                  :: "memory");
+    if constexpr (OWN > 1) tie(transposed[1]);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const uint32_t x = transposed[u] ^ 0x88888888u;
+    for (int unit = 0; unit < 2 * OWN; ++unit) {
+      const int u = unit % 2;
+      const uint32_t dt = wave + unit / 2 * kPromptBatches;
+      const uint32_t x = transposed[unit / 2][u] ^ 0x88888888u;
       const uint32_t y = x >> 8;
       const f16x2 bias_low = {static_cast<_Float16>(-1032.0f),
                               static_cast<_Float16>(-1032.0f)};
@@ -1506,8 +1550,7 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
       operand[1] = __builtin_bit_cast(uint32_t, e1);
       operand[2] = __builtin_bit_cast(uint32_t, e2);
       operand[3] = __builtin_bit_cast(uint32_t, e3);
-      *reinterpret_cast<u32x4*>(target + (wave * 2u + u) * 1024u + lane_now * 16u) =
-          operand;
+      *reinterpret_cast<u32x4*>(target + (dt * 2u + u) * 1024u + lane_now * 16u) = operand;
     }
     if (wave == 6u) {
       *reinterpret_cast<float*>(target + CONV_KS + lane_now * 4u) =
@@ -1525,25 +1568,53 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
   // ---- the first tiles set out, the queries are quantised meanwhile -----------
   const bool any_tile = tile_first < tile_last;
   if (any_tile) {
-    if (wave < 4u) send_values(tile_first);
-    else send_keys(tile_first);
+    if (wave < 4u) send_values(tile_first, page_for(tile_first));
+    else send_keys(tile_first, page_for(tile_first));
   }
-  uint8_t* q_operands_mine = q_operands_all + wave * Q_BYTES;
+  uint8_t* q_operands_mine = q_operands_all + (WIDE ? 0 : wave * Q_BYTES);
   float* exchange_scale = q_scales + wave * RT * 16;
   uint32_t* exchange_limit = q_limits + wave * RT * 16;
+  // Eight high and eight low bytes' worth of a matrix row's k-step; what a lane holds
+  // is the operand as it stands.
+  const auto quantise = [&](const float (&values)[16], float inverse, i32x4& high_operand,
+                            i32x4& low_operand) {
+    uint32_t high_bytes[16], low_bytes[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      int quantized = __float2int_rn(values[j] * inverse);
+      quantized = max(-16319, min(16319, quantized));
+      const int high = (quantized + 64) >> 7;
+      const int low = quantized - (high << 7);
+      high_bytes[j] = static_cast<uint32_t>(high) & 0xffu;
+      low_bytes[j] = static_cast<uint32_t>(low) & 0xffu;
+    }
+    const int order[16] = {0, 2, 4, 6, 1, 3, 5, 7, 8, 10, 12, 14, 9, 11, 13, 15};
+#pragma unroll
+    for (int word = 0; word < 4; ++word) {
+      uint32_t high_word = 0u, low_word = 0u;
+#pragma unroll
+      for (int byte = 0; byte < 4; ++byte) {
+        high_word |= high_bytes[order[4 * word + byte]] << (8 * byte);
+        low_word |= low_bytes[order[4 * word + byte]] << (8 * byte);
+      }
+      high_operand[word] = static_cast<int>(high_word);
+      low_operand[word] = static_cast<int>(low_word);
+    }
+  };
+  i32x4 q_high[KSTEPS], q_low[KSTEPS];
   if (live) {
+    // row tiles one after the other: a lane's share of all k-steps of its matrix row
 #pragma unroll 1
-    for (uint32_t pair = 0; pair < static_cast<uint32_t>(RT * KSTEPS); ++pair) {
-      // k-step pair % KSTEPS of row tile pair / KSTEPS, as in the split kernel
-      const uint32_t rt = pair / KSTEPS;
-      const uint32_t step = pair % KSTEPS;
+    for (uint32_t rt = 0; rt < static_cast<uint32_t>(RT); ++rt) {
       const uint32_t matrix_row = 16u * rt + col;
       const bool valid = matrix_row < matrix_rows;
-      const uint32_t row = valid ? matrix_row / group : 0u;
-      const uint32_t head = kv_head * group + (valid ? matrix_row % group : 0u);
-      const size_t record =
-          static_cast<size_t>(first_row + row) * args.query_heads + head;
-      float values[16];
+      const uint32_t row_of_all = first_matrix_row + (valid ? matrix_row : 0u);
+      const uint32_t row = row_of_all / group;
+      const uint32_t head = kv_head * group + row_of_all % group;
+      const float* source =
+          args.query +
+          (static_cast<size_t>(row) * args.query_heads + head) * args.query_stride;
+      float values[KSTEPS][16];
       float maximum = 0.0f;
 #pragma unroll
       for (int h = 0; h < KSTEPS; ++h) {
@@ -1551,15 +1622,11 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
 #pragma unroll
         for (int piece = 0; piece < 4; ++piece) {
           float4 loaded = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-          if (valid)
-            loaded = *reinterpret_cast<const float4*>(
-                args.query + record * args.query_stride + d0 + 4u * piece);
-          if (static_cast<uint32_t>(h) == step) {
-            values[4 * piece + 0] = loaded.x;
-            values[4 * piece + 1] = loaded.y;
-            values[4 * piece + 2] = loaded.z;
-            values[4 * piece + 3] = loaded.w;
-          }
+          if (valid) loaded = *reinterpret_cast<const float4*>(source + d0 + 4u * piece);
+          values[h][4 * piece + 0] = loaded.x;
+          values[h][4 * piece + 1] = loaded.y;
+          values[h][4 * piece + 2] = loaded.z;
+          values[h][4 * piece + 3] = loaded.w;
           maximum = fmaxf(maximum, fmaxf(fmaxf(fabsf(loaded.x), fabsf(loaded.y)),
                                          fmaxf(fabsf(loaded.z), fabsf(loaded.w))));
         }
@@ -1567,44 +1634,30 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
       maximum = quad_row_max(maximum);
       const float scale = fmaxf(maximum * (1.0f / 16319.0f), 0x1p-100f);
       const float inverse = 1.0f / scale;
-      if (quad == 0u && step == 0u) {
+      if (quad == 0u) {
         exchange_scale[16 * rt + col] =
             scale * (1.4426950408889634f / (16.0f * sqrtf(static_cast<float>(D))));
-        exchange_limit[16 * rt + col] = first_context_tokens + row;
+        exchange_limit[16 * rt + col] =
+            valid ? args.first_context_tokens + row : first_context_tokens;
       }
-      uint32_t high_bytes[16], low_bytes[16];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        int quantized = __float2int_rn(values[j] * inverse);
-        quantized = max(-16319, min(16319, quantized));
-        const int high = (quantized + 64) >> 7;
-        const int low = quantized - (high << 7);
-        high_bytes[j] = static_cast<uint32_t>(high) & 0xffu;
-        low_bytes[j] = static_cast<uint32_t>(low) & 0xffu;
-      }
-      const int order[16] = {0, 2, 4, 6, 1, 3, 5, 7, 8, 10, 12, 14, 9, 11, 13, 15};
-      i32x4 high_operand, low_operand;
-#pragma unroll
-      for (int word = 0; word < 4; ++word) {
-        uint32_t high_word = 0u, low_word = 0u;
-#pragma unroll
-        for (int byte = 0; byte < 4; ++byte) {
-          high_word |= high_bytes[order[4 * word + byte]] << (8 * byte);
-          low_word |= low_bytes[order[4 * word + byte]] << (8 * byte);
+      for (int h = 0; h < KSTEPS; ++h) {
+        quantise(values[h], inverse, q_high[h], q_low[h]);
+        if constexpr (!WIDE) {
+          const uint32_t pair = rt * KSTEPS + h;
+          *reinterpret_cast<i32x4*>(q_operands_mine + (pair * 2u + 0u) * 1024u +
+                                    lane * 16u) = q_high[h];
+          *reinterpret_cast<i32x4*>(q_operands_mine + (pair * 2u + 1u) * 1024u +
+                                    lane * 16u) = q_low[h];
         }
-        high_operand[word] = static_cast<int>(high_word);
-        low_operand[word] = static_cast<int>(low_word);
       }
-      *reinterpret_cast<i32x4*>(q_operands_mine + (pair * 2u + 0u) * 1024u +
-                                lane * 16u) = high_operand;
-      *reinterpret_cast<i32x4*>(q_operands_mine + (pair * 2u + 1u) * 1024u +
-                                lane * 16u) = low_operand;
     }
   }
   vmem_wait<0>();
   __syncthreads();   // the first tile's raw codes and scales are in LDS
   if (any_tile) {
-    if (wave < 4u && tile_first + 1u < tile_last) send_values(tile_first + 1u);
+    if (wave < 4u && tile_first + 1u < tile_last)
+      send_values(tile_first + 1u, page_for(tile_first + 1u));
     convert(tile_first);
   }
   vmem_wait<0>();
@@ -1624,41 +1677,69 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
       for (int i = 0; i < 4; ++i) out[dt][rt][i] = 0.0f;
   }
 
+  float q_scales_of[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) q_scales_of[rt] = live ? exchange_scale[16 * rt + col] : 0.0f;
+  const uint32_t lead = wave < 4u ? 2u : 1u;   // tiles a wave's loads are ahead
+  const void* page = any_tile ? page_for(min(tile_first + lead, tile_last - 1u)) : nullptr;
+
   for (uint32_t tile = tile_first; tile < tile_last; ++tile) {
-    if (wave < 4u) {
-      if (tile + 2u < tile_last) send_values(tile + 2u);
-    } else if (tile + 1u < tile_last) {
-      send_keys(tile + 1u);
+    if (tile + lead < tile_last) {
+      if (wave < 4u)
+        send_values(tile + 2u, page);
+      else
+        send_keys(tile + 1u, page);
+      page = page_for(min(tile + lead + 1u, tile_last - 1u));
+    }
+    // K codes out of LDS (raw), on their way during the conversion
+    constexpr int KC = D / 128;
+    u32x4 key_raw[4 * KC];
+    {
+      // (by address: the compiler sees nothing written to that array)
+      typedef const __attribute__((address_space(3))) u32x4* lds_piece;
+      const uint32_t rows = raw_keys_lds + (tile & 1u) * CODES + col * ROW;
+#pragma unroll
+      for (int i = 0; i < 4 * KC; ++i)
+        key_raw[i] = *(lds_piece)(rows + i / KC * 16 * ROW +
+                                  place(4u * (i % KC) + quad, col) * 16u);
+      asm volatile("" ::: "memory");
     }
     if (tile + 1u < tile_last) convert(tile + 1u);
     if (tile < batch_tiles) {
       const uint32_t tile_begin = tile * 64u;
       const bool needs_mask = tile_begin + 64u > first_context_tokens;
       const uint8_t* operands = converted + (tile & 1u) * CONV;
-      // K codes out of LDS (raw), widened to int8 * 16
-      u32x4 key_raw[4];
-      {
-        const uint32_t key_address =
-            raw_keys_lds + (tile & 1u) * CODES + col * ROW + 16u * quad;
-        key_raw[0] = lds_read16<0 * 16 * ROW>(key_address);
-        key_raw[1] = lds_read16<1 * 16 * ROW>(key_address);
-        key_raw[2] = lds_read16<2 * 16 * ROW>(key_address);
-        key_raw[3] = lds_read16<3 * 16 * ROW>(key_address);
-        lds_wait(key_raw);
-      }
+      // a row tile's query operands, fetched behind the products of the one before
+      const auto fetch_query = [&](int rt) {
+        if constexpr (!WIDE) {
+#pragma unroll
+          for (int h = 0; h < KSTEPS; ++h) {
+            q_high[h] = *reinterpret_cast<const i32x4*>(
+                q_operands + ((rt * KSTEPS + h) * 2 + 0) * 1024);
+            q_low[h] = *reinterpret_cast<const i32x4*>(
+                q_operands + ((rt * KSTEPS + h) * 2 + 1) * 1024);
+          }
+          asm volatile("" ::: "memory");   // set out here
+        }
+      };
+      fetch_query(0);
+      // K codes widened to int8 * 16
       i32x4 key_operand[4][KSTEPS];
       float k_scale[4][4];
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
-        const u32x4 x = key_raw[st];
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          i32x4 operand;
-          operand[0] = static_cast<int>((x[2 * half] << 4) & 0xf0f0f0f0u);
-          operand[1] = static_cast<int>(x[2 * half] & 0xf0f0f0f0u);
-          operand[2] = static_cast<int>((x[2 * half + 1] << 4) & 0xf0f0f0f0u);
-          operand[3] = static_cast<int>(x[2 * half + 1] & 0xf0f0f0f0u);
-          key_operand[st][half] = operand;
+        for (int c = 0; c < KC; ++c) {
+          const u32x4 x = key_raw[st * KC + c];
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            i32x4 operand;
+            operand[0] = static_cast<int>((x[2 * half] << 4) & 0xf0f0f0f0u);
+            operand[1] = static_cast<int>(x[2 * half] & 0xf0f0f0f0u);
+            operand[2] = static_cast<int>((x[2 * half + 1] << 4) & 0xf0f0f0f0u);
+            operand[3] = static_cast<int>(x[2 * half + 1] & 0xf0f0f0f0u);
+            key_operand[st][2 * c + half] = operand;
+          }
         }
         const float4 scales = *reinterpret_cast<const float4*>(
             operands + CONV_KS + (16u * st + 4u * quad) * 4u);
@@ -1676,18 +1757,14 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
         v_scale[u][3] = __builtin_bit_cast(f16x2, pairs.w);
       }
       f16x8 p_operand[RT][2];
+      constexpr int AHEAD = WIDE ? 8 : 2;
+      f16x8 v_ahead[AHEAD];
+      const auto v_at = [&](int i) {
+        return *reinterpret_cast<const f16x8*>(operands + i * 1024 + lane * 16u);
+      };
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        asm volatile("" ::: "memory");
-        i32x4 q_high[KSTEPS], q_low[KSTEPS];
-#pragma unroll
-        for (int h = 0; h < KSTEPS; ++h) {
-          q_high[h] = *reinterpret_cast<const i32x4*>(
-              q_operands + ((rt * KSTEPS + h) * 2 + 0) * 1024);
-          q_low[h] = *reinterpret_cast<const i32x4*>(
-              q_operands + ((rt * KSTEPS + h) * 2 + 1) * 1024);
-        }
-        const float q_scale = exchange_scale[16 * rt + col];
+        const float q_scale = q_scales_of[rt];
         float score[4][4];
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
@@ -1706,6 +1783,7 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
             score[st][i] = static_cast<float>(dot) * k_scale[st][i];
           }
         }
+        if (rt + 1 < RT) fetch_query(rt + 1);
         if (needs_mask) {
           const uint32_t first_token = tile_begin + 4u * quad;
           const uint32_t limit = exchange_limit[16 * rt + col];
@@ -1714,6 +1792,12 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
 #pragma unroll
             for (int i = 0; i < 4; ++i)
               if (first_token + 16u * st + i >= limit) score[st][i] = -INFINITY;
+        }
+        if (rt == RT - 1) {
+          // the first V operands set out before the last probabilities
+#pragma unroll
+          for (int i = 0; i < AHEAD; ++i) v_ahead[i] = v_at(i);
+          asm volatile("" ::: "memory");
         }
         // online softmax, as in the split kernel
         float tile_max = score[0][0];
@@ -1754,16 +1838,17 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
           }
         running_sum[rt] += sum;
       }
+      // V operands, AHEAD of them on their way at a time
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
+      for (int i = 0; i < 2 * DT; ++i) {
+        const f16x8 v_operand = v_ahead[i % AHEAD];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const f16x8 v_operand = *reinterpret_cast<const f16x8*>(
-              operands + (dt * 2 + u) * 1024 + lane * 16u);
-#pragma unroll
-          for (int rt = 0; rt < RT; ++rt)
-            out[dt][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                v_operand, p_operand[rt][u], out[dt][rt], 0, 0, 0);
+        for (int rt = 0; rt < RT; ++rt)
+          out[i / 2][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              v_operand, p_operand[rt][i % 2], out[i / 2][rt], 0, 0, 0);
+        if (i + AHEAD < 2 * DT) {
+          v_ahead[i % AHEAD] = v_at(i + AHEAD);
+          if (i % AHEAD == AHEAD - 1) asm volatile("" ::: "memory");
         }
       }
     }
@@ -1781,8 +1866,8 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
                           : kMaskedMax;
     const uint32_t matrix_row = 16u * rt + col;
     if (matrix_row >= matrix_rows) continue;
-    const uint32_t row = first_row + matrix_row / group;
-    const uint32_t head = kv_head * group + matrix_row % group;
+    const uint32_t row = (first_matrix_row + matrix_row) / group;
+    const uint32_t head = kv_head * group + (first_matrix_row + matrix_row) % group;
     const size_t partial =
         (static_cast<size_t>(row) * args.maximum_splits + split) * args.query_heads +
         head;
@@ -2666,6 +2751,30 @@ extern "C" int32_t qllm_quantize_gqa_queries_q8(
 
 namespace {
 
+// Workgroups of 128 (row, head) pairs each, per key/value head and split.
+uint32_t shared_parts(const qllm_q4h_attention_launch& launch) {
+  const uint64_t pairs = uint64_t{launch.rows} * (launch.query_heads / launch.kv_heads);
+  return static_cast<uint32_t>((pairs + 16u * kPromptBatches - 1u) / (16u * kPromptBatches));
+}
+
+// Shared tiles at head_dim 256 where there are workgroups for two compute units in
+// three, for half of them over a short context or any over a few tiles: a tile takes
+// such a workgroup 3.3 us, a workgroup of one batch 0.86, so few of them over a long
+// context would leave the chip idle.  24 heads on 4, combine included, batches of five
+// rows (eight waves a batch, two from 768 batches on) against shared tiles: 320 / 960 /
+// 3001 rows 31 / 67 / 293 and 30 / 63 / 204 us, 100 and 320 rows after 4000 tokens 65 /
+// 82 and 43 / 66, 48 rows after 1000 32 and 25; left alone: 20 rows after 2000 22 (26),
+// 800 after 3000 188 (152 workgroups).
+bool shares_tiles(const qllm_q4h_attention_launch& launch) {
+  if (launch.head_dim != 256u || launch.split_tokens) return false;
+  const uint64_t tiles = (uint64_t{launch.first_context_tokens} + launch.rows - 1u) / 64u + 1u;
+  const uint64_t splits = launch.maximum_splits;
+  const uint32_t parts = shared_parts(launch);
+  const uint64_t workgroups = launch.kv_heads * splits * parts;
+  return parts <= 65535u && (workgroups >= 176u || tiles <= 3u * splits ||
+                             (workgroups >= 128u && tiles <= 16u * splits));
+}
+
 // any_order: workgroups may deal a batch's tiles otherwise than a launch of its own
 int32_t attend_batches(const qllm_q4h_attention_launch* launch, uint32_t batch_rows,
                        bool any_order) {
@@ -2721,21 +2830,12 @@ int32_t attend_batches(const qllm_q4h_attention_launch* launch, uint32_t batch_r
   args.batch_rows = batch_rows;
   const dim3 grid(launch->kv_heads, splits, batches);
   const hipStream_t stream = as_stream(launch->stream);
-  // At head_dim 256 a workgroup of eight waves fills a compute unit's LDS, and its
-  // prologue and the merge of its states, 20 us, stand between two workgroups; of two
-  // waves three fit and hide each other's, but a tile costs them 1.03 us of the compute
-  // unit against 0.86.  24 heads on 4, five rows a batch (no other geometry was timed):
-  // whole prompts of 960 / 3001 rows (768 / 2404 workgroups, 8 / 24 tiles on average)
-  // 84 / 383 us with eight waves, 68 / 303 with two; 320 rows over 4320 tokens cut
-  // three ways (768, 22) 119 and 101; 1000 rows over 9000 (800, 133) 512 and 603.
-  // Where fewer workgroups than three a compute unit leave waves idle, eight share a
-  // context better: 640 rows over 4640 tokens (512, 66) 171 us against 220.
-  const uint64_t middle = uint64_t{launch->first_context_tokens} + launch->rows / 2u;
   int32_t status = QLLM_OK;
-  if (any_order && launch->head_dim == 256u && row_tiles == 2u &&
-      uint64_t{grid.x} * grid.y * grid.z >= 768u && middle <= uint64_t{splits} * 48u * 64u) {
-    q4h_attention_split_kernel<256, 2, false, 2><<<grid, 128, 0, stream>>>(args);
-    status = launched("Q4H attention split");
+  if (any_order && shares_tiles(*launch)) {
+    const uint32_t parts = shared_parts(*launch);
+    q4h_prompt_attention_kernel<256>
+        <<<dim3(launch->kv_heads, splits, parts), kPromptBatches * 64, 0, stream>>>(args);
+    status = launched("Q4H prompt attention");
   } else {
     status = launch->head_dim == 128u ? launch_split<128>(args, row_tiles, grid, stream)
                                       : launch_split<256>(args, row_tiles, grid, stream);
@@ -2760,6 +2860,11 @@ extern "C" int32_t qllm_attention_paged_q4h_batched(
 extern "C" int32_t qllm_attention_paged_q4h_batched_any_order(
     const qllm_q4h_attention_launch* launch, uint32_t batch_rows) {
   return attend_batches(launch, batch_rows, true);
+}
+
+extern "C" uint32_t qllm_attention_paged_q4h_shares_tiles(
+    const qllm_q4h_attention_launch* launch, uint32_t batch_rows) {
+  return launch && launch->kv_heads && batch_rows && shares_tiles(*launch) ? 1u : 0u;
 }
 
 extern "C" int32_t qllm_attention_paged_q4h_prompt(

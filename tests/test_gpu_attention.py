@@ -258,11 +258,11 @@ def test_splits_are_added_alike_in_every_form(device, splits, d, gated, kind, sh
 
 
 @pytest.mark.parametrize("total,first,Q,KV,batch,splits", [
-    (958, 1, 24, 4, 5, 1),      # 768 workgroups: two waves each; the last has 3 rows
+    (958, 1, 24, 4, 5, 1),      # 768 workgroups of a batch; the last has 3 rows
     (93, 70, 16, 8, 16, 16),    # splits without a tile
     (120, 1000, 12, 2, 5, 16)])
 def test_large_batched_launches_of_256_dimensions(device, total, first, Q, KV, batch, splits):
-    """Batches enough for workgroups of two waves: the launch that is free in its
+    """Batches enough to share tiles: the launch that is free in its
     order takes them and gives the oracle's attention and, up to the rounding of the
     probabilities, what launches of a batch each compute; the other one gives those
     bit for bit."""
@@ -303,6 +303,44 @@ def test_large_batched_launches_of_256_dimensions(device, total, first, Q, KV, b
         gu.assert_close(got[row:row + rows], single, rtol=3e-3, atol=3e-4,
                         what="batched vs single")
         assert np.array_equal(exact_order[row:row + rows], single), row
+
+
+@pytest.mark.parametrize("total,first,Q,KV,gated,page_tokens,splits", [
+    (1, 1, 3, 1, False, 64, 1),          # one row at the cache's first token
+    (43, 1, 3, 1, True, 64, 1),          # 129 (row, head) pairs: a workgroup for the last
+    (50, 60, 10, 2, False, 64, 3),       # row tiles begin inside a row; a batch across pages
+    (64, 700, 16, 8, True, 256, 8),      # splits of a tile or two
+    (200, 1, 8, 1, False, 64, 2),        # splits that the first rows do not reach
+    (97, 129, 26, 2, True, 256, 2)])     # thirteen heads to a key/value head
+def test_shared_tiles_of_256_dimensions(device, total, first, Q, KV, gated, page_tokens, splits):
+    """128 (row, head) pairs per workgroup on shared tiles: the oracle's attention."""
+    d = 256
+    rng = np.random.default_rng(total + Q)
+    tokens = first + total - 1
+    keys = rng.standard_normal((tokens, KV, d)).astype(np.float32)
+    values = rng.standard_normal((tokens, KV, d)).astype(np.float32)
+    pages = synth.q4h_pages(keys, values, page_tokens, 1, 0)
+    stride = d * (2 if gated else 1)
+    query = ol.bf16_round(rng.standard_normal((total, Q, stride)).astype(np.float32))
+    d_pages = [gu.device_tensor(page, device) for page in pages]
+    table = torch.tensor([page.data_ptr() for page in d_pages], dtype=torch.int64,
+                         device=device)
+    d_query = gu.device_tensor(query, device)
+    maxima = torch.zeros((total, splits, Q), device=device)
+    sums = torch.zeros_like(maxima)
+    outputs = torch.zeros((total, splits, Q, d), device=device)
+    out = torch.full((total, Q, d), float("nan"), device=device)
+    launch = qh.Q4hAttentionLaunch(
+        qh.ptr(d_query), 0, 0, qh.ptr(table), qh.ptr(out), qh.ptr(maxima), qh.ptr(sums),
+        qh.ptr(outputs), first, total, 0, page_tokens, Q, KV, d, 0, splits, stride,
+        int(gated), qh.OUT_F32, None)
+    batch = 32 // (Q // KV)
+    assert qh.call("qllm_attention_paged_q4h_shares_tiles", launch, batch) == 1
+    qh.call("qllm_attention_paged_q4h_batched_any_order", launch, batch)
+    torch.cuda.synchronize()
+    shape = ol.AttentionShape(total, Q, KV, d, first, page_tokens, 0, int(gated))
+    gu.assert_close(out.cpu().numpy(), ol.attention_q4h(shape, query, pages, "f64"),
+                    what="shared tiles")
 
 
 @pytest.mark.parametrize("total,first,Q,KV,gated,batch,splits", [
