@@ -2032,6 +2032,9 @@ __global__ __launch_bounds__(256) void attention_few_splits_kernel(
   float sum = sums[0];
   f32x4 result = part[0];
   if constexpr (SPLITS > 1u) {
+    // (the weighted sums are rounded before they are added, as where they are
+    // exchanged between lanes)
+#pragma clang fp contract(off)
     float top = kMaskedMax;
 #pragma unroll
     for (uint32_t s = 0; s < SPLITS; ++s) top = fmaxf(top, maximum[s]);
@@ -2039,7 +2042,7 @@ __global__ __launch_bounds__(256) void attention_few_splits_kernel(
 #pragma unroll
     for (uint32_t s = 0; s < SPLITS; ++s) {
       const float weight = __builtin_amdgcn_exp2f(maximum[s] - top);
-      sums[s] = __fmul_rn(sums[s], weight);
+      sums[s] *= weight;
 #pragma unroll
       for (int i = 0; i < 4; ++i) result[i] = fmaf(part[s][i], weight, result[i]);
     }
@@ -2047,7 +2050,7 @@ __global__ __launch_bounds__(256) void attention_few_splits_kernel(
 #pragma unroll
     for (uint32_t step = SPLITS / 2u; step > 0u; step /= 2u)
 #pragma unroll
-      for (uint32_t s = 0; s < step; ++s) sums[s] = __fadd_rn(sums[s], sums[s + step]);
+      for (uint32_t s = 0; s < step; ++s) sums[s] += sums[s + step];
     sum = sums[0];
   }
 #pragma unroll
