@@ -87,9 +87,11 @@ __device__ __forceinline__ void copy_carry(const RecurrenceArgs& args) {
 // A token's launch is a workgroup per head and bound by its chain of round trips:
 // whatever does not depend on another load is asked for before the first barrier,
 // sums over groups or waves read their parts side by side, and where every thread has
-// all its rows no read waits behind a condition.  A gated step of 16 heads of 64 x 128:
-// 7.9 -> 6.6 us, a delta or bonus step of 32 heads of 64 7.2 -> 6.7.  (256 threads with
-// sixteen rows each take the same time.)
+// as many rows as the kernel holds (FULL) no read waits behind a condition.  Launches
+// back to back, rank 64, against every read behind a condition and sums one part after
+// the other: gated steps of 16 heads of 64 x 64 / 64 x 128 / 128 x 128 5.7 / 6.8 / 8.1
+// -> 4.6 / 4.9 / 5.7 us, delta steps of 32 heads of 64 / 128 / 256 6.6 / 9.2 / 26.1 ->
+// 5.6 / 6.9 / 22.3.  (256 threads with sixteen rows each take the same time.)
 
 // A channel's row of the low-rank map: four threads to a channel, each every fourth
 // piece of eight.  Ranks past 128, and rows not made of such pieces, are read where
@@ -156,15 +158,25 @@ __device__ __forceinline__ float owners_sum(float value, float* scratch, uint32_
   return total;
 }
 
-// Sum of `groups` parts, `stride` apart.
+// Sum of `groups` parts, `stride` apart: sixteen at a time, what is left four at a time
+// (with the last of sixteen read again and again, the five parts of a state of 192 rows
+// and columns cost a delta step 3 us).
 __device__ __forceinline__ float parts_sum(const float* part, uint32_t groups, uint32_t stride) {
   float sum = 0.0f;
-  for (uint32_t first = 0; first < groups; first += 16u) {
+  uint32_t first = 0;
+  for (; first + 16u <= groups; first += 16u) {
     float mine[16];
 #pragma unroll
-    for (uint32_t i = 0; i < 16u; ++i) mine[i] = part[min(first + i, groups - 1u) * stride];
+    for (uint32_t i = 0; i < 16u; ++i) mine[i] = part[(first + i) * stride];
 #pragma unroll
-    for (uint32_t i = 0; i < 16u; ++i) sum += first + i < groups ? mine[i] : 0.0f;
+    for (uint32_t i = 0; i < 16u; ++i) sum += mine[i];
+  }
+  for (; first < groups; first += 4u) {
+    float mine[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; ++i) mine[i] = part[min(first + i, groups - 1u) * stride];
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; ++i) sum += first + i < groups ? mine[i] : 0.0f;
   }
   return sum;
 }
@@ -952,6 +964,9 @@ void launch_chunks_of(const RecurrenceArgs& args, hipStream_t stream) {
   }
 }
 
+// Few rows a thread have an instance of four: of sixteen conditional ones, delta steps of
+// 32 heads of 16 / 32 / 48 took 11.4 / 8.6 / 8.7 us, of four 7.3 / 6.3 / 6.5; gated ones
+// of 16 heads of 16 x 16 6.1 and 5.1.
 template <typename T>
 void launch_gated_step(const RecurrenceArgs& args, hipStream_t stream) {
   const uint32_t dim = args.layer.dim;
@@ -960,8 +975,14 @@ void launch_gated_step(const RecurrenceArgs& args, hipStream_t stream) {
   const uint32_t rows = (dim + groups - 1u) / groups;
   const bool whole = groups * vdim == 1024u && rows * groups == dim;
   const dim3 grid(args.layer.heads);
-  if (rows == 8u && whole)
+  if (whole && rows == 4u)
+    gated_step_kernel<T, 4, true><<<grid, 1024, 0, stream>>>(args);
+  else if (whole && rows == 8u)
     gated_step_kernel<T, 8, true><<<grid, 1024, 0, stream>>>(args);
+  else if (whole && rows == 16u)
+    gated_step_kernel<T, 16, true><<<grid, 1024, 0, stream>>>(args);
+  else if (rows <= 4u)
+    gated_step_kernel<T, 4, false><<<grid, 1024, 0, stream>>>(args);
   else if (rows <= 16u)
     gated_step_kernel<T, 16, false><<<grid, 1024, 0, stream>>>(args);
   else
@@ -982,6 +1003,8 @@ void launch_step(const RecurrenceArgs& args, hipStream_t stream) {
     recurrence_step_kernel<T, 4, true><<<grid, 1024, 0, stream>>>(args);
   else if (dim == 128u)
     recurrence_step_kernel<T, 16, true><<<grid, 1024, 0, stream>>>(args);
+  else if (rows <= 4u)
+    recurrence_step_kernel<T, 4, false><<<grid, 1024, 0, stream>>>(args);
   else if (rows <= 16u)
     recurrence_step_kernel<T, 16, false><<<grid, 1024, 0, stream>>>(args);
   else

@@ -459,6 +459,27 @@ def test_gated_linear_attention_in_portions(device, element, heads, dim, vdim, r
     close(layer.run(projections), want, element, "whole", factor=2.0)
 
 
+# (state rows of a thread, and whether all threads have as many: 1024 / vdim groups share dim)
+@pytest.mark.parametrize("element", [F32, BF16])
+@pytest.mark.parametrize("heads,dim,vdim,rank", [
+    (2, 64, 64, 64), (2, 16, 256, 8),        # 4, all
+    (2, 64, 128, 64), (1, 128, 64, 128),     # 8, all
+    (1, 128, 128, 136), (1, 64, 256, 120),   # 16, all; a rank past what a thread holds
+    (3, 16, 16, 24), (2, 32, 64, 64),        # 1 and 2 of 4
+    (1, 48, 96, 16), (1, 200, 60, 7)])       # 5 and 12 of 16
+def test_gated_steps_of_every_form(device, element, heads, dim, vdim, rank):
+    """Single tokens one after the other, each from the state that the one before left."""
+    rng = np.random.default_rng(dim + vdim)
+    layer = Gated(device, element, heads, dim, vdim, rank, 9.0, rng)
+    projections = mm.bf16(rng.standard_normal((6, layer.stride)))
+    want, states = layer.expected(projections)
+    got = np.concatenate([layer.run(projections[at:at + 1]) for at in range(6)])
+    close(got, want, element, "outputs", factor=2.0)
+    n = heads * dim * vdim
+    state = layer.state[layer.slot_stride:layer.slot_stride + n].cpu().numpy()
+    close(state.reshape(heads, dim, vdim).astype(np.float64), states, F32, "state", factor=4.0)
+
+
 def test_decays_near_both_ends(device):
     """Gates that keep nearly everything over the whole sequence, and gates that
     forget at once (whose logarithm a plain exponential would lose)."""

@@ -820,7 +820,8 @@ class Recurrence:
 
 @pytest.mark.parametrize("kind", [qh.RECURRENCE_DELTA, qh.RECURRENCE_BONUS])
 @pytest.mark.parametrize("dim,rank", [(64, 8), (64, 36), (24, 96), (64, 120), (256, 128),
-                                      (64, 136), (1, 256)])
+                                      (64, 136), (1, 256), (16, 64), (32, 64), (48, 16),
+                                      (96, 64), (128, 64), (192, 40)])
 def test_recurrence_steps_of_any_rank(device, kind, dim, rank):
     """Single tokens at the edges of the low-rank rows that a thread holds (pieces of
     eight, at most sixteen of them) and of the parts that are added side by side."""
