@@ -10,6 +10,8 @@ namespace qllm {
 namespace {
 
 constexpr int kHeld = 4;   // most 16-byte pieces of a row a thread keeps in registers
+// Rows up to which a thread per piece asks for all that it needs at first
+constexpr uint32_t kFewRows = 512;
 
 struct NormArgs {
   qllm_stream_norm_launch launch;
@@ -96,10 +98,14 @@ __device__ __forceinline__ void pad_row(void* output, uint32_t row, uint32_t wid
 // For a decoded token this is one workgroup whose time is the memory round trips it
 // waits for one after the other, 0.7 to 1.5 us each.  So all that it needs - partial
 // sums, norm weights, the previous token's row and the blends - is asked for before
-// the first sum over the row, with HELD = 1 (a thread per 16 bytes; registers of more
-// pieces would not hold it, and many rows hide each other's trips).  With the lookup of
+// the first sum over the row, with HELD = 1 (a thread per 16 bytes).  With the lookup of
 // the first layer's rows in the same launch (TABLE) a token of four layers takes 236 ->
 // 227 us at width 2048, 263 -> 253 in 32 bits.
+// More pieces a thread fetch weights and blends where they use them, and none for
+// pieces that the row does not have: all of it asked for first cost norms of 3000 rows of
+// 5120 (plain / with blends) 38 -> 45 / 80 -> 97 us, of one row 4.0 -> 4.5, and of rows
+// enough to hide each other's trips also with one piece a thread: 3000 rows of 512 with
+// four partial sums 8.2 -> 9.5 us (from 800 rows on the two differ by less than 4 %).
 template <typename T, int HELD, bool TABLE>
 __global__ __launch_bounds__(1024) void stream_norm_wide_kernel(NormArgs args) {
   __shared__ float scratch[16];
@@ -116,25 +122,30 @@ __global__ __launch_bounds__(1024) void stream_norm_wide_kernel(NormArgs args) {
                                            l.step[kStepSlot] * shift.slot_stride)
           : nullptr;
   const bool writes = TABLE || (l.partial_count && !l.branch_weight);
-  f32x4 held[HELD], weight[2][HELD], before[HELD], mu[HELD == 1 ? 6 : 1];
+  constexpr bool kFirst = HELD == 1;   // all loads set out before the first sum
+  f32x4 held[HELD], before[HELD], weight[2], branch, mu[6];
   float squares = 0.0f;
-#pragma unroll
-  for (int i = 0; i < HELD; ++i) {
-    const uint32_t piece = min(threadIdx.x + i * blockDim.x, pieces - 1u);
+  if constexpr (kFirst) {
+    const uint32_t piece = min(threadIdx.x, pieces - 1u);
 #pragma unroll
     for (int output = 0; output < 2; ++output)
       if (l.weight[output])
-        weight[output][i] = reinterpret_cast<const f32x4*>(l.weight[output])[piece];
-    if (l.branch_weight)
-      before[i] = reinterpret_cast<const f32x4*>(l.input + size_t{row} * l.width)[piece];
-    if constexpr (HELD == 1)
-      if (shifted) {
+        weight[output] = reinterpret_cast<const f32x4*>(l.weight[output])[piece];
+    if (l.branch_weight) {
+      before[0] = reinterpret_cast<const f32x4*>(l.input + size_t{row} * l.width)[piece];
+      branch = reinterpret_cast<const f32x4*>(l.branch_weight)[piece];
+    }
+    if (shifted) {
 #pragma unroll
-        for (uint32_t s = 0; s < 6u; ++s)
-          if (s < shift.count) mu[s] = reinterpret_cast<const f32x4*>(shift.mu[s])[piece];
-        if (carried) before[i] = carried[piece];
-      }
+      for (uint32_t s = 0; s < 6u; ++s)
+        if (s < shift.count) mu[s] = reinterpret_cast<const f32x4*>(shift.mu[s])[piece];
+      if (carried) before[0] = carried[piece];
+    }
   }
+  const auto weight_at = [&](int output, uint32_t piece) {
+    return kFirst ? weight[output]
+                  : reinterpret_cast<const f32x4*>(l.weight[output])[piece];
+  };
 #pragma unroll
   for (int i = 0; i < HELD; ++i) {
     const uint32_t piece = threadIdx.x + i * blockDim.x;
@@ -147,11 +158,15 @@ __global__ __launch_bounds__(1024) void stream_norm_wide_kernel(NormArgs args) {
     for (int c = 0; c < 4; ++c) squares = fmaf(held[i][c], held[i][c], squares);
   }
   if (!TABLE && l.branch_weight) {
-    f32x4 branch[HELD];
+    f32x4 branches[HELD];
 #pragma unroll
-    for (int i = 0; i < HELD; ++i)
-      branch[i] = reinterpret_cast<const f32x4*>(
-          l.branch_weight)[min(threadIdx.x + i * blockDim.x, pieces - 1u)];
+    for (int i = 0; i < HELD; ++i) {
+      const uint32_t piece = threadIdx.x + i * blockDim.x;
+      if (kFirst) branches[i] = branch;
+      if (kFirst || piece >= pieces) continue;
+      before[i] = reinterpret_cast<const f32x4*>(l.input + size_t{row} * l.width)[piece];
+      branches[i] = reinterpret_cast<const f32x4*>(l.branch_weight)[piece];
+    }
     const float unit =
         inverse_rms(block_sum(squares, scratch), l.width, l.branch_epsilon);
     squares = 0.0f;
@@ -159,7 +174,7 @@ __global__ __launch_bounds__(1024) void stream_norm_wide_kernel(NormArgs args) {
     for (int i = 0; i < HELD; ++i) {
       const uint32_t piece = threadIdx.x + i * blockDim.x;
       if (piece >= pieces) continue;
-      held[i] = before[i] + held[i] * unit * branch[i] * l.branch_scale;
+      held[i] = before[i] + held[i] * unit * branches[i] * l.branch_scale;
       reinterpret_cast<f32x4*>(l.stream_out + size_t{row} * l.width)[piece] = held[i];
 #pragma unroll
       for (int c = 0; c < 4; ++c) squares = fmaf(held[i][c], held[i][c], squares);
@@ -174,28 +189,23 @@ __global__ __launch_bounds__(1024) void stream_norm_wide_kernel(NormArgs args) {
       const uint32_t piece = threadIdx.x + i * blockDim.x;
       if (piece >= pieces) continue;
       put4<T>(l.output[output], size_t{row} * l.stride[output] + piece * 4u,
-              held[i] * inverse * weight[output][i]);
+              held[i] * inverse * weight_at(output, piece));
     }
     pad_row<T>(l.output[output], row, l.width, l.stride[output]);
   }
   if (!shifted) return;
 
   float before_inverse = 0.0f;
-  if (row == 0u) {   // takes the norm the request carries, already weighted
-    if constexpr (HELD > 1) {
-#pragma unroll
-      for (int i = 0; i < HELD; ++i)
-        before[i] = carried[min(threadIdx.x + i * blockDim.x, pieces - 1u)];
-    }
-  } else {
+  if (!kFirst || row) {   // row 0 takes the norm the request carries, already weighted
     float before_squares = 0.0f;
 #pragma unroll
     for (int i = 0; i < HELD; ++i) {
       const uint32_t piece = threadIdx.x + i * blockDim.x;
       before[i] = f32x4{};
       if (piece >= pieces) continue;
-      before[i] = TABLE ? table_value4(args, row - 1u, piece)
-                        : stream_value4(l, row - 1u, piece);
+      before[i] = !kFirst && row == 0u ? carried[piece]
+                  : TABLE              ? table_value4(args, row - 1u, piece)
+                                       : stream_value4(l, row - 1u, piece);
 #pragma unroll
       for (int c = 0; c < 4; ++c)
         before_squares = fmaf(before[i][c], before[i][c], before_squares);
@@ -206,17 +216,20 @@ __global__ __launch_bounds__(1024) void stream_norm_wide_kernel(NormArgs args) {
   for (int i = 0; i < HELD; ++i) {
     const uint32_t piece = threadIdx.x + i * blockDim.x;
     if (piece >= pieces) continue;
-    const f32x4 here = held[i] * inverse * weight[0][i];
-    const f32x4 there =
-        row == 0u ? before[i] : before[i] * before_inverse * weight[0][i];
-#pragma unroll
-    for (uint32_t s = 0; s < 6u; ++s) {
-      if (s >= shift.count) break;
-      const f32x4 blend =
-          HELD == 1 ? mu[s % (HELD == 1 ? 6u : 1u)]
-                    : reinterpret_cast<const f32x4*>(shift.mu[s])[piece];
+    const f32x4 own = weight_at(0, piece);
+    const f32x4 here = held[i] * inverse * own;
+    const f32x4 there = row == 0u ? before[i] : before[i] * before_inverse * own;
+    const auto blend = [&](uint32_t s, const f32x4& share) {
       put4<T>(shift.output[s], size_t{row} * l.stride[0] + piece * 4u,
-              here + (there - here) * blend);
+              here + (there - here) * share);
+    };
+    if constexpr (kFirst) {
+#pragma unroll
+      for (uint32_t s = 0; s < 6u; ++s)
+        if (s < shift.count) blend(s, mu[s]);
+    } else {
+      for (uint32_t s = 0; s < shift.count; ++s)
+        blend(s, reinterpret_cast<const f32x4*>(shift.mu[s])[piece]);
     }
     if (row + 1u == l.rows) reinterpret_cast<f32x4*>(shift.last)[piece] = here;
   }
@@ -339,7 +352,7 @@ void launch_norm(const NormArgs& args, bool wide, hipStream_t stream) {
   if (pieces > threads * kHeld) threads = 1024u;
   if (!wide || pieces > threads * kHeld)
     stream_norm_narrow_kernel<T, TABLE><<<l.rows, 256, 0, stream>>>(args);
-  else if (pieces <= threads)
+  else if (pieces <= threads && l.rows <= kFewRows)
     stream_norm_wide_kernel<T, 1, TABLE><<<l.rows, threads, 0, stream>>>(args);
   else
     stream_norm_wide_kernel<T, kHeld, TABLE><<<l.rows, threads, 0, stream>>>(args);

@@ -369,7 +369,7 @@ def test_token_shift_carries_the_last_norm(device, element, width):
 
 @pytest.mark.parametrize("element", [F32, BF16])
 @pytest.mark.parametrize("width,rows", [(64, 1), (90, 3), (2048, 1), (2048, 20), (4096, 17),
-                                        (8192, 2)])
+                                        (8192, 2), (5120, 4), (512, 512), (512, 513)])
 @pytest.mark.parametrize("shifted", [False, True])
 def test_first_norm_looks_its_rows_up(device, element, width, rows, shifted):
     """Rows of a thread per piece, of several and of no whole pieces: the same bits as the
