@@ -674,16 +674,22 @@ int32_t qllm_attention_paged_q4h_batched(const qllm_q4h_attention_launch* launch
                                          uint32_t batch_rows);
 /* The same batches, free in the order in which a batch's tiles are added up: at
  * head_dim 256 launches of many rows, or over a short context, share every cache tile
- * between 128 (row, head) pairs.  Such a batch differs from a launch of its own by
+ * between 128 (row, head) pairs (qllm_attention_paged_q4h_shares_tiles).  Such a batch differs from a launch of its own by
  * other F32 sums and by binary16 probabilities that were rounded relative to other
  * running maxima (a few 1e-4 of the values' magnitude), and by how much depends on
  * the launch's other rows; against 64 bits neither is closer.  For prompts. */
 int32_t qllm_attention_paged_q4h_batched_any_order(
     const qllm_q4h_attention_launch* launch, uint32_t batch_rows);
 /* 1 where that launch, with the maximum_splits it has, shares cache tiles between
- * 128 (row, head) pairs (head_dim 256, rows enough or a short context), else 0. */
+ * 128 (row, head) pairs (head_dim 256; chosen by estimates of the two forms), else 0. */
 uint32_t qllm_attention_paged_q4h_shares_tiles(
     const qllm_q4h_attention_launch* launch, uint32_t batch_rows);
+/* Splits, 1 to `most`, with which that launch takes the least time on shared tiles, or
+ * 0 where batches of their own in `batch_splits` splits (qllm_attention_paged_q4h_batched)
+ * take no more.  Reads the launch's sizes alone. */
+uint32_t qllm_attention_paged_q4h_shared_splits(
+    const qllm_q4h_attention_launch* launch, uint32_t batch_rows, uint32_t batch_splits,
+    uint32_t most);
 
 /* The same attention for a long run of prompt rows (head_dim 128,
  * split_tokens 0): eight consecutive batches share a workgroup, which fetches

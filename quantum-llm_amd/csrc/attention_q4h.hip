@@ -26,6 +26,7 @@
 #include "attention_common.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <utility>
 
 namespace qllm {
@@ -2760,22 +2761,72 @@ uint32_t shared_parts(const qllm_q4h_attention_launch& launch) {
   return static_cast<uint32_t>((pairs + 16u * kPromptBatches - 1u) / (16u * kPromptBatches));
 }
 
-// Shared tiles at head_dim 256 where there are workgroups for two compute units in
-// three, for half of them over a short context or any over a few tiles: a tile takes
-// such a workgroup 3.3 us, a workgroup of one batch 0.86, so few of them over a long
-// context would leave the chip idle.  24 heads on 4, combine included, batches of five
-// rows (eight waves a batch, two from 768 batches on) against shared tiles: 320 / 960 /
-// 3001 rows 31 / 67 / 293 and 30 / 63 / 204 us, 100 and 320 rows after 4000 tokens 65 /
-// 82 and 43 / 66, 48 rows after 1000 32 and 25; left alone: 20 rows after 2000 22 (26),
-// 800 after 3000 188 (152 workgroups).
-bool shares_tiles(const qllm_q4h_attention_launch& launch) {
-  if (launch.head_dim != 256u || launch.split_tokens) return false;
-  const uint64_t tiles = (uint64_t{launch.first_context_tokens} + launch.rows - 1u) / 64u + 1u;
-  const uint64_t splits = launch.maximum_splits;
+// What a launch at head_dim 256 takes, combine included, in microseconds: with cache
+// tiles shared by 128 (row, head) pairs, and with a workgroup of eight waves to a batch.
+// A workgroup of either has a compute unit to itself, so what counts is the rounds of
+// them and the tiles that a round walks; a batch's waves walk a tile each and merge
+// their states, a wave of the others walks all and has no state to merge.  Fitted to
+// 5500 launches over eight head layouts (24 on 4, 16 on 8, 16 on 2, 64 on 8, 16 on 16,
+// 8 on 1, 24 on 2, 32 on 32), 2 to 3000 rows after 0 to 9000 tokens, one to eight
+// splits: 5 and 9 % root mean square error.
+struct LaunchTiles {
+  double rounds;     // of workgroups over the compute units
+  double longest;    // tiles of the last rows' workgroup
+  double all;        // tiles of the mean workgroup in every round
+  double combine_us; // partial outputs written and read
+};
+
+LaunchTiles tiles_of_launch(const qllm_q4h_attention_launch& launch, uint64_t workgroups,
+                            uint64_t rows_of_one, uint32_t splits) {
+  const auto tiles = [&](uint64_t rows) {
+    return static_cast<double>((launch.first_context_tokens + rows + 62u) / 64u);
+  };
+  LaunchTiles out{};
+  out.rounds = static_cast<double>((workgroups + 255u) / 256u);
+  out.longest = tiles(launch.rows) / splits;
+  out.all = (tiles(std::min<uint64_t>(rows_of_one, launch.rows)) + tiles(launch.rows)) /
+            (2.0 * splits) * out.rounds;
+  out.combine_us = static_cast<double>(launch.rows) * launch.query_heads * splits * 2048.0 / 5.3e6;
+  return out;
+}
+
+double shared_us(const qllm_q4h_attention_launch& launch, uint32_t splits) {
+  const uint32_t group = launch.query_heads / launch.kv_heads;
   const uint32_t parts = shared_parts(launch);
-  const uint64_t workgroups = launch.kv_heads * splits * parts;
-  return parts <= 65535u && (workgroups >= 176u || tiles <= 3u * splits ||
-                             (workgroups >= 128u && tiles <= 16u * splits));
+  const uint64_t waves =   // that have rows
+      std::min<uint64_t>((uint64_t{launch.rows} * group + 15u) / 16u, kPromptBatches);
+  const LaunchTiles t = tiles_of_launch(launch, uint64_t{launch.kv_heads} * parts * splits,
+                                        (16u * kPromptBatches + group - 1u) / group, splits);
+  const double walked = std::max(std::ceil(t.longest), t.all);
+  // (from five waves on two share a SIMD)
+  return 9.2 + t.combine_us +
+         (waves > 4u ? 6.1 * t.rounds + 2.32 * walked
+                     : 0.86 * (waves - 1.0) * t.rounds + 1.55 * walked);
+}
+
+double batched_us(const qllm_q4h_attention_launch& launch, uint32_t batch_rows,
+                  uint32_t splits) {
+  const uint32_t group = launch.query_heads / launch.kv_heads;
+  const uint64_t batches = (uint64_t{launch.rows} + batch_rows - 1u) / batch_rows;
+  const LaunchTiles t =
+      tiles_of_launch(launch, launch.kv_heads * batches * splits, batch_rows, splits);
+  const double walked = std::max(t.longest, t.all) / kSplitWaves;
+  const bool two = uint64_t{std::min(batch_rows, launch.rows)} * group > 16u;   // row tiles
+  return (two ? 7.0 + 11.9 * t.rounds + 6.6 * walked : 12.6 + 4.3 * walked) + t.combine_us;
+}
+
+bool can_share_tiles(const qllm_q4h_attention_launch& launch) {
+  return launch.head_dim == 256u && !launch.split_tokens && shared_parts(launch) <= 65535u;
+}
+
+// 24 heads on 4, batches of five rows against shared tiles: 320 / 960 / 3001 rows from
+// the first token on 31 / 67 / 293 and 30 / 63 / 204 us, 100 rows after 9000 tokens 91
+// and 66.  Left alone: few rows over a long context, where eight waves share a row's
+// tiles (20 rows after 9000: 34, 58 with shared tiles).
+bool shares_tiles(const qllm_q4h_attention_launch& launch, uint32_t batch_rows) {
+  return can_share_tiles(launch) &&
+         shared_us(launch, launch.maximum_splits) <=
+             batched_us(launch, batch_rows, launch.maximum_splits);
 }
 
 // any_order: workgroups may deal a batch's tiles otherwise than a launch of its own
@@ -2834,7 +2885,7 @@ int32_t attend_batches(const qllm_q4h_attention_launch* launch, uint32_t batch_r
   const dim3 grid(launch->kv_heads, splits, batches);
   const hipStream_t stream = as_stream(launch->stream);
   int32_t status = QLLM_OK;
-  if (any_order && shares_tiles(*launch)) {
+  if (any_order && shares_tiles(*launch, batch_rows)) {
     const uint32_t parts = shared_parts(*launch);
     q4h_prompt_attention_kernel<256>
         <<<dim3(launch->kv_heads, splits, parts), kPromptBatches * 64, 0, stream>>>(args);
@@ -2865,9 +2916,35 @@ extern "C" int32_t qllm_attention_paged_q4h_batched_any_order(
   return attend_batches(launch, batch_rows, true);
 }
 
+namespace {
+bool sizes_known(const qllm_q4h_attention_launch* launch, uint32_t batch_rows) {
+  return launch && batch_rows && launch->rows && launch->kv_heads &&
+         launch->query_heads >= launch->kv_heads;
+}
+}  // namespace
+
 extern "C" uint32_t qllm_attention_paged_q4h_shares_tiles(
     const qllm_q4h_attention_launch* launch, uint32_t batch_rows) {
-  return launch && launch->kv_heads && batch_rows && shares_tiles(*launch) ? 1u : 0u;
+  return sizes_known(launch, batch_rows) && launch->maximum_splits &&
+                 shares_tiles(*launch, batch_rows)
+             ? 1u
+             : 0u;
+}
+
+extern "C" uint32_t qllm_attention_paged_q4h_shared_splits(
+    const qllm_q4h_attention_launch* launch, uint32_t batch_rows, uint32_t batch_splits,
+    uint32_t most) {
+  if (!sizes_known(launch, batch_rows) || !batch_splits || !can_share_tiles(*launch)) return 0u;
+  // (by a margin: within it the estimates say nothing)
+  double least = 0.94 * batched_us(*launch, batch_rows, batch_splits);
+  uint32_t best = 0;
+  for (uint32_t splits = 1; splits <= most; ++splits) {
+    const double time = shared_us(*launch, splits);
+    if (time >= least) continue;
+    least = time;
+    best = splits;
+  }
+  return best;
 }
 
 extern "C" int32_t qllm_attention_paged_q4h_prompt(

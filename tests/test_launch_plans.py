@@ -48,3 +48,43 @@ def test_part_rows_of_linears_cover_what_is_advised(rows, columns, element):
             # (asked for 64 rows at a time)
             assert needed <= room <= max(needed * 1.35, 16 * 128)
     assert qh.call("qllm_linear_part_rows", rows, columns, 64, element) == 0
+
+
+def attention(rows, first, query_heads, kv_heads, splits=1, head_dim=256, split_tokens=0):
+    """A prompt's attention that is planned for and never run."""
+    return qh.Q4hAttentionLaunch(
+        rows=rows, first_context_tokens=first + 1, query_heads=query_heads, kv_heads=kv_heads,
+        head_dim=head_dim, split_tokens=split_tokens, maximum_splits=splits, page_tokens=64)
+
+
+@pytest.mark.parametrize("query_heads,kv_heads,rows,first,shared", [
+    (24, 4, 20, 9000, False), (24, 4, 2, 2000, False),       # few rows over a long context
+    (16, 16, 8, 4000, False), (32, 32, 2, 9000, False),      # ... also with workgroups enough
+    (24, 4, 48, 1000, True), (24, 4, 100, 9000, True),
+    (24, 4, 683, 2000, True), (24, 4, 800, 3000, True), (24, 4, 938, 500, True),
+    (24, 2, 800, 500, True), (8, 1, 3000, 1000, True), (24, 4, 3001, 0, True)])
+def test_prompts_share_cache_tiles_where_that_takes_less(query_heads, kv_heads, rows, first,
+                                                         shared):
+    """The form of a prompt's attention at head_dim 256 and its splits, on either side of
+    a full round of workgroups."""
+    batch = 32 // (query_heads // kv_heads)
+    alone = min(8, max(1, -(-256 // (-(-rows // batch) * kv_heads))))
+    splits = qh.call("qllm_attention_paged_q4h_shared_splits",
+                     attention(rows, first, query_heads, kv_heads), batch, alone, 8)
+    assert (splits > 0) == shared and splits <= 8
+    if shared and rows >= 100:   # (of few rows the batches may take those splits as well)
+        launch = attention(rows, first, query_heads, kv_heads, splits)
+        assert qh.call("qllm_attention_paged_q4h_shares_tiles", launch, batch) == 1
+    # the few heads' shorter round is cut so that compute units do not idle
+    if (query_heads, rows) == (8, 3000):
+        assert splits > 1
+
+
+@pytest.mark.parametrize("change", [dict(head_dim=128), dict(split_tokens=64), dict(rows=0),
+                                    dict(kv_heads=0), dict(query_heads=2)])
+def test_launches_that_cannot_share_tiles(change):
+    sizes = dict(rows=1000, first=0, query_heads=24, kv_heads=4)
+    assert qh.call("qllm_attention_paged_q4h_shared_splits", attention(**sizes), 5, 1, 8) > 0
+    launch = attention(**{**sizes, **change})
+    assert qh.call("qllm_attention_paged_q4h_shared_splits", launch, 5, 1, 8) == 0
+    assert qh.call("qllm_attention_paged_q4h_shares_tiles", launch, 5) == 0
