@@ -895,9 +895,16 @@ constexpr uint32_t kMostPieces = 2u * kComputeUnits;   // of cut tiles
 struct ChunkCost {
   float alone, shared;   // ns
 };
-// Workgroups of 80 and 112 rows and cut tiles: not for matrices of fewer rows, which
-// were not timed with them.
-constexpr uint32_t kLowestTimedRows = 3072;
+// Workgroups of 80 and 112 rows and cut tiles are for matrices of these rows: with fewer
+// they were not timed, and of 32000 rows by 2048, where the estimate errs most, 224 rows
+// of a batch took 48 us instead of 41.  Thirteen matrices in between, 2048 to 17408
+// columns (the widths of 2048, 3072, 4096 and 5120), 40 to 3000 rows of a batch, both
+// scale schemes: the launches for which they are chosen take 0.92 of the time on average
+// and at most 1.04 (one in 300 1.09: 1300 rows by [5120, 3072], UE8M0 scales, 59 us for
+// 54).  A launch whose parts the next norm adds takes those heights only where they
+// gain clearly, since the norm pays for more parts.
+constexpr uint32_t kFewestTimedRows = 3072, kMostTimedRows = 17408;
+constexpr double kClearly = 1.025;
 constexpr uint32_t kHeights[] = {1u, 2u, 3u, 4u, 5u, 7u, 8u};
 // [scheme][SwiGLU][height].  Those of 80 and 112 rows are a fit of their own, to 410
 // launches of the 27B widths over 80 to 784 rows (4 to 8 % root mean square error), brought
@@ -965,11 +972,12 @@ TallPlan plan_tall(uint32_t rows, uint32_t padded_columns, uint32_t batch,
     best = plan;
     least = time;
   };
-  const bool timed = rows >= kLowestTimedRows;
+  const bool timed = rows >= kFewestTimedRows && rows <= kMostTimedRows;
   uint32_t lower = 0;   // the height before
   for (uint32_t index = 0; index < std::size(kHeights); ++index) {
     const uint32_t height = kHeights[index];
-    if (!timed && (height == 5u || height == 7u)) continue;
+    const bool between = height == 5u || height == 7u;
+    if (!timed && between) continue;
     // one or two tiles of rows where they hold the batch, else the higher ones, and
     // none of which a lower one would hold the batch
     if (height < 3u ? batch > 16u * height : batch <= 32u) continue;
@@ -988,7 +996,7 @@ TallPlan plan_tall(uint32_t rows, uint32_t padded_columns, uint32_t batch,
       const double time = (chunks + splits - 1u) / splits * chunk +
                           (separate ? 2.0 : 1.0) * bytes / 6200.0 +
                           (separate && splits > 1u ? 4300.0 : 0.0);
-      offer({height, splits, 0u}, time);
+      offer({height, splits, 0u}, between && !separate ? time * kClearly : time);
     }
     // (whole tiles on every CU, so that two workgroups share it all the way)
     const uint32_t tail = tail_tiles_of(workgroups);
@@ -1193,7 +1201,8 @@ extern "C" size_t qllm_fp4_tall_parts_bytes(const qllm_fp4_matrix* matrix, int32
     const uint32_t row = static_cast<uint32_t>(first);
     if (parts_bytes(rows, row, 2u, swiglu) > kPartsBytes) {
       // no launch of so many rows is cut as a whole: the room of the most pieces
-      if (rows >= kLowestTimedRows && rows % 4u == 0u && matrix->padded_columns >= 16u * kChunk)
+      if (rows >= kFewestTimedRows && rows <= kMostTimedRows && rows % 4u == 0u &&
+          matrix->padded_columns >= 16u * kChunk)
         most = std::max(most, kMostPieces * piece_bytes(kHeights[std::size(kHeights) - 1u],
                                                         swiglu));
       break;

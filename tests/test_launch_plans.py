@@ -1,4 +1,6 @@
 """How launches are laid out and what they need, asked of the library without a GPU."""
+import ctypes
+
 import pytest
 
 import qllm_hip as qh
@@ -31,6 +33,23 @@ def test_parts_of_prompts_fit_what_is_set_aside(rows, padded, most, scheme):
             assert room <= max(needed * 1.35, 16 * 16 * 16 * rows)
     assert room <= most and (room > 0) == (most > 0)
     assert qh.call("qllm_fp4_tall_parts_bytes", m, 1, 40) <= 16 * 2 * 48 * rows * 4
+
+
+@pytest.mark.parametrize("scheme", [UE8M0, F16])
+@pytest.mark.parametrize("rows,timed", [(3068, False), (3072, True), (17408, True),
+                                        (17412, False), (32000, False)])
+def test_untimed_matrices_keep_the_old_heights(rows, timed, scheme):
+    """Workgroups of 80 and 112 batch rows and tiles that are cut alone."""
+    m = matrix(rows, 2048, scheme)
+    room = qh.call("qllm_fp4_tall_workspace_bytes")
+    new = set()
+    for batch in range(33, 2400, 7):
+        for swiglu in (0, 1):
+            layout = qh.LaunchLayout()
+            qh.call("qllm_fp4_tall_layout", m, swiglu, batch, room, 0, ctypes.byref(layout))
+            cut = qh.call("qllm_fp4_tall_tail_parts", m, swiglu, batch, room)
+            new.add(layout.batch_rows in (80, 112) or cut > 0)
+    assert new == ({True, False} if timed else {False})
 
 
 @pytest.mark.parametrize("element", [qh.ELEMENT_BF16, qh.ELEMENT_F32])
