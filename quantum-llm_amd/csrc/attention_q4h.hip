@@ -2476,7 +2476,8 @@ int32_t launch_attention_combine(const float* query, uint32_t query_stride,
   const size_t elements = static_cast<size_t>(rows) * query_heads * head_dim;
   if ((maximum_splits == 1u ||
        (maximum_splits <= 8u && static_cast<size_t>(rows) * query_heads >= 256u)) &&
-      !split_tokens && head_dim % 4u == 0u && query_stride % 4u == 0u && !(addresses & 15u) && elements / 4u < 0xffffff00u) {
+      !split_tokens && head_dim % 4u == 0u && query_stride % 4u == 0u &&
+      !(addresses & 15u) && elements / 4u < 0xffffff00u) {
     const auto launch = [&](auto splits) {
       attention_few_splits_kernel<decltype(splits)::value>
           <<<static_cast<unsigned>((elements / 4u + 255u) / 256u), 256, 0, stream>>>(
@@ -2786,7 +2787,8 @@ LaunchTiles tiles_of_launch(const qllm_q4h_attention_launch& launch, uint64_t wo
   out.longest = tiles(launch.rows) / splits;
   out.all = (tiles(std::min<uint64_t>(rows_of_one, launch.rows)) + tiles(launch.rows)) /
             (2.0 * splits) * out.rounds;
-  out.combine_us = static_cast<double>(launch.rows) * launch.query_heads * splits * 2048.0 / 5.3e6;
+  out.combine_us =
+      static_cast<double>(launch.rows) * launch.query_heads * splits * 2048.0 / 5.3e6;
   return out;
 }
 

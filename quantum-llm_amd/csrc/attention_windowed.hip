@@ -1509,9 +1509,9 @@ uint32_t score_splits_for(uint32_t tiles) {
 
 // Up to two tiles a wave, one workgroup of eight waves per key/value head saves the
 // launch that adds the splits: one row of 16 heads on 4, 128 dimensions, 16.2 -> 13.6
-// us over 6 tiles, 16.5 -> 15.4 over 11 and 16.5 -> 16.1 over 16 (with the scores).  (More heads to a
-// key/value head want more registers than eight waves have.)  `tiles` are the most
-// that a row up to the launch's maximum_position sees.  A captured step names the
+// us over 6 tiles, 16.5 -> 15.4 over 11 and 16.5 -> 16.1 over 16 (with the scores).
+// (More heads to a key/value head want more registers than eight waves have.)  `tiles`
+// are the most that a row up to the launch's maximum_position sees.  A captured step names the
 // model's last position there: it comes this way where the window and the kept
 // tokens, or the model's context, are within 16 tiles, however short the request is
 // so far.  (A turn of 100 + 32 tokens with a window of 1024: 8.01 ms in a model of 140

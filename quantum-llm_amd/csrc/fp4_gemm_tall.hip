@@ -1000,7 +1000,8 @@ TallPlan plan_tall(uint32_t rows, uint32_t padded_columns, uint32_t batch,
     }
     // (whole tiles on every CU, so that two workgroups share it all the way)
     const uint32_t tail = tail_tiles_of(workgroups);
-    if (!separate || whole || !timed || height < kLowestTail || tail == workgroups || !tail) continue;
+    if (!separate || whole || !timed || height < kLowestTail || tail == workgroups || !tail)
+      continue;
     for (uint32_t cut = 2u; cut <= last && tail * cut <= kMostPieces; ++cut) {
       const TallPlan plan{height, 1u, cut};
       const size_t bytes = plan_bytes(plan, rows, batch, swiglu);

@@ -636,7 +636,10 @@ __host__ __device__ __forceinline__ uint32_t added_quads(const Latent& a) {
 // a workgroup per head that held all of its values, one row of 16 heads of 512 latent
 // and 128 own values took 8.5 us for 33 parts (200 KiB a workgroup), and 9.2 - 10.4
 // with parts and weights all asked for at once; here a workgroup adds the parts again
-// for every 32 values but fetches a quarter of the weights: 6.6 us.
+// for every 32 values but fetches a quarter of the weights: 6.6 us.  Query, walk and
+// values together, 8 / 16 / 32 rows over 2100 tokens: 33.6 / 39.4 / 42.3 us with a
+// workgroup per head, 26.9 / 31.9 / 35.0 here; one row over 30000 tokens (128 parts) 35.5
+// and 30.4.  At rank 256 and two or three parts 16 and 32 rows lose: 16.3 and 16.9.
 //
 // Everything that depends on nothing is asked for first, in the order in which it is
 // waited for: the row's maxima (a wave per row), this thread's first parts, this

@@ -1,9 +1,9 @@
 // The residual stream of mixed-layer decoders: embedding lookup (by itself or as the
-// first norm's input) and the norm kernel every layer starts with - the partial sums of the projection before
-// it added to the stream, the row's root mean square taken once, up to two
-// normalised copies written (a parallel layer feeds its mixer and its
-// feed-forward from the same row), or the token-shift blends of a mixer that
-// reads the previous token's normalised input as well.
+// first norm's input) and the norm kernel every layer starts with - the partial sums of
+// the projection before it added to the stream, the row's root mean square taken once,
+// up to two normalised copies written (a parallel layer feeds its mixer and its
+// feed-forward from the same row), or the token-shift blends of a mixer that reads the
+// previous token's normalised input as well.
 #include "mixed_common.hpp"
 
 namespace qllm {
