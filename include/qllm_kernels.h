@@ -675,9 +675,10 @@ int32_t qllm_attention_paged_q4h_batched(const qllm_q4h_attention_launch* launch
 /* The same batches, free in the order in which a batch's tiles are added up: at
  * head_dim 256 launches of many rows, or over a short context, share every cache tile
  * between 128 (row, head) pairs (qllm_attention_paged_q4h_shares_tiles).  Such a batch
- * differs from a launch of its own by other F32 sums and by binary16 probabilities that were rounded relative to other
- * running maxima (a few 1e-4 of the values' magnitude), and by how much depends on
- * the launch's other rows; against 64 bits neither is closer.  For prompts. */
+ * differs from a launch of its own by other F32 sums and by binary16 probabilities that
+ * were rounded relative to other running maxima (a few 1e-4 of the values' magnitude),
+ * and by how much depends on the launch's other rows; against 64 bits neither is
+ * closer.  For prompts. */
 int32_t qllm_attention_paged_q4h_batched_any_order(
     const qllm_q4h_attention_launch* launch, uint32_t batch_rows);
 /* 1 where that launch, with the maximum_splits it has, shares cache tiles between
