@@ -72,6 +72,44 @@ __device__ __forceinline__ bf16x2 fp4x2_to_bf16(uint32_t packed, float scale) {
   return __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(packed, scale, Sel);
 }
 
+// A wave-uniform range of memory for buffer loads and copies, whose addresses are a
+// lane's 32-bit offset and a scalar one.  A lane whose own offset lies past the end
+// fetches nothing and reads zero; the scalar one is not checked.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t memory_range(const void* first,
+                                                               size_t bytes) {
+  constexpr size_t kMost = 0xffffffffu;
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(first), 0,
+                                           static_cast<uint32_t>(bytes < kMost ? bytes : kMost),
+                                           0x00020000);
+}
+
+// Copies 16 bytes a lane from a range to the LDS, lane i's to lds + 16 i (`lds` is the
+// wave's).  The compiler knows of the copy and has reads of the same array wait for it,
+// but not reads by other waves: those need wait_for_loads() and a barrier.
+__device__ __forceinline__ void copy16_to_lds(__amdgpu_buffer_rsrc_t source, uint32_t offset,
+                                              uint32_t scalar_offset, void* lds) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      source, (__attribute__((address_space(3))) void*)lds, 16, offset, scalar_offset, 0, 0);
+}
+
+// At most COUNT of this wave's loads and copies are still on their way.
+template <uint32_t COUNT>
+__device__ __forceinline__ void wait_for_loads() {
+  static_assert(COUNT < 64u);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(COUNT) : "memory");
+}
+
+// A workgroup's barrier that waits for no load or copy, which __syncthreads does for
+// all of them where copies to the LDS are on their way.  The wave's own LDS reads must
+// have been used before it (no instruction moves across), its LDS stores have none here.
+__device__ __forceinline__ void barrier_beside_copies() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 __device__ __forceinline__ float wave_sum(float value) {
 #pragma unroll
   for (int offset = 32; offset > 0; offset >>= 1)

@@ -13,9 +13,9 @@
 //    once; a small batch costs one matrix instruction per KiB of weights.
 //  * more rows (prompts): four waves side by side along the weight rows, each
 //    with NT x MT accumulator tiles; the activation tile of 64 columns is
-//    shared through LDS (double-buffered, one barrier per step, 16-byte pieces
-//    swizzled by row so that a fragment read touches every bank), weights are
-//    prefetched one step ahead in registers.  An XCD gets a contiguous range
+//    shared through LDS (copied there ahead of its step, one barrier per step,
+//    16-byte pieces swizzled by row so that a fragment read touches every bank),
+//    weights are prefetched one step ahead in registers.  An XCD gets a contiguous range
 //    of the grid walked in bands of activation tiles, so operands are shared
 //    in its L2.
 //  * F32 mode runs on the same kernels: a 32-bit activation is the sum of three
@@ -32,6 +32,7 @@
 #include <algorithm>
 #include <cmath>
 #include <iterator>
+#include <utility>
 
 namespace qllm {
 namespace {
@@ -169,6 +170,7 @@ __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_
                                            uint32_t batch, f32x4* scratch) {
   const uint32_t wave = threadIdx.x / kWave;
   const uint32_t lane = threadIdx.x % kWave;
+  const uint32_t first_row = blockIdx.y * (16u * MT);
   const uint32_t tiles = s.rows / (16u * TILES);
   const uint32_t parts = s.epilogue == QLLM_LINEAR_PARTIALS ? s.splits : 1u;
   const uint32_t part = unit / tiles;
@@ -186,7 +188,7 @@ __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_
   const Element* input[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    const uint32_t row = min(mt * 16u + lane % 16u, batch - 1u);
+    const uint32_t row = min(first_row + mt * 16u + lane % 16u, batch - 1u);
     input[mt] = static_cast<const Element*>(s.input) + size_t{row} * s.input_stride +
                 8u * (lane / 16u);
   }
@@ -258,7 +260,7 @@ __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_
       for (uint32_t other = 1; other < kSmallWaves; ++other)
         total[t] += scratch[((t * MT + mt) * kSmallWaves + other) * kWave + at];
     }
-    const uint32_t m = mt * 16u + at % 16u;
+    const uint32_t m = first_row + mt * 16u + at % 16u;
     const uint32_t n = tile * 16u + 4u * (at / 16u);
     if (m >= batch) continue;
     if constexpr (TILES == 2) {
@@ -288,17 +290,14 @@ __global__ __launch_bounds__(kSmallWaves* kWave) void linear_small_kernel(Linear
 
 // ---- tall batches --------------------------------------------------------------
 
-template <bool F32, int NT, int MT>
-__global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
-  using In = Input<F32>;
-  using Element = typename In::Element;
-  constexpr int kParts = In::kParts;
-  constexpr uint32_t kRowsM = MT * 16u;
-  constexpr uint32_t kPieces = kRowsM * 8u;           // 16-byte pieces of a tile
-  constexpr uint32_t kLoads = kPieces / 256u;
-  static_assert(kPieces % 256u == 0u);
-  __shared__ i32x4 tile[2][kParts][kPieces];
+// What a workgroup of 64 NT weight rows by 16 MT batch rows works on.
+struct TallPlace {
+  uint32_t segment, part, m_tile, n_tile;
+};
 
+template <int NT, int MT>
+__device__ __forceinline__ TallPlace tall_place(const LinearArgs& args) {
+  constexpr uint32_t kRowsM = MT * 16u;
   const uint32_t m_tiles = (args.batch + kRowsM - 1u) / kRowsM;
   // contiguous ranges of workgroups per XCD (consecutive ids go round the XCDs)
   uint32_t work = blockIdx.x;
@@ -309,24 +308,246 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
   const uint32_t index = segment_of(args, work);
   const qllm_linear_segment& s = args.segment[index];
   const uint32_t n_tiles = (s.rows + 64u * NT - 1u) / (64u * NT);
-  const uint32_t parts = s.epilogue == QLLM_LINEAR_PARTIALS ? s.splits : 1u;
   const uint32_t part = (work - args.first_unit[index]) / (n_tiles * m_tiles);
   const uint32_t unit = (work - args.first_unit[index]) % (n_tiles * m_tiles);
   // bands of kBandTiles activation tiles, walked column by column
   const uint32_t band = unit / (kBandTiles * n_tiles);
   const uint32_t band_rows = min(kBandTiles, m_tiles - band * kBandTiles);
   const uint32_t in_band = unit - band * kBandTiles * n_tiles;
-  const uint32_t m_tile = band * kBandTiles + in_band % band_rows;
-  const uint32_t n_tile = in_band / band_rows;
+  return {index, part, band * kBandTiles + in_band % band_rows, in_band / band_rows};
+}
 
+// Stores a wave's sums: weight tiles first_tile + t, batch rows m_tile 16 MT + 16 mt.
+template <bool F32, int NT, int MT>
+__device__ __forceinline__ void store_tall(const LinearArgs& args, const TallPlace& place,
+                                           uint32_t first_tile, f32x4 (&sum)[NT][MT]) {
+  using Element = typename Input<F32>::Element;
+  constexpr uint32_t kRowsM = MT * 16u;
+  const qllm_linear_segment& s = args.segment[place.segment];
+  const uint32_t m_tile = place.m_tile;
+  const uint32_t part = place.part;
+  const uint32_t lane = threadIdx.x % kWave;
+  const uint32_t weight_tiles = s.rows / 16u;
+  // What the sums are added to is fetched before anything is stored, and - where
+  // the wave's tiles are whole - all of it at once: every load after a store would
+  // wait for all before it.
+  if (s.epilogue == QLLM_LINEAR_ADD) {
+    const bool whole =
+        s.output_stride % 4u == 0u && (first_tile + NT) * 16u <= s.output_columns;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const uint32_t m = min(m_tile * kRowsM + mt * 16u + lane % 16u, args.batch - 1u);
+      const float* out = static_cast<const float*>(s.output) + size_t{m} * s.output_stride +
+                         first_tile * 16u + 4u * (lane / 16u);
+      if (whole) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          sum[t][mt] += *reinterpret_cast<const f32x4*>(out + t * 16);
+        continue;
+      }
+      for (int t = 0; t < NT; ++t)
+        for (uint32_t i = 0; i < 4u; ++i)
+          if (first_tile * 16u + 4u * (lane / 16u) + t * 16u + i < s.output_columns)
+            sum[t][mt][i] += out[t * 16 + i];
+    }
+  }
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const uint32_t m = m_tile * kRowsM + mt * 16u + lane % 16u;
+    if (m >= args.batch) continue;
+    if (s.epilogue == QLLM_LINEAR_GATED) {
+      if constexpr (NT % 2 == 0) {
+#pragma unroll
+        for (int t = 0; t < NT; t += 2) {
+          const uint32_t at = first_tile + t;
+          if (at >= weight_tiles) continue;
+          const uint32_t n = at / 2u * 16u + 4u * (lane / 16u);
+          if (!F32 && n + 4u <= s.output_columns && s.output_stride % 4u == 0u) {
+            const f32x4 gate = sum[t][mt];
+            const f32x4 up = sum[t + 1][mt];
+            uint32_t bits[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              bits[i] = f32_to_bf16_bits(activate(s.activation, gate[i]) * up[i]);
+            *reinterpret_cast<i32x2*>(static_cast<uint16_t*>(s.output) +
+                                      size_t{m} * s.output_stride + n) =
+                i32x2{static_cast<int>(bits[0] | bits[1] << 16),
+                      static_cast<int>(bits[2] | bits[3] << 16)};
+          } else {
+            store_gated<Element>(s, m, n, sum[t][mt], sum[t + 1][mt]);
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        if (first_tile + t < weight_tiles)
+          store_four(s,
+                     static_cast<float*>(s.output) +
+                         size_t{part} * args.batch * s.output_stride,
+                     m, (first_tile + t) * 16u + 4u * (lane / 16u), sum[t][mt], false);
+    }
+  }
+}
+
+// bf16 input.  Bound by the matrix cores and by what their waves wait for: with the
+// activation tile staged through registers a step ahead they were busy 63 % of the time
+// over thousands of rows.  Here the tile goes from memory straight to the LDS two or three
+// steps ahead, without a register, an address or a store of the wave's; weights go to
+// registers a step ahead, and a half's activations are read in between the products of
+// the half before.  6000 rows by [28672, 4096] 1208 -> 1120 us (1160 -> 1250 TFLOP/s), by
+// [4096, 18432] 800 -> 718, by [11264, 2048] 271 -> 247; 300 rows of the three 105 -> 99,
+// 67 -> 66, 29.5 -> 29.2.  The tiles are arrays of their own: of one array's parts the
+// compiler would have every read wait for all copies.
+//
+// LOADS_FIRST: a workgroup that has a CU to itself waits for its loads, so they go out
+// before anything else (70 rows by [8192, 2048], 128 workgroups, 20.4 -> 18.0 us); where
+// workgroups share a CU they go out between the products (70 rows by [2048, 5632], 480
+// workgroups, 9.7 us, and 10.2 the other way).
+template <int NT, int MT, bool LOADS_FIRST>
+__global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
+  constexpr uint32_t kRowsM = MT * 16u;
+  constexpr uint32_t kPieces = kRowsM * 8u;           // 16-byte pieces of a tile
+  constexpr uint32_t kLoads = kPieces / 256u;
+  static_assert(kPieces % 256u == 0u);
+  // (three workgroups of 128 weight rows fit a CU, with a fourth tile two)
+  constexpr int kTiles = NT > 2 ? 4 : 3;
+  constexpr uint32_t kStepLoads = kLoads + 2u * NT;
+  __shared__ i32x4 tile0[kPieces];
+  __shared__ i32x4 tile1[kPieces];
+  __shared__ i32x4 tile2[kPieces];
+  __shared__ i32x4 tile3[kTiles > 3 ? kPieces : 1u];
+
+  const TallPlace place = tall_place<NT, MT>(args);
+  const qllm_linear_segment& s = args.segment[place.segment];
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t lane = threadIdx.x % kWave;
+  const uint32_t chunks = s.columns / 32u;
+  const uint32_t steps = s.columns / 64u;
+  const uint32_t parts = s.epilogue == QLLM_LINEAR_PARTIALS ? s.splits : 1u;
+  const uint32_t first_step = steps * place.part / parts;
+  const uint32_t end_step = steps * (place.part + 1u) / parts;
+  const uint32_t weight_tiles = s.rows / 16u;
+  const uint32_t first_tile = (place.n_tile * 4u + wave) * NT;
+
+  const i32x4* weights[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+    weights[t] = static_cast<const i32x4*>(s.weights) +
+                 size_t{min(first_tile + t, weight_tiles - 1u)} * chunks * kWave;
+
+  // piece p of the tile: row p / 8, swizzled slot p % 8; rows past the batch are not read
+  const size_t first_row = size_t{place.m_tile} * kRowsM;
+  const auto input = memory_range(
+      static_cast<const uint16_t*>(s.input) + first_row * s.input_stride,
+      (args.batch - first_row) * s.input_stride * 2u);
+  uint32_t source[kLoads];
+#pragma unroll
+  for (uint32_t i = 0; i < kLoads; ++i) {
+    const uint32_t piece = i * 256u + threadIdx.x;
+    const uint32_t row = piece / 8u;
+    source[i] = (row * s.input_stride + ((piece % 8u) ^ (row % 8u)) * 8u) * 2u;
+  }
+  const uint32_t fragment[2] = {(lane % 16u) * 8u + ((lane / 16u) ^ (lane % 8u)),
+                                (lane % 16u) * 8u + ((4u + lane / 16u) ^ (lane % 8u))};
+
+  f32x4 sum[NT][MT] = {};
+  i32x4 held[2][2][NT];   // [step parity][half of 32 columns][tile]
+  const auto copy_input = [&](i32x4* to, uint32_t step) {
+#pragma unroll
+    for (uint32_t i = 0; i < kLoads; ++i)
+      copy16_to_lds(input, source[i], step * 128u, to + i * 256u + wave * kWave);
+  };
+  const auto fetch_weights = [&](uint32_t slot, uint32_t step) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        held[slot][half][t] = weights[t][(step * 2u + half) * kWave + lane];
+  };
+  // (a part without steps, of more parts than steps, loads the last one for nothing)
+  const uint32_t last = end_step > first_step ? end_step - 1u : min(first_step, steps - 1u);
+  const auto tile_of = [&](int position) {
+    position %= kTiles;
+    return position == 0 ? tile0 : position == 1 ? tile1 : position == 2 ? tile2 : tile3;
+  };
+#pragma unroll
+  for (int ahead = 0; ahead + 1 < kTiles; ++ahead)
+    copy_input(tile_of(ahead), min(first_step + ahead, last));
+  fetch_weights(0u, min(first_step, last));
+  wait_for_loads<(kTiles - 2u) * kLoads + 2u * NT>();
+
+  const auto step_at = [&]<int P>(std::integral_constant<int, P>, uint32_t step) {
+    const i32x4* current = tile_of(P);
+    // this step's copies are there: what later steps asked for may be on its way
+    wait_for_loads<(kTiles - 2u) * kStepLoads>();
+    barrier_beside_copies();   // everybody's are, and the tile before has been read
+    i32x4 x[MT];
+    const auto read_first_half = [&] {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) x[mt] = current[mt * 128 + fragment[0]];
+    };
+    if constexpr (!LOADS_FIRST) read_first_half();
+    fetch_weights((P + 1) % 2, min(step + 1u, last));
+    copy_input(tile_of(P + kTiles - 1), min(step + kTiles - 1u, last));
+    if constexpr (LOADS_FIRST) {
+      __builtin_amdgcn_sched_barrier(0);
+      read_first_half();
+    }
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          sum[t][mt] = mfma_bf16(held[P % 2][half][t], x[mt], sum[t][mt]);
+        if (half == 0) x[mt] = current[mt * 128 + fragment[1]];
+      }
+    // loads and the second half's reads go between the products
+    __builtin_amdgcn_sched_group_barrier(0x100, MT, 0);
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        __builtin_amdgcn_sched_group_barrier(0x008, NT, 0);
+        if (!LOADS_FIRST) __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+        if (half == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr int kRound = kTiles % 2 ? 2 * kTiles : kTiles;
+  for (uint32_t step = first_step; step < end_step; step += kRound)
+    [&]<int... P>(std::integer_sequence<int, P...>) {
+      (void)((step_at(std::integral_constant<int, P>{}, step + P), step + P + 1u < end_step) &&
+             ...);
+    }(std::make_integer_sequence<int, kRound>{});
+  wait_for_loads<0>();   // no copy outlives its workgroup
+  store_tall<false, NT, MT>(args, place, first_tile, sum);
+}
+
+// 32-bit input, which is cut into its three parts on its way to the LDS.
+template <int NT, int MT>
+__global__ __launch_bounds__(256, 2) void linear_tall_f32_kernel(LinearArgs args) {
+  using In = Input<true>;
+  using Element = float;
+  constexpr int kParts = In::kParts;
+  constexpr uint32_t kRowsM = MT * 16u;
+  constexpr uint32_t kPieces = kRowsM * 8u;           // 16-byte pieces of a tile
+  constexpr uint32_t kLoads = kPieces / 256u;
+  static_assert(kPieces % 256u == 0u);
+  __shared__ i32x4 tile[2][kParts][kPieces];
+
+  const TallPlace place = tall_place<NT, MT>(args);
+  const qllm_linear_segment& s = args.segment[place.segment];
   const uint32_t wave = threadIdx.x / kWave;
   const uint32_t lane = threadIdx.x % kWave;
   const uint32_t chunks = s.columns / 32u;
   const uint32_t steps = s.columns / 64u;
-  const uint32_t first_step = steps * part / parts;
-  const uint32_t end_step = steps * (part + 1u) / parts;
+  const uint32_t parts = s.epilogue == QLLM_LINEAR_PARTIALS ? s.splits : 1u;
+  const uint32_t first_step = steps * place.part / parts;
+  const uint32_t end_step = steps * (place.part + 1u) / parts;
   const uint32_t weight_tiles = s.rows / 16u;
-  const uint32_t first_tile = (n_tile * 4u + wave) * NT;
+  const uint32_t first_tile = (place.n_tile * 4u + wave) * NT;
 
   const i32x4* weights[NT];
 #pragma unroll
@@ -341,7 +562,7 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
     const uint32_t piece = i * 256u + threadIdx.x;
     const uint32_t row = piece / 8u;
     const uint32_t column = (piece % 8u) ^ (row % 8u);
-    const uint32_t batch_row = min(m_tile * kRowsM + row, args.batch - 1u);
+    const uint32_t batch_row = min(place.m_tile * kRowsM + row, args.batch - 1u);
     source[i] = static_cast<const Element*>(s.input) +
                 size_t{batch_row} * s.input_stride + column * 8u;
   }
@@ -409,90 +630,30 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
     step_at(step + 1u, odd);
   }
   if (step < end_step) step_at(step, even);
-  if constexpr (F32)
-    if (__any(any_nan(sum))) {   // this wave's alone, its inputs past the LDS
+  if (__any(any_nan(sum))) {   // this wave's alone, its inputs past the LDS
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) sum[t][mt] = f32x4{};
-      for (uint32_t chunk = 2u * first_step; chunk < 2u * end_step; ++chunk)
+      for (int mt = 0; mt < MT; ++mt) sum[t][mt] = f32x4{};
+    for (uint32_t chunk = 2u * first_step; chunk < 2u * end_step; ++chunk)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          const uint32_t row = min(m_tile * kRowsM + mt * 16u + lane % 16u, args.batch - 1u);
-          i32x4 x[kParts];
-          In::split(In::load(static_cast<const Element*>(s.input) +
-                             size_t{row} * s.input_stride + chunk * 32u + 8u * (lane / 16u)),
-                    x);
+      for (int mt = 0; mt < MT; ++mt) {
+        const uint32_t row = min(place.m_tile * kRowsM + mt * 16u + lane % 16u, args.batch - 1u);
+        i32x4 x[kParts];
+        In::split(In::load(static_cast<const Element*>(s.input) +
+                           size_t{row} * s.input_stride + chunk * 32u + 8u * (lane / 16u)),
+                  x);
 #pragma unroll
-          for (int t = 0; t < NT; ++t) {
-            const i32x4 w = weights[t][chunk * kWave];
+        for (int t = 0; t < NT; ++t) {
+          const i32x4 w = weights[t][chunk * kWave];
 #pragma unroll
-            for (int p = 0; p < kParts; ++p)
-              sum[t][mt] = mfma_bf16(p ? finite_weights(w) : w, x[p], sum[t][mt]);
-          }
+          for (int p = 0; p < kParts; ++p)
+            sum[t][mt] = mfma_bf16(p ? finite_weights(w) : w, x[p], sum[t][mt]);
         }
-    }
+      }
+  }
 
-  // What the sums are added to is fetched before anything is stored, and - where
-  // the wave's tiles are whole - all of it at once: every load after a store would
-  // wait for all before it.
-  if (s.epilogue == QLLM_LINEAR_ADD) {
-    const bool whole =
-        s.output_stride % 4u == 0u && (first_tile + NT) * 16u <= s.output_columns;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const uint32_t m = min(m_tile * kRowsM + mt * 16u + lane % 16u, args.batch - 1u);
-      const float* out = static_cast<const float*>(s.output) + size_t{m} * s.output_stride +
-                         first_tile * 16u + 4u * (lane / 16u);
-      if (whole) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-          sum[t][mt] += *reinterpret_cast<const f32x4*>(out + t * 16);
-        continue;
-      }
-      for (int t = 0; t < NT; ++t)
-        for (uint32_t i = 0; i < 4u; ++i)
-          if (first_tile * 16u + 4u * (lane / 16u) + t * 16u + i < s.output_columns)
-            sum[t][mt][i] += out[t * 16 + i];
-    }
-  }
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const uint32_t m = m_tile * kRowsM + mt * 16u + lane % 16u;
-    if (m >= args.batch) continue;
-    if (s.epilogue == QLLM_LINEAR_GATED) {
-      if constexpr (NT % 2 == 0) {
-#pragma unroll
-        for (int t = 0; t < NT; t += 2) {
-          const uint32_t at = first_tile + t;
-          if (at >= weight_tiles) continue;
-          const uint32_t n = at / 2u * 16u + 4u * (lane / 16u);
-          if (!F32 && n + 4u <= s.output_columns && s.output_stride % 4u == 0u) {
-            const f32x4 gate = sum[t][mt];
-            const f32x4 up = sum[t + 1][mt];
-            uint32_t bits[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              bits[i] = f32_to_bf16_bits(activate(s.activation, gate[i]) * up[i]);
-            *reinterpret_cast<i32x2*>(static_cast<uint16_t*>(s.output) +
-                                      size_t{m} * s.output_stride + n) =
-                i32x2{static_cast<int>(bits[0] | bits[1] << 16),
-                      static_cast<int>(bits[2] | bits[3] << 16)};
-          } else {
-            store_gated<Element>(s, m, n, sum[t][mt], sum[t + 1][mt]);
-          }
-        }
-      }
-    } else {
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        if (first_tile + t < weight_tiles)
-          store_four(s,
-                     static_cast<float*>(s.output) +
-                         size_t{part} * args.batch * s.output_stride,
-                     m, (first_tile + t) * 16u + 4u * (lane / 16u), sum[t][mt], false);
-    }
-  }
+  store_tall<true, NT, MT>(args, place, first_tile, sum);
 }
 
 __global__ void linear_pack_kernel(const uint16_t* source, uint32_t rows, uint32_t columns,
@@ -589,6 +750,10 @@ uint32_t tall_form(const LinearArgs& args, bool f32) {
   return best;
 }
 
+// Workgroups up to which most have a CU to themselves (192 to 320: 1 to 5 % faster with
+// their loads first, 480: 3 % slower).
+constexpr uint32_t kAlone = 320;
+
 template <bool F32, int NT, int MT>
 int32_t launch_tall(LinearArgs& args, hipStream_t stream) {
   args.first_unit[0] = 0;
@@ -598,15 +763,24 @@ int32_t launch_tall(LinearArgs& args, hipStream_t stream) {
         static_cast<uint32_t>(tall_units({NT, MT, 0.f, 0.f}, args.segment[i].rows,
                                          args.batch)) *
             parts_of(args.segment[i]);
-  linear_tall_kernel<F32, NT, MT>
-      <<<args.first_unit[args.count], 256, 0, stream>>>(args);
+  const uint32_t grid = args.first_unit[args.count];
+  if constexpr (F32) {
+    linear_tall_f32_kernel<NT, MT><<<grid, 256, 0, stream>>>(args);
+  } else if constexpr (NT == 2 && MT == 4) {
+    if (grid <= kAlone)
+      linear_tall_kernel<NT, MT, true><<<grid, 256, 0, stream>>>(args);
+    else
+      linear_tall_kernel<NT, MT, false><<<grid, 256, 0, stream>>>(args);
+  } else {
+    linear_tall_kernel<NT, MT, false><<<grid, 256, 0, stream>>>(args);
+  }
   return launched("tall linear");
 }
 
 template <bool F32, int MT>
 void launch_small(const LinearArgs& args, hipStream_t stream) {
-  linear_small_kernel<F32, MT>
-      <<<args.first_unit[args.count], kSmallWaves * kWave, 0, stream>>>(args);
+  const dim3 grid(args.first_unit[args.count], (args.batch + 16u * MT - 1u) / (16u * MT));
+  linear_small_kernel<F32, MT><<<grid, kSmallWaves * kWave, 0, stream>>>(args);
 }
 
 }  // namespace
@@ -679,6 +853,14 @@ int32_t linear_arguments(const qllm_linear_segment* segments, uint32_t count,
 // batch rows of a workgroup of the form for up to 64
 uint32_t small_rows(uint32_t batch) { return batch <= 16u ? 16u : batch <= 32u ? 32u : 64u; }
 
+// Whether the form for up to 64 rows takes the batch: a longer one of bf16 too, 64 rows at
+// a time, where a lane's 32-bit offset does not reach over 128 rows.
+bool takes_small(const LinearArgs& args, bool f32) {
+  bool far = false;
+  for (uint32_t i = 0; i < args.count; ++i) far |= args.segment[i].input_stride >= 1u << 24;
+  return args.batch <= 64u || (far && !f32);
+}
+
 }  // namespace
 
 extern "C" int32_t qllm_linear_layout(const qllm_linear_segment* segments, uint32_t count,
@@ -689,7 +871,7 @@ extern "C" int32_t qllm_linear_layout(const qllm_linear_segment* segments, uint3
   if (const int32_t status = linear_arguments(segments, count, batch, element, args))
     return status;
   const bool f32 = element == QLLM_ELEMENT_F32;
-  if (batch <= 64u) {
+  if (takes_small(args, f32)) {
     *layout = {small_rows(batch), 16u, parts_of(args.segment[0])};
     return QLLM_OK;
   }
@@ -706,7 +888,7 @@ extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32
     return status;
   const auto hip_stream = as_stream(stream);
   const bool f32 = element == QLLM_ELEMENT_F32;
-  if (batch <= 64u) {
+  if (takes_small(args, f32)) {
     for (uint32_t i = 0; i < count; ++i) {
       const qllm_linear_segment& s = segments[i];
       const uint32_t parts = s.epilogue == QLLM_LINEAR_PARTIALS ? s.splits : 1u;

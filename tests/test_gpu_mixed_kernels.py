@@ -284,6 +284,51 @@ def test_linear_tall_forms_of_every_epilogue(device, element, rows, columns, bat
     assert torch.all(out[:, half:] == 0)
 
 
+@pytest.mark.parametrize("rows,batch,form", [
+    (70, 65, (64, 128)),          # a workgroup to a CU: loads first
+    (3088, 777, (64, 128)),       # several to a CU
+    (2090, 2900, (128, 128)), (8170, 1901, (128, 256))])
+@pytest.mark.parametrize("columns,stride", [(64, 64), (128, 192), (256, 264), (448, 448),
+                                            (576, 1024), (640, 640)])
+def test_linear_tall_steps_ahead(device, rows, batch, form, columns, stride):
+    """Launches of one to ten steps of K, fewer and more than the steps that a workgroup
+    asks for ahead, over input rows with a gap between them."""
+    rng = np.random.default_rng(rows + columns)
+    w = mm.bf16(rng.standard_normal((rows, columns)) / np.sqrt(columns))
+    x = mm.bf16(rng.standard_normal((batch, columns)))
+    weights = packed(device, [(w, 0, 1, 0)], rows, columns)
+    d_x = torch.full((batch, stride), float("nan"), dtype=torch.bfloat16, device=device)
+    d_x[:, :columns] = on(device, x)
+    out = torch.zeros((batch, padded(rows, 4)), device=device)
+    segment = qh.LinearSegment(qh.ptr(weights), qh.ptr(d_x), qh.ptr(out), padded(rows, 16),
+                               columns, stride, padded(rows, 4), rows, qh.LINEAR_STORE, 0, 0)
+    found = qh.LaunchLayout()
+    qh.call("qllm_linear_layout", ctypes.byref(segment), 1, batch, BF16, ctypes.byref(found))
+    assert (found.batch_rows, found.weight_rows) == form
+    qh.call("qllm_linear_batch", ctypes.byref(segment), 1, batch, BF16, None)
+    got = out[:, :rows].double()
+    x, w = on(device, x).double(), on(device, w).double()
+    # exact products, every one of `columns` additions of a sum rounds by at most 2^-24
+    bound = columns * 2.0 ** -24 * (x.abs() @ w.abs().T)
+    assert ((got - x @ w.T).abs() <= bound).all()
+
+
+def test_linear_of_rows_far_apart(device):
+    """Rows 2^24 values apart, past a lane's 32-bit offset over 128 of them."""
+    rng = np.random.default_rng(5)
+    rows, batch, columns, stride = 40, 70, 128, 1 << 24
+    w = mm.bf16(rng.standard_normal((rows, columns)) / 8)
+    x = mm.bf16(rng.standard_normal((batch, columns)))
+    weights = packed(device, [(w, 0, 1, 0)], rows, columns)
+    d_x = torch.empty((batch, stride), dtype=torch.bfloat16, device=device)
+    d_x[:, :columns] = on(device, x)
+    out = torch.zeros((batch, rows), device=device)
+    segment = qh.LinearSegment(qh.ptr(weights), qh.ptr(d_x), qh.ptr(out), 48, columns, stride,
+                               rows, rows, qh.LINEAR_STORE, 0, 0)
+    qh.call("qllm_linear_batch", ctypes.byref(segment), 1, batch, BF16, None)
+    close(out, x.astype(np.float64) @ w.T.astype(np.float64), F32)
+
+
 # ---- stream ---------------------------------------------------------------------
 
 
