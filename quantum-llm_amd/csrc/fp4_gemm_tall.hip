@@ -6,15 +6,14 @@
 // bf16 with their block scale, bf16 activations, 16x16x16 tensor-core tiles,
 // F32 accumulation).  Here the contraction is compute-bound, so it is laid out
 // for the matrix cores: a workgroup of four waves owns 128 activation rows x
-// 256 weight rows; every wave keeps the 128 x 64 accumulator of its two
-// 32-row weight tiles in registers (8 x 4 tiles of v_mfma_f32_16x16x32), takes
+// 256 weight rows (or fewer); every wave keeps the 128 x 64 accumulator of its
+// two 32-row weight tiles in registers (8 x 4 tiles of v_mfma_f32_16x16x32), takes
 // its weights straight from the provider's streaming layout - the 16-byte
 // piece a lane loads per (tile, chunk) is its B operand for the chunk's four
 // instructions, no LDS and no shuffle - and shares the activation tile of the
-// chunk through LDS (double-buffered, one barrier per 64 columns of K).  Batches
-// whose tiles are too few for the GPU - short prompts, and long ones against
-// matrices of few rows - are cut along K and use lower workgroups
-// (fp4_gemm_short_kernel, plan_tall).
+// chunk through LDS (one barrier per 64 columns of K).  Batches whose tiles are
+// too few for the GPU - short prompts, and long ones against matrices of few
+// rows - are cut along K and use lower workgroups (plan_tall).
 //
 // Scale schemes:
 //  * UE8M0 per 32: the power-of-two scale is folded into the nibble -> bf16
@@ -38,6 +37,7 @@
 #include <algorithm>
 #include <iterator>
 #include <type_traits>
+#include <utility>
 
 namespace qllm {
 namespace {
@@ -388,199 +388,56 @@ __device__ __forceinline__ void store_tiles(const TallArgs& args, uint32_t part,
   }
 }
 
-// Workgroup (part, m_tile, n_tile): activation rows [128 m_tile, +128), weight
-// rows [256 n_tile, +256), chunks of the part.
+constexpr uint32_t kPastTheEnd = 0x80000000u;   // an offset that fetches nothing
+
+// A workgroup of 16 MT activation rows by 128 T weight rows and the chunks of its part or
+// piece.  SWIGLU: 128 rows of the gate and of the up matrix each, a wave's two tiles are
+// the same 32 rows of both, and the epilogue writes silu(gate) * up in bf16 with the
+// rounding points of the separate SiLU-product launch - no F32 round trip of the two.
 //
-// SWIGLU: a wave's two tiles are the same 32 rows of the gate and of the up
-// matrix (a workgroup covers 128 rows of each), and the epilogue writes
-// silu(gate) * up in bf16 with the rounding points of the separate
-// SiLU-product launch - no F32 round trip of the two projections.
-template <int SCHEME, bool SWIGLU = false>
-__global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_tall_kernel(
-    const TallArgs args) {
-  using Op = Operand<SCHEME>;
-  using Vector = typename Op::Vector;
-  constexpr bool F16 = SCHEME == kSchemeF16;
-  __shared__ __attribute__((aligned(16))) uint8_t tile[2][kRowsM * kLdsRow];
-
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t n = lane & 15u;
-  const uint32_t g = lane >> 4;
-  const uint32_t K = args.padded_columns;
-  const uint32_t chunks = K / kChunk;
-
-  const Work work = work_of<true>(args, chunks);
-  const uint32_t first_chunk = work.first_chunk;
-  const uint32_t end_chunk = work.end_chunk;
-  const uint32_t first_m = work.m_tile * kRowsM;
-
-  // weight streams of this wave's tiles (tiles past the matrix repeat the last
-  // one and are not stored)
-  const uint32_t tile_count = (args.rows + kTileRows - 1u) / kTileRows;
-  const uint8_t* weight_stream[kTilesPerWave];
-  const uint8_t* scale_stream[kTilesPerWave];
-  uint32_t tile_index[kTilesPerWave];
-#pragma unroll
-  for (uint32_t t = 0; t < kTilesPerWave; ++t) {
-    tile_index[t] = weight_tile<kTilesPerWave, SWIGLU>(work.n_tile, wave, t);
-    const size_t stream = min(tile_index[t], tile_count - 1u);
-    weight_stream[t] = (SWIGLU && t ? args.up_weights : args.weights) +
-                       stream * chunks * (kTileRows * 32u) + (g * 16u + n) * 16u;
-    scale_stream[t] =
-        (SWIGLU && t ? args.up_scales : args.scales) +
-        stream * chunks * (kTileRows * (F16 ? 8u : 2u)) +
-        (F16 ? ((g >> 1) * 16u + n) * 8u : n * 4u);
-  }
-
-  // activation tile: thread -> (row, half of the 64 columns), 64 bytes.  Rows
-  // past the batch stage row 0 again: their results are never stored, and a
-  // load under a branch would make every wait for the weights conservative.
-  const uint32_t stage_row = threadIdx.x >> 1;
-  const uint32_t stage_half = threadIdx.x & 1u;
-  const bool stage_live = first_m + stage_row < args.batch;
-  const uint8_t* stage_source =
-      reinterpret_cast<const uint8_t*>(args.activations) +
-      (static_cast<size_t>(stage_live ? first_m + stage_row : 0u) * K +
-       stage_half * 32u) * 2u;
-  const uint32_t stage_target = stage_row * kLdsRow;
-  // fragment of m-tile mt, span s: row 16 mt + n, columns 32 s + 8 g .. + 8
-  const uint32_t fragment_offset[2] = {n * kLdsRow + swizzled(g, n),
-                                       n * kLdsRow + swizzled(g + 4u, n)};
-
-  f32x4 acc[kTilesM][kTilesPerWave][2];
-#pragma unroll
-  for (uint32_t mt = 0; mt < kTilesM; ++mt)
-#pragma unroll
-    for (uint32_t t = 0; t < kTilesPerWave; ++t)
-#pragma unroll
-      for (uint32_t j = 0; j < 2u; ++j) acc[mt][t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  uint4 staged[4];
-  const auto fetch_activations = [&](uint32_t chunk) {
-#pragma unroll
-    for (uint32_t piece = 0; piece < 4u; ++piece)
-      staged[piece] = *reinterpret_cast<const uint4*>(
-          stage_source + static_cast<size_t>(chunk) * 128u + piece * 16u);
-  };
-  const auto store_activations = [&](uint32_t buffer) {
-#pragma unroll
-    for (uint32_t piece = 0; piece < 4u; ++piece) {
-      uint4 v = staged[piece];
-      v.x = Op::stage(v.x); v.y = Op::stage(v.y);
-      v.z = Op::stage(v.z); v.w = Op::stage(v.w);
-      *reinterpret_cast<uint4*>(
-          &tile[buffer][stage_target + swizzled(stage_half * 4u + piece, stage_row)]) = v;
-    }
-  };
-  // (slot indices are compile-time constants throughout: an array indexed by a
-  // run-time slot would live in scratch memory, and every reload from there
-  // would wait for the prefetch that was just issued)
-  uint4 codes[2][kTilesPerWave];
-  uint2 scales[2][kTilesPerWave];
-  const auto fetch_weights = [&]<int slot>(std::integral_constant<int, slot>,
-                                           uint32_t chunk) {
-#pragma unroll
-    for (uint32_t t = 0; t < kTilesPerWave; ++t) {
-      codes[slot][t] = *reinterpret_cast<const uint4*>(
-          weight_stream[t] + static_cast<size_t>(chunk) * (kTileRows * 32u));
-      if constexpr (F16) {
-        scales[slot][t] = *reinterpret_cast<const uint2*>(
-            scale_stream[t] + static_cast<size_t>(chunk) * (kTileRows * 8u));
-      } else {
-        scales[slot][t].x = *reinterpret_cast<const uint32_t*>(
-            scale_stream[t] + static_cast<size_t>(chunk) * (kTileRows * 2u));
-        scales[slot][t].y = 0u;
-      }
-    }
-  };
-
-  fetch_activations(first_chunk);
-  fetch_weights(std::integral_constant<int, 0>{}, first_chunk);
-  store_activations(0u);
-
-  const auto step = [&]<int slot>(std::integral_constant<int, slot>,
-                                  uint32_t chunk) {
-    __syncthreads();   // tile[slot] is complete; tile[slot ^ 1] is free
-    const uint32_t next = chunk + 1u < end_chunk ? chunk + 1u : chunk;
-    fetch_activations(next);
-    fetch_weights(std::integral_constant<int, slot ^ 1>{}, next);
-    // the loads stay here, a whole step ahead of their use (left alone, the
-    // scheduler sinks them to the end of the step to shorten live ranges)
-    __builtin_amdgcn_sched_barrier(0);
-
-    const uint8_t* current = tile[slot];
-#pragma unroll
-    for (uint32_t s = 0; s < 2u; ++s) {
-      Vector a[kTilesM];
-#pragma unroll
-      for (uint32_t mt = 0; mt < kTilesM; ++mt)
-        a[mt] = __builtin_bit_cast(
-            Vector, *reinterpret_cast<const uint4*>(
-                        current + mt * 16u * kLdsRow + fragment_offset[s]));
-#pragma unroll
-      for (uint32_t t = 0; t < kTilesPerWave; ++t) {
-        const uint4 q = codes[slot][t];
-        const uint32_t packed[4] = {q.x, q.y, q.z, q.w};   // index 2j + s
-#pragma unroll
-        for (uint32_t j = 0; j < 2u; ++j) {
-          // scale of (j, s): binary16 halves of the two words, or UE8M0 bytes
-          const uint32_t word = j ? scales[slot][t].y : scales[slot][t].x;
-          const uint32_t f16_bits = s ? word >> 16 : word & 0xffffu;
-          const float fold =
-              F16 ? 1.0f
-                  : ue8m0_to_f32((scales[slot][t].x >> (8u * (2u * j + s))) & 0xffu);
-          Vector w[Op::kParts];
-          Op::weights(packed[2u * j + s], fold, f16_bits, w);
-#pragma unroll
-          for (int part = 0; part < Op::kParts; ++part)
-#pragma unroll
-            for (uint32_t mt = 0; mt < kTilesM; ++mt)
-              acc[mt][t][j] = Op::mfma(a[mt], w[part], acc[mt][t][j]);
-        }
-      }
-    }
-    if (chunk + 1u < end_chunk) store_activations(slot ^ 1u);
-  };
-  for (uint32_t chunk = first_chunk; chunk < end_chunk; chunk += 2u) {
-    step(std::integral_constant<int, 0>{}, chunk);
-    if (chunk + 1u < end_chunk) step(std::integral_constant<int, 1>{}, chunk + 1u);
-  }
-
-  if (work.is_piece)
-    store_piece<kTilesM, kTilesPerWave>(args, work.piece, acc);
-  else
-    store_tiles<kTilesM, kTilesPerWave, SWIGLU>(args, work.part, first_m, tile_index,
-                                                tile_count, acc);
-}
-
-// Short batches: 16 MT rows a workgroup, 128 T weight rows (SWIGLU: 128 of each of
-// the two matrices).  Up to 64 rows the weights' way from memory is what there is to
-// hide, not the matrix cores' time: a wave keeps its weights of the next four chunks
-// on their way in registers (with the one of fp4_gemm_tall_kernel a step waits out
-// most of a memory round trip), the activations of the next two steps likewise, and a
-// step covers so many chunks that its barrier costs about the same whatever the
-// height.  80 and 112 rows, where registers hold two chunks of weights, stand between
-// those and fp4_gemm_tall_kernel's 128 so that fewer rows of a batch's last workgroups
-// are padding; a weight's conversion, three vector instructions a pair of binary16
-// scaled ones, serves that many more rows (gate and up of [17408, 5120], two
-// workgroups a CU: matrix cores busy 60 % of the time with 64 rows, 65 with 80, 75
-// with 112, 74 with 128).
+// Up to 64 rows the weights' way from memory is what there is to hide, not the matrix
+// cores' time: a wave keeps its weights of the next four chunks on their way in registers
+// (two where accumulators leave no room), activations are two or three steps ahead, and
+// a step covers so many chunks that its barrier costs about the same whatever the height.
+// With 128 rows it is the matrix cores, as far as the card's power lets them: gate and up
+// of [17408, 5120] with binary16 scales over 8192 rows kept them busy 73 % of the time at
+// 2.10 GHz when a unit's weights were converted before its products and a half chunk's
+// activations waited for; with both done in between the products 80 % at 2.00 GHz, 3660 ->
+// 3560 us.  UE8M0 scales, whose activations need no conversion and are copied to the LDS
+// without passing through registers: 63 -> 73 %, 2190 -> 1980 us; 300 rows by [10240, 5120]
+// 47.5 -> 42.1 (binary16: 76 -> 70), 48 rows 17.5 -> 16.7 (21.7 -> 21.2).  80 and 112 rows
+// stand between so that fewer rows of a batch's last workgroups are padding; a weight's
+// conversion, three vector instructions a pair of binary16 scaled ones, serves that many
+// more rows.
 template <int SCHEME, int MT, int T, bool SWIGLU>
-__global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
-    const TallArgs args) {
+__global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_rows_kernel(const TallArgs args) {
   using Op = Operand<SCHEME>;
   using Vector = typename Op::Vector;
   constexpr bool F16 = SCHEME == kSchemeF16;
   static_assert(!SWIGLU || T == 2);
-  constexpr uint32_t kAhead = MT > 4 ? 2 : 4;       // chunks of weights in flight
-  constexpr uint32_t kSpan = MT > 4 ? 1 : MT == 3 ? 2 : 4 / MT;  // chunks per step
+  constexpr int kAhead = MT > 4 ? 2 : 4;            // chunks of weights in flight
+  constexpr int kSpan = MT > 4 ? 1 : MT == 3 ? 2 : 4 / MT;   // chunks per step
+  // Activations that stay bf16 are copied straight to the LDS, into one of four tiles;
+  // those converted on the way pass through registers and two tiles.  (Tiles are arrays of
+  // their own: of one array's parts the compiler would have every read wait for all copies.)
+  constexpr bool kCopied = !F16;
+  constexpr int kTiles = kCopied ? 4 : 2;
+  constexpr int kStages = MT > 7 ? 1 : 2;           // steps of activations in registers
   constexpr uint32_t kRow = kSpan * kLdsRow;
+  constexpr uint32_t kTileBytes = 16u * MT * kRow;
   // 16-byte pieces of a step's activations, of the workgroup and of a thread (an odd
-  // height's last ones are the same piece for half of the threads)
-  constexpr uint32_t kAllPieces = 16u * MT * kSpan * 8u;
+  // height's last ones are the same pieces for half of the waves)
+  constexpr uint32_t kAllPieces = kTileBytes / 16u;
   constexpr uint32_t kPieces = (kAllPieces + kWaves * 64u - 1u) / (kWaves * 64u);
-  __shared__ __attribute__((aligned(16))) uint8_t tile[2][16 * MT * kRow];
+  constexpr uint32_t kStepLoads = kPieces + 2u * T * kSpan;
+  __shared__ __attribute__((aligned(16))) uint8_t tile0[kTileBytes];
+  __shared__ __attribute__((aligned(16))) uint8_t tile1[kTileBytes];
+  __shared__ __attribute__((aligned(16))) uint8_t tile2[kTiles > 2 ? kTileBytes : 16u];
+  __shared__ __attribute__((aligned(16))) uint8_t tile3[kTiles > 2 ? kTileBytes : 16u];
+  const auto tile_of = [&](int position) {
+    position %= kTiles;
+    return position == 0 ? tile0 : position == 1 ? tile1 : position == 2 ? tile2 : tile3;
+  };
 
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -597,35 +454,39 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
   const uint32_t first_chunk = work.first_chunk;
   const uint32_t end_chunk = work.end_chunk;
 
+  // weight streams of this wave's tiles (tiles past the matrix repeat the last
+  // one and are not stored)
+  constexpr uint32_t kCodes = kTileRows * 32u, kScales = kTileRows * (F16 ? 8u : 2u);
   const uint32_t tile_count = (args.rows + kTileRows - 1u) / kTileRows;
-  const uint8_t* weight_stream[T];
-  const uint8_t* scale_stream[T];
+  __amdgpu_buffer_rsrc_t code_stream[T], scale_stream[T];
   uint32_t tile_index[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) {
     tile_index[t] = weight_tile<T, SWIGLU>(work.n_tile, wave, t);
-    const size_t stream = min(tile_index[t], tile_count - 1u);
-    weight_stream[t] = (SWIGLU && t ? args.up_weights : args.weights) +
-                       stream * chunks * (kTileRows * 32u) + lane * 16u;
-    scale_stream[t] = (SWIGLU && t ? args.up_scales : args.scales) +
-                      stream * chunks * (kTileRows * (F16 ? 8u : 2u)) +
-                      (F16 ? ((g >> 1) * 16u + n) * 8u : n * 4u);
+    const size_t stream = static_cast<size_t>(min(tile_index[t], tile_count - 1u)) * chunks;
+    code_stream[t] =
+        memory_range((SWIGLU && t ? args.up_weights : args.weights) + stream * kCodes,
+                     size_t{chunks} * kCodes);
+    scale_stream[t] =
+        memory_range((SWIGLU && t ? args.up_scales : args.scales) + stream * kScales,
+                     size_t{chunks} * kScales);
   }
+  const uint32_t code_offset = lane * 16u;
+  const uint32_t scale_offset = F16 ? ((g >> 1) * 16u + n) * 8u : n * 4u;
 
-  // piece p of a step's activations: row p / (8 kSpan), 16 bytes at column
-  // piece p % (8 kSpan).  Rows past the batch read its last row and are not
-  // stored; columns past K read its last ones and meet no weights.
-  const uint8_t* source_row[kPieces];
-  uint32_t source_column[kPieces], target[kPieces];
+  // Piece p of a step's tile: row p / (8 kSpan) and, of its chunk p / 8 % kSpan, the eight
+  // columns that the swizzle puts there.  Rows past the batch read as zero and are not
+  // stored; columns past K read what follows, or zero, and meet no weights.
+  const auto activations = memory_range(args.activations + static_cast<size_t>(first_m) * K,
+                                        static_cast<size_t>(args.batch - first_m) * K * 2u);
+  uint32_t source[kPieces], target[kPieces];
 #pragma unroll
   for (uint32_t p = 0; p < kPieces; ++p) {
-    const uint32_t piece = min(p * kWaves * 64u + threadIdx.x, kAllPieces - 1u);
+    const uint32_t wave_piece = min(p * kWaves + wave, kAllPieces / 64u - 1u) * 64u;
+    const uint32_t piece = wave_piece + lane;
     const uint32_t row = piece / (8u * kSpan);
-    source_column[p] = piece % (8u * kSpan) * 16u;
-    target[p] = row * kRow + source_column[p] / kLdsRow * kLdsRow +
-                swizzled(source_column[p] % kLdsRow / 16u, row);
-    source_row[p] = reinterpret_cast<const uint8_t*>(args.activations) +
-                    static_cast<size_t>(min(first_m + row, args.batch - 1u)) * K * 2u;
+    source[p] = row * K * 2u + (piece / 8u % kSpan * 8u + ((piece ^ row) % 8u)) * 16u;
+    target[p] = (kCopied ? wave_piece : piece) * 16u;
   }
   const uint32_t fragment_offset[2] = {n * kRow + swizzled(g, n),
                                        n * kRow + swizzled(g + 4u, n)};
@@ -638,145 +499,182 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_short_kernel(
 #pragma unroll
       for (uint32_t j = 0; j < 2u; ++j) acc[mt][t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  uint4 staged[2][kPieces];
-  const auto fetch_activations = [&]<int slot>(std::integral_constant<int, slot>,
-                                               uint32_t chunk) {
+  const auto source_at = [&](uint32_t p, uint32_t chunk) {
+    return source[p] + min(chunk, end_chunk - 1u) * (kChunk * 2u);
+  };
+  const auto copy_activations = [&](uint8_t* tile, uint32_t chunk) {
 #pragma unroll
     for (uint32_t p = 0; p < kPieces; ++p)
-      staged[slot][p] = *reinterpret_cast<const uint4*>(
-          source_row[p] + min(chunk * (kChunk * 2u) + source_column[p], K * 2u - 16u));
+      copy16_to_lds(activations, source_at(p, chunk), 0u, tile + target[p]);
   };
-  const auto store_activations = [&]<int slot>(std::integral_constant<int, slot>) {
+  i32x4 staged[kStages][kPieces];
+  const auto fetch_activations = [&](int slot, uint32_t chunk) {
+#pragma unroll
+    for (uint32_t p = 0; p < kPieces; ++p)
+      staged[slot][p] = __builtin_bit_cast(
+          i32x4,
+          __builtin_amdgcn_raw_buffer_load_b128(activations, source_at(p, chunk), 0, 0));
+  };
+  const auto store_activations = [&](int slot, uint8_t* tile) {
 #pragma unroll
     for (uint32_t p = 0; p < kPieces; ++p) {
-      uint4 v = staged[slot][p];
-      v.x = Op::stage(v.x); v.y = Op::stage(v.y);
-      v.z = Op::stage(v.z); v.w = Op::stage(v.w);
-      *reinterpret_cast<uint4*>(&tile[slot][target[p]]) = v;
+      i32x4 v = staged[slot][p];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v[i] = static_cast<int>(Op::stage(static_cast<uint32_t>(v[i])));
+      *reinterpret_cast<i32x4*>(tile + target[p]) = v;
     }
   };
-  uint4 codes[kAhead][T];
-  uint2 scales[kAhead][T];
-  const auto fetch_weights = [&]<int slot>(std::integral_constant<int, slot>,
-                                           uint32_t chunk) {
-    // past the part's end every lane reads one line of the activations: the
-    // next chunk would go to memory for nothing
-    const auto* idle = reinterpret_cast<const uint8_t*>(args.activations);
-    const bool live = chunk < end_chunk;
-    const size_t at = chunk;
+  i32x4 codes[kAhead][T];
+  i32x2 scales[kAhead][T];
+  const auto fetch_weights = [&](int slot, uint32_t chunk) {
+    // nothing is fetched past the part's end
+    const uint32_t at = min(chunk, end_chunk - 1u);
+    const uint32_t past = chunk < end_chunk ? 0u : kPastTheEnd;
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-      codes[slot][t] = *reinterpret_cast<const uint4*>(
-          live ? weight_stream[t] + at * (kTileRows * 32u) : idle);
-      if constexpr (F16) {
-        scales[slot][t] = *reinterpret_cast<const uint2*>(
-            live ? scale_stream[t] + at * (kTileRows * 8u) : idle);
-      } else {
-        scales[slot][t].x = *reinterpret_cast<const uint32_t*>(
-            live ? scale_stream[t] + at * (kTileRows * 2u) : idle);
-        scales[slot][t].y = 0u;
-      }
+      codes[slot][t] = __builtin_bit_cast(
+          i32x4, __builtin_amdgcn_raw_buffer_load_b128(code_stream[t], code_offset | past,
+                                                       at * kCodes, 0));
+      if constexpr (F16)
+        scales[slot][t] = __builtin_bit_cast(
+            i32x2, __builtin_amdgcn_raw_buffer_load_b64(scale_stream[t], scale_offset | past,
+                                                        at * kScales, 0));
+      else
+        scales[slot][t][0] = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(
+            scale_stream[t], scale_offset | past, at * kScales, 0));
     }
   };
 
-  const auto multiply = [&]<int slot, int buffer, int c>(
-                            std::integral_constant<int, slot>,
-                            std::integral_constant<int, buffer>,
-                            std::integral_constant<int, c>) {
+  // Unit u of a chunk: 16 weight rows by 32 columns, u = 2 T s + 2 t + j.
+  constexpr int kUnits = 4 * T;
+  const auto convert = [&](int slot, int unit, Vector (&w)[Op::kParts]) {
+    const int s = unit / (2 * T), t = unit / 2 % T, j = unit % 2;
+    const uint32_t packed = static_cast<uint32_t>(codes[slot][t][2 * j + s]);
+    // scale of (j, s): binary16 halves of the two words, or UE8M0 bytes
+    const uint32_t word = static_cast<uint32_t>(scales[slot][t][F16 ? j : 0]);
+    const uint32_t f16_bits = s ? word >> 16 : word & 0xffffu;
+    const float fold = F16 ? 1.0f : ue8m0_to_f32(word >> (8 * (2 * j + s)) & 0xffu);
+    Op::weights(packed, fold, f16_bits, w);
+  };
+  Vector w[2][Op::kParts];   // of this unit and of the next
+  // activations of this half chunk and of the next, or - heights whose accumulators
+  // leave no room for two - each of the next in the place of the one just used
+  constexpr int kHalves = MT > 5 ? 1 : 2;
+  Vector a[kHalves][MT];
+  const auto fragment = [&](const uint8_t* tile, int c, int s, int mt) {
+    return __builtin_bit_cast(Vector,
+                              *reinterpret_cast<const i32x4*>(
+                                  tile + mt * 16u * kRow + fragment_offset[s] + c * kLdsRow));
+  };
+  // Matrix instructions of a chunk with what the next ones need in between: an
+  // instruction keeps the matrix cores for sixteen cycles and the wave's issue for four.
+  // Told where to put them only where the products outweigh them: heights of up to 64 rows
+  // (binary16 scales: 48) are up to 6 % faster as the compiler orders them.
+  constexpr bool kPaced = MT > (F16 ? 3 : 4);
+  constexpr int kProducts = MT * Op::kParts;               // of a unit
+  constexpr int kConversion = F16 ? 13 : 6;                // vector instructions of a unit
+  const auto multiply = [&](int slot, const uint8_t* tile,
+                            int c) __attribute__((always_inline)) {
+    const bool last_of_step = c + 1 == kSpan;
+    __builtin_amdgcn_sched_barrier(0);
+    if (c == 0)
 #pragma unroll
-    for (uint32_t s = 0; s < 2u; ++s) {
-      Vector a[MT];
+      for (int mt = 0; mt < MT; ++mt) a[0][mt] = fragment(tile, 0, 0, mt);
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-        a[mt] = __builtin_bit_cast(
-            Vector, *reinterpret_cast<const uint4*>(&tile[buffer][
-                        mt * 16u * kRow + fragment_offset[s] + c * kLdsRow]));
+    for (int unit = 0; unit < kUnits; ++unit) {
+      const int s = unit / (2 * T), t = unit / 2 % T, j = unit % 2;
+      const bool reads =
+          unit % (2 * T) == (kHalves > 1 ? 0 : 2 * T - 1) && !(last_of_step && s == 1);
+      const auto read = [&](int mt) {
+        if (reads)
+          a[(1 - s) % kHalves][mt] = fragment(tile, s ? c + 1 : c, s ? 0 : 1, mt);
+      };
+      if constexpr (kHalves > 1)
 #pragma unroll
-      for (int t = 0; t < T; ++t) {
-        const uint4 q = codes[slot][t];
-        const uint32_t packed[4] = {q.x, q.y, q.z, q.w};   // index 2j + s
+        for (int mt = 0; mt < MT; ++mt) read(mt);
+      if (unit + 1 < kUnits)
+        convert(slot, unit + 1, w[(unit + 1) % 2]);
+      else
+        convert((slot + 1) % kAhead, 0, w[(unit + 1) % 2]);
 #pragma unroll
-        for (uint32_t j = 0; j < 2u; ++j) {
-          const uint32_t word = j ? scales[slot][t].y : scales[slot][t].x;
-          const uint32_t f16_bits = s ? word >> 16 : word & 0xffffu;
-          const float fold =
-              F16 ? 1.0f
-                  : ue8m0_to_f32((scales[slot][t].x >> (8u * (2u * j + s))) & 0xffu);
-          Vector w[Op::kParts];
-          Op::weights(packed[2u * j + s], fold, f16_bits, w);
+      for (int part = 0; part < Op::kParts; ++part)
 #pragma unroll
-          for (int half = 0; half < Op::kParts; ++half)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-              acc[mt][t][j] = Op::mfma(a[mt], w[half], acc[mt][t][j]);
+        for (int mt = 0; mt < MT; ++mt) {
+          acc[mt][t][j] = Op::mfma(a[s % kHalves][mt], w[unit % 2][part], acc[mt][t][j]);
+          if (kHalves == 1 && part + 1 == Op::kParts) read(mt);
         }
+      if constexpr (!kPaced) continue;
+#pragma unroll
+      for (int i = 0; i < kProducts; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (reads && (kHalves > 1 ? i < MT : i >= kProducts - MT))
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, (kConversion + kProducts - 1) / kProducts,
+                                             0);
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  using std::integral_constant;
-  // in the order in which the loop waits for them
-  fetch_activations(integral_constant<int, 0>{}, first_chunk);
-  fetch_weights(integral_constant<int, 0>{}, first_chunk);
-  __builtin_amdgcn_sched_barrier(0);
-  fetch_activations(integral_constant<int, 1>{}, first_chunk + kSpan);
-  fetch_weights(integral_constant<int, 1>{}, first_chunk + 1u);
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (kAhead > 2) {
-    fetch_weights(integral_constant<int, 2>{}, first_chunk + 2u);
-    __builtin_amdgcn_sched_barrier(0);
-    fetch_weights(integral_constant<int, 3>{}, first_chunk + 3u);
+  // About in the order in which the loop waits for them.  (The copies' waits count on a
+  // step's weights at least behind those of the second tile.)
+  static_assert(kAhead >= kSpan && kAhead <= 4);
+  constexpr int kWeightsFirst = kAhead > kSpan ? 0 : kTiles - 2;
+#pragma unroll
+  for (int ahead = 0; ahead < std::max(kTiles - 1, kAhead + kWeightsFirst); ++ahead) {
+    if constexpr (kCopied) {
+      if (ahead + 1 < kTiles) copy_activations(tile_of(ahead), first_chunk + ahead * kSpan);
+    } else {
+      if (ahead < kStages) fetch_activations(ahead, first_chunk + ahead * kSpan);
+    }
+    if (ahead >= kWeightsFirst && ahead < kAhead + kWeightsFirst)
+      fetch_weights(ahead - kWeightsFirst, first_chunk + ahead - kWeightsFirst);
     __builtin_amdgcn_sched_barrier(0);
   }
-  store_activations(integral_constant<int, 0>{});
+  if constexpr (kCopied)
+    wait_for_loads<(kTiles - 2) * kPieces + 2u * T * kAhead>();
+  else
+    store_activations(0, tile0);
+  convert(0, 0, w[0]);
 
-  // a chunk's weights are refilled as soon as they have been multiplied
-  const auto one_chunk = [&]<int slot, int buffer, int c>(
-                             integral_constant<int, slot> s,
-                             integral_constant<int, buffer> b,
-                             integral_constant<int, c> in_step, uint32_t chunk) {
-    if (chunk < end_chunk) multiply(s, b, in_step);
-    // the loads stay here: moved up they would need registers of their own and
-    // copies at the loop's end, which wait for them, moved down they come late
-    __builtin_amdgcn_sched_barrier(0);
-    fetch_weights(s, chunk + kAhead);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  const auto step = [&]<int first_slot, int buffer>(integral_constant<int, first_slot>,
-                                                    integral_constant<int, buffer> b,
-                                                    uint32_t chunk) {
-    __syncthreads();   // tile[buffer] is complete; the other one is free
-    fetch_activations(b, chunk + 2u * kSpan);
-    __builtin_amdgcn_sched_barrier(0);
-    one_chunk(integral_constant<int, first_slot>{}, b, integral_constant<int, 0>{}, chunk);
-    if constexpr (kSpan > 1)
-      one_chunk(integral_constant<int, first_slot + 1>{}, b,
-                integral_constant<int, 1>{}, chunk + 1u);
-    if constexpr (kSpan > 2) {
-      one_chunk(integral_constant<int, first_slot + 2>{}, b,
-                integral_constant<int, 2>{}, chunk + 2u);
-      one_chunk(integral_constant<int, first_slot + 3>{}, b,
-                integral_constant<int, 3>{}, chunk + 3u);
+  // Step P of a round.  A chunk's weights are refilled as soon as they have been
+  // multiplied; one past the part's end makes its loads, which fetch nothing, and
+  // multiplies nothing, so that every wait can count on the same loads having been made.
+  const auto step_at = [&]<int P>(std::integral_constant<int, P>,
+                                  uint32_t chunk) __attribute__((always_inline)) {
+    if constexpr (kCopied) {
+      // this step's tile is there: what later steps asked for may be on its way
+      wait_for_loads<(kTiles - 2) * kStepLoads>();
+      barrier_beside_copies();   // everybody's is, and the tile before has been read
+      copy_activations(tile_of(P + kTiles - 1), chunk + (kTiles - 1) * kSpan);
+    } else {
+      __syncthreads();   // this step's tile is complete; the other one is free
+      fetch_activations(P % kStages, chunk + kStages * kSpan);
     }
-    store_activations(integral_constant<int, buffer ^ 1>{});
-  };
-  constexpr integral_constant<int, 0> even;
-  constexpr integral_constant<int, 1> odd;
-  // Whole rounds of kAhead chunks (eight at MT = 1): a step past the part's end
-  // makes its loads and multiplies nothing, so that every wait can count on the
-  // same loads having been made since.
-  for (uint32_t chunk = first_chunk; chunk < end_chunk;) {
-    step(even, even, chunk);
-    chunk += kSpan;
-    step(integral_constant<int, kSpan % kAhead>{}, odd, chunk);
-    chunk += kSpan;
-    if constexpr (kSpan == 1 && kAhead == 4) {
-      step(integral_constant<int, 2>{}, even, chunk);
-      chunk += kSpan;
-      step(integral_constant<int, 3>{}, odd, chunk);
-      chunk += kSpan;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < kSpan; ++c) {
+      const int slot = (P * kSpan + c) % kAhead;
+      if (chunk + c < end_chunk) multiply(slot, tile_of(P), c);
+      // the loads stay here: moved up they would need registers of their own and
+      // copies at the loop's end, which wait for them, moved down they come late
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_weights(slot, chunk + c + kAhead);
+      __builtin_amdgcn_sched_barrier(0);
     }
-  }
+    if constexpr (!kCopied) store_activations((P + 1) % kStages, tile_of(P + 1));
+  };
+  // Rounds of steps, after which every tile, stage and slot has had its turn: of two
+  // stages whole ones (left in between, the compiler waits for more loads than it needs).
+  constexpr int kRound = std::max(kTiles, (kAhead + kSpan - 1) / kSpan);
+  for (uint32_t chunk = first_chunk; chunk < end_chunk; chunk += kRound * kSpan)
+    [&]<int... P>(std::integer_sequence<int, P...>) {
+      (void)((step_at(std::integral_constant<int, P>{}, chunk + P * kSpan),
+              !kCopied || chunk + (P + 1) * kSpan < end_chunk) &&
+             ...);
+    }(std::make_integer_sequence<int, kRound>{});
+  if constexpr (kCopied) wait_for_loads<0>();   // no copy outlives its workgroup
   if (kTailed && work.is_piece)
     store_piece<MT, T>(args, work.piece, acc);
   else
@@ -847,12 +745,16 @@ __global__ __launch_bounds__(256) void tall_parts_kernel(const TallArgs args) {
   }
 }
 
+// Columns from which on a lane's 32-bit offset does not reach over 128 activation rows:
+// such matrices take workgroups of 16 rows.
+constexpr uint32_t kFarColumns = 1u << 24;
+
 bool tall_matrix_ok(const qllm_fp4_matrix* m) {
   return m && m->weights && m->scales && m->rows && m->columns &&
          m->padded_columns >= m->columns && m->padded_columns % kChunk == 0u &&
          (m->scale_scheme == QLLM_SCALE_UE8M0_BLOCK32 ||
           m->scale_scheme == QLLM_SCALE_F16_BLOCK16) &&
-         m->layout == QLLM_LAYOUT_TILED &&
+         m->padded_columns < 8u * kFarColumns && m->layout == QLLM_LAYOUT_TILED &&
          (m->tile_rows == 0u || m->tile_rows == kTileRows);
 }
 
@@ -978,9 +880,11 @@ TallPlan plan_tall(uint32_t rows, uint32_t padded_columns, uint32_t batch,
     const uint32_t height = kHeights[index];
     const bool between = height == 5u || height == 7u;
     if (!timed && between) continue;
+    const bool far = padded_columns >= kFarColumns;
+    if (far && height > 1u) break;
     // one or two tiles of rows where they hold the batch, else the higher ones, and
     // none of which a lower one would hold the batch
-    if (height < 3u ? batch > 16u * height : batch <= 32u) continue;
+    if (height < 3u ? batch > 16u * height && !far : batch <= 32u) continue;
     if (index && batch <= 16u * lower) continue;
     lower = height;
     const ChunkCost cost = kChunkCost[scheme][swiglu][index];
@@ -1023,45 +927,45 @@ void start_tall(const TallArgs& args, uint32_t height, bool swiglu, uint32_t gri
   switch (height) {
     case 1:
       if (swiglu)
-        fp4_gemm_short_kernel<SCHEME, 1, 2, true><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 1, 2, true><<<grid, kThreads, 0, stream>>>(args);
       else
-        fp4_gemm_short_kernel<SCHEME, 1, 1, false><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 1, 1, false><<<grid, kThreads, 0, stream>>>(args);
       break;
     case 2:
       if (swiglu)
-        fp4_gemm_short_kernel<SCHEME, 2, 2, true><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 2, 2, true><<<grid, kThreads, 0, stream>>>(args);
       else
-        fp4_gemm_short_kernel<SCHEME, 2, 1, false><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 2, 1, false><<<grid, kThreads, 0, stream>>>(args);
       break;
     case 3:
       if (swiglu)
-        fp4_gemm_short_kernel<SCHEME, 3, 2, true><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 3, 2, true><<<grid, kThreads, 0, stream>>>(args);
       else
-        fp4_gemm_short_kernel<SCHEME, 3, 1, false><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 3, 1, false><<<grid, kThreads, 0, stream>>>(args);
       break;
     case 4:
       if (swiglu)
-        fp4_gemm_short_kernel<SCHEME, 4, 2, true><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 4, 2, true><<<grid, kThreads, 0, stream>>>(args);
       else
-        fp4_gemm_short_kernel<SCHEME, 4, 1, false><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 4, 1, false><<<grid, kThreads, 0, stream>>>(args);
       break;
     case 5:
       if (swiglu)
-        fp4_gemm_short_kernel<SCHEME, 5, 2, true><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 5, 2, true><<<grid, kThreads, 0, stream>>>(args);
       else
-        fp4_gemm_short_kernel<SCHEME, 5, 2, false><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 5, 2, false><<<grid, kThreads, 0, stream>>>(args);
       break;
     case 7:
       if (swiglu)
-        fp4_gemm_short_kernel<SCHEME, 7, 2, true><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 7, 2, true><<<grid, kThreads, 0, stream>>>(args);
       else
-        fp4_gemm_short_kernel<SCHEME, 7, 2, false><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 7, 2, false><<<grid, kThreads, 0, stream>>>(args);
       break;
     default:
       if (swiglu)
-        fp4_gemm_tall_kernel<SCHEME, true><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 8, 2, true><<<grid, kThreads, 0, stream>>>(args);
       else
-        fp4_gemm_tall_kernel<SCHEME><<<grid, kThreads, 0, stream>>>(args);
+        fp4_gemm_rows_kernel<SCHEME, 8, 2, false><<<grid, kThreads, 0, stream>>>(args);
   }
 }
 

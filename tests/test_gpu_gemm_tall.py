@@ -50,6 +50,49 @@ def test_tall_gemm_matches_oracle(device, scheme, rows, padded, batch):
         assert error < 2e-6 * np.sqrt(padded)
 
 
+@pytest.mark.parametrize("batch", [16, 31, 45, 64, 125])
+@pytest.mark.parametrize("scheme", [ol.SCALE_UE8M0_BLOCK32, ol.SCALE_F16_BLOCK16])
+def test_tall_gemm_steps_ahead(device, scheme, batch):
+    """One to eighteen chunks of K: fewer and more than a workgroup asks for ahead, ends
+    at every place of a round of its tiles and of a step of several chunks."""
+    rng = np.random.default_rng(batch)
+    for chunks in (1, 2, 3, 4, 5, 6, 7, 9, 13, 15, 16, 17, 18):
+        padded = 64 * chunks
+        codes, scales = synth.fp4_matrix(rng, 77, padded, scheme)
+        act = ol.bf16_round(rng.standard_normal((batch, padded)).astype(np.float32))
+        got = tall(device, codes, scales, scheme, 77, padded, act)
+        want = ol.fp4_linear_f64(codes, scales, scheme, 77, padded, act)
+        magnitude = ol.fp4_linear_f64(codes & 0x77, scales, scheme, 77, padded, np.abs(act))
+        # exact products (binary16 scales: two halves each); an addition rounds by 2^-24
+        assert (np.abs(got - want) <= 2 * padded * 2.0 ** -24 * magnitude).all(), chunks
+
+
+@pytest.mark.parametrize("scheme", [ol.SCALE_UE8M0_BLOCK32, ol.SCALE_F16_BLOCK16])
+def test_tall_gemm_of_far_columns(device, scheme):
+    """2^24 columns, past a lane's 32-bit offset over 128 rows of activations."""
+    rows, padded, batch = 40, 1 << 24, 20
+    block = 32 if scheme == ol.SCALE_UE8M0_BLOCK32 else 16
+    codes = torch.randint(0, 256, (rows, padded // 2), dtype=torch.uint8, device=device)
+    scales = (torch.full((rows, padded // 32), 127, dtype=torch.uint8, device=device)
+              if block == 32 else
+              torch.full((rows, padded // 16), 1.0, dtype=torch.float16, device=device))
+    matrix, keep = qh.prepack(qh.fp4_matrix(codes, scales, rows, padded, padded, scheme),
+                              device)
+    columns = [0, 63, 64, padded // 2 + 5, padded - 1]
+    act = torch.zeros((batch, padded), dtype=torch.bfloat16, device=device)
+    x = torch.randn((batch, len(columns)), device=device).bfloat16()
+    act[:, columns] = x
+    out = torch.zeros((batch, rows), device=device)
+    qh.call("qllm_fp4_gemm_bf16_tall", matrix, qh.ptr(act), act.numel() * 2, qh.ptr(out),
+            qh.OUT_F32, None, batch, None)
+    values = torch.tensor([0, .5, 1, 1.5, 2, 3, 4, 6, -0., -.5, -1, -1.5, -2, -3, -4, -6],
+                          dtype=torch.float64, device=device)
+    picked = torch.stack([codes[:, c // 2] >> 4 * (c % 2) & 15 for c in columns], dim=1)
+    want = x.double() @ values[picked.long()].T
+    bound = len(columns) * 2.0 ** -24 * (x.double().abs() @ values[picked.long()].abs().T)
+    assert ((out.double() - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("scheme", [ol.SCALE_UE8M0_BLOCK32, ol.SCALE_F16_BLOCK16])
 def test_tall_gemm_residual_and_bf16_output(device, scheme):
     rng = np.random.default_rng(5)
