@@ -952,6 +952,15 @@ int32_t qllm_mark_presence(uint8_t* emitted, const uint32_t* tokens,
 int32_t qllm_mark_presence_values(uint8_t* emitted, const uint32_t* host_tokens,
                                   uint32_t count, uint32_t vocabulary, void* stream);
 
+/* Hands `count` words of device memory to the host: they go to host_words and then
+ * `sequence` to *host_sequence, both in pinned host memory that the device writes
+ * (hipHostMalloc), after everything enqueued before.  A host that sees the sequence
+ * sees the words, without waiting for the stream.  With `emitted`, emitted[word] = 1
+ * for every word below `vocabulary` in the same launch. */
+int32_t qllm_publish_words(const uint32_t* words, uint32_t count, uint32_t* host_words,
+                           uint32_t* host_sequence, uint32_t sequence, uint8_t* emitted,
+                           uint32_t vocabulary, void* stream);
+
 /* Up to 16 words from host memory (read before the call returns) to device memory:
  * a launch that carries them instead of a copy. */
 int32_t qllm_store_words(uint32_t* destination, const uint32_t* host_words,

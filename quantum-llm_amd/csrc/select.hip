@@ -430,6 +430,23 @@ __global__ __launch_bounds__(64) void mark_values_kernel(uint8_t* emitted, Words
   if (token < vocabulary) emitted[token] = 1u;
 }
 
+// Words to pinned host memory, then the sequence number that says they are there.  In
+// place of a copy, a wait for the stream and a launch that marks the token, a decoded
+// token's turn between two replays of its graph takes 9 us instead of 20.
+__global__ __launch_bounds__(256) void publish_words_kernel(
+    const uint32_t* words, uint32_t count, uint32_t* host_words, uint32_t* host_sequence,
+    uint32_t sequence, uint8_t* emitted, uint32_t vocabulary) {
+  for (uint32_t i = threadIdx.x; i < count; i += 256u) {
+    const uint32_t word = words[i];
+    __hip_atomic_store(host_words + i, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (emitted && word < vocabulary) emitted[word] = 1u;
+  }
+  __threadfence_system();
+  __syncthreads();   // every thread's words are out
+  if (threadIdx.x == 0u)
+    __hip_atomic_store(host_sequence, sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ __launch_bounds__(64) void mark_presence_kernel(
     uint8_t* emitted, const uint32_t* tokens, uint32_t token_count,
     uint32_t count) {
@@ -661,6 +678,17 @@ extern "C" int32_t qllm_mark_presence_values(uint8_t* emitted, const uint32_t* h
   std::copy_n(host_tokens, count, tokens.value);
   mark_values_kernel<<<1, 64, 0, as_stream(stream)>>>(emitted, tokens, count, vocabulary);
   return launched("presence marks");
+}
+
+extern "C" int32_t qllm_publish_words(const uint32_t* words, uint32_t count,
+                                      uint32_t* host_words, uint32_t* host_sequence,
+                                      uint32_t sequence, uint8_t* emitted,
+                                      uint32_t vocabulary, void* stream) {
+  if (!words || !count || !host_words || !host_sequence || (emitted && !vocabulary))
+    return fail(QLLM_INVALID_ARGUMENT, "invalid words to publish");
+  publish_words_kernel<<<1, 256, 0, as_stream(stream)>>>(
+      words, count, host_words, host_sequence, sequence, emitted, vocabulary);
+  return launched("words to the host");
 }
 
 extern "C" int32_t qllm_mark_presence(uint8_t* emitted, const uint32_t* tokens,

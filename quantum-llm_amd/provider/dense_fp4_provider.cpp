@@ -146,21 +146,18 @@ Mi355DenseFp4Provider::Mi355DenseFp4Provider(const DenseGeometry& geometry)
 Mi355DenseFp4Provider::~Mi355DenseFp4Provider() { release(); }
 
 void Mi355DenseFp4Provider::release() {
+  // (a pass's words are read before the runtime knows that the pass has ended)
+  if (stream_) (void)hipStreamSynchronize(static_cast<hipStream_t>(stream_));
   for (void* graph : graphs_)
     if (graph) (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(graph));
   graphs_.clear();
   for (void* graph : mtp_graphs_)
     if (graph) (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(graph));
   mtp_graphs_.clear();
-  if (stream_) (void)hipStreamSynchronize(static_cast<hipStream_t>(stream_));
   for (void* pointer : allocations_) (void)hipFree(pointer);
   allocations_.clear();
   for (void* pointer : prefill_allocations_) (void)hipFree(pointer);
   prefill_allocations_.clear();
-  if (staging_) {
-    (void)hipHostFree(staging_);
-    staging_ = nullptr;
-  }
   selector_.reset();
   kv_slots_ = {};
   slots_.clear();
@@ -199,13 +196,6 @@ void Mi355DenseFp4Provider::allocate_workspaces() {
   // so that one launch brings both
   tokens_ = static_cast<std::uint32_t*>(device_alloc((8U + 4U) * 4U));
   positions_ = tokens_ + 8U;
-  {
-    void* pinned = nullptr;
-    hip_check(hipHostMalloc(&pinned, sizeof(HostStaging), hipHostMallocDefault),
-              "allocate pinned staging");
-    staging_ = static_cast<HostStaging*>(pinned);
-    *staging_ = HostStaging{};
-  }
   graphs_.assign(max_rows_ + 1U, nullptr);
   if (const char* eager = std::getenv("QLLM_PROVIDER_EAGER"))
     use_graphs_ = eager[0] == '0';
@@ -2646,10 +2636,7 @@ std::optional<DraftPrediction> Mi355DenseFp4Provider::run_mtp(
         er::counter_uniform(request_parameter(*request, "sampling_seed"),
                             sample_position, random_stream));
   } else {
-    hip_check(hipMemcpyAsync(&result.token, mtp_argmax_, sizeof(result.token),
-                             hipMemcpyDeviceToHost, hip_stream),
-              "copy final MTP draft token");
-    hip_check(hipStreamSynchronize(hip_stream), "copy final MTP draft token");
+    result.token = selector_->read_token(mtp_argmax_);
     result.distribution.entries.push_back({result.token, 1.0});
   }
   // logits without a finite maximum select no token
@@ -2698,11 +2685,7 @@ void Mi355DenseFp4Provider::propose_with_graphs(
       request_parameter(request, "sampling_temperature_ppm") == 0U;
   if (greedy) {
     launch_mtp_graph(rows, false, drafts);
-    std::uint32_t* const chosen = staging_->download;
-    hip_check(hipMemcpyAsync(chosen, mtp_draft_tokens_, drafts * 4U,
-                             hipMemcpyDeviceToHost, stream),
-              "copy MTP draft tokens");
-    hip_check(hipStreamSynchronize(stream), "copy MTP draft tokens");
+    const std::uint32_t* const chosen = selector_->read_words(mtp_draft_tokens_, drafts);
     for (std::uint32_t depth = 0; depth < drafts; ++depth) {
       // logits without a finite maximum select no token (0xffffffff); the
       // chained pass embedded a row of zeros for it and every kernel ran
@@ -2830,20 +2813,15 @@ er::ExactDecodeExecutionHandle Mi355DenseFp4Provider::execute_exact_decode(
     std::vector<er::SamplingDistribution> target_distributions;
     target_distributions.reserve(rows);
     if (greedy) {
-      // greedy: the rows' arg-max tokens in one copy and one wait
-      const auto stream = static_cast<hipStream_t>(stream_);
-      hip_check(hipMemcpyAsync(staging_->download, argmax_tokens_,
-                               rows * sizeof(std::uint32_t),
-                               hipMemcpyDeviceToHost, stream),
-                "copy exact greedy tokens");
-      hip_check(hipStreamSynchronize(stream), "copy exact greedy tokens");
+      // greedy: the rows' arg-max tokens in one hand-over
+      const std::uint32_t* const chosen = selector_->read_words(argmax_tokens_, rows);
       // a row without a finite logit selects nothing (0xffffffff): reported
       // here, before the proposer or the request state is touched
       for (std::uint32_t row = 0; row < rows; ++row)
-        if (staging_->download[row] >= g_.vocabulary)
+        if (chosen[row] >= g_.vocabulary)
           throw std::runtime_error("target logits have no finite maximum");
       for (std::uint32_t row = 0; row < rows; ++row)
-        target_distributions.push_back({{{staging_->download[row], 1.0}}});
+        target_distributions.push_back({{{chosen[row], 1.0}}});
     } else if (request_parameter(invocation.request, "sampling_top_k") != 0U) {
       target_distributions = selector_->top_k_distributions(
           logits_, g_.vocabulary, g_.vocabulary, rows, invocation.request);

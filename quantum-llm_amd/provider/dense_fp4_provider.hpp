@@ -443,12 +443,6 @@ class Mi355DenseFp4Provider final : public DecoderProvider {
   std::int8_t* query_operands_{};       // Q4H attention operands of a batch
   float* query_operand_scales_{};
   float* rope_table_{};                 // [max_rows, rotary_dim / 2] (cos, sin)
-  // Pinned host words for the chosen tokens that come down after a pass (what
-  // goes up - 8 tokens, 4 position words - travels in a launch's arguments).
-  struct HostStaging {
-    std::uint32_t download[8];
-  };
-  HostStaging* staging_ = nullptr;
   float* projection_partials_ = nullptr;   // [splits][rows][hidden]
   std::uint32_t projection_splits_ = 3U;   // 0 / 1: residual in the epilogue
   // The q/k/v projection cut along K the same way (QLLM_PROVIDER_QKV_SPLITS);

@@ -746,11 +746,11 @@ void Mi355MixedProvider::ensure_workspace(std::uint32_t rows, std::uint32_t last
   std::uint32_t size = 64U;
   while (size < rows) size *= 2U;
   size = std::min(std::max({size, rows, workspace_rows_}), std::max(g_.chunk_rows, 64U));
+  hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream_)), "grow workspace");
   if (step_graph_) {   // it addresses the buffers that are about to go
     (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(step_graph_));
     step_graph_ = nullptr;
   }
-  hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream_)), "grow workspace");
   const std::size_t element = g_.element == QLLM_ELEMENT_F32 ? 4U : 2U;
   const auto zeroed = [](std::size_t bytes, const char* what) {
     DeviceBuffer buffer(std::max<std::size_t>(bytes, 16U), what);

@@ -6,7 +6,10 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
+#include <chrono>
 #include <cmath>
+#include <cstring>
 #include <numeric>
 #include <stdexcept>
 
@@ -46,15 +49,32 @@ void TokenSelector::mark(
                                          vocabulary_, stream_));
 }
 
-// One word of device memory, through pinned memory: a copy to pageable memory is
-// staged and waited for twice.
-std::uint32_t TokenSelector::read_token(const std::uint32_t* device_token) {
-  const auto stream = static_cast<hipStream_t>(stream_);
-  hip_check(hipMemcpyAsync(&staging_->token, device_token, sizeof(std::uint32_t),
-                           hipMemcpyDeviceToHost, stream),
-            "copy greedy token");
-  hip_check(hipStreamSynchronize(stream), "copy greedy token");
-  return staging_->token;
+std::uint32_t TokenSelector::read_token(const std::uint32_t* device_token,
+                                        std::uint8_t* emitted) {
+  return *read_words(device_token, 1U, emitted);
+}
+
+// The device writes the words into pinned memory and the host watches them arrive: a
+// copy and a wait for the stream after it took 8 us longer.  What has not arrived after
+// two milliseconds - a long prompt, or a device that has failed - is waited for with the
+// stream, which reports what went wrong.
+const std::uint32_t* TokenSelector::read_words(const std::uint32_t* device_words,
+                                               std::uint32_t count, std::uint8_t* emitted) {
+  if (!count || count > kMostWords) throw std::runtime_error("invalid device words to read");
+  const std::uint32_t sequence = ++sequence_;
+  status_check(qllm_publish_words(device_words, count, staging_->words, &staging_->sequence,
+                                  sequence, emitted, vocabulary_, stream_));
+  const auto arrived = [&] {
+    return __atomic_load_n(&staging_->sequence, __ATOMIC_ACQUIRE) == sequence;
+  };
+  const auto deadline = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+  while (!arrived()) {
+    for (int turn = 0; turn < 64 && !arrived(); ++turn) __builtin_ia32_pause();
+    if (std::chrono::steady_clock::now() < deadline) continue;
+    hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream_)), "wait for the device");
+    if (!arrived()) throw std::runtime_error("the device's words have not arrived");
+  }
+  return staging_->words;
 }
 
 // The head's token for a request (run_head with a request, :8433-8517): the
@@ -82,7 +102,7 @@ std::uint32_t TokenSelector::select(float* logits, std::uint8_t* presence,
   const auto temperature = request_parameter(request, "sampling_temperature_ppm");
   std::uint32_t selected{};
   if (temperature == 0U) {
-    selected = read_token(argmax_tokens);
+    selected = read_token(argmax_tokens, output_sampling ? presence : nullptr);
     // a row without a finite logit selects nothing (0xffffffff): reported
     // before the presence bytes or the caller's state change
     if (selected >= vocabulary_)
@@ -137,7 +157,7 @@ std::uint32_t TokenSelector::select(float* logits, std::uint8_t* presence,
                               sample_position, 0U));
     }
   }
-  if (output_sampling) {
+  if (output_sampling && temperature != 0U) {   // (read_token has marked the other)
     const std::uint32_t token[1] = {selected};
     mark(presence, token);
   }
@@ -231,24 +251,21 @@ TokenSelector::top_k_distributions(
                                       workspace_bytes_, stream_));
   // logits of all rows, then tokens of all rows (the device buffers are
   // adjacent with room for 8 rows of 64)
-  constexpr std::size_t kCapacity = 8U * kMaximumTopK;
-  hip_check(hipMemcpyAsync(staging_->top_logits, top_logits_,
-                           kCapacity * 4U + std::size_t{rows} * top_k * 4U,
-                           hipMemcpyDeviceToHost, stream),
-            "copy speculative top-k");
-  hip_check(hipStreamSynchronize(stream), "copy speculative top-k");
+  constexpr std::uint32_t kCapacity = 8U * kMaximumTopK;
+  const std::uint32_t* words = read_words(reinterpret_cast<const std::uint32_t*>(top_logits_),
+                                          kCapacity + rows * top_k);
   ++gpu_calls_;
   logit_transfer_bytes_ += std::size_t{rows} * top_k * 8U;
   std::vector<er::SamplingDistribution> result;
   result.reserve(rows);
   for (std::uint32_t row = 0; row < rows; ++row) {
-    const std::span<const float> row_logits(
-        staging_->top_logits + std::size_t{row} * top_k, top_k);
+    std::array<float, kMaximumTopK> row_logits;
+    std::memcpy(row_logits.data(), words + std::size_t{row} * top_k, top_k * sizeof(float));
     const std::span<const std::uint32_t> row_tokens(
-        staging_->top_tokens + std::size_t{row} * top_k, top_k);
+        words + kCapacity + std::size_t{row} * top_k, top_k);
     result.push_back(er::make_sampling_distribution(
-        row_logits, row_tokens, static_cast<std::uint32_t>(temperature), top_p,
-        min_p));
+        std::span<const float>(row_logits.data(), top_k), row_tokens,
+        static_cast<std::uint32_t>(temperature), top_p, min_p));
   }
   return result;
 }

@@ -42,8 +42,16 @@ class TokenSelector final {
   [[nodiscard]] std::vector<er::SamplingDistribution> top_k_distributions(
       const float* logits, std::uint32_t vocabulary, std::size_t stride,
       std::uint32_t rows, const er::ProgramRequestContext& request);
-  // A selection on the device, after everything enqueued so far.
-  [[nodiscard]] std::uint32_t read_token(const std::uint32_t* device_token);
+  // A selection on the device, after everything enqueued so far; with `emitted` it is
+  // marked there (if it is a token).
+  [[nodiscard]] std::uint32_t read_token(const std::uint32_t* device_token,
+                                         std::uint8_t* emitted = nullptr);
+  // Up to kMostWords words of device memory, after everything enqueued so far: there
+  // until the next call.
+  static constexpr std::uint32_t kMostWords = 2U * 8U * kMaximumTopK;
+  [[nodiscard]] const std::uint32_t* read_words(const std::uint32_t* device_words,
+                                                std::uint32_t count,
+                                                std::uint8_t* emitted = nullptr);
   // emitted[token] = 1 for every token (one launch)
   void mark(std::uint8_t* emitted, std::span<const std::uint32_t> tokens);
 
@@ -53,10 +61,10 @@ class TokenSelector final {
   }
 
  private:
+  // Pinned: written by the device, the sequence number after the words it stands for.
   struct Staging final {
-    float top_logits[8 * kMaximumTopK];            // top-k readback: logits of all
-    std::uint32_t top_tokens[8 * kMaximumTopK];    // rows, then their tokens
-    std::uint32_t token;                           // one row's selection
+    std::uint32_t words[kMostWords];
+    alignas(64) std::uint32_t sequence;
   };
   void* stream_{};
   std::uint32_t vocabulary_{};
@@ -66,6 +74,7 @@ class TokenSelector final {
   float* top_logits_{};
   std::uint32_t* top_tokens_{};
   Staging* staging_{};
+  std::uint32_t sequence_{};
   std::uint64_t gpu_calls_{};
   std::uint64_t logit_transfer_bytes_{};
 };

@@ -287,6 +287,7 @@ SIGNATURES = {
     "qllm_apply_presence_penalty": (c_int32, [c_void_p, c_void_p, c_uint32, c_float, c_void_p]),
     "qllm_apply_presence_penalty_rows": (c_int32, [c_void_p, c_size_t, c_void_p, c_void_p, c_uint32, c_uint32, c_float, c_void_p]),
     "qllm_mark_presence_values": (c_int32, [c_void_p, c_void_p, c_uint32, c_uint32, c_void_p]),
+    "qllm_publish_words": (c_int32, [c_void_p, c_uint32, c_void_p, c_void_p, c_uint32, c_void_p, c_uint32, c_void_p]),
     "qllm_store_words": (c_int32, [c_void_p, c_void_p, c_uint32, c_void_p]),
     "qllm_mark_presence": (c_int32, [c_void_p, c_void_p, c_uint32, c_uint32, c_void_p]),
     "qllm_linear_packed_bytes": (c_size_t, [c_uint32, c_uint32]),

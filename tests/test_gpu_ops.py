@@ -1,4 +1,6 @@
 """Small per-row kernels and token selection on the GPU against the oracle."""
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -500,3 +502,36 @@ def test_words_and_marks_travel_in_a_launch(device, count):
         with pytest.raises(qh.QllmError, match="invalid"):
             qh.call(name, qh.ptr(target), np.zeros(17, np.uint32).ctypes.data, 17, *arguments,
                     None)
+
+
+@pytest.mark.parametrize("count", [1, 5, 256, 257, 1024])
+def test_words_reach_pinned_memory_before_their_sequence_number(device, count):
+    """The host sees the words as soon as it sees the number, also while work enqueued
+    behind them is running; words below the vocabulary are marked."""
+    words = torch.randint(-2 ** 31, 2 ** 31 - 1, (count,), dtype=torch.int32)
+    words[::2] %= 64
+    source = words.to(device)
+    host = torch.zeros(count, dtype=torch.int32).pin_memory()
+    sequence = torch.zeros(1, dtype=torch.int32).pin_memory()
+    emitted = torch.zeros(40, dtype=torch.uint8, device=device)
+    busy = torch.zeros(1 << 28, dtype=torch.uint8, device=device)
+    torch.cuda.synchronize()
+    stream = torch.cuda.current_stream().cuda_stream
+    for number in range(1, 4):
+        host.zero_()
+        qh.call("qllm_publish_words", qh.ptr(source), count, qh.ptr(host), qh.ptr(sequence),
+                number, qh.ptr(emitted) if number == 1 else None, 40, stream)
+        busy.add_(1)
+        deadline = time.monotonic() + 5.0
+        while int(sequence[0]) != number and time.monotonic() < deadline:
+            pass
+        assert int(sequence[0]) == number
+        assert torch.equal(host, words)
+    torch.cuda.synchronize()
+    expected = torch.zeros(40, dtype=torch.uint8)
+    expected[words[(words >= 0) & (words < 40)].long()] = 1
+    assert torch.equal(emitted.cpu(), expected)
+    for bad in ((None, 1), (qh.ptr(source), 0)):
+        with pytest.raises(qh.QllmError, match="invalid"):
+            qh.call("qllm_publish_words", *bad, qh.ptr(host), qh.ptr(sequence), 1, None, 0,
+                    stream)
