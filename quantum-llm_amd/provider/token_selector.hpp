@@ -66,13 +66,13 @@ class TokenSelector final {
     std::uint32_t words[kMostWords];
     alignas(64) std::uint32_t sequence;
   };
+  static constexpr std::uint32_t kPassesBetweenWaits = 16U;
   void* stream_{};
   std::uint32_t vocabulary_{};
   void* workspace_{};
   std::size_t workspace_bytes_{};
   DeviceBuffer device_;
   float* top_logits_{};
-  std::uint32_t* top_tokens_{};
   Staging* staging_{};
   std::uint32_t sequence_{};
   std::uint64_t gpu_calls_{};
