@@ -344,6 +344,26 @@ int32_t qllm_fp4_embedding_batch(const qllm_fp4_matrix* matrix,
                                  const uint32_t* tokens, float* output,
                                  uint32_t batch, void* stream);
 
+/* The rotary table of qllm_rope_table beside another launch. */
+typedef struct qllm_rope_rows {
+  float* table;
+  uint32_t rotary_dim;
+  uint32_t first_rotary_position;
+  float theta;
+  int32_t bf16_activations;
+  const uint32_t* device_positions;
+} qllm_rope_rows;
+
+/* qllm_fp4_embedding_batch into `hidden`, the norm of its rows as qllm_rms_norm_batch
+ * (output_bf16, rows of `columns`) or qllm_rms_norm_q8_batch (output_q8, output_scales)
+ * gives it, and with `rope` qllm_rope_table's rows, in one launch and with the same bits.
+ * Up to 16384 columns, a multiple of 4; `hidden` and `weight` aligned to 16 bytes. */
+int32_t qllm_fp4_embedding_norm_batch(const qllm_fp4_matrix* matrix, const uint32_t* tokens,
+                                      float* hidden, const float* weight, void* output_bf16,
+                                      int8_t* output_q8, float* output_scales, uint32_t rows,
+                                      float epsilon, int32_t zero_centered,
+                                      const qllm_rope_rows* rope, void* stream);
+
 /* ---- normalisation and elementwise ---------------------------------------- */
 
 /* replaces rms_norm_batch / weightless_rms_norm_batch and the zero-centred

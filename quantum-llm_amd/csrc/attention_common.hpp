@@ -120,6 +120,22 @@ __device__ __forceinline__ uint32_t lds_address(const void* pointer) {
       (__attribute__((address_space(3))) const void*)pointer));
 }
 
+// (cos, sin) of a row's rotary angle for one pair of dimensions.
+__device__ __forceinline__ float2 rotary_angle(uint32_t position, uint32_t pair,
+                                               uint32_t rotary_dim, float theta,
+                                               bool bf16_activations) {
+  const float angle = static_cast<float>(position) *
+                      powf(theta, -2.0f * static_cast<float>(pair) /
+                                      static_cast<float>(rotary_dim));
+  float sine, cosine;
+  sincosf(angle, &sine, &cosine);
+  if (bf16_activations) {
+    cosine = bf16_round(cosine);
+    sine = bf16_round(sine);
+  }
+  return make_float2(cosine, sine);
+}
+
 // A word of a small device-side parameter block (step positions) that no
 // kernel writes: fetched with a scalar load, like the page table.
 __device__ __forceinline__ uint32_t uniform_word(const uint32_t* words,

@@ -402,19 +402,9 @@ __global__ void rope_table_kernel(float2* table, uint32_t rotary_dim,
     first_rotary_position = uniform_word(device_positions, 1u);
   const uint32_t half = rotary_dim / 2u;
   const uint32_t row = blockIdx.x;
-  for (uint32_t pair = threadIdx.x; pair < half; pair += blockDim.x) {
-    const float angle =
-        static_cast<float>(first_rotary_position + row) *
-        powf(theta, -2.0f * static_cast<float>(pair) /
-                        static_cast<float>(rotary_dim));
-    float sine, cosine;
-    sincosf(angle, &sine, &cosine);
-    if (bf16_activations) {
-      cosine = bf16_round(cosine);
-      sine = bf16_round(sine);
-    }
-    table[row * half + pair] = make_float2(cosine, sine);
-  }
+  for (uint32_t pair = threadIdx.x; pair < half; pair += blockDim.x)
+    table[row * half + pair] = rotary_angle(first_rotary_position + row, pair, rotary_dim,
+                                            theta, bf16_activations);
 }
 
 // D = head_dim (128 or 256), RT = number of 16-row tiles (rows*group <= 16*RT).

@@ -11,6 +11,7 @@
 #include <cstring>
 #include <numeric>
 #include <stdexcept>
+#include <utility>
 
 namespace qllm {
 namespace {
@@ -1403,12 +1404,13 @@ void Mi355DenseFp4Provider::enqueue_attention_block(std::uint32_t index,
                                                     std::uint32_t rows,
                                                     std::uint32_t first_position,
                                                     bool deferred_positions,
-                                                    bool leave_partials) {
+                                                    bool leave_partials,
+                                                    bool normalised) {
   const auto& layer = layers_[index];
   const std::size_t hidden_bytes = std::size_t{rows} * g_.hidden * 2U;
   const std::size_t attention_bytes =
       std::size_t{rows} * g_.query_heads * g_.head_dim * 2U;
-  enqueue_normalise(layer.input_norm, rows);
+  if (!normalised) enqueue_normalise(layer.input_norm, rows);
   // query, key and value projections (:7004-7011) in one launch
   const std::uint32_t kv_rows = g_.kv_heads * g_.head_dim;
   if (g_.activation_q8) {
@@ -1550,7 +1552,21 @@ void Mi355DenseFp4Provider::enqueue_target(const std::uint32_t* device_tokens,
     enqueue();
     end_gpu_phase(events);
   };
+  // the lookup, the rotary table and the first norm in one launch (phases are timed one
+  // by one, and longer rows take the launches of their own)
+  const bool together = !g_.profile_gpu_phases && g_.layers != 0U &&
+                        g_.hidden % 4U == 0U && g_.hidden <= 16384U;
   timed(GpuPhase::embedding, [&] {
+    if (together) {
+      const qllm_rope_rows rope{rope_table_, g_.rotary_dim, first_position, g_.rope_theta, 0,
+                                deferred_positions ? positions_ : nullptr};
+      status_check(qllm_fp4_embedding_norm_batch(
+          &embedding_.descriptor, device_tokens, hidden_, layers_.front().input_norm,
+          g_.activation_q8 ? nullptr : normalized_, g_.activation_q8 ? q8_ : nullptr,
+          g_.activation_q8 ? q8_scales_ : nullptr, rows, g_.norm_epsilon,
+          g_.zero_centered_norm, &rope, stream_));
+      return;
+    }
     status_check(qllm_fp4_embedding_batch(&embedding_.descriptor, device_tokens,
                                           hidden_, rows, stream_));
     enqueue_rope_table(rows, first_position, deferred_positions);
@@ -1559,7 +1575,7 @@ void Mi355DenseFp4Provider::enqueue_target(const std::uint32_t* device_tokens,
   for (std::uint32_t index = 0; index < g_.layers; ++index) {
     timed(GpuPhase::full_attention, [&] {
       enqueue_attention_block(index, rows, first_position, deferred_positions,
-                              true);
+                              true, together && index == 0U);
     });
     timed(GpuPhase::ffn, [&] { enqueue_ffn_block(index, rows, true); });
   }
@@ -1768,16 +1784,28 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
       hip_check(hipMemcpyAsync(prefill_tokens_, tokens.data() + done, rows * 4U,
                                hipMemcpyHostToDevice, hip_stream),
                 "upload prompt tokens");
-      status_check(qllm_fp4_embedding_batch(&embedding_.descriptor,
-                                            prefill_tokens_, prefill_hidden_,
-                                            rows, stream));
-      status_check(qllm_rope_table(prefill_rope_table_, rows, g_.rotary_dim, position,
-                                   g_.rope_theta, 0, nullptr, stream));
+      // (as a verify step starts)
+      bool normalised = g_.layers != 0U && g_.hidden % 4U == 0U && g_.hidden <= 16384U;
+      if (normalised) {
+        const qllm_rope_rows rope{prefill_rope_table_, g_.rotary_dim, position,
+                                  g_.rope_theta, 0, nullptr};
+        status_check(qllm_fp4_embedding_norm_batch(
+            &embedding_.descriptor, prefill_tokens_, prefill_hidden_,
+            layers_.front().input_norm, prefill_normalized_, nullptr, nullptr, rows,
+            g_.norm_epsilon, g_.zero_centered_norm, &rope, stream));
+      } else {
+        status_check(qllm_fp4_embedding_batch(&embedding_.descriptor,
+                                              prefill_tokens_, prefill_hidden_,
+                                              rows, stream));
+        status_check(qllm_rope_table(prefill_rope_table_, rows, g_.rotary_dim, position,
+                                     g_.rope_theta, 0, nullptr, stream));
+      }
       const std::size_t hidden_bytes = std::size_t{rows} * g_.hidden * 2U;
       // A projection onto the residual stream whose launch is cut along K leaves
       // its parts to the norm that follows, as in a verify step.
       std::uint32_t parts = 0U;
       const auto normalise = [&](const float* weight) {
+        if (std::exchange(normalised, false)) return;
         if (parts)
           status_check(qllm_rms_norm_residual_batch(
               prefill_hidden_, prefill_parts_, parts, weight, prefill_normalized_,

@@ -309,7 +309,8 @@ class Mi355DenseFp4Provider final : public DecoderProvider {
                           bool deferred_positions);
   void enqueue_attention_block(std::uint32_t index, std::uint32_t rows,
                                std::uint32_t first_position,
-                               bool deferred_positions, bool leave_partials);
+                               bool deferred_positions, bool leave_partials,
+                               bool normalised = false);
   void enqueue_ffn_block(std::uint32_t index, std::uint32_t rows,
                          bool leave_partials);
   void enqueue_head(std::uint32_t first_row, std::uint32_t rows);

@@ -110,6 +110,12 @@ class LinearSegment(Structure):
                 ("epilogue", c_uint32), ("activation", c_uint32), ("splits", c_uint32)]
 
 
+class RopeRows(Structure):
+    _fields_ = [("table", c_void_p), ("rotary_dim", c_uint32),
+                ("first_rotary_position", c_uint32), ("theta", c_float),
+                ("bf16_activations", c_int32), ("device_positions", c_void_p)]
+
+
 class TokenShift(Structure):
     _fields_ = [("count", c_uint32), ("mu", c_void_p * 6), ("output", c_void_p * 6),
                 ("previous", c_void_p), ("slot_stride", c_uint64), ("last", c_void_p)]
@@ -287,6 +293,7 @@ SIGNATURES = {
     "qllm_apply_presence_penalty": (c_int32, [c_void_p, c_void_p, c_uint32, c_float, c_void_p]),
     "qllm_apply_presence_penalty_rows": (c_int32, [c_void_p, c_size_t, c_void_p, c_void_p, c_uint32, c_uint32, c_float, c_void_p]),
     "qllm_mark_presence_values": (c_int32, [c_void_p, c_void_p, c_uint32, c_uint32, c_void_p]),
+    "qllm_fp4_embedding_norm_batch": (c_int32, [POINTER(Fp4Matrix), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_uint32, c_float, c_int32, POINTER(RopeRows), c_void_p]),
     "qllm_publish_words": (c_int32, [c_void_p, c_uint32, c_void_p, c_void_p, c_uint32, c_void_p, c_uint32, c_void_p]),
     "qllm_store_words": (c_int32, [c_void_p, c_void_p, c_uint32, c_void_p]),
     "qllm_mark_presence": (c_int32, [c_void_p, c_void_p, c_uint32, c_uint32, c_void_p]),

@@ -1,4 +1,5 @@
 """Small per-row kernels and token selection on the GPU against the oracle."""
+import ctypes
 import time
 
 import numpy as np
@@ -535,3 +536,52 @@ def test_words_reach_pinned_memory_before_their_sequence_number(device, count):
         with pytest.raises(qh.QllmError, match="invalid"):
             qh.call("qllm_publish_words", *bad, qh.ptr(host), qh.ptr(sequence), 1, None, 0,
                     stream)
+
+
+@pytest.mark.parametrize("columns", [4, 252, 2048, 5120, 16384])
+@pytest.mark.parametrize("scheme", [ol.SCALE_UE8M0_BLOCK32, ol.SCALE_F16_BLOCK16])
+@pytest.mark.parametrize("rows,rotary,q8,zero_centered", [
+    (1, 128, False, False), (5, 64, True, True), (33, 6, False, True), (7, 256, True, False)])
+def test_the_start_of_a_pass_equals_its_launches(device, columns, scheme, rows, rotary, q8,
+                                                 zero_centered):
+    """Lookup, norm (or norm and quantisation) and rotary table in one launch, a token
+    outside the vocabulary among them: the bits of the launches one by one."""
+    rng = np.random.default_rng(columns + rows)
+    padded, vocabulary, epsilon, theta = -(-columns // 32) * 32, 37, 1e-6, 1e6
+    codes, scales = synth.fp4_matrix(rng, vocabulary, padded, scheme)
+    codes, scales = gu.device_tensor(codes, device), gu.device_tensor(scales, device)
+    matrix = qh.fp4_matrix(codes, scales, vocabulary, columns, padded, scheme)
+    tokens = torch.from_numpy(rng.integers(0, vocabulary, rows).astype(np.int32)).to(device)
+    tokens[rows // 2] = vocabulary
+    weight = torch.from_numpy(rng.standard_normal(columns).astype(np.float32)).to(device)
+    positions = torch.tensor([11, 12, 13, 0], dtype=torch.int32, device=device)
+
+    def buffers():
+        return (torch.full((rows, columns), 7.0, device=device),
+                torch.full((rows, columns), 7, device=device,
+                           dtype=torch.int8 if q8 else torch.bfloat16),
+                torch.full((rows,), 7.0, device=device),
+                torch.full((rows, rotary), 7.0, device=device))
+
+    hidden, out, out_scales, table = apart = buffers()
+    qh.call("qllm_fp4_embedding_batch", matrix, qh.ptr(tokens), qh.ptr(hidden), rows, None)
+    if q8:
+        qh.call("qllm_rms_norm_q8_batch", qh.ptr(hidden), qh.ptr(weight), qh.ptr(out),
+                qh.ptr(out_scales), rows, columns, epsilon, zero_centered, None)
+    else:
+        qh.call("qllm_rms_norm_batch", qh.ptr(hidden), qh.ptr(weight), None, qh.ptr(out),
+                columns, rows, columns, epsilon, zero_centered, None)
+    qh.call("qllm_rope_table", qh.ptr(table), rows, rotary, 12, theta, 0, None, None)
+    for on_device in (False, True):
+        together = hidden, out, out_scales, table = buffers()
+        rope = qh.RopeRows(qh.ptr(table), rotary, 0 if on_device else 12, theta, 0,
+                           qh.ptr(positions) if on_device else None)
+        qh.call("qllm_fp4_embedding_norm_batch", matrix, qh.ptr(tokens), qh.ptr(hidden),
+                qh.ptr(weight), None if q8 else qh.ptr(out), qh.ptr(out) if q8 else None,
+                qh.ptr(out_scales) if q8 else None, rows, epsilon, zero_centered,
+                ctypes.byref(rope), None)
+        for one, other in zip(together, apart):
+            assert torch.equal(one.view(torch.uint8), other.view(torch.uint8))
+    with pytest.raises(qh.QllmError, match="invalid"):
+        qh.call("qllm_fp4_embedding_norm_batch", matrix, qh.ptr(tokens), qh.ptr(hidden),
+                qh.ptr(weight), None, None, None, rows, epsilon, 0, None, None)
