@@ -1143,6 +1143,14 @@ typedef struct qllm_token_rows {
 int32_t qllm_stream_norm_tokens(const qllm_stream_norm_launch* launch,
                                 const qllm_token_rows* tokens, void* stream);
 
+/* qllm_stream_norm (with `tokens`, not NULL, qllm_stream_norm_tokens) followed by
+ * qllm_linear_batch of its rows, whose results it has.  For a single row that is one launch
+ * where every segment stores or gates what it reads from the norm's outputs and the row is
+ * not too long; the normalised rows themselves are then not written. */
+int32_t qllm_linear_normed(const qllm_stream_norm_launch* norm, const qllm_token_rows* tokens,
+                           const qllm_linear_segment* segments, uint32_t count,
+                           void* stream);
+
 /* ---- windowed attention with mixed heads ---------------------------------- */
 
 /* Geometry of one attention layer.  A page holds, from layer_offset on, the

@@ -27,7 +27,7 @@
 //    over K was (of [11264, 2048] 1.9e-7 up to 64 rows and 4.9e-7 above, 8.1e-7
 //    before), and it takes 13 us for one row and 73 for 333 instead of 330 and 440.
 #include "common.hpp"
-#include "mixed_common.hpp"
+#include "mixed_norm.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -50,7 +50,9 @@ struct LinearArgs {
 
 __device__ __forceinline__ uint32_t segment_of(const LinearArgs& args, uint32_t unit) {
   uint32_t index = 0;
-  while (index + 1u < args.count && unit >= args.first_unit[index + 1u]) ++index;
+#pragma unroll
+  for (uint32_t i = 1; i < kMaximumSegments; ++i)   // (one trip to memory for all of them)
+    index += i < args.count && unit >= args.first_unit[i] ? 1u : 0u;
   return index;
 }
 
@@ -286,6 +288,292 @@ __global__ __launch_bounds__(kSmallWaves* kWave) void linear_small_kernel(Linear
                                                                   scratch);
   else
     small_unit<F32, MT, 1, kUnroll>(s, unit, args.batch, scratch);
+}
+
+// ---- one token with its norm ----------------------------------------------------
+//
+// A token's norm is one workgroup that everything waits for: 4 - 5 us of launch and memory
+// latency, one or two of them a layer.  Here every workgroup of the projection takes
+// the norm by itself instead, from the caches (up to ten rows, 80 KB at width 2048, as much
+// as its weights), after its weight loads have set out, so that a token waits for one memory
+// latency instead of two.  The weights stream through the registers: each is loaded for the
+// next tile as soon as it has been used.  In 32-bit mode the activation is split into its
+// parts once a workgroup instead of once for every matrix instruction.
+// Norm of a row with six partial sums and projection, us, two launches and this one:
+//   2048 columns, bf16: 545 tiles 12.2 -> 10.0, 996 15.6 -> 13.1, 2000 26.0 -> 22.9
+//   2048 columns, F32: 545 tiles 14.6 -> 10.5, 996 19.1 -> 13.5, 2000 30.1 -> 23.0
+//   4096 columns, bf16: 545 tiles 20.1 -> 16.5, 996 gated 56.9 -> 47.2
+
+constexpr uint32_t kNormedThreads = kSmallWaves * kWave;
+constexpr uint32_t kNormedWidth = 4u * kNormedThreads;   // values of a piece of every thread
+constexpr uint32_t kNormedParts = 8;                     // most partial sums of the stream
+
+struct NormedArgs {
+  LinearArgs linear;                     // first_unit counts workgroups
+  NormArgs norm;
+  uint32_t source[kMaximumSegments];     // what a segment reads: weight[0 or 1], 2 + shift
+};
+
+// The norm's row `source` as operands of the matrix instructions (of 32-bit mode its three
+// parts one after the other, kNormedWidth * PIECES apart), to `values`, zeros from the width
+// on to `columns`: the sums, products and roundings of stream_norm_wide_kernel for one row,
+// whose waves these are with PIECES == 1 and two by two with 2.  Workgroup `first` leaves
+// the stream and the carried row.  `set_out` runs once all that the norm reads is asked for.
+template <bool F32, int PIECES, typename SetOut>
+__device__ __forceinline__ void normed_row(const NormArgs& args, uint32_t source,
+                                           uint32_t columns, bool first, uint16_t* values,
+                                           float* scratch, const SetOut& set_out) {
+  constexpr uint32_t kRow = PIECES * kNormedWidth;
+  const qllm_stream_norm_launch& l = args.launch;
+  const qllm_token_shift& shift = args.shift;
+  const uint32_t pieces = l.width / 4u;
+  const uint32_t wave = threadIdx.x / kWave;
+  const bool table = args.tokens.table != nullptr;
+  const bool blended = source >= 2u;
+  const auto row_of = [](const float* rows, uint32_t piece) {
+    return reinterpret_cast<const f32x4*>(rows)[piece];
+  };
+  f32x4 held[PIECES], before[PIECES], weight[PIECES], share[PIECES];
+  i32x4 part[PIECES][kNormedParts];
+  // (absent partial sums lie past the end of the range: nothing is fetched)
+  const auto parts =
+      memory_range(l.partials, size_t{l.partial_count} * l.partial_stride * 4u);
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const uint32_t piece = min(threadIdx.x + i * kNormedThreads, pieces - 1u);
+    held[i] = f32x4{};
+    if (table) {
+      if (const uint16_t* values16 = table_row(args, 0u)) {
+        const i32x2 bits = reinterpret_cast<const i32x2*>(values16)[piece];
+        held[i][0] = __int_as_float(bits[0]);
+        held[i][1] = __int_as_float(bits[1]);
+      }
+    } else if (!l.branch_weight) {
+      held[i] = row_of(l.input, piece);
+    }
+#pragma unroll
+    for (uint32_t p = 0; p < kNormedParts; ++p)
+      part[i][p] = __builtin_bit_cast(
+          i32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     parts, piece * 16u + p * l.partial_stride * 4u, 0, 0));
+    if (l.branch_weight) {
+      before[i] = row_of(l.input, piece);
+      share[i] = row_of(l.branch_weight, piece);
+    }
+    if (blended) {
+      before[i] = row_of(shift.previous + l.step[kStepSlot] * shift.slot_stride, piece);
+      share[i] = row_of(shift.mu[source - 2u], piece);
+    }
+    weight[i] = row_of(l.weight[source == 1u ? 1 : 0], piece);
+  }
+  set_out();
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    if (table)
+      held[i] = bf16_values4(i32x2{__float_as_int(held[i][0]), __float_as_int(held[i][1])},
+                             args.tokens.scale);
+    if (l.partial_count)
+#pragma unroll
+      for (uint32_t p = 0; p < kNormedParts; ++p)
+        held[i] += __builtin_bit_cast(f32x4, part[i][p]);
+  }
+  const auto inside = [&](int i) { return threadIdx.x + i * kNormedThreads < pieces; };
+  const auto inverse_of = [&](float epsilon) __attribute__((always_inline)) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      float squares = 0.0f;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) squares = fmaf(held[i][c], held[i][c], squares);
+      squares = wave_sum(inside(i) ? squares : 0.0f);
+      if (threadIdx.x % kWave == 0u) scratch[i * kSmallWaves + wave] = squares;
+    }
+    __syncthreads();
+    float total = 0.0f;
+#pragma unroll
+    for (uint32_t w = 0; w < PIECES * kSmallWaves; ++w) total += scratch[w];
+    return inverse_rms(total, l.width, epsilon);
+  };
+  if (l.branch_weight) {
+    const float unit = inverse_of(l.branch_epsilon);
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        held[i][c] = fmaf(held[i][c] * unit * share[i][c], l.branch_scale, before[i][c]);
+  }
+  if (first && (table || l.partial_count))
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+      if (inside(i))
+        reinterpret_cast<f32x4*>(l.stream_out)[threadIdx.x + i * kNormedThreads] = held[i];
+  const float inverse = inverse_of(l.epsilon);
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    if (!inside(i)) continue;
+    const uint32_t piece = threadIdx.x + i * kNormedThreads;
+    const f32x4 unit = held[i] * inverse;
+    const f32x4 here = unit * weight[i];
+    f32x4 value = here;
+    if (blended)   // (rounded as the compiler does it there)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        value[c] = fmaf(fmaf(-unit[c], weight[i][c], before[i][c]), share[i][c], here[c]);
+    if constexpr (F32) {
+      i32x4 split[3];
+      Input<true>::split({value, f32x4{}}, split);
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        *reinterpret_cast<i32x2*>(values + p * kRow + piece * 4u) =
+            i32x2{split[p][0], split[p][1]};
+    } else {
+      put4<uint16_t>(values, piece * 4u, value);
+    }
+    if (first && blended) reinterpret_cast<f32x4*>(shift.last)[piece] = here;
+  }
+  for (uint32_t c = l.width + threadIdx.x; c < columns; c += kNormedThreads)
+#pragma unroll
+    for (int p = 0; p < Input<F32>::kParts; ++p) values[p * kRow + c] = 0;
+  __syncthreads();
+}
+
+// What a wave reads of a unit of TILES weight tiles: its eighth of the columns.
+struct NormedPart {
+  const i32x4* weights;
+  uint32_t chunks, begin, end;   // of 32 columns: of the tile, of the wave
+};
+
+// A lane's 16 bytes of a chunk of a unit's tile `tile` of `tiles`.  Past the wave's part
+// nothing is fetched, but there is a load all the same: the compiler knows how many are on
+// their way.
+__device__ __forceinline__ i32x4 load_weights(const NormedPart& part, uint32_t tiles,
+                                              uint32_t unit, uint32_t chunk,
+                                              uint32_t tile) {
+  const uint32_t tile_bytes = part.chunks * kWave * 16u;
+  const auto range = memory_range(part.weights + size_t{unit} * tiles * part.chunks * kWave,
+                                  size_t{tiles} * tile_bytes);
+  const uint32_t from =
+      chunk < part.end ? chunk * (kWave * 16u) + tile * tile_bytes : 0x80000000u;
+  return __builtin_bit_cast(
+      i32x4, __builtin_amdgcn_raw_buffer_load_b128(range, threadIdx.x % kWave * 16u + from, 0,
+                                                   2 /* non-temporal */));
+}
+
+// The units unit, unit + step, ... of a segment.  The first one's loads are in flight when
+// this begins; afterwards every register is loaded again as soon as it has been used.
+template <bool F32, int TILES, int PIECES>
+__device__ __forceinline__ void normed_units(const qllm_linear_segment& s,
+                                             const NormedPart& part, uint32_t unit,
+                                             uint32_t step, const uint16_t* values,
+                                             f32x4* scratch, i32x4 (&w)[8 * PIECES]) {
+  constexpr uint32_t kRow = PIECES * kNormedWidth;
+  constexpr uint32_t kUnroll = 8u * PIECES / TILES;
+  constexpr int kParts = Input<F32>::kParts;
+  const uint32_t wave = threadIdx.x / kWave;
+  const uint32_t lane = threadIdx.x % kWave;
+  const uint32_t units = s.rows / (16u * TILES);
+  const uint16_t* input = values + 8u * (lane / 16u);
+  const auto operand = [&](int p, uint32_t chunk) __attribute__((always_inline)) {
+    return *reinterpret_cast<const i32x4*>(input + p * kRow + chunk * 32u);
+  };
+  for (; unit < units; unit += step) {
+    const bool more = unit + step < units;
+    f32x4 sum[TILES][1] = {};
+    uint32_t chunk = part.begin;
+    const auto multiply = [&](auto again, uint32_t next, uint32_t from)
+                              __attribute__((always_inline)) {
+#pragma unroll
+      for (uint32_t u = 0; u < kUnroll; ++u) {
+        if (chunk + u < part.end) {
+#pragma unroll
+          for (int p = 0; p < kParts; ++p)
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+              sum[t][0] = mfma_bf16(w[u * TILES + t], operand(p, chunk + u), sum[t][0]);
+        }
+        if constexpr (again())
+#pragma unroll
+          for (int t = 0; t < TILES; ++t)
+            w[u * TILES + t] = load_weights(part, TILES, next, from + u, t);
+      }
+    };
+    for (; chunk + kUnroll < part.end; chunk += kUnroll)
+      multiply(std::true_type{}, unit, chunk + kUnroll);
+    if (more)
+      multiply(std::true_type{}, unit + step, part.begin);
+    else
+      multiply(std::false_type{}, 0u, 0u);
+    if constexpr (F32)
+      if (__any(any_nan(sum))) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) sum[t][0] = f32x4{};
+        for (uint32_t chunk = part.begin; chunk < part.end; ++chunk)
+#pragma unroll
+          for (int t = 0; t < TILES; ++t) {
+            const i32x4 tile = load_weights(part, TILES, unit, chunk, t);
+#pragma unroll
+            for (int p = 0; p < kParts; ++p)
+              sum[t][0] = mfma_bf16(p ? finite_weights(tile) : tile, operand(p, chunk),
+                                    sum[t][0]);
+          }
+      }
+#pragma unroll
+    for (int t = 0; t < TILES; ++t)
+      scratch[(t * kSmallWaves + wave) * kWave + lane] = sum[t][0];
+    __syncthreads();
+    if (wave == 0u) {
+      f32x4 total[TILES];
+#pragma unroll
+      for (int t = 0; t < TILES; ++t) {
+        total[t] = scratch[t * kSmallWaves * kWave + lane];
+#pragma unroll
+        for (uint32_t other = 1; other < kSmallWaves; ++other)
+          total[t] += scratch[(t * kSmallWaves + other) * kWave + lane];
+      }
+      const uint32_t n = unit * 16u + 4u * (lane / 16u);
+      if (lane % 16u == 0u) {
+        if constexpr (TILES == 2)
+          store_gated<typename Input<F32>::Element>(s, 0u, n, total[0], total[1]);
+        else
+          store_four(s, static_cast<float*>(s.output), 0u, n, total[0], false);
+      }
+    }
+    if (more) __syncthreads();
+  }
+}
+
+template <bool F32, int PIECES>
+__global__ __launch_bounds__(kNormedThreads, PIECES == 1 ? 4 : 2) void linear_normed_kernel(
+    NormedArgs args) {
+  __shared__ f32x4 scratch[2 * kNormedThreads];
+  __shared__ __attribute__((aligned(16))) uint16_t values[Input<F32>::kParts * PIECES *
+                                                           kNormedWidth];
+  __shared__ __attribute__((aligned(16))) float sums[PIECES * kSmallWaves];
+  const uint32_t index = segment_of(args.linear, blockIdx.x);
+  const qllm_linear_segment& s = args.linear.segment[index];
+  const uint32_t first = args.linear.first_unit[index];
+  const uint32_t step = args.linear.first_unit[index + 1u] - first;
+  const uint32_t unit = blockIdx.x - first;
+  const bool gated = s.epilogue == QLLM_LINEAR_GATED;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t chunks = s.columns / 32u;
+  const NormedPart part{static_cast<const i32x4*>(s.weights), chunks,
+                        chunks * wave / kSmallWaves, chunks * (wave + 1u) / kSmallWaves};
+  const uint32_t tiles = __builtin_amdgcn_readfirstlane(gated ? 2u : 1u);
+  i32x4 w[8 * PIECES];
+  normed_row<F32, PIECES>(
+      args.norm, args.source[index], s.columns, blockIdx.x == 0u, values, sums,
+      [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t j = 0; j < 8u * PIECES; ++j)
+          w[j] = gated ? load_weights(part, tiles, unit, part.begin + j / 2u, j % 2u)
+                       : load_weights(part, tiles, unit, part.begin + j, 0u);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+  if (gated)
+    normed_units<F32, 2, PIECES>(s, part, unit, step, values, scratch, w);
+  else
+    normed_units<F32, 1, PIECES>(s, part, unit, step, values, scratch, w);
 }
 
 // ---- tall batches --------------------------------------------------------------
@@ -679,10 +967,6 @@ __global__ void linear_pack_kernel(const uint16_t* source, uint32_t rows, uint32
   }
 }
 
-bool aligned16(const void* pointer) {
-  return (reinterpret_cast<uintptr_t>(pointer) & 15u) == 0u;
-}
-
 uint32_t parts_of(const qllm_linear_segment& s) {
   return s.epilogue == QLLM_LINEAR_PARTIALS ? s.splits : 1u;
 }
@@ -861,6 +1145,62 @@ bool takes_small(const LinearArgs& args, bool f32) {
   return args.batch <= 64u || (far && !f32);
 }
 
+// Which row of the norm every segment reads; false where the launch is not one of
+// linear_normed_kernel: rows it does not hold, and where two launches are faster.  Those are
+// many short tiles, which leave the workgroups too little to read at a time (256 columns,
+// two launches against one: 2000 gated tiles 13.5 and 13.1 us, 3000 16.7 and 18.0, 8000 31.9
+// and 38.4), and heads of a workgroup a CU that are long enough to hide a norm (4096 columns
+// of bf16: 3000 tiles 66.1 and 65.1 us, 4500 94.1 and 94.3, 8000 159.4 and 161.4).
+bool normed_sources(NormedArgs& args) {
+  const qllm_stream_norm_launch& l = args.norm.launch;
+  if (l.rows != 1u || l.gather || l.width > 2u * kNormedWidth ||
+      l.partial_count > kNormedParts || l.partial_stride >= 1u << 24)
+    return false;
+  bool carried = !l.shift;   // the shift's last row is left by workgroup 0
+  uint64_t stored = 0, gated = 0;
+  uint32_t columns = ~0u;
+  for (uint32_t i = 0; i < args.linear.count; ++i) {
+    const qllm_linear_segment& s = args.linear.segment[i];
+    const uint32_t most = l.width <= kNormedWidth ? kNormedWidth : 2u * kNormedWidth;
+    uint32_t source = ~0u;
+    if (l.shift)
+      for (uint32_t b = 0; b < l.shift->count; ++b)
+        if (l.shift->output[b] == s.input) source = 2u + b;
+    for (uint32_t o = l.shift ? 1u : 0u; o < 2u && source == ~0u; ++o)
+      if (l.weight[o] && l.output[o] == s.input) source = o;
+    if (source == ~0u || s.columns > most ||
+        s.columns > l.stride[source == 1u ? 1 : 0] || s.epilogue == QLLM_LINEAR_ADD ||
+        s.epilogue == QLLM_LINEAR_PARTIALS)
+      return false;
+    carried |= i == 0u && source >= 2u;
+    args.source[i] = source;
+    (s.epilogue == QLLM_LINEAR_GATED ? gated : stored) +=
+        s.rows / (s.epilogue == QLLM_LINEAR_GATED ? 32u : 16u);
+    columns = std::min(columns, s.columns);
+  }
+  if (columns < 512u && stored + gated > 2048u) return false;
+  if (l.element == QLLM_ELEMENT_BF16 && l.width > kNormedWidth && !gated && stored > 4096u)
+    return false;
+  return carried;
+}
+
+// Workgroups of a launch: one a tile as long as `most` fit the chip at once, beyond that as
+// many as fit, dealt to the segments by their tiles.
+void normed_workgroups(LinearArgs& args, uint32_t most) {
+  const auto units = [](const qllm_linear_segment& s) {
+    return s.rows / (s.epilogue == QLLM_LINEAR_GATED ? 32u : 16u);
+  };
+  uint64_t total = 0;
+  for (uint32_t i = 0; i < args.count; ++i) total += units(args.segment[i]);
+  for (uint32_t i = 0; i < args.count; ++i) {
+    const uint64_t own = units(args.segment[i]);
+    const uint64_t groups = total <= most
+                                ? own
+                                : std::max<uint64_t>(own * most / total, 1u);
+    args.first_unit[i + 1] = args.first_unit[i] + static_cast<uint32_t>(groups);
+  }
+}
+
 }  // namespace
 
 extern "C" int32_t qllm_linear_layout(const qllm_linear_segment* segments, uint32_t count,
@@ -910,6 +1250,38 @@ extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32
   if (form == 2u) return launch_tall<false, 4, 8>(args, hip_stream);
   return form ? launch_tall<false, 2, 8>(args, hip_stream)
               : launch_tall<false, 2, 4>(args, hip_stream);
+}
+
+extern "C" int32_t qllm_linear_normed(const qllm_stream_norm_launch* norm,
+                                      const qllm_token_rows* tokens,
+                                      const qllm_linear_segment* segments, uint32_t count,
+                                      void* stream) {
+  NormedArgs args{};
+  bool wide = false;
+  if (const int32_t status = stream_norm_arguments(norm, tokens, args.norm, wide))
+    return status;
+  if (const int32_t status =
+          linear_arguments(segments, count, norm->rows, norm->element, args.linear))
+    return status;
+  if (!wide || !normed_sources(args)) {
+    if (const int32_t status = tokens ? qllm_stream_norm_tokens(norm, tokens, stream)
+                                      : qllm_stream_norm(norm, stream))
+      return status;
+    return qllm_linear_batch(segments, count, norm->rows, norm->element, stream);
+  }
+  // (128 registers a lane up to kNormedWidth values, 256 beyond: two workgroups a CU, or one)
+  normed_workgroups(args.linear, norm->width <= kNormedWidth ? 512u : 256u);
+  const uint32_t grid = args.linear.first_unit[count];
+  const auto hip_stream = as_stream(stream);
+  const bool f32 = norm->element == QLLM_ELEMENT_F32;
+  const auto launch = [&](auto kernel) {
+    kernel<<<grid, kNormedThreads, 0, hip_stream>>>(args);
+  };
+  if (norm->width <= kNormedWidth)
+    f32 ? launch(linear_normed_kernel<true, 1>) : launch(linear_normed_kernel<false, 1>);
+  else
+    f32 ? launch(linear_normed_kernel<true, 2>) : launch(linear_normed_kernel<false, 2>);
+  return launched("linear of a norm");
 }
 
 extern "C" uint32_t qllm_linear_part_rows(uint32_t rows, uint32_t columns, uint32_t batch,

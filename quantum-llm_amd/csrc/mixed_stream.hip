@@ -4,7 +4,7 @@
 // up to two normalised copies written (a parallel layer feeds its mixer and its
 // feed-forward from the same row), or the token-shift blends of a mixer that reads the
 // previous token's normalised input as well.
-#include "mixed_common.hpp"
+#include "mixed_norm.hpp"
 
 namespace qllm {
 namespace {
@@ -12,79 +12,6 @@ namespace {
 constexpr int kHeld = 4;   // most 16-byte pieces of a row a thread keeps in registers
 // Rows up to which a thread per piece asks for all that it needs at first
 constexpr uint32_t kFewRows = 512;
-
-struct NormArgs {
-  qllm_stream_norm_launch launch;
-  qllm_token_shift shift;
-  qllm_token_rows tokens;   // TABLE: the stream's rows are these, not launch.input
-};
-
-__device__ __forceinline__ const uint16_t* table_row(const NormArgs& args, uint32_t row) {
-  const uint32_t token = args.tokens.tokens[row];
-  return token < args.tokens.vocabulary
-             ? static_cast<const uint16_t*>(args.tokens.table) +
-                   size_t{token} * args.launch.width
-             : nullptr;
-}
-
-__device__ __forceinline__ f32x4 table_value4(const NormArgs& args, uint32_t row,
-                                              uint32_t piece) {
-  const uint16_t* values = table_row(args, row);
-  if (!values) return f32x4{};
-  const i32x2 bits = reinterpret_cast<const i32x2*>(values)[piece];
-  f32x4 value;
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-    value[c] = bf16_bits_to_f32(static_cast<uint32_t>(bits[c / 2]) >> (16 * (c % 2)) & 0xffffu) *
-               args.tokens.scale;
-  return value;
-}
-
-// The stream with the partial sums added; with a branch norm the sums alone.
-__device__ __forceinline__ f32x4 stream_value4(const qllm_stream_norm_launch& l,
-                                               uint32_t row, uint32_t piece) {
-  f32x4 value = l.branch_weight
-                    ? f32x4{}
-                    : reinterpret_cast<const f32x4*>(l.input + size_t{row} * l.width)[piece];
-  // eight loads in flight at a time
-  for (uint32_t first = 0; first < l.partial_count; first += 8u) {
-    f32x4 part[8];
-#pragma unroll
-    for (uint32_t i = 0; i < 8u; ++i)
-      part[i] = first + i < l.partial_count
-                    ? reinterpret_cast<const f32x4*>(
-                          l.partials +
-                          (size_t{first + i} * l.rows + row) * l.partial_stride)[piece]
-                    : f32x4{};
-#pragma unroll
-    for (uint32_t i = 0; i < 8u; ++i) value += part[i];
-  }
-  return value;
-}
-
-__device__ __forceinline__ float stream_value(const qllm_stream_norm_launch& l,
-                                              uint32_t row, uint32_t column) {
-  float value = l.branch_weight ? 0.0f : l.input[size_t{row} * l.width + column];
-  for (uint32_t p = 0; p < l.partial_count; ++p)
-    value += l.partials[(size_t{p} * l.rows + row) * l.partial_stride + column];
-  return value;
-}
-
-__device__ __forceinline__ float inverse_rms(float squares, uint32_t width, float epsilon) {
-  return 1.0f / sqrtf(squares / static_cast<float>(width) + epsilon);
-}
-
-template <typename T>
-__device__ __forceinline__ void put4(void* output, size_t index, f32x4 value) {
-  if constexpr (sizeof(T) == 4) {
-    *reinterpret_cast<f32x4*>(static_cast<float*>(output) + index) = value;
-  } else {
-    const uint32_t low = f32_to_bf16_bits(value[0]) | f32_to_bf16_bits(value[1]) << 16;
-    const uint32_t high = f32_to_bf16_bits(value[2]) | f32_to_bf16_bits(value[3]) << 16;
-    *reinterpret_cast<i32x2*>(static_cast<uint16_t*>(output) + index) =
-        i32x2{static_cast<int>(low), static_cast<int>(high)};
-  }
-}
 
 template <typename T>
 __device__ __forceinline__ void pad_row(void* output, uint32_t row, uint32_t width,
@@ -321,10 +248,6 @@ __global__ void embedding_bf16_kernel(const uint16_t* table, uint32_t vocabulary
             : 0.0f;
 }
 
-bool aligned16(const void* pointer) {
-  return (reinterpret_cast<uintptr_t>(pointer) & 15u) == 0u;
-}
-
 }  // namespace
 }  // namespace qllm
 
@@ -358,18 +281,28 @@ void launch_norm(const NormArgs& args, bool wide, hipStream_t stream) {
     stream_norm_wide_kernel<T, kHeld, TABLE><<<l.rows, threads, 0, stream>>>(args);
 }
 
-int32_t norm_rows(const qllm_stream_norm_launch* launch, const qllm_token_rows* tokens,
-                  void* stream) {
-  if (!launch || !launch->input || !launch->rows || !launch->width ||
+}  // namespace
+
+namespace qllm {
+
+int32_t stream_norm_arguments(const qllm_stream_norm_launch* launch,
+                              const qllm_token_rows* tokens, NormArgs& args, bool& wide) {
+  if (tokens && (!launch || !tokens->table || !tokens->tokens || !tokens->vocabulary ||
+                 !launch->stream_out || launch->gather || launch->partial_count))
+    return fail(QLLM_INVALID_ARGUMENT, "invalid stream norm of tokens");
+  qllm_stream_norm_launch own{};
+  if (launch) own = *launch;
+  if (tokens) own.input = own.stream_out;
+  if (!launch || !own.input || !launch->rows || !launch->width ||
       launch->element > QLLM_ELEMENT_F32 ||
       (launch->partial_count &&
-       (tokens || !launch->partials || !launch->stream_out || launch->stream_out == launch->input ||
+       (tokens || !launch->partials || !launch->stream_out || launch->stream_out == own.input ||
         launch->partial_stride < launch->width || launch->gather)) ||
       (launch->branch_weight && (!launch->partial_count || launch->shift)))
     return fail(QLLM_INVALID_ARGUMENT, "invalid stream norm");
-  bool wide = launch->width % 4u == 0u && launch->partial_stride % 4u == 0u &&
-              aligned16(launch->input) && aligned16(launch->stream_out) &&
-              aligned16(launch->partials) && aligned16(launch->branch_weight);
+  wide = launch->width % 4u == 0u && launch->partial_stride % 4u == 0u &&
+         aligned16(own.input) && aligned16(launch->stream_out) &&
+         aligned16(launch->partials) && aligned16(launch->branch_weight);
   for (int i = 0; i < 2; ++i) {
     if (!launch->weight[i]) continue;
     const bool blended = i == 0 && launch->shift;
@@ -378,7 +311,7 @@ int32_t norm_rows(const qllm_stream_norm_launch* launch, const qllm_token_rows* 
     wide = wide && aligned16(launch->weight[i]) && aligned16(launch->output[i]) &&
            launch->stride[i] % 4u == 0u;
   }
-  NormArgs args{*launch, {}, {}};
+  args = {own, {}, {}};
   if (const auto* shift = launch->shift) {
     if (!shift->count || shift->count > 6u || !shift->previous || !shift->last ||
         !launch->step || launch->gather || !launch->weight[0])
@@ -396,6 +329,18 @@ int32_t norm_rows(const qllm_stream_norm_launch* launch, const qllm_token_rows* 
     args.tokens = *tokens;
     wide = wide && (reinterpret_cast<uintptr_t>(tokens->table) & 7u) == 0u;
   }
+  return QLLM_OK;
+}
+
+}  // namespace qllm
+
+namespace {
+
+int32_t norm_rows(const qllm_stream_norm_launch* launch, const qllm_token_rows* tokens,
+                  void* stream) {
+  NormArgs args{};
+  bool wide = false;
+  if (const int32_t status = stream_norm_arguments(launch, tokens, args, wide)) return status;
   const auto hip_stream = as_stream(stream);
   if (launch->element == QLLM_ELEMENT_F32)
     tokens ? launch_norm<float, true>(args, wide, hip_stream)
@@ -414,10 +359,6 @@ extern "C" int32_t qllm_stream_norm(const qllm_stream_norm_launch* launch, void*
 
 extern "C" int32_t qllm_stream_norm_tokens(const qllm_stream_norm_launch* launch,
                                            const qllm_token_rows* tokens, void* stream) {
-  if (!launch || !tokens || !tokens->table || !tokens->tokens || !tokens->vocabulary ||
-      !launch->stream_out || launch->gather || launch->partial_count)
-    return fail(QLLM_INVALID_ARGUMENT, "invalid stream norm of tokens");
-  qllm_stream_norm_launch own = *launch;
-  own.input = own.stream_out;
-  return norm_rows(&own, tokens, stream);
+  if (!tokens) return fail(QLLM_INVALID_ARGUMENT, "invalid stream norm of tokens");
+  return norm_rows(launch, tokens, stream);
 }

@@ -943,16 +943,21 @@ void Mi355MixedProvider::enqueue_embedding(std::uint32_t rows, bool with_norm) {
       hidden_[0].as<float>(), rows, g_.hidden, embedding_scale_, stream_));
 }
 
-void Mi355MixedProvider::enqueue_norm(const qllm_stream_norm_launch& norm) {
+// The norm and the projections that read its rows.
+void Mi355MixedProvider::enqueue_normed(const qllm_stream_norm_launch& norm,
+                                        const qllm_linear_segment* segments,
+                                        std::size_t count) {
   if (!std::exchange(pending_tokens_, false)) {
-    status_check(qllm_stream_norm(&norm, stream_));
+    status_check(qllm_linear_normed(&norm, nullptr, segments,
+                                    static_cast<std::uint32_t>(count), stream_));
     return;
   }
   const qllm_token_rows tokens{embedding_.get(), step_.as<std::uint32_t>() + kStepWords,
                                g_.vocabulary, embedding_scale_};
   qllm_stream_norm_launch first = norm;
   first.stream_out = hidden_[0].as<float>();
-  status_check(qllm_stream_norm_tokens(&first, &tokens, stream_));
+  status_check(qllm_linear_normed(&first, &tokens, segments,
+                                  static_cast<std::uint32_t>(count), stream_));
 }
 
 void Mi355MixedProvider::enqueue_attention(Block& block, std::uint32_t rows,
@@ -1113,7 +1118,7 @@ void Mi355MixedProvider::enqueue_sandwich(Block& block, std::uint32_t rows,
     norm.weight[0] = weight.as<float>();
     norm.output[0] = inputs_.get();
     norm.stride[0] = mixer_stride_;
-    enqueue_norm(norm);
+    return norm;
   };
   const auto project = [&](const Matrix& matrix, std::uint32_t splits,
                            const DeviceBuffer& post_norm) {
@@ -1137,7 +1142,7 @@ void Mi355MixedProvider::enqueue_sandwich(Block& block, std::uint32_t rows,
   s.input = inputs_.get();
   s.input_stride = mixer_stride_;
 
-  normed(block.mixer_norm);
+  auto norm = normed(block.mixer_norm);
   const auto& projection = block.projections.front();
   s.weights = projection.matrix.data.get();
   s.output = projections_.get();
@@ -1146,12 +1151,12 @@ void Mi355MixedProvider::enqueue_sandwich(Block& block, std::uint32_t rows,
   s.output_stride = projection_stride_;
   s.output_columns = projection.matrix.rows;
   s.epilogue = QLLM_LINEAR_STORE;
-  status_check(qllm_linear_batch(&s, 1U, rows, g_.element, stream_));
+  enqueue_normed(norm, &s, 1U);
   enqueue_mixer(block, rows, last_position);
   project(block.output, block.splits, block.mixer_post_norm);
   if (!block.intermediate) return;
 
-  normed(block.ffn_norm);
+  norm = normed(block.ffn_norm);
   s.weights = block.gate_up.data.get();
   s.output = joined_.get();
   s.rows = block.gate_up.rows;
@@ -1160,7 +1165,7 @@ void Mi355MixedProvider::enqueue_sandwich(Block& block, std::uint32_t rows,
   s.output_columns = block.intermediate;
   s.epilogue = QLLM_LINEAR_GATED;
   s.activation = block.activation;
-  status_check(qllm_linear_batch(&s, 1U, rows, g_.element, stream_));
+  enqueue_normed(norm, &s, 1U);
   project(block.down, block.down_splits, block.ffn_post_norm);
 }
 
@@ -1195,7 +1200,6 @@ void Mi355MixedProvider::enqueue_block(Block& block, std::uint32_t rows,
     shift.last = shift_last_.as<float>();
     norm.shift = &shift;
   }
-  enqueue_norm(norm);
 
   std::vector<qllm_linear_segment> segments;
   for (const auto& projection : block.projections) {
@@ -1225,8 +1229,7 @@ void Mi355MixedProvider::enqueue_block(Block& block, std::uint32_t rows,
     s.activation = block.activation;
     segments.push_back(s);
   }
-  status_check(qllm_linear_batch(segments.data(), static_cast<std::uint32_t>(segments.size()),
-                                 rows, g_.element, stream_));
+  enqueue_normed(norm, segments.data(), segments.size());
   enqueue_mixer(block, rows, last_position);
 
   qllm_linear_segment s{};
@@ -1254,7 +1257,7 @@ void Mi355MixedProvider::enqueue_block(Block& block, std::uint32_t rows,
 void Mi355MixedProvider::settle_stream(std::uint32_t rows) {
   if (!pending_partials_) return;
   const auto norm = stream_norm(rows, final_epsilon_);
-  enqueue_norm(norm);
+  status_check(qllm_stream_norm(&norm, stream_));
 }
 
 // Final norm and head on `count` rows: those from `first` on, or with `gather`
@@ -1268,7 +1271,6 @@ void Mi355MixedProvider::enqueue_head(std::uint32_t batch_rows, std::uint32_t fi
   norm.output[0] = head_input_.get();
   norm.stride[0] = mixer_stride_;
   norm.gather = gather ? gather_.as<std::uint32_t>() : nullptr;
-  enqueue_norm(norm);
   qllm_linear_segment s{};
   s.weights = head_.data.get();
   s.input = head_input_.get();
@@ -1279,7 +1281,7 @@ void Mi355MixedProvider::enqueue_head(std::uint32_t batch_rows, std::uint32_t fi
   s.output_stride = round_up(g_.vocabulary, 4U);
   s.output_columns = g_.vocabulary;
   s.epilogue = QLLM_LINEAR_STORE;
-  status_check(qllm_linear_batch(&s, 1U, count, g_.element, stream_));
+  enqueue_normed(norm, &s, 1U);
 }
 
 // Logits of the rows asked for and the token of the last row.  The request has

@@ -151,7 +151,8 @@ class Mi355MixedProvider final : public DecoderProvider {
   void begin_batch(MixedRequestState& state, std::span<const std::uint32_t> tokens,
                    std::uint32_t first_position);
   void enqueue_embedding(std::uint32_t rows, bool with_norm);
-  void enqueue_norm(const qllm_stream_norm_launch& norm);
+  void enqueue_normed(const qllm_stream_norm_launch& norm, const qllm_linear_segment* segments,
+                      std::size_t count);
   void enqueue_block(Block& block, std::uint32_t rows, std::uint32_t last_position);
   void enqueue_sandwich(Block& block, std::uint32_t rows, std::uint32_t last_position);
   void enqueue_mixer(Block& block, std::uint32_t rows, std::uint32_t last_position);

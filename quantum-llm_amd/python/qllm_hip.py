@@ -307,6 +307,7 @@ SIGNATURES = {
     "qllm_embedding_bf16_batch": (c_int32, [c_void_p, c_uint32, c_void_p, c_void_p, c_uint32, c_uint32, c_float, c_void_p]),
     "qllm_stream_norm": (c_int32, [POINTER(StreamNormLaunch), c_void_p]),
     "qllm_stream_norm_tokens": (c_int32, [POINTER(StreamNormLaunch), POINTER(TokenRows), c_void_p]),
+    "qllm_linear_normed": (c_int32, [POINTER(StreamNormLaunch), POINTER(TokenRows), POINTER(LinearSegment), c_uint32, c_void_p]),
     "qllm_windowed_layer_bytes": (c_size_t, [c_uint32, c_uint32, c_uint32, c_uint32, c_uint32]),
     "qllm_windowed_rope_store": (c_int32, [POINTER(WindowedAttention), POINTER(RopeStoreLaunch), c_void_p]),
     "qllm_windowed_attention_workspace_bytes": (c_size_t, [POINTER(WindowedAttention), c_uint32, c_uint32]),

@@ -458,6 +458,80 @@ def test_first_norm_looks_its_rows_up(device, element, width, rows, shifted):
         assert torch.equal(one, two)
 
 
+@pytest.mark.parametrize("element", [F32, BF16])
+@pytest.mark.parametrize("width", [64, 90, 132, 2048, 2052, 4096, 4100])
+@pytest.mark.parametrize("form,partials", [("plain", 0), ("plain", 1), ("plain", 8),
+                                           ("plain", 9), ("branch", 3), ("shift", 5),
+                                           ("tokens", 0), ("tokens shift", 0)])
+def test_projection_takes_its_norm_in(device, element, width, form, partials):
+    """One token's norm and its projections in one launch against the two launches, bit for
+    bit: rows of one and two pieces a thread, of no whole pieces and of too many, a stored
+    and a gated matrix of more tiles than workgroups, one infinite weight."""
+    rng = np.random.default_rng(width + partials)
+    columns, stride = padded(width, 64), padded(width, 64) + 8
+    rows = [9040, 9056] if width <= 2052 else [4208, 64]
+    torch.manual_seed(width)
+    packs = []
+    for r in rows:
+        source = torch.randn(r, width, device=device).bfloat16()
+        source[5, 3] = torch.inf
+        packs.append(torch.empty(qh.call("qllm_linear_packed_bytes", r, columns),
+                                 dtype=torch.uint8, device=device))
+        qh.call("qllm_linear_pack", qh.ptr(source), r, width, qh.ptr(packs[-1]), columns, 0, 1,
+                0, None)
+        torch.cuda.synchronize()
+    table = on(device, mm.bf16(rng.standard_normal((9, width))), torch.bfloat16)
+    ids = on(device, np.array([4], dtype=np.int32), torch.int32)
+    x = on(device, rng.standard_normal((1, width)).astype(np.float32))
+    sums = on(device, rng.standard_normal((max(partials, 1), 1, padded(width, 4)))
+              .astype(np.float32))
+    norms = [on(device, w) for w in rng.standard_normal((3, width)).astype(np.float32)]
+    mus = [on(device, m) for m in rng.uniform(0, 1, (2, width)).astype(np.float32)]
+    carried = on(device, rng.standard_normal(padded(width, 4)).astype(np.float32))
+    step = steps(device, 0, slot=0)
+    shifted, tokens = "shift" in form, "tokens" in form
+
+    def run(together):
+        stream = torch.full((1, width), 7.0, device=device)
+        ins = [torch.full((1, stride), 9.0, dtype=torch_type(element), device=device)
+               for _ in range(4)]
+        last = torch.zeros(padded(width, 4), device=device)
+        shift = qh.TokenShift(2, (ctypes.c_void_p * 6)(*map(qh.ptr, mus)),
+                              (ctypes.c_void_p * 6)(*map(qh.ptr, ins[2:])), qh.ptr(carried),
+                              padded(width, 4), qh.ptr(last))
+        norm = qh.StreamNormLaunch(
+            None if tokens else qh.ptr(x), qh.ptr(stream), qh.ptr(sums), partials,
+            padded(width, 4), (ctypes.c_void_p * 2)(*map(qh.ptr, norms[:2])),
+            (ctypes.c_void_p * 2)(*map(qh.ptr, ins[:2])),
+            (ctypes.c_uint32 * 2)(stride, stride), 1, width, 1e-5, element,
+            ctypes.pointer(shift) if shifted else None, None, qh.ptr(step),
+            qh.ptr(norms[2]) if form == "branch" else None, 0.5, 1e-6)
+        out = torch.zeros((1, padded(rows[0], 4)), device=device)
+        gated = torch.zeros((1, rows[1] // 2), dtype=torch_type(element), device=device)
+        segments = (qh.LinearSegment * 2)(
+            qh.LinearSegment(qh.ptr(packs[0]), qh.ptr(ins[3 if shifted else 0]), qh.ptr(out),
+                             padded(rows[0], 16), columns, stride, padded(rows[0], 4), rows[0],
+                             0, 0, 1),
+            qh.LinearSegment(qh.ptr(packs[1]), qh.ptr(ins[1]), qh.ptr(gated), rows[1], columns,
+                             stride, rows[1] // 2, rows[1] // 2 - 3, 2, 0, 1))
+        row = qh.TokenRows(qh.ptr(table), qh.ptr(ids), 9, 0.75)
+        if together:
+            qh.call("qllm_linear_normed", ctypes.byref(norm),
+                    ctypes.byref(row) if tokens else None, segments, 2, None)
+        else:
+            if tokens:
+                qh.call("qllm_stream_norm_tokens", ctypes.byref(norm), ctypes.byref(row), None)
+            else:
+                qh.call("qllm_stream_norm", ctypes.byref(norm), None)
+            qh.call("qllm_linear_batch", segments, 2, 1, element, None)
+        torch.cuda.synchronize()
+        return stream, last, out, gated
+
+    for one, two in zip(run(True), run(False)):
+        assert torch.equal(one.isnan(), two.isnan())
+        assert torch.equal(one.nan_to_num(), two.nan_to_num())
+
+
 # ---- attention -------------------------------------------------------------------
 
 
