@@ -9,7 +9,7 @@
 //
 //  * up to 64 rows (decode): a workgroup owns one 16-row tile (two for the
 //    gated epilogue), its eight waves split K and add their accumulators
-//    through LDS in a fixed order.  All of a wave's loads are in flight at
+//    through LDS in a fixed order.  Up to eight of a wave's loads are in flight at
 //    once; a small batch costs one matrix instruction per KiB of weights.
 //  * more rows (prompts): four waves side by side along the weight rows, each
 //    with NT x MT accumulator tiles; the activation tile of 64 columns is
@@ -43,7 +43,7 @@ constexpr uint32_t kBandTiles = 8;       // activation tiles per band of the gri
 
 struct LinearArgs {
   qllm_linear_segment segment[kMaximumSegments];
-  uint32_t first_unit[kMaximumSegments + 1];   // workgroups before segment s
+  uint32_t first_unit[kMaximumSegments + 1];   // workgroups before segment s; ~0 past the last
   uint32_t count;
   uint32_t batch;
 };
@@ -52,7 +52,7 @@ __device__ __forceinline__ uint32_t segment_of(const LinearArgs& args, uint32_t 
   uint32_t index = 0;
 #pragma unroll
   for (uint32_t i = 1; i < kMaximumSegments; ++i)   // (one trip to memory for all of them)
-    index += i < args.count && unit >= args.first_unit[i] ? 1u : 0u;
+    index = unit >= args.first_unit[i] ? i : index;
   return index;
 }
 
@@ -170,7 +170,8 @@ __device__ __forceinline__ bool any_nan(const f32x4 (&sum)[N][MT]) {
 template <bool F32, int MT, int TILES, int UNROLL>
 __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_t unit,
                                            uint32_t batch, f32x4* scratch) {
-  const uint32_t wave = threadIdx.x / kWave;
+  const uint32_t wave =
+      MT == 1 && !F32 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : threadIdx.x / kWave;
   const uint32_t lane = threadIdx.x % kWave;
   const uint32_t first_row = blockIdx.y * (16u * MT);
   const uint32_t tiles = s.rows / (16u * TILES);
@@ -236,7 +237,45 @@ __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) multiply(w[u], x[u][mt], mt, std::false_type{});
   }
-  one_by_one(chunk, std::false_type{});
+  if constexpr (F32 || MT > 1) {
+    one_by_one(chunk, std::false_type{});
+  } else {
+    // What is left, its loads all in flight at once.  A wave's part is no whole number of
+    // rounds in most layers (decoding one row, us, chunk by chunk and so: [2048, 7680] in
+    // six parts 8.1 and 7.5, [3072, 1536] 6.2 and 4.1, [32000, 1024] 16.7 and 14.2; with
+    // more registers for it 32-bit inputs would lose a workgroup a CU, 10.1 and 11.0).
+    const auto rest = [&](auto count) __attribute__((always_inline)) {
+      constexpr int N = count();
+      // (one chunk a wave is a matrix of up to 511 columns, which may well lie in the L2)
+      const auto stream = [](const i32x4* from) __attribute__((always_inline)) {
+        return N > 1 ? __builtin_nontemporal_load(from) : *from;
+      };
+      if constexpr (N < UNROLL) {
+        i32x4 w[N][TILES];
+        typename In::Raw x[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+#pragma unroll
+          for (int t = 0; t < TILES; ++t)
+            w[u][t] = stream(weights + (size_t{static_cast<uint32_t>(t)} * chunks + chunk + u) *
+                                           kWave);
+#pragma unroll
+        for (int u = 0; u < N; ++u) x[u] = In::load(input[0] + (chunk + u) * 32u);
+#pragma unroll
+        for (int u = 0; u < N; ++u) multiply(w[u], x[u], 0, std::false_type{});
+      }
+    };
+    switch (end - chunk) {
+      case 1: rest(std::integral_constant<int, 1>{}); break;
+      case 2: rest(std::integral_constant<int, 2>{}); break;
+      case 3: rest(std::integral_constant<int, 3>{}); break;
+      case 4: rest(std::integral_constant<int, 4>{}); break;
+      case 5: rest(std::integral_constant<int, 5>{}); break;
+      case 6: rest(std::integral_constant<int, 6>{}); break;
+      case 7: rest(std::integral_constant<int, 7>{}); break;
+      default: break;
+    }
+  }
   if constexpr (F32)
     if (__any(any_nan(sum))) {
 #pragma unroll
@@ -1116,6 +1155,7 @@ int32_t linear_arguments(const qllm_linear_segment* segments, uint32_t count,
     return fail(QLLM_INVALID_ARGUMENT, "invalid linear batch");
   args.count = count;
   args.batch = batch;
+  std::fill(std::begin(args.first_unit) + 1, std::end(args.first_unit), ~0u);
   for (uint32_t i = 0; i < count; ++i) {
     const qllm_linear_segment& s = segments[i];
     const bool gated = s.epilogue == QLLM_LINEAR_GATED;

@@ -458,6 +458,33 @@ def test_first_norm_looks_its_rows_up(device, element, width, rows, shifted):
         assert torch.equal(one, two)
 
 
+@pytest.mark.parametrize("columns", [64, 192, 320, 768, 1088, 1472, 1856, 2176, 3904])
+@pytest.mark.parametrize("epilogue,splits", [(0, 1), (2, 1), (3, 3)])
+def test_linear_parts_of_no_whole_rounds(device, columns, epilogue, splits):
+    """Waves with zero to fifteen chunks: few rows have the bits that they have among 17,
+    whose chunks are taken one by one, and are the products to bf16's rounding."""
+    rng = np.random.default_rng(columns)
+    matrix = mm.bf16(rng.standard_normal((96, columns)) / np.sqrt(columns))
+    weights = packed(device, [(matrix, 0, 1, 0)], 96, columns)
+    x = on(device, rng.standard_normal((17, columns)), torch.bfloat16)
+    outputs = 48 if epilogue == 2 else 96
+
+    def run(batch):
+        out = torch.full((splits, batch, outputs), 7.0, device=device,
+                         dtype=torch.bfloat16 if epilogue == 2 else torch.float32)
+        segment = qh.LinearSegment(qh.ptr(weights), qh.ptr(x), qh.ptr(out), 96, columns, columns,
+                                   outputs, outputs, epilogue, 0, splits)
+        qh.call("qllm_linear_batch", ctypes.byref(segment), 1, batch, BF16, None)
+        torch.cuda.synchronize()
+        return out
+
+    whole = run(17)
+    for batch in (1, 16):
+        assert torch.equal(run(batch), whole[:, :batch])
+    if epilogue != 2:
+        close(whole.sum(0), x.double().cpu().numpy() @ matrix.astype(np.float64).T, F32)
+
+
 @pytest.mark.parametrize("element", [F32, BF16])
 @pytest.mark.parametrize("width", [64, 90, 132, 2048, 2052, 4096, 4100])
 @pytest.mark.parametrize("form,partials", [("plain", 0), ("plain", 1), ("plain", 8),
