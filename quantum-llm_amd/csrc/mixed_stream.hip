@@ -22,12 +22,12 @@ __device__ __forceinline__ void pad_row(void* output, uint32_t row, uint32_t wid
 
 // Rows whose width is a multiple of 4 and fits HELD pieces per thread.
 //
-// For a decoded token this is one workgroup whose time is the memory round trips it
-// waits for one after the other, 0.7 to 1.5 us each.  So all that it needs - partial
-// sums, norm weights, the previous token's row and the blends - is asked for before
-// the first sum over the row, with HELD = 1 (a thread per 16 bytes).  With the lookup of
-// the first layer's rows in the same launch (TABLE) a token of four layers takes 236 ->
-// 227 us at width 2048, 263 -> 253 in 32 bits.
+// A row by itself is one workgroup whose time is the memory round trips it waits for one
+// after the other, 0.7 to 1.5 us each (4 - 5 us: a decoded token's projections take its
+// norm in where they can, linear_normed_kernel).  So all that it needs - partial sums, norm
+// weights, the previous token's row and the blends - is asked for before the first sum over
+// the row, with HELD = 1 (a thread per 16 bytes).  The lookup of the first layer's rows in
+// the same launch (TABLE) saves the launch before it: 1 to 3000 rows 0.64 of the two.
 // More pieces a thread fetch weights and blends where they use them, and none for
 // pieces that the row does not have: all of it asked for first cost norms of 3000 rows of
 // 5120 (plain / with blends) 38 -> 45 / 80 -> 97 us, of one row 4.0 -> 4.5, and of rows
