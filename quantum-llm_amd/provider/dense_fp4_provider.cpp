@@ -2076,6 +2076,7 @@ er::Status Mi355DenseFp4Provider::run_target_graph(const std::uint32_t* tokens,
     }
     hip_check(hipGraphLaunch(static_cast<hipGraphExec_t>(graphs_[rows]), stream),
               "launch target graph");
+    selector_->replayed();
     last_graph_rows_ = rows;
     return er::Status::success();
   } catch (const std::exception& error) {
@@ -2086,7 +2087,9 @@ er::Status Mi355DenseFp4Provider::run_target_graph(const std::uint32_t* tokens,
 er::Status Mi355DenseFp4Provider::capture_target_graph(
     const std::uint32_t* tokens, std::uint32_t rows,
     std::uint32_t first_position) {
-  return run_target_graph(tokens, rows, first_position);
+  const auto status = run_target_graph(tokens, rows, first_position);
+  selector_->replayed(false);   // whoever replays the graph waits for it
+  return status;
 }
 
 er::Status Mi355DenseFp4Provider::replay_target_graph() {
@@ -2624,6 +2627,7 @@ void Mi355DenseFp4Provider::launch_mtp_graph(std::uint32_t rows, bool chained,
   }
   hip_check(hipGraphLaunch(static_cast<hipGraphExec_t>(slot), stream),
             "launch proposer graph");
+  selector_->replayed();
 }
 
 std::optional<DraftPrediction> Mi355DenseFp4Provider::run_mtp(

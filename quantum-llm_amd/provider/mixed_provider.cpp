@@ -887,7 +887,7 @@ void Mi355MixedProvider::release_pages(const MixedRequestState& state) {
 // ---- execution -----------------------------------------------------------------
 
 // Uploads a batch's words and makes its pages exist.  The pinned words are
-// free: every batch ends with a wait.
+// free: every batch ends with its token, which the device hands over last.
 void Mi355MixedProvider::begin_batch(MixedRequestState& state,
                                      std::span<const std::uint32_t> tokens,
                                      std::uint32_t first_position) {
@@ -1378,6 +1378,7 @@ void Mi355MixedProvider::launch_step_graph() {
   stream_index_ = step_stream_index_;
   hip_check(hipGraphLaunch(static_cast<hipGraphExec_t>(step_graph_), stream),
             "launch step graph");
+  selector_->replayed();
   ++graph_launches_;
 }
 

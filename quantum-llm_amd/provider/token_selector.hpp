@@ -46,6 +46,8 @@ class TokenSelector final {
   // marked there (if it is a token).
   [[nodiscard]] std::uint32_t read_token(const std::uint32_t* device_token,
                                          std::uint8_t* emitted = nullptr);
+  // Whether the pass whose words are read next is a replayed graph.
+  void replayed(bool graph = true) noexcept { replayed_ = graph; }
   // Up to kMostWords words of device memory, after everything enqueued so far: there
   // until the next call.
   static constexpr std::uint32_t kMostWords = 2U * 8U * kMaximumTopK;
@@ -66,7 +68,9 @@ class TokenSelector final {
     std::uint32_t words[kMostWords];
     alignas(64) std::uint32_t sequence;
   };
-  static constexpr std::uint32_t kPassesBetweenWaits = 16U;
+  // hand-overs in a row without a wait for the stream, for which the runtime keeps a
+  // little of every launch
+  static constexpr std::uint32_t kMostUnwaited = 256U;
   void* stream_{};
   std::uint32_t vocabulary_{};
   void* workspace_{};
@@ -75,6 +79,8 @@ class TokenSelector final {
   float* top_logits_{};
   Staging* staging_{};
   std::uint32_t sequence_{};
+  std::uint32_t unwaited_{};
+  bool replayed_{};
   std::uint64_t gpu_calls_{};
   std::uint64_t logit_transfer_bytes_{};
 };
