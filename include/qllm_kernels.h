@@ -1145,11 +1145,19 @@ int32_t qllm_stream_norm_tokens(const qllm_stream_norm_launch* launch,
 
 /* qllm_stream_norm (with `tokens`, not NULL, qllm_stream_norm_tokens) followed by
  * qllm_linear_batch of its rows, whose results it has.  For a single row that is one launch
- * where every segment stores or gates what it reads from the norm's outputs and the row is
- * not too long; the normalised rows themselves are then not written. */
+ * where every segment stores or gates what it reads from the norm's outputs, the row is
+ * not too long, and nothing that is written - outputs, the stream, the shift's last row -
+ * overlaps what is read; the normalised rows themselves are then not written.  (Of the
+ * carried rows, whose slot the device knows, that is looked at for slot 0 and for a last
+ * row that is one of them; outputs have to be apart from the others.) */
 int32_t qllm_linear_normed(const qllm_stream_norm_launch* norm, const qllm_token_rows* tokens,
                            const qllm_linear_segment* segments, uint32_t count,
                            void* stream);
+/* How many launches that is: 1, or 2. */
+int32_t qllm_linear_normed_launches(const qllm_stream_norm_launch* norm,
+                                    const qllm_token_rows* tokens,
+                                    const qllm_linear_segment* segments, uint32_t count,
+                                    uint32_t* launches);
 
 /* ---- windowed attention with mixed heads ---------------------------------- */
 

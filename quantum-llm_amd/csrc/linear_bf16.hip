@@ -1227,6 +1227,74 @@ bool normed_sources(NormedArgs& args) {
   return carried;
 }
 
+// Whether the launch writes nothing that it reads or writes elsewhere: a workgroup takes the
+// norm whenever it starts, when others may have stored their outputs and the first one the
+// stream and the carried row.  Two launches read all of it before, and leave the
+// normalised rows in memory.
+bool normed_apart(const NormedArgs& args) {
+  struct Range {
+    uintptr_t first, end;
+  };
+  const auto range = [](const void* first, uint64_t bytes) {
+    const auto at = reinterpret_cast<uintptr_t>(first);
+    return Range{at, first ? at + bytes : at};
+  };
+  const auto meet = [](Range a, Range b) {
+    return a.first < b.end && b.first < a.end && a.first < a.end && b.first < b.end;
+  };
+  const qllm_stream_norm_launch& l = args.norm.launch;
+  const qllm_token_shift& shift = args.norm.shift;
+  const qllm_token_rows& tokens = args.norm.tokens;
+  const uint64_t element = l.element == QLLM_ELEMENT_F32 ? 4u : 2u;
+  const uint64_t row = uint64_t{l.width} * 4u;
+  const bool leaves_stream = tokens.table || l.partial_count;
+  const Range stream = range(leaves_stream ? l.stream_out : nullptr, row);
+  const Range last = range(l.shift ? shift.last : nullptr, row);
+  if (meet(stream, last)) return false;
+  const auto output = [&](const qllm_linear_segment& s) {
+    return range(s.output, s.output_columns *
+                               (s.epilogue == QLLM_LINEAR_GATED ? element : uint64_t{4u}));
+  };
+  const auto written = [&](Range with) {
+    bool any = meet(stream, with) || meet(last, with);
+    for (uint32_t i = 0; i < args.linear.count; ++i)
+      any |= meet(output(args.linear.segment[i]), with);
+    return any;
+  };
+  for (uint32_t i = 0; i < args.linear.count; ++i) {
+    const qllm_linear_segment& s = args.linear.segment[i];
+    if (meet(output(s), stream) || meet(output(s), last) ||
+        written(range(s.weights, uint64_t{s.rows} * s.columns * 2u)))
+      return false;
+  }
+  for (int i = 0; i < 2; ++i)
+    if (l.weight[i] &&
+        (written(range(l.weight[i], row)) || written(range(l.output[i], l.stride[i] * element))))
+      return false;
+  if (l.partial_count &&
+      (written(range(l.partials, (uint64_t{l.partial_count} - 1u) * l.partial_stride * 4u + row)) ||
+       written(range(l.branch_weight, row))))
+    return false;
+  if (tokens.table) {
+    if (written(range(tokens.table, uint64_t{tokens.vocabulary} * l.width * 2u)) ||
+        written(range(tokens.tokens, 4u)))
+      return false;
+  } else if (written(range(l.input, row))) {
+    return false;
+  }
+  if (!l.shift) return true;
+  for (uint32_t b = 0; b < shift.count; ++b)
+    if (written(range(shift.mu[b], row)) || written(range(shift.output[b], l.stride[0] * element)))
+      return false;
+  // (which slot's row is read is known on the device alone: any row may be `last`)
+  const uint64_t slot = shift.slot_stride * 4u;
+  const uint64_t into = last.first - reinterpret_cast<uintptr_t>(shift.previous);
+  if (last.first >= reinterpret_cast<uintptr_t>(shift.previous) && slot && into % slot == 0u)
+    return false;
+  return !written(range(shift.previous, row)) &&
+         !written(range(l.step, (kStepSlot + 1) * sizeof(uint32_t)));
+}
+
 // Workgroups of a launch: one a tile as long as `most` fit the chip at once, beyond that as
 // many as fit, dealt to the segments by their tiles.
 void normed_workgroups(LinearArgs& args, uint32_t most) {
@@ -1242,6 +1310,20 @@ void normed_workgroups(LinearArgs& args, uint32_t most) {
                                 : std::max<uint64_t>(own * most / total, 1u);
     args.first_unit[i + 1] = args.first_unit[i] + static_cast<uint32_t>(groups);
   }
+}
+
+// The arguments of qllm_linear_normed, checked and collected; `together`: one launch.
+int32_t normed_arguments(const qllm_stream_norm_launch* norm, const qllm_token_rows* tokens,
+                         const qllm_linear_segment* segments, uint32_t count, NormedArgs& args,
+                         bool& together) {
+  bool wide = false;
+  if (const int32_t status = stream_norm_arguments(norm, tokens, args.norm, wide))
+    return status;
+  if (const int32_t status =
+          linear_arguments(segments, count, norm->rows, norm->element, args.linear))
+    return status;
+  together = wide && normed_sources(args) && normed_apart(args);
+  return QLLM_OK;
 }
 
 }  // namespace
@@ -1295,18 +1377,28 @@ extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32
               : launch_tall<false, 2, 4>(args, hip_stream);
 }
 
+extern "C" int32_t qllm_linear_normed_launches(const qllm_stream_norm_launch* norm,
+                                               const qllm_token_rows* tokens,
+                                               const qllm_linear_segment* segments,
+                                               uint32_t count, uint32_t* launches) {
+  NormedArgs args{};
+  bool together = false;
+  if (!launches) return fail(QLLM_INVALID_ARGUMENT, "invalid linear of a norm");
+  if (const int32_t status = normed_arguments(norm, tokens, segments, count, args, together))
+    return status;
+  *launches = together ? 1u : 2u;
+  return QLLM_OK;
+}
+
 extern "C" int32_t qllm_linear_normed(const qllm_stream_norm_launch* norm,
                                       const qllm_token_rows* tokens,
                                       const qllm_linear_segment* segments, uint32_t count,
                                       void* stream) {
   NormedArgs args{};
-  bool wide = false;
-  if (const int32_t status = stream_norm_arguments(norm, tokens, args.norm, wide))
+  bool together = false;
+  if (const int32_t status = normed_arguments(norm, tokens, segments, count, args, together))
     return status;
-  if (const int32_t status =
-          linear_arguments(segments, count, norm->rows, norm->element, args.linear))
-    return status;
-  if (!wide || !normed_sources(args)) {
+  if (!together) {
     if (const int32_t status = tokens ? qllm_stream_norm_tokens(norm, tokens, stream)
                                       : qllm_stream_norm(norm, stream))
       return status;

@@ -308,6 +308,7 @@ SIGNATURES = {
     "qllm_stream_norm": (c_int32, [POINTER(StreamNormLaunch), c_void_p]),
     "qllm_stream_norm_tokens": (c_int32, [POINTER(StreamNormLaunch), POINTER(TokenRows), c_void_p]),
     "qllm_linear_normed": (c_int32, [POINTER(StreamNormLaunch), POINTER(TokenRows), POINTER(LinearSegment), c_uint32, c_void_p]),
+    "qllm_linear_normed_launches": (c_int32, [POINTER(StreamNormLaunch), POINTER(TokenRows), POINTER(LinearSegment), c_uint32, POINTER(c_uint32)]),
     "qllm_windowed_layer_bytes": (c_size_t, [c_uint32, c_uint32, c_uint32, c_uint32, c_uint32]),
     "qllm_windowed_rope_store": (c_int32, [POINTER(WindowedAttention), POINTER(RopeStoreLaunch), c_void_p]),
     "qllm_windowed_attention_workspace_bytes": (c_size_t, [POINTER(WindowedAttention), c_uint32, c_uint32]),

@@ -492,8 +492,9 @@ def test_linear_parts_of_no_whole_rounds(device, columns, epilogue, splits):
                                            ("tokens", 0), ("tokens shift", 0)])
 def test_projection_takes_its_norm_in(device, element, width, form, partials):
     """One token's norm and its projections in one launch against the two launches, bit for
-    bit: rows of one and two pieces a thread, of no whole pieces and of too many, a stored
-    and a gated matrix of more tiles than workgroups, one infinite weight."""
+    bit: rows of one and two pieces a thread, of no whole pieces and of too many (which stay
+    two launches), a stored and a gated matrix of more tiles than workgroups, one infinite
+    weight.  One launch leaves the normalised rows as they were."""
     rng = np.random.default_rng(width + partials)
     columns, stride = padded(width, 64), padded(width, 64) + 8
     rows = [9040, 9056] if width <= 2052 else [4208, 64]
@@ -517,6 +518,7 @@ def test_projection_takes_its_norm_in(device, element, width, form, partials):
     carried = on(device, rng.standard_normal(padded(width, 4)).astype(np.float32))
     step = steps(device, 0, slot=0)
     shifted, tokens = "shift" in form, "tokens" in form
+    one_launch = width % 4 == 0 and width <= 4096 and partials <= 8
 
     def run(together):
         stream = torch.full((1, width), 7.0, device=device)
@@ -525,7 +527,7 @@ def test_projection_takes_its_norm_in(device, element, width, form, partials):
         last = torch.zeros(padded(width, 4), device=device)
         shift = qh.TokenShift(2, (ctypes.c_void_p * 6)(*map(qh.ptr, mus)),
                               (ctypes.c_void_p * 6)(*map(qh.ptr, ins[2:])), qh.ptr(carried),
-                              padded(width, 4), qh.ptr(last))
+                              1 << 40, qh.ptr(last))
         norm = qh.StreamNormLaunch(
             None if tokens else qh.ptr(x), qh.ptr(stream), qh.ptr(sums), partials,
             padded(width, 4), (ctypes.c_void_p * 2)(*map(qh.ptr, norms[:2])),
@@ -543,8 +545,11 @@ def test_projection_takes_its_norm_in(device, element, width, form, partials):
                              stride, rows[1] // 2, rows[1] // 2 - 3, 2, 0, 1))
         row = qh.TokenRows(qh.ptr(table), qh.ptr(ids), 9, 0.75)
         if together:
-            qh.call("qllm_linear_normed", ctypes.byref(norm),
-                    ctypes.byref(row) if tokens else None, segments, 2, None)
+            arguments = ctypes.byref(norm), ctypes.byref(row) if tokens else None, segments, 2
+            launches = ctypes.c_uint32()
+            qh.call("qllm_linear_normed_launches", *arguments, ctypes.byref(launches))
+            assert launches.value == (1 if one_launch else 2)
+            qh.call("qllm_linear_normed", *arguments, None)
         else:
             if tokens:
                 qh.call("qllm_stream_norm_tokens", ctypes.byref(norm), ctypes.byref(row), None)
@@ -552,11 +557,65 @@ def test_projection_takes_its_norm_in(device, element, width, form, partials):
                 qh.call("qllm_stream_norm", ctypes.byref(norm), None)
             qh.call("qllm_linear_batch", segments, 2, 1, element, None)
         torch.cuda.synchronize()
+        assert all(bool((rows == 9.0).all()) for rows in ins) == (together and one_launch)
         return stream, last, out, gated
 
     for one, two in zip(run(True), run(False)):
         assert torch.equal(one.isnan(), two.isnan())
         assert torch.equal(one.nan_to_num(), two.nan_to_num())
+
+
+@pytest.mark.parametrize("element", [F32, BF16])
+@pytest.mark.parametrize("over", ["partials", "input", "branch", "carried", "stream"])
+def test_projections_that_write_over_what_the_norm_reads(device, element, over):
+    """The results of the two launches also where one launch would still read what its
+    workgroups write: sums, stream, branch weights, and a carried row that is the next."""
+    rng = np.random.default_rng(3)
+    width, rows = 512, 9040
+    weights = on(device, rng.standard_normal((rows, width)) / 16, torch.bfloat16)
+    pack = torch.empty(qh.call("qllm_linear_packed_bytes", rows, width), dtype=torch.uint8,
+                       device=device)
+    qh.call("qllm_linear_pack", qh.ptr(weights), rows, width, qh.ptr(pack), width, 0, 1, 0, None)
+    norms = [on(device, w) for w in rng.standard_normal((2, width)).astype(np.float32)]
+    mu = on(device, rng.uniform(0, 1, width).astype(np.float32))
+    step = steps(device, 0, slot=0)
+    torch.manual_seed(7)
+    values = {name: torch.randn(size, device=device) for name, size in (
+        ("input", rows), ("partials", rows), ("branch", rows), ("carried", width),
+        ("stream", rows))}
+
+    def run(together):
+        held = {name: value.clone() for name, value in values.items()}
+        held["out"] = torch.zeros(rows, device=device)
+        ins = [torch.zeros(width, dtype=torch_type(element), device=device) for _ in range(2)]
+        last = held["carried"] if over == "carried" else torch.zeros(width, device=device)
+        shift = qh.TokenShift(1, (ctypes.c_void_p * 6)(qh.ptr(mu)),
+                              (ctypes.c_void_p * 6)(qh.ptr(ins[1])), qh.ptr(held["carried"]),
+                              width, qh.ptr(last))
+        norm = qh.StreamNormLaunch(
+            qh.ptr(held["input"]), qh.ptr(held["stream"]), qh.ptr(held["partials"]), 3, width,
+            (ctypes.c_void_p * 2)(qh.ptr(norms[0])), (ctypes.c_void_p * 2)(qh.ptr(ins[0])),
+            (ctypes.c_uint32 * 2)(width, width), 1, width, 1e-5, element,
+            ctypes.pointer(shift) if over == "carried" else None, None, qh.ptr(step),
+            qh.ptr(held["branch"]) if over == "branch" else None, 0.5, 1e-6)
+        output = held["out" if over == "carried" else over]
+        segment = qh.LinearSegment(qh.ptr(pack), qh.ptr(ins[over == "carried"]), qh.ptr(output),
+                                   rows, width, width, rows, rows, 0, 0, 1)
+        if together:
+            launches = ctypes.c_uint32()
+            qh.call("qllm_linear_normed_launches", ctypes.byref(norm), None,
+                    ctypes.byref(segment), 1, ctypes.byref(launches))
+            assert launches.value == 2   # (and nothing is run that would race)
+            qh.call("qllm_linear_normed", ctypes.byref(norm), None, ctypes.byref(segment), 1,
+                    None)
+        else:
+            qh.call("qllm_stream_norm", ctypes.byref(norm), None)
+            qh.call("qllm_linear_batch", ctypes.byref(segment), 1, 1, element, None)
+        torch.cuda.synchronize()
+        return [*held.values(), last]
+
+    for one, two in zip(run(True), run(False)):
+        assert torch.equal(one, two)
 
 
 # ---- attention -------------------------------------------------------------------

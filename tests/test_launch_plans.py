@@ -107,3 +107,118 @@ def test_launches_that_cannot_share_tiles(change):
     launch = attention(**{**sizes, **change})
     assert qh.call("qllm_attention_paged_q4h_shared_splits", launch, 5, 1, 8) == 0
     assert qh.call("qllm_attention_paged_q4h_shares_tiles", launch, 5) == 0
+
+
+# ---- a norm with its projections ------------------------------------------------
+
+MIB = 1 << 20
+
+
+def normed(form, element, changes=(), width=2048, rows=(4096, 4096), partials=0):
+    """How many launches qllm_linear_normed makes of one row whose buffers lie a MiB apart
+    (nothing is read), a stored and a gated matrix."""
+    place = {name: MIB * (16 + i) for i, name in enumerate((
+        "input", "stream", "partials", "weight0", "weight1", "ins0", "ins1", "ins2", "ins3",
+        "mu0", "mu1", "previous", "last", "step", "branch", "table", "ids", "out", "gated",
+        "matrix0"))}
+    place["matrix1"] = 256 * MIB
+    other = dict(changes)
+    for name in list(other):
+        if name in place:
+            value = other.pop(name)
+            place[name] = (place[value[0]] + value[1]) if isinstance(value, tuple) else value
+    columns = -(-width // 64) * 64
+    shifted, tokens = "shift" in form, "tokens" in form
+    pointers = ctypes.c_void_p * 6
+    shift = qh.TokenShift(2, pointers(place["mu0"], place["mu1"]),
+                          pointers(place["ins2"], place["ins3"]), place["previous"],
+                          other.pop("slot_stride", (1 << 14) + 16), place["last"])
+    norm = qh.StreamNormLaunch(
+        None if tokens else place["input"], place["stream"], place["partials"], partials, width,
+        (ctypes.c_void_p * 2)(place["weight0"], place["weight1"]),
+        (ctypes.c_void_p * 2)(place["ins0"], place["ins1"]),
+        (ctypes.c_uint32 * 2)(columns, columns), 1, width, 1e-5, element,
+        ctypes.pointer(shift) if shifted else None, None, place["step"],
+        place["branch"] if form == "branch" else None, 0.5, 1e-6)
+    segments = (qh.LinearSegment * 2)(
+        qh.LinearSegment(place["matrix0"], place["ins3" if shifted else "ins0"], place["out"],
+                         rows[0], columns, columns, rows[0], rows[0], 0, 0, 1),
+        qh.LinearSegment(place["matrix1"], place["ins1"], place["gated"], rows[1], columns,
+                         columns, rows[1] // 2, rows[1] // 2, 2, 0, 1))
+    norm.rows = other.pop("batch", 1)
+    for name, value in other.items():
+        setattr(segments[0], name, value)
+    row = qh.TokenRows(place["table"], place["ids"], 9, 0.75)
+    launches = ctypes.c_uint32()
+    qh.call("qllm_linear_normed_launches", ctypes.byref(norm),
+            ctypes.byref(row) if tokens else None, segments, 2, ctypes.byref(launches))
+    return launches.value
+
+
+FORMS = [("plain", 0), ("plain", 8), ("branch", 3), ("shift", 5), ("tokens", 0),
+         ("tokens shift", 0)]
+
+
+@pytest.mark.parametrize("element", [qh.ELEMENT_BF16, qh.ELEMENT_F32])
+@pytest.mark.parametrize("form,partials", FORMS)
+def test_a_row_and_its_projections_are_one_launch(form, partials, element):
+    for width in (64, 132, 2048, 2052, 4096):
+        rows = (4096, 4096) if width > 448 else (1024, 1024)
+        assert normed(form, element, width=width, rows=rows, partials=partials) == 1
+    assert normed(form, element, width=90, partials=partials) == 2     # no whole pieces
+    assert normed(form, element, width=4100, partials=partials) == 2
+    assert normed(form, element, dict(batch=2), partials=partials) == 2
+    assert normed(form, element, dict(epilogue=1), partials=partials) == 2
+    assert normed(form, element, dict(epilogue=3), partials=partials) == 2
+    assert normed(form, element, dict(weight0=MIB + 4), partials=partials) == 2   # not aligned
+    assert normed("plain", element, partials=9) == 2
+    # many short tiles, and a long stored head of bf16
+    assert normed("plain", element, width=256, rows=(32784, 32)) == 2
+    assert normed("plain", element, width=448, rows=(32784, 32)) == 2
+    assert normed("plain", element, width=512, rows=(32784, 32)) == 1
+
+
+@pytest.mark.parametrize("element", [qh.ELEMENT_BF16, qh.ELEMENT_F32])
+@pytest.mark.parametrize("form,partials", FORMS)
+def test_a_norm_whose_inputs_are_written_over_is_two_launches(form, partials, element):
+    """Projections that write over what the norm or another projection reads, the stream
+    and the shift's last row likewise: the first and the last bytes of every range, and
+    just past both."""
+    width, size = 2048, 2 if element == qh.ELEMENT_BF16 else 4
+    row = 4 * width
+    reads = {"weight0": row, "weight1": row, "ins1": width * size, "matrix1": 4096 * width * 2}
+    if "tokens" in form:
+        reads |= {"table": 9 * width * 2}
+    else:
+        reads |= {"input": row}
+    if partials:
+        reads |= {"partials": partials * row}
+    if form == "branch":
+        reads |= {"branch": row}
+    if "shift" in form:
+        reads |= {"mu0": row, "mu1": row, "previous": row, "last": row}
+    writes = {"out": 4096 * 4, "gated": 2048 * size}
+    if partials or "tokens" in form:
+        writes["stream"] = row
+        reads["stream"] = row
+    if "shift" in form:
+        writes["last"] = row
+
+    def launches(changes):
+        return normed(form, element, dict(changes, slot_stride=1 << 26), partials=partials)
+
+    for writer, written in writes.items():
+        for reader, read in reads.items():
+            if writer == reader or (writer, reader) == ("stream", "input"):
+                continue
+            # (the carried rows: every slot's)
+            for place, apart in ((0, False), (read - 16, False), (16 - written, False),
+                                 (read, True), (-written, True)):
+                assert launches({writer: (reader, place)}) == (1 if apart else 2), (
+                    writer, reader, place)
+
+
+def test_a_last_row_that_is_a_carried_one_is_two_launches():
+    for slot, launches in ((0, 2), (3, 2), (3.5, 1)):
+        assert normed("shift", qh.ELEMENT_F32, {"last": ("previous", int(slot * ((1 << 16) + 64)))},
+                      partials=2) == launches
