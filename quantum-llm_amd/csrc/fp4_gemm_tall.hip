@@ -617,14 +617,16 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_rows_kernel(const Tal
     }
   };
 
-  // About in the order in which the loop waits for them.  (The copies' waits count on a
-  // step's weights at least behind those of the second tile.)
+  // About in the order in which the loop waits for them, and in just this order: the
+  // copies' waits count on all weights behind the first tile, and on a step's at least
+  // behind the second.
   static_assert(kAhead >= kSpan && kAhead <= 4);
   constexpr int kWeightsFirst = kAhead > kSpan ? 0 : kTiles - 2;
 #pragma unroll
   for (int ahead = 0; ahead < std::max(kTiles - 1, kAhead + kWeightsFirst); ++ahead) {
     if constexpr (kCopied) {
       if (ahead + 1 < kTiles) copy_activations(tile_of(ahead), first_chunk + ahead * kSpan);
+      __builtin_amdgcn_sched_barrier(0);
     } else {
       if (ahead < kStages) fetch_activations(ahead, first_chunk + ahead * kSpan);
     }

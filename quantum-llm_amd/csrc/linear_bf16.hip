@@ -801,10 +801,14 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
     position %= kTiles;
     return position == 0 ? tile0 : position == 1 ? tile1 : position == 2 ? tile2 : tile3;
   };
+  // (in this order: the waits count on the tiles one after the other, weights behind them)
 #pragma unroll
-  for (int ahead = 0; ahead + 1 < kTiles; ++ahead)
+  for (int ahead = 0; ahead + 1 < kTiles; ++ahead) {
     copy_input(tile_of(ahead), min(first_step + ahead, last));
+    __builtin_amdgcn_sched_barrier(0);
+  }
   fetch_weights(0u, min(first_step, last));
+  __builtin_amdgcn_sched_barrier(0);
   wait_for_loads<(kTiles - 2u) * kLoads + 2u * NT>();
 
   const auto step_at = [&]<int P>(std::integral_constant<int, P>, uint32_t step) {
