@@ -92,6 +92,13 @@ __device__ __forceinline__ void copy16_to_lds(__amdgpu_buffer_rsrc_t source, uin
       source, (__attribute__((address_space(3))) void*)lds, 16, offset, scalar_offset, 0, 0);
 }
 
+// The same from an address of every lane's own, for what 32-bit offsets do not reach.
+__device__ __forceinline__ void copy16_to_lds(const void* source, void* lds) {
+  __builtin_amdgcn_global_load_lds(
+      (const __attribute__((address_space(1))) void*)source,
+      (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+
 // At most COUNT of this wave's loads and copies are still on their way.
 template <uint32_t COUNT>
 __device__ __forceinline__ void wait_for_loads() {

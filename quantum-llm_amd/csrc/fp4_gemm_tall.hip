@@ -409,7 +409,10 @@ constexpr uint32_t kPastTheEnd = 0x80000000u;   // an offset that fetches nothin
 // stand between so that fewer rows of a batch's last workgroups are padding; a weight's
 // conversion, three vector instructions a pair of binary16 scaled ones, serves that many
 // more rows.
-template <int SCHEME, int MT, int T, bool SWIGLU>
+//
+// FAR: matrices of 2^24 columns and more, whose activation rows and weight tiles lie past
+// 32-bit offsets: 64-bit addresses of every lane's own and a range a chunk.
+template <int SCHEME, int MT, int T, bool SWIGLU, bool FAR = false>
 __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_rows_kernel(const TallArgs args) {
   using Op = Operand<SCHEME>;
   using Vector = typename Op::Vector;
@@ -460,16 +463,21 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_rows_kernel(const Tal
   const uint32_t tile_count = (args.rows + kTileRows - 1u) / kTileRows;
   __amdgpu_buffer_rsrc_t code_stream[T], scale_stream[T];
   uint32_t tile_index[T];
+  const auto codes_of = [&](int t) { return SWIGLU && t ? args.up_weights : args.weights; };
+  const auto scales_of = [&](int t) { return SWIGLU && t ? args.up_scales : args.scales; };
+  // `count` chunks of tile t from chunk `at` on, `bytes` each
+  const auto stream_of = [&](const uint8_t* first, int t, uint32_t at, uint32_t count,
+                             uint32_t bytes) __attribute__((always_inline)) {
+    const size_t stream = static_cast<size_t>(min(tile_index[t], tile_count - 1u)) * chunks;
+    return memory_range(first + (stream + at) * bytes, size_t{count} * bytes);
+  };
 #pragma unroll
   for (int t = 0; t < T; ++t) {
     tile_index[t] = weight_tile<T, SWIGLU>(work.n_tile, wave, t);
-    const size_t stream = static_cast<size_t>(min(tile_index[t], tile_count - 1u)) * chunks;
-    code_stream[t] =
-        memory_range((SWIGLU && t ? args.up_weights : args.weights) + stream * kCodes,
-                     size_t{chunks} * kCodes);
-    scale_stream[t] =
-        memory_range((SWIGLU && t ? args.up_scales : args.scales) + stream * kScales,
-                     size_t{chunks} * kScales);
+    if constexpr (!FAR) {
+      code_stream[t] = stream_of(codes_of(t), t, 0u, chunks, kCodes);
+      scale_stream[t] = stream_of(scales_of(t), t, 0u, chunks, kScales);
+    }
   }
   const uint32_t code_offset = lane * 16u;
   const uint32_t scale_offset = F16 ? ((g >> 1) * 16u + n) * 8u : n * 4u;
@@ -502,18 +510,33 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_rows_kernel(const Tal
   const auto source_at = [&](uint32_t p, uint32_t chunk) {
     return source[p] + min(chunk, end_chunk - 1u) * (kChunk * 2u);
   };
+  // (rows past the batch are its last one here)
+  const auto far_source = [&](uint32_t p, uint32_t chunk) {
+    const uint32_t piece = min(p * kWaves + wave, kAllPieces / 64u - 1u) * 64u + lane;
+    const uint32_t row = piece / (8u * kSpan);
+    const size_t at = min(chunk + piece / 8u % kSpan, end_chunk - 1u);
+    return reinterpret_cast<const uint8_t*>(
+               args.activations + static_cast<size_t>(min(first_m + row, args.batch - 1u)) * K) +
+           at * (kChunk * 2u) + (piece ^ row) % 8u * 16u;
+  };
   const auto copy_activations = [&](uint8_t* tile, uint32_t chunk) {
 #pragma unroll
     for (uint32_t p = 0; p < kPieces; ++p)
-      copy16_to_lds(activations, source_at(p, chunk), 0u, tile + target[p]);
+      if constexpr (FAR)
+        copy16_to_lds(far_source(p, chunk), tile + target[p]);
+      else
+        copy16_to_lds(activations, source_at(p, chunk), 0u, tile + target[p]);
   };
   i32x4 staged[kStages][kPieces];
   const auto fetch_activations = [&](int slot, uint32_t chunk) {
 #pragma unroll
     for (uint32_t p = 0; p < kPieces; ++p)
-      staged[slot][p] = __builtin_bit_cast(
-          i32x4,
-          __builtin_amdgcn_raw_buffer_load_b128(activations, source_at(p, chunk), 0, 0));
+      if constexpr (FAR)
+        staged[slot][p] = *reinterpret_cast<const i32x4*>(far_source(p, chunk));
+      else
+        staged[slot][p] = __builtin_bit_cast(
+            i32x4,
+            __builtin_amdgcn_raw_buffer_load_b128(activations, source_at(p, chunk), 0, 0));
   };
   const auto store_activations = [&](int slot, uint8_t* tile) {
 #pragma unroll
@@ -533,16 +556,18 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_rows_kernel(const Tal
     const uint32_t past = chunk < end_chunk ? 0u : kPastTheEnd;
 #pragma unroll
     for (int t = 0; t < T; ++t) {
+      const auto code = FAR ? stream_of(codes_of(t), t, at, 1u, kCodes) : code_stream[t];
+      const auto scale = FAR ? stream_of(scales_of(t), t, at, 1u, kScales) : scale_stream[t];
       codes[slot][t] = __builtin_bit_cast(
-          i32x4, __builtin_amdgcn_raw_buffer_load_b128(code_stream[t], code_offset | past,
-                                                       at * kCodes, 0));
+          i32x4, __builtin_amdgcn_raw_buffer_load_b128(code, code_offset | past,
+                                                       FAR ? 0u : at * kCodes, 0));
       if constexpr (F16)
         scales[slot][t] = __builtin_bit_cast(
-            i32x2, __builtin_amdgcn_raw_buffer_load_b64(scale_stream[t], scale_offset | past,
-                                                        at * kScales, 0));
+            i32x2, __builtin_amdgcn_raw_buffer_load_b64(scale, scale_offset | past,
+                                                        FAR ? 0u : at * kScales, 0));
       else
         scales[slot][t][0] = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(
-            scale_stream[t], scale_offset | past, at * kScales, 0));
+            scale, scale_offset | past, FAR ? 0u : at * kScales, 0));
     }
   };
 
@@ -748,7 +773,7 @@ __global__ __launch_bounds__(256) void tall_parts_kernel(const TallArgs args) {
 }
 
 // Columns from which on a lane's 32-bit offset does not reach over 128 activation rows:
-// such matrices take workgroups of 16 rows.
+// such matrices take the kernel's FAR form.
 constexpr uint32_t kFarColumns = 1u << 24;
 
 bool tall_matrix_ok(const qllm_fp4_matrix* m) {
@@ -756,7 +781,7 @@ bool tall_matrix_ok(const qllm_fp4_matrix* m) {
          m->padded_columns >= m->columns && m->padded_columns % kChunk == 0u &&
          (m->scale_scheme == QLLM_SCALE_UE8M0_BLOCK32 ||
           m->scale_scheme == QLLM_SCALE_F16_BLOCK16) &&
-         m->padded_columns < 8u * kFarColumns && m->layout == QLLM_LAYOUT_TILED &&
+         m->layout == QLLM_LAYOUT_TILED &&
          (m->tile_rows == 0u || m->tile_rows == kTileRows);
 }
 
@@ -882,11 +907,12 @@ TallPlan plan_tall(uint32_t rows, uint32_t padded_columns, uint32_t batch,
     const uint32_t height = kHeights[index];
     const bool between = height == 5u || height == 7u;
     if (!timed && between) continue;
-    const bool far = padded_columns >= kFarColumns;
-    if (far && height > 1u) break;
+    // (far matrices, which no decoder has: 128 rows pay from 256 workgroups on, a hundred
+    // GB of operands)
+    if (padded_columns >= kFarColumns && (height == 3u || height > 4u)) continue;
     // one or two tiles of rows where they hold the batch, else the higher ones, and
     // none of which a lower one would hold the batch
-    if (height < 3u ? batch > 16u * height && !far : batch <= 32u) continue;
+    if (height < 3u ? batch > 16u * height : batch <= 32u) continue;
     if (index && batch <= 16u * lower) continue;
     lower = height;
     const ChunkCost cost = kChunkCost[scheme][swiglu][index];
@@ -922,52 +948,33 @@ TallPlan plan_tall(uint32_t rows, uint32_t padded_columns, uint32_t batch,
   return best;
 }
 
+template <int SCHEME, int MT, int T, bool FAR>
+void start_rows(const TallArgs& args, bool swiglu, uint32_t grid, hipStream_t stream) {
+  constexpr uint32_t kThreads = kWaves * 64;
+  if (swiglu)
+    fp4_gemm_rows_kernel<SCHEME, MT, 2, true, FAR><<<grid, kThreads, 0, stream>>>(args);
+  else
+    fp4_gemm_rows_kernel<SCHEME, MT, T, false, FAR><<<grid, kThreads, 0, stream>>>(args);
+}
+
 template <int SCHEME>
 void start_tall(const TallArgs& args, uint32_t height, bool swiglu, uint32_t grid,
                 hipStream_t stream) {
-  constexpr uint32_t kThreads = kWaves * 64;
+  if (args.padded_columns >= kFarColumns) {
+    switch (height) {
+      case 1: return start_rows<SCHEME, 1, 1, true>(args, swiglu, grid, stream);
+      case 2: return start_rows<SCHEME, 2, 1, true>(args, swiglu, grid, stream);
+      default: return start_rows<SCHEME, 4, 1, true>(args, swiglu, grid, stream);
+    }
+  }
   switch (height) {
-    case 1:
-      if (swiglu)
-        fp4_gemm_rows_kernel<SCHEME, 1, 2, true><<<grid, kThreads, 0, stream>>>(args);
-      else
-        fp4_gemm_rows_kernel<SCHEME, 1, 1, false><<<grid, kThreads, 0, stream>>>(args);
-      break;
-    case 2:
-      if (swiglu)
-        fp4_gemm_rows_kernel<SCHEME, 2, 2, true><<<grid, kThreads, 0, stream>>>(args);
-      else
-        fp4_gemm_rows_kernel<SCHEME, 2, 1, false><<<grid, kThreads, 0, stream>>>(args);
-      break;
-    case 3:
-      if (swiglu)
-        fp4_gemm_rows_kernel<SCHEME, 3, 2, true><<<grid, kThreads, 0, stream>>>(args);
-      else
-        fp4_gemm_rows_kernel<SCHEME, 3, 1, false><<<grid, kThreads, 0, stream>>>(args);
-      break;
-    case 4:
-      if (swiglu)
-        fp4_gemm_rows_kernel<SCHEME, 4, 2, true><<<grid, kThreads, 0, stream>>>(args);
-      else
-        fp4_gemm_rows_kernel<SCHEME, 4, 1, false><<<grid, kThreads, 0, stream>>>(args);
-      break;
-    case 5:
-      if (swiglu)
-        fp4_gemm_rows_kernel<SCHEME, 5, 2, true><<<grid, kThreads, 0, stream>>>(args);
-      else
-        fp4_gemm_rows_kernel<SCHEME, 5, 2, false><<<grid, kThreads, 0, stream>>>(args);
-      break;
-    case 7:
-      if (swiglu)
-        fp4_gemm_rows_kernel<SCHEME, 7, 2, true><<<grid, kThreads, 0, stream>>>(args);
-      else
-        fp4_gemm_rows_kernel<SCHEME, 7, 2, false><<<grid, kThreads, 0, stream>>>(args);
-      break;
-    default:
-      if (swiglu)
-        fp4_gemm_rows_kernel<SCHEME, 8, 2, true><<<grid, kThreads, 0, stream>>>(args);
-      else
-        fp4_gemm_rows_kernel<SCHEME, 8, 2, false><<<grid, kThreads, 0, stream>>>(args);
+    case 1: return start_rows<SCHEME, 1, 1, false>(args, swiglu, grid, stream);
+    case 2: return start_rows<SCHEME, 2, 1, false>(args, swiglu, grid, stream);
+    case 3: return start_rows<SCHEME, 3, 1, false>(args, swiglu, grid, stream);
+    case 4: return start_rows<SCHEME, 4, 1, false>(args, swiglu, grid, stream);
+    case 5: return start_rows<SCHEME, 5, 2, false>(args, swiglu, grid, stream);
+    case 7: return start_rows<SCHEME, 7, 2, false>(args, swiglu, grid, stream);
+    default: return start_rows<SCHEME, 8, 2, false>(args, swiglu, grid, stream);
   }
 }
 

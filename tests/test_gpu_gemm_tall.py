@@ -93,6 +93,49 @@ def test_tall_gemm_of_far_columns(device, scheme):
     assert ((out.double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("padded,batch", [((1 << 24) + 192, 1), ((1 << 24) + 192, 50),
+                                          ((1 << 24) + 192, 130), (1 << 27, 20)])
+@pytest.mark.parametrize("scheme", [ol.SCALE_UE8M0_BLOCK32, ol.SCALE_F16_BLOCK16])
+def test_tall_gemm_and_swiglu_past_32_bit_offsets(device, scheme, padded, batch):
+    """Workgroups of 16, 64 and 32 rows over matrices whose activation rows, and of
+    2^27 columns weight tiles too, lie further apart than a 32-bit offset; one that ends
+    within a step of several chunks."""
+    rows, columns = 40, [0, 63, 64, padded // 2 + 5, padded - 130, padded - 1]
+    block = 32 if scheme == ol.SCALE_UE8M0_BLOCK32 else 16
+    values = torch.tensor([0, .5, 1, 1.5, 2, 3, 4, 6, -0., -.5, -1, -1.5, -2, -3, -4, -6],
+                          dtype=torch.float64, device=device)
+    act = torch.zeros((batch, padded), dtype=torch.bfloat16, device=device)
+    x = torch.randn((batch, len(columns)), device=device).bfloat16()
+    act[:, columns] = x
+    matrices, sums, bounds = [], [], []
+    for _ in range(1 if padded == 1 << 27 else 2):
+        codes = torch.randint(0, 256, (rows, padded // 2), dtype=torch.uint8, device=device)
+        scales = (torch.full((rows, padded // 32), 127, dtype=torch.uint8, device=device)
+                  if block == 32 else
+                  torch.full((rows, padded // 16), 1.0, dtype=torch.float16, device=device))
+        matrices.append(qh.prepack(qh.fp4_matrix(codes, scales, rows, padded, padded, scheme),
+                                   device))
+        picked = torch.stack([codes[:, c // 2] >> 4 * (c % 2) & 15 for c in columns], dim=1)
+        sums.append(x.double() @ values[picked.long()].T)
+        bounds.append(len(columns) * 2.0 ** -24 *
+                      (x.double().abs() @ values[picked.long()].abs().T))
+        del codes, scales
+    out = torch.zeros((batch, rows), device=device)
+    qh.call("qllm_fp4_gemm_bf16_tall", matrices[0][0], qh.ptr(act), act.numel() * 2, qh.ptr(out),
+            qh.OUT_F32, None, batch, None)
+    torch.cuda.synchronize()
+    assert ((out.double() - sums[0]).abs() <= bounds[0]).all()
+    if len(matrices) == 1:
+        return
+    gated = torch.zeros((batch, rows), dtype=torch.bfloat16, device=device)
+    qh.call("qllm_fp4_swiglu_bf16_tall", matrices[0][0], matrices[1][0], qh.ptr(act),
+            act.numel() * 2, qh.ptr(gated), batch, None)
+    torch.cuda.synchronize()
+    # two roundings to bf16, each by at most 2^-9, and twice that for the exponential
+    want = torch.nn.functional.silu(sums[0]) * sums[1]
+    assert ((gated.double() - want).abs() <= 2.0 ** -7 * want.abs() + 1e-5).all()
+
+
 @pytest.mark.parametrize("scheme", [ol.SCALE_UE8M0_BLOCK32, ol.SCALE_F16_BLOCK16])
 def test_tall_gemm_residual_and_bf16_output(device, scheme):
     rng = np.random.default_rng(5)

@@ -52,6 +52,17 @@ def test_untimed_matrices_keep_the_old_heights(rows, timed, scheme):
     assert new == ({True, False} if timed else {False})
 
 
+@pytest.mark.parametrize("scheme", [UE8M0, F16])
+@pytest.mark.parametrize("padded", [1 << 24, 1 << 27, (1 << 31) + 64])
+def test_matrices_past_32_bit_offsets_are_taken(padded, scheme):
+    for swiglu in (0, 1):
+        for batch, height in ((1, 16), (20, 32), (40, 64), (700, 64)):
+            layout = qh.LaunchLayout()
+            qh.call("qllm_fp4_tall_layout", matrix(40, padded, scheme), swiglu, batch, 0, 0,
+                    ctypes.byref(layout))
+            assert (layout.batch_rows, layout.parts) == (height, 1)
+
+
 @pytest.mark.parametrize("element", [qh.ELEMENT_BF16, qh.ELEMENT_F32])
 @pytest.mark.parametrize("rows,columns", [(2048, 640), (2048, 7680), (4096, 16384), (512, 1024),
                                           (16, 64), (5120, 5120)])
