@@ -173,7 +173,6 @@ __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_
   const uint32_t wave =
       MT == 1 && !F32 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : threadIdx.x / kWave;
   const uint32_t lane = threadIdx.x % kWave;
-  const uint32_t first_row = blockIdx.y * (16u * MT);
   const uint32_t tiles = s.rows / (16u * TILES);
   const uint32_t parts = s.epilogue == QLLM_LINEAR_PARTIALS ? s.splits : 1u;
   const uint32_t part = unit / tiles;
@@ -191,7 +190,7 @@ __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_
   const Element* input[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    const uint32_t row = min(first_row + mt * 16u + lane % 16u, batch - 1u);
+    const uint32_t row = min(mt * 16u + lane % 16u, batch - 1u);
     input[mt] = static_cast<const Element*>(s.input) + size_t{row} * s.input_stride +
                 8u * (lane / 16u);
   }
@@ -304,7 +303,7 @@ __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_
       for (uint32_t other = 1; other < kSmallWaves; ++other)
         total[t] += scratch[((t * MT + mt) * kSmallWaves + other) * kWave + at];
     }
-    const uint32_t m = first_row + mt * 16u + at % 16u;
+    const uint32_t m = mt * 16u + at % 16u;
     const uint32_t n = tile * 16u + 4u * (at / 16u);
     if (m >= batch) continue;
     if constexpr (TILES == 2) {
@@ -734,7 +733,10 @@ __device__ __forceinline__ void store_tall(const LinearArgs& args, const TallPla
 // before anything else (70 rows by [8192, 2048], 128 workgroups, 20.4 -> 18.0 us); where
 // workgroups share a CU they go out between the products (70 rows by [2048, 5632], 480
 // workgroups, 9.7 us, and 10.2 the other way).
-template <int NT, int MT, bool LOADS_FIRST>
+//
+// FAR: input rows 2^24 values apart and more, past a 32-bit offset over 128 of them; every
+// lane has a 64-bit address of its own.
+template <int NT, int MT, bool LOADS_FIRST, bool FAR = false>
 __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
   constexpr uint32_t kRowsM = MT * 16u;
   constexpr uint32_t kPieces = kRowsM * 8u;           // 16-byte pieces of a tile
@@ -786,7 +788,15 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
   const auto copy_input = [&](i32x4* to, uint32_t step) {
 #pragma unroll
     for (uint32_t i = 0; i < kLoads; ++i)
-      copy16_to_lds(input, source[i], step * 128u, to + i * 256u + wave * kWave);
+      if constexpr (FAR) {   // (rows past the batch are its last one here)
+        const uint32_t piece = i * 256u + threadIdx.x;
+        const size_t row = min(first_row + piece / 8u, size_t{args.batch - 1u});
+        copy16_to_lds(static_cast<const uint16_t*>(s.input) + row * s.input_stride +
+                          step * 64u + ((piece ^ piece / 8u) % 8u) * 8u,
+                      to + i * 256u + wave * kWave);
+      } else {
+        copy16_to_lds(input, source[i], step * 128u, to + i * 256u + wave * kWave);
+      }
   };
   const auto fetch_weights = [&](uint32_t slot, uint32_t step) {
 #pragma unroll
@@ -1084,6 +1094,9 @@ uint32_t tall_form(const LinearArgs& args, bool f32) {
 // their loads first, 480: 3 % slower).
 constexpr uint32_t kAlone = 320;
 
+// Values between input rows from which on a lane's 32-bit offset does not reach over 128.
+constexpr uint32_t kFarStride = 1u << 24;
+
 template <bool F32, int NT, int MT>
 int32_t launch_tall(LinearArgs& args, hipStream_t stream) {
   args.first_unit[0] = 0;
@@ -1094,8 +1107,13 @@ int32_t launch_tall(LinearArgs& args, hipStream_t stream) {
                                          args.batch)) *
             parts_of(args.segment[i]);
   const uint32_t grid = args.first_unit[args.count];
+  bool far = false;
+  for (uint32_t i = 0; i < args.count; ++i)
+    far |= args.segment[i].input_stride >= kFarStride;
   if constexpr (F32) {
     linear_tall_f32_kernel<NT, MT><<<grid, 256, 0, stream>>>(args);
+  } else if (far) {
+    linear_tall_kernel<NT, MT, false, true><<<grid, 256, 0, stream>>>(args);
   } else if constexpr (NT == 2 && MT == 4) {
     if (grid <= kAlone)
       linear_tall_kernel<NT, MT, true><<<grid, 256, 0, stream>>>(args);
@@ -1109,8 +1127,8 @@ int32_t launch_tall(LinearArgs& args, hipStream_t stream) {
 
 template <bool F32, int MT>
 void launch_small(const LinearArgs& args, hipStream_t stream) {
-  const dim3 grid(args.first_unit[args.count], (args.batch + 16u * MT - 1u) / (16u * MT));
-  linear_small_kernel<F32, MT><<<grid, kSmallWaves * kWave, 0, stream>>>(args);
+  linear_small_kernel<F32, MT>
+      <<<args.first_unit[args.count], kSmallWaves * kWave, 0, stream>>>(args);
 }
 
 }  // namespace
@@ -1183,14 +1201,6 @@ int32_t linear_arguments(const qllm_linear_segment* segments, uint32_t count,
 
 // batch rows of a workgroup of the form for up to 64
 uint32_t small_rows(uint32_t batch) { return batch <= 16u ? 16u : batch <= 32u ? 32u : 64u; }
-
-// Whether the form for up to 64 rows takes the batch: a longer one of bf16 too, 64 rows at
-// a time, where a lane's 32-bit offset does not reach over 128 rows.
-bool takes_small(const LinearArgs& args, bool f32) {
-  bool far = false;
-  for (uint32_t i = 0; i < args.count; ++i) far |= args.segment[i].input_stride >= 1u << 24;
-  return args.batch <= 64u || (far && !f32);
-}
 
 // Which row of the norm every segment reads; false where the launch is not one of
 // linear_normed_kernel: rows it does not hold, and where two launches are faster.  Those are
@@ -1340,7 +1350,7 @@ extern "C" int32_t qllm_linear_layout(const qllm_linear_segment* segments, uint3
   if (const int32_t status = linear_arguments(segments, count, batch, element, args))
     return status;
   const bool f32 = element == QLLM_ELEMENT_F32;
-  if (takes_small(args, f32)) {
+  if (batch <= 64u) {
     *layout = {small_rows(batch), 16u, parts_of(args.segment[0])};
     return QLLM_OK;
   }
@@ -1357,7 +1367,7 @@ extern "C" int32_t qllm_linear_batch(const qllm_linear_segment* segments, uint32
     return status;
   const auto hip_stream = as_stream(stream);
   const bool f32 = element == QLLM_ELEMENT_F32;
-  if (takes_small(args, f32)) {
+  if (batch <= 64u) {
     for (uint32_t i = 0; i < count; ++i) {
       const qllm_linear_segment& s = segments[i];
       const uint32_t parts = s.epilogue == QLLM_LINEAR_PARTIALS ? s.splits : 1u;

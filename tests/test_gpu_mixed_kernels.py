@@ -329,6 +329,39 @@ def test_linear_of_rows_far_apart(device):
     close(out, x.astype(np.float64) @ w.T.astype(np.float64), F32)
 
 
+@pytest.mark.parametrize("rows,batch,form", [(70, 130, (64, 128)), (40000, 200, (128, 128)),
+                                             (40000, 300, (128, 256))])
+@pytest.mark.parametrize("columns", [64, 448])
+def test_linear_tall_forms_of_rows_far_apart(device, rows, batch, form, columns):
+    """Every tall form over rows 2^24 + 8 values apart, in the workgroups that rows side by
+    side get and with their bits: a batch that ends within a tile, one and seven steps."""
+    stride = (1 << 24) + 8
+    torch.manual_seed(rows + columns)
+    w = torch.randn(rows, columns, device=device).bfloat16()
+    x = torch.randn(batch, columns, device=device).bfloat16()
+    weights = torch.empty(qh.call("qllm_linear_packed_bytes", rows, columns), dtype=torch.uint8,
+                          device=device)
+    qh.call("qllm_linear_pack", qh.ptr(w), rows, columns, qh.ptr(weights), columns, 0, 1, 0, None)
+    d_x = torch.empty((batch, stride), dtype=torch.bfloat16, device=device)
+    d_x[:, :columns] = x
+    outs = []
+    for source, gap in ((x, columns), (d_x, stride)):
+        out = torch.zeros((batch, padded(rows, 4)), device=device)
+        segment = qh.LinearSegment(qh.ptr(weights), qh.ptr(source), qh.ptr(out),
+                                   padded(rows, 16), columns, gap, padded(rows, 4), rows,
+                                   qh.LINEAR_STORE, 0, 0)
+        found = qh.LaunchLayout()
+        qh.call("qllm_linear_layout", ctypes.byref(segment), 1, batch, BF16,
+                ctypes.byref(found))
+        assert (found.batch_rows, found.weight_rows) == form
+        qh.call("qllm_linear_batch", ctypes.byref(segment), 1, batch, BF16, None)
+        torch.cuda.synchronize()
+        outs.append(out[:, :rows])
+    assert torch.equal(*outs)
+    bound = columns * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((outs[0].double() - x.double() @ w.double().T).abs() <= bound).all()
+
+
 # ---- stream ---------------------------------------------------------------------
 
 

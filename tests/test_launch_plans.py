@@ -80,6 +80,19 @@ def test_part_rows_of_linears_cover_what_is_advised(rows, columns, element):
     assert qh.call("qllm_linear_part_rows", rows, columns, 64, element) == 0
 
 
+def test_rows_far_apart_have_the_layout_of_rows_side_by_side():
+    for rows, batch in ((64, 65), (8192, 300), (40000, 200), (40000, 300), (40000, 3000)):
+        found = []
+        for stride in (128, 1 << 24, 1 << 30):
+            segment = qh.LinearSegment(1 << 12, 1 << 13, 1 << 14, rows, 128, stride, rows, rows,
+                                       0, 0, 0)
+            layout = qh.LaunchLayout()
+            qh.call("qllm_linear_layout", ctypes.byref(segment), 1, batch, qh.ELEMENT_BF16,
+                    ctypes.byref(layout))
+            found.append((layout.batch_rows, layout.weight_rows))
+        assert found[0][1] > 64 and found == found[:1] * 3
+
+
 def attention(rows, first, query_heads, kv_heads, splits=1, head_dim=256, split_tokens=0):
     """A prompt's attention that is planned for and never run."""
     return qh.Q4hAttentionLaunch(
