@@ -668,8 +668,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_rows_kernel(const Tal
   // Step P of a round.  A chunk's weights are refilled as soon as they have been
   // multiplied; one past the part's end makes its loads, which fetch nothing, and
   // multiplies nothing, so that every wait can count on the same loads having been made.
-  const auto step_at = [&]<int P>(std::integral_constant<int, P>,
-                                  uint32_t chunk) __attribute__((always_inline)) {
+  const auto step_at = [&]<int P, bool WHOLE>(std::integral_constant<int, P>,
+                                              std::bool_constant<WHOLE>,
+                                              uint32_t chunk) __attribute__((always_inline)) {
     if constexpr (kCopied) {
       // this step's tile is there: what later steps asked for may be on its way
       wait_for_loads<(kTiles - 2) * kStepLoads>();
@@ -683,7 +684,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_rows_kernel(const Tal
 #pragma unroll
     for (int c = 0; c < kSpan; ++c) {
       const int slot = (P * kSpan + c) % kAhead;
-      if (chunk + c < end_chunk) multiply(slot, tile_of(P), c);
+      if (WHOLE || chunk + c < end_chunk) multiply(slot, tile_of(P), c);
       // the loads stay here: moved up they would need registers of their own and
       // copies at the loop's end, which wait for them, moved down they come late
       __builtin_amdgcn_sched_barrier(0);
@@ -692,13 +693,24 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_rows_kernel(const Tal
     }
     if constexpr (!kCopied) store_activations((P + 1) % kStages, tile_of(P + 1));
   };
-  // Rounds of steps, after which every tile, stage and slot has had its turn: of two
-  // stages whole ones (left in between, the compiler waits for more loads than it needs).
+  // Rounds of steps, after which every tile, stage and slot has had its turn.  Of copied
+  // activations whole ones and what is left (of a loop that is left within a round the
+  // compiler takes every step for the one before the next round, which then starts with a
+  // wait for copies and weights just asked for); of two stages whole ones alone, steps past
+  // the end among them (the same, for what passes through registers).
   constexpr int kRound = std::max(kTiles, (kAhead + kSpan - 1) / kSpan);
-  for (uint32_t chunk = first_chunk; chunk < end_chunk; chunk += kRound * kSpan)
+  uint32_t chunk = first_chunk;
+  for (; kCopied ? chunk + kRound * kSpan <= end_chunk : chunk < end_chunk;
+       chunk += kRound * kSpan)
     [&]<int... P>(std::integer_sequence<int, P...>) {
-      (void)((step_at(std::integral_constant<int, P>{}, chunk + P * kSpan),
-              !kCopied || chunk + (P + 1) * kSpan < end_chunk) &&
+      (step_at(std::integral_constant<int, P>{}, std::bool_constant<kCopied>{},
+               chunk + P * kSpan),
+       ...);
+    }(std::make_integer_sequence<int, kRound>{});
+  if (kCopied && chunk < end_chunk)
+    [&]<int... P>(std::integer_sequence<int, P...>) {
+      (void)((step_at(std::integral_constant<int, P>{}, std::false_type{}, chunk + P * kSpan),
+              chunk + (P + 1) * kSpan < end_chunk) &&
              ...);
     }(std::make_integer_sequence<int, kRound>{});
   if constexpr (kCopied) wait_for_loads<0>();   // no copy outlives its workgroup

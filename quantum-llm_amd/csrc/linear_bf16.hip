@@ -860,11 +860,19 @@ __global__ __launch_bounds__(256, 2) void linear_tall_kernel(LinearArgs args) {
     __builtin_amdgcn_sched_barrier(0);
   };
   constexpr int kRound = kTiles % 2 ? 2 * kTiles : kTiles;
-  for (uint32_t step = first_step; step < end_step; step += kRound)
+  // Rounds of steps, after which every tile and slot has had its turn, and what is left.
+  // (Of a loop that is left within a round the compiler takes every step for the one before
+  // the next round, which then starts with a wait for copies and weights just asked for.)
+  uint32_t step = first_step;
+  for (; step + kRound <= end_step; step += kRound)
+    [&]<int... P>(std::integer_sequence<int, P...>) {
+      (step_at(std::integral_constant<int, P>{}, step + P), ...);
+    }(std::make_integer_sequence<int, kRound>{});
+  if (step < end_step)
     [&]<int... P>(std::integer_sequence<int, P...>) {
       (void)((step_at(std::integral_constant<int, P>{}, step + P), step + P + 1u < end_step) &&
              ...);
-    }(std::make_integer_sequence<int, kRound>{});
+    }(std::make_integer_sequence<int, kRound - 1>{});
   wait_for_loads<0>();   // no copy outlives its workgroup
   store_tall<false, NT, MT>(args, place, first_tile, sum);
 }
@@ -1068,11 +1076,23 @@ void each_form(bool f32, const Visit& visit) {
     for (uint32_t i = 0; i < std::size(kTallForms); ++i) visit(kTallForms[i], i);
 }
 
+// Values between input rows from which on a lane's 32-bit offset does not reach over 128.
+constexpr uint32_t kFarStride = 1u << 24;
+
+bool rows_far_apart(const LinearArgs& args) {
+  bool far = false;
+  for (uint32_t i = 0; i < args.count; ++i)
+    far |= args.segment[i].input_stride >= kFarStride;
+  return far;
+}
+
 // The form for a launch whose parts are given.
 uint32_t tall_form(const LinearArgs& args, bool f32) {
+  const bool far = !f32 && rows_far_apart(args);
   uint32_t best = 0;
   double least = 0.0;
   each_form(f32, [&](const TallForm& form, uint32_t index) {
+    if (far && form.nt > 2u) return;   // (no registers left for addresses)
     double units = 0.0;
     double work = 0.0;
     for (uint32_t i = 0; i < args.count; ++i) {
@@ -1094,9 +1114,6 @@ uint32_t tall_form(const LinearArgs& args, bool f32) {
 // their loads first, 480: 3 % slower).
 constexpr uint32_t kAlone = 320;
 
-// Values between input rows from which on a lane's 32-bit offset does not reach over 128.
-constexpr uint32_t kFarStride = 1u << 24;
-
 template <bool F32, int NT, int MT>
 int32_t launch_tall(LinearArgs& args, hipStream_t stream) {
   args.first_unit[0] = 0;
@@ -1107,18 +1124,14 @@ int32_t launch_tall(LinearArgs& args, hipStream_t stream) {
                                          args.batch)) *
             parts_of(args.segment[i]);
   const uint32_t grid = args.first_unit[args.count];
-  bool far = false;
-  for (uint32_t i = 0; i < args.count; ++i)
-    far |= args.segment[i].input_stride >= kFarStride;
   if constexpr (F32) {
     linear_tall_f32_kernel<NT, MT><<<grid, 256, 0, stream>>>(args);
-  } else if (far) {
+  } else if constexpr (NT > 2) {
+    linear_tall_kernel<NT, MT, false><<<grid, 256, 0, stream>>>(args);
+  } else if (rows_far_apart(args)) {
     linear_tall_kernel<NT, MT, false, true><<<grid, 256, 0, stream>>>(args);
-  } else if constexpr (NT == 2 && MT == 4) {
-    if (grid <= kAlone)
-      linear_tall_kernel<NT, MT, true><<<grid, 256, 0, stream>>>(args);
-    else
-      linear_tall_kernel<NT, MT, false><<<grid, 256, 0, stream>>>(args);
+  } else if (MT == 4 && grid <= kAlone) {
+    linear_tall_kernel<NT, MT, MT == 4><<<grid, 256, 0, stream>>>(args);
   } else {
     linear_tall_kernel<NT, MT, false><<<grid, 256, 0, stream>>>(args);
   }

@@ -329,11 +329,10 @@ def test_linear_of_rows_far_apart(device):
     close(out, x.astype(np.float64) @ w.T.astype(np.float64), F32)
 
 
-@pytest.mark.parametrize("rows,batch,form", [(70, 130, (64, 128)), (40000, 200, (128, 128)),
-                                             (40000, 300, (128, 256))])
+@pytest.mark.parametrize("rows,batch,form", [(70, 130, (64, 128)), (40000, 200, (128, 128))])
 @pytest.mark.parametrize("columns", [64, 448])
 def test_linear_tall_forms_of_rows_far_apart(device, rows, batch, form, columns):
-    """Every tall form over rows 2^24 + 8 values apart, in the workgroups that rows side by
+    """The tall forms over rows 2^24 + 8 values apart, in the workgroups that rows side by
     side get and with their bits: a batch that ends within a tile, one and seven steps."""
     stride = (1 << 24) + 8
     torch.manual_seed(rows + columns)

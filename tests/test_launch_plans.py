@@ -80,7 +80,8 @@ def test_part_rows_of_linears_cover_what_is_advised(rows, columns, element):
     assert qh.call("qllm_linear_part_rows", rows, columns, 64, element) == 0
 
 
-def test_rows_far_apart_have_the_layout_of_rows_side_by_side():
+def test_rows_far_apart_have_tall_layouts():
+    """Those of rows side by side, but for the largest."""
     for rows, batch in ((64, 65), (8192, 300), (40000, 200), (40000, 300), (40000, 3000)):
         found = []
         for stride in (128, 1 << 24, 1 << 30):
@@ -90,7 +91,8 @@ def test_rows_far_apart_have_the_layout_of_rows_side_by_side():
             qh.call("qllm_linear_layout", ctypes.byref(segment), 1, batch, qh.ELEMENT_BF16,
                     ctypes.byref(layout))
             found.append((layout.batch_rows, layout.weight_rows))
-        assert found[0][1] > 64 and found == found[:1] * 3
+        near = {(128, 256): (128, 128)}.get(found[0], found[0])
+        assert near in ((64, 128), (128, 128)) and found[1:] == [near] * 2
 
 
 def attention(rows, first, query_heads, kv_heads, splits=1, head_dim=256, split_tokens=0):
