@@ -597,12 +597,19 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_rows_kernel(const Tal
   // Told where to put them only where the products outweigh them: heights of up to 64 rows
   // (binary16 scales: 48) are up to 6 % faster as the compiler orders them.
   constexpr bool kPaced = MT > (F16 ? 3 : 4);
+  // Whether a chunk's last unit converts the next chunk's first: that waits for its weights
+  // before those of four chunks on are asked for.  Low workgroups, which wait for weights
+  // and nothing else, ask first (16 rows, UE8M0 scales: [32000, 2048] 12.3 -> 11.4 us,
+  // [5120, 17408] 20.9 -> 19.1, where one unit at a time had taken 11.4 and 19.3; with 32
+  // rows and binary16 scales it gains nothing).
+  constexpr bool kAcross = MT > (F16 ? 1 : 2);
   constexpr int kProducts = MT * Op::kParts;               // of a unit
   constexpr int kConversion = F16 ? 13 : 6;                // vector instructions of a unit
   const auto multiply = [&](int slot, const uint8_t* tile,
                             int c) __attribute__((always_inline)) {
     const bool last_of_step = c + 1 == kSpan;
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!kAcross) convert(slot, 0, w[0]);
     if (c == 0)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) a[0][mt] = fragment(tile, 0, 0, mt);
@@ -620,7 +627,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_rows_kernel(const Tal
         for (int mt = 0; mt < MT; ++mt) read(mt);
       if (unit + 1 < kUnits)
         convert(slot, unit + 1, w[(unit + 1) % 2]);
-      else
+      else if constexpr (kAcross)
         convert((slot + 1) % kAhead, 0, w[(unit + 1) % 2]);
 #pragma unroll
       for (int part = 0; part < Op::kParts; ++part)
@@ -663,7 +670,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void fp4_gemm_rows_kernel(const Tal
     wait_for_loads<(kTiles - 2) * kPieces + 2u * T * kAhead>();
   else
     store_activations(0, tile0);
-  convert(0, 0, w[0]);
+  if constexpr (kAcross) convert(0, 0, w[0]);
 
   // Step P of a round.  A chunk's weights are refilled as soon as they have been
   // multiplied; one past the part's end makes its loads, which fetch nothing, and
