@@ -729,10 +729,10 @@ __device__ __forceinline__ void store_tall(const LinearArgs& args, const TallPla
 // 67 -> 66, 29.5 -> 29.2.  The tiles are arrays of their own: of one array's parts the
 // compiler would have every read wait for all copies.
 //
-// LOADS_FIRST: a workgroup that has a CU to itself waits for its loads, so they go out
-// before anything else (70 rows by [8192, 2048], 128 workgroups, 20.4 -> 18.0 us); where
-// workgroups share a CU they go out between the products (70 rows by [2048, 5632], 480
-// workgroups, 9.7 us, and 10.2 the other way).
+// LOADS_FIRST: a workgroup that has a CU to itself, or shares it with one other that is as
+// high as wide, waits for its loads, so they go out before anything else (70 rows by [8192,
+// 2048], 128 workgroups, 20.4 -> 18.0 us); where more share a CU they go out between the
+// products (70 rows by [2048, 5632], 480 workgroups, 9.7 us, and 10.2 the other way).
 //
 // FAR: input rows 2^24 values apart and more, past a 32-bit offset over 128 of them; every
 // lane has a 64-bit address of its own.
@@ -1110,9 +1110,11 @@ uint32_t tall_form(const LinearArgs& args, bool f32) {
   return best;
 }
 
-// Workgroups up to which most have a CU to themselves (192 to 320: 1 to 5 % faster with
-// their loads first, 480: 3 % slower).
-constexpr uint32_t kAlone = 320;
+// Workgroups up to which a launch asks for its loads first.  64 x 128: as many as CUs (128 to
+// 256: 5 to 12 % faster so; 286 to 312: 2 to 5 % slower, 500 rows by [8192, 2048], 512, 6 %).
+// 128 x 128: two a CU (448 to 512: 2 to 4 % faster, 65 rows by [5120, 17408] in twelve parts
+// 45.4 -> 43.8 us; 752: 2 to 4 % slower).
+constexpr uint32_t loads_first_up_to(int mt) { return mt == 4 ? 256u : 512u; }
 
 template <bool F32, int NT, int MT>
 int32_t launch_tall(LinearArgs& args, hipStream_t stream) {
@@ -1130,8 +1132,8 @@ int32_t launch_tall(LinearArgs& args, hipStream_t stream) {
     linear_tall_kernel<NT, MT, false><<<grid, 256, 0, stream>>>(args);
   } else if (rows_far_apart(args)) {
     linear_tall_kernel<NT, MT, false, true><<<grid, 256, 0, stream>>>(args);
-  } else if (MT == 4 && grid <= kAlone) {
-    linear_tall_kernel<NT, MT, MT == 4><<<grid, 256, 0, stream>>>(args);
+  } else if (grid <= loads_first_up_to(MT)) {
+    linear_tall_kernel<NT, MT, true><<<grid, 256, 0, stream>>>(args);
   } else {
     linear_tall_kernel<NT, MT, false><<<grid, 256, 0, stream>>>(args);
   }
