@@ -1079,6 +1079,14 @@ void each_form(bool f32, const Visit& visit) {
 // Values between input rows from which on a lane's 32-bit offset does not reach over 128.
 constexpr uint32_t kFarStride = 1u << 24;
 
+// More than two workgroups of 64 x 128 a CU share more of its cache's rate than it has: a
+// step of 64 columns is 24 KB for half the products of 128 x 128 with 32.  Large matrices in
+// many steps show it: 400 rows by [12288, 4096] 71.4 us and with 128 x 128 62.2, 160 rows by
+// [4096, 18432] in eight parts 54.1 and 45.8, by [32000, 2048] 46.5 and 40.8, 26 others 0.87
+// to 1.02.  Smaller ones, or of fewer steps, are up to 1.2 times as fast with 64 x 128 (1500
+// rows by [2816, 1024] 18.2 and 21.9, by [3072, 3072] 44.7 and 47.2).
+constexpr double kMostSmall = 2.0, kManySteps = 24.0, kLargeMatrix = 1 << 24;
+
 bool rows_far_apart(const LinearArgs& args) {
   bool far = false;
   for (uint32_t i = 0; i < args.count; ++i)
@@ -1095,14 +1103,19 @@ uint32_t tall_form(const LinearArgs& args, bool f32) {
     if (far && form.nt > 2u) return;   // (no registers left for addresses)
     double units = 0.0;
     double work = 0.0;
+    double weights = 0.0;
     for (uint32_t i = 0; i < args.count; ++i) {
       const auto& s = args.segment[i];
+      weights += static_cast<double>(s.rows) * s.columns;
       const double own = static_cast<double>(tall_units(form, s.rows, args.batch));
       units += own * parts_of(s);
       work += own * (s.columns / 64u);
     }
     const double time = tall_time(form, units, work / units);
-    if (index == 0u || time < least) {
+    if (!f32 && index == 0u && units > kMostSmall * 256.0 && work / units >= kManySteps &&
+        weights >= kLargeMatrix)
+      return;
+    if (least == 0.0 || time < least) {
       best = index;
       least = time;
     }

@@ -80,6 +80,21 @@ def test_part_rows_of_linears_cover_what_is_advised(rows, columns, element):
     assert qh.call("qllm_linear_part_rows", rows, columns, 64, element) == 0
 
 
+@pytest.mark.parametrize("rows,columns,batch,parts,form", [
+    (12288, 4096, 300, 0, (64, 128)), (12288, 4096, 340, 0, (128, 128)),   # 480, 576 workgroups
+    (10912, 1536, 400, 0, (64, 128)), (10944, 1536, 400, 0, (128, 128)),   # 2^24 weights
+    (16384, 1472, 300, 0, (64, 128)), (16384, 1536, 300, 0, (128, 128)),   # 24 steps
+    (4096, 12288, 160, 8, (128, 128)), (4096, 12224, 160, 8, (64, 128)),   # of a part
+    (2816, 1024, 1500, 0, (64, 128)), (3072, 3072, 1500, 0, (64, 128))])
+def test_small_workgroups_of_large_matrices_are_two_a_cu(rows, columns, batch, parts, form):
+    segment = qh.LinearSegment(1 << 12, 1 << 13, 1 << 14, rows, columns, columns, rows, rows,
+                               qh.LINEAR_PARTIALS if parts else 0, 0, parts)
+    layout = qh.LaunchLayout()
+    qh.call("qllm_linear_layout", ctypes.byref(segment), 1, batch, qh.ELEMENT_BF16,
+            ctypes.byref(layout))
+    assert (layout.batch_rows, layout.weight_rows) == form
+
+
 def test_rows_far_apart_have_tall_layouts():
     """Those of rows side by side, but for the largest."""
     for rows, batch in ((64, 65), (8192, 300), (40000, 200), (40000, 300), (40000, 3000)):
