@@ -402,10 +402,11 @@ constexpr uint32_t kPastTheEnd = 0x80000000u;   // an offset that fetches nothin
 // With 128 rows it is the matrix cores, as far as the card's power lets them: gate and up
 // of [17408, 5120] with binary16 scales over 8192 rows kept them busy 73 % of the time at
 // 2.10 GHz when a unit's weights were converted before its products and a half chunk's
-// activations waited for; with both done in between the products 80 % at 2.00 GHz, 3660 ->
-// 3560 us.  UE8M0 scales, whose activations need no conversion and are copied to the LDS
-// without passing through registers: 63 -> 73 %, 2190 -> 1980 us; 300 rows by [10240, 5120]
-// 47.5 -> 42.1 (binary16: 76 -> 70), 48 rows 17.5 -> 16.7 (21.7 -> 21.2).  80 and 112 rows
+// activations waited for; with both done in between the products 80 % at 2.00 GHz, 3750 ->
+// 3650 us.  UE8M0 scales, whose activations need no conversion and are copied to the LDS
+// without passing through registers: 63 -> 75 %, 2245 -> 2037 us; 300 rows by [10240, 5120]
+// 50.9 -> 42.4 (binary16: 80 -> 71), 64 by [32000, 2048] 21.7 -> 19.5 (28.7 -> 26.8); 48 rows
+// by [10240, 5120] stay within 3 % of 20 (25).  80 and 112 rows
 // stand between so that fewer rows of a batch's last workgroups are padding; a weight's
 // conversion, three vector instructions a pair of binary16 scaled ones, serves that many
 // more rows.
@@ -814,12 +815,14 @@ bool tall_matrix_ok(const qllm_fp4_matrix* m) {
 // once more, at 6.2 TB/s, and take a launch of their own where no norm adds
 // them.  The constants are a fit to 1300 timed launches over weights that come
 // from memory (nine matrices of [2048, 2048] to [17408, 5120], 8 to 3000 rows,
-// heights 1, 2, 4 and 8; 7 % root mean square error; the chosen layout is 1.5 %
-// slower than the best of those timed on average).  What it gives over one workgroup per 128 rows and
-// tile: [5120, 17408] with binary16 scales, 48 rows 400 -> 27 us, 300 rows
-// 404 -> 97, 1000 rows 405 -> 254, 2000 rows 668 -> 498; [10240, 5120] 127 ->
-// 25, 135 -> 73, 211 -> 190, 333 -> 327; gate and up of [17408, 5120] 129 -> 54,
-// 221 -> 195, then unchanged.
+// heights 1, 2, 4 and 8; 7 % root mean square error) of the kernels that converted a unit's
+// weights before its products; the chosen layout was 1.5 % slower than the best of those
+// timed on average, and of the present kernel 4 % (20000 layouts of twelve matrices, 8 to
+// 3001 rows; most with 40 to 80 rows, whose K is cut into more parts than pay).  What the
+// rule gives over one workgroup per 128 rows and tile: [5120, 17408] with binary16 scales,
+// 48 rows 400 -> 27 us, 300 rows 404 -> 97, 1000 rows 405 -> 254, 2000 rows 668 -> 498;
+// [10240, 5120] 127 -> 25, 135 -> 73, 211 -> 190, 333 -> 327; gate and up of [17408, 5120]
+// 129 -> 54, 221 -> 195, then unchanged.
 //
 // Where parts are added by a launch of their own, the tiles past the last full round of
 // the CUs may be cut instead of all of them: `cut` pieces each, the others run whole, as

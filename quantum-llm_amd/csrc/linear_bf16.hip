@@ -248,7 +248,7 @@ __device__ __forceinline__ void small_unit(const qllm_linear_segment& s, uint32_
     // turn of 32 tokens 6.46 and 6.24 ms (with plain loads 6.47).
     const auto rest = [&](auto count) __attribute__((always_inline)) {
       constexpr int N = count();
-      // (one chunk a wave is a matrix of up to 511 columns, which may well lie in the L2)
+      // (of a single chunk, a matrix of few columns in the main, what the L2 may well hold)
       const auto stream = [](const i32x4* from) __attribute__((always_inline)) {
         return N > 1 ? __builtin_nontemporal_load(from) : *from;
       };
@@ -724,15 +724,15 @@ __device__ __forceinline__ void store_tall(const LinearArgs& args, const TallPla
 // over thousands of rows.  Here the tile goes from memory straight to the LDS two or three
 // steps ahead, without a register, an address or a store of the wave's; weights go to
 // registers a step ahead, and a half's activations are read in between the products of
-// the half before.  6000 rows by [28672, 4096] 1208 -> 1120 us (1160 -> 1250 TFLOP/s), by
-// [4096, 18432] 800 -> 718, by [11264, 2048] 271 -> 247; 300 rows of the three 105 -> 99,
-// 67 -> 66, 29.5 -> 29.2.  The tiles are arrays of their own: of one array's parts the
+// the half before.  6000 rows by [28672, 4096] 1285 -> 1153 us (1097 -> 1222 TFLOP/s), by
+// [4096, 18432] 833 -> 721, by [11264, 2048] 294 -> 258; 300 rows of the three 110 -> 104,
+// 69.5 -> 68.2, 29.8 -> 29.2.  The tiles are arrays of their own: of one array's parts the
 // compiler would have every read wait for all copies.
 //
 // LOADS_FIRST: a workgroup that has a CU to itself, or shares it with one other that is as
 // high as wide, waits for its loads, so they go out before anything else (70 rows by [8192,
-// 2048], 128 workgroups, 20.4 -> 18.0 us); where more share a CU they go out between the
-// products (70 rows by [2048, 5632], 480 workgroups, 9.7 us, and 10.2 the other way).
+// 2048], 128 workgroups, 19.8 -> 17.8 us); where more share a CU they go out between the
+// products (500 rows by the same, 512 workgroups, 28.2 us, and 29.8 the other way).
 //
 // FAR: input rows 2^24 values apart and more, past a 32-bit offset over 128 of them; every
 // lane has a 64-bit address of its own.
@@ -1044,10 +1044,14 @@ uint32_t parts_of(const qllm_linear_segment& s) {
 // hide each other's round trips, and parts written and read at 6.5 TB/s.  The
 // constants are a fit to 1150 timed launches over weights from memory (eight
 // matrices of [2048, 2048] to [24576, 4096], 66 to 3000 rows; 8 % root mean square
-// error); the layout it picks is 0.7 % slower than the best of those timed, the
-// rule before it - largest tiles that give two workgroups a CU, K never cut - 68 %:
-// [2048, 7680] 100 rows 62 -> 13 us, 1000 rows 60 -> 40, 3000 rows 117 -> 93; in 32
-// bits 100 rows 141 -> 20, 500 rows 143 -> 47.
+// error) of the kernel that staged its activation tile through registers; 32-bit input
+// still runs it.  What they picked there was 0.7 % slower than the best of those timed, the
+// rule before it - largest tiles that give two workgroups a CU, K never cut - 68 %: [2048,
+// 7680] 100 rows 62 -> 13 us, 1000 rows 60 -> 40, 3000 rows 117 -> 93; in 32 bits 100 rows
+// 141 -> 20, 500 rows 143 -> 47.  With the tiles copied straight to the LDS the form they
+// pick for given parts is 2.1 % slower than the best of the three (368 launches of twenty
+// matrices, 65 to 3000 rows; 1.23 at worst).  A fit of those took 0.9 % and lost up to 1.2
+// in launches that are at their best now.
 struct TallForm {
   uint32_t nt, mt;
   float alone, shared;
