@@ -402,6 +402,14 @@ int32_t qllm_rms_norm_residual_batch(float* hidden, const float* partials,
                                      float epsilon, int32_t zero_centered,
                                      void* stream);
 
+/* One row of it, the last of a prompt: sum = residual + partials[0] + ... of `count`
+ * parts `partial_stride` floats apart (0 parts: a copy of the residual), output_bf16 =
+ * RMSNorm(sum).  `sum` may be `residual`.  elements and partial_stride % 4 == 0. */
+int32_t qllm_rms_norm_row(const float* residual, float* sum, const float* partials,
+                          uint32_t count, size_t partial_stride, const float* weight,
+                          void* output_bf16, uint32_t elements, float epsilon,
+                          int32_t zero_centered, void* stream);
+
 /* The same with the sum written elsewhere: sum[r] = residual[r] + partials[0][r]
  * + ... (from zero when residual is NULL), output_bf16[r] = RMSNorm(sum[r]).
  * The proposer's projections use it: the fusion projection has no residual
@@ -896,6 +904,35 @@ int32_t qllm_fp4_head_argmax(const qllm_fp4_matrix* matrix, const void* input,
                              uint32_t* tokens, void* workspace,
                              size_t workspace_bytes,
                              const qllm_rollout_step* advance, void* stream);
+
+/* Hands the tokens of an arg-max to the host in its last launch: host[m] = *sequence << 32
+ * | token of row m, in pinned host memory that the device writes (hipHostMalloc), one
+ * 8-byte store a row.  A host that sees its sequence number in a row has the row's token.
+ * `sequence` is a device word, so a captured launch is handed a new one every time (NULL:
+ * sequence_value).  With
+ * `emitted`, emitted[*slot * vocabulary + token] = 1 for every token below `vocabulary`
+ * (slot NULL: 0), where *mark is not 0 (mark NULL: always). */
+typedef struct qllm_token_handover {
+  uint64_t* host;              /* [batch] */
+  const uint32_t* sequence;    /* or NULL */
+  uint32_t sequence_value;
+  uint8_t* emitted;            /* or NULL */
+  const uint32_t* mark;        /* device words, or NULL */
+  const uint32_t* slot;
+  uint32_t vocabulary;
+} qllm_token_handover;
+
+/* qllm_fp4_head_argmax and qllm_argmax_batch (below) with such a handover, or NULL. */
+int32_t qllm_fp4_head_argmax_handed(const qllm_fp4_matrix* matrix, const void* input,
+                                    size_t input_bytes, float* logits, uint32_t batch,
+                                    uint32_t* tokens, void* workspace,
+                                    size_t workspace_bytes,
+                                    const qllm_rollout_step* advance,
+                                    const qllm_token_handover* handover, void* stream);
+int32_t qllm_argmax_batch_handed(const float* values, uint32_t count, uint32_t batch,
+                                 uint32_t* output, void* workspace,
+                                 size_t workspace_bytes,
+                                 const qllm_token_handover* handover, void* stream);
 
 /* replaces argmax_batch (transformer_kernels.hpp:1266-1269): ties to the
  * lower index, NaN never wins.  workspace: at least

@@ -171,11 +171,13 @@ struct RolloutAdvance {
 
 // Stage 2 of an arg-max whose stage-1 partials lie in [batch][blocks] arrays
 // (select.hip); with `advance` (batch 1) the same launch also advances the
-// rollout with the winner.
+// rollout with the winner, with `handover` it also hands the winners to the host.
 int32_t launch_argmax_final(const float* partial_values,
                             const uint32_t* partial_indices, uint32_t blocks,
                             uint32_t batch, uint32_t* output,
-                            const RolloutAdvance* advance, hipStream_t stream);
+                            const RolloutAdvance* advance,
+                            const qllm_token_handover* handover, hipStream_t stream);
+bool handover_ok(const qllm_token_handover* handover);
 
 // splitmix64 counter generator shared with the host-side restatement.
 __host__ __device__ inline uint64_t mix64(uint64_t seed, uint64_t index) {

@@ -482,15 +482,14 @@ __global__ __launch_bounds__(1024) void rms_norm_residual_q8_kernel(
 // folded into the norm that follows it.  `sum` may be `residual`.
 __global__ __launch_bounds__(1024) void rms_norm_residual_kernel(
     const float* residual, float* sum, const float* partials,
-    uint32_t partial_count, const float* weight, uint16_t* output_bf16,
-    uint32_t elements, float epsilon, bool zero_centered) {
+    uint32_t partial_count, size_t partial_stride, const float* weight,
+    uint16_t* output_bf16, uint32_t elements, float epsilon, bool zero_centered) {
   __shared__ float scratch[16];
   const size_t row = blockIdx.x;
   rms_norm_row_wide(residual ? residual + row * elements : nullptr, weight, nullptr,
                     output_bf16 + row * elements, elements, elements, epsilon,
                     zero_centered, scratch, partials + row * elements,
-                    partial_count, static_cast<size_t>(gridDim.x) * elements,
-                    sum + row * elements);
+                    partial_count, partial_stride, sum + row * elements);
 }
 
 // Row r of the output is [RMSNorm(first[r]) | RMSNorm(second[r])] in bf16:
@@ -791,9 +790,28 @@ extern "C" int32_t qllm_rms_norm_residual_batch(
   // (measured on rows of 5120: 320 threads, four float4 each, take 6.0 us
   // against 4.75 us with 1024: one CU's few waves wait longer for the row)
   rms_norm_residual_kernel<<<rows, 1024, 0, as_stream(stream)>>>(
-      hidden, hidden, partials, partial_count, weight,
+      hidden, hidden, partials, partial_count, size_t{rows} * elements, weight,
       static_cast<uint16_t*>(output_bf16), elements, epsilon, zero_centered != 0);
   return launched("residual RMSNorm");
+}
+
+extern "C" int32_t qllm_rms_norm_row(const float* residual, float* sum, const float* partials,
+                                     uint32_t count, size_t partial_stride,
+                                     const float* weight, void* output_bf16,
+                                     uint32_t elements, float epsilon,
+                                     int32_t zero_centered, void* stream) {
+  const auto aligned = [](const void* pointer) {
+    return reinterpret_cast<uintptr_t>(pointer) % 16u == 0u;
+  };
+  if (!residual || !sum || !output_bf16 || (count && !partials) || count > 16u ||
+      partial_stride % 4u || !elements || elements % 4u || elements > 16384u ||
+      !aligned(residual) || !aligned(sum) || !aligned(partials) || !aligned(output_bf16) ||
+      (weight && !aligned(weight)))
+    return fail(QLLM_INVALID_ARGUMENT, "invalid RMSNorm of a row");
+  rms_norm_residual_kernel<<<1, 1024, 0, as_stream(stream)>>>(
+      residual, sum, partials, count, partial_stride, weight,
+      static_cast<uint16_t*>(output_bf16), elements, epsilon, zero_centered != 0);
+  return launched("RMSNorm of a row");
 }
 
 extern "C" int32_t qllm_rms_norm_partials_batch(
@@ -810,7 +828,7 @@ extern "C" int32_t qllm_rms_norm_partials_batch(
       (weight && !aligned(weight)))
     return fail(QLLM_INVALID_ARGUMENT, "invalid RMSNorm of partial sums");
   rms_norm_residual_kernel<<<rows, 1024, 0, as_stream(stream)>>>(
-      residual, sum, partials, partial_count, weight,
+      residual, sum, partials, partial_count, size_t{rows} * elements, weight,
       static_cast<uint16_t*>(output_bf16), elements, epsilon, zero_centered != 0);
   return launched("RMSNorm of partial sums");
 }

@@ -1073,7 +1073,15 @@ extern "C" int32_t qllm_fp4_head_argmax(const qllm_fp4_matrix* matrix,
                                         size_t workspace_bytes,
                                         const qllm_rollout_step* advance,
                                         void* stream) {
-  if (!matrix_ok(matrix) || !input || !logits || !batch || batch > 8u || !tokens ||
+  return qllm_fp4_head_argmax_handed(matrix, input, input_bytes, logits, batch, tokens,
+                                     workspace, workspace_bytes, advance, nullptr, stream);
+}
+
+extern "C" int32_t qllm_fp4_head_argmax_handed(
+    const qllm_fp4_matrix* matrix, const void* input, size_t input_bytes, float* logits,
+    uint32_t batch, uint32_t* tokens, void* workspace, size_t workspace_bytes,
+    const qllm_rollout_step* advance, const qllm_token_handover* handover, void* stream) {
+  if (!handover_ok(handover) || !matrix_ok(matrix) || !input || !logits || !batch || batch > 8u || !tokens ||
       !workspace || matrix->padded_columns % kChunk != 0u ||
       workspace_bytes < qllm_fp4_head_workspace_bytes(matrix, batch) ||
       input_bytes < static_cast<size_t>(batch) * matrix->padded_columns * 2u ||
@@ -1103,7 +1111,8 @@ extern "C" int32_t qllm_fp4_head_argmax(const qllm_fp4_matrix* matrix,
     step = {advance->next_token, advance->draft_tokens, advance->capacity,
             advance->rows, advance->device_positions};
   return launch_argmax_final(args.argmax_values, args.argmax_indices, tiles, batch,
-                             tokens, advance ? &step : nullptr, as_stream(stream));
+                             tokens, advance ? &step : nullptr, handover,
+                             as_stream(stream));
 }
 
 extern "C" int32_t qllm_fp4_gemm_bf16_partial(const qllm_fp4_matrix* matrix,

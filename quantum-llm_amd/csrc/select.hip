@@ -106,13 +106,23 @@ __global__ __launch_bounds__(256) void argmax_partial_kernel(
 }
 
 // `advance.positions` non-null (one row): thread 0 also does what
-// rollout_advance_kernel does with the winner.
+// rollout_advance_kernel does with the winner.  `handover.host` non-null: it also stores
+// the winner for the host, which needs no launch after this one then (publish_words_kernel,
+// and the way to it, were 3 - 5 us of every decoded token).  Token and sequence number are
+// one 8-byte store, so nothing has to be ordered between rows or before it.
 __global__ __launch_bounds__(256) void argmax_final_kernel(
     const float* partial_values, const uint32_t* partial_indices,
-    uint32_t blocks_per_row, uint32_t* output, RolloutAdvance advance) {
+    uint32_t blocks_per_row, uint32_t* output, RolloutAdvance advance,
+    qllm_token_handover handover) {
   __shared__ float shared_values[4];
   __shared__ uint32_t shared_indices[4];
   const uint32_t request = blockIdx.x;
+  // (asked for with the partials, not after them)
+  const uint32_t sequence =
+      handover.sequence ? handover.sequence[0] : handover.sequence_value;
+  const bool marked =
+      handover.host && handover.emitted && (!handover.mark || handover.mark[0] != 0u);
+  const uint32_t slot_marked = marked && handover.slot ? handover.slot[0] : 0u;
   float best = -INFINITY;
   uint32_t index = kNoIndex;
   for (uint32_t item = threadIdx.x; item < blocks_per_row; item += blockDim.x) {
@@ -126,6 +136,12 @@ __global__ __launch_bounds__(256) void argmax_final_kernel(
   block_best(best, index, shared_values, shared_indices);
   if (threadIdx.x != 0u) return;
   output[request] = index;
+  if (handover.host) {
+    __hip_atomic_store(handover.host + request, uint64_t{sequence} << 32 | index,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (marked && index < handover.vocabulary)
+      handover.emitted[size_t{slot_marked} * handover.vocabulary + index] = 1u;
+  }
   if (advance.positions && request == 0u) {
     const uint32_t slot = advance.positions[3];
     advance.next_token[0] = index;
@@ -459,11 +475,19 @@ __global__ __launch_bounds__(64) void mark_presence_kernel(
 int32_t launch_argmax_final(const float* partial_values,
                             const uint32_t* partial_indices, uint32_t blocks,
                             uint32_t batch, uint32_t* output,
-                            const RolloutAdvance* advance, hipStream_t stream) {
+                            const RolloutAdvance* advance,
+                            const qllm_token_handover* handover, hipStream_t stream) {
   argmax_final_kernel<<<batch, 256, 0, stream>>>(
       partial_values, partial_indices, blocks, output,
-      advance ? *advance : RolloutAdvance{});
+      advance ? *advance : RolloutAdvance{},
+      handover ? *handover : qllm_token_handover{});
   return launched("argmax of the head's tile maxima");
+}
+
+bool handover_ok(const qllm_token_handover* handover) {
+  return !handover ||
+         (handover->host && reinterpret_cast<uintptr_t>(handover->host) % 8u == 0u &&
+          (!handover->emitted || handover->vocabulary));
 }
 
 }  // namespace qllm
@@ -479,7 +503,16 @@ extern "C" int32_t qllm_argmax_batch(const float* values, uint32_t count,
                                      uint32_t batch, uint32_t* output,
                                      void* workspace, size_t workspace_bytes,
                                      void* stream) {
-  if (!values || !count || !batch || !output || !workspace ||
+  return qllm_argmax_batch_handed(values, count, batch, output, workspace, workspace_bytes,
+                                  nullptr, stream);
+}
+
+extern "C" int32_t qllm_argmax_batch_handed(const float* values, uint32_t count,
+                                            uint32_t batch, uint32_t* output,
+                                            void* workspace, size_t workspace_bytes,
+                                            const qllm_token_handover* handover,
+                                            void* stream) {
+  if (!values || !count || !batch || !output || !workspace || !handover_ok(handover) ||
       workspace_bytes < qllm_argmax_workspace_bytes(count, batch))
     return fail(QLLM_INVALID_ARGUMENT, "invalid argmax batch");
   const uint32_t blocks = (count + kArgmaxChunk - 1u) / kArgmaxChunk;
@@ -489,7 +522,8 @@ extern "C" int32_t qllm_argmax_batch(const float* values, uint32_t count,
   argmax_partial_kernel<<<dim3(blocks, batch), 256, 0, as_stream(stream)>>>(
       values, count, partial_values, partial_indices, blocks);
   argmax_final_kernel<<<batch, 256, 0, as_stream(stream)>>>(
-      partial_values, partial_indices, blocks, output, RolloutAdvance{});
+      partial_values, partial_indices, blocks, output, RolloutAdvance{},
+      handover ? *handover : qllm_token_handover{});
   return launched("argmax batch");
 }
 
@@ -558,7 +592,8 @@ extern "C" int32_t qllm_argmax_batch_static(const float* values, uint32_t count,
   argmax_partial_kernel<<<dim3(blocks, batch), 256, 0, as_stream(stream)>>>(
       values, count, partial_values, partial_indices, blocks);
   argmax_final_kernel<<<batch, 256, 0, as_stream(stream)>>>(
-      partial_values, partial_indices, blocks, output, RolloutAdvance{});
+      partial_values, partial_indices, blocks, output, RolloutAdvance{},
+      qllm_token_handover{});
   return launched("argmax batch static");
 }
 

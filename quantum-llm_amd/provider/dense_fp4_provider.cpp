@@ -195,7 +195,7 @@ void Mi355DenseFp4Provider::allocate_workspaces() {
                              std::size_t{g_.query_heads} * g_.head_dim});
   // tokens (up to 8) and the four position words of a pass lie side by side,
   // so that one launch brings both
-  tokens_ = static_cast<std::uint32_t*>(device_alloc((8U + 4U) * 4U));
+  tokens_ = static_cast<std::uint32_t*>(device_alloc((8U + 4U + 1U) * 4U));
   positions_ = tokens_ + 8U;
   graphs_.assign(max_rows_ + 1U, nullptr);
   if (const char* eager = std::getenv("QLLM_PROVIDER_EAGER"))
@@ -1485,8 +1485,8 @@ void Mi355DenseFp4Provider::enqueue_ffn_block(std::uint32_t index,
 // hidden_: logits_ [rows, vocabulary] and their arg-max tokens.  The norm
 // also completes hidden_ when partials are pending, which is only so for a
 // head over all rows.
-void Mi355DenseFp4Provider::enqueue_head(std::uint32_t first_row,
-                                         std::uint32_t rows) {
+void Mi355DenseFp4Provider::enqueue_head(std::uint32_t first_row, std::uint32_t rows,
+                                         const qllm_token_handover* handover) {
   if (pending_partials_ && first_row != 0U)
     throw std::runtime_error("head over a row range needs a complete hidden state");
   if (g_.activation_q8) {
@@ -1497,9 +1497,9 @@ void Mi355DenseFp4Provider::enqueue_head(std::uint32_t first_row,
                            rows);
     status_check(qllm_fp4_gemm_q8(&head_.descriptor, q8_, q8_scales_, logits_,
                                   QLLM_OUT_F32, nullptr, rows, stream_));
-    status_check(qllm_argmax_batch(logits_, g_.vocabulary, rows, argmax_tokens_,
-                                   select_workspace_, select_workspace_bytes_,
-                                   stream_));
+    status_check(qllm_argmax_batch_handed(logits_, g_.vocabulary, rows, argmax_tokens_,
+                                          select_workspace_, select_workspace_bytes_,
+                                          handover, stream_));
     return;
   }
   if (first_row == 0U) {
@@ -1511,7 +1511,7 @@ void Mi355DenseFp4Provider::enqueue_head(std::uint32_t first_row,
         g_.zero_centered_norm, stream_));
   }
   enqueue_head_projection(head_.descriptor, normalized_, logits_, rows,
-                          argmax_tokens_, nullptr);
+                          argmax_tokens_, nullptr, handover);
 }
 
 // logits = head . normalized_ and their arg-max tokens: the projection's
@@ -1520,19 +1520,21 @@ void Mi355DenseFp4Provider::enqueue_head(std::uint32_t first_row,
 // the matrix-core kernel does not take go through the plain arg-max.
 void Mi355DenseFp4Provider::enqueue_head_projection(
     const qllm_fp4_matrix& head, const std::uint16_t* input, float* logits,
-    std::uint32_t rows, std::uint32_t* tokens, const qllm_rollout_step* advance) {
+    std::uint32_t rows, std::uint32_t* tokens, const qllm_rollout_step* advance,
+    const qllm_token_handover* handover) {
   const std::size_t input_bytes = std::size_t{rows} * g_.hidden * 2U;
   if (head.padded_columns % 64U == 0U &&
       qllm_fp4_head_workspace_bytes(&head, rows) <= select_workspace_bytes_) {
-    status_check(qllm_fp4_head_argmax(&head, input, input_bytes, logits, rows,
-                                      tokens, select_workspace_,
-                                      select_workspace_bytes_, advance, stream_));
+    status_check(qllm_fp4_head_argmax_handed(&head, input, input_bytes, logits, rows,
+                                             tokens, select_workspace_,
+                                             select_workspace_bytes_, advance, handover,
+                                             stream_));
     return;
   }
   status_check(qllm_fp4_gemm_bf16(&head, input, input_bytes, logits,
                                   QLLM_OUT_F32, nullptr, rows, stream_));
-  status_check(qllm_argmax_batch(logits, head.rows, rows, tokens, select_workspace_,
-                                 select_workspace_bytes_, stream_));
+  status_check(qllm_argmax_batch_handed(logits, head.rows, rows, tokens, select_workspace_,
+                                        select_workspace_bytes_, handover, stream_));
   if (advance)
     status_check(qllm_rollout_advance(tokens, advance->next_token,
                                       advance->draft_tokens, advance->capacity,
@@ -1579,7 +1581,12 @@ void Mi355DenseFp4Provider::enqueue_target(const std::uint32_t* device_tokens,
     });
     timed(GpuPhase::ffn, [&] { enqueue_ffn_block(index, rows, true); });
   }
-  timed(GpuPhase::head, [&] { enqueue_head(0U, rows); });
+  // (a captured pass reads the number of its hand-over from the word behind its positions)
+  const qllm_token_handover handover{selector_->handed_words(),
+                                     deferred_positions ? tokens_ + 12 : nullptr,
+                                     deferred_positions ? 0U : selector_->next_handover(),
+                                     nullptr, nullptr, nullptr, 0U};
+  timed(GpuPhase::head, [&] { enqueue_head(0U, rows, &handover); });
 }
 
 // The proposer's pass over a prompt chunk: row r pairs tokens[r] (the token
@@ -1778,6 +1785,8 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
       state->mtp_length = first_position;
     }
 
+    const bool head_normalised =
+        !feed_proposer && g_.hidden % 4U == 0U && g_.hidden <= 16384U;
     for (std::uint32_t done = 0; done < count;) {
       const std::uint32_t rows = std::min(prefill_rows_, count - done);
       const std::uint32_t position = first_position + done;
@@ -1932,17 +1941,25 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
             &layer.gate.descriptor, &layer.up.descriptor, prefill_normalized_,
             hidden_bytes, prefill_activation_, rows, prefill_parts_,
             prefill_parts_bytes_, stream));
-        // (the last layer's sum is complete: its rows are read as they are)
+        // (the proposer reads the last layer's sums, otherwise the head its last row's)
         project(layer.down.descriptor, prefill_activation_,
                 std::size_t{rows} * g_.intermediate * 2U,
-                index + 1U < g_.layers);
+                index + 1U < g_.layers || head_normalised);
       }
       if (done + rows == count) {
-        // last row -> the verify step's buffers, then the head on that row
-        hip_check(hipMemcpyAsync(
-                      hidden_, prefill_hidden_ + std::size_t{rows - 1U} * g_.hidden,
-                      g_.hidden * 4U, hipMemcpyDeviceToDevice, hip_stream),
-                  "retain the prompt's last hidden state");
+        // last row -> the verify step's buffers, with the norm of the head on that row
+        // (which comes by itself where the proposer's passes are still to use the buffers)
+        const float* const last = prefill_hidden_ + std::size_t{rows - 1U} * g_.hidden;
+        if (head_normalised)
+          status_check(qllm_rms_norm_row(
+              last, hidden_,
+              parts ? prefill_parts_ + std::size_t{rows - 1U} * g_.hidden : nullptr, parts,
+              std::size_t{rows} * g_.hidden, final_norm_, normalized_, g_.hidden,
+              g_.norm_epsilon, g_.zero_centered_norm, stream));
+        else
+          hip_check(hipMemcpyAsync(hidden_, last, g_.hidden * 4U, hipMemcpyDeviceToDevice,
+                                   hip_stream),
+                    "retain the prompt's last hidden state");
       }
       // the proposer sees (token at p + 1, target hidden at p) for every prompt
       // position but the last, whose successor is not known yet
@@ -1966,23 +1983,27 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
       }
       done += rows;
     }
-    status_check(qllm_rms_norm_batch(hidden_, final_norm_, nullptr, normalized_,
-                                     g_.hidden, 1U, g_.hidden, g_.norm_epsilon,
-                                     g_.zero_centered_norm, stream));
-    status_check(qllm_fp4_gemm_bf16(&head_.descriptor, normalized_,
-                                    std::size_t{g_.hidden} * 2U, logits_,
-                                    QLLM_OUT_F32, nullptr, 1U, stream));
-    status_check(qllm_argmax_batch(logits_, g_.vocabulary, 1U, argmax_tokens_,
-                                   select_workspace_, select_workspace_bytes_,
-                                   stream));
+    if (!head_normalised)
+      status_check(qllm_rms_norm_batch(hidden_, final_norm_, nullptr, normalized_,
+                                       g_.hidden, 1U, g_.hidden, g_.norm_epsilon,
+                                       g_.zero_centered_norm, stream));
+    const bool sampled = request.parameters.contains("sampling_temperature_ppm");
+    const bool marked =
+        sampled && TokenSelector::marks_handed(request, first_position + count - 1U);
+    const qllm_token_handover handover{selector_->handed_words(), nullptr,
+                                       selector_->next_handover(),
+                                       marked ? presence_ : nullptr, nullptr, nullptr,
+                                       g_.vocabulary};
+    enqueue_head_projection(head_.descriptor, normalized_, logits_, 1U, argmax_tokens_,
+                            nullptr, &handover);
     std::uint32_t predicted{};
-    if (request.parameters.contains("sampling_temperature_ppm")) {
+    if (sampled) {
       // the head under the request's sampling profile, at the position of the
       // prompt's last token (run_head with a request, :8433-8517)
       predicted = selector_->select(logits_, presence_, argmax_tokens_, request,
-                                    first_position + count - 1U);
+                                    first_position + count - 1U, true);
     } else {
-      predicted = selector_->read_token(argmax_tokens_);
+      predicted = *selector_->read_handed(1U);
     }
     prefill_tokens_total_ += count;
     if (state) {
@@ -2024,10 +2045,7 @@ er::Status Mi355DenseFp4Provider::run_target(const std::uint32_t* tokens,
     if (!embedding_ready_ || !head_ready_)
       return {er::ErrorCode::invalid_argument, "target program is not prepared"};
     ensure_pages(first_position + rows - 1U);
-    hip_check(hipMemcpyAsync(tokens_, tokens, rows * sizeof(std::uint32_t),
-                             hipMemcpyHostToDevice,
-                             static_cast<hipStream_t>(stream_)),
-              "upload target tokens");
+    status_check(qllm_store_words(tokens_, tokens, rows, stream_));
     enqueue_target(tokens_, rows, first_position, false);
     collect_gpu_phases();
     return er::Status::success();
@@ -2049,12 +2067,13 @@ er::Status Mi355DenseFp4Provider::run_target_graph(const std::uint32_t* tokens,
       return {er::ErrorCode::invalid_argument, "target program is not prepared"};
     ensure_pages(first_position + rows - 1U);
     const auto stream = static_cast<hipStream_t>(stream_);
-    std::uint32_t words[12]{};
+    std::uint32_t words[13]{};
     std::copy(tokens, tokens + rows, words);
     const std::uint32_t positions[4] = {first_position, first_position,
                                         first_position + 1U, rows};
     std::copy(positions, positions + 4, words + 8);
-    status_check(qllm_store_words(tokens_, words, 12U, stream_));
+    words[12] = selector_->next_handover();
+    status_check(qllm_store_words(tokens_, words, 13U, stream_));
     if (!graphs_[rows]) {
       hip_check(hipStreamSynchronize(stream), "drain stream before capture");
       hipGraph_t graph{};
@@ -2585,7 +2604,7 @@ void Mi355DenseFp4Provider::enqueue_mtp(std::uint32_t rows,
   enqueue_head_projection(mtp_.head_prefix,
                           normalized_ + std::size_t{rows - 1U} * g_.hidden,
                           mtp_logits_, 1U, mtp_argmax_,
-                          deferred_positions ? &advance : nullptr);
+                          deferred_positions ? &advance : nullptr, nullptr);
 }
 
 // Replays the proposer pass captured for (rows, source of the previous hidden
@@ -2846,7 +2865,9 @@ er::ExactDecodeExecutionHandle Mi355DenseFp4Provider::execute_exact_decode(
     target_distributions.reserve(rows);
     if (greedy) {
       // greedy: the rows' arg-max tokens in one hand-over
-      const std::uint32_t* const chosen = selector_->read_words(argmax_tokens_, rows);
+      const std::uint32_t* const chosen =
+          penalty == 0.0 ? selector_->read_handed(rows)
+                         : selector_->read_words(argmax_tokens_, rows);
       // a row without a finite logit selects nothing (0xffffffff): reported
       // here, before the proposer or the request state is touched
       for (std::uint32_t row = 0; row < rows; ++row)

@@ -313,11 +313,13 @@ class Mi355DenseFp4Provider final : public DecoderProvider {
                                bool normalised = false);
   void enqueue_ffn_block(std::uint32_t index, std::uint32_t rows,
                          bool leave_partials);
-  void enqueue_head(std::uint32_t first_row, std::uint32_t rows);
+  void enqueue_head(std::uint32_t first_row, std::uint32_t rows,
+                    const qllm_token_handover* handover = nullptr);
   void enqueue_head_projection(const qllm_fp4_matrix& head,
                                const std::uint16_t* input, float* logits,
                                std::uint32_t rows, std::uint32_t* tokens,
-                               const qllm_rollout_step* advance);
+                               const qllm_rollout_step* advance,
+                               const qllm_token_handover* handover);
   [[nodiscard]] er::ExecutionValue device_hidden_value(std::uint32_t rows) const;
   [[nodiscard]] std::uint32_t require_hidden_value(
       const er::ExecutionValue& value) const;

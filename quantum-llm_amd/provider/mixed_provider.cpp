@@ -14,7 +14,10 @@ namespace qllm {
 namespace {
 
 constexpr std::uint32_t kSmallBatch = 64U;   // rows that stream the weights once
-constexpr std::uint32_t kStepWords = 4U;     // ahead of the tokens
+// first position, slot, rows; whether the token is marked as emitted, and the number of
+// its hand-over
+constexpr std::uint32_t kStepWords = 6U;     // ahead of the tokens
+constexpr std::uint32_t kStepMark = 3U, kStepSequence = 4U;
 
 std::uint32_t round_up(std::uint32_t value, std::uint32_t to) {
   return (value + to - 1U) / to * to;
@@ -890,7 +893,8 @@ void Mi355MixedProvider::release_pages(const MixedRequestState& state) {
 // free: every batch ends with its token, which the device hands over last.
 void Mi355MixedProvider::begin_batch(MixedRequestState& state,
                                      std::span<const std::uint32_t> tokens,
-                                     std::uint32_t first_position) {
+                                     std::uint32_t first_position,
+                                     const er::ProgramRequestContext& request) {
   const auto rows = static_cast<std::uint32_t>(tokens.size());
   if (!rows || rows > g_.chunk_rows)
     throw std::runtime_error("program batch holds too many or no tokens");
@@ -919,7 +923,9 @@ void Mi355MixedProvider::begin_batch(MixedRequestState& state,
   words[0] = first_position;
   words[1] = state.slot;
   words[2] = rows;
-  words[3] = 0U;
+  words[kStepMark] = TokenSelector::marks_handed(request, first_position + rows - 1U);
+  words[kStepSequence] = selector_->next_handover();
+  words[5] = 0U;
   std::copy(tokens.begin(), tokens.end(), words + kStepWords);
   if (rows == 1U)
     status_check(qllm_store_words(step_.as<std::uint32_t>(), words, kStepWords + 1U,
@@ -1284,6 +1290,18 @@ void Mi355MixedProvider::enqueue_head(std::uint32_t batch_rows, std::uint32_t fi
   enqueue_normed(norm, &s, 1U);
 }
 
+// The arg-max of the first row of logits, which hands itself over.
+void Mi355MixedProvider::enqueue_selection() {
+  const auto* step = step_.as<std::uint32_t>();
+  const qllm_token_handover handover{selector_->handed_words(), step + kStepSequence, 0U,
+                                     presence_.as<std::uint8_t>(), step + kStepMark,
+                                     step + 1, g_.vocabulary};
+  status_check(qllm_argmax_batch_handed(logits_.as<float>(), g_.vocabulary, 1U,
+                                        argmax_.as<std::uint32_t>(),
+                                        select_workspace_.get(), select_workspace_bytes_,
+                                        &handover, stream_));
+}
+
 // Logits of the rows asked for and the token of the last row.  The request has
 // advanced when this returns.
 Mi355MixedProvider::HeadResult Mi355MixedProvider::finish_batch(
@@ -1321,9 +1339,7 @@ Mi355MixedProvider::HeadResult Mi355MixedProvider::finish_batch(
   }
   if (!head_enqueued) {
     enqueue_head(rows, rows - 1U, 1U, false);
-    status_check(qllm_argmax_batch(logits_.as<float>(), g_.vocabulary, 1U,
-                                   argmax_.as<std::uint32_t>(), select_workspace_.get(),
-                                   select_workspace_bytes_, stream_));
+    enqueue_selection();
   }
   if (last_wanted) copy_rows(before, 1U);
   const std::uint32_t last_position = state.position + rows - 1U;
@@ -1331,7 +1347,7 @@ Mi355MixedProvider::HeadResult Mi355MixedProvider::finish_batch(
   result.token = selector_->select(
       logits_.as<float>(),
       presence_.as<std::uint8_t>() + std::size_t{state.slot} * g_.vocabulary,
-      argmax_.as<std::uint32_t>(), request, last_position);
+      argmax_.as<std::uint32_t>(), request, last_position, true);
   release_pages(state);
   program_steps_ += rows;
   if (rows > 1U) prompt_rows_ += rows;
@@ -1346,9 +1362,7 @@ void Mi355MixedProvider::launch_step_graph() {
     enqueue_embedding(1U, true);
     for (auto& block : blocks_) enqueue_block(*block, 1U, g_.max_context - 1U);
     enqueue_head(1U, 0U, 1U, false);
-    status_check(qllm_argmax_batch(logits_.as<float>(), g_.vocabulary, 1U,
-                                   argmax_.as<std::uint32_t>(), select_workspace_.get(),
-                                   select_workspace_bytes_, stream_));
+    enqueue_selection();
   };
   // the first token runs uncaptured: it loads every kernel it needs
   if (!use_graphs_ || !step_warm_) {
@@ -1460,7 +1474,7 @@ er::OperationExecutionHandle Mi355MixedProvider::execute(
     if (operation->kind == Kind::embedding) {
       const auto tokens = host_u32_batch(input("token_ids"), kTokenAbi,
                                          "embedding token batch", g_.chunk_rows);
-      begin_batch(*state, tokens, state->position);
+      begin_batch(*state, tokens, state->position, invocation.request);
       enqueue_embedding(batch_rows_, false);
       values.emplace("hidden", hidden_value(batch_rows_));
     } else if (operation->kind == Kind::head) {
@@ -1507,7 +1521,7 @@ er::OperationExecutionHandle Mi355MixedProvider::execute_program_sequence(
     const auto positions =
         host_u32_batch(input("positions"), kPositionAbi, "position batch", g_.chunk_rows);
     const auto first = contiguous_first(positions, tokens.size());
-    begin_batch(*state, tokens, first);
+    begin_batch(*state, tokens, first, invocation.request);
     const bool single = batch_rows_ == 1U;
     if (single) {
       launch_step_graph();

@@ -54,28 +54,21 @@ std::uint32_t TokenSelector::read_token(const std::uint32_t* device_token,
   return *read_words(device_token, 1U, emitted);
 }
 
-// A kernel writes the words into pinned memory, a sequence number after them.  After a
+// A kernel writes words into pinned memory, and a sequence number that says so.  After a
 // replayed graph the host watches the number: a wait for the stream takes 7.5 us longer, and
 // whoever waits for it later, if anybody does, finds 10 to 15 us of it left, as many after
 // 4096 replays as after one.  Launches of a pass one by one are waited for here: watching
 // saves 5 us of a pass of 40 and leaves 31 to the next wait, which is the next capture's,
 // copy's or the caller's.  What has not arrived after two milliseconds - a device that has
 // failed - is waited for with the stream, which reports what went wrong.
-const std::uint32_t* TokenSelector::read_words(const std::uint32_t* device_words,
-                                               std::uint32_t count, std::uint8_t* emitted) {
-  if (!count || count > kMostWords) throw std::runtime_error("invalid device words to read");
+template <typename Arrived>
+void TokenSelector::await(const Arrived& arrived) {
   const bool watched = std::exchange(replayed_, false);
-  const std::uint32_t sequence = ++sequence_;
-  status_check(qllm_publish_words(device_words, count, staging_->words, &staging_->sequence,
-                                  sequence, emitted, vocabulary_, stream_));
-  const auto arrived = [&] {
-    return __atomic_load_n(&staging_->sequence, __ATOMIC_ACQUIRE) == sequence;
-  };
   if (watched && ++unwaited_ < kMostUnwaited) {
     const auto deadline = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
     do {
       for (int turn = 0; turn < 64; ++turn) {
-        if (arrived()) return staging_->words;
+        if (arrived()) return;
         __builtin_ia32_pause();
       }
     } while (std::chrono::steady_clock::now() < deadline);
@@ -83,7 +76,41 @@ const std::uint32_t* TokenSelector::read_words(const std::uint32_t* device_words
   hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream_)), "wait for the device");
   unwaited_ = 0U;
   if (!arrived()) throw std::runtime_error("the device's words have not arrived");
+}
+
+const std::uint32_t* TokenSelector::read_words(const std::uint32_t* device_words,
+                                               std::uint32_t count, std::uint8_t* emitted) {
+  if (!count || count > kMostWords) throw std::runtime_error("invalid device words to read");
+  const std::uint32_t sequence = ++sequence_;
+  status_check(qllm_publish_words(device_words, count, staging_->words, &staging_->sequence,
+                                  sequence, emitted, vocabulary_, stream_));
+  await([&] {
+    return __atomic_load_n(&staging_->sequence, __ATOMIC_ACQUIRE) == sequence;
+  });
   return staging_->words;
+}
+
+const std::uint32_t* TokenSelector::read_handed(std::uint32_t rows) {
+  if (!rows || rows > kMostHanded) throw std::runtime_error("invalid tokens to read");
+  await([&] {
+    for (std::uint32_t row = 0; row < rows; ++row) {
+      const std::uint64_t word = __atomic_load_n(&staging_->handed[row], __ATOMIC_ACQUIRE);
+      if (word >> 32 != handed_sequence_) return false;
+      handed_tokens_[row] = static_cast<std::uint32_t>(word);
+    }
+    return true;
+  });
+  return handed_tokens_;
+}
+
+bool TokenSelector::marks_handed(const er::ProgramRequestContext& request,
+                                 std::uint32_t sample_position) {
+  for (const char* name : {"sampling_first_output_position", "sampling_temperature_ppm",
+                           "sampling_presence_penalty_biased_ppm"})
+    if (!request.parameters.contains(name)) return false;   // which select() reports
+  return sample_position >= request_parameter(request, "sampling_first_output_position") &&
+         request_parameter(request, "sampling_temperature_ppm") == 0U &&
+         request_parameter(request, "sampling_presence_penalty_biased_ppm") == 2'000'000U;
 }
 
 // The head's token for a request (run_head with a request, :8433-8517): the
@@ -94,7 +121,7 @@ const std::uint32_t* TokenSelector::read_words(const std::uint32_t* device_words
 std::uint32_t TokenSelector::select(float* logits, std::uint8_t* presence,
                                     std::uint32_t* argmax_tokens,
                                     const er::ProgramRequestContext& request,
-                                    std::uint32_t sample_position) {
+                                    std::uint32_t sample_position, bool handed) {
   const auto stream = static_cast<hipStream_t>(stream_);
   const auto first_output =
       request_parameter(request, "sampling_first_output_position");
@@ -111,7 +138,9 @@ std::uint32_t TokenSelector::select(float* logits, std::uint8_t* presence,
   const auto temperature = request_parameter(request, "sampling_temperature_ppm");
   std::uint32_t selected{};
   if (temperature == 0U) {
-    selected = read_token(argmax_tokens, output_sampling ? presence : nullptr);
+    selected = handed && !(output_sampling && penalty != 0.0)
+                   ? *read_handed(1U)
+                   : read_token(argmax_tokens, output_sampling ? presence : nullptr);
     // a row without a finite logit selects nothing (0xffffffff): reported
     // before the presence bytes or the caller's state change
     if (selected >= vocabulary_)
@@ -167,7 +196,7 @@ std::uint32_t TokenSelector::select(float* logits, std::uint8_t* presence,
                               sample_position, 0U));
     }
   }
-  if (output_sampling && temperature != 0U) {   // (read_token has marked the other)
+  if (output_sampling && temperature != 0U) {   // (the other has been marked with its word)
     const std::uint32_t token[1] = {selected};
     mark(presence, token);
   }

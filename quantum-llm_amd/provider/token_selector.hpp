@@ -31,11 +31,15 @@ class TokenSelector final {
 
   // The head's token for a request (dense_fp4_provider.cpp:8433-8517) from one
   // row of logits whose arg-max lies in `argmax_tokens`; an output token is
-  // marked as emitted in `presence`.
+  // marked as emitted in `presence`.  `handed`: the launch that took the arg-max hands it
+  // over, and has marked it where marks_handed() says so.
   [[nodiscard]] std::uint32_t select(float* logits, std::uint8_t* presence,
                                      std::uint32_t* argmax_tokens,
                                      const er::ProgramRequestContext& request,
-                                     std::uint32_t sample_position);
+                                     std::uint32_t sample_position, bool handed = false);
+  // Whether select() emits the arg-max of the logits as they are.
+  [[nodiscard]] static bool marks_handed(const er::ProgramRequestContext& request,
+                                         std::uint32_t sample_position);
   [[nodiscard]] er::SamplingDistribution distribution(
       float* row_logits, std::uint32_t vocabulary, std::uint32_t* device_argmax,
       const er::ProgramRequestContext& request, const std::uint8_t* presence);
@@ -54,6 +58,13 @@ class TokenSelector final {
   [[nodiscard]] const std::uint32_t* read_words(const std::uint32_t* device_words,
                                                 std::uint32_t count,
                                                 std::uint8_t* emitted = nullptr);
+  // Where an arg-max of up to kMostHanded rows leaves its tokens by itself; the next
+  // sequence number, for the device word that its launch reads; and the tokens handed over
+  // with that number, after everything enqueued so far: there until the next call.
+  static constexpr std::uint32_t kMostHanded = 8U;
+  [[nodiscard]] std::uint64_t* handed_words() const noexcept { return staging_->handed; }
+  [[nodiscard]] std::uint32_t next_handover() noexcept { return ++handed_sequence_; }
+  [[nodiscard]] const std::uint32_t* read_handed(std::uint32_t rows);
   // emitted[token] = 1 for every token (one launch)
   void mark(std::uint8_t* emitted, std::span<const std::uint32_t> tokens);
 
@@ -67,7 +78,11 @@ class TokenSelector final {
   struct Staging final {
     std::uint32_t words[kMostWords];
     alignas(64) std::uint32_t sequence;
+    alignas(64) std::uint64_t handed[kMostHanded];   // sequence << 32 | token
   };
+  // Waits until arrived(): the one way to read what the device writes.
+  template <typename Arrived>
+  void await(const Arrived& arrived);
   // hand-overs in a row without a wait for the stream, for which the runtime keeps a
   // little of every launch
   static constexpr std::uint32_t kMostUnwaited = 256U;
@@ -79,6 +94,8 @@ class TokenSelector final {
   float* top_logits_{};
   Staging* staging_{};
   std::uint32_t sequence_{};
+  std::uint32_t handed_sequence_{};
+  std::uint32_t handed_tokens_[kMostHanded]{};
   std::uint32_t unwaited_{};
   bool replayed_{};
   std::uint64_t gpu_calls_{};

@@ -47,6 +47,12 @@ class RolloutStep(Structure):
                 ("device_positions", c_void_p)]
 
 
+class TokenHandover(Structure):
+    _fields_ = [("host", c_void_p), ("sequence", c_void_p), ("sequence_value", c_uint32),
+                ("emitted", c_void_p), ("mark", c_void_p), ("slot", c_void_p),
+                ("vocabulary", c_uint32)]
+
+
 class Q4hAttentionLaunch(Structure):
     _fields_ = [("query", c_void_p), ("q8_queries", c_void_p),
                 ("query_scales", c_void_p), ("page_table", c_void_p),
@@ -283,6 +289,9 @@ SIGNATURES = {
     "qllm_rollout_advance": (c_int32, [c_void_p, c_void_p, c_void_p, c_uint32, c_uint32, c_void_p, c_void_p]),
     "qllm_attention_paged_q8": (c_int32, [POINTER(Q8AttentionLaunch)]),
     "qllm_argmax_workspace_bytes": (c_size_t, [c_uint32, c_uint32]),
+    "qllm_fp4_head_argmax_handed": (c_int32, [POINTER(Fp4Matrix), c_void_p, c_size_t, c_void_p, c_uint32, c_void_p, c_void_p, c_size_t, POINTER(RolloutStep), POINTER(TokenHandover), c_void_p]),
+    "qllm_argmax_batch_handed": (c_int32, [c_void_p, c_uint32, c_uint32, c_void_p, c_void_p, c_size_t, POINTER(TokenHandover), c_void_p]),
+    "qllm_rms_norm_row": (c_int32, [c_void_p, c_void_p, c_void_p, c_uint32, c_size_t, c_void_p, c_void_p, c_uint32, c_float, c_int32, c_void_p]),
     "qllm_argmax_batch": (c_int32, [c_void_p, c_uint32, c_uint32, c_void_p, c_void_p, c_size_t, c_void_p]),
     "qllm_argmax_static_capacity_bytes": (c_size_t, []),
     "qllm_argmax_batch_static": (c_int32, [c_void_p, c_uint32, c_uint32, c_void_p, c_void_p]),

@@ -538,6 +538,93 @@ def test_words_reach_pinned_memory_before_their_sequence_number(device, count):
                     stream)
 
 
+@pytest.mark.parametrize("count,batch", [(1, 1), (2047, 5), (32000, 1), (32001, 8)])
+@pytest.mark.parametrize("words", [False, True])
+def test_argmax_hands_its_tokens_over(device, count, batch, words):
+    """A captured arg-max leaves token and sequence number in pinned memory on every
+    replay, with the number that its device word holds then, and marks where the device
+    says so; rows without a token hand over 0xffffffff and mark nothing."""
+    generator = torch.Generator().manual_seed(count + batch)
+    host = torch.zeros(batch, dtype=torch.int64).pin_memory()
+    step = torch.zeros(3, dtype=torch.int32, device=device)   # number, mark, slot
+    emitted = torch.zeros(3, count, dtype=torch.uint8, device=device)
+    values = torch.empty(batch, count, device=device)
+    tokens = torch.empty(batch, dtype=torch.int32, device=device)
+    workspace = torch.empty(qh.call("qllm_argmax_workspace_bytes", count, batch),
+                            dtype=torch.uint8, device=device)
+    handover = qh.TokenHandover(qh.ptr(host), qh.ptr(step) if words else None, 41,
+                                qh.ptr(emitted), qh.ptr(step[1:]) if words else None,
+                                qh.ptr(step[2:]) if words else None, count)
+    stream = torch.cuda.Stream()
+
+    def launch():
+        qh.call("qllm_argmax_batch_handed", qh.ptr(values), count, batch, qh.ptr(tokens),
+                qh.ptr(workspace), workspace.numel(), handover, stream.cuda_stream)
+
+    launch()
+    stream.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        launch()
+    emitted.zero_()
+    marks = torch.zeros(3, count, dtype=torch.uint8)
+    for number in range(1, 5):
+        rows = torch.randn(batch, count, generator=generator)
+        if number == 3:
+            rows[0] = float("nan")
+        values.copy_(rows)
+        mark, slot = number % 2, number // 2
+        step.copy_(torch.tensor([number, mark, slot], dtype=torch.int32))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            graph.replay()
+        torch.cuda.synchronize()
+        chosen = rows.argmax(dim=1)
+        if number == 3:
+            chosen[0] = 0xffffffff
+        assert torch.equal(host >> 32, torch.full((batch,), number if words else 41))
+        assert torch.equal(host & 0xffffffff, chosen)
+        assert torch.equal(tokens.cpu().long() & 0xffffffff, chosen)
+        if mark or not words:
+            marks[slot if words else 0, chosen[chosen < count]] = 1
+        assert torch.equal(emitted.cpu(), marks)
+    for bad in (qh.TokenHandover(None, None, 1, None, None, None, 0),
+                qh.TokenHandover(qh.ptr(host) + 4, None, 1, None, None, None, 0),
+                qh.TokenHandover(qh.ptr(host), None, 1, qh.ptr(emitted), None, None, 0)):
+        with pytest.raises(qh.QllmError, match="invalid"):
+            qh.call("qllm_argmax_batch_handed", qh.ptr(values), count, batch, qh.ptr(tokens),
+                    qh.ptr(workspace), workspace.numel(), bad, None)
+
+
+@pytest.mark.parametrize("elements,rows,count", [(4, 1, 0), (2048, 5, 1), (5120, 48, 12),
+                                                 (16384, 3, 16)])
+@pytest.mark.parametrize("zero_centered", [0, 1])
+def test_norm_of_a_row_equals_that_of_its_batch(device, elements, rows, count, zero_centered):
+    """The last row of a batch of partial sums by itself: sum and norm bit for bit."""
+    hidden = torch.randn(rows, elements, device=device)
+    parts = torch.randn(max(count, 1), rows, elements, device=device)
+    weight = torch.randn(elements, device=device)
+    out = torch.empty(rows, elements, dtype=torch.int16, device=device)
+    want = hidden.clone()
+    if count:
+        qh.call("qllm_rms_norm_residual_batch", qh.ptr(want), qh.ptr(parts), count,
+                qh.ptr(weight), qh.ptr(out), rows, elements, 1e-6, zero_centered, None)
+    else:
+        qh.call("qllm_rms_norm_batch", qh.ptr(want), qh.ptr(weight), None, qh.ptr(out),
+                elements, rows, elements, 1e-6, zero_centered, None)
+    total = torch.empty(elements, device=device)
+    row = torch.empty(elements, dtype=torch.int16, device=device)
+    qh.call("qllm_rms_norm_row", qh.ptr(hidden[rows - 1]), qh.ptr(total),
+            qh.ptr(parts[0, rows - 1]) if count else None, count, rows * elements,
+            qh.ptr(weight), qh.ptr(row), elements, 1e-6, zero_centered, None)
+    torch.cuda.synchronize()
+    assert torch.equal(total, want[rows - 1])
+    assert torch.equal(row, out[rows - 1])
+    with pytest.raises(qh.QllmError, match="invalid"):
+        qh.call("qllm_rms_norm_row", qh.ptr(hidden), qh.ptr(total), None, 1, elements,
+                qh.ptr(weight), qh.ptr(row), elements, 1e-6, zero_centered, None)
+
+
 @pytest.mark.parametrize("columns", [4, 252, 2048, 5120, 16384])
 @pytest.mark.parametrize("scheme", [ol.SCALE_UE8M0_BLOCK32, ol.SCALE_F16_BLOCK16])
 @pytest.mark.parametrize("rows,rotary,q8,zero_centered", [

@@ -106,12 +106,70 @@ int main() {
 }
 """
 
+HANDED = DRIVER[:DRIVER.index("int main()")] + r"""
+int main() {
+  qllm::TokenSelector selector(nullptr, 64u, nullptr, 0u);
+  std::uint64_t* const host = selector.handed_words();
+  // tokens that are there with their number are read without a launch; watched after a
+  // replayed graph, waited for otherwise
+  for (std::uint32_t pass = 1; pass <= 40; ++pass) {
+    const std::uint32_t number = selector.next_handover();
+    EXPECT(number == pass);
+    for (std::uint32_t row = 0; row < 8u; ++row)
+      host[row] = std::uint64_t{number} << 32 | (pass + row);
+    waits = 0;
+    if (pass % 2u) selector.replayed();
+    const std::uint32_t* const tokens = selector.read_handed(8u);
+    for (std::uint32_t row = 0; row < 8u; ++row) EXPECT(tokens[row] == pass + row);
+    EXPECT(waits == (pass % 2u ? 0 : 1));
+  }
+  // a row that is late arrives with the stream; one that never does is an error, and so
+  // is the token of an earlier pass
+  const std::uint32_t number = selector.next_handover();
+  host[0] = std::uint64_t{number} << 32 | 5u;
+  pending = [=] { host[1] = std::uint64_t{number} << 32 | 0xffffffffu; };
+  selector.replayed();
+  waits = 0;
+  EXPECT(selector.read_handed(2u)[1] == 0xffffffffu && waits == 1);
+  (void)selector.next_handover();
+  for (const bool graph : {false, true}) {
+    selector.replayed(graph);
+    bool thrown = false;
+    try { (void)selector.read_handed(1u); } catch (const std::runtime_error&) { thrown = true; }
+    EXPECT(thrown);
+  }
+  // which requests emit the arg-max as it is
+  qllm::er::ProgramRequestContext request;
+  EXPECT(!qllm::TokenSelector::marks_handed(request, 9u));
+  request.parameters["sampling_first_output_position"] = 5u;
+  request.parameters["sampling_temperature_ppm"] = 0u;
+  request.parameters["sampling_presence_penalty_biased_ppm"] = 2'000'000u;
+  EXPECT(qllm::TokenSelector::marks_handed(request, 5u));
+  EXPECT(!qllm::TokenSelector::marks_handed(request, 4u));
+  request.parameters["sampling_presence_penalty_biased_ppm"] = 2'000'001u;
+  EXPECT(!qllm::TokenSelector::marks_handed(request, 5u));
+  request.parameters["sampling_presence_penalty_biased_ppm"] = 2'000'000u;
+  request.parameters["sampling_temperature_ppm"] = 1u;
+  EXPECT(!qllm::TokenSelector::marks_handed(request, 5u));
+  std::puts("ok");
+  return 0;
+}
+"""
+
 
 def test_only_replayed_graphs_leave_the_stream_unwaited_for(tmp_path):
+    run_driver(tmp_path, DRIVER)
+
+
+def test_tokens_handed_over_with_their_number(tmp_path):
+    run_driver(tmp_path, HANDED)
+
+
+def run_driver(tmp_path, driver):
     if not os.path.isdir("/opt/rocm/include/hip"):
         pytest.skip("the runtime's headers are not installed")
     source, binary = tmp_path / "driver.cpp", tmp_path / "driver"
-    source.write_text(DRIVER)
+    source.write_text(driver)
     done = subprocess.run(
         ["g++", "-std=c++20", "-O1", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(ROOT, "include"),
          "-I" + os.path.join(PROVIDER, "include"), "-I" + PROVIDER, "-isystem", "/opt/rocm/include",
