@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
+#include <type_traits>
 
 namespace qllm {
 
@@ -263,6 +264,14 @@ __global__ __launch_bounds__(1024) void quantize_q8_wide_kernel(
     target[index] = 0u;
 }
 
+// A row of up to SLOTS x blockDim.x x 4 values.  Bound by round trips to memory: everything
+// is asked for before anything is waited for, of partial sums up to eight pieces a slot,
+// and the sum is stored when the row's square has been added up, not before its barriers.
+// With one slot after the other, four pieces at a time, the store in between and always 1024
+// threads of four slots, five rows of 5120 and three parts took 3.87 us (now 3.41), of 2048
+// 3.25 (2.57), 48 rows of 5120 and twelve parts 7.15 (6.44), 4000 rows and two 80.8 (73.2),
+// 3000 rows of 2048 without parts 15.5 (10.2).
+template <int SLOTS = 4, bool PARTS = false>
 __device__ __forceinline__ void rms_norm_row_wide(
     const float* input_row, const float* weight, float* out_f32,
     uint16_t* out_bf16, uint32_t bf16_columns, uint32_t elements,
@@ -275,66 +284,91 @@ __device__ __forceinline__ void rms_norm_row_wide(
   // with fp4_codes_row the row is an FP4 embedding row, decoded on the way in
   const float4* x = reinterpret_cast<const float4*>(input_row);
   const uint32_t vectors = elements / 4u;
+  // (with one slot the threads are hardly more than the pieces: those past the row take its
+  // last one for nothing, and no load is behind a condition)
+  const auto piece = [&](int slot) {
+    const uint32_t index = slot * blockDim.x + threadIdx.x;
+    return SLOTS == 1 ? min(index, vectors - 1u) : index;
+  };
   // the row and its weights are fetched together, before the reduction
-  float4 values[4];
-  float4 factors[4];
+  float4 values[SLOTS];
+  float4 factors[SLOTS];
   float square = 0.0f;
 #pragma unroll
-  for (int slot = 0; slot < 4; ++slot) {
+  for (int slot = 0; slot < SLOTS; ++slot) {
     const uint32_t index = slot * blockDim.x + threadIdx.x;
     values[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
+    factors[slot] = make_float4(1.f, 1.f, 1.f, 1.f);
+    if constexpr (PARTS) {
+      const uint32_t at = piece(slot);
+      if (at >= vectors) continue;
+      if (input_row) values[slot] = x[at];
+      if (weight) factors[slot] = reinterpret_cast<const float4*>(weight)[at];
+      continue;
+    }
     if (index < vectors)
       values[slot] = fp4_codes_row ? fp4_row_vector(fp4_codes_row, fp4_scales_row,
                                                     fp4_scheme, index)
                      : input_row   ? x[index]
                                    : make_float4(0.f, 0.f, 0.f, 0.f);
-    factors[slot] = make_float4(1.f, 1.f, 1.f, 1.f);
     if (weight && index < vectors)
       factors[slot] = reinterpret_cast<const float4*>(weight)[index];
   }
-  if (partial_count) {
+  if (PARTS && partial_count) {
+    const auto add = [&]<uint32_t COUNT>(std::integral_constant<uint32_t, COUNT>,
+                                         uint32_t first) {
+      float4 early[SLOTS][COUNT];
 #pragma unroll
-    for (int slot = 0; slot < 4; ++slot) {
-      const uint32_t index = slot * blockDim.x + threadIdx.x;
-      if (index >= vectors) continue;
-      // partials are requested four at a time (one round trip each; one at a time,
-      // twelve of a 48-row prompt's rows took 9.0 us, 6.8 so) and added
-      // in index order
-      for (uint32_t first = 0; first < partial_count; first += 4u) {
-        float4 early[4];
+      for (int slot = 0; slot < SLOTS; ++slot)
 #pragma unroll
-        for (uint32_t p = 0; p < 4u; ++p)
-          if (first + p < partial_count)
-            early[p] = reinterpret_cast<const float4*>(
-                partial_row + (first + p) * partial_stride)[index];
+        for (uint32_t p = 0; p < COUNT; ++p)
+          if (const uint32_t at = piece(slot); at < vectors)
+            early[slot][p] = reinterpret_cast<const float4*>(
+                partial_row + (first + p) * partial_stride)[at];
 #pragma unroll
-        for (uint32_t p = 0; p < 4u; ++p)
-          if (first + p < partial_count) {
-            values[slot].x += early[p].x; values[slot].y += early[p].y;
-            values[slot].z += early[p].z; values[slot].w += early[p].w;
-          }
-      }
-      reinterpret_cast<float4*>(sum_out)[index] = values[slot];
+      for (int slot = 0; slot < SLOTS; ++slot)
+#pragma unroll
+        for (uint32_t p = 0; p < COUNT; ++p) {   // in index order
+          values[slot].x += early[slot][p].x; values[slot].y += early[slot][p].y;
+          values[slot].z += early[slot][p].z; values[slot].w += early[slot][p].w;
+        }
+    };
+    constexpr uint32_t kMost = SLOTS > 2 ? 4u : 8u;
+    uint32_t first = 0;
+    for (; first + kMost <= partial_count; first += kMost)
+      add(std::integral_constant<uint32_t, kMost>{}, first);
+    if (kMost > 4u && first + 4u <= partial_count) {
+      add(std::integral_constant<uint32_t, 4u>{}, first);
+      first += 4u;
     }
-  } else if (sum_out) {
-#pragma unroll
-    for (int slot = 0; slot < 4; ++slot) {
-      const uint32_t index = slot * blockDim.x + threadIdx.x;
-      if (index < vectors) reinterpret_cast<float4*>(sum_out)[index] = values[slot];
-    }
+    if (first + 3u == partial_count)
+      add(std::integral_constant<uint32_t, 3u>{}, first);
+    else if (first + 2u == partial_count)
+      add(std::integral_constant<uint32_t, 2u>{}, first);
+    else if (first + 1u == partial_count)
+      add(std::integral_constant<uint32_t, 1u>{}, first);
   }
 #pragma unroll
-  for (int slot = 0; slot < 4; ++slot) {
+  for (int slot = 0; slot < SLOTS; ++slot) {
+    if (slot * blockDim.x + threadIdx.x >= vectors) continue;
     square = fmaf(values[slot].x, values[slot].x, square);
     square = fmaf(values[slot].y, values[slot].y, square);
     square = fmaf(values[slot].z, values[slot].z, square);
     square = fmaf(values[slot].w, values[slot].w, square);
   }
   square = block_sum(square, scratch);
+  // (after the sum's barriers, which wait for stores)
+  if (sum_out) {
+#pragma unroll
+    for (int slot = 0; slot < SLOTS; ++slot) {
+      const uint32_t index = slot * blockDim.x + threadIdx.x;
+      if (index < vectors) reinterpret_cast<float4*>(sum_out)[index] = values[slot];
+    }
+  }
   const float inverse =
       rsqrtf(square / static_cast<float>(elements) + epsilon);
 #pragma unroll
-  for (int slot = 0; slot < 4; ++slot) {
+  for (int slot = 0; slot < SLOTS; ++slot) {
     const uint32_t index = slot * blockDim.x + threadIdx.x;
     if (index >= vectors) continue;
     float4 factor = factors[slot];
@@ -360,7 +394,7 @@ __device__ __forceinline__ void rms_norm_row_wide(
     // output (same operations on the same values)
     float maximum = 0.0f;
 #pragma unroll
-    for (int slot = 0; slot < 4; ++slot) {
+    for (int slot = 0; slot < SLOTS; ++slot) {
       if (slot * blockDim.x + threadIdx.x >= vectors) continue;
       maximum = fmaxf(maximum, fmaxf(fmaxf(fabsf(values[slot].x), fabsf(values[slot].y)),
                                      fmaxf(fabsf(values[slot].z), fabsf(values[slot].w))));
@@ -369,7 +403,7 @@ __device__ __forceinline__ void rms_norm_row_wide(
     const float scale = maximum > 0.0f ? maximum / 127.0f : 1.0f;
     if (threadIdx.x == 0) *out_q8_scale = scale;
 #pragma unroll
-    for (int slot = 0; slot < 4; ++slot) {
+    for (int slot = 0; slot < SLOTS; ++slot) {
       const uint32_t index = slot * blockDim.x + threadIdx.x;
       if (index >= vectors) continue;
       reinterpret_cast<uint32_t*>(out_q8)[index] = q8_pack4(values[slot], scale);
@@ -381,13 +415,14 @@ __device__ __forceinline__ void rms_norm_row_wide(
       out_bf16[index] = 0u;
 }
 
+template <int SLOTS>
 __global__ __launch_bounds__(1024) void rms_norm_batch_wide_kernel(
     const float* input, const float* weight, float* output_f32,
     uint16_t* output_bf16, uint32_t bf16_padded_columns, uint32_t elements,
     float epsilon, bool zero_centered) {
   __shared__ float scratch[16];
   const size_t row = blockIdx.x;
-  rms_norm_row_wide(
+  rms_norm_row_wide<SLOTS>(
       input + row * elements, weight,
       output_f32 ? output_f32 + row * elements : nullptr,
       output_bf16 ? output_bf16 + row * bf16_padded_columns : nullptr,
@@ -451,25 +486,27 @@ __global__ __launch_bounds__(1024) void embedding_norm_kernel(const EmbeddingNor
 
 // RMSNorm of a row straight into its per-row Q8 form (normalize_rows followed
 // by quantize_rows, dense_fp4_provider.cpp:5740-5778, 5983-5992, in one launch).
+template <int SLOTS>
 __global__ __launch_bounds__(1024) void rms_norm_q8_kernel(
     const float* input, const float* weight, int8_t* output_q8, float* scales,
     uint32_t elements, float epsilon, bool zero_centered) {
   __shared__ float scratch[16];
   const size_t row = blockIdx.x;
-  rms_norm_row_wide(input + row * elements, weight, nullptr, nullptr, 0u, elements,
+  rms_norm_row_wide<SLOTS>(input + row * elements, weight, nullptr, nullptr, 0u, elements,
                     epsilon, zero_centered, scratch, nullptr, 0u, 0u, nullptr,
                     output_q8 + row * elements, scales + row);
 }
 
 // The same on a row that is first completed from K-split partial sums
 // (rms_norm_residual_kernel below, with the Q8 output of rms_norm_q8_kernel).
+template <int SLOTS>
 __global__ __launch_bounds__(1024) void rms_norm_residual_q8_kernel(
     const float* residual, float* sum, const float* partials,
     uint32_t partial_count, const float* weight, int8_t* output_q8, float* scales,
     uint32_t elements, float epsilon, bool zero_centered) {
   __shared__ float scratch[16];
   const size_t row = blockIdx.x;
-  rms_norm_row_wide(residual ? residual + row * elements : nullptr, weight, nullptr,
+  rms_norm_row_wide<SLOTS, true>(residual ? residual + row * elements : nullptr, weight, nullptr,
                     nullptr, 0u, elements, epsilon, zero_centered, scratch,
                     partials + row * elements, partial_count,
                     static_cast<size_t>(gridDim.x) * elements, sum + row * elements,
@@ -480,16 +517,30 @@ __global__ __launch_bounds__(1024) void rms_norm_residual_q8_kernel(
 // without a residual), then its RMSNorm in bf16: the residual add of a
 // projection whose K was cut over workgroups (qllm_fp4_gemm_bf16_partial)
 // folded into the norm that follows it.  `sum` may be `residual`.
+template <int SLOTS>
 __global__ __launch_bounds__(1024) void rms_norm_residual_kernel(
     const float* residual, float* sum, const float* partials,
     uint32_t partial_count, size_t partial_stride, const float* weight,
     uint16_t* output_bf16, uint32_t elements, float epsilon, bool zero_centered) {
   __shared__ float scratch[16];
   const size_t row = blockIdx.x;
-  rms_norm_row_wide(residual ? residual + row * elements : nullptr, weight, nullptr,
+  rms_norm_row_wide<SLOTS, true>(residual ? residual + row * elements : nullptr, weight, nullptr,
                     output_bf16 + row * elements, elements, elements, epsilon,
                     zero_centered, scratch, partials + row * elements,
                     partial_count, partial_stride, sum + row * elements);
+}
+
+// Calls launch(SLOTS, threads) for as few pieces a thread as hold a row; `two`: two of them
+// as well.  A piece is the same thread's in all of them: the forms of a norm add up a row's
+// square in one order.  (Two pieces on 640 threads are as fast for 5120 and were in another.)
+template <typename Launch>
+void with_row_slots(uint32_t elements, bool two, const Launch& launch) {
+  if (elements <= 4096u)
+    launch(std::integral_constant<int, 1>{}, (elements / 4u + kWave - 1u) / kWave * kWave);
+  else if (elements <= 8192u && two)
+    launch(std::integral_constant<int, 2>{}, 1024u);
+  else
+    launch(std::integral_constant<int, 4>{}, 1024u);
 }
 
 // Row r of the output is [RMSNorm(first[r]) | RMSNorm(second[r])] in bf16:
@@ -653,8 +704,11 @@ extern "C" int32_t qllm_rms_norm_q8_batch(const float* input, const float* weigh
       elements % 4u != 0u || elements > 16384u || !(epsilon > 0.0f) ||
       !aligned(input) || !aligned(output_q8) || (weight && !aligned(weight)))
     return fail(QLLM_INVALID_ARGUMENT, "invalid Q8 RMSNorm");
-  rms_norm_q8_kernel<<<rows, 1024, 0, as_stream(stream)>>>(
-      input, weight, output_q8, scales, elements, epsilon, zero_centered != 0);
+  with_row_slots(elements, true, [&]<int SLOTS>(std::integral_constant<int, SLOTS>,
+                                                uint32_t threads) {
+    rms_norm_q8_kernel<SLOTS><<<rows, threads, 0, as_stream(stream)>>>(
+        input, weight, output_q8, scales, elements, epsilon, zero_centered != 0);
+  });
   return launched("Q8 RMSNorm");
 }
 
@@ -671,9 +725,12 @@ extern "C" int32_t qllm_rms_norm_partials_q8_batch(
       elements > 16384u || !(epsilon > 0.0f) || !aligned(residual) || !aligned(sum) ||
       !aligned(partials) || !aligned(output_q8) || (weight && !aligned(weight)))
     return fail(QLLM_INVALID_ARGUMENT, "invalid Q8 RMSNorm of partial sums");
-  rms_norm_residual_q8_kernel<<<rows, 1024, 0, as_stream(stream)>>>(
-      residual, sum, partials, partial_count, weight, output_q8, scales, elements,
-      epsilon, zero_centered != 0);
+  with_row_slots(elements, true, [&]<int SLOTS>(std::integral_constant<int, SLOTS>,
+                                                uint32_t threads) {
+    rms_norm_residual_q8_kernel<SLOTS><<<rows, threads, 0, as_stream(stream)>>>(
+        residual, sum, partials, partial_count, weight, output_q8, scales, elements,
+        epsilon, zero_centered != 0);
+  });
   return launched("Q8 RMSNorm of partial sums");
 }
 
@@ -765,9 +822,12 @@ extern "C" int32_t qllm_rms_norm_batch(const float* input, const float* weight,
       (reinterpret_cast<uintptr_t>(output_bf16) & 7u) == 0u;
   if (elements % 4u == 0u && elements <= 16384u && aligned &&
       bf16_padded_columns % 4u == 0u)
-    rms_norm_batch_wide_kernel<<<rows, 1024, 0, as_stream(stream)>>>(
-        input, weight, output_f32, static_cast<uint16_t*>(output_bf16),
-        bf16_padded_columns, elements, epsilon, zero_centered != 0);
+    with_row_slots(elements, false, [&]<int SLOTS>(std::integral_constant<int, SLOTS>,
+                                                   uint32_t threads) {
+      rms_norm_batch_wide_kernel<SLOTS><<<rows, threads, 0, as_stream(stream)>>>(
+          input, weight, output_f32, static_cast<uint16_t*>(output_bf16),
+          bf16_padded_columns, elements, epsilon, zero_centered != 0);
+    });
   else
     rms_norm_batch_kernel<<<rows, 256, 0, as_stream(stream)>>>(
         input, weight, output_f32, static_cast<uint16_t*>(output_bf16),
@@ -789,9 +849,12 @@ extern "C" int32_t qllm_rms_norm_residual_batch(
     return fail(QLLM_INVALID_ARGUMENT, "invalid residual RMSNorm");
   // (measured on rows of 5120: 320 threads, four float4 each, take 6.0 us
   // against 4.75 us with 1024: one CU's few waves wait longer for the row)
-  rms_norm_residual_kernel<<<rows, 1024, 0, as_stream(stream)>>>(
-      hidden, hidden, partials, partial_count, size_t{rows} * elements, weight,
-      static_cast<uint16_t*>(output_bf16), elements, epsilon, zero_centered != 0);
+  with_row_slots(elements, true, [&]<int SLOTS>(std::integral_constant<int, SLOTS>,
+                                                uint32_t threads) {
+    rms_norm_residual_kernel<SLOTS><<<rows, threads, 0, as_stream(stream)>>>(
+        hidden, hidden, partials, partial_count, size_t{rows} * elements, weight,
+        static_cast<uint16_t*>(output_bf16), elements, epsilon, zero_centered != 0);
+  });
   return launched("residual RMSNorm");
 }
 
@@ -808,9 +871,12 @@ extern "C" int32_t qllm_rms_norm_row(const float* residual, float* sum, const fl
       !aligned(residual) || !aligned(sum) || !aligned(partials) || !aligned(output_bf16) ||
       (weight && !aligned(weight)))
     return fail(QLLM_INVALID_ARGUMENT, "invalid RMSNorm of a row");
-  rms_norm_residual_kernel<<<1, 1024, 0, as_stream(stream)>>>(
-      residual, sum, partials, count, partial_stride, weight,
-      static_cast<uint16_t*>(output_bf16), elements, epsilon, zero_centered != 0);
+  with_row_slots(elements, true, [&]<int SLOTS>(std::integral_constant<int, SLOTS>,
+                                                uint32_t threads) {
+    rms_norm_residual_kernel<SLOTS><<<1, threads, 0, as_stream(stream)>>>(
+        residual, sum, partials, count, partial_stride, weight,
+        static_cast<uint16_t*>(output_bf16), elements, epsilon, zero_centered != 0);
+  });
   return launched("RMSNorm of a row");
 }
 
@@ -827,9 +893,12 @@ extern "C" int32_t qllm_rms_norm_partials_batch(
       !aligned(sum) || !aligned(partials) || !aligned(output_bf16) ||
       (weight && !aligned(weight)))
     return fail(QLLM_INVALID_ARGUMENT, "invalid RMSNorm of partial sums");
-  rms_norm_residual_kernel<<<rows, 1024, 0, as_stream(stream)>>>(
-      residual, sum, partials, partial_count, size_t{rows} * elements, weight,
-      static_cast<uint16_t*>(output_bf16), elements, epsilon, zero_centered != 0);
+  with_row_slots(elements, true, [&]<int SLOTS>(std::integral_constant<int, SLOTS>,
+                                                uint32_t threads) {
+    rms_norm_residual_kernel<SLOTS><<<rows, threads, 0, as_stream(stream)>>>(
+        residual, sum, partials, partial_count, size_t{rows} * elements, weight,
+        static_cast<uint16_t*>(output_bf16), elements, epsilon, zero_centered != 0);
+  });
   return launched("RMSNorm of partial sums");
 }
 

@@ -220,7 +220,9 @@ def test_query_q8_quantisation_is_byte_exact(device):
     assert np.array_equal(scales.cpu().numpy(), want_scales)
 
 
-@pytest.mark.parametrize("elements,count", [(5120, 3), (256, 1), (16384, 16), (5124, 2)])
+@pytest.mark.parametrize("elements,count", [(5120, 3), (256, 1), (16384, 16), (5124, 2),
+                                            (4, 4), (4096, 9), (4100, 12), (8192, 15),
+                                            (8196, 7)])
 def test_rms_norm_residual_adds_partials_in_order(device, elements, count):
     """hidden += partial 0 + partial 1 + ... (that order, F32) and the RMSNorm
     of the sum in bf16: the sum bit for bit, the norm equal to the plain norm
