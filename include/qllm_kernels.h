@@ -610,7 +610,9 @@ typedef struct qllm_q4h_attention_launch {
   const float* query_scales;    /* NULL, or the operand scales of the same call */
   const void* const* page_table;
   void* output;                 /* [rows, query_heads, head_dim] */
-  float* partial_maxima;        /* [rows, maximum_splits, query_heads] */
+  float* partial_maxima;        /* [rows, maximum_splits, query_heads]; working
+                                   space, which a launch of one split may leave
+                                   as it is */
   float* partial_sums;          /* same */
   float* partial_outputs;       /* [rows, maximum_splits, query_heads, d] */
   uint32_t first_context_tokens;/* row r attends tokens [0, first + r) */

@@ -5,6 +5,7 @@
 
 #include "common.hpp"
 
+#include <initializer_list>
 #include <type_traits>
 
 namespace qllm {
@@ -215,6 +216,34 @@ __device__ __forceinline__ void wave_tile_range(uint32_t context_tiles,
   }
 }
 
+// Four neighbouring outputs of a row from their sums over the context and the row's
+// probability sum: divided, gated (gate: the four values of the query's second half),
+// stored in the output's type at element `index`.
+__device__ __forceinline__ void store_attention_outputs(f32x4 result, float sum,
+                                                        bool gated, f32x4 gate,
+                                                        void* output,
+                                                        uint32_t output_kind,
+                                                        size_t index) {
+  // (the quotients of one divisor: its reciprocal once, then product and remainder,
+  // which rounds as a division does; infinities have no remainder)
+  const float inverse = 1.0f / sum;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float quotient = result[i] * inverse;
+    const float refined = fmaf(fmaf(-quotient, sum, result[i]), inverse, quotient);
+    result[i] = __builtin_isfinite(quotient) ? refined : quotient;
+    if (gated) result[i] *= 1.0f / (1.0f + expf(-gate[i]));
+  }
+  if (output_kind == QLLM_OUT_BF16) {
+    uint2 packed;
+    packed.x = f32_to_bf16_bits(result[0]) | (f32_to_bf16_bits(result[1]) << 16);
+    packed.y = f32_to_bf16_bits(result[2]) | (f32_to_bf16_bits(result[3]) << 16);
+    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(output) + index) = packed;
+  } else {
+    *reinterpret_cast<f32x4*>(static_cast<float*>(output) + index) = result;
+  }
+}
+
 struct PartialTarget {
   float* partial_maxima;   // [rows, maximum_splits, query_heads]
   float* partial_sums;     // same
@@ -225,10 +254,15 @@ struct PartialTarget {
   uint32_t split;
   uint32_t group;          // query heads per KV head
   uint32_t matrix_rows;    // rows * group
+  // ONE only; gate_query: the rows whose second half gates the outputs, or null
+  void* output;            // [rows, query_heads, D]
+  uint32_t output_kind;
+  const float* gate_query;
+  uint32_t query_stride;
 };
 
 // Merges the wave states of a workgroup (of eight waves unless said otherwise) and
-// writes the split partial.
+// writes the split partial, or the outputs themselves.
 // A wave's state: per row tile rt (16 matrix rows; lane (col = lane%16, quad =
 // lane/16) owns matrix row 16*rt + col) the running maximum (log2 units) and
 // sum, and out[dt][rt] = O^T elements d = 16*dt + 4*quad .. +3 of that row.
@@ -241,7 +275,10 @@ struct PartialTarget {
 //     writes them out.
 // `pool` needs 8 KiB of LDS per wave, `summary` 512*RT bytes per wave; both may
 // overlap whatever the tile loop used (the function starts with a barrier).
-template <int D, int RT, int WAVES = kSplitWaves>
+// ONE (a launch of one split): the outputs themselves, as the combine would leave
+// them.  A parameter and not a test of `output`: with the test in every kernel
+// launches of nine splits took 2 - 4 % longer.
+template <int D, int RT, int WAVES = kSplitWaves, bool ONE = false>
 __device__ __forceinline__ void merge_wave_states(
     float (&running_max)[RT], float (&running_sum)[RT],
     f32x4 (&out)[D / 16][RT], float* pool, float2* summary, uint32_t wave,
@@ -253,6 +290,21 @@ __device__ __forceinline__ void merge_wave_states(
   static_assert(VECTORS % ROUND == 0 && ROUND % WAVES == 0, "vectors are dealt to the waves");
   const uint32_t col = lane & 15u;
   const uint32_t quad = lane >> 4;
+  // (ONE: the gates of the vectors this wave will own travel during the merge)
+  f32x4 gates[ONE ? VECTORS / WAVES : 1] = {};
+  if (ONE && target.gate_query) {
+#pragma unroll
+    for (int group_index = 0; group_index < VECTORS / WAVES; ++group_index) {
+      const uint32_t k = group_index * WAVES + wave;
+      const uint32_t matrix_row = min(16u * (k % RT) + col, target.matrix_rows - 1u);
+      const size_t record =
+          static_cast<size_t>(matrix_row / target.group) * target.query_heads +
+          target.kv_head * target.group + matrix_row % target.group;
+      gates[group_index] = *reinterpret_cast<const f32x4*>(
+          target.gate_query + record * target.query_stride + D + 16u * (k / RT) +
+          4u * quad);
+    }
+  }
   __syncthreads();  // tiles done: the LDS they used is free
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
@@ -313,13 +365,24 @@ __device__ __forceinline__ void merge_wave_states(
     if (matrix_row >= target.matrix_rows) continue;
     const uint32_t row = matrix_row / target.group;
     const uint32_t head = target.kv_head * target.group + matrix_row % target.group;
+    if constexpr (ONE) {
+      float sum = merged_sum[0];
+#pragma unroll
+      for (int other = 1; other < RT; ++other)
+        if (rt == static_cast<uint32_t>(other)) sum = merged_sum[other];
+      const size_t record = static_cast<size_t>(row) * target.query_heads + head;
+      store_attention_outputs(merged[group_index], sum, target.gate_query != nullptr,
+                              gates[group_index], target.output, target.output_kind,
+                              record * D + 16u * dt + 4u * quad);
+      continue;
+    }
     const size_t partial =
         (static_cast<size_t>(row) * target.maximum_splits + target.split) *
             target.query_heads + head;
     *reinterpret_cast<f32x4*>(target.partial_outputs + partial * D + 16u * dt +
                               4u * quad) = merged[group_index];
   }
-  if (wave != 0u || quad != 0u) return;
+  if (ONE || wave != 0u || quad != 0u) return;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const uint32_t matrix_row = 16u * rt + col;
@@ -333,5 +396,18 @@ __device__ __forceinline__ void merge_wave_states(
     target.partial_sums[partial] = merged_sum[rt];
   }
 }
+
+// What a launch reads besides the cache pages.
+struct AttentionInput {
+  const void* data;   // may be null
+  size_t bytes;
+};
+// Whether a launch's workgroups may write its outputs themselves: it has one split, the
+// outputs can be stored four at a time, and they lie over nothing that other workgroups
+// of the launch still read.  Otherwise the partials go through the combine's launch.
+bool one_split_writes_output(const void* output, uint32_t output_kind,
+                             uint32_t maximum_splits, uint32_t split_tokens,
+                             uint32_t rows, uint32_t query_heads, uint32_t head_dim,
+                             std::initializer_list<AttentionInput> inputs);
 
 }  // namespace qllm

@@ -116,6 +116,10 @@ struct F16SplitArgs {
   // Batched launch (prompt prefill): grid layer z takes rows
   // [z * batch_rows, +batch_rows) of `rows`.  0 = one batch holds all rows.
   uint32_t batch_rows;
+  // a launch of one split writes the outputs itself (null: it leaves partials)
+  void* output;
+  uint32_t output_kind;
+  uint32_t output_gated;
 };
 
 constexpr uint32_t kF16Tile = 32;  // tokens per wave step
@@ -131,8 +135,9 @@ constexpr uint32_t kF16Tile = 32;  // tokens per wave step
 //           of bank conflicts, and the score registers of a 16-token sub-tile
 //           are already the B operand.
 // D = head_dim (128 or 256), RT = 16-row tiles of rows*group query rows,
-// Q8 = the cache holds int8 codes and per-record scales instead of binary16.
-template <int D, int RT, bool Q8>
+// Q8 = the cache holds int8 codes and per-record scales instead of binary16,
+// ONE = the launch has one split, whose workgroups write the outputs themselves.
+template <int D, int RT, bool Q8, bool ONE>
 __global__ __launch_bounds__(kSplitWaves * 64) void f16_attention_split_kernel(
     const F16SplitArgs launch_args) {
   // a batched launch narrows the arguments to the batch of this grid layer
@@ -152,6 +157,10 @@ __global__ __launch_bounds__(kSplitWaves * 64) void f16_attention_split_kernel(
     args.partial_maxima = launch_args.partial_maxima + first_partial;
     args.partial_sums = launch_args.partial_sums + first_partial;
     args.partial_outputs = launch_args.partial_outputs + first_partial * D;
+    if constexpr (ONE)
+      args.output = static_cast<uint8_t*>(launch_args.output) +
+                    static_cast<size_t>(first_row) * launch_args.query_heads * D *
+                        (launch_args.output_kind == QLLM_OUT_BF16 ? 2u : 4u);
   }
   constexpr int KSTEPS = D / 32;  // k-steps of the score MFMA over head_dim
   constexpr int DT = D / 16;      // 16-wide tiles of head_dim
@@ -467,8 +476,10 @@ __global__ __launch_bounds__(kSplitWaves * 64) void f16_attention_split_kernel(
   const PartialTarget target{args.partial_maxima, args.partial_sums,
                              args.partial_outputs, args.maximum_splits,
                              args.query_heads, kv_head, split, group,
-                             matrix_rows};
-  merge_wave_states<D, RT>(running_max, running_sum, out,
+                             matrix_rows, args.output, args.output_kind,
+                             args.output_gated ? args.query : nullptr,
+                             args.query_stride};
+  merge_wave_states<D, RT, kSplitWaves, ONE>(running_max, running_sum, out,
                            reinterpret_cast<float*>(stage),
                            reinterpret_cast<float2*>(exchange), wave, lane,
                            target);
@@ -486,7 +497,7 @@ __global__ __launch_bounds__(kSplitWaves * 64) void f16_attention_split_kernel(
 // the choice of which global granule a lane fetches for its LDS slot: K row r
 // keeps granule g at g ^ (r & 15) (the A-operand read takes one granule from
 // each of 16 consecutive rows), V row t at g ^ (2 * (t & 7)) as above.
-template <int RT>
+template <int RT, bool ONE>
 __global__ __launch_bounds__(kSplitWaves * 64) void f16_attention_split_d128_kernel(
     const F16SplitArgs args) {
   constexpr int D = 128;
@@ -742,44 +753,64 @@ __global__ __launch_bounds__(kSplitWaves * 64) void f16_attention_split_d128_ker
   const PartialTarget target{args.partial_maxima, args.partial_sums,
                              args.partial_outputs, args.maximum_splits,
                              args.query_heads, kv_head, split, group,
-                             matrix_rows};
-  merge_wave_states<D, RT>(running_max, running_sum, out,
+                             matrix_rows, args.output, args.output_kind,
+                             args.output_gated ? args.query : nullptr,
+                             args.query_stride};
+  merge_wave_states<D, RT, kSplitWaves, ONE>(running_max, running_sum, out,
                            reinterpret_cast<float*>(stage),
                            reinterpret_cast<float2*>(exchange), wave, lane,
                            target);
 }
 
-int32_t launch_f16_split_d128(const F16SplitArgs& args, uint32_t row_tiles,
-                              dim3 grid, hipStream_t stream) {
+// Whether workgroups of a single split write the outputs themselves: not with two row
+// tiles at head_dim 256, whose sixteen gated outputs a lane take one workgroup a KV head
+// longer than the combine's launch (30 matrix rows over 60 tokens 13.2 -> 14.0 us; two
+// rows of 24 heads on 4 9.6 -> 8.8, five of 16 heads on 4 at head_dim 128 8.6 -> 7.2).
+bool writes_one_split(uint32_t head_dim, uint32_t row_tiles) {
+  return head_dim == 128u || row_tiles == 1u;
+}
+
+template <bool ONE>
+int32_t launch_f16_split_d128_of(const F16SplitArgs& args, uint32_t row_tiles,
+                                 dim3 grid, hipStream_t stream) {
   switch (row_tiles) {
     case 1:
-      f16_attention_split_d128_kernel<1><<<grid, kSplitWaves * 64, 0, stream>>>(args);
+      f16_attention_split_d128_kernel<1, ONE>
+          <<<grid, kSplitWaves * 64, 0, stream>>>(args);
       break;
     case 2:
-      f16_attention_split_d128_kernel<2><<<grid, kSplitWaves * 64, 0, stream>>>(args);
+      f16_attention_split_d128_kernel<2, ONE>
+          <<<grid, kSplitWaves * 64, 0, stream>>>(args);
       break;
     default:
-      f16_attention_split_d128_kernel<3><<<grid, kSplitWaves * 64, 0, stream>>>(args);
+      f16_attention_split_d128_kernel<3, ONE>
+          <<<grid, kSplitWaves * 64, 0, stream>>>(args);
       break;
   }
   return launched("F16 attention split");
 }
 
-template <int D, bool Q8 = false>
-int32_t launch_f16_split(const F16SplitArgs& args, uint32_t row_tiles, dim3 grid,
-                         hipStream_t stream) {
+int32_t launch_f16_split_d128(const F16SplitArgs& args, uint32_t row_tiles,
+                              dim3 grid, hipStream_t stream) {
+  return args.output ? launch_f16_split_d128_of<true>(args, row_tiles, grid, stream)
+                     : launch_f16_split_d128_of<false>(args, row_tiles, grid, stream);
+}
+
+template <int D, bool Q8, bool ONE>
+int32_t launch_f16_split_of(const F16SplitArgs& args, uint32_t row_tiles, dim3 grid,
+                            hipStream_t stream) {
   switch (row_tiles) {
     case 1:
-      f16_attention_split_kernel<D, 1, Q8>
+      f16_attention_split_kernel<D, 1, Q8, ONE>
           <<<grid, kSplitWaves * 64, 0, stream>>>(args);
       break;
     case 2:
-      f16_attention_split_kernel<D, 2, Q8>
+      f16_attention_split_kernel<D, 2, Q8, ONE>
           <<<grid, kSplitWaves * 64, 0, stream>>>(args);
       break;
     default:
       if constexpr (D == 128) {
-        f16_attention_split_kernel<D, 3, Q8>
+        f16_attention_split_kernel<D, 3, Q8, ONE>
             <<<grid, kSplitWaves * 64, 0, stream>>>(args);
         break;
       } else {
@@ -788,6 +819,13 @@ int32_t launch_f16_split(const F16SplitArgs& args, uint32_t row_tiles, dim3 grid
       }
   }
   return launched("F16 attention split");
+}
+
+template <int D, bool Q8 = false>
+int32_t launch_f16_split(const F16SplitArgs& args, uint32_t row_tiles, dim3 grid,
+                         hipStream_t stream) {
+  return args.output ? launch_f16_split_of<D, Q8, true>(args, row_tiles, grid, stream)
+                     : launch_f16_split_of<D, Q8, false>(args, row_tiles, grid, stream);
 }
 
 }  // namespace
@@ -874,13 +912,23 @@ extern "C" int32_t qllm_attention_paged_f16(
   args.kv_heads = launch->kv_heads;
   args.split_tokens = launch->split_tokens;
   args.maximum_splits = launch->maximum_splits;
+  if (writes_one_split(launch->head_dim, row_tiles) &&
+      one_split_writes_output(
+          launch->output, launch->output_kind, launch->maximum_splits,
+          launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
+          {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
+                               launch->query_stride}})) {
+    args.output = launch->output;
+    args.output_kind = launch->output_kind;
+    args.output_gated = launch->output_gated != 0 ? 1u : 0u;
+  }
   const dim3 grid(launch->kv_heads, splits);
   const hipStream_t stream = as_stream(launch->stream);
   const int32_t status =
       launch->head_dim == 128u
           ? launch_f16_split_d128(args, row_tiles, grid, stream)
           : launch_f16_split<256>(args, row_tiles, grid, stream);
-  if (status != QLLM_OK) return status;
+  if (status != QLLM_OK || args.output) return status;
   return launch_attention_combine(
       launch->query, launch->query_stride, launch->output_gated,
       launch->partial_maxima, launch->partial_sums, launch->partial_outputs,
@@ -941,13 +989,23 @@ extern "C" int32_t qllm_attention_paged_f16_batched(
   args.kv_heads = launch->kv_heads;
   args.split_tokens = launch->split_tokens;
   args.maximum_splits = launch->maximum_splits;
+  if (writes_one_split(launch->head_dim, row_tiles) &&
+      one_split_writes_output(
+          launch->output, launch->output_kind, launch->maximum_splits,
+          launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
+          {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
+                               launch->query_stride}})) {
+    args.output = launch->output;
+    args.output_kind = launch->output_kind;
+    args.output_gated = launch->output_gated != 0 ? 1u : 0u;
+  }
   args.batch_rows = batch_rows;
   const dim3 grid(launch->kv_heads, splits, batches);
   const hipStream_t stream = as_stream(launch->stream);
   const int32_t status =
       launch->head_dim == 128u ? launch_f16_split<128>(args, row_tiles, grid, stream)
                                : launch_f16_split<256>(args, row_tiles, grid, stream);
-  if (status != QLLM_OK) return status;
+  if (status != QLLM_OK || args.output) return status;
   return launch_attention_combine(
       launch->query, launch->query_stride, launch->output_gated,
       launch->partial_maxima, launch->partial_sums, launch->partial_outputs,
@@ -1040,6 +1098,16 @@ extern "C" int32_t qllm_attention_paged_q8(const qllm_q8_attention_launch* launc
   args.kv_heads = launch->kv_heads;
   args.split_tokens = launch->split_tokens;
   args.maximum_splits = launch->maximum_splits;
+  if (writes_one_split(launch->head_dim, row_tiles) &&
+      one_split_writes_output(
+          launch->output, launch->output_kind, launch->maximum_splits,
+          launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
+          {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
+                               launch->query_stride}})) {
+    args.output = launch->output;
+    args.output_kind = launch->output_kind;
+    args.output_gated = launch->output_gated != 0 ? 1u : 0u;
+  }
   args.page_offset = launch->page_offset_bytes;
   args.device_positions = launch->device_positions;
   const dim3 grid(launch->kv_heads, splits);
@@ -1048,7 +1116,7 @@ extern "C" int32_t qllm_attention_paged_q8(const qllm_q8_attention_launch* launc
       launch->head_dim == 128u
           ? launch_f16_split<128, true>(args, row_tiles, grid, stream)
           : launch_f16_split<256, true>(args, row_tiles, grid, stream);
-  if (status != QLLM_OK) return status;
+  if (status != QLLM_OK || args.output) return status;
   return launch_attention_combine(
       launch->query, launch->query_stride, launch->output_gated,
       launch->partial_maxima, launch->partial_sums, launch->partial_outputs,
@@ -1108,6 +1176,16 @@ extern "C" int32_t qllm_attention_paged_q8_batched(
   args.kv_heads = launch->kv_heads;
   args.split_tokens = launch->split_tokens;
   args.maximum_splits = launch->maximum_splits;
+  if (writes_one_split(launch->head_dim, row_tiles) &&
+      one_split_writes_output(
+          launch->output, launch->output_kind, launch->maximum_splits,
+          launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
+          {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
+                               launch->query_stride}})) {
+    args.output = launch->output;
+    args.output_kind = launch->output_kind;
+    args.output_gated = launch->output_gated != 0 ? 1u : 0u;
+  }
   args.page_offset = launch->page_offset_bytes;
   args.batch_rows = batch_rows;
   const dim3 grid(launch->kv_heads, splits, batches);
@@ -1116,7 +1194,7 @@ extern "C" int32_t qllm_attention_paged_q8_batched(
       launch->head_dim == 128u
           ? launch_f16_split<128, true>(args, row_tiles, grid, stream)
           : launch_f16_split<256, true>(args, row_tiles, grid, stream);
-  if (status != QLLM_OK) return status;
+  if (status != QLLM_OK || args.output) return status;
   return launch_attention_combine(
       launch->query, launch->query_stride, launch->output_gated,
       launch->partial_maxima, launch->partial_sums, launch->partial_outputs,

@@ -113,6 +113,10 @@ struct SplitArgs {
   float epsilon;
   uint32_t first_cache_position;   // or device_positions[0]
   uint32_t bf16_activations;
+  // a launch of one split writes the outputs itself (null: it leaves partials)
+  void* output;
+  uint32_t output_kind;
+  uint32_t output_gated;
 };
 
 
@@ -423,7 +427,11 @@ __global__ void rope_table_kernel(float2* table, uint32_t rotary_dim,
 // the staged tile before it is read (the cache pages need not hold them yet);
 // the workgroup that owns the context's last tile also writes them to the
 // pages for later steps.
-template <int D, int RT, bool FUSED = false>
+//
+// ONE: the launch has one split, whose workgroups write the outputs themselves; the
+// partials and the combine's launch go (fused, five rows of 16 heads on 4, 60 tokens
+// 12.6 -> 11.3 us in a replayed graph, of 64 heads on 8 15.2 -> 14.6).
+template <int D, int RT, bool FUSED = false, bool ONE = false>
 __global__ __launch_bounds__(kSplitWaves * 64, 2) void q4h_attention_split_kernel(
     const SplitArgs launch_args) {
   constexpr int WAVES = kSplitWaves;
@@ -444,6 +452,10 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void q4h_attention_split_kerne
     args.partial_maxima = launch_args.partial_maxima + first_partial;
     args.partial_sums = launch_args.partial_sums + first_partial;
     args.partial_outputs = launch_args.partial_outputs + first_partial * D;
+    if constexpr (ONE)
+      args.output = static_cast<uint8_t*>(launch_args.output) +
+                    static_cast<size_t>(first_row) * launch_args.query_heads * D *
+                        (launch_args.output_kind == QLLM_OUT_BF16 ? 2u : 4u);
   }
   // Everything the prologue reads from the argument block is asked for here,
   // in one round trip, not piece by piece along its chain of dependencies.
@@ -498,10 +510,11 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void q4h_attention_split_kerne
   // (fused: the workgroup at the end of the context also encodes the batch's
   // K/V records, lays them over its tiles and writes them to their pages -
   // about two tiles' worth of time for each of its waves.  The plain kernel
-  // deals the same way, so that both add up a context in the same order.)
-  constexpr uint32_t kTailWork = 2u * kSplitWaves;
+  // deals the same way, so that both add up a context in the same order.  Where
+  // one workgroup has the whole context every wave has that work.)
+  const uint32_t tail_work = ONE || gridDim.y == 1u ? 0u : 2u * kSplitWaves;
   wave_tile_range<WAVES>(context_tiles, 64u, args.split_tokens, split, gridDim.y, wave,
-                         tile_first, tile_last, kTailWork);
+                         tile_first, tile_last, tail_work);
 
   // the wave's staging areas: tile t of the wave uses area t % DEPTH
   uint8_t* const stage_base = stage + wave * (STAGE * DEPTH);
@@ -669,9 +682,9 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void q4h_attention_split_kerne
     }
     uint32_t workgroup_first, workgroup_last, unused;
     wave_tile_range(context_tiles, 64u, args.split_tokens, split, gridDim.y, 0u,
-                    workgroup_first, unused, kTailWork);
+                    workgroup_first, unused, tail_work);
     wave_tile_range(context_tiles, 64u, args.split_tokens, split, gridDim.y,
-                    kSplitWaves - 1u, unused, workgroup_last, kTailWork);
+                    kSplitWaves - 1u, unused, workgroup_last, tail_work);
     reaches_batch = workgroup_first < workgroup_last &&
                     workgroup_last * 64u > first_cache_position;
     // the wave's first tiles set out first: the work below hides behind them
@@ -1312,8 +1325,10 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void q4h_attention_split_kerne
   const PartialTarget target{args.partial_maxima, args.partial_sums,
                              args.partial_outputs, args.maximum_splits,
                              args.query_heads, kv_head, split, group,
-                             matrix_rows};
-  merge_wave_states<D, RT, WAVES>(running_max, running_sum, out,
+                             matrix_rows, args.output, args.output_kind,
+                             args.output_gated ? args.query : nullptr,
+                             args.query_stride};
+  merge_wave_states<D, RT, WAVES, ONE>(running_max, running_sum, out,
                                   reinterpret_cast<float*>(stage),
                                   reinterpret_cast<float2*>(exchange), wave, lane,
                                   target);
@@ -1355,7 +1370,7 @@ constexpr int kPromptBatches = 8;
 // codes are 128 bytes there, so their 16-byte pieces are swizzled by the row.  3001
 // rows of 24 heads on 4: 281 us with a workgroup of two waves for every five rows,
 // each of which converted its own V codes, 197 here.
-template <int D>
+template <int D, bool ONE = false>
 __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kernel(
     const SplitArgs args) {
   constexpr bool WIDE = D == 256;
@@ -1859,6 +1874,19 @@ __global__ __launch_bounds__(kPromptBatches * 64) void q4h_prompt_attention_kern
     if (matrix_row >= matrix_rows) continue;
     const uint32_t row = (first_matrix_row + matrix_row) / group;
     const uint32_t head = kv_head * group + (first_matrix_row + matrix_row) % group;
+    if constexpr (ONE) {
+      const size_t record = static_cast<size_t>(row) * args.query_heads + head;
+      const float* gate_row = args.query + record * args.query_stride + D + 4u * quad;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        f32x4 gate = {};
+        if (args.output_gated) gate = *reinterpret_cast<const f32x4*>(gate_row + 16 * dt);
+        store_attention_outputs(out[dt][rt], running_sum[rt], args.output_gated != 0u,
+                                gate, args.output, args.output_kind,
+                                record * D + 16u * dt + 4u * quad);
+      }
+      continue;
+    }
     const size_t partial =
         (static_cast<size_t>(row) * args.maximum_splits + split) * args.query_heads +
         head;
@@ -2044,19 +2072,8 @@ __global__ __launch_bounds__(256) void attention_few_splits_kernel(
       for (uint32_t s = 0; s < step; ++s) sums[s] += sums[s + step];
     sum = sums[0];
   }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    result[i] /= sum;
-    if (output_gated) result[i] *= 1.0f / (1.0f + expf(-gate[i]));
-  }
-  if (output_kind == QLLM_OUT_BF16) {
-    uint2 packed;
-    packed.x = f32_to_bf16_bits(result[0]) | (f32_to_bf16_bits(result[1]) << 16);
-    packed.y = f32_to_bf16_bits(result[2]) | (f32_to_bf16_bits(result[3]) << 16);
-    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(output) + index) = packed;
-  } else {
-    *reinterpret_cast<f32x4*>(static_cast<float*>(output) + index) = result;
-  }
+  store_attention_outputs(result, sum, output_gated != 0, gate, output, output_kind,
+                          index);
 }
 
 // ---- K/V store ----------------------------------------------------------------
@@ -2417,22 +2434,22 @@ __global__ __launch_bounds__(64) void quantize_queries_q8_kernel(
   }
 }
 
-template <int D, bool FUSED = false>
-int32_t launch_split(const SplitArgs& args, uint32_t row_tiles, dim3 grid,
-                     hipStream_t stream) {
+template <int D, bool FUSED, bool ONE>
+int32_t launch_split_of(const SplitArgs& args, uint32_t row_tiles, dim3 grid,
+                        hipStream_t stream) {
   const size_t lds = 0;  // all LDS of the split kernel is static
   switch (row_tiles) {
     case 1:
-      q4h_attention_split_kernel<D, 1, FUSED>
+      q4h_attention_split_kernel<D, 1, FUSED, ONE>
           <<<grid, kSplitWaves * 64, lds, stream>>>(args);
       break;
     case 2:
-      q4h_attention_split_kernel<D, 2, FUSED>
+      q4h_attention_split_kernel<D, 2, FUSED, ONE>
           <<<grid, kSplitWaves * 64, lds, stream>>>(args);
       break;
     default:
       if constexpr (D == 128) {
-        q4h_attention_split_kernel<D, 3, FUSED>
+        q4h_attention_split_kernel<D, 3, FUSED, ONE>
             <<<grid, kSplitWaves * 64, lds, stream>>>(args);
         break;
       } else {
@@ -2443,9 +2460,32 @@ int32_t launch_split(const SplitArgs& args, uint32_t row_tiles, dim3 grid,
   return launched("Q4H attention split");
 }
 
+template <int D, bool FUSED = false>
+int32_t launch_split(const SplitArgs& args, uint32_t row_tiles, dim3 grid,
+                     hipStream_t stream) {
+  return args.output ? launch_split_of<D, FUSED, true>(args, row_tiles, grid, stream)
+                     : launch_split_of<D, FUSED, false>(args, row_tiles, grid, stream);
+}
+
 }  // namespace
 
 // shared with the exact-F16 path
+bool one_split_writes_output(const void* output, uint32_t output_kind,
+                             uint32_t maximum_splits, uint32_t split_tokens,
+                             uint32_t rows, uint32_t query_heads, uint32_t head_dim,
+                             std::initializer_list<AttentionInput> inputs) {
+  if (maximum_splits != 1u || split_tokens) return false;
+  const uintptr_t begin = reinterpret_cast<uintptr_t>(output);
+  if (begin & 15u) return false;
+  const uintptr_t end = begin + static_cast<size_t>(rows) * query_heads * head_dim *
+                                    (output_kind == QLLM_OUT_BF16 ? 2u : 4u);
+  for (const AttentionInput& input : inputs) {
+    const uintptr_t first = reinterpret_cast<uintptr_t>(input.data);
+    if (input.data && begin < first + input.bytes && first < end) return false;
+  }
+  return true;
+}
+
 int32_t launch_attention_combine(const float* query, uint32_t query_stride,
                                  int output_gated, const float* partial_maxima,
                                  const float* partial_sums,
@@ -2760,6 +2800,14 @@ uint32_t shared_parts(const qllm_q4h_attention_launch& launch) {
 // 5500 launches over eight head layouts (24 on 4, 16 on 8, 16 on 2, 64 on 8, 16 on 16,
 // 8 on 1, 24 on 2, 32 on 32), 2 to 3000 rows after 0 to 9000 tokens, one to eight
 // splits: 5 and 9 % root mean square error.
+// From this many workgroups of shared tiles on they write the outputs of a single split
+// themselves.  64 heads on 8 at head_dim 128: 6000 rows (1000 workgroups) 792 -> 749 us,
+// 1000 (168) 80.6 -> 75.8, 400 (72) 42.0 -> 41.0, but 300 (56) 36.9 -> 37.6 and 200 (40)
+// 29.2 -> 31.0: a few workgroups take longer over the divisions and the 32-byte pieces
+// of their rows than a launch over all compute units.  (At head_dim 256, whose rows are
+// gated, 3001 rows of 24 heads on 4 in 564 workgroups gain nothing: the combine stays.)
+constexpr uint32_t kDirectWorkgroups = 64u;
+
 struct LaunchTiles {
   double rounds;     // of workgroups over the compute units
   double longest;    // tiles of the last rows' workgroup
@@ -2874,10 +2922,21 @@ int32_t attend_batches(const qllm_q4h_attention_launch* launch, uint32_t batch_r
   args.split_tokens = launch->split_tokens;
   args.maximum_splits = launch->maximum_splits;
   args.batch_rows = batch_rows;
+  const bool shares = any_order && shares_tiles(*launch, batch_rows);
+  if (!shares &&
+      one_split_writes_output(
+          launch->output, launch->output_kind, launch->maximum_splits,
+          launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
+          {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
+                               launch->query_stride}})) {
+    args.output = launch->output;
+    args.output_kind = launch->output_kind;
+    args.output_gated = launch->output_gated != 0 ? 1u : 0u;
+  }
   const dim3 grid(launch->kv_heads, splits, batches);
   const hipStream_t stream = as_stream(launch->stream);
   int32_t status = QLLM_OK;
-  if (any_order && shares_tiles(*launch, batch_rows)) {
+  if (shares) {
     const uint32_t parts = shared_parts(*launch);
     q4h_prompt_attention_kernel<256>
         <<<dim3(launch->kv_heads, splits, parts), kPromptBatches * 64, 0, stream>>>(args);
@@ -2886,7 +2945,7 @@ int32_t attend_batches(const qllm_q4h_attention_launch* launch, uint32_t batch_r
     status = launch->head_dim == 128u ? launch_split<128>(args, row_tiles, grid, stream)
                                       : launch_split<256>(args, row_tiles, grid, stream);
   }
-  if (status != QLLM_OK) return status;
+  if (status != QLLM_OK || args.output) return status;
   // partials are laid out by global row, which is what the combine indexes
   return launch_attention_combine(
       launch->query, launch->query_stride, launch->output_gated,
@@ -2979,12 +3038,26 @@ extern "C" int32_t qllm_attention_paged_q4h_prompt(
   args.kv_heads = launch->kv_heads;
   args.maximum_splits = launch->maximum_splits;
   args.batch_rows = batch_rows;
-  const dim3 grid(launch->kv_heads, launch->maximum_splits,
-                  (batches + kPromptBatches - 1u) / kPromptBatches);
+  const uint32_t parts = (batches + kPromptBatches - 1u) / kPromptBatches;
+  if (launch->kv_heads * parts >= kDirectWorkgroups &&
+      one_split_writes_output(
+          launch->output, launch->output_kind, launch->maximum_splits,
+          launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
+          {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
+                               launch->query_stride}})) {
+    args.output = launch->output;
+    args.output_kind = launch->output_kind;
+    args.output_gated = launch->output_gated != 0 ? 1u : 0u;
+  }
+  const dim3 grid(launch->kv_heads, launch->maximum_splits, parts);
   const hipStream_t stream = as_stream(launch->stream);
-  q4h_prompt_attention_kernel<128><<<grid, kPromptBatches * 64, 0, stream>>>(args);
+  if (args.output)
+    q4h_prompt_attention_kernel<128, true>
+        <<<grid, kPromptBatches * 64, 0, stream>>>(args);
+  else
+    q4h_prompt_attention_kernel<128><<<grid, kPromptBatches * 64, 0, stream>>>(args);
   const int32_t status = launched("Q4H prompt attention");
-  if (status != QLLM_OK) return status;
+  if (status != QLLM_OK || args.output) return status;
   return launch_attention_combine(
       launch->query, launch->query_stride, launch->output_gated,
       launch->partial_maxima, launch->partial_sums, launch->partial_outputs,
@@ -3054,6 +3127,26 @@ int32_t launch_q4h_attention(const qllm_q4h_attention_launch* launch,
   args.split_tokens = launch->split_tokens;
   args.maximum_splits = launch->maximum_splits;
   args.device_positions = launch->device_positions;
+  const size_t width = size_t{launch->kv_heads} * launch->head_dim;
+  if (one_split_writes_output(
+          launch->output, launch->output_kind, launch->maximum_splits,
+          launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
+          {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
+                               launch->query_stride},
+           {args.query_operands,
+            launch->kv_heads * q4h_operand_plane_bytes(row_tiles, launch->head_dim)},
+           {args.query_operand_scales, sizeof(float) * 16u * row_tiles * launch->kv_heads},
+           {rope ? rope->key : nullptr, sizeof(float) * launch->rows * width},
+           {rope ? rope->value : nullptr, sizeof(float) * launch->rows * width},
+           {rope ? rope->q_norm_weight : nullptr, sizeof(float) * launch->head_dim},
+           {rope ? rope->k_norm_weight : nullptr, sizeof(float) * launch->head_dim},
+           {rope ? rope->rope_table : nullptr,
+            rope ? sizeof(float) * launch->rows * rope->rotary_dim : 0u},
+           {launch->device_positions, 3u * sizeof(uint32_t)}})) {
+    args.output = launch->output;
+    args.output_kind = launch->output_kind;
+    args.output_gated = launch->output_gated != 0 ? 1u : 0u;
+  }
   const dim3 grid(launch->kv_heads, splits);
   const hipStream_t stream = as_stream(launch->stream);
   int32_t status;
@@ -3083,7 +3176,7 @@ int32_t launch_q4h_attention(const qllm_q4h_attention_launch* launch,
                  ? launch_split<128>(args, row_tiles, grid, stream)
                  : launch_split<256>(args, row_tiles, grid, stream);
   }
-  if (status != QLLM_OK) return status;
+  if (status != QLLM_OK || args.output) return status;
   return launch_attention_combine(
       launch->query, launch->query_stride, launch->output_gated,
       launch->partial_maxima, launch->partial_sums, launch->partial_outputs,

@@ -265,6 +265,14 @@ void Mi355DenseFp4Provider::allocate_workspaces() {
   split_tokens_ = 0U;
   maximum_splits_ =
       std::min(wanted_splits, std::max(1U, (g_.max_context + 511U) / 512U));
+  prefill_splits_ = std::min(maximum_splits_, 8U);
+  q4h_splits_ = maximum_splits_;
+  // One split of a Q4H launch writes the outputs itself.  Five rows of 16 heads on 4 after
+  // 500 and 760 tokens: 12.9 and 16.1 us against 15.7 and 17.8 with two splits; at 1000
+  // tokens 16.3 against 15.5 with three, at head_dim 256 and 760 tokens 28.3 with either.
+  if (g_.kv_encoding == KvEncoding::q4_f16_per_head && g_.head_dim == 128U &&
+      g_.max_context <= 768U)
+    q4h_splits_ = 1U;
   const std::size_t partials = rows * maximum_splits_ * g_.query_heads;
   partial_maxima_ = static_cast<float*>(device_alloc(partials * 4U));
   partial_sums_ = static_cast<float*>(device_alloc(partials * 4U));
@@ -1220,7 +1228,7 @@ void Mi355DenseFp4Provider::enqueue_attention(
     launch.kv_heads = g_.kv_heads;
     launch.head_dim = g_.head_dim;
     launch.split_tokens = split_tokens_;
-    launch.maximum_splits = maximum_splits_;
+    launch.maximum_splits = q4h_splits_;
     launch.query_stride = query_stride;
     launch.output_gated = g_.output_gated;
     launch.output_kind = g_.activation_q8 ? QLLM_OUT_F32 : QLLM_OUT_BF16;
@@ -1706,9 +1714,8 @@ void Mi355DenseFp4Provider::ensure_prefill_workspace(std::uint32_t rows) {
   prefill_activation_ = static_cast<std::uint16_t*>(allocate(
       n * std::max<std::size_t>(g_.intermediate, 2U * g_.hidden) * 2U));
   {
-    // fewer splits than the verify step: the row batches of a chunk already
-    // fill the GPU, and the partials are per row
-    prefill_splits_ = std::min<std::uint32_t>(maximum_splits_, 8U);
+    // (prefill_splits_ is at most 8: the row batches of a chunk already fill the
+    // GPU, and the partials are per row)
     // partial rows: the most rows x splits any chunk of up to n rows asks for
     // (long chunks are not cut, short ones have few rows)
     const std::uint32_t attention_batch = std::max(
@@ -2276,7 +2283,7 @@ er::Status Mi355DenseFp4Provider::time_kernel(const std::string& which,
         launch.kv_heads = g_.kv_heads;
         launch.head_dim = g_.head_dim;
         launch.split_tokens = split_tokens_;
-        launch.maximum_splits = maximum_splits_;
+        launch.maximum_splits = q4h_splits_;
         launch.query_stride = query_stride;
         launch.output_gated = g_.output_gated;
         launch.output_kind = QLLM_OUT_BF16;

@@ -428,6 +428,7 @@ class Mi355DenseFp4Provider final : public DecoderProvider {
   std::uint64_t mtp_page_offset_{};   // the proposer's Q8 layer inside a page
   std::uint32_t split_tokens_{};
   std::uint32_t maximum_splits_{};
+  std::uint32_t q4h_splits_{};      // of a verify step over the Q4H cache
 
   // workspaces (device)
   std::uint32_t max_rows_{};

@@ -627,3 +627,46 @@ def test_rotary_and_store_from_a_table_equal_their_own_angles(
         qh.call("qllm_qkv_rope_table_batch", qh.ptr(query), stride, qh.ptr(key),
                 qh.ptr(value), None, None, qh.ptr(table), None, 0, 0, 64, 0, rows, heads, kv,
                 64, 64, eps, 0, None)
+
+
+@pytest.mark.parametrize("tokens,rows,Q,KV,d,gated,kind", [
+    (5, 5, 16, 4, 128, False, qh.OUT_BF16),      # the batch is the whole context
+    (64, 2, 16, 4, 128, True, qh.OUT_F32), (65, 4, 8, 8, 128, False, qh.OUT_BF16),
+    (513, 5, 64, 8, 128, True, qh.OUT_BF16), (1030, 5, 64, 8, 128, False, qh.OUT_F32),
+    (300, 5, 24, 4, 256, True, qh.OUT_BF16), (70, 2, 24, 4, 256, False, qh.OUT_F32)])
+def test_one_split_writes_what_the_combine_would(device, tokens, rows, Q, KV, d, gated, kind):
+    """A fused launch of one split into a buffer of its own, and off a 16-byte line or
+    over its table, where the combine writes the outputs: the same bits."""
+    rng = np.random.default_rng(tokens + Q)
+    page, rotary, first = 64, 64, tokens - (rows - 1)
+    pages = synth.q4h_pages(rng.standard_normal((tokens, KV, d)).astype(np.float32),
+                            rng.standard_normal((tokens, KV, d)).astype(np.float32), page, 1, 0)
+    stride = d * (2 if gated else 1)
+    d_q = gu.device_tensor(rng.standard_normal((rows, Q, stride)).astype(np.float32), device)
+    d_k, d_v = (gu.device_tensor(rng.standard_normal((rows, KV, d)).astype(np.float32), device)
+                for _ in range(2))
+    maxima, sums = torch.zeros((2, rows, 1, Q), device=device)
+    partials = torch.zeros((rows, 1, Q, d), device=device)
+    type_ = torch.bfloat16 if kind == qh.OUT_BF16 else torch.float32
+    got = []
+    for where in ("own", "shifted", "over the table"):
+        d_pages = [gu.device_tensor(p, device) for p in pages]
+        table = torch.tensor([p.data_ptr() for p in d_pages], dtype=torch.int64, device=device)
+        out = torch.zeros(rows * Q * d + 16, dtype=type_, device=device)
+        begin = 2 if where == "shifted" else 0
+        cos_sin = (out.view(torch.float32) if where == "over the table"
+                   else torch.zeros(rows * rotary, device=device))
+        qh.call("qllm_rope_table", qh.ptr(cos_sin), rows, rotary, first - 1, 1e6, 0, None, None)
+        launch = qh.Q4hAttentionLaunch(
+            qh.ptr(d_q), 0, 0, qh.ptr(table), out.data_ptr() + begin * out.element_size(),
+            qh.ptr(maxima), qh.ptr(sums), qh.ptr(partials), first, rows, 0, page, Q, KV, d, 0, 1,
+            stride, int(gated), kind, None)
+        rope = qh.Q4hFusedRope(qh.ptr(d_k), qh.ptr(d_v), 0, 0, qh.ptr(cos_sin), rotary, 1e-6,
+                               first - 1, 0)
+        partials.fill_(-1.0)
+        qh.call("qllm_attention_paged_q4h_fused", launch, rope)
+        torch.cuda.synchronize()
+        assert bool((partials == -1.0).all()) == (where == "own")
+        got.append(out[begin:begin + rows * Q * d].float().cpu().numpy())
+    assert np.abs(got[0]).max() > 0.0
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
