@@ -722,6 +722,14 @@ uint32_t qllm_attention_paged_q4h_shared_splits(
     const qllm_q4h_attention_launch* launch, uint32_t batch_rows, uint32_t batch_splits,
     uint32_t most);
 
+/* The form and the splits, 1 to `most`, with which a prompt's launch at head_dim 128
+ * (split_tokens 0) takes the least time: 1 for qllm_attention_paged_q4h_prompt, 0 for
+ * qllm_attention_paged_q4h_batched.  Reads the launch's sizes alone; *splits is 0 for
+ * sizes that neither takes. */
+uint32_t qllm_attention_paged_q4h_prompt_form(
+    const qllm_q4h_attention_launch* launch, uint32_t batch_rows, uint32_t most,
+    uint32_t* splits);
+
 /* The same attention for a long run of prompt rows (head_dim 128,
  * split_tokens 0): eight consecutive batches share a workgroup, which fetches
  * every cache tile once for the eight and converts its V codes and scales to

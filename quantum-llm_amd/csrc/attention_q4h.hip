@@ -2869,6 +2869,59 @@ bool shares_tiles(const qllm_q4h_attention_launch& launch, uint32_t batch_rows) 
              batched_us(launch, batch_rows, launch.maximum_splits);
 }
 
+// partial outputs written and read, and the launch; a single split has none
+double combine_128_us(const qllm_q4h_attention_launch& launch, uint32_t splits) {
+  return splits == 1u ? 0.0
+                      : 2.0 + static_cast<double>(launch.rows) * launch.query_heads *
+                                  splits * 820.0 / 5.3e6;
+}
+
+// A prompt's attention at head_dim 128: as batches of
+// their own, whose workgroups (82 KiB of LDS, one to a compute unit) deal a context's
+// tiles over eight waves, or as shared tiles, eight batches to a workgroup.  Fitted to
+// 320 sizes (9 to 2500 rows after 1 to 8000 tokens; 64 heads on 8, 16 on 4, 32 on 32 and
+// on 8) with 1 to 8 splits: the choice takes 0.3 % longer than the best one on average
+// and 7 % at most.  Batches of their own up to 31 of them, splits for one workgroup a
+// compute unit rounded up, took 19 % on average and 3.1 times at most: 256 workgroups
+// and a few more are two rounds (120 rows of 64 heads after 2048 tokens 42.6 us in two
+// splits, 30.8 in one), and a few hundred rows fill the chip in batches of their own
+// (300 rows from the first on 38 us shared, 27 so).
+double batches_128_us(const qllm_q4h_attention_launch& launch, uint32_t batch_rows,
+                      uint32_t splits) {
+  const uint32_t group = launch.query_heads / launch.kv_heads;
+  const uint32_t first_rows = std::min(batch_rows, launch.rows);
+  const uint64_t batches = (uint64_t{launch.rows} + batch_rows - 1u) / batch_rows;
+  const uint64_t rounds = (batches * launch.kv_heads * splits + 255u) / 256u;
+  const auto walked = [&](uint64_t rows) {
+    const double tiles =
+        static_cast<double>((launch.first_context_tokens + rows + 62u) / 64u);
+    if (splits == 1u) return std::ceil(tiles / kSplitWaves);
+    // (the deal of the split kernel; its last waves walk fewer)
+    const double share = (tiles + 2.0 * kSplitWaves) / (kSplitWaves * splits);
+    return 0.75 * std::ceil(share - 0.03) + 0.25 * share;
+  };
+  const double longest = walked(launch.rows);
+  const double each = rounds == 1u ? longest : 0.5 * (longest + walked(first_rows));
+  const uint32_t row_tiles = std::min((first_rows * group + 15u) / 16u, 3u);
+  const double base[] = {6.0, 7.5, 9.0}, tile[] = {2.3, 3.1, 3.75};
+  return static_cast<double>(rounds) *
+             (base[row_tiles - 1u] + tile[row_tiles - 1u] * each) +
+         combine_128_us(launch, splits);
+}
+
+double shared_128_us(const qllm_q4h_attention_launch& launch, uint32_t batch_rows,
+                     uint32_t splits) {
+  const uint64_t batches = (uint64_t{launch.rows} + batch_rows - 1u) / batch_rows;
+  const uint64_t parts = (batches + kPromptBatches - 1u) / kPromptBatches;
+  const LaunchTiles t =
+      tiles_of_launch(launch, parts * launch.kv_heads * splits,
+                      uint64_t{batch_rows} * kPromptBatches, splits);
+  // (from five waves on two share a SIMD)
+  return 9.0 + 5.0 * t.rounds +
+         (batches > 4u ? 3.5 : 2.0) * std::max(std::ceil(t.longest), t.all) +
+         (splits == 1u ? 1.0 : combine_128_us(launch, splits));
+}
+
 // any_order: workgroups may deal a batch's tiles otherwise than a launch of its own
 int32_t attend_batches(const qllm_q4h_attention_launch* launch, uint32_t batch_rows,
                        bool any_order) {
@@ -2996,6 +3049,37 @@ extern "C" uint32_t qllm_attention_paged_q4h_shared_splits(
     best = splits;
   }
   return best;
+}
+
+extern "C" uint32_t qllm_attention_paged_q4h_prompt_form(
+    const qllm_q4h_attention_launch* launch, uint32_t batch_rows, uint32_t most,
+    uint32_t* splits) {
+  if (!splits) return 0u;
+  *splits = 0u;
+  if (!sizes_known(launch, batch_rows) || !most || launch->head_dim != 128u ||
+      launch->split_tokens)
+    return 0u;
+  const uint64_t batches = (uint64_t{launch->rows} + batch_rows - 1u) / batch_rows;
+  const uint64_t alone = batches * launch->kv_heads;
+  const uint64_t together =
+      (batches + kPromptBatches - 1u) / kPromptBatches * launch->kv_heads;
+  double least = 0.0;
+  uint32_t shared = 0u;
+  const auto consider = [&](double time, uint32_t form, uint32_t cuts) {
+    if (*splits && time >= least) return;
+    least = time;
+    shared = form;
+    *splits = cuts;
+  };
+  // (one round of batches of their own, two of shared tiles: beyond them a cut costs
+  // more than it evens out, and the partials take room)
+  for (uint32_t cuts = 1; cuts <= most; ++cuts) {
+    if (cuts == 1u || alone * cuts <= 256u)
+      consider(batches_128_us(*launch, batch_rows, cuts), 0u, cuts);
+    if (cuts == 1u || together * cuts <= 512u)
+      consider(shared_128_us(*launch, batch_rows, cuts), 1u, cuts);
+  }
+  return shared;
 }
 
 extern "C" int32_t qllm_attention_paged_q4h_prompt(

@@ -1291,24 +1291,21 @@ std::uint32_t Mi355DenseFp4Provider::prefill_splits_for(
   return std::clamp((256U + workgroups - 1U) / workgroups, 1U, prefill_splits_);
 }
 
-// Context splits of the shared-tile prompt attention (eight row batches per
-// workgroup), or 0 where the batched launch of the verify step's kernel serves:
-// fewer than 32 row batches at head_dim 128.  At head_dim 256 the most splits that are
-// tried with it.
+// The most context splits that are tried with shared tiles (eight row batches or, at
+// head_dim 256, 128 (row, head) pairs to a workgroup, one workgroup to a compute unit):
+// for two rounds of them at head_dim 128; at head_dim 256 for one more than a full round
+// (three times as many gain 2 % on average, 30 % for 700 - 900 rows over 9000 tokens, and
+// want three times the room).
 std::uint32_t Mi355DenseFp4Provider::prompt_attention_splits(
     std::uint32_t rows, std::uint32_t attention_batch) const noexcept {
-  const std::uint32_t batches = (rows + attention_batch - 1U) / attention_batch;
   if (g_.head_dim == 256U) {
-    // 128 (row, head) pairs to a workgroup, one workgroup to a compute unit: splits for
-    // one more than a full round of them at most (three times as many gain 2 % on
-    // average, 30 % for 700 - 900 rows over 9000 tokens, and want three times the room)
     const std::uint32_t workgroups =
         (rows * (g_.query_heads / g_.kv_heads) + 127U) / 128U * g_.kv_heads;
     return std::clamp((256U + workgroups - 1U) / workgroups, 1U, prefill_splits_);
   }
-  if (g_.head_dim != 128U || batches < 32U) return 0U;
+  const std::uint32_t batches = (rows + attention_batch - 1U) / attention_batch;
   const std::uint32_t workgroups = (batches + 7U) / 8U * g_.kv_heads;
-  return std::clamp((256U + workgroups - 1U) / workgroups, 1U, prefill_splits_);
+  return std::clamp(512U / workgroups, 1U, prefill_splits_);
 }
 
 // (cos, sin) of the rotary angles of a batch at first_position .. + rows - 1
@@ -1892,22 +1889,26 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
           launch.output_gated = g_.output_gated;
           launch.output_kind = QLLM_OUT_BF16;
           launch.stream = stream;
-          // From 32 row batches on, eight batches share a workgroup and every
-          // cache tile it fetches and converts; the context is then cut as far
-          // as it takes to give every CU one of those workgroups.
-          // At head_dim 256 the estimates of either form decide.
-          std::uint32_t shared = prompt_attention_splits(rows, attention_batch);
-          const std::uint32_t alone = prefill_splits_for(rows, attention_batch);
-          if (g_.head_dim == 256U)
-            shared = qllm_attention_paged_q4h_shared_splits(&launch, attention_batch, alone,
-                                                            shared);
-          launch.maximum_splits = shared != 0U ? shared : alone;
-          status_check(shared == 0U
-                           ? qllm_attention_paged_q4h_batched(&launch, attention_batch)
-                       : g_.head_dim == 128U
-                           ? qllm_attention_paged_q4h_prompt(&launch, attention_batch)
-                           : qllm_attention_paged_q4h_batched_any_order(&launch,
-                                                                        attention_batch));
+          // Batches of their own, or several that share a workgroup and every cache tile
+          // it fetches and converts, and the splits: by estimates of either form.
+          const std::uint32_t most = prompt_attention_splits(rows, attention_batch);
+          if (g_.head_dim == 128U) {
+            const bool shared = qllm_attention_paged_q4h_prompt_form(
+                                    &launch, attention_batch, most,
+                                    &launch.maximum_splits) != 0U;
+            status_check(shared
+                             ? qllm_attention_paged_q4h_prompt(&launch, attention_batch)
+                             : qllm_attention_paged_q4h_batched(&launch, attention_batch));
+          } else {
+            const std::uint32_t alone = prefill_splits_for(rows, attention_batch);
+            const std::uint32_t shared = qllm_attention_paged_q4h_shared_splits(
+                &launch, attention_batch, alone, most);
+            launch.maximum_splits = shared != 0U ? shared : alone;
+            status_check(
+                shared != 0U
+                    ? qllm_attention_paged_q4h_batched_any_order(&launch, attention_batch)
+                    : qllm_attention_paged_q4h_batched(&launch, attention_batch));
+          }
         } else {
           const std::uint32_t query_stride =
               g_.head_dim * (g_.output_gated ? 2U : 1U);

@@ -150,6 +150,36 @@ def test_launches_that_cannot_share_tiles(change):
     assert qh.call("qllm_attention_paged_q4h_shares_tiles", launch, 5) == 0
 
 
+@pytest.mark.parametrize("query_heads,kv_heads,rows,first,form", [
+    (64, 8, 1, 0, (0, 1)), (64, 8, 300, 0, (0, 1)), (64, 8, 16384, 0, (1, 1)),
+    (64, 8, 120, 2048, (0, 1)),        # two splits: 320 workgroups, a second round
+    (64, 8, 48, 8000, (0, 4)),         # 256 workgroups
+    (64, 8, 1000, 2048, (1, 3)),       # 504 workgroups, two rounds
+    (16, 4, 1500, 2048, (0, 1)), (32, 32, 48, 8000, (0, 8)), (3, 1, 65535, 0, (1, 1)),
+    (512, 512, 100, 100, None), (7, 7, 100000, 60000, None)])
+@pytest.mark.parametrize("most", [1, 3, 8])
+def test_prompt_forms_of_128_dimensions(query_heads, kv_heads, rows, first, form, most):
+    batch = 48 // (query_heads // kv_heads)
+    splits = ctypes.c_uint32()
+    shared = qh.call("qllm_attention_paged_q4h_prompt_form",
+                     attention(rows, first, query_heads, kv_heads, head_dim=128), batch, most,
+                     ctypes.byref(splits))
+    assert shared in (0, 1) and 1 <= splits.value <= most
+    workgroups = kv_heads * -(-rows // (batch * (8 if shared else 1)))
+    assert splits.value == 1 or workgroups * splits.value <= (512 if shared else 256)
+    if most == 8 and form:
+        assert (shared, splits.value) == form
+
+
+@pytest.mark.parametrize("change", [dict(head_dim=256), dict(split_tokens=64), dict(rows=0),
+                                    dict(kv_heads=0), dict(query_heads=2)])
+def test_launches_without_a_prompt_form(change):
+    sizes = {**dict(rows=1000, first=0, query_heads=16, kv_heads=4, head_dim=128), **change}
+    splits = ctypes.c_uint32(9)
+    assert qh.call("qllm_attention_paged_q4h_prompt_form", attention(**sizes), 12, 8,
+                   ctypes.byref(splits)) == 0 and splits.value == 0
+
+
 # ---- a norm with its projections ------------------------------------------------
 
 MIB = 1 << 20
