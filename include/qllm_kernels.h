@@ -1388,6 +1388,12 @@ size_t qllm_latent_attention_workspace_bytes(const qllm_latent_attention* attent
                                              uint32_t maximum_position);
 int32_t qllm_latent_attention_rows(const qllm_latent_attention* attention,
                                    const qllm_latent_launch* launch, void* stream);
+/* qllm_latent_store of the same rows, then qllm_latent_attention_rows; in the split form,
+ * without a query latent to store, with a launch less.  The workspace lies over nothing
+ * that the store reads. */
+int32_t qllm_latent_store_attention_rows(const qllm_latent_attention* attention,
+                                         const qllm_latent_store_launch* store,
+                                         const qllm_latent_launch* launch, void* stream);
 
 /* ---- recurrent layers ------------------------------------------------------ */
 

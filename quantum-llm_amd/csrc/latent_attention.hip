@@ -114,14 +114,11 @@ struct StoreArgs {
   qllm_latent_store_launch launch;
 };
 
-// A workgroup per row and task: the cache row, or the query latent.
+// A workgroup of 256 threads: a row's cache row, or its query latent.
 template <typename T>
-__global__ __launch_bounds__(256) void latent_store_kernel(StoreArgs args) {
-  __shared__ float scratch[16];
-  const Latent& a = args.attention;
-  const auto& run = args.launch;
-  const uint32_t row = blockIdx.x;
-  const bool query = blockIdx.y == 1u;
+__device__ __forceinline__ void store_latent(const Latent& a,
+                                             const qllm_latent_store_launch& run,
+                                             uint32_t row, bool query, float* scratch) {
   const float* source = run.projections + size_t{row} * run.stride +
                         (query ? run.query_column : run.latent_column);
   const uint32_t rank = query ? run.query_rank : a.rank;
@@ -172,6 +169,12 @@ __global__ __launch_bounds__(256) void latent_store_kernel(StoreArgs args) {
         },
         chunks_of(a.rank) * 32u);
   }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void latent_store_kernel(StoreArgs args) {
+  __shared__ float scratch[16];
+  store_latent<T>(args.attention, args.launch, blockIdx.x, blockIdx.y == 1u, scratch);
 }
 
 struct AttentionArgs {
@@ -356,9 +359,28 @@ __device__ __forceinline__ i32x4 query_operand(const float* source, uint32_t d, 
 // Split form: the queries of 16 rows and one head through the transposed key
 // map (a wave per 16 latent values), or, in the last workgroup along x, their
 // rotated parts.
-__global__ __launch_bounds__(256) void latent_query_kernel(AttentionArgs args) {
+//
+// STORE: one more workgroup along x, of as many heads as there are rows, leaves a cache row, which the next
+// launch reads; the queries do not.  As a launch of its own that took 4.7 us of a decoded
+// token's layer.
+template <bool STORE>
+__global__ __launch_bounds__(256) void latent_query_kernel(AttentionArgs args,
+                                                           qllm_latent_store_launch store) {
   const Latent& a = args.attention;
   const auto& run = args.launch;
+  if constexpr (STORE) {
+    __shared__ float scratch[16];
+    // (the first along x: a cache row takes longer than a query's part)
+    if (blockIdx.x == 0u) {
+      for (uint32_t row = blockIdx.z * a.heads + blockIdx.y; row < run.rows;
+           row += gridDim.z * a.heads) {
+        store_latent<uint16_t>(a, store, row, false, scratch);
+        __syncthreads();
+      }
+      return;
+    }
+  }
+  const uint32_t block = blockIdx.x - (STORE ? 1u : 0u);
   const uint32_t head = blockIdx.y;
   const uint32_t row0 = blockIdx.z * 16u;
   const uint32_t rows = min(16u, run.rows - row0);
@@ -369,7 +391,7 @@ __global__ __launch_bounds__(256) void latent_query_kernel(AttentionArgs args) {
   const float* source = run.query + size_t{row0} * run.query_stride + size_t{head} * width;
   uint16_t* out = args.query + (size_t{row0} * a.heads + head) * stride;
   const size_t out_row = size_t{a.heads} * stride;
-  if (blockIdx.x * 4u >= tiles) {
+  if (block * 4u >= tiles) {
     const uint32_t padded = chunks_of(a.rot_dim) * 32u;
     const uint32_t first = a.step[kStepPosition] + row0;
     for (uint32_t i = threadIdx.x; i < rows * padded; i += blockDim.x) {
@@ -382,7 +404,7 @@ __global__ __launch_bounds__(256) void latent_query_kernel(AttentionArgs args) {
     }
     return;
   }
-  const uint32_t tile = blockIdx.x * 4u + threadIdx.x / kWave;
+  const uint32_t tile = block * 4u + threadIdx.x / kWave;
   if (tile >= tiles) return;
   const uint32_t lane = threadIdx.x % kWave;
   const uint32_t column = lane % 16u;
@@ -1200,15 +1222,22 @@ extern "C" size_t qllm_latent_layer_bytes(uint32_t page_tokens, uint32_t rank,
          (element == QLLM_ELEMENT_F32 ? 4u : 2u);
 }
 
+namespace {
+bool valid_store(const qllm_latent_attention* attention,
+                 const qllm_latent_store_launch* launch) {
+  return attention && launch && valid_geometry(*attention) && launch->projections &&
+         launch->rows &&
+         launch->latent_column + attention->rank + attention->rot_dim <= launch->stride &&
+         (!launch->query_rank ||
+          (launch->query_norm && launch->query_out &&
+           launch->query_stride >= launch->query_rank &&
+           launch->query_column + launch->query_rank <= launch->stride));
+}
+}  // namespace
+
 extern "C" int32_t qllm_latent_store(const qllm_latent_attention* attention,
                                      const qllm_latent_store_launch* launch, void* stream) {
-  if (!attention || !launch || !valid_geometry(*attention) || !launch->projections ||
-      !launch->rows ||
-      launch->latent_column + attention->rank + attention->rot_dim > launch->stride ||
-      (launch->query_rank &&
-       (!launch->query_norm || !launch->query_out ||
-        launch->query_stride < launch->query_rank ||
-        launch->query_column + launch->query_rank > launch->stride)))
+  if (!valid_store(attention, launch))
     return fail(QLLM_INVALID_ARGUMENT, "invalid latent store");
   const StoreArgs args{*attention, *launch};
   const dim3 grid(launch->rows, launch->query_rank ? 2u : 1u);
@@ -1243,9 +1272,12 @@ extern "C" size_t qllm_latent_attention_workspace_bytes(
   }
 }
 
-extern "C" int32_t qllm_latent_attention_rows(const qllm_latent_attention* attention,
-                                              const qllm_latent_launch* launch,
-                                              void* stream) {
+namespace {
+// `store`: null, or rows that the launch that makes the queries leaves in the pages (split
+// form only).
+int32_t attend_latents(const qllm_latent_attention* attention,
+                       const qllm_latent_launch* launch,
+                       const qllm_latent_store_launch* store, void* stream) {
   if (!attention || !launch || !valid_geometry(*attention) || !launch->query ||
       !launch->output || !launch->rows ||
       launch->query_stride < attention->heads * (attention->dim + attention->rot_dim) ||
@@ -1309,9 +1341,14 @@ extern "C" int32_t qllm_latent_attention_rows(const qllm_latent_attention* atten
   }
   args.splits = splits_for(a, rows, launch->maximum_position);
   const uint32_t row_tiles = (rows + 15u) / 16u;
-  latent_query_kernel<<<dim3((chunks_of(a.rank) * 2u + 3u) / 4u + (a.rot_dim ? 1u : 0u),
-                             a.heads, row_tiles),
-                        256, 0, hip_stream>>>(args);
+  const uint32_t query_parts =
+      (chunks_of(a.rank) * 2u + 3u) / 4u + (a.rot_dim ? 1u : 0u);
+  if (store)
+    latent_query_kernel<true><<<dim3(query_parts + 1u, a.heads, row_tiles), 256, 0,
+                                hip_stream>>>(args, *store);
+  else
+    latent_query_kernel<false><<<dim3(query_parts, a.heads, row_tiles), 256, 0,
+                                 hip_stream>>>(args, {});
   const dim3 grid(args.splits, item_tiles(a, rows));
   if (a.rank <= 64u)
     latent_split_kernel<1><<<grid, 256, 0, hip_stream>>>(args);
@@ -1325,4 +1362,25 @@ extern "C" int32_t qllm_latent_attention_rows(const qllm_latent_attention* atten
   latent_value_kernel<<<dim3(a.heads, row_tiles, value_parts), kValueThreads, value_bytes(a),
                         hip_stream>>>(args);
   return launched("latent split attention");
+}
+}  // namespace
+
+extern "C" int32_t qllm_latent_attention_rows(const qllm_latent_attention* attention,
+                                              const qllm_latent_launch* launch,
+                                              void* stream) {
+  return attend_latents(attention, launch, nullptr, stream);
+}
+
+extern "C" int32_t qllm_latent_store_attention_rows(const qllm_latent_attention* attention,
+                                                    const qllm_latent_store_launch* store,
+                                                    const qllm_latent_launch* launch,
+                                                    void* stream) {
+  if (!valid_store(attention, store) || !launch || store->rows != launch->rows)
+    return fail(QLLM_INVALID_ARGUMENT, "invalid latent store");
+  // (a query latent is read by a projection between the two)
+  if (!store->query_rank &&
+      qllm_latent_attention_form(attention, launch->rows) == QLLM_ATTENTION_SPLIT)
+    return attend_latents(attention, launch, store, stream);
+  if (const int32_t status = qllm_latent_store(attention, store, stream)) return status;
+  return attend_latents(attention, launch, nullptr, stream);
 }

@@ -1035,15 +1035,6 @@ void Mi355MixedProvider::enqueue_latent(Block& block, std::uint32_t rows,
   store.stride = projection_stride_;
   store.latent_column = block.latent_column;
   store.rows = rows;
-  if (block.query_rank) {
-    store.query_column = block.query_column;
-    store.query_rank = block.query_rank;
-    store.query_norm = block.query_norm.as<float>();
-    store.query_out = query_latents_.get();
-    store.query_stride = block.query_up.columns;
-  }
-  status_check(qllm_latent_store(&a, &store, stream_));
-
   qllm_latent_launch launch{};
   launch.query = projections_.as<float>() + block.query_column;
   launch.query_stride = projection_stride_;
@@ -1058,7 +1049,30 @@ void Mi355MixedProvider::enqueue_latent(Block& block, std::uint32_t rows,
     s.output_stride = block.query_up.rows;
     s.output_columns = a.heads * (a.dim + a.rot_dim);
     s.epilogue = QLLM_LINEAR_STORE;
-    status_check(qllm_linear_batch(&s, 1U, rows, g_.element, stream_));
+    // one row's query latent is normed by the projection that reads it, where it can be
+    qllm_stream_norm_launch norm{};
+    norm.input = launch.query;
+    norm.weight[0] = block.query_norm.as<float>();
+    norm.output[0] = query_latents_.get();
+    norm.stride[0] = block.query_up.columns;
+    norm.rows = rows;
+    norm.width = block.query_rank;
+    norm.epsilon = a.epsilon;
+    norm.element = g_.element;
+    std::uint32_t launches = 2U;
+    if (rows == 1U)
+      status_check(qllm_linear_normed_launches(&norm, nullptr, &s, 1U, &launches));
+    if (launches == 1U) {
+      status_check(qllm_linear_normed(&norm, nullptr, &s, 1U, stream_));
+    } else {
+      store.query_column = block.query_column;
+      store.query_rank = block.query_rank;
+      store.query_norm = block.query_norm.as<float>();
+      store.query_out = query_latents_.get();
+      store.query_stride = block.query_up.columns;
+      status_check(qllm_latent_store(&a, &store, stream_));
+      status_check(qllm_linear_batch(&s, 1U, rows, g_.element, stream_));
+    }
     launch.query = queries_.as<float>();
     launch.query_stride = block.query_up.rows;
   }
@@ -1071,7 +1085,10 @@ void Mi355MixedProvider::enqueue_latent(Block& block, std::uint32_t rows,
   launch.maximum_position = last_position;
   launch.workspace = scratch_.get();
   launch.workspace_bytes = scratch_bytes_;
-  status_check(qllm_latent_attention_rows(&a, &launch, stream_));
+  // (a store with query latents is done already)
+  status_check(store.query_rank
+                   ? qllm_latent_attention_rows(&a, &launch, stream_)
+                   : qllm_latent_store_attention_rows(&a, &store, &launch, stream_));
 }
 
 void Mi355MixedProvider::enqueue_mixer(Block& block, std::uint32_t rows,

@@ -330,6 +330,7 @@ SIGNATURES = {
     "qllm_latent_attention_form": (c_uint32, [POINTER(LatentAttention), c_uint32]),
     "qllm_latent_attention_workspace_bytes": (c_size_t, [POINTER(LatentAttention), c_uint32, c_uint32]),
     "qllm_latent_attention_rows": (c_int32, [POINTER(LatentAttention), POINTER(LatentLaunch), c_void_p]),
+    "qllm_latent_store_attention_rows": (c_int32, [POINTER(LatentAttention), POINTER(LatentStoreLaunch), POINTER(LatentLaunch), c_void_p]),
     "qllm_recurrence_workspace_bytes": (c_size_t, [POINTER(Recurrence), c_uint32]),
     "qllm_recurrence_rows": (c_int32, [POINTER(Recurrence), POINTER(RecurrenceLaunch), c_void_p]),
     "qllm_fill_random": (c_int32, [c_void_p, c_size_t, c_uint32, c_uint64, c_void_p]),

@@ -108,6 +108,7 @@ class Latent:
         self.heads, self.dim, self.rot_dim, self.vdim, self.rank = (heads, dim, rot_dim, vdim,
                                                                     rank)
         self.window, self.query_rank = window, query_rank
+        self.together = False   # store and attention by one call
         self.scale = 1.2 / np.sqrt(dim + rot_dim) if scale is None else scale
         self.norm = mm.bf16(1.0 + 0.2 * rng.standard_normal(rank))
         self.key_up = mm.bf16(rng.standard_normal((heads * dim, rank)) / np.sqrt(rank))
@@ -155,7 +156,8 @@ class Latent:
         store = qh.LatentStoreLaunch(qh.ptr(projections), projections.shape[1], self.query_rank,
                                      0, self.query_rank, qh.ptr(self.keep[5]),
                                      qh.ptr(query_out), stride, rows)
-        qh.call("qllm_latent_store", ctypes.byref(self.layer), ctypes.byref(store), None)
+        if not self.together:
+            qh.call("qllm_latent_store", ctypes.byref(self.layer), ctypes.byref(store), None)
         last = position + rows - 1
         size = qh.call("qllm_latent_attention_workspace_bytes", ctypes.byref(self.layer), rows,
                        last)
@@ -165,8 +167,12 @@ class Latent:
         launch = qh.LatentLaunch(
             qh.ptr(query), query.shape[1], qh.ptr(gate), gate.shape[1], qh.ptr(out),
             out.shape[1], rows, last, qh.ptr(workspace), size)
-        qh.call("qllm_latent_attention_rows", ctypes.byref(self.layer), ctypes.byref(launch),
-                None)
+        if self.together:
+            qh.call("qllm_latent_store_attention_rows", ctypes.byref(self.layer),
+                    ctypes.byref(store), ctypes.byref(launch), None)
+        else:
+            qh.call("qllm_latent_attention_rows", ctypes.byref(self.layer),
+                    ctypes.byref(launch), None)
         torch.cuda.synchronize()
         assert torch.all(out[:, self.heads * self.vdim:] == 0)
         if self.query_rank:
@@ -519,3 +525,30 @@ def test_long_prompts_in_segments(device, element, heads, dim, vdim, tau):
         close(state.reshape(heads, dim, vdim).astype(np.float64), states, F32, "state",
               factor=4.0)
         assert torch.all(layer.state[:layer.slot_stride] == 0)
+
+
+@pytest.mark.parametrize("element", [qh.ELEMENT_BF16, qh.ELEMENT_F32])
+@pytest.mark.parametrize("heads,dim,rot_dim,rotary,vdim,rank,query_rank", [
+    (16, 128, 64, 64, 128, 512, 0), (2, 32, 0, 0, 16, 130, 0),   # two heads, no shared key part
+    (3, 48, 16, 8, 40, 64, 0), (4, 64, 32, 32, 64, 256, 96)])    # a query latent: two calls
+def test_store_and_attention_by_one_call(device, element, heads, dim, rot_dim, rotary, vdim,
+                                         rank, query_rank):
+    """The pages and outputs of the two calls, bit for bit: prompts, single tokens, few rows
+    across a page's end, more rows than workgroups leave cache rows at once."""
+    results = []
+    for together in (False, True):
+        layer = Latent(device, element, heads, dim, rot_dim, rotary, vdim, rank, 0, seed=3,
+                       query_rank=query_rank)
+        layer.together = together
+        rng = np.random.default_rng(rank)
+        position, outputs = 0, []
+        for rows in (40, 1, 1, 30, 3, 17, 32, 1):
+            outputs.append(layer.run(layer.inputs(rng, rows), position))
+            position += rows
+        results.append((outputs, [page.cpu().numpy() for page in layer.pages]))
+    (apart, apart_pages), (joined, joined_pages) = results
+    for a, b in zip(apart, joined):
+        assert np.array_equal(a, b)
+    for a, b in zip(apart_pages, joined_pages):
+        assert np.array_equal(a, b)
+    assert any(page.any() for page in joined_pages)
