@@ -989,6 +989,16 @@ int32_t qllm_topk_logits_batch(const float* values, uint32_t count,
                                float* output_values, uint32_t* output_indices,
                                void* workspace, size_t workspace_bytes,
                                void* stream);
+/* The same into pinned host memory, without a copy: row r's values and indices, then
+ * host_sequences[r] = sequence (released to the system, so that a host that acquires the
+ * number sees the row). */
+int32_t qllm_topk_logits_batch_handed(const float* values, uint32_t count,
+                                      size_t row_stride, uint32_t top_k,
+                                      uint32_t rows, float* host_values,
+                                      uint32_t* host_indices,
+                                      uint32_t* host_sequences, uint32_t sequence,
+                                      void* workspace, size_t workspace_bytes,
+                                      void* stream);
 
 /* replaces apply_presence_penalty (transformer_kernels.hpp:1292-1294). */
 int32_t qllm_apply_presence_penalty(float* logits, const uint8_t* emitted,

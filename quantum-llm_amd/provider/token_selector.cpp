@@ -19,10 +19,7 @@ namespace qllm {
 TokenSelector::TokenSelector(void* stream, std::uint32_t vocabulary, void* workspace,
                              std::size_t workspace_bytes)
     : stream_(stream), vocabulary_(vocabulary), workspace_(workspace),
-      workspace_bytes_(workspace_bytes),
-      device_(8U * kMaximumTopK * (4U + 4U), "allocate token selection") {
-  // top-k logits of up to 8 rows, then their tokens: one buffer, one readback
-  top_logits_ = device_.as<float>();
+      workspace_bytes_(workspace_bytes) {
   void* pinned = nullptr;
   hip_check(hipHostMalloc(&pinned, sizeof(Staging), hipHostMallocDefault),
             "allocate pinned staging");
@@ -266,8 +263,8 @@ er::SamplingDistribution TokenSelector::distribution(
 }
 
 // The distributions of `rows` rows of logits (row r at logits + r * stride)
-// for a sampled request with 1 <= top_k <= 64: one selection launch for all
-// rows, one readback, then make_sampling_distribution per row
+// for a sampled request with 1 <= top_k <= 64: one selection for all rows, which
+// leaves them in pinned memory, then make_sampling_distribution per row
 // (distribution_from_logits, dense_fp4_provider.cpp:8331-8391, which selects
 // and reads back row by row).
 std::vector<er::SamplingDistribution>
@@ -287,10 +284,18 @@ TokenSelector::top_k_distributions(
         "sampled exact decode requires top-k of at most 64 (0 = whole row)");
   // logits of all rows, then tokens of all rows
   const std::uint32_t chosen = rows * top_k;
-  status_check(qllm_topk_logits_batch(logits, vocabulary, stride, top_k, rows, top_logits_,
-                                      device_.as<std::uint32_t>() + chosen, workspace_,
-                                      workspace_bytes_, stream_));
-  const std::uint32_t* words = read_words(device_.as<std::uint32_t>(), 2U * chosen);
+  const std::uint32_t sequence = ++sequence_;
+  std::uint32_t* const words = staging_->words;
+  status_check(qllm_topk_logits_batch_handed(
+      logits, vocabulary, stride, top_k, rows, reinterpret_cast<float*>(words),
+      words + chosen, staging_->row_sequences, sequence, workspace_, workspace_bytes_,
+      stream_));
+  await([&] {
+    for (std::uint32_t row = 0; row < rows; ++row)
+      if (__atomic_load_n(&staging_->row_sequences[row], __ATOMIC_ACQUIRE) != sequence)
+        return false;
+    return true;
+  });
   ++gpu_calls_;
   logit_transfer_bytes_ += std::size_t{rows} * top_k * 8U;
   std::vector<er::SamplingDistribution> result;

@@ -78,6 +78,7 @@ class TokenSelector final {
   struct Staging final {
     std::uint32_t words[kMostWords];
     alignas(64) std::uint32_t sequence;
+    alignas(64) std::uint32_t row_sequences[8];      // of a top-k launch's rows
     alignas(64) std::uint64_t handed[kMostHanded];   // sequence << 32 | token
   };
   // Waits until arrived(): the one way to read what the device writes.
@@ -90,8 +91,6 @@ class TokenSelector final {
   std::uint32_t vocabulary_{};
   void* workspace_{};
   std::size_t workspace_bytes_{};
-  DeviceBuffer device_;
-  float* top_logits_{};
   Staging* staging_{};
   std::uint32_t sequence_{};
   std::uint32_t handed_sequence_{};

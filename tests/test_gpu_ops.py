@@ -326,6 +326,34 @@ def test_batched_topk_when_the_threshold_does_not_filter(device):
     assert values[0][:3].tolist() == [1.0, 1.0, -np.inf] and np.all(np.isneginf(values[0][3:]))
 
 
+@pytest.mark.parametrize("rows,count,top_k", [(5, 32000, 20), (8, 300, 64), (1, 64, 1),
+                                              (3, 151936, 64), (2, 65537, 7)])
+def test_batched_topk_by_hand_over(device, rows, count, top_k):
+    """Into pinned memory: the words of the launch into device memory and, once a row's
+    number is there, nothing that was there before; rows of few values, of ties only (the k
+    rounds) and without a single number among them."""
+    rng = np.random.default_rng(count)
+    logits = rng.standard_normal((rows, count)).astype(np.float32)
+    logits[-1] = 1.5                                   # all equal
+    if rows > 2:
+        logits[0, ::3], logits[1] = -np.inf, np.nan
+    want_values, want_indices = batched_topk(device, list(logits), top_k)
+    d_logits = gu.device_tensor(logits, device)
+    workspace = torch.zeros(qh.call("qllm_topk_batch_workspace_bytes", count, top_k, rows),
+                            dtype=torch.uint8, device=device)
+    values = torch.full((rows, top_k), 7.0, pin_memory=True)
+    indices = torch.full((rows, top_k), 77, dtype=torch.int32, pin_memory=True)
+    numbers = torch.zeros(rows + 1, dtype=torch.int32, pin_memory=True)
+    for number in (41, 42):
+        qh.call("qllm_topk_logits_batch_handed", qh.ptr(d_logits), count, count, top_k, rows,
+                values.data_ptr(), indices.data_ptr(), numbers.data_ptr(), number,
+                qh.ptr(workspace), workspace.numel(), None)
+        torch.cuda.synchronize()
+        assert numbers.tolist() == [number] * rows + [0]
+        assert np.array_equal(values.numpy(), want_values)
+        assert np.array_equal(indices.numpy().view(np.uint32), want_indices)
+
+
 def test_batched_topk_rejects_what_it_does_not_take(device):
     values = torch.zeros((2, 1000), device=device)
     out_v = torch.zeros((2, 64), device=device)
