@@ -768,8 +768,7 @@ int32_t launch_mfma_batch(const GemmArgs& args, uint32_t batch, uint32_t grid,
 }
 
 // One tile per workgroup (a gate tile and its up tile for the fused SwiGLU
-// pair), or k_splits workgroups per tile; four waves split K, eight when the
-// launch has too few workgroups to give every CU one.
+// pair), or k_splits workgroups per tile.
 uint32_t compute_units() {
   static const uint32_t count = [] {
     int device = 0, units = 0;
@@ -809,9 +808,18 @@ int32_t launch_mfma(GemmArgs args, int scheme, bool tiled, uint32_t batch,
       tiles = args.balance_first_tile + extra * cut;
     }
   }
-  // four waves split K, eight when the launch has too few workgroups to give
-  // every CU one
-  const uint32_t waves = tiles <= 256u && !swiglu ? 8u : 4u;
+  // Four waves split K; eight where the launch has at most one workgroup a CU, which then
+  // waits for its own chain of chunks, and the chunks are enough to share.  A launch
+  // alone, five rows, four and eight waves: binary16 scales, 2048 rows, 11 and 16 chunks
+  // a workgroup 3.9 / 4.7 and 4.0 / 4.6 us, 21 5.1 / 5.0, 32 5.2 / 4.9, 88 9.8 / 7.8;
+  // UE8M0 4.0 / 4.3, 4.1 / 4.3, 4.8 / 4.5, 5.4 / 4.7.  Gate and up, whose waves have two
+  // tiles' loads in flight, 4096 rows: binary16 16, 32 and 64 chunks 5.3 / 6.6, 7.1 / 7.3
+  // and 10.7 / 9.7, UE8M0 5.4 / 5.9, 7.2 / 6.9 and 11.3 / 9.3.
+  const uint32_t chunks = args.padded_columns / kChunk / splits;
+  uint32_t enough = 20u;
+  if (swiglu) enough = scheme == kSchemeF16 ? 40u : 28u;
+  if (args.activation_scales) enough = swiglu ? ~0u : 0u;
+  const uint32_t waves = tiles <= 256u && chunks >= enough ? 8u : 4u;
 #define QLLM_LAUNCH(SCHEME_, TILES_, TILED_)                                  \
   return launch_mfma_batch<SCHEME_, TILES_, TILED_>(args, batch, tiles, waves, \
                                                     stream)
