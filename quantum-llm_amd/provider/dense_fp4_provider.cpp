@@ -313,7 +313,8 @@ void Mi355DenseFp4Provider::allocate_workspaces() {
   hip_check(hipMemset(proposal_presence_, 0, g_.vocabulary),
             "clear presence bytes");
   selector_ = std::make_unique<TokenSelector>(stream_, g_.vocabulary, select_workspace_,
-                                              select_workspace_bytes_);
+                                              select_workspace_bytes_,
+                                              qllm_topk_logits_batch_handed);
 
   if (g_.mtp_layers) {
     mtp_tokens_ = static_cast<std::uint32_t*>(device_alloc((8U + 4U) * 4U));

@@ -692,7 +692,8 @@ void Mi355MixedProvider::finalize_locked() {
   argmax_ = DeviceBuffer(4U, "allocate arg-max");
   selector_ = std::make_unique<TokenSelector>(stream_, g_.vocabulary,
                                               select_workspace_.get(),
-                                              select_workspace_bytes_);
+                                              select_workspace_bytes_,
+                                              qllm_topk_logits_batch_handed);
   const std::uint32_t element_bytes = g_.element == QLLM_ELEMENT_F32 ? 4U : 2U;
   head_input_ = DeviceBuffer(std::size_t{kLogitRows} * mixer_stride_ * element_bytes,
                              "allocate head input");

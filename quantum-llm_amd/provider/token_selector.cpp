@@ -17,9 +17,9 @@
 namespace qllm {
 
 TokenSelector::TokenSelector(void* stream, std::uint32_t vocabulary, void* workspace,
-                             std::size_t workspace_bytes)
+                             std::size_t workspace_bytes, TopKRows top_k_rows)
     : stream_(stream), vocabulary_(vocabulary), workspace_(workspace),
-      workspace_bytes_(workspace_bytes) {
+      workspace_bytes_(workspace_bytes), top_k_rows_(top_k_rows) {
   void* pinned = nullptr;
   hip_check(hipHostMalloc(&pinned, sizeof(Staging), hipHostMallocDefault),
             "allocate pinned staging");
@@ -286,7 +286,8 @@ TokenSelector::top_k_distributions(
   const std::uint32_t chosen = rows * top_k;
   const std::uint32_t sequence = ++sequence_;
   std::uint32_t* const words = staging_->words;
-  status_check(qllm_topk_logits_batch_handed(
+  if (!top_k_rows_) throw std::logic_error("this selector takes no top k");
+  status_check(top_k_rows_(
       logits, vocabulary, stride, top_k, rows, reinterpret_cast<float*>(words),
       words + chosen, staging_->row_sequences, sequence, workspace_, workspace_bytes_,
       stream_));

@@ -19,10 +19,15 @@ class TokenSelector final {
  public:
   static constexpr std::uint32_t kMaximumTopK = 64U;  // provider.cpp:8359
 
+  // qllm_topk_logits_batch_handed, for requests that sample from a top k (a selector of
+  // arg-max tokens has no need of it).
+  using TopKRows = std::int32_t (*)(const float*, std::uint32_t, std::size_t, std::uint32_t,
+                                    std::uint32_t, float*, std::uint32_t*, std::uint32_t*,
+                                    std::uint32_t, void*, std::size_t, void*);
   // `workspace`: device memory of at least workspace_bytes(), shared with the
   // caller's own arg-max launches on the same stream.
   TokenSelector(void* stream, std::uint32_t vocabulary, void* workspace,
-                std::size_t workspace_bytes);
+                std::size_t workspace_bytes, TopKRows top_k_rows = nullptr);
   ~TokenSelector();
   TokenSelector(const TokenSelector&) = delete;
   TokenSelector& operator=(const TokenSelector&) = delete;
@@ -91,6 +96,7 @@ class TokenSelector final {
   std::uint32_t vocabulary_{};
   void* workspace_{};
   std::size_t workspace_bytes_{};
+  TopKRows top_k_rows_{};
   Staging* staging_{};
   std::uint32_t sequence_{};
   std::uint32_t handed_sequence_{};
