@@ -637,6 +637,12 @@ typedef struct qllm_q4h_attention_launch {
    * maximum_splits, so a captured graph can be replayed as the context
    * grows.  No counterpart in the reference struct. */
   const uint32_t* device_positions;
+  /* How a balanced launch (split_tokens 0) deals the tiles of a verify step or batch.
+   * 0: the end of the context, where the batch's records are encoded, counts as sixteen
+   * tiles.  1: where the workgroups before it can take a tile a wave, the last one has
+   * the last tile alone, and a single one deals evenly - fewer tiles one after the other
+   * in short contexts, F32 sums in another order. */
+  int32_t tail_alone;
 } qllm_q4h_attention_launch;
 
 /* Split phase + split-K combine.  rows * (query_heads/kv_heads) <= 48,

@@ -186,7 +186,8 @@ __device__ __forceinline__ void q8_encode_record(const float* source,
 // tail_work (balanced only): what the waves at the end of the context do
 // besides their tiles, in tiles' worth of time - the deal is over
 // context_tiles + tail_work tiles of which the last tail_work do not exist, so
-// those waves walk that many fewer.
+// those waves walk that many fewer.  tail_alone: where the other workgroups' waves hold
+// all tiles but the last one each, the last workgroup has that one alone.
 template <int WAVES = kSplitWaves>
 __device__ __forceinline__ void wave_tile_range(uint32_t context_tiles,
                                                 uint32_t tile_tokens,
@@ -195,12 +196,20 @@ __device__ __forceinline__ void wave_tile_range(uint32_t context_tiles,
                                                 uint32_t wave,
                                                 uint32_t& tile_first,
                                                 uint32_t& tile_last,
-                                                uint32_t tail_work = 0u) {
+                                                uint32_t tail_work = 0u,
+                                                bool tail_alone = false) {
   if (split_tokens == 0u) {
     // floor(slot * tiles / slots) in 32-bit arithmetic: with tiles = q * slots
     // + r it is slot * q + floor(slot * r / slots), and slot * r < slots^2
     const uint32_t slots = splits * WAVES;
     const uint32_t slot = split * WAVES + wave;
+    const uint32_t others = slots - WAVES;   // slots of the other workgroups
+    if (tail_alone && splits > 1u && context_tiles <= others + 1u) {
+      const uint32_t before = context_tiles - 1u;
+      tile_first = slot < others ? slot * before / others : before + min(slot - others, 1u);
+      tile_last = slot < others ? (slot + 1u) * before / others : context_tiles;
+      return;
+    }
     const uint32_t dealt = context_tiles + tail_work;
     const uint32_t quotient = dealt / slots;
     const uint32_t remainder = dealt - quotient * slots;

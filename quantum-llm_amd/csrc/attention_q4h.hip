@@ -117,6 +117,7 @@ struct SplitArgs {
   void* output;
   uint32_t output_kind;
   uint32_t output_gated;
+  uint32_t tail_alone;
 };
 
 
@@ -510,11 +511,16 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void q4h_attention_split_kerne
   // (fused: the workgroup at the end of the context also encodes the batch's
   // K/V records, lays them over its tiles and writes them to their pages -
   // about two tiles' worth of time for each of its waves.  The plain kernel
-  // deals the same way, so that both add up a context in the same order.  Where
-  // one workgroup has the whole context every wave has that work.)
-  const uint32_t tail_work = ONE || gridDim.y == 1u ? 0u : 2u * kSplitWaves;
+  // deals the same way, so that both add up a context in the same order.
+  // tail_alone: that work is left to one workgroup with no tile but the last, where
+  // there are workgroups enough, and where there is one only every wave has it - five
+  // rows of 16 heads on 4 after 500 tokens, one split, 16.5 us with the uneven deal and a
+  // combine, 12.9 with an even one and without.)
+  const bool tail_alone = args.tail_alone != 0u;
+  const uint32_t tail_work =
+      tail_alone && gridDim.y == 1u ? 0u : 2u * kSplitWaves;
   wave_tile_range<WAVES>(context_tiles, 64u, args.split_tokens, split, gridDim.y, wave,
-                         tile_first, tile_last, tail_work);
+                         tile_first, tile_last, tail_work, tail_alone);
 
   // the wave's staging areas: tile t of the wave uses area t % DEPTH
   uint8_t* const stage_base = stage + wave * (STAGE * DEPTH);
@@ -682,9 +688,9 @@ __global__ __launch_bounds__(kSplitWaves * 64, 2) void q4h_attention_split_kerne
     }
     uint32_t workgroup_first, workgroup_last, unused;
     wave_tile_range(context_tiles, 64u, args.split_tokens, split, gridDim.y, 0u,
-                    workgroup_first, unused, tail_work);
+                    workgroup_first, unused, tail_work, tail_alone);
     wave_tile_range(context_tiles, 64u, args.split_tokens, split, gridDim.y,
-                    kSplitWaves - 1u, unused, workgroup_last, tail_work);
+                    kSplitWaves - 1u, unused, workgroup_last, tail_work, tail_alone);
     reaches_batch = workgroup_first < workgroup_last &&
                     workgroup_last * 64u > first_cache_position;
     // the wave's first tiles set out first: the work below hides behind them
@@ -2896,7 +2902,8 @@ double batches_128_us(const qllm_q4h_attention_launch& launch, uint32_t batch_ro
     const double tiles =
         static_cast<double>((launch.first_context_tokens + rows + 62u) / 64u);
     if (splits == 1u) return std::ceil(tiles / kSplitWaves);
-    // (the deal of the split kernel; its last waves walk fewer)
+    // (the deal of the split kernel: a tile a wave, or its last waves walk fewer)
+    if (tiles <= kSplitWaves * (splits - 1.0) + 1.0) return 1.0;
     const double share = (tiles + 2.0 * kSplitWaves) / (kSplitWaves * splits);
     return 0.75 * std::ceil(share - 0.03) + 0.25 * share;
   };
@@ -2974,6 +2981,7 @@ int32_t attend_batches(const qllm_q4h_attention_launch* launch, uint32_t batch_r
   args.kv_heads = launch->kv_heads;
   args.split_tokens = launch->split_tokens;
   args.maximum_splits = launch->maximum_splits;
+  args.tail_alone = launch->tail_alone != 0 ? 1u : 0u;
   args.batch_rows = batch_rows;
   const bool shares = any_order && shares_tiles(*launch, batch_rows);
   if (!shares &&
@@ -3121,6 +3129,7 @@ extern "C" int32_t qllm_attention_paged_q4h_prompt(
   args.query_heads = launch->query_heads;
   args.kv_heads = launch->kv_heads;
   args.maximum_splits = launch->maximum_splits;
+  args.tail_alone = launch->tail_alone != 0 ? 1u : 0u;
   args.batch_rows = batch_rows;
   const uint32_t parts = (batches + kPromptBatches - 1u) / kPromptBatches;
   if (launch->kv_heads * parts >= kDirectWorkgroups &&
@@ -3210,6 +3219,7 @@ int32_t launch_q4h_attention(const qllm_q4h_attention_launch* launch,
   args.kv_heads = launch->kv_heads;
   args.split_tokens = launch->split_tokens;
   args.maximum_splits = launch->maximum_splits;
+  args.tail_alone = launch->tail_alone != 0 ? 1u : 0u;
   args.device_positions = launch->device_positions;
   const size_t width = size_t{launch->kv_heads} * launch->head_dim;
   if (one_split_writes_output(

@@ -179,6 +179,30 @@ std::uint64_t Mi355DenseFp4Provider::kv_bytes_per_token_layer() const noexcept {
   return std::uint64_t{g_.kv_heads} * 2U * (g_.head_dim / 2U + 2U);
 }
 
+// Context splits of a verify step.  As long as the chip has room for them, as many as it
+// takes for every wave of a workgroup (eight) to have one tile at the longest context -
+// 64 tokens of the Q4H cache, whose last tile has a workgroup of its own, 32 of the exact
+// one - because a second tile takes longer than a further split costs the combine.  Up
+// to 32, which it fetches in one go, and beyond them where a tile of the exact cache is
+// 256 dimensions wide.  Five rows, splits for two tiles a wave (512 tokens a split) and
+// for one: Q4H, 16 heads on 4 of 128 dimensions after 1000 and 4000 tokens 15.4 and 13.0
+// us, 14.3 and 13.0, 24 heads on 4 of 256 after 4000 23.8 and 20.3; exact, 16 on 4 of 128 after 4000 11.4 and 9.7, 24
+// on 4 of 256 after 4000 and 8000 26.2 and 18.0, 33.0 and 21.8.
+std::uint32_t Mi355DenseFp4Provider::verify_splits(std::uint32_t most) const noexcept {
+  const auto cut = [&](std::uint32_t tokens) {
+    return std::max(1U, (g_.max_context - 1U) / tokens + 1U);
+  };
+  const bool q4h = g_.kv_encoding == KvEncoding::q4_f16_per_head;
+  // (the codes of Q8 rows move by one with every other order of the sums between them)
+  if (g_.activation_q8) return std::min(most, cut(512U));
+  // One split writes the outputs itself: five rows of 16 heads on 4 after 500 tokens
+  // 12.8 us, 13.0 in three (15.6 in two that count the tail as sixteen tiles).
+  if (q4h && g_.max_context <= 512U) return 1U;
+  const std::uint32_t single = q4h ? cut(512U) + 1U : cut(256U);
+  const std::uint32_t room = q4h || g_.head_dim == 128U ? std::min(most, 32U) : most;
+  return single <= room ? single : std::min(most, cut(512U));
+}
+
 void Mi355DenseFp4Provider::allocate_workspaces() {
   const auto device_alloc = [this](std::size_t bytes) {
     void* pointer{};
@@ -266,14 +290,9 @@ void Mi355DenseFp4Provider::allocate_workspaces() {
   maximum_splits_ =
       std::min(wanted_splits, std::max(1U, (g_.max_context + 511U) / 512U));
   prefill_splits_ = std::min(maximum_splits_, 8U);
-  q4h_splits_ = maximum_splits_;
-  // One split of a Q4H launch writes the outputs itself.  Five rows of 16 heads on 4 after
-  // 500 and 760 tokens: 12.9 and 16.1 us against 15.7 and 17.8 with two splits; at 1000
-  // tokens 16.3 against 15.5 with three, at head_dim 256 and 760 tokens 28.3 with either.
-  if (g_.kv_encoding == KvEncoding::q4_f16_per_head && g_.head_dim == 128U &&
-      g_.max_context <= 768U)
-    q4h_splits_ = 1U;
-  const std::size_t partials = rows * maximum_splits_ * g_.query_heads;
+  verify_splits_ = verify_splits(wanted_splits);
+  const std::size_t partials =
+      rows * std::max(maximum_splits_, verify_splits_) * g_.query_heads;
   partial_maxima_ = static_cast<float*>(device_alloc(partials * 4U));
   partial_sums_ = static_cast<float*>(device_alloc(partials * 4U));
   partial_outputs_ =
@@ -1229,7 +1248,8 @@ void Mi355DenseFp4Provider::enqueue_attention(
     launch.kv_heads = g_.kv_heads;
     launch.head_dim = g_.head_dim;
     launch.split_tokens = split_tokens_;
-    launch.maximum_splits = q4h_splits_;
+    launch.maximum_splits = verify_splits_;
+    launch.tail_alone = !g_.activation_q8;
     launch.query_stride = query_stride;
     launch.output_gated = g_.output_gated;
     launch.output_kind = g_.activation_q8 ? QLLM_OUT_F32 : QLLM_OUT_BF16;
@@ -1271,7 +1291,7 @@ void Mi355DenseFp4Provider::enqueue_attention(
     launch.kv_heads = g_.kv_heads;
     launch.head_dim = g_.head_dim;
     launch.split_tokens = split_tokens_;
-    launch.maximum_splits = maximum_splits_;
+    launch.maximum_splits = verify_splits_;
     launch.query_stride = query_stride;
     launch.output_gated = g_.output_gated;
     launch.output_kind = g_.activation_q8 ? QLLM_OUT_F32 : QLLM_OUT_BF16;
@@ -1894,6 +1914,7 @@ Mi355DenseFp4Provider::PrefillResult Mi355DenseFp4Provider::prefill(
           // it fetches and converts, and the splits: by estimates of either form.
           const std::uint32_t most = prompt_attention_splits(rows, attention_batch);
           if (g_.head_dim == 128U) {
+            launch.tail_alone = 1;
             const bool shared = qllm_attention_paged_q4h_prompt_form(
                                     &launch, attention_batch, most,
                                     &launch.maximum_splits) != 0U;
@@ -2263,7 +2284,7 @@ er::Status Mi355DenseFp4Provider::time_kernel(const std::string& which,
         launch.kv_heads = g_.kv_heads;
         launch.head_dim = g_.head_dim;
         launch.split_tokens = split_tokens_;
-        launch.maximum_splits = maximum_splits_;
+        launch.maximum_splits = verify_splits_;
         launch.query_stride = query_stride;
         launch.output_gated = g_.output_gated;
         launch.output_kind = QLLM_OUT_BF16;
@@ -2285,7 +2306,8 @@ er::Status Mi355DenseFp4Provider::time_kernel(const std::string& which,
         launch.kv_heads = g_.kv_heads;
         launch.head_dim = g_.head_dim;
         launch.split_tokens = split_tokens_;
-        launch.maximum_splits = q4h_splits_;
+        launch.maximum_splits = verify_splits_;
+        launch.tail_alone = !g_.activation_q8;
         launch.query_stride = query_stride;
         launch.output_gated = g_.output_gated;
         launch.output_kind = QLLM_OUT_BF16;

@@ -64,7 +64,7 @@ class Q4hAttentionLaunch(Structure):
                 ("head_dim", c_uint32), ("split_tokens", c_uint32),
                 ("maximum_splits", c_uint32), ("query_stride", c_uint32),
                 ("output_gated", c_int32), ("output_kind", c_uint32),
-                ("stream", c_void_p), ("device_positions", c_void_p)]
+                ("stream", c_void_p), ("device_positions", c_void_p), ("tail_alone", c_int32)]
 
 
 class Q4hFusedRope(Structure):

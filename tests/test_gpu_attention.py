@@ -670,3 +670,56 @@ def test_one_split_writes_what_the_combine_would(device, tokens, rows, Q, KV, d,
         got.append(out[begin:begin + rows * Q * d].float().cpu().numpy())
     assert np.abs(got[0]).max() > 0.0
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("tokens,rows,Q,KV,d,gated,splits", [
+    (5, 5, 16, 4, 128, False, 2),          # one tile: the other workgroup has none
+    (64 * 9, 5, 16, 4, 128, False, 2),     # nine tiles: one each and the last alone
+    (64 * 9 + 1, 5, 16, 4, 128, False, 2), # ten: the uneven deal
+    (64 * 9 + 2, 4, 64, 8, 128, True, 3),  # a batch across the last tile's edge
+    (1500, 5, 64, 8, 128, False, 4), (64 * 8, 2, 16, 4, 128, False, 1),
+    (4000, 5, 24, 4, 256, True, 9), (700, 1, 24, 4, 256, True, 5)])
+def test_a_last_tile_alone(device, tokens, rows, Q, KV, d, gated, splits):
+    """The deal with tail_alone: the fused launch equals the rotary and the plain launch
+    bit for bit and stores the same pages, and differs from the other deal by the order of
+    F32 sums and probabilities rounded to binary16 relative to other maxima (2^-11 each)."""
+    rng = np.random.default_rng(tokens + splits)
+    page, rotary, first = 64, 64, tokens - (rows - 1)
+    pages = synth.q4h_pages(rng.standard_normal((tokens, KV, d)).astype(np.float32),
+                            rng.standard_normal((tokens, KV, d)).astype(np.float32), page, 1, 0)
+    stride = d * (2 if gated else 1)
+    q = rng.standard_normal((rows, Q, stride)).astype(np.float32)
+    k, v = (rng.standard_normal((rows, KV, d)).astype(np.float32) for _ in range(2))
+    maxima, sums = torch.zeros((2, rows, splits, Q), device=device)
+    partials = torch.zeros((rows, splits, Q, d), device=device)
+    row_tiles = (rows * Q // KV + 15) // 16
+    operands = torch.zeros(KV * row_tiles * (d // 64) * 2048, dtype=torch.uint8, device=device)
+    scales = torch.zeros(KV * row_tiles * 16, device=device)
+    cos_sin = torch.zeros(rows * rotary, device=device)
+    qh.call("qllm_rope_table", qh.ptr(cos_sin), rows, rotary, first - 1, 1e6, 0, None, None)
+    results = []
+    for fused, alone in ((True, 0), (True, 1), (False, 1)):
+        d_pages = [gu.device_tensor(p, device) for p in pages]
+        table = torch.tensor([p.data_ptr() for p in d_pages], dtype=torch.int64, device=device)
+        d_q, d_k, d_v = (gu.device_tensor(x, device) for x in (q, k, v))
+        out = torch.zeros((rows, Q, d), device=device)
+        launch = qh.Q4hAttentionLaunch(
+            qh.ptr(d_q), 0 if fused else qh.ptr(operands), 0 if fused else qh.ptr(scales),
+            qh.ptr(table), qh.ptr(out), qh.ptr(maxima), qh.ptr(sums), qh.ptr(partials), first,
+            rows, 0, page, Q, KV, d, 0, splits, stride, int(gated), qh.OUT_F32, None, None, alone)
+        if fused:
+            rope = qh.Q4hFusedRope(qh.ptr(d_k), qh.ptr(d_v), 0, 0, qh.ptr(cos_sin), rotary, 1e-6,
+                                   first - 1, 0)
+            qh.call("qllm_attention_paged_q4h_fused", launch, rope)
+        else:
+            qh.call("qllm_qkv_rope_cache_paged_q4h_prepared", None, 0, qh.ptr(d_q), stride,
+                    qh.ptr(d_k), qh.ptr(d_v), 0, 0, qh.ptr(table), 0, page, first - 1, first - 1,
+                    None, rows, Q, KV, d, rotary, 1e-6, 1e6, 0, qh.ptr(operands), qh.ptr(scales),
+                    None)
+            qh.call("qllm_attention_paged_q4h", launch)
+        torch.cuda.synchronize()
+        results.append((out.cpu().numpy(), [p.cpu().numpy() for p in d_pages]))
+    assert np.array_equal(results[1][0], results[2][0])
+    for a, b, c in zip(*(r[1] for r in results)):
+        assert np.array_equal(a, b) and np.array_equal(a, c)
+    gu.assert_close(results[1][0], results[0][0].astype(np.float64), what="other deal")
