@@ -263,13 +263,14 @@ __global__ __launch_bounds__(kMergeThreads) void topk_merge_kernel(
 //      LDS and ranked against each other, rank r going to output slot r.
 // With fewer chunks than k the threshold is -inf (every item is a candidate).
 // If more candidates turn up than LDS holds (large values packed into a few
-// chunks), the workgroup falls back to k rounds over the whole row.  Only the chunks
-// that reach the threshold are read a second time: of five rows of 32000 logits and k =
-// 20 some 20 chunks of 125, 17.2 us -> 10.3 with the hand-over to the host (2.8 us as a
-// launch of its own); a row's round trips, one
-// after the other, are what it waits for.  Results
+// chunks), the workgroup falls back to k rounds over the whole row.  Results
 // are those of the rounds: same order, same ties, NaN excluded, missing ranks
 // padded with (-inf, no index).
+//
+// A row's workgroup waits for round trips one after the other.  Only the chunks that
+// reach the threshold are read a second time - some 20 of 125 for k = 20 of 32000
+// logits - and its words go to the host by themselves: 17.2 us and a copy's launch of
+// 2.8 before, 10.3 now.
 constexpr uint32_t kSelectThreads = 1024;
 constexpr uint32_t kSelectCandidates = 4096;
 constexpr uint32_t kSelectMaxChunks = 4096;

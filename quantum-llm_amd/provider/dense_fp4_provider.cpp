@@ -184,10 +184,10 @@ std::uint64_t Mi355DenseFp4Provider::kv_bytes_per_token_layer() const noexcept {
 // 64 tokens of the Q4H cache, whose last tile has a workgroup of its own, 32 of the exact
 // one - because a second tile takes longer than a further split costs the combine.  Up
 // to 32, which it fetches in one go, and beyond them where a tile of the exact cache is
-// 256 dimensions wide.  Five rows, splits for two tiles a wave (512 tokens a split) and
-// for one: Q4H, 16 heads on 4 of 128 dimensions after 1000 and 4000 tokens 15.4 and 13.0
-// us, 14.3 and 13.0, 24 heads on 4 of 256 after 4000 23.8 and 20.3; exact, 16 on 4 of 128 after 4000 11.4 and 9.7, 24
-// on 4 of 256 after 4000 and 8000 26.2 and 18.0, 33.0 and 21.8.
+// 256 dimensions wide.  Five rows, splits of 512 tokens and for a tile a wave: Q4H, 16
+// heads on 4 of 128 dimensions after 1000 tokens 15.4 and 13.0 us, after 4000 14.3 and
+// 13.0, 24 heads on 4 of 256 after 4000 23.8 and 20.3; exact, 16 on 4 of 128 after 4000
+// 11.4 and 9.7, 24 on 4 of 256 after 4000 26.2 and 18.0, after 8000 33.0 and 21.8.
 std::uint32_t Mi355DenseFp4Provider::verify_splits(std::uint32_t most) const noexcept {
   const auto cut = [&](std::uint32_t tokens) {
     return std::max(1U, (g_.max_context - 1U) / tokens + 1U);
