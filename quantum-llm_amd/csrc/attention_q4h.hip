@@ -2929,6 +2929,10 @@ double shared_128_us(const qllm_q4h_attention_launch& launch, uint32_t batch_row
          (splits == 1u ? 1.0 : combine_128_us(launch, splits));
 }
 
+// Rows of a launch in batches of their own, each a layer of the grid; shared tiles take
+// kPromptBatches as many.
+constexpr uint32_t kBatchedRows = 65535u;
+
 // any_order: workgroups may deal a batch's tiles otherwise than a launch of its own
 int32_t attend_batches(const qllm_q4h_attention_launch* launch, uint32_t batch_rows,
                        bool any_order) {
@@ -2947,7 +2951,7 @@ int32_t attend_batches(const qllm_q4h_attention_launch* launch, uint32_t batch_r
           (launch->output_gated ? 2u : 1u) * launch->head_dim ||
       (launch->output_kind != QLLM_OUT_F32 &&
        launch->output_kind != QLLM_OUT_BF16) ||
-      launch->rows > 65535u ||
+      launch->rows > kBatchedRows ||
       launch->first_context_tokens > 0xffffffffu - (launch->rows - 1u))
     return fail(QLLM_INVALID_ARGUMENT, "invalid batched Q4H paged attention");
   const uint32_t group = launch->query_heads / launch->kv_heads;
@@ -3065,8 +3069,16 @@ extern "C" uint32_t qllm_attention_paged_q4h_prompt_form(
   if (!splits) return 0u;
   *splits = 0u;
   if (!sizes_known(launch, batch_rows) || !most || launch->head_dim != 128u ||
-      launch->split_tokens)
+      launch->split_tokens || launch->query_heads % launch->kv_heads ||
+      uint64_t{std::min(batch_rows, launch->rows)} *
+              (launch->query_heads / launch->kv_heads) > 48u ||
+      !launch->first_context_tokens ||
+      launch->first_context_tokens > 0xffffffffu - (launch->rows - 1u))
     return 0u;
+  // (the rows that either form takes, whatever the estimates say beyond them)
+  const bool takes_alone = launch->rows <= kBatchedRows;
+  const bool takes_shared = launch->rows <= kBatchedRows * kPromptBatches;
+  most = std::min(most, kCombineSplitCapacity);
   const uint64_t batches = (uint64_t{launch->rows} + batch_rows - 1u) / batch_rows;
   const uint64_t alone = batches * launch->kv_heads;
   const uint64_t together =
@@ -3082,9 +3094,9 @@ extern "C" uint32_t qllm_attention_paged_q4h_prompt_form(
   // (one round of batches of their own, two of shared tiles: beyond them a cut costs
   // more than it evens out, and the partials take room)
   for (uint32_t cuts = 1; cuts <= most; ++cuts) {
-    if (cuts == 1u || alone * cuts <= 256u)
+    if (takes_alone && (cuts == 1u || alone * cuts <= 256u))
       consider(batches_128_us(*launch, batch_rows, cuts), 0u, cuts);
-    if (cuts == 1u || together * cuts <= 512u)
+    if (takes_shared && (cuts == 1u || together * cuts <= 512u))
       consider(shared_128_us(*launch, batch_rows, cuts), 1u, cuts);
   }
   return shared;
@@ -3106,7 +3118,7 @@ extern "C" int32_t qllm_attention_paged_q4h_prompt(
           (launch->output_gated ? 2u : 1u) * launch->head_dim ||
       (launch->output_kind != QLLM_OUT_F32 &&
        launch->output_kind != QLLM_OUT_BF16) ||
-      launch->rows > 65535u * kPromptBatches ||
+      launch->rows > kBatchedRows * kPromptBatches ||
       launch->first_context_tokens > 0xffffffffu - (launch->rows - 1u))
     return fail(QLLM_INVALID_ARGUMENT, "invalid Q4H prompt attention");
   const uint32_t group = launch->query_heads / launch->kv_heads;

@@ -180,6 +180,31 @@ def test_launches_without_a_prompt_form(change):
                    ctypes.byref(splits)) == 0 and splits.value == 0
 
 
+@pytest.mark.parametrize("query_heads,kv_heads,rows,first,shared", [
+    (8, 1, 65535, 0, 0), (8, 1, 65536, 0, 1), (64, 2, 70000, 0, 1), (7, 7, 65536, 0, 1),
+    (7, 7, 100000, 60000, 1), (1, 1, 300000, 0, 1), (1, 1, 65535 * 8, 0, 1),
+    (1, 1, 65535 * 8 + 1, 0, None), (64, 8, 1 << 20, 0, None)])
+def test_prompt_forms_take_their_rows(query_heads, kv_heads, rows, first, shared):
+    """Batches of their own only for rows that launch takes, 65535, whatever the estimates
+    say; shared tiles up to eight times as many; beyond them no form."""
+    splits = ctypes.c_uint32(9)
+    form = qh.call("qllm_attention_paged_q4h_prompt_form",
+                   attention(rows, first, query_heads, kv_heads, head_dim=128),
+                   48 // (query_heads // kv_heads), 8, ctypes.byref(splits))
+    assert (form, splits.value > 0) == ((shared, True) if shared is not None else (0, False))
+
+
+@pytest.mark.parametrize("change", [dict(query_heads=15), dict(batch=13), dict(first=-1),
+                                    dict(first=0xffffffff - 100)])
+def test_sizes_that_no_prompt_form_takes(change):
+    sizes = {**dict(rows=1000, first=0, query_heads=16, kv_heads=4, head_dim=128, batch=12),
+             **change}
+    batch = sizes.pop("batch")
+    splits = ctypes.c_uint32(9)
+    assert qh.call("qllm_attention_paged_q4h_prompt_form", attention(**sizes), batch, 8,
+                   ctypes.byref(splits)) == 0 and splits.value == 0
+
+
 # ---- a norm with its projections ------------------------------------------------
 
 MIB = 1 << 20
