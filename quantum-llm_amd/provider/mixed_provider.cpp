@@ -892,10 +892,10 @@ void Mi355MixedProvider::release_pages(const MixedRequestState& state) {
 
 // Uploads a batch's words and makes its pages exist.  The pinned words are
 // free: every batch ends with its token, which the device hands over last.
+// `marked`: the step graph marks its token as emitted.
 void Mi355MixedProvider::begin_batch(MixedRequestState& state,
                                      std::span<const std::uint32_t> tokens,
-                                     std::uint32_t first_position,
-                                     const er::ProgramRequestContext& request) {
+                                     std::uint32_t first_position, bool marked) {
   const auto rows = static_cast<std::uint32_t>(tokens.size());
   if (!rows || rows > g_.chunk_rows)
     throw std::runtime_error("program batch holds too many or no tokens");
@@ -924,7 +924,7 @@ void Mi355MixedProvider::begin_batch(MixedRequestState& state,
   words[0] = first_position;
   words[1] = state.slot;
   words[2] = rows;
-  words[kStepMark] = TokenSelector::marks_handed(request, first_position + rows - 1U);
+  words[kStepMark] = marked ? 1U : 0U;
   words[kStepSequence] = selector_->next_handover();
   words[5] = 0U;
   std::copy(tokens.begin(), tokens.end(), words + kStepWords);
@@ -1308,12 +1308,14 @@ void Mi355MixedProvider::enqueue_head(std::uint32_t batch_rows, std::uint32_t fi
   enqueue_normed(norm, &s, 1U);
 }
 
-// The arg-max of the first row of logits, which hands itself over.
-void Mi355MixedProvider::enqueue_selection() {
-  const auto* step = step_.as<std::uint32_t>();
-  const qllm_token_handover handover{selector_->handed_words(), step + kStepSequence, 0U,
-                                     presence_.as<std::uint8_t>(), step + kStepMark,
-                                     step + 1, g_.vocabulary};
+// The arg-max of the first row of logits, which hands itself over and marks itself as
+// emitted in `emitted` (row *slot of it) where *mark is not 0; without `mark` always, with
+// null `emitted` never.
+void Mi355MixedProvider::enqueue_selection(std::uint8_t* emitted, const std::uint32_t* mark,
+                                           const std::uint32_t* slot) {
+  const qllm_token_handover handover{selector_->handed_words(),
+                                     step_.as<std::uint32_t>() + kStepSequence, 0U, emitted,
+                                     mark, slot, g_.vocabulary};
   status_check(qllm_argmax_batch_handed(logits_.as<float>(), g_.vocabulary, 1U,
                                         argmax_.as<std::uint32_t>(),
                                         select_workspace_.get(), select_workspace_bytes_,
@@ -1355,17 +1357,20 @@ Mi355MixedProvider::HeadResult Mi355MixedProvider::finish_batch(
     enqueue_head(rows, 0U, count, true);
     copy_rows(first, count);
   }
+  const std::uint32_t last_position = state.position + rows - 1U;
+  auto* const presence =
+      presence_.as<std::uint8_t>() + std::size_t{state.slot} * g_.vocabulary;
   if (!head_enqueued) {
     enqueue_head(rows, rows - 1U, 1U, false);
-    enqueue_selection();
+    // (the head's request decides, which need not be the one of the embedding)
+    enqueue_selection(
+        TokenSelector::marks_handed(request, last_position) ? presence : nullptr, nullptr,
+        nullptr);
   }
   if (last_wanted) copy_rows(before, 1U);
-  const std::uint32_t last_position = state.position + rows - 1U;
   state.position += rows;
-  result.token = selector_->select(
-      logits_.as<float>(),
-      presence_.as<std::uint8_t>() + std::size_t{state.slot} * g_.vocabulary,
-      argmax_.as<std::uint32_t>(), request, last_position, true);
+  result.token = selector_->select(logits_.as<float>(), presence, argmax_.as<std::uint32_t>(),
+                                   request, last_position, true);
   release_pages(state);
   program_steps_ += rows;
   if (rows > 1U) prompt_rows_ += rows;
@@ -1380,7 +1385,8 @@ void Mi355MixedProvider::launch_step_graph() {
     enqueue_embedding(1U, true);
     for (auto& block : blocks_) enqueue_block(*block, 1U, g_.max_context - 1U);
     enqueue_head(1U, 0U, 1U, false);
-    enqueue_selection();
+    const auto* step = step_.as<std::uint32_t>();
+    enqueue_selection(presence_.as<std::uint8_t>(), step + kStepMark, step + 1);
   };
   // the first token runs uncaptured: it loads every kernel it needs
   if (!use_graphs_ || !step_warm_) {
@@ -1492,7 +1498,7 @@ er::OperationExecutionHandle Mi355MixedProvider::execute(
     if (operation->kind == Kind::embedding) {
       const auto tokens = host_u32_batch(input("token_ids"), kTokenAbi,
                                          "embedding token batch", g_.chunk_rows);
-      begin_batch(*state, tokens, state->position, invocation.request);
+      begin_batch(*state, tokens, state->position, false);
       enqueue_embedding(batch_rows_, false);
       values.emplace("hidden", hidden_value(batch_rows_));
     } else if (operation->kind == Kind::head) {
@@ -1539,7 +1545,10 @@ er::OperationExecutionHandle Mi355MixedProvider::execute_program_sequence(
     const auto positions =
         host_u32_batch(input("positions"), kPositionAbi, "position batch", g_.chunk_rows);
     const auto first = contiguous_first(positions, tokens.size());
-    begin_batch(*state, tokens, first, invocation.request);
+    begin_batch(*state, tokens, first,
+                TokenSelector::marks_handed(
+                    invocation.request,
+                    first + static_cast<std::uint32_t>(tokens.size()) - 1U));
     const bool single = batch_rows_ == 1U;
     if (single) {
       launch_step_graph();

@@ -149,7 +149,7 @@ class Mi355MixedProvider final : public DecoderProvider {
   std::size_t scratch_bytes_for(std::uint32_t rows, std::uint32_t last_position) const;
   void ensure_workspace(std::uint32_t rows, std::uint32_t last_position);
   void begin_batch(MixedRequestState& state, std::span<const std::uint32_t> tokens,
-                   std::uint32_t first_position, const er::ProgramRequestContext& request);
+                   std::uint32_t first_position, bool marked);
   void enqueue_embedding(std::uint32_t rows, bool with_norm);
   void enqueue_normed(const qllm_stream_norm_launch& norm, const qllm_linear_segment* segments,
                       std::size_t count);
@@ -171,7 +171,8 @@ class Mi355MixedProvider final : public DecoderProvider {
     std::shared_ptr<std::vector<float>> logits;
     std::uint32_t token{};
   };
-  void enqueue_selection();
+  void enqueue_selection(std::uint8_t* emitted, const std::uint32_t* mark,
+                         const std::uint32_t* slot);
   HeadResult finish_batch(MixedRequestState& state, std::uint32_t rows,
                           const er::ProgramRequestContext& request, bool head_enqueued);
   void launch_step_graph();

@@ -1,12 +1,15 @@
 """Whole mixed-layer models through the framework's own entry points: the model
 folder, the compiled program, request slots and pages, sampling, the worker -
 against the plain float64 statement."""
+import ctypes
 import os
+from ctypes import c_char_p, c_int32, c_uint32, c_void_p
 
 import numpy as np
 import pytest
 import torch
 
+import artifact_lib as al
 import mixed_model as mm
 import mixer_oracle as mo
 import qllm_provider as qp
@@ -246,6 +249,25 @@ def test_sampling_follows_the_seed(mixed):
     once = generate(presence_ppm=2000000)
     assert once[0] == greedy[0]
     model.close()
+
+
+def test_the_head_request_decides_what_is_marked(mixed):
+    """One operation at a time, the embedding's request without sampling parameters: the
+    tokens of a request that all operations share, also under a penalty on those marked."""
+    al.probe()
+    probe = ctypes.CDLL(al.PROBE_LIBRARY).qprobe_operations
+    probe.argtypes = [c_char_p, c_void_p, c_uint32, c_uint32, c_uint32, c_int32, c_void_p]
+    prompt = np.ascontiguousarray(mixed.tokens[:20], dtype=np.uint32)
+
+    def tokens(penalised, bare):
+        out = np.zeros(41, dtype=np.uint32)
+        assert probe(os.fsencode(mixed.path), prompt.ctypes.data, prompt.size, 40, penalised,
+                     bare, out.ctypes.data) == 0
+        return out.tolist()
+
+    shared = tokens(12, 0)
+    assert shared != tokens(0, 0)         # the penalty has tokens to act on
+    assert tokens(12, 1) == shared
 
 
 def test_trace_replay_program(mixed, tmp_path):
