@@ -609,7 +609,11 @@ typedef struct qllm_q4h_attention_launch {
                                    reference's single Q8 plane) */
   const float* query_scales;    /* NULL, or the operand scales of the same call */
   const void* const* page_table;
-  void* output;                 /* [rows, query_heads, head_dim] */
+  void* output;                 /* [rows, query_heads, head_dim]; over no cache page.
+                                   Outputs over an input are stored when all of it
+                                   has been read; with device_positions the page
+                                   table counts as one up to the context that
+                                   first_context_tokens + rows - 1 names */
   float* partial_maxima;        /* [rows, maximum_splits, query_heads]; working
                                    space, which a launch of one split may leave
                                    as it is */
@@ -770,7 +774,7 @@ int32_t qllm_store_kv_paged_f16_batch(const float* key, const float* value,
 typedef struct qllm_f16_attention_launch {
   const float* query;
   const void* const* device_pages;
-  void* output;
+  void* output;                 /* and the partials: as in qllm_q4h_attention_launch */
   float* partial_maxima;
   float* partial_sums;
   float* partial_outputs;
@@ -852,7 +856,7 @@ int32_t qllm_qkv_rope_store_q8_batch(
 typedef struct qllm_q8_attention_launch {
   const float* query;
   const void* const* device_pages;
-  void* output;
+  void* output;                 /* and the partials: as in qllm_q4h_attention_launch */
   float* partial_maxima;
   float* partial_sums;
   float* partial_outputs;

@@ -411,6 +411,13 @@ struct AttentionInput {
   const void* data;   // may be null
   size_t bytes;
 };
+// The entries of a page table that a context of `tokens` takes (with positions on the
+// device: of the context that the launch's own words name).
+inline AttentionInput page_table_input(const void* const* table, uint32_t tokens,
+                                       uint32_t page_tokens) {
+  const uint64_t pages = (uint64_t{tokens} + page_tokens - 1u) / page_tokens;
+  return {table, sizeof(void*) * (pages ? pages : 1u)};
+}
 // Whether a launch's workgroups may write its outputs themselves: it has one split, the
 // outputs can be stored four at a time, and they lie over nothing that other workgroups
 // of the launch still read.  Otherwise the partials go through the combine's launch.

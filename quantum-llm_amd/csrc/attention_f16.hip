@@ -917,7 +917,9 @@ extern "C" int32_t qllm_attention_paged_f16(
           launch->output, launch->output_kind, launch->maximum_splits,
           launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
           {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
-                               launch->query_stride}})) {
+                               launch->query_stride},
+           page_table_input(launch->device_pages, last_context,
+                            launch->device_page_tokens)})) {
     args.output = launch->output;
     args.output_kind = launch->output_kind;
     args.output_gated = launch->output_gated != 0 ? 1u : 0u;
@@ -994,7 +996,9 @@ extern "C" int32_t qllm_attention_paged_f16_batched(
           launch->output, launch->output_kind, launch->maximum_splits,
           launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
           {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
-                               launch->query_stride}})) {
+                               launch->query_stride},
+           page_table_input(launch->device_pages, last_context,
+                            launch->device_page_tokens)})) {
     args.output = launch->output;
     args.output_kind = launch->output_kind;
     args.output_gated = launch->output_gated != 0 ? 1u : 0u;
@@ -1103,7 +1107,10 @@ extern "C" int32_t qllm_attention_paged_q8(const qllm_q8_attention_launch* launc
           launch->output, launch->output_kind, launch->maximum_splits,
           launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
           {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
-                               launch->query_stride}})) {
+                               launch->query_stride},
+           page_table_input(launch->device_pages, last_context,
+                            launch->page_tokens),
+           {launch->device_positions, 3u * sizeof(uint32_t)}})) {
     args.output = launch->output;
     args.output_kind = launch->output_kind;
     args.output_gated = launch->output_gated != 0 ? 1u : 0u;
@@ -1181,7 +1188,9 @@ extern "C" int32_t qllm_attention_paged_q8_batched(
           launch->output, launch->output_kind, launch->maximum_splits,
           launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
           {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
-                               launch->query_stride}})) {
+                               launch->query_stride},
+           page_table_input(launch->device_pages, last_context,
+                            launch->page_tokens)})) {
     args.output = launch->output;
     args.output_kind = launch->output_kind;
     args.output_gated = launch->output_gated != 0 ? 1u : 0u;

@@ -2993,7 +2993,8 @@ int32_t attend_batches(const qllm_q4h_attention_launch* launch, uint32_t batch_r
           launch->output, launch->output_kind, launch->maximum_splits,
           launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
           {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
-                               launch->query_stride}})) {
+                               launch->query_stride},
+           page_table_input(launch->page_table, last_context, launch->page_tokens)})) {
     args.output = launch->output;
     args.output_kind = launch->output_kind;
     args.output_gated = launch->output_gated != 0 ? 1u : 0u;
@@ -3127,6 +3128,7 @@ extern "C" int32_t qllm_attention_paged_q4h_prompt(
                 "Q4H prompt attention: batch_rows * (query_heads/kv_heads) "
                 "exceeds 48");
   const uint32_t batches = (launch->rows + batch_rows - 1u) / batch_rows;
+  const uint32_t last_context = launch->first_context_tokens + launch->rows - 1u;
   SplitArgs args{};
   args.query = launch->query;
   args.query_stride = launch->query_stride;
@@ -3149,7 +3151,8 @@ extern "C" int32_t qllm_attention_paged_q4h_prompt(
           launch->output, launch->output_kind, launch->maximum_splits,
           launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
           {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
-                               launch->query_stride}})) {
+                               launch->query_stride},
+           page_table_input(launch->page_table, last_context, launch->page_tokens)})) {
     args.output = launch->output;
     args.output_kind = launch->output_kind;
     args.output_gated = launch->output_gated != 0 ? 1u : 0u;
@@ -3239,6 +3242,7 @@ int32_t launch_q4h_attention(const qllm_q4h_attention_launch* launch,
           launch->split_tokens, launch->rows, launch->query_heads, launch->head_dim,
           {{launch->query, sizeof(float) * launch->rows * launch->query_heads *
                                launch->query_stride},
+           page_table_input(launch->page_table, last_context, launch->page_tokens),
            {args.query_operands,
             launch->kv_heads * q4h_operand_plane_bytes(row_tiles, launch->head_dim)},
            {args.query_operand_scales, sizeof(float) * 16u * row_tiles * launch->kv_heads},

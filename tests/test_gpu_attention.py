@@ -8,6 +8,7 @@ import gpu_util as gu
 import oracle_lib as ol
 import qllm_hip as qh
 import synth
+import test_gpu_attention_q8 as q8
 
 pytestmark = pytest.mark.gpu
 
@@ -723,3 +724,80 @@ def test_a_last_tile_alone(device, tokens, rows, Q, KV, d, gated, splits):
     for a, b, c in zip(*(r[1] for r in results)):
         assert np.array_equal(a, b) and np.array_equal(a, c)
     gu.assert_close(results[1][0], results[0][0].astype(np.float64), what="other deal")
+
+
+def pages_of(device, rng, cache, tokens, KV, d, page):
+    """(device pages, the oracle's pages) of random keys and values."""
+    if cache == "q8":
+        return q8.build_cache(device, rng, tokens, KV, d, page, 1024)[::2]
+    keys, values = (rng.standard_normal((tokens, KV, d)).astype(np.float32) for _ in range(2))
+    pages = (synth.q4h_pages(keys, values, page, 1, 0) if cache == "q4h"
+             else synth.f16_pages(keys, values, page))
+    return [gu.device_tensor(p, device) for p in pages], pages
+
+
+@pytest.mark.parametrize("cache,form,tokens,rows,Q,KV,d,gated,kind,batch,direct", [
+    ("q4h", "", 100, 5, 64, 8, 128, False, qh.OUT_BF16, 0, True),
+    ("q4h", "", 300, 5, 24, 4, 256, True, qh.OUT_F32, 0, True),
+    ("q4h", "_batched", 200, 40, 16, 4, 128, True, qh.OUT_F32, 12, True),
+    ("q4h", "_batched", 100, 41, 24, 4, 256, False, qh.OUT_BF16, 5, True),
+    ("q4h", "_prompt", 430, 400, 64, 8, 128, False, qh.OUT_BF16, 6, True),   # 72 workgroups
+    ("q4h", "_prompt", 400, 400, 64, 8, 128, True, qh.OUT_F32, 6, True),
+    ("q4h", "_prompt", 300, 300, 64, 8, 128, False, qh.OUT_F32, 6, False),   # 56
+    ("f16", "", 60, 4, 16, 4, 128, False, qh.OUT_BF16, 0, True),    # one, two, three row tiles
+    ("f16", "", 700, 5, 16, 4, 128, True, qh.OUT_F32, 0, True),
+    ("f16", "", 100, 5, 64, 8, 128, False, qh.OUT_F32, 0, True),
+    ("f16", "", 300, 2, 24, 4, 256, True, qh.OUT_BF16, 0, True),
+    ("f16", "", 300, 5, 24, 4, 256, True, qh.OUT_BF16, 0, False),   # two tiles at 256
+    ("f16", "_batched", 90, 40, 64, 8, 128, False, qh.OUT_BF16, 6, True),
+    ("f16", "_batched", 70, 21, 24, 4, 256, True, qh.OUT_F32, 2, True),
+    ("q8", "", 100, 5, 64, 8, 128, False, qh.OUT_BF16, 0, True),
+    ("q8", "", 40, 1, 24, 4, 256, True, qh.OUT_F32, 0, True),
+    ("q8", "_batched", 90, 40, 16, 4, 128, True, qh.OUT_F32, 12, True),
+    ("q8", "_batched", 70, 21, 24, 4, 256, False, qh.OUT_BF16, 2, True)])
+def test_one_split_of_every_form(device, cache, form, tokens, rows, Q, KV, d, gated, kind, batch,
+                                 direct):
+    """The oracle's attention by a launch of one split into a buffer of its own, and the same
+    bits by way of the partials where the outputs lie off a 16-byte line, over the query or
+    over the page table, which other workgroups still read."""
+    rng = np.random.default_rng(tokens + Q + d)
+    page, first, stride = 64, tokens - (rows - 1), d * (2 if gated else 1)
+    d_pages, pages = pages_of(device, rng, cache, tokens, KV, d, page)
+    query = rng.standard_normal((rows, Q, stride)).astype(np.float32)
+    shape = ol.AttentionShape(rows, Q, KV, d, first, page, 0, int(gated))
+    want = (ol.attention_q4h(shape, query, pages) if cache == "q4h"
+            else ol.attention_f16(shape, query, pages, True) if cache == "f16"
+            else ol.attention_q8(shape, query, pages, 1024))
+    addresses = torch.tensor([p.data_ptr() for p in d_pages], dtype=torch.int64, device=device)
+    type_ = torch.bfloat16 if kind == qh.OUT_BF16 else torch.float32
+    count = rows * Q * d
+    got = []
+    for where in ["own", "shifted", "over the table"] + ([] if gated else ["over the query"]):
+        maxima, sums = torch.zeros((2, rows, 1, Q), device=device)
+        partials = torch.full((rows, 1, Q, d), -1.0, device=device)
+        d_query = gu.device_tensor(query, device)
+        whole = (d_query.view(-1).view(type_) if where == "over the query"
+                 else torch.zeros(count + 16, dtype=type_, device=device))
+        begin = 2 if where == "shifted" else 0
+        table = addresses.clone()
+        if where == "over the table":
+            table = whole.view(torch.uint8)[32:32 + 8 * len(pages)].view(torch.int64)
+            table.copy_(addresses)
+        common = (qh.ptr(table), whole.data_ptr() + begin * whole.element_size(), qh.ptr(maxima),
+                  qh.ptr(sums), qh.ptr(partials))
+        heads = (Q, KV, d, 0, 1, stride, int(gated), kind, None)
+        if cache == "q4h":
+            launch = qh.Q4hAttentionLaunch(qh.ptr(d_query), 0, 0, *common, first, rows, 0, page,
+                                           *heads)
+        elif cache == "f16":
+            launch = qh.F16AttentionLaunch(qh.ptr(d_query), *common, first, rows, 0, page, *heads)
+        else:
+            launch = qh.Q8AttentionLaunch(qh.ptr(d_query), *common, 1024, first, rows, page,
+                                          *heads)
+        qh.call(f"qllm_attention_paged_{cache}{form}", launch, *([batch] if batch else []))
+        torch.cuda.synchronize()
+        assert bool((partials == -1.0).all()) == (direct and where == "own"), where
+        got.append(whole[begin:begin + count].float().cpu().numpy().reshape(rows, Q, d))
+    gu.assert_close(got[0], want, what=f"one split over {cache}")
+    for other in got[1:]:
+        assert np.array_equal(got[0], other)
