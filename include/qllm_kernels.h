@@ -794,6 +794,11 @@ typedef struct qllm_f16_attention_launch {
 } qllm_f16_attention_launch;
 
 int32_t qllm_attention_paged_f16(const qllm_f16_attention_launch* launch);
+/* maximum_splits, 1 to `most` (for a workgroup a compute unit), with which that launch
+ * (split_tokens 0) takes the least time over a context of so many tokens, every wave with
+ * one tile at most; 0 where that takes more splits than `most` or, at head_dim 128, 32. */
+uint32_t qllm_attention_paged_f16_splits(uint32_t context_tokens, uint32_t head_dim,
+                                         uint32_t most);
 /* The batched form for prompt prefill, as qllm_attention_paged_q4h_batched. */
 int32_t qllm_attention_paged_f16_batched(const qllm_f16_attention_launch* launch,
                                          uint32_t batch_rows);

@@ -19,6 +19,8 @@
 // multiplies the score and the V scale the probability.
 #include "attention_common.hpp"
 
+#include <algorithm>
+
 namespace qllm {
 namespace {
 
@@ -861,6 +863,32 @@ extern "C" int32_t qllm_store_kv_paged_f16_batch(
                                           first_cache_position, kv_heads,
                                           head_dim);
   return launched("F16 K/V store");
+}
+
+// A wave with one tile of 32 tokens is as fast as it gets, so the workgroups are as many as
+// that takes - and more of a short context, whose tiles a few compute units would fetch on
+// their own.  At head_dim 128 the combine fetches up to 32 splits in one go; beyond them two
+// tiles a wave are no slower.  Us a launch over splits, in a replayed graph:
+//   16 heads on 4 of 128, one row: 250 tokens 1: 5.9, 2: 7.4, 16: 7.0, 64: 10.5; 700 tokens
+//     3: 7.7, 8: 7.2, 16: 7.1; 4000 tokens 8: 8.7, 16: 7.7, 64: 10.7
+//   64 on 8 of 128, five rows: 700 tokens 2: 12.7, 8: 11.0, 16: 11.7, 32: 12.9
+//   24 on 4 of 256, five rows: 270 tokens 2: 15.4, 16: 13.7, 64: 19.5; 3000 tokens 8: 25.2,
+//     16: 16.9, 32: 15.6, 64: 20.8; 9000 tokens 18: 34.0, 32: 31.0, 36: 22.8, 64: 25.1
+extern "C" uint32_t qllm_attention_paged_f16_splits(uint32_t context_tokens,
+                                                    uint32_t head_dim, uint32_t most) {
+  if (!context_tokens || !most || (head_dim != 128u && head_dim != 256u)) return 0u;
+  const auto cut = [&](uint32_t tokens) { return (context_tokens - 1u) / tokens + 1u; };
+  const uint32_t room = head_dim == 128u ? std::min(most, 32u) : most;
+  const uint32_t single = cut(kSplitWaves * kF16Tile);
+  if (single > room) return 0u;
+  uint32_t splits = single;
+  if (head_dim == 128u) {
+    // (some 64 workgroups: `most` is 256 of them)
+    if (single > 1u) splits = std::max(splits, std::clamp(most / 4u, 8u, 16u));
+  } else if (context_tokens > 64u) {
+    splits = std::max({splits, std::min(16u, cut(32u)), std::min(32u, cut(64u))});
+  }
+  return std::min(splits, room);
 }
 
 extern "C" int32_t qllm_attention_paged_f16(

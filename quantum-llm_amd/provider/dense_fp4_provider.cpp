@@ -179,28 +179,34 @@ std::uint64_t Mi355DenseFp4Provider::kv_bytes_per_token_layer() const noexcept {
   return std::uint64_t{g_.kv_heads} * 2U * (g_.head_dim / 2U + 2U);
 }
 
-// Context splits of a verify step.  As long as the chip has room for them, as many as it
-// takes for every wave of a workgroup (eight) to have one tile at the longest context -
-// 64 tokens of the Q4H cache, whose last tile has a workgroup of its own, 32 of the exact
-// one - because a second tile takes longer than a further split costs the combine.  Up
-// to 32, which it fetches in one go, and beyond them where a tile of the exact cache is
-// 256 dimensions wide.  Five rows, splits of 512 tokens and for a tile a wave: Q4H, 16
-// heads on 4 of 128 dimensions after 1000 tokens 15.4 and 13.0 us, after 4000 14.3 and
-// 13.0, 24 heads on 4 of 256 after 4000 23.8 and 20.3; exact, 16 on 4 of 128 after 4000
-// 11.4 and 9.7, 24 on 4 of 256 after 4000 26.2 and 18.0, after 8000 33.0 and 21.8.
+// Context splits of a verify step over the Q4H cache, fixed for the replayed graph: as long
+// as the chip has room for them, as many as it takes for every wave of a workgroup (eight)
+// to have one tile of 64 tokens at the longest context, the last tile in a workgroup of its
+// own, because a second tile takes longer than a further split costs the combine.  Up to
+// 32, which it fetches in one go.  Five rows, splits of 512 tokens and for a tile a wave: 16
+// heads on 4 of 128 dimensions after 1000 tokens 15.4 and 13.0 us, after 4000 14.3 and 13.0,
+// 24 heads on 4 of 256 after 4000 23.8 and 20.3; a context of one tile within a longest of
+// 4000 13.3 and 13.2, one row alone 9.8 and 10.0.
+// Over the exact cache, whose launches know their context: the splits where that has too
+// many tiles for one a wave.
 std::uint32_t Mi355DenseFp4Provider::verify_splits(std::uint32_t most) const noexcept {
-  const auto cut = [&](std::uint32_t tokens) {
-    return std::max(1U, (g_.max_context - 1U) / tokens + 1U);
-  };
-  const bool q4h = g_.kv_encoding == KvEncoding::q4_f16_per_head;
+  const std::uint32_t cut = std::max(1U, (g_.max_context - 1U) / 512U + 1U);
   // (the codes of Q8 rows move by one with every other order of the sums between them)
-  if (g_.activation_q8) return std::min(most, cut(512U));
+  if (g_.activation_q8 || g_.kv_encoding != KvEncoding::q4_f16_per_head)
+    return std::min(most, cut);
   // One split writes the outputs itself: five rows of 16 heads on 4 after 500 tokens
   // 12.8 us, 13.0 in three (15.6 in two that count the tail as sixteen tiles).
-  if (q4h && g_.max_context <= 512U) return 1U;
-  const std::uint32_t single = q4h ? cut(512U) + 1U : cut(256U);
-  const std::uint32_t room = q4h || g_.head_dim == 128U ? std::min(most, 32U) : most;
-  return single <= room ? single : std::min(most, cut(512U));
+  if (g_.max_context <= 512U) return 1U;
+  const std::uint32_t single = cut + 1U;
+  return single <= std::min(most, 32U) ? single : std::min(most, cut);
+}
+
+// Context splits of a verify step over the exact cache.
+std::uint32_t Mi355DenseFp4Provider::exact_splits(std::uint32_t context) const noexcept {
+  if (g_.activation_q8) return verify_splits_;
+  const std::uint32_t splits =
+      qllm_attention_paged_f16_splits(context, g_.head_dim, most_splits_);
+  return splits ? splits : verify_splits_;
 }
 
 void Mi355DenseFp4Provider::allocate_workspaces() {
@@ -284,15 +290,21 @@ void Mi355DenseFp4Provider::allocate_workspaces() {
   // Context splits: kv_heads * splits workgroups fill the 256 CUs; the
   // attention kernels deal the context's tiles evenly over them themselves
   // (split_tokens 0), whatever the context length.
-  const std::uint32_t wanted_splits =
-      std::max(1U, 256U / std::max(1U, g_.kv_heads));
+  most_splits_ = std::max(1U, 256U / std::max(1U, g_.kv_heads));
   split_tokens_ = 0U;
   maximum_splits_ =
-      std::min(wanted_splits, std::max(1U, (g_.max_context + 511U) / 512U));
+      std::min(most_splits_, std::max(1U, (g_.max_context + 511U) / 512U));
   prefill_splits_ = std::min(maximum_splits_, 8U);
-  verify_splits_ = verify_splits(wanted_splits);
-  const std::size_t partials =
-      rows * std::max(maximum_splits_, verify_splits_) * g_.query_heads;
+  verify_splits_ = verify_splits(most_splits_);
+  // (the most of any context)
+  std::uint32_t partial_splits = std::max(maximum_splits_, verify_splits_);
+  if (g_.kv_encoding == KvEncoding::fp16)
+    for (std::uint64_t context = 32U; context < std::uint64_t{g_.max_context} + 32U;
+         context += 32U)
+      partial_splits = std::max(
+          partial_splits, exact_splits(static_cast<std::uint32_t>(
+                              std::min<std::uint64_t>(context, g_.max_context))));
+  const std::size_t partials = rows * partial_splits * g_.query_heads;
   partial_maxima_ = static_cast<float*>(device_alloc(partials * 4U));
   partial_sums_ = static_cast<float*>(device_alloc(partials * 4U));
   partial_outputs_ =
@@ -1291,7 +1303,7 @@ void Mi355DenseFp4Provider::enqueue_attention(
     launch.kv_heads = g_.kv_heads;
     launch.head_dim = g_.head_dim;
     launch.split_tokens = split_tokens_;
-    launch.maximum_splits = verify_splits_;
+    launch.maximum_splits = exact_splits(first_position + rows);
     launch.query_stride = query_stride;
     launch.output_gated = g_.output_gated;
     launch.output_kind = g_.activation_q8 ? QLLM_OUT_F32 : QLLM_OUT_BF16;
@@ -2284,7 +2296,7 @@ er::Status Mi355DenseFp4Provider::time_kernel(const std::string& which,
         launch.kv_heads = g_.kv_heads;
         launch.head_dim = g_.head_dim;
         launch.split_tokens = split_tokens_;
-        launch.maximum_splits = verify_splits_;
+        launch.maximum_splits = exact_splits(context_tokens + rows);
         launch.query_stride = query_stride;
         launch.output_gated = g_.output_gated;
         launch.output_kind = QLLM_OUT_BF16;

@@ -302,6 +302,7 @@ class Mi355DenseFp4Provider final : public DecoderProvider {
                                    std::size_t input_bytes, std::uint32_t rows,
                                    bool leave_partials);
   [[nodiscard]] std::uint32_t verify_splits(std::uint32_t most) const noexcept;
+  [[nodiscard]] std::uint32_t exact_splits(std::uint32_t context) const noexcept;
   [[nodiscard]] std::uint32_t prefill_splits_for(
       std::uint32_t rows, std::uint32_t attention_batch) const noexcept;
   [[nodiscard]] std::uint32_t prompt_attention_splits(
@@ -429,7 +430,8 @@ class Mi355DenseFp4Provider final : public DecoderProvider {
   std::uint64_t mtp_page_offset_{};   // the proposer's Q8 layer inside a page
   std::uint32_t split_tokens_{};
   std::uint32_t maximum_splits_{};
-  std::uint32_t verify_splits_{};   // of a verify step's attention
+  std::uint32_t verify_splits_{};   // of a verify step's attention (exact_splits)
+  std::uint32_t most_splits_{};     // for a workgroup a compute unit
 
   // workspaces (device)
   std::uint32_t max_rows_{};

@@ -278,6 +278,7 @@ SIGNATURES = {
     "qllm_attention_paged_q4h_prompt_form": (c_uint32, [POINTER(Q4hAttentionLaunch), c_uint32, c_uint32, POINTER(c_uint32)]),
     "qllm_attention_paged_q4h_prompt": (c_int32, [POINTER(Q4hAttentionLaunch), c_uint32]),
     "qllm_store_kv_paged_f16_batch": (c_int32, [c_void_p, c_void_p, c_void_p, c_uint32, c_uint32, c_uint32, c_uint32, c_uint32, c_uint32, c_void_p]),
+    "qllm_attention_paged_f16_splits": (c_uint32, [c_uint32, c_uint32, c_uint32]),
     "qllm_attention_paged_f16": (c_int32, [POINTER(F16AttentionLaunch)]),
     "qllm_attention_paged_f16_batched": (c_int32, [POINTER(F16AttentionLaunch), c_uint32]),
     "qllm_attention_paged_q8_batched": (c_int32, [POINTER(Q8AttentionLaunch), c_uint32]),

@@ -205,6 +205,29 @@ def test_sizes_that_no_prompt_form_takes(change):
                    ctypes.byref(splits)) == 0 and splits.value == 0
 
 
+@pytest.mark.parametrize("head_dim,most", [(128, 64), (128, 32), (128, 8), (256, 64), (256, 16),
+                                           (256, 1)])
+def test_exact_splits_follow_the_context(head_dim, most):
+    """A tile of 32 tokens a wave at most, as long as there is room; never fewer splits for a
+    longer context."""
+    room = min(most, 32) if head_dim == 128 else most
+
+    def splits(context):
+        return qh.call("qllm_attention_paged_f16_splits", context, head_dim, most)
+
+    assert splits(0) == 0 and splits(1) == splits(64) == 1
+    before = 1
+    for context in list(range(1, 20000, 31)) + [256 * room, 256 * room + 1, 0xffffffff]:
+        found = splits(context)
+        if context > 256 * room:
+            assert found == 0
+            continue
+        assert before <= found <= room and found * 256 >= context
+        assert found <= max(-(-context // 32), 16) and (found == 1 or context > 64)
+        before = found if context < 19900 else 1
+    assert qh.call("qllm_attention_paged_f16_splits", 100, 64, most) == 0
+
+
 # ---- a norm with its projections ------------------------------------------------
 
 MIB = 1 << 20
