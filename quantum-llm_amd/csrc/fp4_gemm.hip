@@ -809,15 +809,18 @@ int32_t launch_mfma(GemmArgs args, int scheme, bool tiled, uint32_t batch,
     }
   }
   // Four waves split K; eight where the launch has at most one workgroup a CU, which then
-  // waits for its own chain of chunks, and the chunks are enough to share.  A launch
-  // alone, five rows, four and eight waves: binary16 scales, 2048 rows, 11 and 16 chunks
-  // a workgroup 3.9 / 4.7 and 4.0 / 4.6 us, 21 5.1 / 5.0, 32 5.2 / 4.9, 88 9.8 / 7.8;
-  // UE8M0 4.0 / 4.3, 4.1 / 4.3, 4.8 / 4.5, 5.4 / 4.7.  Gate and up, whose waves have two
-  // tiles' loads in flight, 4096 rows: binary16 16, 32 and 64 chunks 5.3 / 6.6, 7.1 / 7.3
-  // and 10.7 / 9.7, UE8M0 5.4 / 5.9, 7.2 / 6.9 and 11.3 / 9.3.
+  // waits for its own chain of chunks, and the chunks are enough to share.  Eight against
+  // four waves, mean and worst of 4 to 20 matrices of 64 to 8192 rows, a launch alone:
+  //   binary16 scales, 16 chunks a workgroup 1.17 and 1.19, 19 1.00 and 1.03, 21 0.98, 32
+  //   0.94; UE8M0 16 1.07 and 1.10, 17 0.95 and 0.98, 19 0.94 and 0.96, all at five rows
+  //   gate and up, whose waves have two tiles' loads in flight, binary16: five rows, 40
+  //   chunks 1.07 and 1.09, 48 1.02 and 1.07, 52 0.94 and 0.98, 64 0.92; eight rows, 48
+  //   1.08 and 1.09, 72 1.03 and 1.06, 80 1.02 and 1.03, 88 0.95 and 0.97.  UE8M0: five
+  //   rows, 28 0.96 and 1.00, 40 0.96; eight rows, 40 1.02 and 1.09, 48 0.98 and 1.00
   const uint32_t chunks = args.padded_columns / kChunk / splits;
-  uint32_t enough = 20u;
-  if (swiglu) enough = scheme == kSchemeF16 ? 40u : 28u;
+  const bool f16 = scheme == kSchemeF16, many = batch > 6u;
+  uint32_t enough = f16 ? 20u : 17u;
+  if (swiglu) enough = f16 ? (many ? 88u : 52u) : (many ? 48u : 28u);
   if (args.activation_scales) enough = swiglu ? ~0u : 0u;
   const uint32_t waves = tiles <= 256u && chunks >= enough ? 8u : 4u;
 #define QLLM_LAUNCH(SCHEME_, TILES_, TILED_)                                  \

@@ -187,6 +187,36 @@ def test_fused_swiglu_matches_oracle(device, scheme):
                     what="swiglu")
 
 
+@pytest.mark.parametrize("scheme", [ol.SCALE_F16_BLOCK16, ol.SCALE_UE8M0_BLOCK32])
+@pytest.mark.parametrize("batch", [1, 6, 7])
+def test_projections_on_either_side_of_eight_waves(device, scheme, batch):
+    """Chunks of 64 columns from which eight waves share a workgroup's, not four: rows of a
+    projection, and of gate and up, on both sides of the line."""
+    rng = np.random.default_rng(batch + scheme)
+    rows = 96
+    for chunks in (16, 17, 19, 20):
+        codes, scales = synth.fp4_matrix(rng, rows, 64 * chunks, scheme)
+        act = ol.bf16_round(rng.standard_normal((batch, 64 * chunks)).astype(np.float32))
+        want = ol.fp4_linear_f64(codes, scales, scheme, rows, 64 * chunks, act)
+        gu.assert_close(gu.gemm(device, codes, scales, scheme, rows, 64 * chunks, act), want,
+                        what=f"{chunks} chunks")
+    for chunks in (27, 28, 47, 48, 51, 52, 87, 88):
+        padded = 64 * chunks
+        pair = [synth.fp4_matrix(rng, rows, padded, scheme) for _ in range(2)]
+        act = ol.bf16_round(0.02 * rng.standard_normal((batch, padded)).astype(np.float32))
+        want = ol.silu_product(*(ol.fp4_linear_f64(*m, scheme, rows, padded, act)
+                                 for m in pair), True)
+        tensors = [[gu.device_tensor(x, device) for x in m] for m in pair]
+        matrices = [qh.prepack(qh.fp4_matrix(*m, rows, padded, padded, scheme), device)
+                    for m in tensors]
+        d_act = gu.device_tensor(ol.bf16_bits(act), device)
+        out = torch.zeros((batch, rows), dtype=torch.bfloat16, device=device)
+        qh.call("qllm_fp4_swiglu_bf16", matrices[0][0], matrices[1][0], qh.ptr(d_act),
+                d_act.numel() * 2, qh.ptr(out), batch, None)
+        torch.cuda.synchronize()
+        gu.assert_close(out.float().cpu().numpy(), want, what=f"gate and up, {chunks} chunks")
+
+
 def test_q8_gemv_matches_reference_integer_statement(device):
     """Reference arithmetic (ABI 3 weights x Q8 activations), fixture of
     runtime/tools/dense_fp4_cuda_smoke.cpp:139-216, threshold 2e-4 (:4911)."""
