@@ -275,6 +275,7 @@ constexpr uint32_t kSelectThreads = 1024;
 constexpr uint32_t kSelectCandidates = 4096;
 constexpr uint32_t kSelectMaxChunks = 4096;
 constexpr uint32_t kSelectMaxK = 64;
+constexpr uint32_t kSelectItems = 4;   // of a thread on their way at a time
 
 __global__ __launch_bounds__(256) void chunk_max_kernel(
     const float* values, uint32_t count, size_t row_stride, uint32_t chunk,
@@ -332,6 +333,14 @@ __global__ __launch_bounds__(kSelectThreads) void topk_threshold_kernel(
                          __HIP_MEMORY_SCOPE_SYSTEM);
   };
 
+  // (a short row is read once, with the maxima, whatever the threshold will be)
+  const bool whole = count <= kSelectItems * kSelectThreads;
+  float early[kSelectItems];
+  if (whole)
+#pragma unroll
+    for (uint32_t i = 0; i < kSelectItems; ++i)
+      early[i] = row[min(i * kSelectThreads + threadIdx.x, count - 1u)];
+
   // the k-th largest chunk maximum (staged in candidate_values)
   if (threadIdx.x == 0u) {
     threshold = -INFINITY;
@@ -354,32 +363,42 @@ __global__ __launch_bounds__(kSelectThreads) void topk_threshold_kernel(
     }
   __syncthreads();
   const float limit = threshold;
-  // chunks without such an item are not read again
-  for (uint32_t item = threadIdx.x; item < chunks_per_row; item += kSelectThreads)
-    if (candidate_values[item] >= limit)
-      high_chunks[atomicAdd(&high_count, 1u)] = static_cast<uint16_t>(item);
-  __syncthreads();   // the staged maxima are overwritten from here on
+  const auto keep = [&](float value, uint32_t item) {
+    if (!(value >= limit)) return;   // (false for NaN)
+    const uint32_t slot = atomicAdd(&candidates, 1u);
+    if (slot < kSelectCandidates) {
+      candidate_values[slot] = value;
+      candidate_indices[slot] = item;
+    }
+  };
+  if (whole) {
+#pragma unroll
+    for (uint32_t i = 0; i < kSelectItems; ++i)
+      if (const uint32_t item = i * kSelectThreads + threadIdx.x; item < count)
+        keep(early[i], item);
+  } else {
+    // chunks without such an item are not read again
+    for (uint32_t item = threadIdx.x; item < chunks_per_row; item += kSelectThreads)
+      if (candidate_values[item] >= limit)
+        high_chunks[atomicAdd(&high_count, 1u)] = static_cast<uint16_t>(item);
+    __syncthreads();   // the staged maxima are overwritten from here on
 
-  // a wave per chunk, four items a lane on their way at a time
-  const uint32_t lane = threadIdx.x & 63u;
-  for (uint32_t high = threadIdx.x >> 6; high < high_count; high += kSelectThreads / 64u) {
-    const uint32_t begin = high_chunks[high] * chunk;
-    const uint32_t end = min(count, begin + chunk);
-    for (uint32_t first = begin + lane; first < end; first += 256u) {
-      float value[4];
+    // a wave per piece of 256 items, four a lane on their way at a time: of a small k a
+    // few chunks are all that is read again, and long ones (five rows of 151936, k = 1:
+    // 92 us with a wave to a chunk, 82 with all items read again, 66 so)
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t shift = chunk > 256u ? 31u - __clz(chunk) - 8u : 0u;   // pieces of a chunk
+    for (uint32_t work = threadIdx.x >> 6; work < high_count << shift;
+         work += kSelectThreads / 64u) {
+      const uint32_t begin = high_chunks[work >> shift] * chunk;
+      const uint32_t end = min(count, begin + chunk);
+      const uint32_t first = begin + (work & ((1u << shift) - 1u)) * 256u + lane;
+      float value[kSelectItems];
 #pragma unroll
-      for (uint32_t i = 0; i < 4u; ++i) value[i] = row[min(first + 64u * i, end - 1u)];
+      for (uint32_t i = 0; i < kSelectItems; ++i) value[i] = row[min(first + 64u * i, end - 1u)];
 #pragma unroll
-      for (uint32_t i = 0; i < 4u; ++i) {
-        const uint32_t item = first + 64u * i;
-        if (item < end && value[i] >= limit) {   // false for NaN
-          const uint32_t slot = atomicAdd(&candidates, 1u);
-          if (slot < kSelectCandidates) {
-            candidate_values[slot] = value[i];
-            candidate_indices[slot] = item;
-          }
-        }
-      }
+      for (uint32_t i = 0; i < kSelectItems; ++i)
+        if (const uint32_t item = first + 64u * i; item < end) keep(value[i], item);
     }
   }
   __syncthreads();

@@ -327,7 +327,9 @@ def test_batched_topk_when_the_threshold_does_not_filter(device):
 
 
 @pytest.mark.parametrize("rows,count,top_k", [(5, 32000, 20), (8, 300, 64), (1, 64, 1),
-                                              (3, 151936, 64), (2, 65537, 7)])
+                                              (3, 151936, 64), (2, 65537, 7),
+                                              (3, 4096, 9), (3, 4097, 1), (2, 4097, 64),
+                                              (4, 151936, 1), (2, 40000, 2), (1, 262145, 3)])
 def test_batched_topk_by_hand_over(device, rows, count, top_k):
     """Into pinned memory: the words of the launch into device memory and, once a row's
     number is there, nothing that was there before; rows of few values, of ties only (the k
