@@ -180,8 +180,22 @@ def test_launches_without_a_prompt_form(change):
                    ctypes.byref(splits)) == 0 and splits.value == 0
 
 
+@pytest.mark.parametrize("query_heads,kv_heads,rows,first,form", [
+    (48, 8, 1168, 0, (1, 2)), (32, 32, 2196, 193, (1, 2)), (32, 8, 1156, 0, (1, 3)),
+    (16, 8, 4302, 0, (1, 2)), (28, 4, 1199, 0, (1, 3)), (64, 2, 572, 168, (1, 2)),
+    (40, 40, 589, 0, (0, 1))])
+def test_prompt_forms_of_close_estimates(query_heads, kv_heads, rows, first, form):
+    """Where the estimates are close, batches of their own up to 31 of them and splits for
+    one workgroup a compute unit: 6 to 14 % less than the least of the estimates took."""
+    splits = ctypes.c_uint32()
+    shared = qh.call("qllm_attention_paged_q4h_prompt_form",
+                     attention(rows, first, query_heads, kv_heads, head_dim=128),
+                     48 // (query_heads // kv_heads), 8, ctypes.byref(splits))
+    assert (shared, splits.value) == form
+
+
 @pytest.mark.parametrize("query_heads,kv_heads,rows,first,shared", [
-    (8, 1, 65535, 0, 0), (8, 1, 65536, 0, 1), (64, 2, 70000, 0, 1), (7, 7, 65536, 0, 1),
+    (1, 1, 65535, 0, 0), (1, 1, 65536, 0, 1), (8, 1, 65536, 0, 1), (64, 2, 70000, 0, 1), (7, 7, 65536, 0, 1),
     (7, 7, 100000, 60000, 1), (1, 1, 300000, 0, 1), (1, 1, 65535 * 8, 0, 1),
     (1, 1, 65535 * 8 + 1, 0, None), (64, 8, 1 << 20, 0, None)])
 def test_prompt_forms_take_their_rows(query_heads, kv_heads, rows, first, shared):
