@@ -734,8 +734,9 @@ uint32_t qllm_attention_paged_q4h_shared_splits(
 
 /* The form and the splits, 1 to `most`, with which a prompt's launch at head_dim 128
  * (split_tokens 0) takes the least time: 1 for qllm_attention_paged_q4h_prompt, 0 for
- * qllm_attention_paged_q4h_batched, which takes an eighth as many rows.  Reads the
- * launch's sizes alone; *splits is 0 for sizes that neither takes. */
+ * qllm_attention_paged_q4h_batched, which takes an eighth as many rows and is estimated
+ * with tail_alone 1.  Reads the launch's sizes alone; *splits is 0 for sizes that neither
+ * takes. */
 uint32_t qllm_attention_paged_q4h_prompt_form(
     const qllm_q4h_attention_launch* launch, uint32_t batch_rows, uint32_t most,
     uint32_t* splits);

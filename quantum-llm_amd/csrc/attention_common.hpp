@@ -233,8 +233,10 @@ __device__ __forceinline__ void store_attention_outputs(f32x4 result, float sum,
                                                         void* output,
                                                         uint32_t output_kind,
                                                         size_t index) {
-  // (the quotients of one divisor: its reciprocal once, then product and remainder,
-  // which rounds as a division does; infinities have no remainder)
+  // (the quotients of one divisor: its correctly rounded reciprocal once, then the product
+  // and its remainder - P. Markstein, "Computation of elementary functions on the IBM RISC
+  // System/6000 processor", 1990: rounded as the division where the remainder does not
+  // underflow, that is for outputs from some 2^-100 on; infinities have no remainder)
   const float inverse = 1.0f / sum;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {

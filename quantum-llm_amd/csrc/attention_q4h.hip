@@ -2806,14 +2806,6 @@ uint32_t shared_parts(const qllm_q4h_attention_launch& launch) {
 // 5500 launches over eight head layouts (24 on 4, 16 on 8, 16 on 2, 64 on 8, 16 on 16,
 // 8 on 1, 24 on 2, 32 on 32), 2 to 3000 rows after 0 to 9000 tokens, one to eight
 // splits: 5 and 9 % root mean square error.
-// From this many workgroups of shared tiles on they write the outputs of a single split
-// themselves.  64 heads on 8 at head_dim 128: 6000 rows (1000 workgroups) 792 -> 749 us,
-// 1000 (168) 80.6 -> 75.8, 400 (72) 42.0 -> 41.0, but 300 (56) 36.9 -> 37.6 and 200 (40)
-// 29.2 -> 31.0: a few workgroups take longer over the divisions and the 32-byte pieces
-// of their rows than a launch over all compute units.  (At head_dim 256, whose rows are
-// gated, 3001 rows of 24 heads on 4 in 564 workgroups gain nothing: the combine stays.)
-constexpr uint32_t kDirectWorkgroups = 64u;
-
 struct LaunchTiles {
   double rounds;     // of workgroups over the compute units
   double longest;    // tiles of the last rows' workgroup
@@ -2901,8 +2893,9 @@ double batches_128_us(const qllm_q4h_attention_launch& launch, uint32_t batch_ro
   const auto walked = [&](uint64_t rows) {
     const double tiles =
         static_cast<double>((launch.first_context_tokens + rows + 62u) / 64u);
+    // (the deal of the split kernel with tail_alone: an even one of a single split, a tile
+    // a wave where there are enough, otherwise fewer for its last waves)
     if (splits == 1u) return std::ceil(tiles / kSplitWaves);
-    // (the deal of the split kernel: a tile a wave, or its last waves walk fewer)
     if (tiles <= kSplitWaves * (splits - 1.0) + 1.0) return 1.0;
     const double share = (tiles + 2.0 * kSplitWaves) / (kSplitWaves * splits);
     return 0.75 * std::ceil(share - 0.03) + 0.25 * share;
@@ -3118,6 +3111,14 @@ extern "C" uint32_t qllm_attention_paged_q4h_prompt_form(
   return shared;
 }
 
+// From this many workgroups of shared tiles on they write the outputs of a single split
+// themselves.  64 heads on 8 at head_dim 128: 6000 rows (1000 workgroups) 792 -> 749 us,
+// 1000 (168) 80.6 -> 75.8, 400 (72) 42.0 -> 41.0, but 300 (56) 36.9 -> 37.6 and 200 (40)
+// 29.2 -> 31.0: a few workgroups take longer over the divisions and the 32-byte pieces
+// of their rows than a launch over all compute units.  (At head_dim 256, whose rows are
+// gated, 3001 rows of 24 heads on 4 in 564 workgroups gain nothing: the combine stays.)
+constexpr uint32_t kDirectWorkgroups = 64u;
+
 extern "C" int32_t qllm_attention_paged_q4h_prompt(
     const qllm_q4h_attention_launch* launch, uint32_t batch_rows) {
   if (!launch || !launch->query || !launch->page_table || !launch->output ||
@@ -3158,7 +3159,6 @@ extern "C" int32_t qllm_attention_paged_q4h_prompt(
   args.query_heads = launch->query_heads;
   args.kv_heads = launch->kv_heads;
   args.maximum_splits = launch->maximum_splits;
-  args.tail_alone = launch->tail_alone != 0 ? 1u : 0u;
   args.batch_rows = batch_rows;
   const uint32_t parts = (batches + kPromptBatches - 1u) / kPromptBatches;
   if (launch->kv_heads * parts >= kDirectWorkgroups &&

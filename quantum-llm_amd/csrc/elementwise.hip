@@ -493,8 +493,8 @@ __global__ __launch_bounds__(1024) void rms_norm_q8_kernel(
   __shared__ float scratch[16];
   const size_t row = blockIdx.x;
   rms_norm_row_wide<SLOTS>(input + row * elements, weight, nullptr, nullptr, 0u, elements,
-                    epsilon, zero_centered, scratch, nullptr, 0u, 0u, nullptr,
-                    output_q8 + row * elements, scales + row);
+                           epsilon, zero_centered, scratch, nullptr, 0u, 0u, nullptr,
+                           output_q8 + row * elements, scales + row);
 }
 
 // The same on a row that is first completed from K-split partial sums
@@ -506,11 +506,11 @@ __global__ __launch_bounds__(1024) void rms_norm_residual_q8_kernel(
     uint32_t elements, float epsilon, bool zero_centered) {
   __shared__ float scratch[16];
   const size_t row = blockIdx.x;
-  rms_norm_row_wide<SLOTS, true>(residual ? residual + row * elements : nullptr, weight, nullptr,
-                    nullptr, 0u, elements, epsilon, zero_centered, scratch,
-                    partials + row * elements, partial_count,
-                    static_cast<size_t>(gridDim.x) * elements, sum + row * elements,
-                    output_q8 + row * elements, scales + row);
+  rms_norm_row_wide<SLOTS, true>(
+      residual ? residual + row * elements : nullptr, weight, nullptr, nullptr, 0u,
+      elements, epsilon, zero_centered, scratch, partials + row * elements, partial_count,
+      static_cast<size_t>(gridDim.x) * elements, sum + row * elements,
+      output_q8 + row * elements, scales + row);
 }
 
 // sum[r] = residual[r] + partials[0][r] + ... + partials[count-1][r] (from zero
@@ -524,10 +524,10 @@ __global__ __launch_bounds__(1024) void rms_norm_residual_kernel(
     uint16_t* output_bf16, uint32_t elements, float epsilon, bool zero_centered) {
   __shared__ float scratch[16];
   const size_t row = blockIdx.x;
-  rms_norm_row_wide<SLOTS, true>(residual ? residual + row * elements : nullptr, weight, nullptr,
-                    output_bf16 + row * elements, elements, elements, epsilon,
-                    zero_centered, scratch, partials + row * elements,
-                    partial_count, partial_stride, sum + row * elements);
+  rms_norm_row_wide<SLOTS, true>(
+      residual ? residual + row * elements : nullptr, weight, nullptr,
+      output_bf16 + row * elements, elements, elements, epsilon, zero_centered, scratch,
+      partials + row * elements, partial_count, partial_stride, sum + row * elements);
 }
 
 // Calls launch(SLOTS, threads) for as few pieces a thread as hold a row; `two`: two of them
@@ -847,8 +847,6 @@ extern "C" int32_t qllm_rms_norm_residual_batch(
       elements % 4u != 0u || elements > 16384u || !aligned(hidden) ||
       !aligned(partials) || !aligned(output_bf16) || (weight && !aligned(weight)))
     return fail(QLLM_INVALID_ARGUMENT, "invalid residual RMSNorm");
-  // (measured on rows of 5120: 320 threads, four float4 each, take 6.0 us
-  // against 4.75 us with 1024: one CU's few waves wait longer for the row)
   with_row_slots(elements, true, [&]<int SLOTS>(std::integral_constant<int, SLOTS>,
                                                 uint32_t threads) {
     rms_norm_residual_kernel<SLOTS><<<rows, threads, 0, as_stream(stream)>>>(

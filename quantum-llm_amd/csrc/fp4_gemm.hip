@@ -1092,8 +1092,8 @@ extern "C" int32_t qllm_fp4_head_argmax_handed(
     const qllm_fp4_matrix* matrix, const void* input, size_t input_bytes, float* logits,
     uint32_t batch, uint32_t* tokens, void* workspace, size_t workspace_bytes,
     const qllm_rollout_step* advance, const qllm_token_handover* handover, void* stream) {
-  if (!handover_ok(handover) || !matrix_ok(matrix) || !input || !logits || !batch || batch > 8u || !tokens ||
-      !workspace || matrix->padded_columns % kChunk != 0u ||
+  if (!handover_ok(handover) || !matrix_ok(matrix) || !input || !logits || !batch ||
+      batch > 8u || !tokens || !workspace || matrix->padded_columns % kChunk != 0u ||
       workspace_bytes < qllm_fp4_head_workspace_bytes(matrix, batch) ||
       input_bytes < static_cast<size_t>(batch) * matrix->padded_columns * 2u ||
       (advance && (batch != 1u || !advance->next_token || !advance->draft_tokens ||

@@ -360,9 +360,9 @@ __device__ __forceinline__ i32x4 query_operand(const float* source, uint32_t d, 
 // map (a wave per 16 latent values), or, in the last workgroup along x, their
 // rotated parts.
 //
-// STORE: one more workgroup along x, of as many heads as there are rows, leaves a cache row, which the next
-// launch reads; the queries do not.  As a launch of its own that took 4.7 us of a decoded
-// token's layer.
+// STORE: one more workgroup along x, of as many heads as there are rows, leaves a cache
+// row, which the next launch reads; the queries do not.  As a launch of its own that took
+// 4.7 us of a decoded token's layer.
 template <bool STORE>
 __global__ __launch_bounds__(256) void latent_query_kernel(AttentionArgs args,
                                                            qllm_latent_store_launch store) {

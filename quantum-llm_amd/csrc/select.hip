@@ -705,14 +705,10 @@ extern "C" size_t qllm_topk_batch_workspace_bytes(uint32_t count,
 }
 
 namespace {
-int32_t topk_rows(const float* values, uint32_t count,
-                                          size_t row_stride, uint32_t top_k,
-                                          uint32_t rows, float* output_values,
-                                          uint32_t* output_indices,
-                                          void* workspace,
-                                          size_t workspace_bytes,
-                                          uint32_t* host_sequences,
-                                          uint32_t sequence, void* stream) {
+int32_t topk_rows(const float* values, uint32_t count, size_t row_stride, uint32_t top_k,
+                  uint32_t rows, float* output_values, uint32_t* output_indices,
+                  void* workspace, size_t workspace_bytes, uint32_t* host_sequences,
+                  uint32_t sequence, void* stream) {
   if (!values || !count || !top_k || top_k > kSelectMaxK || top_k > count ||
       !rows || rows > 65535u || row_stride < count || !output_values ||
       !output_indices || !workspace ||
