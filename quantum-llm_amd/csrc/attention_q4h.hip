@@ -2867,59 +2867,87 @@ bool shares_tiles(const qllm_q4h_attention_launch& launch, uint32_t batch_rows) 
              batched_us(launch, batch_rows, launch.maximum_splits);
 }
 
-// partial outputs written and read, and the launch; a single split has none
-double combine_128_us(const qllm_q4h_attention_launch& launch, uint32_t splits) {
-  return splits == 1u ? 0.0
-                      : 2.0 + static_cast<double>(launch.rows) * launch.query_heads *
-                                  splits * 820.0 / 5.3e6;
+// From this many workgroups of shared tiles on they write the outputs of a single split
+// themselves.  64 heads on 8 at head_dim 128: 6000 rows (1000 workgroups) 792 -> 749 us,
+// 1000 (168) 80.6 -> 75.8, 400 (72) 42.0 -> 41.0, but 300 (56) 36.9 -> 37.6 and 200 (40)
+// 29.2 -> 31.0: a few workgroups take longer over the divisions and the 32-byte pieces
+// of their rows than a launch over all compute units.  (At head_dim 256, whose rows are
+// gated, 3001 rows of 24 heads on 4 in 564 workgroups gain nothing: the combine stays.)
+constexpr uint32_t kDirectWorkgroups = 64u;
+
+// A prompt's attention at head_dim 128: as batches of their own, whose workgroups (82 KiB
+// of LDS, one to a compute unit) deal a context's tiles over eight waves, or as shared
+// tiles, eight batches to a workgroup.  What either takes, in microseconds, fitted to 1479
+// sizes (7 to 6000 rows after none to 22000 tokens, sixteen head layouts) with 1 to 8
+// splits, 4.6 and 3.1 % off near the best of them.  Batches of their own up to 31 of them,
+// splits for one workgroup a compute unit rounded up, take up to 3.1 times as long: 256
+// workgroups and a few more are two rounds (120 rows of 64 heads after 2048 tokens 42.6 us
+// in two splits, 30.8 in one), and a few hundred rows fill the chip in batches of their own
+// (300 rows from the first on 38 us shared, 27 so).
+//
+// Workgroups that take from `longest` down to `shortest`, in this order, on 256 compute
+// units: one round is as long as the longest; what is left of a second begins where the
+// first ends, and such pairs take the same all along; of more rounds their mean counts,
+// and `left` of a short one where the last round is not full.
+double rounds_us(uint64_t workgroups, double longest, double shortest, double pair,
+                 double mean, double left) {
+  if (workgroups <= 256u) return longest;
+  const double rounds = static_cast<double>(workgroups) / 256.0;
+  return std::max({longest, 2.0 * pair * (longest - (longest - shortest) / rounds),
+                   mean * rounds * 0.5 * (longest + shortest) +
+                       left * shortest * (std::ceil(rounds) - rounds)});
 }
 
-// A prompt's attention at head_dim 128: as batches of
-// their own, whose workgroups (82 KiB of LDS, one to a compute unit) deal a context's
-// tiles over eight waves, or as shared tiles, eight batches to a workgroup.  Fitted to
-// 320 sizes (9 to 2500 rows after 1 to 8000 tokens; 64 heads on 8, 16 on 4, 32 on 32 and
-// on 8) with 1 to 8 splits: the choice takes 0.3 % longer than the best one on average
-// and 7 % at most.  Batches of their own up to 31 of them, splits for one workgroup a
-// compute unit rounded up, took 19 % on average and 3.1 times at most: 256 workgroups
-// and a few more are two rounds (120 rows of 64 heads after 2048 tokens 42.6 us in two
-// splits, 30.8 in one), and a few hundred rows fill the chip in batches of their own
-// (300 rows from the first on 38 us shared, 27 so).
 double batches_128_us(const qllm_q4h_attention_launch& launch, uint32_t batch_rows,
                       uint32_t splits) {
   const uint32_t group = launch.query_heads / launch.kv_heads;
   const uint32_t first_rows = std::min(batch_rows, launch.rows);
   const uint64_t batches = (uint64_t{launch.rows} + batch_rows - 1u) / batch_rows;
-  const uint64_t rounds = (batches * launch.kv_heads * splits + 255u) / 256u;
-  const auto walked = [&](uint64_t rows) {
+  const uint32_t row_tiles = std::min((first_rows * group + 15u) / 16u, 3u);
+  const double base[] = {3.75, 4.9, 6.4}, tile[] = {2.55, 3.2, 4.2};
+  const auto batch_us = [&](uint64_t rows) {
     const double tiles =
         static_cast<double>((launch.first_context_tokens + rows + 62u) / 64u);
     // (the deal of the split kernel with tail_alone: an even one of a single split, a tile
     // a wave where there are enough, otherwise fewer for its last waves)
-    if (splits == 1u) return std::ceil(tiles / kSplitWaves);
-    if (tiles <= kSplitWaves * (splits - 1.0) + 1.0) return 1.0;
-    const double share = (tiles + 2.0 * kSplitWaves) / (kSplitWaves * splits);
-    return 0.75 * std::ceil(share - 0.03) + 0.25 * share;
+    double walked = std::ceil(tiles / kSplitWaves);
+    if (splits > 1u)
+      walked = tiles <= kSplitWaves * (splits - 1.0) + 1.0
+                   ? 1.0
+                   : std::ceil((tiles + 2.0 * kSplitWaves) / (kSplitWaves * splits) - 0.03);
+    return base[row_tiles - 1u] + tile[row_tiles - 1u] * walked;
   };
-  const double longest = walked(launch.rows);
-  const double each = rounds == 1u ? longest : 0.5 * (longest + walked(first_rows));
-  const uint32_t row_tiles = std::min((first_rows * group + 15u) / 16u, 3u);
-  const double base[] = {6.0, 7.5, 9.0}, tile[] = {2.3, 3.1, 3.75};
-  return static_cast<double>(rounds) *
-             (base[row_tiles - 1u] + tile[row_tiles - 1u] * each) +
-         combine_128_us(launch, splits);
+  const double time = 2.5 + rounds_us(batches * launch.kv_heads * splits,
+                                      batch_us(launch.rows), batch_us(first_rows), 0.93,
+                                      1.1, 0.77);
+  // (partial outputs written and read, and the combine's launch)
+  return splits == 1u ? time
+                      : time + 0.52 +
+                            2.5e-4 * static_cast<double>(launch.rows) *
+                                launch.query_heads * splits;
 }
 
 double shared_128_us(const qllm_q4h_attention_launch& launch, uint32_t batch_rows,
                      uint32_t splits) {
   const uint64_t batches = (uint64_t{launch.rows} + batch_rows - 1u) / batch_rows;
   const uint64_t parts = (batches + kPromptBatches - 1u) / kPromptBatches;
-  const LaunchTiles t =
-      tiles_of_launch(launch, parts * launch.kv_heads * splits,
-                      uint64_t{batch_rows} * kPromptBatches, splits);
+  const uint64_t waves = std::min<uint64_t>(batches, kPromptBatches);
   // (from five waves on two share a SIMD)
-  return 9.0 + 5.0 * t.rounds +
-         (batches > 4u ? 3.5 : 2.0) * std::max(std::ceil(t.longest), t.all) +
-         (splits == 1u ? 1.0 : combine_128_us(launch, splits));
+  const double tile = waves > 4u ? 3.5 : 2.23;
+  const auto part_us = [&](uint64_t rows) {
+    const double tiles =
+        static_cast<double>((launch.first_context_tokens + rows + 62u) / 64u);
+    return 1.02 * static_cast<double>(waves) + tile * std::ceil(tiles / splits);
+  };
+  const double time =
+      8.8 + rounds_us(parts * launch.kv_heads * splits, part_us(launch.rows),
+                      part_us(std::min<uint64_t>(uint64_t{batch_rows} * kPromptBatches,
+                                                 launch.rows)),
+                      1.0, 1.08, 0.0);
+  const bool direct = splits == 1u && parts * launch.kv_heads >= kDirectWorkgroups;
+  return direct ? time
+                : time + 1.6e-4 * static_cast<double>(launch.rows) * launch.query_heads *
+                             splits;
 }
 
 // Rows of a launch in batches of their own, each a layer of the grid; shared tiles take
@@ -3086,12 +3114,11 @@ extern "C" uint32_t qllm_attention_paged_q4h_prompt_form(
     *splits = cuts;
   };
   // What the workgroups alone say - batches of their own up to 31 of them, splits for one
-  // workgroup a compute unit - unless the estimates promise a good part less: they are some
-  // 8 % off, and more where the second round is short.  Over 1479 sizes (7 to 6000 rows
-  // after none to 22000 tokens, sixteen head layouts) the estimates alone took up to 14 %
-  // longer than this and more than 3 % in 52; with the margin they take 0.77 of the time on
-  // average and more in two (4 and 6 %).
-  constexpr double kMargin = 0.13;
+  // workgroup a compute unit - unless the estimates promise a part less that is more than
+  // they are off.  Of the time of that rule alone 0.76 on average over the 1479 sizes and
+  // over 787 others, more than 3 % longer in two and one of them (6 and 5 %); without the
+  // margin in 23 of the former, by up to 12 %.
+  constexpr double kMargin = 0.05;
   const bool few = takes_alone && batches < 32u;
   const uint64_t workgroups = few ? alone : together;
   const auto filled =
@@ -3110,14 +3137,6 @@ extern "C" uint32_t qllm_attention_paged_q4h_prompt_form(
   }
   return shared;
 }
-
-// From this many workgroups of shared tiles on they write the outputs of a single split
-// themselves.  64 heads on 8 at head_dim 128: 6000 rows (1000 workgroups) 792 -> 749 us,
-// 1000 (168) 80.6 -> 75.8, 400 (72) 42.0 -> 41.0, but 300 (56) 36.9 -> 37.6 and 200 (40)
-// 29.2 -> 31.0: a few workgroups take longer over the divisions and the 32-byte pieces
-// of their rows than a launch over all compute units.  (At head_dim 256, whose rows are
-// gated, 3001 rows of 24 heads on 4 in 564 workgroups gain nothing: the combine stays.)
-constexpr uint32_t kDirectWorkgroups = 64u;
 
 extern "C" int32_t qllm_attention_paged_q4h_prompt(
     const qllm_q4h_attention_launch* launch, uint32_t batch_rows) {
