@@ -206,8 +206,12 @@ __device__ __forceinline__ void wave_tile_range(uint32_t context_tiles,
     const uint32_t others = slots - WAVES;   // slots of the other workgroups
     if (tail_alone && splits > 1u && context_tiles <= others + 1u) {
       const uint32_t before = context_tiles - 1u;
-      tile_first = slot < others ? slot * before / others : before + min(slot - others, 1u);
-      tile_last = slot < others ? (slot + 1u) * before / others : context_tiles;
+      // (its last wave, which has none of a few rows' records to encode: one row of 24 heads
+      // on 4 of 256 dimensions after 300 tokens 13.2 us with the first wave, 12.7 so)
+      tile_first = slot < others ? slot * before / others : before;
+      tile_last = slot < others       ? (slot + 1u) * before / others
+                  : slot + 1u == slots ? context_tiles
+                                       : before;
       return;
     }
     const uint32_t dealt = context_tiles + tail_work;

@@ -186,7 +186,7 @@ std::uint64_t Mi355DenseFp4Provider::kv_bytes_per_token_layer() const noexcept {
 // 32, which it fetches in one go.  Five rows, splits of 512 tokens and for a tile a wave: 16
 // heads on 4 of 128 dimensions after 1000 tokens 15.4 and 13.0 us, after 4000 14.3 and 13.0,
 // 24 heads on 4 of 256 after 4000 23.8 and 20.3; a context of one tile within a longest of
-// 4000 13.3 and 13.2, one row alone 9.8 and 10.0.
+// 4000 13.2 and 13.0, one row alone 9.6 and 9.7.
 // Over the exact cache, whose launches know their context: the splits where that has too
 // many tiles for one a wave.
 std::uint32_t Mi355DenseFp4Provider::verify_splits(std::uint32_t most) const noexcept {
